@@ -207,6 +207,11 @@ int mi8_gemm_fp8_splitk(const void* a, int a_dtype, int64_t lda, const void* b, 
                         int64_t M, int64_t N, int64_t K, const float* sa, int sa_is_vector, const float* sb,
                         int sb_is_vector, void* out, int out_dtype, int64_t ldc, int splits, void* workspace,
                         int64_t workspace_bytes, void* stream);
+/* out += that product, summed as mi8_gemm_fp8_accumulate does. */
+int mi8_gemm_fp8_splitk_accumulate(const void* a, int a_dtype, int64_t lda, const void* b, int b_dtype, int64_t ldb,
+                                   int64_t M, int64_t N, int64_t K, const float* sa, int sa_is_vector, const float* sb,
+                                   int sb_is_vector, void* out, int out_dtype, int64_t ldc, int splits, void* workspace,
+                                   int64_t workspace_bytes, void* stream);
 int mi8_gemm_splitk_suggest(int64_t M, int64_t N, int64_t K);
 int64_t mi8_gemm_splitk_workspace_bytes(int64_t M, int64_t N, int splits);
 

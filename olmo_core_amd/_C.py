@@ -77,6 +77,11 @@ _SIGNATURES = {
         [c_void_p, c_int, c_int64, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p,
          c_int, c_void_p, c_int, c_int64, c_int, c_void_p, c_int64, c_void_p],
     ),
+    "mi8_gemm_fp8_splitk_accumulate": (
+        c_int,
+        [c_void_p, c_int, c_int64, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p,
+         c_int, c_void_p, c_int, c_int64, c_int, c_void_p, c_int64, c_void_p],
+    ),
     "mi8_gemm_splitk_suggest": (c_int, [c_int64, c_int64, c_int64]),
     "mi8_gemm_splitk_workspace_bytes": (c_int64, [c_int64, c_int64, c_int]),
     "mi8_gemm_num_variants": (c_int, []),

@@ -7,7 +7,6 @@ namespace gemm {
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int BK = 128;  // bytes of K per LDS stage
 
@@ -26,7 +25,13 @@ struct GemmArgs {
 };
 
 
-__device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
+// The 16-byte chunk index of an LDS row r is XORed with swz16(r).  A fragment read of a 16x16x128 MFMA has lane l at row
+// l % 16, chunk 2 (l / 16) + q, i.e. four lanes per 128-byte row.  Which swizzles the LDS of gfx950 serves without bank
+// conflicts was found by timing all 4096 GF(2)-linear maps row -> 3 bits in a loop of ds_read_b128 from four waves: a
+// third of them run at the rate of a contiguous read, this is the one with the fewest terms; (r >> 1) & 7, which
+// would be conflict free if 16 consecutive lanes were served together over 64 banks, measured 28 % slower
+// (SQ_LDS_BANK_CONFLICT: half of the LDS cycles of the GEMM).
+__device__ __forceinline__ int swz16(int r) { return ((r >> 2) & 1) | (((r >> 1) & 1) << 2); }
 
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f)
 {

@@ -1,30 +1,25 @@
 // Scaled float8 GEMM on CDNA4 matrix cores:  C[M,N] = bf16( (A[M,K] . B[N,K]^T) * (1/sa) * (1/sb) ).
 //
-// Both operands are K-contiguous ("TN"), which is what v_mfma_f32_32x32x64_f8f6f4 wants: every lane feeds 32
-// consecutive K bytes of one row.  A workgroup owns a BM x BN tile of C, walks K in 128-byte steps through a
-// double-buffered LDS stage, and each wave accumulates a (BM/WM) x (BN/WN) sub-tile in fp32 registers.
+// Both operands are K-contiguous ("TN"), which is what the fp8 MFMAs want: every lane feeds 32 consecutive K bytes of
+// one row.
 //
-// LDS stage layout: [row][128 bytes]; the 16-byte chunk c of row r sits at chunk position c ^ swz(r),
-// swz(r) = (r ^ (r >> 3)) & 7, so that the 16-byte fragment reads of 32 different rows spread over all banks
-// while the stores (8 lanes per row) stay contiguous.
-//
-// This file holds that general tile kernel (any M, N; K % 16 == 0; bf16 or fp32 output), its split-K form for
-// problems with few output tiles, and the entry points, which pick a kernel by shape: the persistent direct-to-LDS
-// kernel of mi8_gemm_m16.hip for large problems, the weight-streaming kernel of mi8_gemm_skinny.hip for a few
-// rows of A.
-#include "mi8_gemm_body.h"
+// This file holds the kernels over the general tile routine of mi8_gemm_ring.h (any M, N; K % 16 == 0; bf16 or fp32
+// output), their split-K form for problems with few output tiles, and the entry points, which pick a kernel by shape:
+// the persistent direct-to-LDS kernel of mi8_gemm_m16.hip for large problems, the weight-streaming kernel of
+// mi8_gemm_skinny.hip for a few rows of A.
+#include "mi8_gemm_ring.h"
 
 namespace mi8 {
 using namespace gemm;
 namespace {
 
-template <int BM, int BN, int WM, int WN, int CBSZ, int BLGP>
-__global__ __launch_bounds__(WM * WN * 64, 1) void gemm_fp8_kernel(GemmArgs g)
+template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP>
+__global__ __launch_bounds__(kRingThreads, OCC) void gemm_fp8_ring_kernel(GemmArgs g)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     int tm, tn;
     if (!tile_of_block(g, tm, tn)) return;
-    gemm_tile_body<BM, BN, WM, WN, CBSZ, BLGP>(g, tm * BM, tn * BN, lds);
+    ring_tile<BM, BN, ST, CBSZ, BLGP>(g, tm * BM, tn * BN, lds);
 }
 
 // ---- split K ---------------------------------------------------------------------------------------
@@ -34,8 +29,6 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_fp8_kernel(GemmArgs g)
 // the raw fp32 sums into its own plane of a workspace; a second kernel adds the planes in a fixed order (the
 // result does not depend on scheduling), applies the scales and rounds.
 
-constexpr int kSplitTile = 128;
-
 struct SplitArgs {
     GemmArgs g;          // the problem; C, ldc, scales describe the final output
     float* planes;       // [splits][M][ld_plane] fp32
@@ -44,8 +37,8 @@ struct SplitArgs {
     int splits;
 };
 
-template <int CBSZ, int BLGP>
-__global__ __launch_bounds__(256, 1) void gemm_fp8_splitk_kernel(SplitArgs a)
+template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP>
+__global__ __launch_bounds__(kRingThreads, OCC) void gemm_fp8_splitk_kernel(SplitArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     GemmArgs g = a.g;
@@ -59,13 +52,15 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_splitk_kernel(SplitArgs a)
     g.K = left < a.steps_per_split * BK ? left : a.steps_per_split * BK;
     g.C = a.planes + (int64_t)split * g.M * a.ld_plane;
     g.c_f32 = 1;
+    g.accumulate = 0;
     g.ldc = a.ld_plane;
     g.sa = g.sb = nullptr;
     g.sa_vec = g.sb_vec = 0;
-    gemm_tile_body<kSplitTile, kSplitTile, 2, 2, CBSZ, BLGP>(g, tm * kSplitTile, tn * kSplitTile, lds);
+    ring_tile<BM, BN, ST, CBSZ, BLGP>(g, tm * BM, tn * BN, lds);
 }
 
-// out[m][n] = round( (sum over planes, in plane order) * (1/sa) * (1/sb) ); four columns per thread
+// out[m][n] (+)= round( (sum over planes, in plane order) * (1/sa) * (1/sb) ); four columns per thread.  Bound by the
+// latency of the plane reads: four are in flight at a time (one after the other: 7-11 us where this takes 4-6).
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(SplitArgs a)
 {
     const GemmArgs& g = a.g;
@@ -76,107 +71,165 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(SplitArgs a)
     const int n = (int)(q % quads_per_row) * 4;
     const int64_t plane = (int64_t)g.M * a.ld_plane;
     const float* p = a.planes + (int64_t)m * a.ld_plane + n;
-    float4 s = *reinterpret_cast<const float4*>(p);
-    for (int i = 1; i < a.splits; ++i) {
-        const float4 t = *reinterpret_cast<const float4*>(p + i * plane);
-        s.x += t.x;
-        s.y += t.y;
-        s.z += t.z;
-        s.w += t.w;
+    ring_v4f s = *reinterpret_cast<const ring_v4f*>(p);
+    int i = 1;
+    for (; i + 3 < a.splits; i += 4) {
+        ring_v4f t[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) t[u] = *reinterpret_cast<const ring_v4f*>(p + (i + u) * plane);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s += t[u];
     }
+    for (; i < a.splits; ++i) s += *reinterpret_cast<const ring_v4f*>(p + i * plane);
     // same scale arithmetic as the tile routine's own epilogue
     const float isa = g.sa_vec ? __builtin_amdgcn_rcpf(g.sa[m]) : 1.0f / g.sa[0];
-    const float isb_scalar = g.sb_vec ? 0.0f : 1.0f / g.sb[0];
-    const float v[4] = {s.x, s.y, s.z, s.w};
+    const float isb_single = g.sb_vec ? 0.0f : 1.0f / g.sb[0];
+    const bool both_single = !g.sa_vec && !g.sb_vec;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         if (n + j >= g.N) break;
-        const float isb = g.sb_vec ? __builtin_amdgcn_rcpf(g.sb[n + j]) : isb_scalar;
-        const float r = v[j] * isa * isb;
-        if (g.c_f32)
-            reinterpret_cast<float*>(g.C)[(int64_t)m * g.ldc + n + j] = r;
-        else
-            reinterpret_cast<uint16_t*>(g.C)[(int64_t)m * g.ldc + n + j] = f32_to_bf16_bits(r);
+        const float isb = g.sb_vec ? __builtin_amdgcn_rcpf(g.sb[n + j]) : isb_single;
+        const float r = both_single ? s[j] * (isa * isb) : s[j] * isa * isb;
+        if (g.c_f32) {
+            float* c = reinterpret_cast<float*>(g.C) + (int64_t)m * g.ldc + n + j;
+            *c = g.accumulate ? *c + r : r;
+        } else {
+            uint16_t* c = reinterpret_cast<uint16_t*>(g.C) + (int64_t)m * g.ldc + n + j;
+            uint16_t h = f32_to_bf16_bits(r);
+            if (g.accumulate) h = f32_to_bf16_bits(bits_to_f32((uint32_t)*c << 16) + bits_to_f32((uint32_t)h << 16));
+            *c = h;
+        }
     }
 }
 
-template <int CBSZ, int BLGP>
-int launch_splitk_typed(const SplitArgs& a, hipStream_t st)
+// ---- tile shapes of the ring kernels and what a problem costs on them ---------------------------------------------
+
+struct RingShape {
+    const char* name;
+    int bm, bn;
+    float step1;  // us per 128-byte K step with one workgroup on a compute unit ...
+    float step2;  // ... and for a pair of them sharing one (0: only one fits)
+    float tile;   // us per tile outside the K loop
+};
+
+// (measured on shapes from 300 x 2048 x 768 to 4096 x 2048 x 8192; the model below meets them within 15 %)
+constexpr RingShape kRing[] = {
+    {"64x64_ring4", 64, 64, 0.28f, 0.39f, 1.2f},
+    {"128x64_ring3", 128, 64, 0.40f, 0.64f, 1.2f},
+    {"64x128_ring3", 64, 128, 0.40f, 0.64f, 1.2f},
+    {"128x128_ring2", 128, 128, 0.72f, 1.0f, 1.5f},
+    {"128x128_ring3", 128, 128, 0.60f, 0.0f, 1.5f},
+};
+constexpr int kNumRing = sizeof(kRing) / sizeof(kRing[0]);
+constexpr float kLaunchUs = 2.6f;
+
+// time of a problem of `slices` independent slices of `steps` K steps on tile shape r, launch included
+float ring_cost(const RingShape& r, int64_t M, int64_t N, int64_t steps, int64_t slices)
 {
-    auto kern = gemm_fp8_splitk_kernel<CBSZ, BLGP>;
-    constexpr int lds_bytes = 2 * (kSplitTile + kSplitTile) * BK;
-    static std::atomic<uint64_t> configured{0};
-    if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, configured, "mi8_gemm_fp8_splitk"))
-        return rc;
-    const int total = a.g.tiles_m * a.g.tiles_n;
-    hipLaunchKernelGGL(kern, dim3(((total + 7) / 8) * 8, a.splits), dim3(256), lds_bytes, st, a);
-    const int64_t quads = (int64_t)a.g.M * (a.ld_plane / 4);
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, a);
-    return launch_status("mi8_gemm_fp8_splitk");
+    const int64_t tiles = ((M + r.bm - 1) / r.bm) * ((N + r.bn - 1) / r.bn) * slices;
+    const int64_t per_cu = (tiles + 255) / 256;
+    if (per_cu == 1 || r.step2 == 0.0f) return kLaunchUs + per_cu * (steps * r.step1 + r.tile);
+    return kLaunchUs + 0.5f * per_cu * (steps * r.step2 + r.tile);
 }
 
-// slices for a problem, 1 = do not split: aim at two workgroups per compute unit, at least four K steps a slice
+int best_ring(int64_t M, int64_t N, int64_t steps, int64_t slices, float* cost)
+{
+    int best = 0;
+    float c = 0.0f;
+    for (int i = 0; i < kNumRing; ++i) {
+        const float t = ring_cost(kRing[i], M, N, steps, slices);
+        if (i == 0 || t < c) {
+            best = i;
+            c = t;
+        }
+    }
+    *cost = c;
+    return best;
+}
+
+// the same for the persistent kernel: rounds of 256 tiles, a full round running at the clock the power limit leaves
+float persistent_cost(int64_t M, int64_t N, int64_t steps)
+{
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
+    const int64_t full = tiles / 256, rest = tiles % 256;
+    float t = 3.0f + full * (steps * 1.35f + 5.0f);
+    if (rest) t += steps * (1.0f + 0.35f * (rest > 128 ? (rest - 128) / 128.0f : 0.0f)) + 5.0f;
+    return t;
+}
+
+// Slices for a problem, 1 = do not split: a summation order of its own, so it depends on the product alone.  Splitting
+// pays where the whole of K in one workgroup is the time (few tiles, a long K) and costs a second launch that reads the
+// planes; up to 192 tiles of 64 x 64 it is at worst even.  At least four K steps a slice.
 int suggested_splits(int64_t M, int64_t N, int64_t K)
 {
-    const int64_t tiles = ((M + kSplitTile - 1) / kSplitTile) * ((N + kSplitTile - 1) / kSplitTile);
+    const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256), tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
     const int64_t steps = (K + BK - 1) / BK;
-    if (M <= 16 || tiles > 256 || steps < 8) return 1;  // (up to 16 rows: the few-rows kernel reads B once)
-    int64_t s = 512 / tiles;
-    if (s > steps / 4) s = steps / 4;
-    if (s > 32) s = 32;
-    if (s < 2) return 1;
-    const int64_t per = (steps + s - 1) / s;
-    return (int)((steps + per - 1) / per);  // no empty slice
+    if (M <= 16 || tiles256 > 96 || steps < 8) return 1;  // (up to 16 rows: the few-rows kernel reads B once)
+    float best;
+    best_ring(M, N, steps, 1, &best);
+    if (tiles64 <= 192) best = 1e30f;
+    int64_t splits = 1;
+    for (int64_t s = 2; s <= 32 && s <= steps / 4; ++s) {
+        const int64_t per = (steps + s - 1) / s;
+        if ((s - 1) * per >= steps) continue;  // the last slice would be empty
+        float t;
+        best_ring(M, N, per, s, &t);
+        t += 2.2f + (float)(M * N) * (4.0f * s + 2.0f) / 4.0e6f;
+        if (t < best) {
+            best = t;
+            splits = s;
+        }
+    }
+    return (int)splits;
 }
 
-// ---- variants --------------------------------------------------------------------------------------
+// ---- variants: the ring tile shapes, then the other two kernels ----------------------------------------------------
 
-struct Variant {
-    const char* name;
-    int bm, bn, threads;
-};
+constexpr int kM16 = kNumRing, kSkinny = kNumRing + 1, kNumVariants = kNumRing + 2;
 
-constexpr Variant kVariants[] = {
-    {"256x256_w2x2", 256, 256, 256},
-    {"256x256_w2x4", 256, 256, 512},
-    {"128x128_w2x2", 128, 128, 256},
-    {"256x128_w2x2", 256, 128, 256},
-    {"128x256_w2x2", 128, 256, 256},
-    {"256x256_dma_w4x128_m16x128", 256, 256, 256},
-    {"rows64x16_k8_m16x128", 64, 16, 512},
-};
-constexpr int kSmallTile = 2, kM16 = 5, kSkinny = 6;
-constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
-
-template <int BM, int BN, int WM, int WN, int CBSZ, int BLGP>
-int launch_one(const GemmArgs& g, hipStream_t st)
+template <typename Args, typename Kernel>
+int launch_ring_kernel(Kernel kern, std::atomic<uint64_t>& configured, int lds_bytes, const Args& a, int tiles, int slices,
+                       hipStream_t st, const char* what)
 {
-    auto kern = gemm_fp8_kernel<BM, BN, WM, WN, CBSZ, BLGP>;
-    constexpr int lds_bytes = 2 * (BM + BN) * BK;
-    static std::atomic<uint64_t> configured{0};
-    if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, configured, "mi8_gemm_fp8"))
-        return rc;
-    const int total = g.tiles_m * g.tiles_n;
-    const int blocks = ((total + 7) / 8) * 8;
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(WM * WN * 64), lds_bytes, st, g);
-    return launch_status("mi8_gemm_fp8");
+    if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, configured, what)) return rc;
+    hipLaunchKernelGGL(kern, dim3((tiles + 7) / 8 * 8, slices), dim3(kRingThreads), lds_bytes, st, a);
+    return launch_status(what);
+}
+
+template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP>
+int launch_ring(GemmArgs& g, SplitArgs* split, hipStream_t st)
+{
+    GemmArgs& p = split ? split->g : g;
+    p.tiles_m = (p.M + BM - 1) / BM;
+    p.tiles_n = (p.N + BN - 1) / BN;
+    const int tiles = p.tiles_m * p.tiles_n;
+    static std::atomic<uint64_t> configured[2];
+    if (split)
+        return launch_ring_kernel(gemm_fp8_splitk_kernel<BM, BN, ST, OCC, CBSZ, BLGP>, configured[1], kRingLdsBytes<BM, BN, ST>,
+                                  *split, tiles, split->splits, st, "mi8_gemm_fp8_splitk");
+    return launch_ring_kernel(gemm_fp8_ring_kernel<BM, BN, ST, OCC, CBSZ, BLGP>, configured[0], kRingLdsBytes<BM, BN, ST>, g,
+                              tiles, 1, st, "mi8_gemm_fp8");
 }
 
 template <int CBSZ, int BLGP>
-int launch_variant(int variant, GemmArgs& g, hipStream_t st)
+int launch_ring_shape(int shape, GemmArgs& g, SplitArgs* split, hipStream_t st)
 {
-    const Variant& v = kVariants[variant];
-    g.tiles_m = (g.M + v.bm - 1) / v.bm;
-    g.tiles_n = (g.N + v.bn - 1) / v.bn;
-    switch (variant) {
-        case 0: return launch_one<256, 256, 2, 2, CBSZ, BLGP>(g, st);
-        case 1: return launch_one<256, 256, 2, 4, CBSZ, BLGP>(g, st);
-        case 2: return launch_one<128, 128, 2, 2, CBSZ, BLGP>(g, st);
-        case 3: return launch_one<256, 128, 2, 2, CBSZ, BLGP>(g, st);
-        case 4: return launch_one<128, 256, 2, 2, CBSZ, BLGP>(g, st);
+    switch (shape) {
+        case 0: return launch_ring<64, 64, 4, 2, CBSZ, BLGP>(g, split, st);
+        case 1: return launch_ring<128, 64, 3, 2, CBSZ, BLGP>(g, split, st);
+        case 2: return launch_ring<64, 128, 3, 2, CBSZ, BLGP>(g, split, st);
+        case 3: return launch_ring<128, 128, 2, 2, CBSZ, BLGP>(g, split, st);
+        case 4: return launch_ring<128, 128, 3, 1, CBSZ, BLGP>(g, split, st);
     }
-    set_error("mi8_gemm_fp8: unknown variant %d", variant);
+    set_error("mi8_gemm_fp8: unknown variant %d", shape);
     return MI8_ERR_ARG;
+}
+
+int launch_ring_typed(int shape, int a_dtype, int b_dtype, GemmArgs& g, SplitArgs* split, hipStream_t st)
+{
+    if (a_dtype == MI8_E4M3)
+        return b_dtype == MI8_E4M3 ? launch_ring_shape<0, 0>(shape, g, split, st) : launch_ring_shape<0, 1>(shape, g, split, st);
+    return b_dtype == MI8_E4M3 ? launch_ring_shape<1, 0>(shape, g, split, st) : launch_ring_shape<1, 1>(shape, g, split, st);
 }
 
 }  // namespace
@@ -188,7 +241,8 @@ extern "C" int mi8_gemm_num_variants(void) { return kNumVariants; }
 
 extern "C" const char* mi8_gemm_variant_name(int variant)
 {
-    return (variant >= 0 && variant < kNumVariants) ? kVariants[variant].name : nullptr;
+    if (variant < 0 || variant >= kNumVariants) return nullptr;
+    return variant == kM16 ? "256x256_dma_w4x128_m16x128" : variant == kSkinny ? "rows64x16_k8_m16x128" : kRing[variant].name;
 }
 
 namespace {
@@ -221,22 +275,19 @@ int gemm_fp8_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b
     const bool dma_ok = (K % 128 == 0) && M >= 256 && N >= 256 && N % 8 == 0 && ldc % 8 == 0 && ldc < (1 << 22) && aligned16(out) &&
                         out_dtype == MI8_BF16 && (!sb_is_vector || aligned16(sb)) &&
                         (sa_is_vector != 0) == (sb_is_vector != 0) && (!accumulate || (M % 256 == 0 && N % 256 == 0));
-    // measured on MI355X on the benchmark configurations' shapes: the four-wave layout beats the eight-wave one
-    // by 0-14 %, and its 16x16x128 form beats its 32x32x64 form by 3-9 % (random operands, power-limited clocks).
-    // Problems with few 256 x 256 tiles leave most compute units idle and pay one memory latency per K step:
-    // 128 x 128 tiles put four times the workgroups to work (512 x 11008 x 4096: 42 us against 70 us), and a few
-    // rows of A go to the kernel that streams B once.
+    // A few rows of A go to the kernel that streams B once; everything else to whichever of the ring tile shapes and the
+    // persistent kernel the measured costs above say is fastest for this number of tiles and K steps (all of them give
+    // the same bits).
     if (variant < 0) {
-        const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
-        if (M <= kSkinnyMaxM && !accumulate)
+        if (M <= kSkinnyMaxM) {
             variant = kSkinny;
-        else if (dma_ok)
-            variant = tiles256 <= 96 ? kSmallTile : kM16;  // (mi8_gemm_fp8_swiglu_matches_separate mirrors this)
-        else
-            variant = tiles256 <= 384 ? kSmallTile : 1;
+        } else {
+            const int64_t steps = ceil_div(K, BK);
+            float cost;
+            variant = best_ring(M, N, steps, 1, &cost);
+            if (dma_ok && persistent_cost(M, N, steps) < cost) variant = kM16;
+        }
     }
-    MI8_REQUIRE(!(accumulate && variant == kSkinny), MI8_ERR_UNSUPPORTED,
-                "mi8_gemm_fp8_accumulate: the few-rows variant does not accumulate");
     if (variant == kSkinny) return launch_skinny(g, a_dtype, b_dtype, st);
     if (variant == kM16) {
         MI8_REQUIRE(dma_ok, MI8_ERR_UNSUPPORTED,
@@ -245,9 +296,7 @@ int gemm_fp8_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b
                     (long long)M, (long long)N, (long long)K, (long long)ldc);
         return launch_m16(g, a_dtype, b_dtype, st);
     }
-    if (a_dtype == MI8_E4M3)
-        return b_dtype == MI8_E4M3 ? launch_variant<0, 0>(variant, g, st) : launch_variant<0, 1>(variant, g, st);
-    return b_dtype == MI8_E4M3 ? launch_variant<1, 0>(variant, g, st) : launch_variant<1, 1>(variant, g, st);
+    return launch_ring_typed(variant, a_dtype, b_dtype, g, nullptr, st);
 }
 }  // namespace
 
@@ -268,8 +317,9 @@ extern "C" int mi8_gemm_fp8_accumulate(const void* a, int a_dtype, int64_t lda, 
                           ldc, -1, true, stream);
 }
 
-// 1 if mi8_gemm_fp8_swiglu takes the shape AND mi8_gemm_fp8 would run both projections on the same persistent
-// kernel (then the fused launch reproduces the three-call route bit for bit; other tile kernels sum in another order)
+// 1 if mi8_gemm_fp8_swiglu takes the shape AND the library would not cut either projection along K (then the fused
+// launch reproduces the three-call route bit for bit: all kernels that do not split sum in one order); fewer tiles go to
+// the separate calls
 extern "C" int mi8_gemm_fp8_swiglu_matches_separate(int64_t M, int64_t H, int64_t K)
 {
     if (M < 256 || H < 256 || K <= 0 || K % 128 || H % 8) return 0;
@@ -307,8 +357,8 @@ extern "C" int mi8_gemm_fp8_swiglu(const void* a, int a_dtype, int64_t lda, cons
     return rc;
 }
 
-// 1 if mi8_gemm_fp8_codes takes the shape: the shapes mi8_gemm_fp8 runs on the persistent tile kernel (so that the
-// output has the bits of the plain call) whose row segments line up with the output tiles
+// 1 if mi8_gemm_fp8_codes takes the shape: shapes that the library never cuts along K (so that the output has the bits
+// of the plain call) whose row segments line up with the output tiles
 extern "C" int mi8_gemm_fp8_codes_supported(int64_t M, int64_t N, int64_t K)
 {
     if (M < 256 || N < 256 || K <= 0 || K % 128 || N % 64) return 0;
@@ -349,10 +399,11 @@ extern "C" int64_t mi8_gemm_splitk_workspace_bytes(int64_t M, int64_t N, int spl
     return (int64_t)splits * M * ((N + 3) / 4 * 4) * (int64_t)sizeof(float);
 }
 
-extern "C" int mi8_gemm_fp8_splitk(const void* a, int a_dtype, int64_t lda, const void* b, int b_dtype, int64_t ldb,
+namespace {
+int splitk_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b_dtype, int64_t ldb,
                                    int64_t M, int64_t N, int64_t K, const float* sa, int sa_is_vector,
                                    const float* sb, int sb_is_vector, void* out, int out_dtype, int64_t ldc,
-                                   int splits, void* workspace, int64_t workspace_bytes, void* stream)
+                                   int splits, void* workspace, int64_t workspace_bytes, bool accumulate, void* stream)
 {
     MI8_REQUIRE(a && b && sa && sb && out && workspace, MI8_ERR_ARG, "mi8_gemm_fp8_splitk: null pointer");
     MI8_REQUIRE((a_dtype == MI8_E4M3 || a_dtype == MI8_E5M2) && (b_dtype == MI8_E4M3 || b_dtype == MI8_E5M2),
@@ -381,14 +432,35 @@ extern "C" int mi8_gemm_fp8_splitk(const void* a, int a_dtype, int64_t lda, cons
                 (long long)mi8_gemm_splitk_workspace_bytes(M, N, used));
     SplitArgs s{};
     s.g = GemmArgs{(const uint8_t*)a, (const uint8_t*)b, out, out_dtype == MI8_F32 ? 1 : 0, lda, ldb, ldc, (int)M,
-                   (int)N, (int)K, sa, sb, sa_is_vector ? 1 : 0, sb_is_vector ? 1 : 0,
-                   (int)((M + kSplitTile - 1) / kSplitTile), (int)((N + kSplitTile - 1) / kSplitTile)};
+                   (int)N, (int)K, sa, sb, sa_is_vector ? 1 : 0, sb_is_vector ? 1 : 0, 0, 0, accumulate ? 1 : 0};
     s.planes = (float*)workspace;
     s.ld_plane = (N + 3) / 4 * 4;
     s.steps_per_split = (int)per;
     s.splits = used;
     hipStream_t st = (hipStream_t)stream;
-    if (a_dtype == MI8_E4M3)
-        return b_dtype == MI8_E4M3 ? launch_splitk_typed<0, 0>(s, st) : launch_splitk_typed<0, 1>(s, st);
-    return b_dtype == MI8_E4M3 ? launch_splitk_typed<1, 0>(s, st) : launch_splitk_typed<1, 1>(s, st);
+    float cost;
+    const int shape = best_ring(M, N, per, used, &cost);
+    if (int rc = launch_ring_typed(shape, a_dtype, b_dtype, s.g, &s, st)) return rc;
+    const int64_t quads = M * (s.ld_plane / 4);
+    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, s);
+    return launch_status("mi8_gemm_fp8_splitk");
+}
+}  // namespace
+
+extern "C" int mi8_gemm_fp8_splitk(const void* a, int a_dtype, int64_t lda, const void* b, int b_dtype, int64_t ldb,
+                                   int64_t M, int64_t N, int64_t K, const float* sa, int sa_is_vector,
+                                   const float* sb, int sb_is_vector, void* out, int out_dtype, int64_t ldc,
+                                   int splits, void* workspace, int64_t workspace_bytes, void* stream)
+{
+    return splitk_entry(a, a_dtype, lda, b, b_dtype, ldb, M, N, K, sa, sa_is_vector, sb, sb_is_vector, out, out_dtype, ldc,
+                        splits, workspace, workspace_bytes, false, stream);
+}
+
+extern "C" int mi8_gemm_fp8_splitk_accumulate(const void* a, int a_dtype, int64_t lda, const void* b, int b_dtype, int64_t ldb,
+                                              int64_t M, int64_t N, int64_t K, const float* sa, int sa_is_vector,
+                                              const float* sb, int sb_is_vector, void* out, int out_dtype, int64_t ldc,
+                                              int splits, void* workspace, int64_t workspace_bytes, void* stream)
+{
+    return splitk_entry(a, a_dtype, lda, b, b_dtype, ldb, M, N, K, sa, sa_is_vector, sb, sb_is_vector, out, out_dtype, ldc,
+                        splits, workspace, workspace_bytes, true, stream);
 }

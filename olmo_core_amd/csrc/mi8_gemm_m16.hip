@@ -62,14 +62,6 @@ constexpr int WT = 128;                      // wave tile edge
 constexpr int NT = WT / 16;                  // MFMA tiles per wave tile edge
 constexpr int kLoads = 8;                    // direct loads per operand, step and wave (8 rows each)
 
-// The 16-byte chunk index of row r is XORed with swz16(r).  A fragment read has lane l at row l % 16, chunk
-// 2 (l / 16) + q, i.e. four lanes per 128-byte row.  Which swizzles the LDS of gfx950 serves without bank conflicts
-// was found by timing all 4096 GF(2)-linear maps row -> 3 bits in a loop of ds_read_b128 from four waves: a third
-// of them run at the rate of a contiguous read, this is the one with the fewest terms; (r >> 1) & 7, which
-// would be conflict free if 16 consecutive lanes were served together over 64 banks, measured 28 % slower
-// (SQ_LDS_BANK_CONFLICT: half of the LDS cycles of the GEMM).
-__device__ __forceinline__ int swz16(int r) { return ((r >> 2) & 1) | (((r >> 1) & 1) << 2); }
-
 // Maximum over every aligned group of eight lanes, of two independent 16-bit halves per register, by DPP moves (no
 // LDS traffic: an LDS instruction the compiler knows of would make it wait for the direct-to-LDS loads in flight);
 // all eight lanes end up with the result.

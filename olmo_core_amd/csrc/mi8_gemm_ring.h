@@ -1,0 +1,253 @@
+// The fp8 GEMM tile routine for everything the persistent kernel (mi8_gemm_m16.hip) is too coarse for: any M, N,
+// K % 16 == 0, bf16 or fp32 output, single scales or scale vectors; shared by the dense, split-K and grouped kernels.
+//
+// What bounds it: these are products with fewer tiles than fill the chip once or twice at 256 x 256, so a tile's time is
+// latency (the first operand bytes, one barrier and one LDS round trip per 128-byte K step, the epilogue) and, once two
+// workgroups share a compute unit, the operand bytes that come out of L2: (BM + BN) * 128 per step at about 80 B/ns and
+// compute unit.  Hence small tiles (64 or 128 on a side, four waves of (BM / 2) x (BN / 2)), operands that go from L2
+// straight to LDS (buffer loads with the LDS destination, no registers and no vector address arithmetic: one resident
+// lane offset per load and a uniform K offset), a ring of ST stages so that ST - 1 steps are in flight, and an LDS
+// footprint that lets two workgroups live on a compute unit, one computing while the other waits.
+//
+// The MFMA (v_mfma_f32_16x16x128_f8f6f4), the order of K and the scale arithmetic are those of the persistent kernel: a
+// product has the same bits on either.  Measured against the register-staged 128 x 128 tiles that were here before
+// (32x32x64 MFMAs, split along K where tiles were few), us per launch in a graph: 305 x 2816 x 1024 15.7 -> 5.6,
+// 1537 x 2048 x 2048 25.7 -> 12.3, 1999 x 1024 x 2816 23.4 -> 12.2, 512 x 4096 x 4096 27.9 -> 15.6.
+//
+// LDS stage: [row][128 bytes], A rows then B rows; 16-byte chunk c of row r sits at c ^ swz16(r) (the swizzle of the
+// persistent kernel), applied by permuting which global chunk a lane fetches.
+#pragma once
+#include "mi8_gemm.h"
+
+namespace mi8 {
+namespace gemm {
+namespace {
+
+typedef float ring_v4f __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* ring_lds_t;
+typedef const __attribute__((address_space(3))) v4i* ring_frag_t;
+
+// 16 bytes per lane from a raw buffer into LDS at dst + 16 * lane (dst uniform); lanes past the descriptor's end write zeros
+__device__ __forceinline__ void ring_load(__amdgpu_buffer_rsrc_t d, uint8_t* dst, int lane_offset, int offset)
+{
+#ifdef __HIP_DEVICE_COMPILE__  // (the builtin exists in the device pass only)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (ring_lds_t)dst, 16, lane_offset, offset, 0, 0);
+#endif
+}
+
+// all but the last N vector memory operations and every LDS operation of this wave have completed
+template <int N>
+__device__ __forceinline__ void ring_wait()
+{
+    static_assert(N < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x70);
+}
+
+template <int BM, int BN, int ST>
+constexpr int kRingLdsBytes = ST * (BM + BN) * BK;
+
+constexpr int kRingThreads = 256;
+
+// C[m0 .. m0 + BM, n0 .. n0 + BN] of g's product (K may be 0: zeros).  g.sa == null: the raw fp32 sums are wanted.
+template <int BM, int BN, int ST, int CBSZ, int BLGP>
+__device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const int n0, uint8_t* lds)
+{
+    constexpr int NW = kRingThreads / 64;
+    constexpr int WTM = BM / 2, WTN = BN / 2;  // wave tile
+    constexpr int TM = WTM / 16, TN = WTN / 16;
+    constexpr int STAGE = (BM + BN) * BK;
+    constexpr int LA = BM / 8 / NW, LB = BN / 8 / NW, LD = LA + LB;  // loads per wave and step: 8 rows x 128 bytes each
+    static_assert(LA * 8 * NW == BM && LB * 8 * NW == BN && ST >= 2 && ST <= 4 && LD * (ST - 2) < 64, "tile shape");
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const int r16 = lane & 15, kb = lane >> 4;
+
+    // ---- operand loads: load i of wave w fills rows 8 (4 i + w) .. + 7; rows past the edge re-read the last one
+    const int rows_a = g.M - m0 < BM ? g.M - m0 : BM, rows_b = g.N - n0 < BN ? g.N - n0 : BN;
+    const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(g.A + (int64_t)m0 * g.lda), 0, (int)(uint32_t)((int64_t)(rows_a - 1) * g.lda + g.K), 0x00020000);
+    const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(g.B + (int64_t)n0 * g.ldb), 0, (int)(uint32_t)((int64_t)(rows_b - 1) * g.ldb + g.K), 0x00020000);
+    const int lr = lane >> 3, chunk16 = ((lane & 7) ^ swz16(lr)) * 16;
+    int off[LD];
+#pragma unroll
+    for (int i = 0; i < LD; ++i) {
+        const bool is_a = i < LA;
+        int r = 8 * (NW * (is_a ? i : i - LA) + wave) + lr;
+        const int last = (is_a ? rows_a : rows_b) - 1;
+        r = r < last ? r : last;
+        off[i] = (int)((uint32_t)r * (uint32_t)(is_a ? g.lda : g.ldb)) + chunk16;
+    }
+    const int nk = (g.K + BK - 1) / BK;
+    const bool ragged = g.K < nk * BK;
+    auto issue = [&](int k, int slot) __attribute__((always_inline)) {
+        uint8_t* st = lds + slot * STAGE;
+        const int at = k * BK;
+        if (ragged && k == nk - 1) {  // bytes past K are fed as zeros: those lanes point past the descriptor's end
+#pragma unroll
+            for (int i = 0; i < LD; ++i) {
+                const bool is_a = i < LA;
+                ring_load(is_a ? da : db, st + ((is_a ? 0 : BM) + 8 * (NW * (is_a ? i : i - LA) + wave)) * BK,
+                          at + chunk16 < g.K ? off[i] + at : (int)0xFFFFFFF0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < LD; ++i) {
+                const bool is_a = i < LA;
+                ring_load(is_a ? da : db, st + ((is_a ? 0 : BM) + 8 * (NW * (is_a ? i : i - LA) + wave)) * BK, off[i], at);
+            }
+        }
+    };
+
+    // ---- fragment reads: half q of a lane's 32 K bytes; MFMA tile t adds 2048 t
+    uint32_t fa_at[2], fb_at[2];
+    {
+        const uint32_t lds0 = (uint32_t)(uintptr_t)(ring_lds_t)lds;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const uint32_t chunk = (uint32_t)((2 * kb + q) ^ swz16(r16)) << 4;
+            fa_at[q] = lds0 + (uint32_t)((wm * WTM + r16) * BK) + chunk;
+            fb_at[q] = lds0 + (uint32_t)((BM + wn * WTN + r16) * BK) + chunk;
+        }
+    }
+
+    ring_v4f acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = (ring_v4f){0, 0, 0, 0};
+
+#pragma unroll
+    for (int s = 0; s < ST - 1; ++s)
+        if (s < nk) issue(s, s);
+    int slot = 0;
+    for (int k = 0; k < nk; ++k) {
+        // this wave's loads of step k have landed (those of up to ST - 2 later steps may be in flight) ...
+        const int ahead = nk - 1 - k;
+        if (ahead >= ST - 2)
+            ring_wait<LD * (ST - 2)>();
+        else if (ST > 3 && ahead == 1)
+            ring_wait<LD>();
+        else
+            ring_wait<0>();
+        // ... every wave's have, and every wave has its fragments of step k - 1, whose slot is filled next
+        asm volatile("s_barrier" ::: "memory");
+        if (k + ST - 1 < nk) issue(k + ST - 1, slot == 0 ? ST - 1 : slot - 1);
+        const uint32_t at = (uint32_t)(slot * STAGE);
+        v4i fa[TM][2], fb[TN][2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) fa[i][q] = *reinterpret_cast<ring_frag_t>((uintptr_t)(fa_at[q] + at + i * 16 * BK));
+#pragma unroll
+            for (int j = 0; j < TN; ++j) fb[j][q] = *reinterpret_cast<ring_frag_t>((uintptr_t)(fb_at[q] + at + j * 16 * BK));
+        }
+        // D' = B . A^T: the first operand is the B fragment (its type code goes to cbsz)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                    __builtin_shufflevector(fb[j][0], fb[j][1], 0, 1, 2, 3, 4, 5, 6, 7),
+                    __builtin_shufflevector(fa[i][0], fa[i][1], 0, 1, 2, 3, 4, 5, 6, 7), acc[i][j], BLGP, CBSZ, 0, 0, 0, 0);
+        slot = slot == ST - 1 ? 0 : slot + 1;
+    }
+
+    // ---- epilogue: acc[i][j][e] of lane l is C[row = 16 i + l % 16][col = 16 j + 4 (l / 16) + e] of the wave tile.
+    // Single scales are inverted with an IEEE division, scale vectors with v_rcp_f32 (exact for the power-of-two scales
+    // of the axiswise recipes, within 1 ulp otherwise).
+    const int row0 = m0 + wm * WTM + r16, col0 = n0 + wn * WTN + 4 * kb;
+    const float isa1 = g.sa && !g.sa_vec ? 1.0f / g.sa[0] : 1.0f, isb1 = g.sb && !g.sb_vec ? 1.0f / g.sb[0] : 1.0f;
+    const bool both_single = !g.sa_vec && !g.sb_vec;
+    float isb[TN][4];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            isb[j][e] = g.sb_vec ? (col0 + 16 * j + e < g.N ? __builtin_amdgcn_rcpf(g.sb[col0 + 16 * j + e]) : 0.0f) : isb1;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int row = row0 + 16 * i;
+        const float isa = g.sa_vec ? (row < g.M ? __builtin_amdgcn_rcpf(g.sa[row]) : 0.0f) : isa1;
+        const float one = isa1 * isb1;
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][j][e] = both_single ? acc[i][j][e] * one : acc[i][j][e] * isa * isb[j][e];
+    }
+    if (g.c_f32) {
+        float* C = reinterpret_cast<float*>(g.C);
+        const bool wide = ((g.ldc | g.N) & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int row = row0 + 16 * i;
+            if (row >= g.M) continue;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int col = col0 + 16 * j;
+                float* c = C + (int64_t)row * g.ldc + col;
+                if (wide) {
+                    if (col < g.N) {
+                        ring_v4f* c4 = reinterpret_cast<ring_v4f*>(c);
+                        *c4 = g.accumulate ? *c4 + acc[i][j] : acc[i][j];
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (col + e < g.N) c[e] = g.accumulate ? c[e] + acc[i][j][e] : acc[i][j][e];
+                }
+            }
+        }
+        return;
+    }
+    uint16_t* C = reinterpret_cast<uint16_t*>(g.C);
+    if (((g.ldc | g.N) & 7) != 0 || (reinterpret_cast<uintptr_t>(C) & 15) != 0) {  // rows that are not whole 16-byte chunks
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int row = row0 + 16 * i;
+            if (row >= g.M) continue;
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int col = col0 + 16 * j + e;
+                    if (col >= g.N) continue;
+                    uint16_t* c = C + (int64_t)row * g.ldc + col;
+                    uint16_t r = f32_to_bf16_bits(acc[i][j][e]);
+                    if (g.accumulate)  // both terms are bf16 values, summed in float32 and rounded once
+                        r = f32_to_bf16_bits(bits_to_f32((uint32_t)*c << 16) + bits_to_f32((uint32_t)r << 16));
+                    *c = r;
+                }
+        }
+        return;
+    }
+    // bf16 rows leave through LDS (the ring is free now): whole row segments of the wave tile, 16 bytes per lane
+    constexpr int PITCH = WTN * 2 + 16;  // (the pad spreads the rows of a store over the banks)
+    static_assert(NW * WTM * PITCH <= ST * STAGE, "output staging");
+    __syncthreads();
+    uint8_t* stg = lds + wave * (WTM * PITCH);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+            *reinterpret_cast<uint2*>(stg + (16 * i + r16) * PITCH + (16 * j + 4 * kb) * 2) =
+                make_uint2(pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3]));
+    constexpr int LPR = WTN / 8, RPI = 64 / LPR;  // lanes per row, rows per store
+#pragma unroll
+    for (int it = 0; it < WTM / RPI; ++it) {
+        const int rw = it * RPI + lane / LPR, c8 = (lane % LPR) * 8;
+        v4i v = *reinterpret_cast<const v4i*>(stg + rw * PITCH + c8 * 2);
+        const int row = m0 + wm * WTM + rw, col = n0 + wn * WTN + c8;
+        if (row < g.M && col < g.N) {
+            v4i* c = reinterpret_cast<v4i*>(C + (int64_t)row * g.ldc + col);
+            if (g.accumulate) v = add_bf16x8(v, *c);
+            *c = v;
+        }
+    }
+}
+
+}  // namespace
+}  // namespace gemm
+}  // namespace mi8

@@ -106,6 +106,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_fp8_skinny_kernel(Gemm
     const bool m_ok = wave < MT && m < g.M;
     const float isa = !m_ok ? 0.0f : g.sa_vec ? __builtin_amdgcn_rcpf(g.sa[m]) : 1.0f / g.sa[0];
     const float isb_scalar = g.sb_vec ? 0.0f : 1.0f / g.sb[0];
+    const bool both_single = !g.sa_vec && !g.sb_vec;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         if (nb > 0) __syncthreads();  // the previous block's sums have been read
@@ -121,11 +122,16 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_fp8_skinny_kernel(Gemm
             const int n = n0 + nb * 16 + kg * 4 + j;
             if (n >= g.N) continue;
             const float isb = g.sb_vec ? __builtin_amdgcn_rcpf(g.sb[n]) : isb_scalar;
-            const float v = sum[j] * isa * isb;
-            if (g.c_f32)
-                reinterpret_cast<float*>(g.C)[(int64_t)m * g.ldc + n] = v;
-            else
-                reinterpret_cast<uint16_t*>(g.C)[(int64_t)m * g.ldc + n] = f32_to_bf16_bits(v);
+            const float v = both_single ? sum[j] * (isa * isb) : sum[j] * isa * isb;
+            if (g.c_f32) {
+                float* c = reinterpret_cast<float*>(g.C) + (int64_t)m * g.ldc + n;
+                *c = g.accumulate ? *c + v : v;
+            } else {
+                uint16_t* c = reinterpret_cast<uint16_t*>(g.C) + (int64_t)m * g.ldc + n;
+                uint16_t h = f32_to_bf16_bits(v);
+                if (g.accumulate) h = f32_to_bf16_bits(bits_to_f32((uint32_t)*c << 16) + bits_to_f32((uint32_t)h << 16));
+                *c = h;
+            }
         }
     }
 }

@@ -5,18 +5,14 @@
 //   grouped_wgrad : out[e]         = A_t[:, seg_e] . B_t[:, seg_e]^T     (grad_weight; ragged K, segments padded
 //                                                                          to multiples of 128 with zero bytes)
 //
-// Each workgroup finds its group by walking the (at most a few hundred) group sizes, builds a per-group view of
-// the operands and runs the general tile routine on it; workgroups beyond the real number of tiles exit.
-#include "mi8_gemm_body.h"
+// Each workgroup finds its group in the device-resident sizes, builds a per-group view of the operands and runs the
+// general tile routine on it; workgroups beyond the real number of tiles exit.
+#include "mi8_gemm_ring.h"
+#include "mi8_groups.h"
 
 namespace mi8 {
 using namespace gemm;
 namespace {
-
-constexpr int GBM = 256, GBN = 256;  // 8 waves of 128 x 64: the best general-shape configuration measured
-constexpr int GWM = 2, GWN = 4;
-constexpr int kGroupedThreads = GWM * GWN * 64;
-constexpr int kGroupedLds = 2 * (GBM + GBN) * BK;
 
 struct GroupedArgs {
     const uint8_t* A;  // [T, lda]
@@ -34,47 +30,30 @@ struct GroupedArgs {
     int accumulate;   // C += the rounded product
 };
 
-template <int CBSZ, int BLGP>
-__global__ __launch_bounds__(kGroupedThreads, 1) void grouped_gemm_kernel(GroupedArgs a)
+template <int BM, int BN, int ST, int CBSZ, int BLGP>
+__global__ __launch_bounds__(kRingThreads, 2) void grouped_gemm_kernel(GroupedArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int mt = (int)blockIdx.x / a.tiles_n, nt = (int)blockIdx.x % a.tiles_n;
-    int64_t row0 = 0;
-    int tiles_before = 0, e = 0, m_e = 0;
-    bool found = false;
-    for (e = 0; e < a.E; ++e) {
-        int64_t m = a.sizes[e];
-        m = m < 0 ? 0 : m;
-        m = (row0 + m > a.T) ? a.T - row0 : m;  // never touch rows past the activation matrix
-        const int t = (int)((m + GBM - 1) / GBM);
-        if (mt < tiles_before + t) {
-            m_e = (int)m;
-            found = true;
-            break;
-        }
-        tiles_before += t;
-        row0 += m;
-    }
-    if (!found) return;
+    const GroupSpan s = locate_group<BM, true>(a.sizes, a.E, a.T, mt);
+    if (s.e >= a.E) return;
     GemmArgs g;
-    g.A = a.A + row0 * a.lda;
-    g.B = a.B + (int64_t)e * a.b_group_stride;
-    g.C = reinterpret_cast<uint8_t*>(a.C) + row0 * a.ldc * (a.c_f32 ? 4 : 2);
+    g.A = a.A + s.rows_before * a.lda;
+    g.B = a.B + (int64_t)s.e * a.b_group_stride;
+    g.C = reinterpret_cast<uint8_t*>(a.C) + s.rows_before * a.ldc * (a.c_f32 ? 4 : 2);
     g.c_f32 = a.c_f32;
     g.lda = a.lda;
     g.ldb = a.ldb;
     g.ldc = a.ldc;
-    g.M = m_e;
+    g.M = (int)s.m;
     g.N = a.N;
     g.K = a.K;
-    g.sa = a.sa + row0;
-    g.sb = a.sb + (int64_t)e * a.sb_group_stride;
+    g.sa = a.sa + s.rows_before;
+    g.sb = a.sb + (int64_t)s.e * a.sb_group_stride;
     g.sa_vec = 1;
     g.sb_vec = 1;
-    g.tiles_m = 0;
-    g.tiles_n = a.tiles_n;
     g.accumulate = a.accumulate;
-    gemm_tile_body<GBM, GBN, GWM, GWN, CBSZ, BLGP>(g, (mt - tiles_before) * GBM, nt * GBN, lds);
+    ring_tile<BM, BN, ST, CBSZ, BLGP>(g, (int)(mt - s.units_before) * BM, nt * BN, lds);
 }
 
 struct GroupedWgradArgs {
@@ -92,8 +71,8 @@ struct GroupedWgradArgs {
     int tiles_n, tiles_k;
 };
 
-template <int CBSZ, int BLGP>
-__global__ __launch_bounds__(kGroupedThreads, 1) void grouped_wgrad_kernel(GroupedWgradArgs a)
+template <int BM, int BN, int ST, int CBSZ, int BLGP>
+__global__ __launch_bounds__(kRingThreads, 2) void grouped_wgrad_kernel(GroupedWgradArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int per_group = a.tiles_n * a.tiles_k;
@@ -101,20 +80,9 @@ __global__ __launch_bounds__(kGroupedThreads, 1) void grouped_wgrad_kernel(Group
     const int rem = (int)blockIdx.x % per_group;
     const int tn = rem / a.tiles_k, tk = rem % a.tiles_k;
     // segment of group e in the padded token axis: starts at 128 * (tiles of the groups before it)
-    int64_t rows_before = 0, tiles_before = 0, m_e = 0;
-    for (int i = 0; i <= e; ++i) {
-        int64_t m = a.sizes[i];
-        m = m < 0 ? 0 : m;
-        m = (rows_before + m > a.T) ? a.T - rows_before : m;
-        if (i == e) {
-            m_e = m;
-            break;
-        }
-        tiles_before += (m + 127) / 128;
-        rows_before += m;
-    }
-    const int64_t seg0 = 128 * tiles_before;
-    int64_t seg = 128 * ((m_e + 127) / 128);
+    const GroupSpan s = locate_group<128, false>(a.sizes, a.E, a.T, e);
+    const int64_t seg0 = 128 * s.units_before;
+    int64_t seg = 128 * ((s.m + 127) / 128);
     if (seg0 + seg > a.ld_t) seg = 0;
     GemmArgs g;
     g.A = a.At + seg0;
@@ -127,38 +95,60 @@ __global__ __launch_bounds__(kGroupedThreads, 1) void grouped_wgrad_kernel(Group
     g.M = a.N;
     g.N = a.Kl;
     g.K = (int)seg;  // 0 for an empty group: the tile routine then writes zeros
-    // an empty group has no scales (nothing was quantised): give the epilogue a finite stand-in
-    static __device__ const float kOne = 1.0f;
-    g.sa = seg ? a.sa + (int64_t)e * a.N : &kOne;
-    g.sb = seg ? a.sb + (int64_t)e * a.Kl : &kOne;
+    // an empty group has no scales (nothing was quantised): the raw sums, zeros, are what is wanted
+    g.sa = seg ? a.sa + (int64_t)e * a.N : nullptr;
+    g.sb = seg ? a.sb + (int64_t)e * a.Kl : nullptr;
     g.sa_vec = seg ? 1 : 0;
     g.sb_vec = seg ? 1 : 0;
-    g.tiles_m = 0;
-    g.tiles_n = a.tiles_k;
     g.accumulate = 0;
-    gemm_tile_body<GBM, GBN, GWM, GWN, CBSZ, BLGP>(g, tn * GBM, tk * GBN, lds);
+    ring_tile<BM, BN, ST, CBSZ, BLGP>(g, tn * BM, tk * BN, lds);
 }
 
-template <int CBSZ, int BLGP>
-int launch_grouped(const GroupedArgs& a, int blocks, hipStream_t st)
+template <int BM, int BN, int ST, int CBSZ, int BLGP>
+int launch_grouped(GroupedArgs& a, hipStream_t st)
 {
-    auto kern = grouped_gemm_kernel<CBSZ, BLGP>;
+    auto kern = grouped_gemm_kernel<BM, BN, ST, CBSZ, BLGP>;
     static std::atomic<uint64_t> configured{0};
-    if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), kGroupedLds, configured, "mi8_grouped_gemm_fp8"))
+    if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), kRingLdsBytes<BM, BN, ST>, configured, "mi8_grouped_gemm_fp8"))
         return rc;
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kGroupedThreads), kGroupedLds, st, a);
+    a.tiles_n = (a.N + BN - 1) / BN;
+    const int64_t blocks = (ceil_div(a.T, BM) + a.E) * a.tiles_n;  // every group adds at most one partial tile
+    MI8_REQUIRE(blocks < ((int64_t)1 << 31), MI8_ERR_UNSUPPORTED, "mi8_grouped_gemm_fp8: grid too large");
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kRingThreads), (kRingLdsBytes<BM, BN, ST>), st, a);
     return launch_status("mi8_grouped_gemm_fp8");
 }
 
+// tile height by the rows a group has on average: what lies below a group's last row is work for nothing
 template <int CBSZ, int BLGP>
-int launch_wgrad(const GroupedWgradArgs& a, int blocks, hipStream_t st)
+int launch_grouped_shape(GroupedArgs& a, hipStream_t st)
 {
-    auto kern = grouped_wgrad_kernel<CBSZ, BLGP>;
+    const int64_t rows = a.T / a.E;
+    if (rows <= 24) return launch_grouped<32, 128, 4, CBSZ, BLGP>(a, st);
+    if (rows <= 128) return launch_grouped<64, 128, 3, CBSZ, BLGP>(a, st);
+    return launch_grouped<128, 128, 2, CBSZ, BLGP>(a, st);
+}
+
+template <int BM, int BN, int ST, int CBSZ, int BLGP>
+int launch_wgrad(GroupedWgradArgs& a, hipStream_t st)
+{
+    auto kern = grouped_wgrad_kernel<BM, BN, ST, CBSZ, BLGP>;
     static std::atomic<uint64_t> configured{0};
-    if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), kGroupedLds, configured, "mi8_grouped_wgrad_fp8"))
+    if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), kRingLdsBytes<BM, BN, ST>, configured, "mi8_grouped_wgrad_fp8"))
         return rc;
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kGroupedThreads), kGroupedLds, st, a);
+    a.tiles_n = (a.N + BM - 1) / BM;
+    a.tiles_k = (a.Kl + BN - 1) / BN;
+    const int64_t blocks = (int64_t)a.E * a.tiles_n * a.tiles_k;
+    MI8_REQUIRE(blocks < ((int64_t)1 << 31), MI8_ERR_UNSUPPORTED, "mi8_grouped_wgrad_fp8: grid too large");
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kRingThreads), (kRingLdsBytes<BM, BN, ST>), st, a);
     return launch_status("mi8_grouped_wgrad_fp8");
+}
+
+// small tiles until the large ones would put two workgroups on every compute unit
+template <int CBSZ, int BLGP>
+int launch_wgrad_shape(GroupedWgradArgs& a, hipStream_t st)
+{
+    if ((int64_t)a.E * ceil_div(a.N, 128) * ceil_div(a.Kl, 128) < 512) return launch_wgrad<64, 64, 4, CBSZ, BLGP>(a, st);
+    return launch_wgrad<128, 128, 2, CBSZ, BLGP>(a, st);
 }
 
 bool fp8_code(int v) { return v == MI8_E4M3 || v == MI8_E5M2; }
@@ -184,13 +174,10 @@ int grouped_gemm_entry(const void* a, int a_dtype, int64_t lda, const void* b, i
     MI8_REQUIRE(aligned16(a) && aligned16(b), MI8_ERR_UNSUPPORTED, "mi8_grouped_gemm_fp8: operands must be 16-byte aligned");
     MI8_REQUIRE(N * ldb < ((int64_t)1 << 32) && T < (1 << 30) && N < (1 << 30) && K < (1 << 30), MI8_ERR_UNSUPPORTED,
                 "mi8_grouped_gemm_fp8: operand too large");
-    const int tiles_n = (int)ceil_div(N, GBN);
-    const int64_t m_tiles = ceil_div(T, GBM) + num_groups;  // every group adds at most one partial tile
-    MI8_REQUIRE(m_tiles * tiles_n < ((int64_t)1 << 31), MI8_ERR_UNSUPPORTED, "mi8_grouped_gemm_fp8: grid too large");
+    MI8_REQUIRE(lda < (1 << 25), MI8_ERR_UNSUPPORTED, "mi8_grouped_gemm_fp8: lda (%lld) of 2^25 or more", (long long)lda);
     GroupedArgs g{(const uint8_t*)a, (const uint8_t*)b, out, out_dtype == MI8_F32 ? 1 : 0, lda, ldb, ldc,
-                  b_group_stride, sb_group_stride, group_sizes, num_groups, T, (int)N, (int)K, sa, sb, tiles_n,
+                  b_group_stride, sb_group_stride, group_sizes, num_groups, T, (int)N, (int)K, sa, sb, 0,
                   accumulate ? 1 : 0};
-    const int blocks = (int)(m_tiles * tiles_n);
     hipStream_t st = (hipStream_t)stream;
     // full-tile shapes with bf16 output run on the persistent direct-to-LDS kernel (which rewrites the overlap of its
     // shifted last tile column when N is not a multiple of 256: not possible when accumulating)
@@ -201,8 +188,8 @@ int grouped_gemm_entry(const void* a, int a_dtype, int64_t lda, const void* b, i
                                    group_sizes, num_groups, T, (int)N, (int)K, sa, sb, sb_group_stride, (uint16_t*)out,
                                    ldc, accumulate, st);
     if (a_dtype == MI8_E4M3)
-        return b_dtype == MI8_E4M3 ? launch_grouped<0, 0>(g, blocks, st) : launch_grouped<0, 1>(g, blocks, st);
-    return b_dtype == MI8_E4M3 ? launch_grouped<1, 0>(g, blocks, st) : launch_grouped<1, 1>(g, blocks, st);
+        return b_dtype == MI8_E4M3 ? launch_grouped_shape<0, 0>(g, st) : launch_grouped_shape<0, 1>(g, st);
+    return b_dtype == MI8_E4M3 ? launch_grouped_shape<1, 0>(g, st) : launch_grouped_shape<1, 1>(g, st);
 }
 }  // namespace
 
@@ -278,16 +265,14 @@ extern "C" int mi8_grouped_wgrad_fp8(const void* a_t, int a_dtype, const void* b
     MI8_REQUIRE(aligned16(a_t) && aligned16(b_t), MI8_ERR_UNSUPPORTED, "mi8_grouped_wgrad_fp8: operands must be 16-byte aligned");
     MI8_REQUIRE(N * ld_t < ((int64_t)1 << 32) && Kl * ld_t < ((int64_t)1 << 32), MI8_ERR_UNSUPPORTED,
                 "mi8_grouped_wgrad_fp8: operand larger than 4 GiB");
-    const int tiles_n = (int)ceil_div(N, GBM), tiles_k = (int)ceil_div(Kl, GBN);
     GroupedWgradArgs g{(const uint8_t*)a_t, (const uint8_t*)b_t, ld_t, group_sizes, num_groups, T, (int)N, (int)Kl,
-                       sa, sb, out, out_dtype == MI8_F32 ? 1 : 0, tiles_n, tiles_k};
-    const int blocks = num_groups * tiles_n * tiles_k;
+                       sa, sb, out, out_dtype == MI8_F32 ? 1 : 0, 0, 0};
     hipStream_t st = (hipStream_t)stream;
     if (out_dtype == MI8_BF16 && N >= 256 && Kl >= 256 && Kl % 8 == 0 && aligned16(out) && aligned16(sb) &&
         ld_t % 128 == 0 && ld_t < (1 << 23))
         return launch_m16_grouped_wgrad((const uint8_t*)a_t, a_dtype, (const uint8_t*)b_t, b_dtype, ld_t, group_sizes,
                                          num_groups, T, (int)N, (int)Kl, sa, sb, (uint16_t*)out, st);
     if (a_dtype == MI8_E4M3)
-        return b_dtype == MI8_E4M3 ? launch_wgrad<0, 0>(g, blocks, st) : launch_wgrad<0, 1>(g, blocks, st);
-    return b_dtype == MI8_E4M3 ? launch_wgrad<1, 0>(g, blocks, st) : launch_wgrad<1, 1>(g, blocks, st);
+        return b_dtype == MI8_E4M3 ? launch_wgrad_shape<0, 0>(g, st) : launch_wgrad_shape<0, 1>(g, st);
+    return b_dtype == MI8_E4M3 ? launch_wgrad_shape<1, 0>(g, st) : launch_wgrad_shape<1, 1>(g, st);
 }

@@ -289,10 +289,11 @@ def gemm_fp8(
         ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         ev0.record()
     L = _C.lib()
-    if accumulate and variant < 0 and splits != 1 and L.mi8_gemm_splitk_suggest(M, N, K) > 1:
-        # few output tiles: the plain call cuts K into slices (another summation order); the sum keeps its bits
-        return out.add_(gemm_fp8(a, sa, b, sb, k=K, out_dtype=out_dtype, splits=splits))
-    if accumulate:
+    if variant >= 0:
+        splits = 1
+    elif splits < 0:
+        splits = L.mi8_gemm_splitk_suggest(M, N, K)
+    if accumulate and splits == 1:
         _C.check(
             L.mi8_gemm_fp8_accumulate(
                 a.data_ptr(), _FP8_CODE[a.dtype], a.stride(0), b.data_ptr(), _FP8_CODE[b.dtype], b.stride(0), M, N, K,
@@ -301,19 +302,11 @@ def gemm_fp8(
             ),
             "mi8_gemm_fp8_accumulate",
         )
-        if sink is not None:
-            ev1.record()
-            sink.append((ev0, ev1, (M, N, K)))
-        return out
-    if variant >= 0:
-        splits = 1
-    elif splits < 0:
-        splits = L.mi8_gemm_splitk_suggest(M, N, K)
-    if splits > 1:
+    elif splits > 1:
         # the planes come from torch's caching allocator: reuse is ordered on the stream like any other tensor
         planes = torch.empty(L.mi8_gemm_splitk_workspace_bytes(M, N, splits), dtype=torch.uint8, device=a.device)
         _C.check(
-            L.mi8_gemm_fp8_splitk(
+            (L.mi8_gemm_fp8_splitk_accumulate if accumulate else L.mi8_gemm_fp8_splitk)(
                 a.data_ptr(), _FP8_CODE[a.dtype], a.stride(0), b.data_ptr(), _FP8_CODE[b.dtype], b.stride(0), M, N, K,
                 sa.data_ptr(), int(sa.numel() != 1),
                 sb.data_ptr(), int(sb.numel() != 1),

@@ -355,3 +355,62 @@ def test_accumulating_gemm_equals_gemm_plus_add(dev, shape, vec, out_dtype):
         assert torch.equal(wide[:, :N], want) and bool((wide[:, N:] == 7.0).all())
     with pytest.raises(ValueError):
         ops.gemm_fp8(aq, sa, bq, sb, out_dtype=out_dtype, accumulate=True)
+
+
+RING = [n for n in ("64x64_ring4", "128x64_ring3", "64x128_ring3", "128x128_ring2", "128x128_ring3")]
+
+
+@pytest.mark.parametrize("name", RING)
+@pytest.mark.parametrize("mnk", [(1, 1, 16), (63, 65, 128), (65, 127, 144), (129, 136, 240), (128, 128, 384), (200, 72, 656)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_ring_tiles_at_their_edges(dev, name, mnk):
+    """The ring tile shapes one row / column / K step around their tile sizes: K shorter than a step, a ragged last step
+    whose padding bytes are poison, output rows that are not whole 16-byte chunks, C += product in both output types.
+    Integer operands and power-of-two scales: exact."""
+    M, N, K = mnk
+    v = ops.gemm_variants().index(name)
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.full((M, K + 48), 3.0)
+    b = torch.full((N, K + 16), float("nan"))
+    a[:, :K] = torch.randint(-2, 3, (M, K), generator=g).float()
+    b[:, :K] = torch.randint(-2, 3, (N, K), generator=g).float()
+    ref = a[:, :K] @ b[:, :K].t()
+    aq, bq = a.to(E5M2).to(dev), b.to(E4M3).to(dev)
+    sa, sb = 2.0 ** torch.randint(-3, 4, (M,), generator=g).float(), 2.0 ** torch.randint(-3, 4, (N,), generator=g).float()
+    for sa_t, sb_t in ((torch.tensor([4.0]), torch.tensor([0.5])), (sa, sb), (sa, torch.tensor([2.0]))):
+        want = ref / (sa_t[:, None] if sa_t.numel() > 1 else sa_t) / (sb_t[None, :] if sb_t.numel() > 1 else sb_t)
+        for dt in (torch.bfloat16, torch.float32):
+            for pad in (8, 3):
+                out = torch.full((M, N + pad), 7.0, device=dev, dtype=dt)
+                ops.gemm_fp8(aq, sa_t.to(dev), bq, sb_t.to(dev), k=K, out_dtype=dt, out=out[:, :N], variant=v)
+                assert torch.equal(out[:, :N].float().cpu(), want.to(dt).float()), (dt, pad)
+                assert bool((out[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("mnk", [(300, 264, 384), (1000, 520, 1152)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
+def test_ring_tiles_have_the_bits_of_the_persistent_kernel(dev, mnk, vec):
+    """One MFMA shape, one order of K, one scale arithmetic: which kernel a shape is dispatched to does not show."""
+    M, N, K = mnk
+    a, b = seeded((M, K), 91).to(E5M2).to(dev), seeded((N, K), 92).to(E4M3).to(dev)
+    g = torch.Generator().manual_seed(93)
+    sa = (torch.rand(M if vec else 1, generator=g) + 0.5).to(dev)
+    sb = (torch.rand(N if vec else 1, generator=g) + 0.5).to(dev)
+    names = ops.gemm_variants()
+    want = ops.gemm_fp8(a, sa, b, sb, variant=names.index("256x256_dma_w4x128_m16x128"))
+    for name in RING:
+        got = ops.gemm_fp8(a, sa, b, sb, variant=names.index(name))
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), name
+
+
+@pytest.mark.parametrize("mnk", [(100, 200, 1040), (257, 130, 4096)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_split_k_accumulates_as_an_add(dev, mnk, dt):
+    """C += product summed in slices of K: the bits of the sliced product and an elementwise add."""
+    M, N, K = mnk
+    a, b = seeded((M, K), 5).to(E4M3).to(dev), seeded((N, K), 6).to(E4M3).to(dev)
+    s = torch.full((1,), 1.7, device=dev)
+    first = seeded((M, N), 7).to(dt).to(dev)
+    want = first + ops.gemm_fp8(a, s, b, s, out_dtype=dt, splits=5)
+    got = ops.gemm_fp8(a, s, b, s, out_dtype=dt, splits=5, out=first.clone(), accumulate=True)
+    assert torch.equal(got, want)
