@@ -147,16 +147,6 @@ int best_ring(int64_t M, int64_t N, int64_t steps, int64_t slices, float* cost)
     return best;
 }
 
-// the same for the persistent kernel: rounds of 256 tiles, a full round running at the clock the power limit leaves
-float persistent_cost(int64_t M, int64_t N, int64_t steps)
-{
-    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
-    const int64_t full = tiles / 256, rest = tiles % 256;
-    float t = 3.0f + full * (steps * 1.35f + 5.0f);
-    if (rest) t += steps * (1.0f + 0.35f * (rest > 128 ? (rest - 128) / 128.0f : 0.0f)) + 5.0f;
-    return t;
-}
-
 // Slices for a problem, 1 = do not split: a summation order of its own, so it depends on the product alone.  Splitting
 // pays where the whole of K in one workgroup is the time (few tiles, a long K) and costs a second launch that reads the
 // planes; up to 192 tiles of 64 x 64 it is at worst even.  At least four K steps a slice.
@@ -167,6 +157,10 @@ int suggested_splits(int64_t M, int64_t N, int64_t K)
     if (M <= 16 || tiles256 > 96 || steps < 8) return 1;  // (up to 16 rows: the few-rows kernel reads B once)
     float best;
     best_ring(M, N, steps, 1, &best);
+    if (M >= 256 && N >= 256 && K % BK == 0 && N % 8 == 0) {
+        const float t = m16_cost(M, N, K);
+        best = t < best ? t : best;
+    }
     if (tiles64 <= 192) best = 1e30f;
     int64_t splits = 1;
     for (int64_t s = 2; s <= 32 && s <= steps / 4; ++s) {
@@ -270,11 +264,11 @@ int gemm_fp8_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b
                sa, sb, sa_is_vector ? 1 : 0, sb_is_vector ? 1 : 0, 0, 0, accumulate ? 1 : 0};
     hipStream_t st = (hipStream_t)stream;
     // (the persistent kernel shifts its last tile row / column back over the previous one when M or N is not a
-    // multiple of 256 and rewrites the overlap with identical values: not possible when accumulating)
+    // whole number of half tiles (128 x 256) and rewrites the overlap with identical values: not possible when accumulating)
     // (its output stores address a tile's 256 rows with 32-bit byte offsets: ldc < 2^22)
     const bool dma_ok = (K % 128 == 0) && M >= 256 && N >= 256 && N % 8 == 0 && ldc % 8 == 0 && ldc < (1 << 22) && aligned16(out) &&
                         out_dtype == MI8_BF16 && (!sb_is_vector || aligned16(sb)) &&
-                        (sa_is_vector != 0) == (sb_is_vector != 0) && (!accumulate || (M % 256 == 0 && N % 256 == 0));
+                        (sa_is_vector != 0) == (sb_is_vector != 0) && (!accumulate || (M % 128 == 0 && N % 256 == 0));
     // A few rows of A go to the kernel that streams B once; everything else to whichever of the ring tile shapes and the
     // persistent kernel the measured costs above say is fastest for this number of tiles and K steps (all of them give
     // the same bits).
@@ -285,7 +279,7 @@ int gemm_fp8_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b
             const int64_t steps = ceil_div(K, BK);
             float cost;
             variant = best_ring(M, N, steps, 1, &cost);
-            if (dma_ok && persistent_cost(M, N, steps) < cost) variant = kM16;
+            if (dma_ok && m16_cost(M, N, K) < cost) variant = kM16;
         }
     }
     if (variant == kSkinny) return launch_skinny(g, a_dtype, b_dtype, st);

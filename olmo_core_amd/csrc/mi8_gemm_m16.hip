@@ -40,6 +40,7 @@ constexpr int STAGE = (BM + BN) * BK;        // 64 KB
 constexpr int OUT_STAGING = 4 * 4096;        // 4 KB of output staging per wave
 constexpr int SCALE_SLOT = 2 * 256 * 4;      // one tile's 256 row scales and 256 column scales
 constexpr int SCALE_SLOTS = 4;
+static_assert(3 * (BM / 2 + BN) * BK <= 2 * STAGE + OUT_STAGING, "the three stages of a half tile end before the scale slots");
 // Tile timeline (only in the diagnostics library, which compiles this file with -DMI8_TILE_TIMELINE): wave 0 of every
 // workgroup records the shader clock at fixed points of each of its tiles - K loop start, after three K steps, epilogue
 // start, every epilogue pass, last store issued, tile end - in 1 KB of LDS of its own and copies them out when the
@@ -89,10 +90,20 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t out_rows(void* p, int bytes)
     return __builtin_amdgcn_make_buffer_rsrc(p, 0, bytes, 0x00020000);
 }
 
-template <typename Problem, int CBSZ_A, int BLGP_B>
-__global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
+// s_waitcnt: at most n vector memory operations of this wave outstanding, the other counters untouched
+constexpr int vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
+
+// Workgroup `block` of `blocks` that walk the problem's whole tiles (kHalf: one half tile each, 128 x 256: the waves take
+// 64 x 128).
+template <typename Problem, int CBSZ_A, int BLGP_B, bool kHalf>
+__device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, const int blocks)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    constexpr int WTM = kHalf ? WT / 2 : WT;          // rows of a wave's part of the tile
+    constexpr int kRowsA = kHalf ? BM / 2 : BM;       // A rows of a stage
+    constexpr int kStage = (kRowsA + BN) * BK;
+    constexpr int kLoadsA = kHalf ? kLoads / 2 : kLoads;
+    constexpr int kPasses = kHalf ? 2 : 4;            // epilogue: blocks of 32 rows of the wave's part
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -129,8 +140,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const uint32_t chunk = (uint32_t)((2 * kb + q) ^ swz16(r16));
-            ra[q] = lds0 + (uint32_t)((wm * WT + r16) * BK) + (chunk << 4);
-            rb[q] = lds0 + (uint32_t)(BM * BK + (wn * WT + r16) * BK) + (chunk << 4);
+            ra[q] = lds0 + (uint32_t)((wm * WTM + r16) * BK) + (chunk << 4);
+            rb[q] = lds0 + (uint32_t)(kRowsA * BK + (wn * WT + r16) * BK) + (chunk << 4);
         }
     }
     auto flip_read_stage = [&](int to_stage) __attribute__((always_inline)) {
@@ -161,15 +172,17 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
         const int64_t ld = k < 2 ? pb.lda : pb.ldb;
         dv[k] = (uint32_t)((int64_t)lr * ld) + ((uint32_t)((lane & 7) ^ swz16(8 * (k & 1) + lr)) << 4);
     }
-    // x in 0..15: the first eight -> A rows 8 x, the rest -> B rows 8 (x - 8)
+    // x in 0..15: the first eight -> A rows 8 x, the rest -> B rows 8 (x - 8).  A half tile has 128 rows of A: wave w fetches
+    // rows [32 w, +32) with the first four.
     auto dma_one = [&](const uint8_t* a_origin, const uint8_t* b_origin, int stage, int x) __attribute__((always_inline)) {
         const bool is_a = x < kLoads;
         const int p = x % kLoads;
-        uint32_t rows = (uint32_t)((int64_t)(wave * 64 + 8 * p) * (is_a ? pb.lda : pb.ldb));
+        const int row = wave * 8 * (is_a ? kLoadsA : kLoads) + 8 * p;
+        uint32_t rows = (uint32_t)((int64_t)row * (is_a ? pb.lda : pb.ldb));
         asm volatile("" : "+s"(rows));  // opaque: the sum stays one add at the load instead of sixteen resident registers
         const uint32_t o = dv[(is_a ? 0 : 2) + (p & 1)] + rows;
         const uint8_t* src = (is_a ? a_origin : b_origin) + o;
-        uint8_t* dst = lds + stage * STAGE + (is_a ? 0 : BM * BK) + (wave * 64 + 8 * (x % kLoads)) * BK;
+        uint8_t* dst = lds + stage * kStage + (is_a ? 0 : kRowsA * BK) + row * BK;
         __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)dst, 16, 0, 0);
     };
 
@@ -202,7 +215,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
     auto scale_dma = [&](const TileDesc& d) __attribute__((always_inline)) {
         if constexpr (Problem::kVecScales) {
             uint8_t* slot = lds + 2 * STAGE + OUT_STAGING + (ld_seq & kSlotMask) * kSlotBytes + wave * 256;
-            __builtin_amdgcn_global_load_lds((gptr_t)(d.sa + wave * 64 + lane), (lptr_t)slot, 4, 0, 0);
+            // (a half tile has 128 rows, and the scales may end with them: its upper half repeats the lower one)
+            const int row = (wave * 64 + lane) & (kHalf ? 127 : 255);
+            __builtin_amdgcn_global_load_lds((gptr_t)(d.sa + row), (lptr_t)slot, 4, 0, 0);
             __builtin_amdgcn_global_load_lds((gptr_t)(d.sb + wave * 64 + lane), (lptr_t)(slot + 1024), 4, 0, 0);
             if constexpr (Problem::kTwoSegments) {
                 __builtin_amdgcn_global_load_lds((gptr_t)(d.sa2 + wave * 64 + lane), (lptr_t)(slot + 2048), 4, 0, 0);
@@ -216,13 +231,17 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
     // of equal cost every XCD takes a contiguous range of the tile order (neighbouring tiles share operand panels),
     // its workgroups striding through it; tiles of unequal cost are strided over the whole grid instead
     const typename Problem::Cache cache = pb.prepare();
-    const int total = pb.total_tiles(cache);
+    int total;
+    if constexpr (kHalf)
+        total = pb.half_tiles();
+    else
+        total = pb.total_tiles(cache);
     int first_tile, tile_stride, my_tiles;
     if constexpr (Problem::kXcdRanges) {
         const int per_xcd = (total + 7) / 8;
-        const int xcd = (int)blockIdx.x & 7;
-        const int slot = (int)blockIdx.x >> 3;
-        const int slots = ((int)gridDim.x + 7 - xcd) >> 3;
+        const int xcd = block & 7;
+        const int slot = block >> 3;
+        const int slots = (blocks + 7 - xcd) >> 3;
         const int first = xcd * per_xcd;
         int last = first + per_xcd;
         last = last < total ? last : total;
@@ -230,8 +249,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
         tile_stride = slots;
         my_tiles = (first_tile < last) ? (last - first_tile + slots - 1) / slots : 0;
     } else {
-        first_tile = (int)blockIdx.x;
-        tile_stride = (int)gridDim.x;
+        first_tile = block;
+        tile_stride = blocks;
         my_tiles = (first_tile < total) ? (total - first_tile + tile_stride - 1) / tile_stride : 0;
     }
     if (my_tiles == 0) {
@@ -239,7 +258,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
             if (lane == 0) pb.h_slots[(int)blockIdx.x * 4 + wave] = 0;
         return;
     }
-    auto my_tile = [&](int idx) __attribute__((always_inline)) { return pb.tile(first_tile + idx * tile_stride, cache); };
+    auto my_tile = [&](int idx) __attribute__((always_inline)) {
+        if constexpr (kHalf)
+            return pb.half_tile(first_tile + idx * tile_stride);
+        else
+            return pb.tile(first_tile + idx * tile_stride, cache);
+    };
 
     // Fused SwiGLU problem: LDS B rows [64 w, 64 w + 64), the rows this wave fetches, are rows 64 (w / 2) .. of B1
     // (even w) or of B3 (odd w); folded into the wave's B cursor once per tile.
@@ -292,9 +316,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
         }
         if (ld_kt >= ld_nk) next_load_tile();
     };
-    next_load_tile();
+    if constexpr (!kHalf) next_load_tile();
 
-    v4f acc[NT][NT];
+    v4f acc[2 * kPasses][NT];
     // D' = B . A^T : the first MFMA operand is the B fragment (its type code goes to cbsz).  `fresh`: the tile's
     // first touch of this accumulator; the MFMA then takes the constant 0 as its addend, so the accumulators
     // never have to be cleared between tiles.
@@ -340,7 +364,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
     };
 
     // ---- prologue: stages of steps 0 and 1, fragments of step 0 ----------------------------------------
-    if (ld_a != nullptr) {  // uniform
+    if (!kHalf && ld_a != nullptr) {  // uniform
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
 #pragma unroll
@@ -364,9 +388,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
             read_b(fb[0][t], t, 1);
         }
     };
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's direct loads have landed
-    __syncthreads();
-    read_step_head();
+    if constexpr (!kHalf) {
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's direct loads have landed
+        __syncthreads();
+        read_step_head();
+    }
 
     int step = 0;
     for (int cp_tile = 0; cp_tile < my_tiles; ++cp_tile) {
@@ -412,6 +438,23 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
         // issued, the last tile's at the very end of the step - and the first MFMA of the next step then waited out the
         // LDS latency (the wait at a loop head covers every read in flight).  Now all reads of a step are issued in the
         // first three quarters of phase B.
+        // The wait between the phases: all loads but the eight the step's first phase has issued have landed, so the other
+        // stage (step + 1) is complete.  (The compiler does not track direct-to-LDS loads across a barrier.)  A tile's
+        // first step follows the previous tile's epilogue, whose stores - 32, 40 with row-segment codes, 48 or 52 of
+        // the fused SwiGLU problem - are younger than the loads waited for here (one in-order
+        // counter): they may stay outstanding as well.
+        auto wait_step = [&](bool fresh) __attribute__((always_inline)) {
+            if (!fresh) {
+                __builtin_amdgcn_s_waitcnt(vmcnt(8));
+            } else if constexpr (Problem::kSwiglu) {
+                if (pb.x_codes)  // (uniform)
+                    __builtin_amdgcn_s_waitcnt(vmcnt(8 + 13 * kPasses));
+                else
+                    __builtin_amdgcn_s_waitcnt(vmcnt(8 + 12 * kPasses));
+            } else {
+                __builtin_amdgcn_s_waitcnt(vmcnt(8 + (Problem::kOutCodes ? 10 : 8) * kPasses));
+            }
+        };
         auto k_step = [&](bool fresh, auto set_tag) __attribute__((always_inline)) {
             constexpr int S = decltype(set_tag)::value;
             const int cur = step & 1;
@@ -427,22 +470,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
                 if (x >= 8 && x % 3 == 2) dma_one(ld_a, ld_b, cur, kLoads + (x - 8) / 3);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            // All but this phase's eight loads have landed: the other stage (step + 1) is complete.  (The
-            // compiler does not track direct-to-LDS loads across a barrier.)
-            // A tile's first step follows the previous tile's epilogue, whose 32 stores (40 with row-segment codes, 48
-            // or 52 of the fused SwiGLU problem) are younger than the loads waited for here (one in-order counter):
-            // they may stay outstanding as well.
-            if (fresh) {
-                if constexpr (Problem::kSwiglu) {
-                    if (pb.x_codes)  // (uniform)
-                        __builtin_amdgcn_s_waitcnt(0xCF7C);  // vmcnt(60): 8 loads, 48 + 4 stores
-                    else
-                        __builtin_amdgcn_s_waitcnt(0xCF78);  // vmcnt(56)
-                } else {
-                    __builtin_amdgcn_s_waitcnt(Problem::kOutCodes ? 0xCF70 : 0x8F78);  // vmcnt(48) / vmcnt(40)
-                }
-            } else
-                __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8)
+            wait_step(fresh);
             asm volatile("s_barrier" ::: "memory");
             flip_read_stage(cur ^ 1);
             // phase B: the next step's fragments - all B tiles (into the other set), then A tiles 0-3 - are read
@@ -459,7 +487,87 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
             advance_load_cursor();
             ++step;
         };
-        if (td.nk > 0) {
+        if constexpr (kHalf) {
+            // A half tile: half the rows of A, hence a third less of a stage, half the accumulators and room for a second set of
+            // A fragments too.  So there are three stages, every fragment of a step is read during the step before, and a
+            // stage is free for step s + 3 as soon as step s starts: one barrier a step, its loads two steps ahead of
+            // their wait, its 24 fragment reads (1140 cycles of LDS for the four waves, against 1024 of MFMAs) spread over
+            // all of it.  Without its loads and reads the loop takes 0.53 us a step, with either 0.60, with both 0.65;
+            // operands that come from HBM make it 0.85.  One tile per workgroup: nothing is prefetched across tiles, and the
+            // output staging takes the place of the stages.
+            const uint8_t* a_src = td.a;
+            const uint8_t* b_src = td.b + b_wave_shift;
+            constexpr int kStepLoads = kLoadsA + kLoads;
+            auto fetch = [&](int x, int slot) __attribute__((always_inline)) {  // x-th load of the step a_src / b_src point at
+                dma_one(a_src, b_src, slot, x < kLoadsA ? x : kLoads + x - kLoadsA);
+            };
+            scale_dma(td);
+#pragma unroll
+            for (int s = 0; s < 3; ++s)
+                if (s < td.nk) {
+#pragma unroll
+                    for (int x = 0; x < kStepLoads; ++x) fetch(x, s);
+                    a_src += BK;
+                    b_src += BK;
+                }
+            if (td.nk > 2)
+                __builtin_amdgcn_s_waitcnt(vmcnt(2 * kStepLoads));
+            else if (td.nk == 2)
+                __builtin_amdgcn_s_waitcnt(vmcnt(kStepLoads));
+            else
+                __builtin_amdgcn_s_waitcnt(vmcnt(0));
+            asm volatile("s_barrier" ::: "memory");
+            read_step_head();
+#pragma unroll
+            for (int i = 0; i < 2 * kPasses; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[i][j] = (v4f){0, 0, 0, 0};
+            int slot = 0;
+            auto half_step = [&](int kt, auto set_tag) __attribute__((always_inline)) {
+                constexpr int S = decltype(set_tag)::value;
+                auto& fa = S ? fa_hi : fa_lo;
+                auto& fa_next = S ? fa_lo : fa_hi;
+                // this wave's loads of step kt + 1 have landed and its fragments of step kt arrived; then every wave's have
+                if (kt + 2 < td.nk)
+                    __builtin_amdgcn_s_waitcnt(vmcnt(kStepLoads) & 0xF0FF);
+                else
+                    __builtin_amdgcn_s_waitcnt(vmcnt(0) & 0xF0FF);
+                asm volatile("s_barrier" ::: "memory");
+                const int next = slot == 2 ? -2 * kStage : kStage;
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    ra[q] += (uint32_t)next;
+                    rb[q] += (uint32_t)next;
+                }
+                auto body = [&](auto with_loads) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int x = 0; x < 32; ++x) {
+                        const int j = x >> 2, i = x & 3;
+                        mma(fa[i], fb[S][j], acc[i][j], false, i, j);
+                        if (x < 8) read_a(fa_next[x >> 1], x >> 1, x & 1);
+                        if (x >= 8 && x < 24) read_b(fb[S ^ 1][(x - 8) >> 1], (x - 8) >> 1, x & 1);
+                        if (decltype(with_loads)::value && x % 2 == 1 && x / 2 < kStepLoads) fetch(x / 2, slot);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                };
+                if (kt + 3 < td.nk) {
+                    body(std::true_type{});
+                    a_src += BK;
+                    b_src += BK;
+                } else {
+                    body(std::false_type{});
+                }
+                slot = slot == 2 ? 0 : slot + 1;
+            };
+            int kt = 0;
+            for (; kt + 1 < td.nk; kt += 2) {
+                half_step(kt, std::integral_constant<int, 0>{});
+                half_step(kt + 1, std::integral_constant<int, 1>{});
+            }
+            if (kt < td.nk) half_step(kt, std::integral_constant<int, 0>{});
+            __builtin_amdgcn_s_waitcnt(vmcnt(0) & 0xF0FF);
+            asm volatile("s_barrier" ::: "memory");  // nobody reads the stages any more
+        } else if (td.nk > 0) {
             // a tile starts from set 0 (read_step_head) and alternates; what the last step prefetched for the next
             // tile is read again after the epilogue, into set 0
             const std::integral_constant<int, 0> set0;
@@ -486,7 +594,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
             }
         } else {  // nothing is accumulated (empty group): the tile is all zeros
 #pragma unroll
-            for (int i = 0; i < NT; ++i)
+            for (int i = 0; i < 2 * kPasses; ++i)
 #pragma unroll
                 for (int j = 0; j < NT; ++j) acc[i][j] = (v4f){0, 0, 0, 0};
         }
@@ -500,7 +608,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
         // (the copies below are opaque to the compiler's hazard handling: the last MFMA has retired after these)
         MI8_TL(2);
         asm volatile("s_nop 15\n\ts_nop 15");
-        uint8_t* stg = lds + 2 * STAGE + wave * 4096;
+        uint8_t* stg = lds + (kHalf ? 0 : 2 * STAGE) + wave * 4096;
         const uint32_t stg_lds = (uint32_t)(uintptr_t)(lptr_t)stg;
         const bool zero_tile = td.nk == 0;  // nothing accumulated; the scales may be unset
         const uint8_t* sc_slot = lds + 2 * STAGE + OUT_STAGING + (cp_seq & kSlotMask) * kSlotBytes;
@@ -519,7 +627,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
         // an elementwise bf16 add would (float32 sum of the two bf16 values, one rounding).
         v4i held[4];
         auto load_held = [&](int jq, int ih) __attribute__((always_inline)) {
-            const int rt = wm * WT + ih * 32;
+            const int rt = wm * WTM + ih * 32;
             if constexpr (Problem::kMaskRows) {
                 const int voff = (rt + (lane >> 3) - td.row_lo) * ldc_bytes + (wn * WT + jq * 64 + (lane & 7) * 8) * 2;
 #pragma unroll
@@ -557,17 +665,17 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
             c23 = dpp_pk_umax16_over8(c23);
             const uint32_t w = (lane & 2) ? c23 : c01;
             const uint16_t code = (uint16_t)((lane & 1) ? (w >> 16) : (w & 0xFFFFu));
-            if ((lane & 7) < 4) codes[(int64_t)col_block * rows_total + td.m0 + wm * WT + ih * 32 + code_lane] = code;
+            if ((lane & 7) < 4) codes[(int64_t)col_block * rows_total + td.m0 + wm * WTM + ih * 32 + code_lane] = code;
         };
-        auto record_codes = [&](int p) __attribute__((always_inline)) {  // p = 4 * jq + ih: the pass whose rows are staged
+        auto record_codes = [&](int jq, int ih) __attribute__((always_inline)) {  // of the pass whose rows are staged
             if constexpr (Problem::kOutCodes) {
                 uint32_t c01, c23;
                 lane_codes(c01, c23);
-                store_codes(pb.codes, pb.g.M, td.n0 / 64 + wn * 2 + (p >> 2), p & 3, c01, c23);
+                store_codes(pb.codes, pb.g.M, td.n0 / 64 + wn * 2 + jq, ih, c01, c23);
             }
         };
         auto store_staged = [&](int jq, int ih) __attribute__((always_inline)) {
-            const int rt = wm * WT + ih * 32;  // first tile row of the pass
+            const int rt = wm * WTM + ih * 32;  // first tile row of the pass
             if constexpr (Problem::kMaskRows) {
                 // Only rows [row_lo, row_hi) of the tile belong to this tile's group.  The stores go through a
                 // buffer descriptor that spans exactly those rows: a lane whose row lies outside gets an offset
@@ -594,7 +702,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
             const float* aux = reinterpret_cast<const float*>(lds + 2 * STAGE + OUT_STAGING);
             uint32_t hmax = 0;
             auto store_out = [&](int which, int ih) __attribute__((always_inline)) {
-                const int rt = wm * WT + ih * 32;
+                const int rt = wm * WTM + ih * 32;
                 const int64_t shift = which == 0 ? 0 : (which == 1 ? pb.x3_offset : pb.h_offset);
                 const __amdgpu_buffer_rsrc_t c_tile = out_rows(td.c + shift, 256 * ldc_bytes);
 #pragma unroll
@@ -648,7 +756,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
                 }
             };
 #pragma unroll
-            for (int ih = 0; ih < 4; ++ih) {
+            for (int ih = 0; ih < kPasses; ++ih) {
                 uint2 o1[2][4], o3[2][4], oh[2][4];
                 scaled(o1, ih, 0, aux[0]);
                 stage(o1, ih == 0 ? -1 : 2, ih - 1);
@@ -674,7 +782,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
                 stage(oh, 1, ih);
             }
             __builtin_amdgcn_s_waitcnt(0xc07f);
-            store_out(2, 3);
+            store_out(2, kPasses - 1);
             {   // fold this tile's maximum into the lane's slot (an LDS atomic the compiler need not order against
                 // the direct loads in flight)
                 const uint32_t maddr = (uint32_t)(uintptr_t)(lptr_t)(lds + 2 * STAGE + OUT_STAGING) + (64 + tid) * 4;
@@ -699,8 +807,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
                 }
             }
 #pragma unroll
-            for (int ih = 0; ih < 4; ++ih) {
-                const int rt = wm * WT + ih * 32;  // first tile row of this pass
+            for (int ih = 0; ih < kPasses; ++ih) {
+                const int rt = wm * WTM + ih * 32;  // first tile row of this pass
                 uint2 o[2][4];
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
@@ -740,12 +848,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
                     // the previous pass's rows have arrived in registers (so its staging area is free again)
                     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
                     if constexpr (Problem::kAccumulate) add_held();
-                    record_codes(4 * jq + ih - 1);
+                    record_codes(ih == 0 ? jq - 1 : jq, ih == 0 ? kPasses - 1 : ih - 1);
                 }
                 // (this pass's old C values are requested before the previous pass's stores are issued: the wait for
                 // them, one pass later, then leaves those stores outstanding)
                 if constexpr (Problem::kAccumulate) load_held(jq, ih);
-                if (jq + ih > 0) store_staged(ih == 0 ? jq - 1 : jq, ih == 0 ? 3 : ih - 1);
+                if (jq + ih > 0) store_staged(ih == 0 ? jq - 1 : jq, ih == 0 ? kPasses - 1 : ih - 1);
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -772,8 +880,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
         }
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
         if constexpr (Problem::kAccumulate) add_held();
-        record_codes(7);
-        store_staged(1, 3);
+        record_codes(1, kPasses - 1);
+        store_staged(1, kPasses - 1);
         MI8_TL(11);
         };
         if constexpr (Problem::kTwoSegments) {
@@ -791,7 +899,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
         // again here makes those 96 registers free during the epilogue, which otherwise spills (and every
         // reload from scratch waits on the in-order vector memory counter, i.e. on the stores above).
         __builtin_amdgcn_sched_barrier(0);  // (or the scheduler moves these reads up into the epilogue)
-        read_step_head();
+        if constexpr (!kHalf) read_step_head();
         MI8_TL(12);
         MI8_TL_NEXT_TILE();
     }
@@ -812,6 +920,22 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
         uint32_t m = reinterpret_cast<const uint32_t*>(lds + 2 * STAGE + OUT_STAGING)[64 + tid];
         m = wave_umax(m);
         if (lane == 0) pb.h_slots[(int)blockIdx.x * 4 + wave] = m;
+    }
+}
+
+// Workgroups [0, whole_blocks) walk the whole tiles, the others have a half tile each; the dispatcher starts those as compute
+// units fall free.  (Two separate bodies: as branches of one tile loop they share 256 accumulators across control flow and the
+// kernel spills.)
+template <typename Problem, int CBSZ_A, int BLGP_B>
+__global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
+{
+    if constexpr (Problem::kHalves) {
+        if ((int)blockIdx.x < pb.rows.whole_blocks)
+            m16_tiles<Problem, CBSZ_A, BLGP_B, false>(pb, (int)blockIdx.x, pb.rows.whole_blocks);
+        else
+            m16_tiles<Problem, CBSZ_A, BLGP_B, true>(pb, (int)blockIdx.x - pb.rows.whole_blocks, (int)gridDim.x - pb.rows.whole_blocks);
+    } else {
+        m16_tiles<Problem, CBSZ_A, BLGP_B, false>(pb, (int)blockIdx.x, (int)gridDim.x);
     }
 }
 
@@ -837,7 +961,8 @@ int launch(const Problem& pb, int max_tiles, bool persistent, hipStream_t st)
     static std::atomic<uint64_t> configured{0};
     if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), LDS_BYTES, configured, "mi8 16x16x128 GEMM"))
         return rc;
-    const int blocks = persistent ? persistent_blocks(max_tiles) : max_tiles;
+    int blocks = persistent ? persistent_blocks(max_tiles) : max_tiles;
+    if constexpr (Problem::kHalves) blocks = pb.rows.blocks();
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), LDS_BYTES, st, pb);
     return launch_status("mi8 16x16x128 GEMM");
 }
@@ -854,38 +979,93 @@ int launch_typed(const Problem& pb, int max_tiles, bool persistent, int a_dtype,
 
 }  // namespace
 
+namespace {
+
+// Which tiles of a dense problem are halves (tiles_n columns of tiles, nk K steps), and g.tiles_m = pairs of half rows.
+// Splitting tiles of a partial last round pays when its halves fit into one round: 2048 x 11008 x 4096 is 344 tiles, two
+// rounds of 256 workgroups for 1.34 rounds of work; as 256 whole and 176 half tiles it takes 79 us instead of 84.
+// 4096 x 2048 x 8192, 128 tiles, is 256 half tiles: 59 us instead of 76.  (A step of a half tile takes 0.65 us with its
+// operands in the memory-side cache, 0.85 us from HBM; a whole tile's 1.0 us, 1.35 us when all compute units have one.)
+HalfRows plan_halves(GemmArgs& g, int most_halves = 1 << 30)
+{
+    const int half_rows = (g.M + 127) / 128;
+    g.tiles_m = half_rows / 2;
+    const int pairs = g.tiles_m * g.tiles_n, odd = (half_rows & 1) * g.tiles_n;
+    const int cus = num_compute_units();
+    const float steps = (float)(g.K / BK), whole = steps * 1.05f + 5.0f, half = steps * 0.78f + 3.5f;
+    // the longest share of a workgroup: half tiles are dealt first to those with fewer whole ones
+    auto longest = [&](int split) {
+        const int n_full = pairs - split, n_half = 2 * split + odd;
+        const int q = n_full / cus, r = n_full % cus, h = n_half / cus, hr = n_half % cus;
+        const float less = q * whole + (h + (hr > 0 ? 1 : 0)) * half;
+        const float more = r > 0 ? (q + 1) * whole + (h + (hr > cus - r ? 1 : 0)) * half : 0.0f;
+        return less > more ? less : more;
+    };
+    if (odd > most_halves) {
+        g.tiles_m = (g.M + BM - 1) / BM;
+        return HalfRows{g.tiles_m * g.tiles_n, 0, 0, persistent_blocks(g.tiles_m * g.tiles_n), 0};
+    }
+    int split = 0;
+    float best = longest(0);
+    const int candidates[2] = {pairs % cus, pairs < cus ? pairs : pairs % cus + cus};
+    for (int c : candidates)
+        if (c > 0 && c <= pairs && 2 * c + odd <= most_halves && longest(c) < 0.97f * best) {
+            split = c;
+            best = longest(c);
+        }
+    return HalfRows{pairs - split, 2 * split + odd, 2 * split, persistent_blocks(pairs - split), (2 * split + odd + 7) / 8 * 8};
+}
+
+}  // namespace
+
+float m16_cost(int64_t M, int64_t N, int64_t K)
+{
+    // (the plan's own arithmetic, with the fixed cost of a launch; a full machine runs whole tiles at 1.35 us a step)
+    GemmArgs g{};
+    g.M = (int)M;
+    g.N = (int)N;
+    g.K = (int)K;
+    g.tiles_n = (int)((N + BN - 1) / BN);
+    const HalfRows h = plan_halves(g);
+    const float steps = (float)(K / BK);
+    const int cus = num_compute_units();
+    const int q = h.n_full / cus, r = h.n_full % cus, halves = (h.n_half + cus - 1) / cus;
+    float t = 3.0f + q * (steps * 1.35f + 5.0f);
+    if (r) t += steps * (1.0f + 0.35f * (r > cus / 2 ? (float)(2 * r - cus) / cus : 0.0f)) + 5.0f;
+    if (halves && !(r && h.n_half <= cus - r)) t += halves * (steps * 0.78f + 3.5f);
+    return t;
+}
+
 int launch_m16(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st)
 {
-    g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
-    const int tiles = g.tiles_m * g.tiles_n;
+    const HalfRows rows = plan_halves(g);
     if (g.sa_vec) {
-        if (g.accumulate) return launch_typed(DenseProblem<true, true>{g, g.lda, g.ldb, g.ldc}, tiles, true, a_dtype, b_dtype, st);
-        return launch_typed(DenseProblem<true>{g, g.lda, g.ldb, g.ldc}, tiles, true, a_dtype, b_dtype, st);
+        if (g.accumulate) return launch_typed(DenseProblem<true, true>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);
+        return launch_typed(DenseProblem<true>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);
     }
-    if (g.accumulate) return launch_typed(DenseProblem<false, true>{g, g.lda, g.ldb, g.ldc}, tiles, true, a_dtype, b_dtype, st);
-    return launch_typed(DenseProblem<false>{g, g.lda, g.ldb, g.ldc}, tiles, true, a_dtype, b_dtype, st);
+    if (g.accumulate) return launch_typed(DenseProblem<false, true>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);
+    return launch_typed(DenseProblem<false>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);
 }
 
 int launch_m16_codes(GemmArgs& g, uint16_t* codes, int a_dtype, int b_dtype, hipStream_t st)
 {
-    g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
-    DenseProblem<false, false, true> pb{g, g.lda, g.ldb, g.ldc};
+    const HalfRows rows = plan_halves(g);
+    DenseProblem<false, false, true> pb{g, g.lda, g.ldb, g.ldc, rows};
     pb.codes = codes;
-    return launch_typed(pb, g.tiles_m * g.tiles_n, true, a_dtype, b_dtype, st);
+    return launch_typed(pb, 0, true, a_dtype, b_dtype, st);
 }
 
 int launch_m16_swiglu(GemmArgs& g, const uint8_t* b3, const float* sb3, uint16_t* x3, uint16_t* h, uint32_t* h_slots,
                       int* n_slots, uint16_t* x_codes, int a_dtype, int b_dtype, hipStream_t st)
 {
-    g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + 127) / 128;
-    SwigluProblem pb{g, g.lda, g.ldb, g.ldc, (int64_t)(b3 - g.B), (int64_t)(x3 - reinterpret_cast<uint16_t*>(g.C)),
+    const HalfRows rows = plan_halves(g, 256);  // (4 partial maxima per workgroup, MI8_AMAX_SLOTS in all)
+    SwigluProblem pb{g, g.lda, g.ldb, g.ldc, rows, (int64_t)(b3 - g.B), (int64_t)(x3 - reinterpret_cast<uint16_t*>(g.C)),
                      (int64_t)(h - reinterpret_cast<uint16_t*>(g.C)), sb3, h_slots, x_codes};
-    const int tiles = g.tiles_m * g.tiles_n;
-    *n_slots = 4 * persistent_blocks(tiles);  // one partial maximum per wave of the grid launch() forms from `tiles`
-    return launch_typed(pb, tiles, true, a_dtype, b_dtype, st);
+    *n_slots = 4 * rows.blocks();  // one partial maximum per wave of the grid
+    return launch_typed(pb, 0, true, a_dtype, b_dtype, st);
 }
 
 int launch_m16_grouped(const uint8_t* a, int a_dtype, int64_t lda, const uint8_t* b, int b_dtype, int64_t ldb,

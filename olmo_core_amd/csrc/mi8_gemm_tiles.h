@@ -32,6 +32,33 @@ struct TileDesc {
 
 struct NoCache {};
 
+// Rows of a kHalves problem.  The M rows are ceil(M / 128) half rows of tiles: pairs of them make the 256-row tiles, an odd
+// one at the end is a row of half tiles (128 x 256).  The last tiles of the order may be split into their two halves, so
+// that a partial last round of whole tiles becomes a round of half tiles on twice as many compute units.  Half tiles
+// are numbered by themselves: the halves of the split pairs, then the odd half row.  Every tile is complete: the last one
+// of either kind is shifted back over its predecessor (M >= 256), recomputes the overlap with the same K order and
+// rewrites identical values.
+struct HalfRows {
+    int n_full;       // whole tiles
+    int n_half;       // half tiles
+    int n_split;      // how many of these are halves of split tiles (the rest: the odd half row)
+    int whole_blocks;  // workgroups that walk the whole tiles
+    int half_blocks;   // workgroups with a half tile each
+    __host__ __device__ int blocks() const { return whole_blocks + half_blocks; }
+    __device__ __forceinline__ void half(const GemmArgs& g, int i, int& m0, int& tn) const
+    {
+        int tm, row;
+        if (i < n_split) {
+            tile_coords(g, n_full + (i >> 1), tm, tn);
+            row = 2 * tm + (i & 1);
+        } else {
+            tn = i - n_split;
+            row = 2 * g.tiles_m;
+        }
+        m0 = (row * 128 + 128 <= g.M) ? row * 128 : g.M - 128;
+    }
+};
+
 // Dense problem: C[M, N] = A[M, K] . B[N, K]^T.  The last tile row / column is shifted back so that every tile
 // is full (M, N >= 256): the overlap is recomputed with the same K order and rewritten with identical values.
 // CODES: the epilogue also records, per row segment (64 consecutive columns of a row) of C, the largest magnitude it
@@ -41,7 +68,9 @@ template <bool VEC, bool ACC = false, bool CODES = false>
 struct DenseProblem {
     GemmArgs g;
     int64_t lda, ldb, ldc;
+    HalfRows rows;
     uint16_t* codes = nullptr;  // (CODES)
+    static constexpr bool kHalves = true;
     static constexpr bool kVecScales = VEC;  // both scales are vectors (per row / per column) or both single
     static constexpr bool kAccumulate = ACC;  // C += the rounded product
     static constexpr bool kOutCodes = CODES;
@@ -52,15 +81,25 @@ struct DenseProblem {
     static constexpr bool kMaskRows = false, kXcdRanges = true;
     using Cache = NoCache;
     __device__ __forceinline__ Cache prepare() const { return Cache{}; }
-    __device__ __forceinline__ int total_tiles(const Cache&) const { return g.tiles_m * g.tiles_n; }
     // (single-scale problems only) the two scales, the same for every tile
     __device__ __forceinline__ float single_sa() const { return g.sa[0]; }
     __device__ __forceinline__ float single_sb() const { return g.sb[0]; }
+    __device__ __forceinline__ int total_tiles(const Cache&) const { return rows.n_full; }
+    __device__ __forceinline__ int half_tiles() const { return rows.n_half; }
     __device__ __forceinline__ TileDesc tile(int t, const Cache&) const
     {
         int tm, tn;
         tile_coords(g, t, tm, tn);
-        const int m0 = (tm * BM + BM <= g.M) ? tm * BM : g.M - BM;
+        return at((tm * BM + BM <= g.M) ? tm * BM : g.M - BM, tn, BM);
+    }
+    __device__ __forceinline__ TileDesc half_tile(int i) const
+    {
+        int m0, tn;
+        rows.half(g, i, m0, tn);
+        return at(m0, tn, BM / 2);
+    }
+    __device__ __forceinline__ TileDesc at(int m0, int tn, int height) const
+    {
         const int n0 = (tn * BN + BN <= g.N) ? tn * BN : g.N - BN;
         TileDesc d;
         d.a = g.A + (int64_t)m0 * g.lda;
@@ -70,7 +109,7 @@ struct DenseProblem {
         d.sb = g.sb + (VEC ? n0 : 0);
         d.c = reinterpret_cast<uint16_t*>(g.C) + (int64_t)m0 * g.ldc + n0;
         d.row_lo = 0;
-        d.row_hi = BM;
+        d.row_hi = height;
         d.m0 = m0;
         d.n0 = n0;
         return d;
@@ -85,6 +124,7 @@ struct DenseProblem {
 struct SwigluProblem {
     GemmArgs g;             // A, B = B1, C = x1; N = H; tiles_n counts 128-column tiles; sa, sb = scale of A, of B1
     int64_t lda, ldb, ldc;
+    HalfRows rows;
     int64_t b3_offset;      // bytes from B1 to B3
     int64_t x3_offset;      // elements from x1 to x3 and to h (same pitch ldc)
     int64_t h_offset;
@@ -92,17 +132,27 @@ struct SwigluProblem {
     uint32_t* h_slots;      // [4 * workgroups] partial maxima of |h| (float32 bit patterns)
     uint16_t* x_codes;      // null, or [H / 64][M] codes of the larger of x1 and x3 per row segment (H % 64 == 0)
     static constexpr bool kVecScales = false, kAccumulate = false, kSwiglu = true, kOutCodes = false;
-    static constexpr bool kMaskRows = false, kXcdRanges = true, kMfmaScale = false, kTwoSegments = false;
+    static constexpr bool kMaskRows = false, kXcdRanges = true, kMfmaScale = false, kTwoSegments = false, kHalves = true;
     using Cache = NoCache;
     __device__ __forceinline__ Cache prepare() const { return Cache{}; }
-    __device__ __forceinline__ int total_tiles(const Cache&) const { return g.tiles_m * g.tiles_n; }
     __device__ __forceinline__ float single_sa() const { return g.sa[0]; }
     __device__ __forceinline__ float single_sb() const { return g.sb[0]; }
+    __device__ __forceinline__ int total_tiles(const Cache&) const { return rows.n_full; }
+    __device__ __forceinline__ int half_tiles() const { return rows.n_half; }
     __device__ __forceinline__ TileDesc tile(int t, const Cache&) const
     {
         int tm, tn;
         tile_coords(g, t, tm, tn);
-        const int m0 = (tm * BM + BM <= g.M) ? tm * BM : g.M - BM;
+        return at((tm * BM + BM <= g.M) ? tm * BM : g.M - BM, tn, BM);
+    }
+    __device__ __forceinline__ TileDesc half_tile(int i) const
+    {
+        int m0, tn;
+        rows.half(g, i, m0, tn);
+        return at(m0, tn, BM / 2);
+    }
+    __device__ __forceinline__ TileDesc at(int m0, int tn, int height) const
+    {
         const int n0 = (tn * 128 + 128 <= g.N) ? tn * 128 : g.N - 128;
         TileDesc d;
         d.a = g.A + (int64_t)m0 * g.lda;
@@ -112,7 +162,7 @@ struct SwigluProblem {
         d.sb = g.sb;
         d.c = reinterpret_cast<uint16_t*>(g.C) + (int64_t)m0 * g.ldc + n0;
         d.row_lo = 0;
-        d.row_hi = BM;
+        d.row_hi = height;
         d.m0 = m0;
         d.n0 = n0;
         return d;
@@ -189,7 +239,7 @@ struct GroupedProblem {
     int N, K, tiles_n;
     const float* sa;
     const float* sb;
-    static constexpr bool kVecScales = true, kMaskRows = true, kXcdRanges = true;
+    static constexpr bool kVecScales = true, kMaskRows = true, kXcdRanges = true, kHalves = false;
     using Cache = GroupCache;
     __device__ __forceinline__ Cache prepare() const { return build_group_cache<BM>(sizes, E, T); }
     __device__ __forceinline__ int total_tiles(const Cache& c) const
@@ -229,7 +279,7 @@ struct GroupedProblem {
 // the column scales a group stride; K1, K2 are multiples of 256 (an even number of steps each).
 struct GroupedDualProblem {
     static constexpr bool kAccumulate = false, kSwiglu = false, kOutCodes = false, kMfmaScale = true, kTwoSegments = true;
-    static constexpr bool kVecScales = true, kMaskRows = true, kXcdRanges = true;
+    static constexpr bool kVecScales = true, kMaskRows = true, kXcdRanges = true, kHalves = false;
     GroupedProblem<false> first;  // A1, B1, C, pitches, sizes, N, K = K1, sa1, sb1
     int64_t lda, ldb, ldc;        // (copies of first's, under the names the kernel reads)
     const uint8_t* A2;
@@ -282,7 +332,7 @@ struct GroupedWgradProblem {
     int N, Kl, tiles_n, tiles_k;
     const float* sa;  // [E, N]
     const float* sb;  // [E, Kl]
-    static constexpr bool kVecScales = true, kMaskRows = false, kXcdRanges = false;
+    static constexpr bool kVecScales = true, kMaskRows = false, kXcdRanges = false, kHalves = false;
     static constexpr bool kAccumulate = false, kSwiglu = false, kOutCodes = false, kMfmaScale = false, kTwoSegments = false;
     using Cache = WgradCache;
     __device__ __forceinline__ Cache prepare() const

@@ -414,3 +414,49 @@ def test_split_k_accumulates_as_an_add(dev, mnk, dt):
     want = first + ops.gemm_fp8(a, s, b, s, out_dtype=dt, splits=5)
     got = ops.gemm_fp8(a, s, b, s, out_dtype=dt, splits=5, out=first.clone(), accumulate=True)
     assert torch.equal(got, want)
+
+
+# half rows of tiles (128 x 256): every tile split, a partial last round split, an odd half row at the end (alone, and
+# shifted back over its predecessor), whole tiles only
+HALF_SHAPES = [(4096, 2048, 256), (2048, 4352, 384), (2560, 2816, 128), (384, 512, 640), (777, 1032, 256), (1300, 6400, 384)]
+
+
+@pytest.mark.parametrize("mnk", HALF_SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
+def test_half_tiles_of_the_persistent_kernel(dev, mnk, vec):
+    """The persistent kernel's plan of whole and half tiles against the ring tiles (same bits), with C += product where the
+    tiles do not overlap and, for single scales, the row-segment codes recorded by its epilogue."""
+    M, N, K = mnk
+    a, b = seeded((M, K), 91).to(E5M2).to(dev), seeded((N, K), 92).to(E4M3).to(dev)
+    g = torch.Generator().manual_seed(93)
+    sa = (torch.rand(M if vec else 1, generator=g) + 0.5).to(dev)
+    sb = (torch.rand(N if vec else 1, generator=g) + 0.5).to(dev)
+    names = ops.gemm_variants()
+    ring = names.index("128x128_ring2")
+    want = ops.gemm_fp8(a, sa, b, sb, variant=ring)
+    got = ops.gemm_fp8(a, sa, b, sb, variant=names.index("256x256_dma_w4x128_m16x128"))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    first = seeded((M, N), 94).to(dev)
+    res = ops.gemm_fp8(a, sa, b, sb, out=first.clone(), accumulate=True, splits=1)
+    assert torch.equal(res, first + want)
+    if not vec and ops.gemm_codes_supported(M, N, K):
+        out, codes = ops.gemm_fp8_codes(a, sa, b, sb)
+        assert torch.equal(out, want) and torch.equal(codes, ops.rowseg_max_codes(want))
+
+
+@pytest.mark.parametrize("mhk", [(4096, 1024, 256), (777, 1416, 384), (2048, 2176, 256)], ids=lambda s: "x".join(map(str, s)))
+def test_half_tiles_of_the_fused_swiglu_launch(dev, mhk):
+    M, H, K = mhk
+    xq, _, sx = ops.cast_tensorwise(seeded((M, K), 61).to(dev), E4M3)
+    w1q, _, s1 = ops.cast_tensorwise(seeded((H, K), 62, std=0.05).to(dev), E4M3)
+    w3q, _, s3 = ops.cast_tensorwise(seeded((H, K), 63, std=0.02).to(dev), E4M3)
+    ring = ops.gemm_variants().index("128x128_ring2")
+    want_codes = H % 64 == 0
+    x1, x3, h, (slots, n), *codes = ops.gemm_fp8_swiglu(xq, sx, w1q, s1, w3q, s3, want_codes=want_codes)
+    assert torch.equal(x1, ops.gemm_fp8(xq, sx, w1q, s1, variant=ring))
+    assert torch.equal(x3, ops.gemm_fp8(xq, sx, w3q, s3, variant=ring))
+    rh, (rslots, rn) = ops.swiglu_fwd(x1, x3)
+    assert torch.equal(h.view(torch.int16), rh.view(torch.int16))
+    assert int(slots[:n].max()) == int(rslots[:rn].max())
+    if want_codes:
+        assert torch.equal(codes[0], ops.rowseg_max_codes(x1, x3))
