@@ -128,8 +128,10 @@ float ring_cost(const RingShape& r, int64_t M, int64_t N, int64_t steps, int64_t
 {
     const int64_t tiles = ((M + r.bm - 1) / r.bm) * ((N + r.bn - 1) / r.bn) * slices;
     const int64_t per_cu = (tiles + 255) / 256;
-    if (per_cu == 1 || r.step2 == 0.0f) return kLaunchUs + per_cu * (steps * r.step1 + r.tile);
-    return kLaunchUs + 0.5f * per_cu * (steps * r.step2 + r.tile);
+    const float work = per_cu == 1 || r.step2 == 0.0f ? per_cu * (steps * r.step1 + r.tile) : 0.5f * per_cu * (steps * r.step2 + r.tile);
+    // A short K leaves the stores: these kernels write 3.2 MB a us (27648 x 5120 x 256: 91-100 us, the persistent kernel 66-76).
+    const float stores = (float)(M * N) * (slices > 1 ? 4.0f * slices : 2.0f) / 3.2e6f;
+    return kLaunchUs + (work > stores ? work : stores);
 }
 
 int best_ring(int64_t M, int64_t N, int64_t steps, int64_t slices, float* cost)
