@@ -108,8 +108,11 @@ __global__ __launch_bounds__(kThreads) void swiglu_max_sum_kernel(const uint16_t
 // leaves its two maxima as partials (a thousand atomics on one word would take longer than the scan).  Otherwise:
 // the thresholds are the maxima of those partials, and the remaining segments whose sums exceed them are computed;
 // what they find is merged with the thresholds by atomics (few: only a wave that can raise a value asks).
-// A wave lists the flagged ones among its 512 segments in LDS, and its eight groups of eight lanes compute them,
-// eight segments at a time.
+// A wave lists the flagged ones among its 512 segments in LDS, and its eight groups of eight lanes compute them, 32
+// segments at a time: the time is the chain of load latencies, so every lane has four segments' loads in flight, and
+// segments that what has been found meanwhile (by any wave) rules out are passed over.  Where the thresholds from the
+// seeds leave a large share of the segments (4096 x 8192, x1 of unit variance) the second launch took 74 us with eight
+// at a time and fixed thresholds.
 template <bool SEED>
 __global__ __launch_bounds__(kThreads) void swiglu_sparse_amax_kernel(const uint16_t* __restrict__ x1,
                                                                       const uint16_t* __restrict__ x3,
@@ -119,7 +122,7 @@ __global__ __launch_bounds__(kThreads) void swiglu_sparse_amax_kernel(const uint
                                                                       const uint16_t* __restrict__ xc,
                                                                       uint32_t* __restrict__ state)
 {
-    __shared__ uint16_t picked[kThreads / 64][kSegsPerWave];
+    __shared__ uint32_t picked[kThreads / 64][kSegsPerWave];  // sum << 9 | index in the wave's range
     __shared__ int32_t n_picked[kThreads / 64];
     __shared__ uint32_t smem[3][kThreads / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -163,24 +166,50 @@ __global__ __launch_bounds__(kThreads) void swiglu_sparse_amax_kernel(const uint
         const bool in_range = wave_first + lane * kSegsPerLane + k < nseg;
         const bool seed = s[k] >= 0x7F80u || s[k] + kSeedSlack >= top;
         const bool need = in_range && (SEED ? seed : (!seed && swiglu_segment_needed(s[k], t1, t3)));
-        if (need) picked[wave][atomicAdd(&n_picked[wave], 1)] = (uint16_t)(lane * kSegsPerLane + k);
+        if (need) picked[wave][atomicAdd(&n_picked[wave], 1)] = s[k] << 9 | (uint32_t)(lane * kSegsPerLane + k);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int count = n_picked[wave];
+    constexpr int kInFlight = 4;
     uint32_t m1 = 0, m3 = 0;
-    for (int k = grp; k < count; k += 8) {
-        const int64_t seg = wave_first + picked[wave][k];
-        const int64_t cb = seg / rows, r = seg % rows;
-        const int64_t c = cb * kSegCols + sub * 8;
-        if (c < cols) {
+    for (int base = 0; base < count; base += 8 * kInFlight) {
+        uint4 a[kInFlight], b[kInFlight], g[kInFlight];
+#pragma unroll
+        for (int u = 0; u < kInFlight; ++u) {
+            a[u] = b[u] = g[u] = make_uint4(0, 0, 0, 0);  // (a segment passed over computes to zero)
+            const int k = base + 8 * u + grp;
+            if (k >= count) continue;
+            const uint32_t pick = picked[wave][k];
+            if (!SEED && !swiglu_segment_needed(pick >> 9, t1, t3)) continue;
+            const int64_t seg = wave_first + (pick & 511u);
+            const int64_t cb = seg / rows, r = seg % rows;
+            const int64_t c = cb * kSegCols + sub * 8;
+            if (c >= cols) continue;
             const int64_t off = r * cols + c;
+            a[u] = *reinterpret_cast<const uint4*>(x1 + off);
+            b[u] = *reinterpret_cast<const uint4*>(x3 + off);
+            g[u] = *reinterpret_cast<const uint4*>(gh + off);
+        }
+#pragma unroll
+        for (int u = 0; u < kInFlight; ++u) {
             uint4 p1, p3;
-            swiglu_bwd8(*reinterpret_cast<const uint4*>(x1 + off), *reinterpret_cast<const uint4*>(x3 + off),
-                        *reinterpret_cast<const uint4*>(gh + off), p1, p3);
+            swiglu_bwd8(a[u], b[u], g[u], p1, p3);
             m1 = umax32(m1, absmax_packed8(p1));
             m3 = umax32(m3, absmax_packed8(p3));
+        }
+        if (!SEED && base + 8 * kInFlight < count) {
+            // a wave with more to do publishes what it found and takes over what others did: thresholds only rise to
+            // values that some element reached
+            m1 = wave_umax(m1);
+            m3 = wave_umax(m3);
+            if (lane == 0) {
+                if (m1 > t1) atomicMax(&state[0], m1);
+                if (m3 > t3) atomicMax(&state[1], m3);
+            }
+            t1 = umax32(t1, umax32(m1, __hip_atomic_load(&state[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
+            t3 = umax32(t3, umax32(m3, __hip_atomic_load(&state[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
         }
     }
     m1 = wave_umax(m1);
@@ -196,8 +225,8 @@ __global__ __launch_bounds__(kThreads) void swiglu_sparse_amax_kernel(const uint
             seed3[blockIdx.x] = umax32(umax32(smem[2][0], smem[2][1]), umax32(smem[2][2], smem[2][3]));
         }
     } else if (lane == 0) {
-        if (m1 > t1 && m1 > __hip_atomic_load(&state[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&state[0], m1);
-        if (m3 > t3 && m3 > __hip_atomic_load(&state[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&state[1], m3);
+        if (m1 >= t1 && m1 > __hip_atomic_load(&state[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&state[0], m1);
+        if (m3 >= t3 && m3 > __hip_atomic_load(&state[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&state[1], m3);
     }
 }
 

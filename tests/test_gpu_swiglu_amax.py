@@ -221,3 +221,19 @@ def test_mlp_backward_same_bits_with_and_without_codes(dev):
             feed_forward.SWIGLU_AMAX_FROM_CODES = True
     for name, u, v in zip(("y", "gx", "gw1", "gw2", "gw3"), *outs):
         assert torch.equal(u, v), f"{name}: results differ between the two amax routes"
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 64), (40, 13 * 64), (513, 128), (2048, 1024)])
+def test_many_segments_above_the_seed_thresholds(dev, rows, cols):
+    """Segment maxima that never meet in one element: bounds far above the amax, so that most segments are computed."""
+    g = torch.Generator().manual_seed(rows)
+    x1, x3 = (torch.randn(rows, cols, generator=g).bfloat16().to(dev) for _ in range(2))
+    gh = (torch.randn(rows, cols, generator=g) * 1e-3).bfloat16().to(dev)
+    x1[:, ::64] *= 16
+    gh[:, ::64] *= 2.0 ** -6
+    gh[:, 1::64] *= 16
+    x1[:, 1::64] *= 2.0 ** -6
+    x3[:, 1::64] *= 2.0 ** -6
+    _, _, s1, s3 = ops.swiglu_bwd(x1, x3, gh)
+    state = ops.swiglu_bwd_amax_from_codes(x1, x3, gh, ops.rowseg_max_codes(gh), ops.rowseg_max_codes(x1, x3))
+    assert int(state[0]) == int(s1[0][: s1[1]].max()) and int(state[1]) == int(s3[0][: s3[1]].max())
