@@ -32,6 +32,14 @@ from .native_config import CastConfig, Float8LinearConfig, ScalingGranularity, S
 __all__ = ["Float8Linear", "convert_to_float8_training", "float8_linear_function", "float8_projections"]
 
 
+def needs_autograd(*tensors: torch.Tensor) -> bool:
+    """Whether a call on these tensors has to go through an autograd function: some gradient is wanted, or
+    forward-mode differentiation is on (the function then refuses, where plain kernels would drop the tangent)."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return True
+    return torch.autograd.forward_ad._current_level >= 0
+
+
 def _is_tensorwise(c: CastConfig) -> bool:
     return c.scaling_type is ScalingType.DYNAMIC and c.scaling_granularity is ScalingGranularity.TENSORWISE
 

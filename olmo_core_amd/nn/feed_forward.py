@@ -17,7 +17,7 @@ import torch
 import torch.nn as nn
 
 from ..float8 import ops
-from ..float8.linear import Float8Linear, _is_tensorwise, _shared_tensorwise
+from ..float8.linear import Float8Linear, _shared_tensorwise, needs_autograd
 
 __all__ = ["FeedForward", "swiglu"]
 
@@ -259,10 +259,15 @@ class FeedForward(nn.Module):
                 return y.reshape(*x.shape[:-1], self.w2.weight.shape[0])
         elif xa.is_cuda and act_dtype == torch.bfloat16 and _fusable_modules(self):
             x2 = xa.reshape(-1, xa.shape[-1])
-            y = _fused_mlp(x2, self.w1.weight, self.w2.weight, self.w3.weight, self.w1.config,
-                           self.w1.precomputed_weight_scale(), self.w2.precomputed_weight_scale(),
-                           self.w3.precomputed_weight_scale(), self.w1.weight_operands(), self.w2.weight_operands(),
-                           self.w3.weight_operands())
+            weights = (self.w1.weight, self.w2.weight, self.w3.weight)
+            scales = tuple(m.precomputed_weight_scale() for m in (self.w1, self.w2, self.w3))
+            operands = tuple(m.weight_operands() for m in (self.w1, self.w2, self.w3))
+            if needs_autograd(x2, *weights):
+                y = _fused_mlp(x2, *weights, self.w1.config, *scales, *operands)
+            else:
+                # nothing to differentiate: no transposed float8 copies, nothing kept for a backward (an autograd
+                # function reports its inputs' requires_grad also where gradients are off)
+                y = _mlp_forward(x2, *weights, self.w1.config, (False,) * 4, scales, operands)[0]
             return y.reshape(*x.shape[:-1], self.w2.weight.shape[0])
         x1, x3 = self.w1(x), self.w3(x)
         if x1.is_cuda and x1.dtype == torch.bfloat16 and not compiling:
