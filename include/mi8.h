@@ -303,6 +303,23 @@ int mi8_grouped_wgrad_fp8(const void* a_t, int a_dtype, const void* b_t, int b_d
                           const int64_t* group_sizes, int32_t num_groups, int64_t T, int64_t N, int64_t Kl,
                           const float* sa, const float* sb, void* out, int out_dtype, void* stream);
 
+/* A generation step of a SwiGLU block (tensorwise e4m3, evaluation): h = silu(x1) * x3 in bf16 [M, H], x1 = x B1^T,
+ * x3 = x B3^T, with the partial maxima of |h| (slots_h: uint32 [MI8_AMAX_SLOTS], *n_slots_used of them written), in one
+ * launch; x1 and x3 are not written.  1 <= M <= 64, H % 8 == 0 and H <= 16 * MI8_AMAX_SLOTS, K % 16 == 0, pitches multiples
+ * of 16, pointers 16-byte aligned.
+ *   x_is_fp8 != 0: x is e4m3 [M, lda] with its scale sx; otherwise bf16, contiguous (lda == K), at most 16 rows and 16384
+ *   elements: every workgroup then takes the amax and quantises (flags: MI8_FLAG_POW2_SCALE) what it reads. */
+int mi8_few_rows_swiglu(const void* x, int x_is_fp8, int64_t lda, const float* sx, const void* b1, const void* b3,
+                        int64_t ldb, int64_t M, int64_t H, int64_t K, const float* sb1, const float* sb3, uint32_t flags,
+                        void* h, uint32_t* slots_h, int32_t* n_slots_used, void* stream);
+
+/* out[M, ldc] (bf16) = q(x) B^T scaled, x bf16 [M, lda], M <= 16, quantised to e4m3 by the launch with the scale of the
+ * partial maxima `slots` (mi8_scale_from_partials): the bits of mi8_cast_tensorwise followed by mi8_gemm_fp8.
+ * N % 8 == 0, K % 16 == 0, lda % 8 == 0, ldb % 16 == 0, ldc % 4 == 0, pointers 16-byte aligned. */
+int mi8_few_rows_cast_gemm(const void* x, int64_t lda, const uint32_t* slots, int32_t n_slots, const void* b, int64_t ldb,
+                           int64_t M, int64_t N, int64_t K, const float* sb, uint32_t flags, void* out, int64_t ldc,
+                           void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * SwiGLU pointwise kernels between the projections of the feed-forward block
  * (reference: src/olmo_core/nn/feed_forward.py:171  w2(silu(w1 x) * w3 x)).

@@ -18,6 +18,7 @@
 // traffic would exceed the read of B, so a workgroup then takes 32 rows of B per pass over A.  Rows of A past M and rows of B past N
 // are clamped to the last valid row and their results dropped; K bytes past K (K % 16 == 0) are fed as zeros.
 #include "mi8_gemm.h"
+#include "mi8_swiglu.h"
 
 namespace mi8 {
 namespace gemm {
@@ -148,6 +149,196 @@ int launch_skinny_typed(const GemmArgs& g, int a_dtype, int b_dtype, hipStream_t
     return launch_status("mi8_gemm_fp8");
 }
 
+// ---- the same for a generation step of a SwiGLU block: activations quantised by the GEMM that reads them ------------
+//
+// A step on one token is a chain of launches that each wait for the one before: cast, two projections, SwiGLU, cast,
+// projection.  The arithmetic on the activations is so small that every workgroup can repeat it: kind_x says how the
+// kernel gets its float8 rows of A,
+//   kFp8      they are in memory with their scale,
+//   kSlots    A is bf16 and partial maxima of |A| are in memory (left by the launch that produced A): every workgroup
+//             folds them into the scale and converts its fragments on the way into the MFMAs,
+//   kAmax     A is bf16 and small: every workgroup takes the amax itself as well.
+// DUAL: 16 rows of B and the same 16 rows of a second matrix B3 per workgroup, x1 = A B^T, x3 = A B3^T; the epilogue
+// rounds both to bf16 and stores only h = silu(x1) * x3, with a partial maximum of |h| per workgroup.
+// Bytes, scales and sums are those of the separate launches.  One token, 4096 -> 11008 -> 4096: two launches instead of six.
+enum FewRowsInput { kFp8, kSlots, kAmax };
+
+struct FewRowsArgs {
+    GemmArgs g;  // kSlots, kAmax: A is bf16, lda counts its elements, sa is unused
+    const uint8_t* B3;
+    const float* sb3;
+    const uint32_t* slots_in;  // kSlots
+    int n_slots;
+    bool pow2;
+    uint32_t* slots_out;  // DUAL: one per workgroup
+};
+
+constexpr int kFewThreads = kSkinnyWaves * 64;
+constexpr int kAmaxVecs = 4;  // 8-element groups of A per lane where every workgroup takes the amax
+
+// 16 quantised K bytes of one row (zeros past the end of K) from 16 bf16 values
+__device__ __forceinline__ v4i quantise16(const uint4 (&v)[2], float s, bool ok)
+{
+    v4i r{0, 0, 0, 0};
+    if (!ok) return r;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        r[2 * h] = (int)quant4<MI8_E4M3, false>(bits_to_f32(v[h].x << 16), bits_to_f32(v[h].x & 0xFFFF0000u),
+                                                bits_to_f32(v[h].y << 16), bits_to_f32(v[h].y & 0xFFFF0000u), s, s, s, s);
+        r[2 * h + 1] = (int)quant4<MI8_E4M3, false>(bits_to_f32(v[h].z << 16), bits_to_f32(v[h].z & 0xFFFF0000u),
+                                                    bits_to_f32(v[h].w << 16), bits_to_f32(v[h].w & 0xFFFF0000u), s, s, s, s);
+    }
+    return r;
+}
+
+template <int MT, int U, int KIND, bool DUAL>
+__global__ __launch_bounds__(kFewThreads) void few_rows_kernel(FewRowsArgs a)
+{
+    constexpr int NB = DUAL ? 2 : 1;
+    __shared__ v4f red[kSkinnyWaves][MT][64];
+    __shared__ uint32_t smem[kSkinnyWaves];
+    const GemmArgs& g = a.g;
+
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r16 = lane & 15, kg = lane >> 4;
+    const int n0 = (int)blockIdx.x * 16;
+    const int n_row = n0 + r16 < g.N ? n0 + r16 : g.N - 1;
+
+    float scale;
+    if constexpr (KIND == kFp8) {
+        scale = g.sa[0];
+    } else {
+        uint32_t m = 0;
+        if constexpr (KIND == kSlots) {
+            for (int i = threadIdx.x; i < a.n_slots; i += kFewThreads) m = umax32(m, a.slots_in[i]);
+        } else {
+            const uint4* x = reinterpret_cast<const uint4*>(g.A);  // contiguous, at most kFewThreads * kAmaxVecs groups
+            const int groups = g.M * (g.K / 8);
+            uint4 v[kAmaxVecs];
+#pragma unroll
+            for (int i = 0; i < kAmaxVecs; ++i) {
+                const int k = (int)threadIdx.x + kFewThreads * i;
+                v[i] = k < groups ? x[k] : make_uint4(0, 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < kAmaxVecs; ++i) m = umax32(m, (max_code8(v[i].x, v[i].y, v[i].z, v[i].w) & 0xFFFFu) << 16);
+        }
+        m = wave_umax(m);
+        if (lane == 0) smem[wave] = m;
+        __syncthreads();
+        m = 0;
+#pragma unroll
+        for (int w = 0; w < kSkinnyWaves; ++w) m = umax32(m, smem[w]);
+        scale = scale_from_amax_bits<MI8_E4M3>(m, a.pow2);
+    }
+
+    const uint8_t* wp[NB];
+    wp[0] = g.B + (int64_t)n_row * g.ldb + kg * 32;
+    if constexpr (DUAL) wp[1] = a.B3 + (int64_t)n_row * g.ldb + kg * 32;
+    constexpr int kXBytes = KIND == kFp8 ? 1 : 2;
+    const uint8_t* xp[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int m = mt * 16 + r16 < g.M ? mt * 16 + r16 : g.M - 1;
+        xp[mt] = g.A + ((int64_t)m * g.lda + kg * 32) * kXBytes;
+    }
+
+    const int steps = (g.K + kStep - 1) / kStep;
+    const int per_wave = (steps + kSkinnyWaves - 1) / kSkinnyWaves;
+    const int s_begin = wave * per_wave;
+    const int s_end = s_begin + per_wave < steps ? s_begin + per_wave : steps;
+
+    v4f acc[NB][MT];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[nb][mt] = v4f{0, 0, 0, 0};
+
+    for (int s = s_begin; s < s_end; s += U) {
+        v4i w[U][NB][2];
+        uint4 x[U][MT][2][kXBytes];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t off = (int64_t)(s + u) * kStep;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const bool ok = s + u < s_end && (s + u) * kStep + kg * 32 + 16 * h < g.K;
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) w[u][nb][h] = load16(wp[nb] + off + 16 * h, ok);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int q = 0; q < kXBytes; ++q)
+                        x[u][mt][h][q] = __builtin_bit_cast(uint4, load16(xp[mt] + (off + 16 * h) * kXBytes + 16 * q, ok));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                v4i half[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if constexpr (KIND == kFp8) {
+                        half[h] = __builtin_bit_cast(v4i, x[u][mt][h][0]);
+                    } else {
+                        const bool ok = s + u < s_end && (s + u) * kStep + kg * 32 + 16 * h < g.K;
+                        half[h] = quantise16(x[u][mt][h], scale, ok);
+                    }
+                }
+                const v8i fx = __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    const v8i fw = __builtin_shufflevector(w[u][nb][0], w[u][nb][1], 0, 1, 2, 3, 4, 5, 6, 7);
+                    acc[nb][mt] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fw, fx, acc[nb][mt], 0, 0, 0, 0, 0, 0);
+                }
+            }
+        }
+    }
+
+    const int m = (wave < MT ? wave : 0) * 16 + r16;  // wave mt finishes block mt of the rows of A
+    const int n = n0 + kg * 4;                        // four columns of C per lane (N % 4 == 0)
+    const bool ok = wave < MT && m < g.M && n < g.N;
+    const float isa = 1.0f / scale;
+    uint2 c[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+        if (nb > 0) __syncthreads();  // the previous matrix's sums have been read
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) red[wave][mt][lane] = acc[nb][mt];
+        __syncthreads();
+        c[nb] = make_uint2(0, 0);
+        if (!ok) continue;
+        v4f sum = red[0][wave][lane];
+#pragma unroll
+        for (int w2 = 1; w2 < kSkinnyWaves; ++w2) sum += red[w2][wave][lane];
+        const float f = isa * (1.0f / (nb ? a.sb3[0] : g.sb[0]));
+        c[nb] = make_uint2(pack_bf16x2(sum[0] * f, sum[1] * f), pack_bf16x2(sum[2] * f, sum[3] * f));
+    }
+    uint2 out = c[0];
+    if constexpr (DUAL) out = swiglu_fwd4(c[0], c[NB - 1]);
+    if (ok) *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.C) + (int64_t)m * g.ldc + n) = out;
+    if constexpr (DUAL) {
+        uint32_t hm = ok ? (max_code8(out.x, out.y, out.x, out.y) & 0xFFFFu) << 16 : 0u;
+        hm = wave_umax(hm);
+        if (lane == 0) smem[wave] = hm;  // (the reads of smem above are two barriers back)
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            hm = 0;
+#pragma unroll
+            for (int w2 = 0; w2 < MT; ++w2) hm = umax32(hm, smem[w2]);
+            a.slots_out[blockIdx.x] = hm;
+        }
+    }
+}
+
+template <int MT, int U, int KIND, bool DUAL>
+int launch_few_rows(const FewRowsArgs& a, hipStream_t st, const char* what)
+{
+    hipLaunchKernelGGL((few_rows_kernel<MT, U, KIND, DUAL>), dim3((a.g.N + 15) / 16), dim3(kFewThreads), 0, st, a);
+    return launch_status(what);
+}
+
 }  // namespace
 
 int launch_skinny(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st)
@@ -163,3 +354,60 @@ int launch_skinny(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st)
 
 }  // namespace gemm
 }  // namespace mi8
+
+using namespace mi8;
+using namespace mi8::gemm;
+
+extern "C" int mi8_few_rows_swiglu(const void* x, int x_is_fp8, int64_t lda, const float* sx, const void* b1, const void* b3,
+                                   int64_t ldb, int64_t M, int64_t H, int64_t K, const float* sb1, const float* sb3,
+                                   uint32_t flags, void* h, uint32_t* slots_h, int32_t* n_slots_used, void* stream)
+{
+    MI8_REQUIRE(x && b1 && b3 && sb1 && sb3 && h && slots_h && n_slots_used && (!x_is_fp8 || sx), MI8_ERR_ARG,
+                "mi8_few_rows_swiglu: null pointer");
+    MI8_REQUIRE(M > 0 && M <= kSkinnyMaxM && H > 0 && H <= 16 * MI8_AMAX_SLOTS && H % 8 == 0 && K > 0 && K % 16 == 0 &&
+                    K < (1 << 30),
+                MI8_ERR_UNSUPPORTED,
+                "mi8_few_rows_swiglu: needs 1..%d rows, H %% 8 == 0 up to %d, K %% 16 == 0 (got %lld x %lld x %lld)", kSkinnyMaxM,
+                16 * MI8_AMAX_SLOTS, (long long)M, (long long)H, (long long)K);
+    MI8_REQUIRE(x_is_fp8 || (M * K <= (int64_t)kFewThreads * kAmaxVecs * 8 && M <= 16 && lda == K), MI8_ERR_UNSUPPORTED,
+                "mi8_few_rows_swiglu: bf16 rows must be contiguous, at most 16 of them and at most %d elements (got %lld x %lld); "
+                "use mi8_cast_tensorwise",
+                kFewThreads * kAmaxVecs * 8, (long long)M, (long long)K);
+    MI8_REQUIRE(lda >= K && ldb >= K && lda % 16 == 0 && ldb % 16 == 0, MI8_ERR_UNSUPPORTED,
+                "mi8_few_rows_swiglu: pitches must be multiples of 16 and at least K");
+    MI8_REQUIRE(aligned16(x) && aligned16(b1) && aligned16(b3) && aligned16(h), MI8_ERR_UNSUPPORTED,
+                "mi8_few_rows_swiglu: pointers must be 16-byte aligned");
+    FewRowsArgs a{};
+    a.g = GemmArgs{(const uint8_t*)x, (const uint8_t*)b1, h, 0, lda, ldb, H, (int)M, (int)H, (int)K, sx, sb1, 0, 0, 0, 0, 0};
+    a.B3 = (const uint8_t*)b3;
+    a.sb3 = sb3;
+    a.pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
+    a.slots_out = slots_h;
+    *n_slots_used = (int32_t)((H + 15) / 16);
+    hipStream_t st = (hipStream_t)stream;
+    if (!x_is_fp8) return launch_few_rows<1, 2, kAmax, true>(a, st, "mi8_few_rows_swiglu");
+    if (M <= 16) return launch_few_rows<1, 4, kFp8, true>(a, st, "mi8_few_rows_swiglu");
+    if (M <= 32) return launch_few_rows<2, 2, kFp8, true>(a, st, "mi8_few_rows_swiglu");
+    return launch_few_rows<4, 2, kFp8, true>(a, st, "mi8_few_rows_swiglu");
+}
+
+extern "C" int mi8_few_rows_cast_gemm(const void* x, int64_t lda, const uint32_t* slots, int32_t n_slots, const void* b,
+                                      int64_t ldb, int64_t M, int64_t N, int64_t K, const float* sb, uint32_t flags,
+                                      void* out, int64_t ldc, void* stream)
+{
+    MI8_REQUIRE(x && slots && b && sb && out, MI8_ERR_ARG, "mi8_few_rows_cast_gemm: null pointer");
+    MI8_REQUIRE(M > 0 && M <= 16 && N > 0 && N < (1 << 30) && N % 8 == 0 && K > 0 && K % 16 == 0 && K < (1 << 30),
+                MI8_ERR_UNSUPPORTED, "mi8_few_rows_cast_gemm: needs 1..16 rows, N %% 8 == 0, K %% 16 == 0 (got %lld x %lld x %lld)",
+                (long long)M, (long long)N, (long long)K);
+    MI8_REQUIRE(n_slots > 0 && n_slots <= MI8_AMAX_SLOTS, MI8_ERR_ARG, "mi8_few_rows_cast_gemm: n_slots %d out of range", n_slots);
+    MI8_REQUIRE(lda >= K && ldb >= K && lda % 8 == 0 && ldb % 16 == 0 && ldc >= N && ldc % 4 == 0, MI8_ERR_UNSUPPORTED,
+                "mi8_few_rows_cast_gemm: lda must be a multiple of 8, ldb of 16 (both at least K), ldc of 4 and at least N");
+    MI8_REQUIRE(aligned16(x) && aligned16(b) && aligned16(out), MI8_ERR_UNSUPPORTED,
+                "mi8_few_rows_cast_gemm: pointers must be 16-byte aligned");
+    FewRowsArgs a{};
+    a.g = GemmArgs{(const uint8_t*)x, (const uint8_t*)b, out, 0, lda, ldb, ldc, (int)M, (int)N, (int)K, nullptr, sb, 0, 0, 0, 0, 0};
+    a.slots_in = slots;
+    a.n_slots = n_slots;
+    a.pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
+    return launch_few_rows<1, 2, kSlots, false>(a, (hipStream_t)stream, "mi8_few_rows_cast_gemm");
+}

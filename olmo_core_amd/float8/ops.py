@@ -424,6 +424,68 @@ def gemm_fp8_codes(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch
     return out, codes
 
 
+FEW_ROWS = 64  # rows up to which the entry points below take a generation step
+_FEW_ROWS_SELF_AMAX = 16384  # elements of x up to which few_rows_swiglu quantises x itself (at most 16 rows)
+
+
+def few_rows_supported(M: int, H: int, x_dtype: torch.dtype, w_dtype: torch.dtype) -> bool:
+    """Whether :func:`few_rows_swiglu` (and, up to 16 rows, :func:`few_rows_cast_gemm`) takes the block."""
+    return (M <= FEW_ROWS and H % 16 == 0 and H <= 16 * _C.AMAX_SLOTS and x_dtype == w_dtype == torch.float8_e4m3fn
+            and not FORCE_SW_CVT)
+
+
+def few_rows_quantises(M: int, K: int) -> bool:
+    """Whether :func:`few_rows_swiglu` takes the bf16 rows themselves."""
+    return M <= 16 and M * K <= _FEW_ROWS_SELF_AMAX
+
+
+def few_rows_swiglu(x: torch.Tensor, sx: Optional[torch.Tensor], w1q, s1, w3q, s3, *, pow2: bool = False):
+    """
+    ``h = silu(x1) * x3`` (bf16) and its amax partials ``(slots, n_slots)`` for a few rows, ``x1`` and ``x3`` the two
+    input projections, in one launch; ``x`` is e4m3 with its scale ``sx``, or (:func:`few_rows_quantises`) bf16 with
+    ``sx=None``.  Up to 16 rows ``h`` has the bits of the separate launches.
+    """
+    _require_gpu(x, "few_rows_swiglu")
+    if sx is None:
+        x = _hp2d(x, "few_rows_swiglu")
+    if x.dtype != (torch.bfloat16 if sx is None else torch.float8_e4m3fn) or w1q.dtype != torch.float8_e4m3fn or w3q.dtype != w1q.dtype:
+        raise TypeError("few_rows_swiglu: x must be bfloat16, or float8_e4m3fn with a scale; weights float8_e4m3fn")
+    M, K = x.shape
+    H = w1q.shape[0]
+    if w1q.shape != (H, K) or w3q.shape != (H, K) or w1q.stride(0) != w3q.stride(0) or x.stride(1) != 1 or w1q.stride(1) != 1:
+        raise ValueError("few_rows_swiglu: operands do not fit together")
+    h = torch.empty((M, H), dtype=torch.bfloat16, device=x.device)
+    slots = torch.empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x.device)
+    used = _C.c_int32(0)
+    _C.check(
+        _C.lib().mi8_few_rows_swiglu(
+            x.data_ptr(), int(sx is not None), x.stride(0) if M > 1 else K, sx.data_ptr() if sx is not None else None,
+            w1q.data_ptr(), w3q.data_ptr(), w1q.stride(0), M, H, K, s1.data_ptr(), s3.data_ptr(), _flags(pow2),
+            h.data_ptr(), slots.data_ptr(), used, _stream(x),
+        ),
+        "mi8_few_rows_swiglu",
+    )
+    return h, (slots, used.value)
+
+
+def few_rows_cast_gemm(x: torch.Tensor, slots: Tuple[torch.Tensor, int], wq, sw, *, pow2: bool = False) -> torch.Tensor:
+    """``gemm_fp8(*cast_tensorwise(x, e4m3, slots=slots), wq, sw)`` for at most 16 rows in one launch, with its bits."""
+    x = _hp2d(x, "few_rows_cast_gemm")
+    if x.dtype != torch.bfloat16 or wq.dtype != torch.float8_e4m3fn or wq.shape[1] != x.shape[1] or wq.stride(1) != 1:
+        raise ValueError("few_rows_cast_gemm: expects bfloat16 rows and a float8_e4m3fn weight of the same row length")
+    M, K = x.shape
+    N = wq.shape[0]
+    out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    _C.check(
+        _C.lib().mi8_few_rows_cast_gemm(
+            x.data_ptr(), K, slots[0].data_ptr(), slots[1], wq.data_ptr(), wq.stride(0), M, N, K, sw.data_ptr(),
+            _flags(pow2), out.data_ptr(), N, _stream(x),
+        ),
+        "mi8_few_rows_cast_gemm",
+    )
+    return out
+
+
 def gemm_variants() -> list:
     L = _C.lib()
     return [L.mi8_gemm_variant_name(i).decode() for i in range(L.mi8_gemm_num_variants())]

@@ -65,14 +65,14 @@ def _fused_launch_ok(M: int, D: int, H: int) -> bool:
     return FUSE_SWIGLU_EPILOGUE and ops.swiglu_gemm_matches_separate(M, H, D)
 
 
-def _mlp_forward(x, w1, w2, w3, c, need, ws=(None, None, None), wo=(None, None, None)):
+def _mlp_forward(x, w1, w2, w3, c, need, ws=(None, None, None), wo=(None, None, None), keep=True):
     """y = (silu(x W1^T) * (x W3^T)) W2^T with tensorwise float8 GEMMs; x [M, D], W1/W3 [H, D], W2 [D, H].  x is
     converted to bfloat16 first if it is of another type (float32 activations under autocast: each of the three
     modules would convert its own input).
     need: which of (x, w1, w2, w3) get a gradient.  ws: weight scales precomputed after the optimizer step (None: reduce
     the amax here); wo: float8 copies the modules keep between calls (None: quantise the weight here); both in the
     order (w1, w2, w3).  Returns ``(y, saved)``, ``saved`` being the 13 tensors :func:`_mlp_backward` takes (an empty
-    tensor where nothing is kept)."""
+    tensor where nothing is kept).  keep=False: only ``y`` is wanted (no gradients, ``saved`` is not to be used)."""
     pow2 = c.round_scales_to_power_of_2
     in_dt, w_dt = c.cast_config_input.target_dtype, c.cast_config_weight.target_dtype
     any_grad = any(need)
@@ -81,19 +81,31 @@ def _mlp_forward(x, w1, w2, w3, c, need, ws=(None, None, None), wo=(None, None, 
     x_codes = None
     if x.dtype != torch.bfloat16:
         x = x.to(torch.bfloat16)
+    M, D, H = x.shape[0], x.shape[1], w1.shape[0]
+    # a generation step: launches that wait for one another are the time, so the activations are quantised by the GEMMs
+    few_rows = not keep and STAGE_SINK is None and ops.few_rows_supported(M, H, in_dt, w_dt) and w2.shape[0] % 8 == 0
+    x_in_gemm = few_rows and ops.few_rows_quantises(M, D)
     # The amax of x and of every weight that still needs one is taken in a single launch.
-    todo = [x] + [w for w, s, o in ((w1, ws1, wo1), (w3, ws3, wo3), (w2, ws2, wo2)) if s is None and o is None]
+    todo = [w for w, s, o in ((w1, ws1, wo1), (w3, ws3, wo3), (w2, ws2, wo2)) if s is None and o is None]
+    if not x_in_gemm:
+        todo.insert(0, x)
     part = {}
-    if len(todo) > 1 and all(t.dtype == x.dtype and t.is_contiguous() for t in todo):
+    if len(todo) > 1 and all(t.dtype == todo[0].dtype and t.is_contiguous() for t in todo):
         part = {id(t): p for t, p in zip(todo, ops.amax_partials_batch(todo))}
-    xq, xq_t, sx = ops.cast_tensorwise(x, in_dt, pow2=pow2, want_transposed=need[1] or need[3], slots=part.get(id(x)))
+    xq, xq_t, sx = (x, None, None) if x_in_gemm else ops.cast_tensorwise(
+        x, in_dt, pow2=pow2, want_transposed=need[1] or need[3], slots=part.get(id(x)))
     w1q, w1q_t, s1 = wo1 or ops.cast_tensorwise(w1, w_dt, pow2=pow2, want_transposed=need[0], scale=ws1,
                                                 slots=part.get(id(w1)))
     w3q, w3q_t, s3 = wo3 or ops.cast_tensorwise(w3, w_dt, pow2=pow2, want_transposed=need[0], scale=ws3,
                                                 slots=part.get(id(w3)))
     w2q, w2q_t, s2 = wo2 or ops.cast_tensorwise(w2, w_dt, pow2=pow2, want_transposed=any_grad, scale=ws2,
                                                 slots=part.get(id(w2)))
-    M, D, H = x.shape[0], x.shape[1], w1.shape[0]
+    if few_rows:
+        h, h_slots = ops.few_rows_swiglu(xq, sx, w1q, s1, w3q, s3, pow2=pow2)
+        if M <= 16:
+            return ops.few_rows_cast_gemm(h, h_slots, w2q, s2, pow2=pow2), ()
+        hq, _, sh = ops.cast_tensorwise(h, in_dt, pow2=pow2, slots=h_slots)
+        return ops.gemm_fp8(hq, sh, w2q, s2, out_dtype=x.dtype), ()
     if _fused_launch_ok(M, D, H):
         # both input projections and the activation in one launch: x1 and x3 are never read back
         if _use_codes(M, D, H, any_grad):
@@ -267,7 +279,7 @@ class FeedForward(nn.Module):
             else:
                 # nothing to differentiate: no transposed float8 copies, nothing kept for a backward (an autograd
                 # function reports its inputs' requires_grad also where gradients are off)
-                y = _mlp_forward(x2, *weights, self.w1.config, (False,) * 4, scales, operands)[0]
+                y = _mlp_forward(x2, *weights, self.w1.config, (False,) * 4, scales, operands, keep=False)[0]
             return y.reshape(*x.shape[:-1], self.w2.weight.shape[0])
         x1, x3 = self.w1(x), self.w3(x)
         if x1.is_cuda and x1.dtype == torch.bfloat16 and not compiling:

@@ -9,19 +9,19 @@ from oracle import float8_oracle as O
 
 pytestmark = pytest.mark.gpu
 
-from olmo_core_amd.float8 import AOFloat8LinearRecipe, Float8Config  # noqa: E402
+from olmo_core_amd.float8 import AOFloat8LinearConfig, AOFloat8LinearRecipe, Float8Config  # noqa: E402
 from olmo_core_amd.float8 import ops  # noqa: E402
 from olmo_core_amd.nn import FeedForward  # noqa: E402
 
 
-def _make(dev, D, H, fuse, recipe="tensorwise", seed=0):
+def _make(dev, D, H, fuse, recipe="tensorwise", seed=0, ao=None):
     g = torch.Generator().manual_seed(seed)
     ff = FeedForward(d_model=D, hidden_size=H, bias=False, dtype=torch.bfloat16, fuse_float8=fuse)
     with torch.no_grad():
         for p in ff.parameters():
             p.copy_((torch.randn(p.shape, generator=g) * 0.02).bfloat16())
     ff = ff.to(dev)
-    Float8Config(ao_recipe=AOFloat8LinearRecipe(recipe)).apply_float8_linear(ff)
+    (Float8Config(ao=ao) if ao else Float8Config(ao_recipe=AOFloat8LinearRecipe(recipe))).apply_float8_linear(ff)
     return ff
 
 
@@ -303,3 +303,31 @@ def test_compiled_modules_use_their_kept_weights(dev, monkeypatch):
             p.mul_(1.5)
     y = compiled(xs[0])
     assert len(casts) == 8 and torch.equal(y, fwd(model, xs[0]))
+
+
+@pytest.mark.parametrize("kept", [True, False], ids=["kept_weights", "plain"])
+@pytest.mark.parametrize("mdh", [(1, 4096, 11008), (1, 1040, 2768), (4, 4096, 528), (5, 4096, 528), (16, 1024, 2816), (17, 1040, 2768),
+                                 (33, 768, 2048), (64, 1024, 528), (65, 1024, 528)], ids=lambda s: "x".join(map(str, s)))
+def test_evaluation_gives_the_training_forward(dev, mdh, kept):
+    """Without gradients the block takes other launches (activations quantised by the GEMMs, no transposed copies)."""
+    M, D, H = mdh
+    ff = _make(dev, D, H, fuse=True, ao=AOFloat8LinearConfig.recommended() if kept else None)
+    x = seeded((M, D), 1).to(dev)
+    x[0, 3] = 40.0
+    want = ff(x.clone().requires_grad_(True)).detach()
+    for ctx in (torch.no_grad(), torch.inference_mode()):
+        with ctx:
+            got = ff(x)
+        if M <= 16 or M > 64:
+            assert torch.equal(got, want)
+        else:
+            # sums in another order: bf16 roundings of h, a few of which move a float8 code of the second product
+            assert_gemm_close(got, want.cpu(), "y")
+    for v in (float("nan"), float("inf"), 0.0):
+        x[0, 5] = v
+        if v == 0.0:
+            x.zero_()
+        want = ff(x.clone().requires_grad_(True)).detach()
+        with torch.no_grad():
+            got = ff(x)
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(), want.nan_to_num())
