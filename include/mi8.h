@@ -315,7 +315,7 @@ int mi8_few_rows_swiglu(const void* x, int x_is_fp8, int64_t lda, const float* s
 
 /* out[M, ldc] (bf16) = q(x) B^T scaled, x bf16 [M, lda], M <= 16, quantised to e4m3 by the launch with the scale of the
  * partial maxima `slots` (mi8_scale_from_partials): the bits of mi8_cast_tensorwise followed by mi8_gemm_fp8.
- * N % 8 == 0, K % 16 == 0, lda % 8 == 0, ldb % 16 == 0, ldc % 4 == 0, pointers 16-byte aligned. */
+ * M * K <= 65536, N % 8 == 0, K % 16 == 0, lda % 8 == 0, ldb % 16 == 0, ldc % 4 == 0, pointers 16-byte aligned. */
 int mi8_few_rows_cast_gemm(const void* x, int64_t lda, const uint32_t* slots, int32_t n_slots, const void* b, int64_t ldb,
                            int64_t M, int64_t N, int64_t K, const float* sb, uint32_t flags, void* out, int64_t ldc,
                            void* stream);

@@ -152,15 +152,18 @@ int launch_skinny_typed(const GemmArgs& g, int a_dtype, int b_dtype, hipStream_t
 // ---- the same for a generation step of a SwiGLU block: activations quantised by the GEMM that reads them ------------
 //
 // A step on one token is a chain of launches that each wait for the one before: cast, two projections, SwiGLU, cast,
-// projection.  The arithmetic on the activations is so small that every workgroup can repeat it: kind_x says how the
+// projection.  The arithmetic on the activations is so small that every workgroup can repeat it: KIND says how the
 // kernel gets its float8 rows of A,
 //   kFp8      they are in memory with their scale,
 //   kSlots    A is bf16 and partial maxima of |A| are in memory (left by the launch that produced A): every workgroup
-//             folds them into the scale and converts its fragments on the way into the MFMAs,
+//             folds them into the scale and converts A into LDS,
 //   kAmax     A is bf16 and small: every workgroup takes the amax itself as well.
 // DUAL: 16 rows of B and the same 16 rows of a second matrix B3 per workgroup, x1 = A B^T, x3 = A B3^T; the epilogue
 // rounds both to bf16 and stores only h = silu(x1) * x3, with a partial maximum of |h| per workgroup.
-// Bytes, scales and sums are those of the separate launches.  One token, 4096 -> 11008 -> 4096: two launches instead of six.
+// The time is streaming B: a wave's next step is on its way while it works on one, the first while A is quantised, and
+// the registers leave room for three workgroups a compute unit, so that the 688 of 11008 rows run in one round (with two
+// fitting: 28 us for 90 MB; converting in registers instead of LDS: 17.7 us for 45 MB).
+// Bytes, scales and sums are those of the separate launches.
 enum FewRowsInput { kFp8, kSlots, kAmax };
 
 struct FewRowsArgs {
@@ -175,26 +178,22 @@ struct FewRowsArgs {
 
 constexpr int kFewThreads = kSkinnyWaves * 64;
 constexpr int kAmaxVecs = 4;  // 8-element groups of A per lane where every workgroup takes the amax
+constexpr int kLdsElems = 65536;  // bytes of LDS for A where partial maxima are given
 
-// 16 quantised K bytes of one row (zeros past the end of K) from 16 bf16 values
-__device__ __forceinline__ v4i quantise16(const uint4 (&v)[2], float s, bool ok)
+// eight bf16 values -> eight e4m3 bytes
+__device__ __forceinline__ uint2 quantise8(uint4 v, float s)
 {
-    v4i r{0, 0, 0, 0};
-    if (!ok) return r;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        r[2 * h] = (int)quant4<MI8_E4M3, false>(bits_to_f32(v[h].x << 16), bits_to_f32(v[h].x & 0xFFFF0000u),
-                                                bits_to_f32(v[h].y << 16), bits_to_f32(v[h].y & 0xFFFF0000u), s, s, s, s);
-        r[2 * h + 1] = (int)quant4<MI8_E4M3, false>(bits_to_f32(v[h].z << 16), bits_to_f32(v[h].z & 0xFFFF0000u),
-                                                    bits_to_f32(v[h].w << 16), bits_to_f32(v[h].w & 0xFFFF0000u), s, s, s, s);
-    }
-    return r;
+    float f[8];
+    unpack8(v, f);
+    return make_uint2(quant4<MI8_E4M3, false>(f[0], f[1], f[2], f[3], s, s, s, s),
+                      quant4<MI8_E4M3, false>(f[4], f[5], f[6], f[7], s, s, s, s));
 }
 
 template <int MT, int U, int KIND, bool DUAL>
-__global__ __launch_bounds__(kFewThreads) void few_rows_kernel(FewRowsArgs a)
+__global__ __launch_bounds__(kFewThreads, MT == 1 ? 6 : MT == 2 ? 4 : 2) void few_rows_kernel(FewRowsArgs a)
 {
     constexpr int NB = DUAL ? 2 : 1;
+    extern __shared__ __attribute__((aligned(16))) uint8_t aq[];  // kSlots, kAmax: A in e4m3, [M][K]
     __shared__ v4f red[kSkinnyWaves][MT][64];
     __shared__ uint32_t smem[kSkinnyWaves];
     const GemmArgs& g = a.g;
@@ -204,21 +203,41 @@ __global__ __launch_bounds__(kFewThreads) void few_rows_kernel(FewRowsArgs a)
     const int n0 = (int)blockIdx.x * 16;
     const int n_row = n0 + r16 < g.N ? n0 + r16 : g.N - 1;
 
+    const int steps = (g.K + kStep - 1) / kStep;
+    const int per_wave = (steps + kSkinnyWaves - 1) / kSkinnyWaves;
+    const int s_begin = wave * per_wave;
+    const int s_end = s_begin + per_wave < steps ? s_begin + per_wave : steps;
+
+    const uint8_t* wp[NB];
+    wp[0] = g.B + (int64_t)n_row * g.ldb + kg * 32;
+    if constexpr (DUAL) wp[1] = a.B3 + (int64_t)n_row * g.ldb + kg * 32;
+    v4i w[U][NB][2], w_next[U][NB][2];
+    auto inside = [&](int s, int h) { return s < s_end && s * kStep + kg * 32 + 16 * h < g.K; };
+    auto load_w = [&](v4i(&to)[U][NB][2], int s) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+                    to[u][nb][h] = load16(wp[nb] + (int64_t)(s + u) * kStep + 16 * h, inside(s + u, h));
+    };
+    load_w(w, s_begin);
+
     float scale;
     if constexpr (KIND == kFp8) {
         scale = g.sa[0];
     } else {
         uint32_t m = 0;
+        const int per_row = g.K / 8, groups = g.M * per_row;
+        uint4 v[KIND == kAmax ? kAmaxVecs : 1];
         if constexpr (KIND == kSlots) {
             for (int i = threadIdx.x; i < a.n_slots; i += kFewThreads) m = umax32(m, a.slots_in[i]);
-        } else {
-            const uint4* x = reinterpret_cast<const uint4*>(g.A);  // contiguous, at most kFewThreads * kAmaxVecs groups
-            const int groups = g.M * (g.K / 8);
-            uint4 v[kAmaxVecs];
+        } else {  // contiguous, at most kFewThreads * kAmaxVecs groups
 #pragma unroll
             for (int i = 0; i < kAmaxVecs; ++i) {
                 const int k = (int)threadIdx.x + kFewThreads * i;
-                v[i] = k < groups ? x[k] : make_uint4(0, 0, 0, 0);
+                v[i] = k < groups ? reinterpret_cast<const uint4*>(g.A)[k] : make_uint4(0, 0, 0, 0);
             }
 #pragma unroll
             for (int i = 0; i < kAmaxVecs; ++i) m = umax32(m, (max_code8(v[i].x, v[i].y, v[i].z, v[i].w) & 0xFFFFu) << 16);
@@ -228,25 +247,30 @@ __global__ __launch_bounds__(kFewThreads) void few_rows_kernel(FewRowsArgs a)
         __syncthreads();
         m = 0;
 #pragma unroll
-        for (int w = 0; w < kSkinnyWaves; ++w) m = umax32(m, smem[w]);
+        for (int i = 0; i < kSkinnyWaves; ++i) m = umax32(m, smem[i]);
         scale = scale_from_amax_bits<MI8_E4M3>(m, a.pow2);
+        if constexpr (KIND == kAmax) {
+#pragma unroll
+            for (int i = 0; i < kAmaxVecs; ++i) {
+                const int k = (int)threadIdx.x + kFewThreads * i;
+                if (k < groups) reinterpret_cast<uint2*>(aq)[k] = quantise8(v[i], scale);
+            }
+        } else {
+            for (int k = threadIdx.x; k < groups; k += kFewThreads) {
+                const int r = k / per_row, c = k - r * per_row;
+                const uint16_t* row = reinterpret_cast<const uint16_t*>(g.A) + (int64_t)r * g.lda;
+                reinterpret_cast<uint2*>(aq)[k] = quantise8(*reinterpret_cast<const uint4*>(row + 8 * c), scale);
+            }
+        }
+        __syncthreads();
     }
 
-    const uint8_t* wp[NB];
-    wp[0] = g.B + (int64_t)n_row * g.ldb + kg * 32;
-    if constexpr (DUAL) wp[1] = a.B3 + (int64_t)n_row * g.ldb + kg * 32;
-    constexpr int kXBytes = KIND == kFp8 ? 1 : 2;
     const uint8_t* xp[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         const int m = mt * 16 + r16 < g.M ? mt * 16 + r16 : g.M - 1;
-        xp[mt] = g.A + ((int64_t)m * g.lda + kg * 32) * kXBytes;
+        xp[mt] = (KIND == kFp8 ? g.A + (int64_t)m * g.lda : aq + m * g.K) + kg * 32;
     }
-
-    const int steps = (g.K + kStep - 1) / kStep;
-    const int per_wave = (steps + kSkinnyWaves - 1) / kSkinnyWaves;
-    const int s_begin = wave * per_wave;
-    const int s_end = s_begin + per_wave < steps ? s_begin + per_wave : steps;
 
     v4f acc[NB][MT];
 #pragma unroll
@@ -254,39 +278,25 @@ __global__ __launch_bounds__(kFewThreads) void few_rows_kernel(FewRowsArgs a)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[nb][mt] = v4f{0, 0, 0, 0};
 
-    for (int s = s_begin; s < s_end; s += U) {
-        v4i w[U][NB][2];
-        uint4 x[U][MT][2][kXBytes];
+    v4i x[U][MT][2], x_next[U][MT][2];
+    auto load_x = [&](v4i(&to)[U][MT][2], int s) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t off = (int64_t)(s + u) * kStep;
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const bool ok = s + u < s_end && (s + u) * kStep + kg * 32 + 16 * h < g.K;
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) w[u][nb][h] = load16(wp[nb] + off + 16 * h, ok);
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int q = 0; q < kXBytes; ++q)
-                        x[u][mt][h][q] = __builtin_bit_cast(uint4, load16(xp[mt] + (off + 16 * h) * kXBytes + 16 * q, ok));
-            }
-        }
+                    to[u][mt][h] = load16(xp[mt] + (int64_t)(s + u) * kStep + 16 * h, inside(s + u, h));
+    };
+    load_x(x, s_begin);
+    for (int s = s_begin; s < s_end; s += U) {
+        load_w(w_next, s + U);
+        load_x(x_next, s + U);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-                v4i half[2];
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    if constexpr (KIND == kFp8) {
-                        half[h] = __builtin_bit_cast(v4i, x[u][mt][h][0]);
-                    } else {
-                        const bool ok = s + u < s_end && (s + u) * kStep + kg * 32 + 16 * h < g.K;
-                        half[h] = quantise16(x[u][mt][h], scale, ok);
-                    }
-                }
-                const v8i fx = __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                const v8i fx = __builtin_shufflevector(x[u][mt][0], x[u][mt][1], 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
                     const v8i fw = __builtin_shufflevector(w[u][nb][0], w[u][nb][1], 0, 1, 2, 3, 4, 5, 6, 7);
@@ -294,6 +304,18 @@ __global__ __launch_bounds__(kFewThreads) void few_rows_kernel(FewRowsArgs a)
                 }
             }
         }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) w[u][nb][h] = w_next[u][nb][h];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) x[u][mt][h] = x_next[u][mt][h];
     }
 
     const int m = (wave < MT ? wave : 0) * 16 + r16;  // wave mt finishes block mt of the rows of A
@@ -335,7 +357,12 @@ __global__ __launch_bounds__(kFewThreads) void few_rows_kernel(FewRowsArgs a)
 template <int MT, int U, int KIND, bool DUAL>
 int launch_few_rows(const FewRowsArgs& a, hipStream_t st, const char* what)
 {
-    hipLaunchKernelGGL((few_rows_kernel<MT, U, KIND, DUAL>), dim3((a.g.N + 15) / 16), dim3(kFewThreads), 0, st, a);
+    static std::atomic<uint64_t> configured;
+    if constexpr (KIND == kSlots)
+        if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(few_rows_kernel<MT, U, KIND, DUAL>), kLdsElems, configured, what))
+            return rc;
+    const int lds = KIND == kFp8 ? 0 : a.g.M * a.g.K;  // (K % 16 == 0)
+    hipLaunchKernelGGL((few_rows_kernel<MT, U, KIND, DUAL>), dim3((a.g.N + 15) / 16), dim3(kFewThreads), lds, st, a);
     return launch_status(what);
 }
 
@@ -385,10 +412,10 @@ extern "C" int mi8_few_rows_swiglu(const void* x, int x_is_fp8, int64_t lda, con
     a.slots_out = slots_h;
     *n_slots_used = (int32_t)((H + 15) / 16);
     hipStream_t st = (hipStream_t)stream;
-    if (!x_is_fp8) return launch_few_rows<1, 2, kAmax, true>(a, st, "mi8_few_rows_swiglu");
-    if (M <= 16) return launch_few_rows<1, 4, kFp8, true>(a, st, "mi8_few_rows_swiglu");
-    if (M <= 32) return launch_few_rows<2, 2, kFp8, true>(a, st, "mi8_few_rows_swiglu");
-    return launch_few_rows<4, 2, kFp8, true>(a, st, "mi8_few_rows_swiglu");
+    if (!x_is_fp8) return launch_few_rows<1, 1, kAmax, true>(a, st, "mi8_few_rows_swiglu");
+    if (M <= 16) return launch_few_rows<1, 1, kFp8, true>(a, st, "mi8_few_rows_swiglu");
+    if (M <= 32) return launch_few_rows<2, 1, kFp8, true>(a, st, "mi8_few_rows_swiglu");
+    return launch_few_rows<4, 1, kFp8, true>(a, st, "mi8_few_rows_swiglu");
 }
 
 extern "C" int mi8_few_rows_cast_gemm(const void* x, int64_t lda, const uint32_t* slots, int32_t n_slots, const void* b,
@@ -399,6 +426,8 @@ extern "C" int mi8_few_rows_cast_gemm(const void* x, int64_t lda, const uint32_t
     MI8_REQUIRE(M > 0 && M <= 16 && N > 0 && N < (1 << 30) && N % 8 == 0 && K > 0 && K % 16 == 0 && K < (1 << 30),
                 MI8_ERR_UNSUPPORTED, "mi8_few_rows_cast_gemm: needs 1..16 rows, N %% 8 == 0, K %% 16 == 0 (got %lld x %lld x %lld)",
                 (long long)M, (long long)N, (long long)K);
+    MI8_REQUIRE(M * K <= kLdsElems, MI8_ERR_UNSUPPORTED, "mi8_few_rows_cast_gemm: at most %d elements (got %lld x %lld); use "
+                "mi8_cast_tensorwise and mi8_gemm_fp8", kLdsElems, (long long)M, (long long)K);
     MI8_REQUIRE(n_slots > 0 && n_slots <= MI8_AMAX_SLOTS, MI8_ERR_ARG, "mi8_few_rows_cast_gemm: n_slots %d out of range", n_slots);
     MI8_REQUIRE(lda >= K && ldb >= K && lda % 8 == 0 && ldb % 16 == 0 && ldc >= N && ldc % 4 == 0, MI8_ERR_UNSUPPORTED,
                 "mi8_few_rows_cast_gemm: lda must be a multiple of 8, ldb of 16 (both at least K), ldc of 4 and at least N");

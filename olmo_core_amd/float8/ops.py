@@ -434,9 +434,9 @@ def few_rows_supported(M: int, H: int, x_dtype: torch.dtype, w_dtype: torch.dtyp
             and not FORCE_SW_CVT)
 
 
-def few_rows_quantises(M: int, K: int) -> bool:
-    """Whether :func:`few_rows_swiglu` takes the bf16 rows themselves."""
-    return M <= 16 and M * K <= _FEW_ROWS_SELF_AMAX
+def few_rows_quantises(M: int, K: int, have_slots: bool = False) -> bool:
+    """Whether :func:`few_rows_swiglu` (with ``have_slots``: :func:`few_rows_cast_gemm`) takes bf16 rows of this size."""
+    return M <= 16 and M * K <= (_SMALL_CAST if have_slots else _FEW_ROWS_SELF_AMAX)
 
 
 def few_rows_swiglu(x: torch.Tensor, sx: Optional[torch.Tensor], w1q, s1, w3q, s3, *, pow2: bool = False):
@@ -469,7 +469,8 @@ def few_rows_swiglu(x: torch.Tensor, sx: Optional[torch.Tensor], w1q, s1, w3q, s
 
 
 def few_rows_cast_gemm(x: torch.Tensor, slots: Tuple[torch.Tensor, int], wq, sw, *, pow2: bool = False) -> torch.Tensor:
-    """``gemm_fp8(*cast_tensorwise(x, e4m3, slots=slots), wq, sw)`` for at most 16 rows in one launch, with its bits."""
+    """``gemm_fp8(*cast_tensorwise(x, e4m3, slots=slots), wq, sw)`` in one launch, with its bits, for the
+    sizes of ``few_rows_quantises(..., have_slots=True)``."""
     x = _hp2d(x, "few_rows_cast_gemm")
     if x.dtype != torch.bfloat16 or wq.dtype != torch.float8_e4m3fn or wq.shape[1] != x.shape[1] or wq.stride(1) != 1:
         raise ValueError("few_rows_cast_gemm: expects bfloat16 rows and a float8_e4m3fn weight of the same row length")

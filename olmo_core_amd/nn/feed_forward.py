@@ -102,7 +102,7 @@ def _mlp_forward(x, w1, w2, w3, c, need, ws=(None, None, None), wo=(None, None, 
                                                 slots=part.get(id(w2)))
     if few_rows:
         h, h_slots = ops.few_rows_swiglu(xq, sx, w1q, s1, w3q, s3, pow2=pow2)
-        if M <= 16:
+        if ops.few_rows_quantises(M, H, have_slots=True):
             return ops.few_rows_cast_gemm(h, h_slots, w2q, s2, pow2=pow2), ()
         hq, _, sh = ops.cast_tensorwise(h, in_dt, pow2=pow2, slots=h_slots)
         return ops.gemm_fp8(hq, sh, w2q, s2, out_dtype=x.dtype), ()
