@@ -52,6 +52,7 @@ typedef enum mi8_hp {
 /* flags shared by the cast entry points */
 #define MI8_FLAG_POW2_SCALE 1u /* round every scale down to a power of two (ao.py:167 round_scales_to_power_of_2) */
 #define MI8_FLAG_SW_CVT 2u     /* convert with integer arithmetic instead of v_cvt_pk_{fp8,bf8}_f32 (same bytes) */
+#define MI8_FLAG_PAD_T128 8u   /* transposed copies of tensorwise casts: zero columns up to a multiple of 128 instead of 16 */
 #define MI8_FLAG_AMAX_READY 4u /* grouped casts: the amax workspaces already hold the amax of x (see mi8_grouped_swiglu_*) */
 
 /* Number of uint32 slots a tensorwise amax workspace must have. */
@@ -109,7 +110,9 @@ int mi8_multi_tensor_scales(const void* const* ptrs, const int64_t* numels, int3
  *                        bytes cols..ld_out-1 of a row are not touched.
  *   out_t (may be NULL): fp8 [cols, ld_t], the transposed copy; ld_t >= rows, ld_t % 16 == 0; columns
  *                        rows..round_up(rows,16)-1 of out_t are written as zero (so that a GEMM may contract
- *                        over round_up(rows,16)), columns beyond are not touched.
+ *                        over round_up(rows,16)), columns beyond are not touched.  With MI8_FLAG_PAD_T128 both
+ *                        are multiples of 128: ld_t >= round_up(rows,128), zeros up to there (the persistent GEMM
+ *                        contracts whole 128-byte steps).
  * cols % 16 == 0 is required.  The GEMMs accept any operand pitch that is a multiple of 16. */
 int mi8_cast_tensorwise(const void* x, int hp_dtype, int64_t rows, int64_t cols, const uint32_t* slots,
                         int32_t n_slots, const float* scale_in, int fp8_dtype, uint32_t flags, void* out,

@@ -24,6 +24,7 @@ MI8_BF16, MI8_F32, MI8_F16, MI8_RAW8 = 0, 1, 2, 3
 FLAG_POW2_SCALE = 1
 FLAG_SW_CVT = 2
 FLAG_AMAX_READY = 4
+FLAG_PAD_T128 = 8
 AMAX_SLOTS = 2048
 
 # name -> (restype, argtypes); mirrors include/mi8.h one to one

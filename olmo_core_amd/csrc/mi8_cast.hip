@@ -176,6 +176,7 @@ struct TileCastArgs {
     uint8_t* out_t;  // [cols, ld_t] or null
     int64_t ld_t;
     float* scale_out;  // scalar modes: [1]; per-column mode: [cols]; may be null
+    int64_t t_end;     // columns of out_t written: rows and the zeros after them
 };
 
 // Source row of logical row r when the casts read their input through a token permutation (the rows of a
@@ -362,7 +363,7 @@ __global__ __launch_bounds__(kThreads) void tile_cast_kernel(TileCastArgs a)
     }
 
     tile_cast_body<HP, FP8, SW>(a.x, a.rows, a.cols, row0, col0, sc, a.out, a.ld_out, a.out_t, a.ld_t, row0,
-                                (a.rows + 15) / 16 * 16, lds_t);
+                                a.t_end, lds_t);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -647,6 +648,7 @@ struct SwigluBwdCastArgs {
     int64_t ld_t;
     float* scale_out1;  // [1]
     float* scale_out3;
+    int64_t t_end;  // columns of the transposed copies written
 };
 
 template <int FP8, bool SW>
@@ -726,7 +728,7 @@ __global__ __launch_bounds__(kThreads) void swiglu_bwd_cast_kernel(SwigluBwdCast
     }
     if (want_t) {
         __syncthreads();
-        const int64_t dst_end = (a.rows + 15) / 16 * 16;
+        const int64_t dst_end = a.t_end;
 #pragma unroll
         for (int o = 0; o < 2; ++o)
 #pragma unroll
@@ -1156,6 +1158,7 @@ extern "C" int mi8_cast_tensorwise(const void* x, int hp_dtype, int64_t rows, in
                                    int32_t n_slots, const float* scale_in, int fp8_dtype, uint32_t flags, void* out,
                                    int64_t ld_out, void* out_t, int64_t ld_t, float* scale_out, void* stream)
 {
+    const int64_t t_end = round_up(rows, flags & MI8_FLAG_PAD_T128 ? 128 : 16);
     MI8_REQUIRE(x, MI8_ERR_ARG, "mi8_cast_tensorwise: x is null");
     MI8_REQUIRE(out || out_t, MI8_ERR_ARG, "mi8_cast_tensorwise: no output requested");
     MI8_REQUIRE(valid_hp(hp_dtype) && valid_fp8(fp8_dtype), MI8_ERR_ARG, "mi8_cast_tensorwise: unknown dtype");
@@ -1177,8 +1180,9 @@ extern "C" int mi8_cast_tensorwise(const void* x, int hp_dtype, int64_t rows, in
         MI8_REQUIRE(ld_out >= cols && ld_out % 16 == 0, MI8_ERR_UNSUPPORTED,
                     "mi8_cast_tensorwise: ld_out (%lld) must be a multiple of 16 and at least cols", (long long)ld_out);
     if (out_t)
-        MI8_REQUIRE(ld_t >= rows && ld_t % 16 == 0, MI8_ERR_UNSUPPORTED,
-                    "mi8_cast_tensorwise: ld_t (%lld) must be a multiple of 16 and at least rows", (long long)ld_t);
+        MI8_REQUIRE(ld_t >= rows && ld_t % 16 == 0 && (!(flags & MI8_FLAG_PAD_T128) || ld_t >= t_end), MI8_ERR_UNSUPPORTED,
+                    "mi8_cast_tensorwise: ld_t (%lld) must be a multiple of 16 and at least rows (rounded up to 128 with MI8_FLAG_PAD_T128)",
+                    (long long)ld_t);
     if (fused_amax) {
         const bool sw = (flags & MI8_FLAG_SW_CVT) != 0, pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
         if (hp_dtype == MI8_BF16)
@@ -1188,7 +1192,7 @@ extern "C" int mi8_cast_tensorwise(const void* x, int hp_dtype, int64_t rows, in
         return launch_status("mi8_cast_tensorwise");
     }
     TileCastArgs a{x, rows, cols, slots, n_slots, scale_in, (flags & MI8_FLAG_POW2_SCALE) != 0,
-                   (uint8_t*)out, ld_out, (uint8_t*)out_t, ld_t, scale_out};
+                   (uint8_t*)out, ld_out, (uint8_t*)out_t, ld_t, scale_out, t_end};
     dispatch_tile_cast(hp_dtype, fp8_dtype, (flags & MI8_FLAG_SW_CVT) != 0, slots ? kScalarFromSlots : kScalarFromPtr,
                        a, (hipStream_t)stream);
     return launch_status("mi8_cast_tensorwise");
@@ -1266,6 +1270,7 @@ extern "C" int mi8_swiglu_bwd_cast(const void* x1, const void* x3, const void* g
                                    uint32_t flags, void* out1, void* out3, int64_t ld_out, void* out1_t, void* out3_t,
                                    int64_t ld_t, float* scale_out1, float* scale_out3, void* stream)
 {
+    const int64_t t_end = round_up(rows, flags & MI8_FLAG_PAD_T128 ? 128 : 16);
     MI8_REQUIRE(x1 && x3 && gh && slots_g1 && slots_g3 && scale_out1 && scale_out3, MI8_ERR_ARG,
                 "mi8_swiglu_bwd_cast: null pointer");
     MI8_REQUIRE((out1 != nullptr) == (out3 != nullptr) && (out1_t != nullptr) == (out3_t != nullptr) && (out1 || out1_t),
@@ -1282,11 +1287,12 @@ extern "C" int mi8_swiglu_bwd_cast(const void* x1, const void* x3, const void* g
         MI8_REQUIRE(ld_out >= cols && ld_out % 16 == 0, MI8_ERR_UNSUPPORTED,
                     "mi8_swiglu_bwd_cast: ld_out (%lld) must be a multiple of 16 and at least cols", (long long)ld_out);
     if (out1_t)
-        MI8_REQUIRE(ld_t >= rows && ld_t % 16 == 0, MI8_ERR_UNSUPPORTED,
-                    "mi8_swiglu_bwd_cast: ld_t (%lld) must be a multiple of 16 and at least rows", (long long)ld_t);
+        MI8_REQUIRE(ld_t >= rows && ld_t % 16 == 0 && (!(flags & MI8_FLAG_PAD_T128) || ld_t >= t_end), MI8_ERR_UNSUPPORTED,
+                    "mi8_swiglu_bwd_cast: ld_t (%lld) must be a multiple of 16 and at least rows (rounded up to 128 with MI8_FLAG_PAD_T128)",
+                    (long long)ld_t);
     SwigluBwdCastArgs a{(const uint4*)x1, (const uint4*)x3, (const uint4*)gh, rows, cols, slots_g1, slots_g3, n_slots,
                         (flags & MI8_FLAG_POW2_SCALE) != 0, (uint8_t*)out1, (uint8_t*)out3, ld_out, (uint8_t*)out1_t,
-                        (uint8_t*)out3_t, ld_t, scale_out1, scale_out3};
+                        (uint8_t*)out3_t, ld_t, scale_out1, scale_out3, t_end};
     const dim3 grid((unsigned)ceil_div(cols, kTile), (unsigned)ceil_div(rows, kTile));
     hipStream_t st = (hipStream_t)stream;
     const bool sw = flags & MI8_FLAG_SW_CVT;
@@ -1357,7 +1363,7 @@ extern "C" int mi8_cast_colwise_t(const void* x, int hp_dtype, int64_t rows, int
     int rc = launch_status("mi8_cast_colwise_t(amax)");
     if (rc != MI8_OK) return rc;
     TileCastArgs a{x, rows, cols, workspace, n_chunks, nullptr, (flags & MI8_FLAG_POW2_SCALE) != 0,
-                   nullptr, 0, (uint8_t*)out_t, ld_t, scale_out};
+                   nullptr, 0, (uint8_t*)out_t, ld_t, scale_out, round_up(rows, 16)};
     dispatch_tile_cast(hp_dtype, fp8_dtype, (flags & MI8_FLAG_SW_CVT) != 0, kPerColumnFromWorkspace, a, st);
     return launch_status("mi8_cast_colwise_t(cast)");
 }

@@ -43,16 +43,16 @@ def _(x2, weight, weight_scale, cfg, need_gx, need_gw, module_id):
     N = weight.shape[0]
     x_is_q, w_is_q = _saves_quantised(c, need_gx, need_gw)
 
-    def saved(is_q, rows, cols, cast):
+    def saved(is_q, rows, cols, cast, pad):
         if not is_q:
             return x2.new_empty(0), x2.new_empty(0)
         if _is_axiswise(cast):  # transposed copy padded to 128 rows, one scale per column
-            return (x2.new_empty((cols, (rows + 127) // 128 * 128), dtype=cast.target_dtype),
+            return (x2.new_empty((cols, ops.pad128(rows)), dtype=cast.target_dtype),
                     x2.new_empty(cols, dtype=torch.float32))
-        return x2.new_empty((cols, (rows + 15) // 16 * 16), dtype=cast.target_dtype), x2.new_empty(1, dtype=torch.float32)
+        return x2.new_empty((cols, pad(rows)), dtype=cast.target_dtype), x2.new_empty(1, dtype=torch.float32)
 
-    xa, xb = saved(x_is_q, M, K, c.cast_config_input)
-    wa, wb = saved(w_is_q, N, K, c.cast_config_weight)
+    xa, xb = saved(x_is_q, M, K, c.cast_config_input, ops.pad128)
+    wa, wb = saved(w_is_q, N, K, c.cast_config_weight, ops.pad16)
     return x2.new_empty((M, N)), xa, xb, wa, wb
 
 
@@ -141,18 +141,17 @@ def _(x, w1, w2, w3, cfg, need_x, need_w1, need_w2, need_w3, id1, id2, id3):
     H = w1.shape[0]
     any_grad = need_x or need_w1 or need_w2 or need_w3
     in_dt, w_dt = c.cast_config_input.target_dtype, c.cast_config_weight.target_dtype
-    pad16 = lambda n: (n + 15) // 16 * 16  # noqa: E731
     none = lambda: x.new_empty(0, dtype=torch.bfloat16)  # noqa: E731
     f32 = lambda: x.new_empty(1, dtype=torch.float32)  # noqa: E731
-    q_t = lambda rows, cols, dt, wanted: x.new_empty((cols, pad16(rows)), dtype=dt) if wanted else none()  # noqa: E731
+    q_t = lambda rows, cols, dt, wanted, pad=ops.pad16: x.new_empty((cols, pad(rows)), dtype=dt) if wanted else none()  # noqa: E731
     codes = none()
     if ff._fused_launch_ok(M, D, H) and ff._use_codes(M, D, H, any_grad):
         codes = x.new_empty(((H + 63) // 64) * M, dtype=torch.int16)
     bf16 = torch.bfloat16
     return [
         x.new_empty((M, w2.shape[0]), dtype=bf16),
-        q_t(M, D, in_dt, need_w1 or need_w3), f32(), x.new_empty((M, H), dtype=bf16), x.new_empty((M, H), dtype=bf16),
-        q_t(M, H, in_dt, need_w2), f32(),
+        q_t(M, D, in_dt, need_w1 or need_w3, ops.pad128), f32(), x.new_empty((M, H), dtype=bf16), x.new_empty((M, H), dtype=bf16),
+        q_t(M, H, in_dt, need_w2, ops.pad128), f32(),
         q_t(H, D, w_dt, need_x), f32(), q_t(w2.shape[0], H, w_dt, any_grad), f32(), q_t(H, D, w_dt, need_x), f32(),
         codes,
     ]

@@ -72,9 +72,10 @@ def _rows_operand(x: torch.Tensor, c: CastConfig, pow2: bool) -> Tuple[torch.Ten
 
 
 def _cols_operand(x: torch.Tensor, c: CastConfig, pow2: bool) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Operand whose K is x's first dim: transposed fp8 [cols, pad16(rows)] + scale [1] or [cols]."""
+    """Operand whose K is x's first dim: transposed fp8 [cols, rows padded with zeros] + scale [1] or [cols]."""
     if _is_tensorwise(c):
-        _, q_t, s = ops.cast_tensorwise(x, c.target_dtype, pow2=pow2, want_rowmajor=False, want_transposed=True)
+        _, q_t, s = ops.cast_tensorwise(x, c.target_dtype, pow2=pow2, want_rowmajor=False, want_transposed=True,
+                                       whole_steps=True)
         return q_t, s
     return ops.cast_colwise_t(x, c.target_dtype, pow2=pow2)
 
@@ -96,7 +97,8 @@ def _input_operands(x2, c: Float8LinearConfig, pow2: bool, share_x: bool):
     ci = c.cast_config_input
     x_saved = None
     if _is_tensorwise(ci):
-        xq, xq_t, sx = ops.cast_tensorwise(x2, ci.target_dtype, pow2=pow2, want_rowmajor=True, want_transposed=share_x)
+        xq, xq_t, sx = ops.cast_tensorwise(x2, ci.target_dtype, pow2=pow2, want_rowmajor=True, want_transposed=share_x,
+                                           whole_steps=True)
         if share_x:
             x_saved = (xq_t, sx)
     elif share_x:  # per-row copy for this GEMM, per-column transposed copy for grad_weight, one cast
@@ -157,7 +159,8 @@ def _backward_impl(go2, c: Float8LinearConfig, N: int, x_dtype, w_dtype, x_part,
     go_rows = go_cols = None
     cg, cgw = c.cast_config_grad_output, c.cast_config_grad_output_for_grad_weight
     if need_gx and need_gw and _shared_tensorwise(cg, cgw):
-        q, q_t, s = ops.cast_tensorwise(go2, cg.target_dtype, pow2=pow2, want_rowmajor=True, want_transposed=True)
+        q, q_t, s = ops.cast_tensorwise(go2, cg.target_dtype, pow2=pow2, want_rowmajor=True, want_transposed=True,
+                                        whole_steps=True)
         go_rows, go_cols = (q, s), (q_t, s)
     elif need_gx and need_gw and _shared_axiswise(cg, cgw):
         q, rs, q_t, cs = ops.cast_rows_and_colwise_t(go2, cg.target_dtype, pow2=pow2)

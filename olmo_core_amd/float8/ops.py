@@ -68,6 +68,10 @@ def pad16(n: int) -> int:
     return (n + 15) // 16 * 16
 
 
+def pad128(n: int) -> int:
+    return (n + 127) // 128 * 128
+
+
 def amax_partials(x: torch.Tensor) -> Tuple[torch.Tensor, int]:
     """Per-workgroup partial maxima of |x| (as float32 bit patterns); returns (slots, n_used)."""
     _require_gpu(x, "amax_partials")
@@ -172,11 +176,14 @@ def cast_tensorwise(
     scale: Optional[torch.Tensor] = None,
     pitch: Optional[int] = None,
     pitch_t: Optional[int] = None,
+    whole_steps: bool = False,
 ) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor], torch.Tensor]:
     """
     Quantise ``x [rows, cols]`` with one scale.  Returns ``(q, q_t, scale)``: ``q`` fp8 ``[rows, cols]``,
     ``q_t`` fp8 ``[cols, pad16(rows)]`` (zero padded), ``scale`` float32 ``[1]``.  The scale comes from
     ``scale`` if given, else from amax partials (``slots`` if already computed by a producer kernel).
+    ``whole_steps``: ``q_t`` is ``[cols, pad128(rows)]``, for a GEMM that contracts over the rows in steps of 128 whatever
+    their number (the persistent kernel takes no other).
     """
     x = _hp2d(x, "cast_tensorwise")
     rows, cols = x.shape
@@ -186,7 +193,7 @@ def cast_tensorwise(
     if scale is None and slots is None and not fused_amax:
         slots = amax_partials(x)
     q = _operand((rows, cols), fp8_dtype, dev, pitch) if want_rowmajor else None
-    q_t = _operand((cols, pad16(rows)), fp8_dtype, dev, pitch_t) if want_transposed else None
+    q_t = _operand((cols, (pad128 if whole_steps else pad16)(rows)), fp8_dtype, dev, pitch_t) if want_transposed else None
     scale_out = torch.empty(1, dtype=torch.float32, device=dev)
     if scale is not None:
         scale = scale.reshape(1).to(torch.float32)
@@ -196,7 +203,7 @@ def cast_tensorwise(
             slots[0].data_ptr() if slots is not None and scale is None else None,
             slots[1] if slots is not None and scale is None else 0,
             scale.data_ptr() if scale is not None else None,
-            _FP8_CODE[fp8_dtype], _flags(pow2),
+            _FP8_CODE[fp8_dtype], _flags(pow2) | (_C.FLAG_PAD_T128 if whole_steps else 0),
             q.data_ptr() if q is not None else None, q.stride(0) if q is not None else 0,
             q_t.data_ptr() if q_t is not None else None, q_t.stride(0) if q_t is not None else 0,
             scale_out.data_ptr(), _stream(x),
@@ -569,7 +576,7 @@ def swiglu_bwd_amax_from_codes(x1: torch.Tensor, x3: torch.Tensor, gh: torch.Ten
 
 def swiglu_bwd_cast(
     x1: torch.Tensor, x3: torch.Tensor, gh: torch.Tensor, fp8_dtype: torch.dtype, *, pow2: bool = False,
-    want_rowmajor: bool = True, want_transposed: bool = False, codes: Optional[tuple] = None,
+    want_rowmajor: bool = True, want_transposed: bool = False, codes: Optional[tuple] = None, whole_steps: bool = False,
 ):
     """
     ``swiglu_bwd`` followed by ``cast_tensorwise`` of both gradients, without ever writing them in bf16: a first
@@ -577,7 +584,7 @@ def swiglu_bwd_cast(
     ``(g1q, g1q_t, scale1, g3q, g3q_t, scale3)`` with the bytes and scales of the two-step route.
     ``codes`` = ``(gh_codes, x_codes)`` (from :func:`gemm_fp8_codes` / :func:`gemm_fp8_swiglu`, or
     :func:`rowseg_max_codes`): the amax is then found by computing only the row segments that can hold it, instead
-    of by the pass over all three tensors.
+    of by the pass over all three tensors.  ``whole_steps``: as for :func:`cast_tensorwise`.
     """
     _require_gpu(x1, "swiglu_bwd_cast")
     if not (x1.dtype == x3.dtype == gh.dtype == torch.bfloat16) or not (x1.shape == x3.shape == gh.shape) or x1.dim() != 2:
@@ -601,13 +608,13 @@ def swiglu_bwd_cast(
         )
         used = _C.lib().mi8_amax_slots_for(n)
     q = [_operand((rows, cols), fp8_dtype, dev) if want_rowmajor else None for _ in range(2)]
-    q_t = [_operand((cols, pad16(rows)), fp8_dtype, dev) if want_transposed else None for _ in range(2)]
+    q_t = [_operand((cols, (pad128 if whole_steps else pad16)(rows)), fp8_dtype, dev) if want_transposed else None for _ in range(2)]
     scales = [torch.empty(1, dtype=torch.float32, device=dev) for _ in range(2)]
     ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
     _C.check(
         _C.lib().mi8_swiglu_bwd_cast(
             x1.data_ptr(), x3.data_ptr(), gh.data_ptr(), rows, cols, s1.data_ptr(), s3.data_ptr(), used,
-            _FP8_CODE[fp8_dtype], _flags(pow2), ptr(q[0]), ptr(q[1]), q[0].stride(0) if want_rowmajor else 0,
+            _FP8_CODE[fp8_dtype], _flags(pow2) | (_C.FLAG_PAD_T128 if whole_steps else 0), ptr(q[0]), ptr(q[1]), q[0].stride(0) if want_rowmajor else 0,
             ptr(q_t[0]), ptr(q_t[1]), q_t[0].stride(0) if want_transposed else 0,
             scales[0].data_ptr(), scales[1].data_ptr(), _stream(x1),
         ),

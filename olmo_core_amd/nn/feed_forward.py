@@ -93,7 +93,7 @@ def _mlp_forward(x, w1, w2, w3, c, need, ws=(None, None, None), wo=(None, None, 
     if len(todo) > 1 and all(t.dtype == todo[0].dtype and t.is_contiguous() for t in todo):
         part = {id(t): p for t, p in zip(todo, ops.amax_partials_batch(todo))}
     xq, xq_t, sx = (x, None, None) if x_in_gemm else ops.cast_tensorwise(
-        x, in_dt, pow2=pow2, want_transposed=need[1] or need[3], slots=part.get(id(x)))
+        x, in_dt, pow2=pow2, want_transposed=need[1] or need[3], slots=part.get(id(x)), whole_steps=True)
     w1q, w1q_t, s1 = wo1 or ops.cast_tensorwise(w1, w_dt, pow2=pow2, want_transposed=need[0], scale=ws1,
                                                 slots=part.get(id(w1)))
     w3q, w3q_t, s3 = wo3 or ops.cast_tensorwise(w3, w_dt, pow2=pow2, want_transposed=need[0], scale=ws3,
@@ -118,7 +118,7 @@ def _mlp_forward(x, w1, w2, w3, c, need, ws=(None, None, None), wo=(None, None, 
         h, h_slots = ops.swiglu_fwd(x1, x3, want_amax=True)
     if STAGE_SINK is not None:
         STAGE_SINK.update(x1=x1.clone(), x3=x3.clone(), h=h.clone())
-    hq, hq_t, sh = ops.cast_tensorwise(h, in_dt, pow2=pow2, want_transposed=need[2], slots=h_slots)
+    hq, hq_t, sh = ops.cast_tensorwise(h, in_dt, pow2=pow2, want_transposed=need[2], slots=h_slots, whole_steps=True)
     if STAGE_SINK is not None:
         STAGE_SINK.update(sh=sh.clone(), hq=hq.clone())
     y = ops.gemm_fp8(hq, sh, w2q, s2, out_dtype=x.dtype)
@@ -143,7 +143,8 @@ def _mlp_backward(gy, saved, c, dims, dtypes, need):
     if gy.dtype != x_dt:
         gy = gy.to(x_dt)
     need_gh = need_x or need_w1 or need_w3
-    gyq, gyq_t, sgy = ops.cast_tensorwise(gy, go_dt, pow2=pow2, want_rowmajor=need_gh, want_transposed=need_w2)
+    gyq, gyq_t, sgy = ops.cast_tensorwise(gy, go_dt, pow2=pow2, want_rowmajor=need_gh, want_transposed=need_w2,
+                                           whole_steps=True)
     gw2 = ops.gemm_fp8(gyq_t, sgy, hq_t, sh, out_dtype=x_dt) if need_w2 else None
     gx = gw1 = gw3 = None
     if need_gh:
@@ -161,7 +162,7 @@ def _mlp_backward(gy, saved, c, dims, dtypes, need):
         need_t = need_w1 or need_w3
         # then the recompute-and-cast pass (no bf16 round trip of g1, g3)
         g1q, g1q_t, sg1, g3q, g3q_t, sg3 = ops.swiglu_bwd_cast(
-            x1, x3, gh, go_dt, pow2=pow2, want_rowmajor=need_x, want_transposed=need_t, codes=codes)
+            x1, x3, gh, go_dt, pow2=pow2, want_rowmajor=need_x, want_transposed=need_t, codes=codes, whole_steps=True)
         del gh
         if STAGE_SINK is not None:
             STAGE_SINK.update(sg1=sg1.clone(), sg3=sg3.clone(), amax_from_codes=codes is not None,

@@ -318,3 +318,22 @@ def test_argument_errors(dev):
         ops.cast_tensorwise(torch.zeros(4, 16, dtype=torch.bfloat16), E4M3)  # CPU tensor: no CPU path
     with pytest.raises(TypeError):
         ops.cast_rowwise(torch.zeros(4, 16, dtype=torch.float16, device=dev), E4M3)
+
+
+@pytest.mark.parametrize("rows", [1, 112, 127, 128, 129, 1999])
+def test_transposed_copy_in_whole_steps(dev, rows):
+    """whole_steps pads the transposed copy with zeros to a multiple of 128 rows (pad16(rows) without)."""
+    x = seeded((rows, 144), rows).to(dev)
+    _, want, _ = ops.cast_tensorwise(x, E4M3, want_transposed=True)
+    # freed memory of another content, so that an unwritten tail shows
+    torch.full((144, ops.pad128(rows)), 0x55, dtype=torch.uint8, device=dev)
+    _, q_t, _ = ops.cast_tensorwise(x, E4M3, want_transposed=True, whole_steps=True)
+    assert q_t.shape == (144, ops.pad128(rows))
+    assert torch.equal(u8(q_t)[:, :rows], u8(want)[:, :rows]) and not u8(q_t)[:, rows:].any()
+    x1, x3, gh = (seeded((rows, 144), s).to(dev) for s in (1, 2, 3))
+    a = ops.swiglu_bwd_cast(x1, x3, gh, E5M2, want_transposed=True)
+    torch.full((144, ops.pad128(rows)), 0x55, dtype=torch.uint8, device=dev)
+    b = ops.swiglu_bwd_cast(x1, x3, gh, E5M2, want_transposed=True, whole_steps=True)
+    for i in (1, 4):
+        assert b[i].shape == (144, ops.pad128(rows))
+        assert torch.equal(u8(a[i])[:, :rows], u8(b[i])[:, :rows]) and not u8(b[i])[:, rows:].any()
