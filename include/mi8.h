@@ -145,6 +145,15 @@ int mi8_cast_tensorwise_static(const void* x, int hp_dtype, int64_t rows, int64_
 int mi8_cast_rowwise(const void* x, int hp_dtype, int64_t rows, int64_t cols, int fp8_dtype, uint32_t flags,
                      void* out, int64_t ld_out, float* scale_out, void* stream);
 
+/* The two per-row casts of an expert layer that is not differentiated, bf16 to e4m3, with the bytes and scales of the
+ * separate steps.  gather_cast_rows: row r of out [tokens * top_k, ld_out] is row indices[r] / top_k of x
+ * [tokens, cols] (an index outside [0, tokens * top_k): a row of zeros).  swiglu_cast_rows: rows of silu(x1) * x3,
+ * rounded to bf16 first.  Same limits as mi8_cast_rowwise. */
+int mi8_moe_gather_cast_rows(const void* x, int64_t tokens, int64_t cols, const int32_t* indices, int32_t top_k,
+                             uint32_t flags, void* out, int64_t ld_out, float* scale_out, void* stream);
+int mi8_swiglu_cast_rows(const void* x1, const void* x3, int64_t rows, int64_t cols, uint32_t flags, void* out,
+                         int64_t ld_out, float* scale_out, void* stream);
+
 /* Number of uint32 a column-amax workspace needs for a [rows, cols] input. */
 int64_t mi8_colamax_workspace_slots(int64_t rows, int64_t cols);
 

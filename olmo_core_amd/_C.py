@@ -52,6 +52,14 @@ _SIGNATURES = {
         c_int,
         [c_void_p, c_int, c_int64, c_int64, c_int, c_uint32, c_void_p, c_int64, c_void_p, c_void_p],
     ),
+    "mi8_moe_gather_cast_rows": (
+        c_int,
+        [c_void_p, c_int64, c_int64, c_void_p, c_int32, c_uint32, c_void_p, c_int64, c_void_p, c_void_p],
+    ),
+    "mi8_swiglu_cast_rows": (
+        c_int,
+        [c_void_p, c_void_p, c_int64, c_int64, c_uint32, c_void_p, c_int64, c_void_p, c_void_p],
+    ),
     "mi8_colamax_workspace_slots": (c_int64, [c_int64, c_int64]),
     "mi8_cast_colwise_t": (
         c_int,

@@ -793,6 +793,45 @@ def gather_cast_rows_and_colwise_t(
     return q, row_scale, q_t, scale
 
 
+def gather_cast_rows(x: torch.Tensor, indices: torch.Tensor, top_k: int, *, pow2: bool = False):
+    """The row-major product of :func:`gather_cast_rows_and_colwise_t` alone, in one pass (bf16 to e4m3):
+    ``(q [tokens * top_k, cols], scale)``."""
+    x = _hp2d(x, "gather_cast_rows")
+    tokens, cols = x.shape
+    T = tokens * top_k
+    if x.dtype != torch.bfloat16:
+        raise TypeError(f"gather_cast_rows: expected bfloat16, got {x.dtype}")
+    if indices.dim() != 1 or indices.shape[0] != T or indices.device != x.device:
+        raise ValueError(f"gather_cast_rows: expected {T} indices on {x.device}")
+    if indices.dtype != torch.int32 or not indices.is_contiguous():
+        indices = indices.to(torch.int32).contiguous()
+    q = torch.empty((T, cols), dtype=torch.float8_e4m3fn, device=x.device)
+    s = torch.empty(T, dtype=torch.float32, device=x.device)
+    _C.check(
+        _C.lib().mi8_moe_gather_cast_rows(x.data_ptr(), tokens, cols, indices.data_ptr(), top_k, _flags(pow2), q.data_ptr(),
+                                          cols, s.data_ptr(), _stream(x)),
+        "mi8_moe_gather_cast_rows",
+    )
+    return q, s
+
+
+def swiglu_cast_rows(x1: torch.Tensor, x3: torch.Tensor, *, pow2: bool = False):
+    """``cast_rowwise(silu(x1) * x3, e4m3)`` in one pass over bf16 ``x1``, ``x3`` ``[rows, cols]``: ``(q, scale)``."""
+    _require_gpu(x1, "swiglu_cast_rows")
+    if not (x1.dtype == x3.dtype == torch.bfloat16) or x1.dim() != 2 or x1.shape != x3.shape or x3.device != x1.device:
+        raise ValueError("swiglu_cast_rows: expects two bfloat16 matrices of one shape")
+    x1, x3 = x1.contiguous(), x3.contiguous()
+    rows, cols = x1.shape
+    q = torch.empty((rows, cols), dtype=torch.float8_e4m3fn, device=x1.device)
+    s = torch.empty(rows, dtype=torch.float32, device=x1.device)
+    _C.check(
+        _C.lib().mi8_swiglu_cast_rows(x1.data_ptr(), x3.data_ptr(), rows, cols, _flags(pow2), q.data_ptr(), cols,
+                                      s.data_ptr(), _stream(x1)),
+        "mi8_swiglu_cast_rows",
+    )
+    return q, s
+
+
 _ONE_GROUP: dict = {}
 
 

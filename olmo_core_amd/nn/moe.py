@@ -19,6 +19,7 @@ import torch
 import torch.nn as nn
 
 from ..float8 import ops
+from ..float8.linear import needs_autograd
 
 __all__ = ["DroplessMoEMLP", "float8_dropless_mlp"]
 
@@ -197,6 +198,34 @@ class _Float8DroplessMLP(torch.autograd.Function):
                 g_router)
 
 
+def _forward_only(x, w1, w2, w3, sizes, E, pow2, indices, top_k, kept, scatter_weights):
+    """The forward of :class:`_Float8DroplessMLP` where nothing is differentiated: no transposed float8 copies of the
+    activations, nothing kept."""
+    D, H = x.shape[1], w1.shape[0] // E
+    if indices is not None:
+        xq, sx = ops.gather_cast_rows(x, indices, top_k, pow2=pow2)
+    else:
+        xq, sx = ops.cast_rowwise(x, _E4M3, pow2=pow2)
+    if kept is not None:
+        (w1q, s1, _, _), (w3q, s3, _, _), (_, _, w2t, s2) = kept
+    else:
+        w1q, s1 = ops.cast_rowwise(w1, _E4M3, pow2=pow2)
+        w3q, s3 = ops.cast_rowwise(w3, _E4M3, pow2=pow2)
+        equal = torch.full((E,), H, dtype=torch.int64, device=x.device)
+        w2t, s2 = ops.grouped_cast_colwise_t(w2, equal, _E4M3, pow2=pow2)
+    x1 = ops.grouped_gemm_fp8(xq, sx, w1q, s1, sizes, n=H, k=D, b_group_stride=H * w1q.stride(0), sb_group_stride=H)
+    x2 = ops.grouped_gemm_fp8(xq, sx, w3q, s3, sizes, n=H, k=D, b_group_stride=H * w3q.stride(0), sb_group_stride=H)
+    hq, sh = ops.swiglu_cast_rows(x1, x2, pow2=pow2)
+    y = ops.grouped_gemm_fp8(hq, sh, w2t, s2, sizes, n=D, k=H, b_group_stride=(H + 127) // 128 * 128, sb_group_stride=D)
+    if scatter_weights is not None:
+        from ..ops import moe as moe_ops
+
+        if indices is None:
+            raise ValueError("scatter_weights needs the permutation (indices)")
+        y = moe_ops._scatter(y, indices, scatter_weights, top_k)
+    return y
+
+
 @torch.compiler.disable
 def float8_dropless_mlp(x, w1, w2, w3, batch_size_per_expert, num_experts: int, pow2: bool = True, indices=None,
                         top_k: int = 1, kept=None, scatter_weights=None):
@@ -206,6 +235,10 @@ def float8_dropless_mlp(x, w1, w2, w3, batch_size_per_expert, num_experts: int, 
     ``[tokens * top_k, d_model]``, and the gather never writes its bf16 result.  With ``scatter_weights`` (one router
     weight per slot) the weighted scatter back to token order happens here as well (result ``[tokens, d_model]``), and
     the backward quantises the weighted gather of the incoming gradient without writing it in bf16 either."""
+    differentiable = (x, w1, w2, w3) if scatter_weights is None else (x, w1, w2, w3, scatter_weights)
+    if (STAGE_SINK is None and x.dtype == torch.bfloat16 and x.numel() and max(x.shape[1], w1.shape[0] // num_experts) <= 65536
+            and not needs_autograd(*differentiable)):  # (the per-row casts hold a row of at most 65536 in registers)
+        return _forward_only(x, w1, w2, w3, batch_size_per_expert, num_experts, pow2, indices, top_k, kept, scatter_weights)
     return _Float8DroplessMLP.apply(x, w1, w2, w3, batch_size_per_expert, num_experts, pow2, indices, top_k, kept,
                                     scatter_weights)
 

@@ -190,3 +190,53 @@ def test_gather_fused_with_the_grouped_cast(dev, sl, hs, ne, top_k, pow2):
     assert int(u8(qb[0]).max()) == 0
     assert_scale_equal(srb[0:1], O.amax_to_scale(torch.zeros(1, 1, dtype=torch.bfloat16), E4M3, pow2))
     assert torch.equal(u8(qb[1:]), u8(q[1:]))
+
+
+@pytest.mark.parametrize("tokens,cols,top_k", [(1, 16, 1), (5, 1040, 3), (67, 2064, 2), (3, 4112, 8), (2, 8208, 4), (3, 65536, 1)],
+                         ids=lambda v: str(v))
+@pytest.mark.parametrize("pow2", [True, False], ids=["pow2", ""])
+def test_row_casts_of_an_undifferentiated_expert_layer(dev, tokens, cols, top_k, pow2):
+    """gather -> per-row cast and SwiGLU -> per-row cast in one pass each: bytes and scales of the separate steps, at
+    row lengths on either side of each kernel variant; a dropped token reads as zeros, NaN and inf reach their row alone."""
+    from helpers import E4M3, u8
+    from olmo_core_amd.float8 import ops as f8
+
+    g = torch.Generator().manual_seed(cols + tokens)
+    x = torch.randn(tokens, cols, generator=g).bfloat16()
+    if tokens > 1:
+        x[0, 3], x[1, 5] = float("nan"), float("inf")
+    indices = torch.randperm(tokens * top_k, generator=g).int()
+    indices[-1] = -1
+    q, s = f8.gather_cast_rows(x.to(dev), indices.to(dev), top_k, pow2=pow2)
+    rows = x.repeat_interleave(top_k, 0)[indices.long()]
+    rows[-1] = 0
+    q2, s2 = f8.cast_rowwise(rows.to(dev), E4M3, pow2=pow2)
+    assert torch.equal(u8(q), u8(q2)) and torch.equal(s.view(torch.int32), s2.view(torch.int32))
+
+    x3 = torch.randn(tokens, cols, generator=g).bfloat16().to(dev)
+    h, _ = f8.swiglu_fwd(x.to(dev), x3, want_amax=False)
+    q, s = f8.swiglu_cast_rows(x.to(dev), x3, pow2=pow2)
+    q2, s2 = f8.cast_rowwise(h, E4M3, pow2=pow2)
+    assert torch.equal(u8(q), u8(q2)) and torch.equal(s.view(torch.int32), s2.view(torch.int32))
+
+
+@pytest.mark.parametrize("keep", [False, True], ids=["", "kept"])
+@pytest.mark.parametrize("tokens", [1, 48, 333])
+def test_routed_layer_without_gradients_has_the_same_bits(dev, tokens, keep):
+    from olmo_core_amd.nn import DroplessMoEMLP, ParallelDroplessMLP
+
+    d, h, ne, top_k = 256, 144, 8, 2
+    g = torch.Generator().manual_seed(tokens)
+    mlp = DroplessMoEMLP(d_model=d, hidden_size=h, num_experts=ne, dtype=torch.bfloat16, init_device="cuda",
+                         keep_float8_weights=keep)
+    layer = ParallelDroplessMLP(mlp=mlp, top_k=top_k)
+    x = torch.randn(tokens, d, generator=g).bfloat16().to(dev)
+    # expert 3 gets no token
+    idx = torch.rand(tokens, ne, generator=g).index_fill(1, torch.tensor([3]), -1.0).topk(top_k, dim=-1).indices.to(dev)
+    sizes = torch.bincount(idx.flatten(), minlength=ne)
+    w = torch.rand(tokens, top_k, generator=g).bfloat16().to(dev)
+    want = layer(x, w, idx, sizes)
+    assert want.requires_grad
+    with torch.no_grad():
+        got = layer(x, w, idx, sizes)
+    assert torch.equal(got, want.detach())
