@@ -118,13 +118,38 @@ int launch_grouped(GroupedArgs& a, hipStream_t st)
     return launch_status("mi8_grouped_gemm_fp8");
 }
 
-// tile height by the rows a group has on average: what lies below a group's last row is work for nothing
-template <int CBSZ, int BLGP>
-int launch_grouped_shape(GroupedArgs& a, hipStream_t st)
+// Which kernel a grouped product runs on, by estimated microseconds.  The sizes of the groups are on the device; with
+// popularity as skewed as routers make it, T rows in E groups fill about T / BM + E / 2 tiles of BM rows.  Measured, with
+// s = K / 128 steps: the persistent kernel has 256 workgroups and takes 3.3 + 1.1 s a round, a ring tile 32, 64 or 128 rows
+// high 3.4 + 0.53 s, 2 + s or 3 + 1.38 s for 512 of them, half of that where each has a compute unit to itself; any launch
+// 5 more.  64 groups, N 1024, K 2048 (us: persistent, rings of 32, 64 and 128 rows), T = 384: 26, 13.5, 13.5, 17.5;
+// 2048: 27, 29, 22, 23; 4096: 29, 46, 38, 30; 8 groups, N 1024, K 1792, T = 1024: 22, 12, 11.5, 15; 4096: 23, 30, 25, 20;
+// 8192: 24, 50, 39, 37.  The lines lie where the estimates cross.  All four give the same bits.
+enum GroupedKernel { kRing32, kRing64, kRing128, kPersistent };
+
+GroupedKernel choose_grouped(int64_t T, int64_t E, int64_t N, int64_t K, bool persistent_fits)
 {
-    const int64_t rows = a.T / a.E;
-    if (rows <= 24) return launch_grouped<32, 128, 4, CBSZ, BLGP>(a, st);
-    if (rows <= 128) return launch_grouped<64, 128, 3, CBSZ, BLGP>(a, st);
+    const double steps = (double)ceil_div(K, 128), columns = (double)ceil_div(N, 128);
+    const double rows = (double)T, partial = 0.5 * (double)(E < T ? E : T);
+    const auto ring = [&](double round, int bm) {
+        const double blocks = (rows / bm + partial) * columns / 512;
+        return round * (blocks > 0.5 ? blocks : 0.5);
+    };
+    const double cost[4] = {ring(3.4 + 0.53 * steps, 32), ring(2.0 + steps, 64), ring(3.0 + 1.38 * steps, 128), [&] {
+                                const double tiles = (rows / 256 + partial) * (double)ceil_div(N, 256) / 256;
+                                return (3.3 + 1.1 * steps) * (tiles > 1 ? tiles : 1);
+                            }()};
+    int best = kRing32;
+    for (int k = kRing64; k <= (persistent_fits ? kPersistent : kRing128); ++k)
+        if (cost[k] < cost[best]) best = k;
+    return (GroupedKernel)best;
+}
+
+template <int CBSZ, int BLGP>
+int launch_grouped_shape(GroupedArgs& a, GroupedKernel k, hipStream_t st)
+{
+    if (k == kRing32) return launch_grouped<32, 128, 4, CBSZ, BLGP>(a, st);
+    if (k == kRing64) return launch_grouped<64, 128, 3, CBSZ, BLGP>(a, st);
     return launch_grouped<128, 128, 2, CBSZ, BLGP>(a, st);
 }
 
@@ -179,17 +204,19 @@ int grouped_gemm_entry(const void* a, int a_dtype, int64_t lda, const void* b, i
                   b_group_stride, sb_group_stride, group_sizes, num_groups, T, (int)N, (int)K, sa, sb, 0,
                   accumulate ? 1 : 0};
     hipStream_t st = (hipStream_t)stream;
-    // full-tile shapes with bf16 output run on the persistent direct-to-LDS kernel (which rewrites the overlap of its
-    // shifted last tile column when N is not a multiple of 256: not possible when accumulating)
-    if (out_dtype == MI8_BF16 && T >= 256 && N >= 256 && K % 128 == 0 && N % 8 == 0 && ldc % 8 == 0 && aligned16(out) &&
+    // the persistent kernel takes full-tile shapes with bf16 output (it rewrites the overlap of its shifted last tile
+    // column when N is not a multiple of 256: not possible when accumulating)
+    const bool fits = out_dtype == MI8_BF16 && T >= 256 && N >= 256 && K % 128 == 0 && N % 8 == 0 && ldc % 8 == 0 && aligned16(out) &&
         sb_group_stride % 4 == 0 && aligned16(sb) && lda < (1 << 23) && ldb < (1 << 23) && ldc < (1 << 22) &&
-        (!accumulate || N % 256 == 0))
+        (!accumulate || N % 256 == 0);
+    const GroupedKernel k = choose_grouped(T, num_groups, N, K, fits);
+    if (k == kPersistent)
         return launch_m16_grouped((const uint8_t*)a, a_dtype, lda, (const uint8_t*)b, b_dtype, ldb, b_group_stride,
                                    group_sizes, num_groups, T, (int)N, (int)K, sa, sb, sb_group_stride, (uint16_t*)out,
                                    ldc, accumulate, st);
     if (a_dtype == MI8_E4M3)
-        return b_dtype == MI8_E4M3 ? launch_grouped_shape<0, 0>(g, st) : launch_grouped_shape<0, 1>(g, st);
-    return b_dtype == MI8_E4M3 ? launch_grouped_shape<1, 0>(g, st) : launch_grouped_shape<1, 1>(g, st);
+        return b_dtype == MI8_E4M3 ? launch_grouped_shape<0, 0>(g, k, st) : launch_grouped_shape<0, 1>(g, k, st);
+    return b_dtype == MI8_E4M3 ? launch_grouped_shape<1, 0>(g, k, st) : launch_grouped_shape<1, 1>(g, k, st);
 }
 }  // namespace
 

@@ -517,3 +517,36 @@ def test_grouped_dual_gemm_against_separate_products(dev, sizes):
             b = wt[:, e * k:(e + 1) * k].float().double().cpu() / sc[e][:, None].double().cpu()
             ref = ref + a @ b.t()
         assert_gemm_close(got[s:s + m], ref, f"group {e}")
+
+
+@pytest.mark.parametrize("accumulate", [False, True], ids=["", "accumulate"])
+@pytest.mark.parametrize("sizes,n,k", [
+    ([3, 0, 31, 1, 33, 0, 64, 32] * 6, 1024, 1024),   # tiles of 32 rows
+    ([64, 65, 0, 700, 63, 1] * 2, 512, 1792),         # of 64 rows
+    ([130, 0, 2900, 1000], 1024, 1792),               # of 128 rows
+    ([300, 0, 17, 20000, 9700], 320, 384),            # the persistent kernel, its last tile column shifted
+    ([7000, 255, 0, 257, 9000], 1024, 1024),          # the persistent kernel
+    ([40, 0, 301], 264, 144),                         # no multiple of a step
+], ids=["32", "64", "128", "persistent-shifted", "persistent", "ragged-k"])
+def test_grouped_gemm_choice_exact_integers(dev, sizes, n, k, accumulate):
+    """Integer operands and power-of-two scales: the product is exact in float32 whichever kernel the sizes lead to, so
+    the result is its bf16 rounding (accumulating: the bf16 sum of that and the old value), and rows of no group stay."""
+    E, T = len(sizes), sum(sizes)
+    g = torch.Generator(device="cuda").manual_seed(T + n)
+    a = torch.randint(-4, 5, (T, k), generator=g, device=dev).float()
+    b = torch.randint(-4, 5, (E * n, k), generator=g, device=dev).float()
+    sa = torch.exp2(torch.randint(-3, 4, (T,), generator=g, device=dev).float())
+    sb = torch.exp2(torch.randint(-3, 4, (E, n), generator=g, device=dev).float())
+    old = torch.randint(-64, 65, (T, n), generator=g, device=dev).bfloat16()
+    got = old.clone() if accumulate else None
+    out = ops.grouped_gemm_fp8(a.to(E4M3), sa, b.to(E4M3), sb, torch.tensor(sizes), n=n, k=k, b_group_stride=n * k,
+                               sb_group_stride=n, **({"accumulate_into": got} if accumulate else {}))
+    start = 0
+    for e, m in enumerate(sizes):
+        rows = slice(start, start + m)
+        if m:
+            want = (a[rows] @ b[e * n:(e + 1) * n].t() / sa[rows, None] / sb[e]).bfloat16()
+            if accumulate:
+                want = old[rows] + want
+            assert torch.equal(out[rows], want), f"group {e}"
+        start += m
