@@ -398,6 +398,12 @@ int mi8_gemm_fp8_codes(const void* a, int a_dtype, int64_t lda, const void* b, i
  * aligned, element by element otherwise.  An index outside [0, tokens * top_k) is treated as a dropped token.
  * ------------------------------------------------------------------------------------------- */
 
+/* indices [n]: the slots 0..n-1 stably sorted by expert id (ids: int32 or int64 [n], taken modulo 2^32); bin_ids [n]:
+ * their ids; bins [experts]: inclusive prefix sums of sizes.  n up to mi8_moe_sort_slots_max(). */
+int64_t mi8_moe_sort_slots_max(void);
+int mi8_moe_sort_slots(const void* ids, int ids_are_64, int64_t n, const int64_t* sizes, int32_t experts, int32_t* indices,
+                       int32_t* bin_ids, int32_t* bins, void* stream);
+
 /* out[i, :] = x[indices[i] / top_k, :] * weights[indices[i]]           out: [tokens * top_k, hidden] */
 int mi8_moe_gather(const void* x, int dtype, int64_t tokens, int64_t hidden, const int32_t* indices,
                    const void* weights, int w_dtype, int32_t top_k, void* out, void* stream);

@@ -52,6 +52,11 @@ _SIGNATURES = {
         c_int,
         [c_void_p, c_int, c_int64, c_int64, c_int, c_uint32, c_void_p, c_int64, c_void_p, c_void_p],
     ),
+    "mi8_moe_sort_slots_max": (c_int64, []),
+    "mi8_moe_sort_slots": (
+        c_int,
+        [c_void_p, c_int, c_int64, c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_void_p],
+    ),
     "mi8_moe_gather_cast_rows": (
         c_int,
         [c_void_p, c_int64, c_int64, c_void_p, c_int32, c_uint32, c_void_p, c_int64, c_void_p, c_void_p],

@@ -411,10 +411,86 @@ int launch_wgrad(PermuteArgs& a, int dtype, int64_t rows, hipStream_t st)
     return launch_status(BINNED ? "mi8_moe_binned_scatter_wgrad" : "mi8_moe_scatter_wgrad");
 }
 
+// ---- slots sorted by expert -----------------------------------------------------------------------------
+// Stable sort of up to kSortSlots expert ids in one launch: the place of slot e is the number of slots before it that
+// have its id or a smaller one, plus the number of slots after it with a smaller one.  A workgroup places 64 slots, one
+// per lane; its 16 waves count over a sixteenth of the ids each (wave-uniform, so scalar loads and two vector
+// instructions an id).  A call with few tokens is a chain of short launches: the conversion, sort, prefix sum and their
+// copies were eleven of them.  Counting is n^2, so larger inputs stay with the radix sort.  us on the device, this and the
+// chain it replaces: 384 slots 3.6 / 27, 2048 7.4 / 30, 8192 15.8 / 37.
+constexpr int kSortThreads = 1024;
+constexpr int64_t kSortSlots = 8192;
+
+template <typename ID>
+__global__ __launch_bounds__(kSortThreads) void sort_slots_kernel(const ID* __restrict__ ids, int n,
+                                                                  const int64_t* __restrict__ sizes, int experts,
+                                                                  int32_t* __restrict__ indices, int32_t* __restrict__ bin_ids,
+                                                                  int32_t* __restrict__ bins)
+{
+    __shared__ int32_t part[kSortThreads / 64][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int first = (int)blockIdx.x * 64, e = first + lane;
+    const int32_t id = e < n ? (int32_t)ids[e] : 0;
+    const int per = (n + kSortThreads / 64 - 1) / (kSortThreads / 64);
+    const int lo = per * wave < n ? per * wave : n, hi = lo + per < n ? lo + per : n;
+    int32_t before = 0;
+    int j = lo;
+    const int end_before = hi < first ? hi : first;
+#pragma unroll 8
+    for (; j < end_before; ++j) before += (int32_t)ids[j] <= id ? 1 : 0;
+    const int end_own = hi < first + 64 ? hi : first + 64;
+    for (; j < end_own; ++j) {
+        const int32_t other = (int32_t)ids[j];
+        before += other < id || (other == id && j < e) ? 1 : 0;
+    }
+#pragma unroll 8
+    for (; j < hi; ++j) before += (int32_t)ids[j] < id ? 1 : 0;
+    part[wave][lane] = before;
+    __syncthreads();
+    if (wave == 0 && e < n) {
+        int32_t at = 0;
+#pragma unroll
+        for (int w = 0; w < kSortThreads / 64; ++w) at += part[w][lane];
+        indices[at] = e;
+        bin_ids[at] = id;
+    }
+    if (wave == 1 && blockIdx.x == 0) {  // the inclusive prefix sums of the experts' counts
+        int64_t sum = 0;
+        for (int base = 0; base < experts; base += 64) {
+            int64_t v = base + lane < experts ? sizes[base + lane] : 0;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int64_t o = __shfl_up(v, d, 64);
+                if (lane >= d) v += o;
+            }
+            if (base + lane < experts) bins[base + lane] = (int32_t)(sum + v);
+            sum += __shfl(v, 63, 64);
+        }
+    }
+}
+
 }  // namespace
 }  // namespace mi8
 
 using namespace mi8;
+
+extern "C" int64_t mi8_moe_sort_slots_max(void) { return kSortSlots; }
+
+extern "C" int mi8_moe_sort_slots(const void* ids, int ids_are_64, int64_t n, const int64_t* sizes, int32_t experts,
+                                  int32_t* indices, int32_t* bin_ids, int32_t* bins, void* stream)
+{
+    MI8_REQUIRE(ids && sizes && indices && bin_ids && bins, MI8_ERR_ARG, "mi8_moe_sort_slots: null pointer");
+    MI8_REQUIRE(n > 0 && n <= kSortSlots && experts > 0, MI8_ERR_UNSUPPORTED,
+                "mi8_moe_sort_slots: needs 1..%lld slots and an expert (got %lld, %d)", (long long)kSortSlots, (long long)n, experts);
+    const dim3 grid((unsigned)ceil_div(n, 64));
+    if (ids_are_64)
+        hipLaunchKernelGGL(sort_slots_kernel<int64_t>, grid, dim3(kSortThreads), 0, (hipStream_t)stream, (const int64_t*)ids,
+                           (int)n, sizes, experts, indices, bin_ids, bins);
+    else
+        hipLaunchKernelGGL(sort_slots_kernel<int32_t>, grid, dim3(kSortThreads), 0, (hipStream_t)stream, (const int32_t*)ids,
+                           (int)n, sizes, experts, indices, bin_ids, bins);
+    return launch_status("mi8_moe_sort_slots");
+}
 
 extern "C" int mi8_moe_gather(const void* x, int dtype, int64_t tokens, int64_t hidden, const int32_t* indices,
                               const void* weights, int w_dtype, int32_t top_k, void* out, void* stream)

@@ -364,9 +364,9 @@ class ParallelDroplessMLP(nn.Module):
     def indices_and_bins(self, expert_indices: torch.Tensor, batch_size_per_expert: torch.Tensor):
         """``(indices, bin_ids, bins)``: argsort of the flattened expert assignment, the sorted expert ids and
         the inclusive prefix sums of the per-expert counts (all int32)."""
-        bin_ids, indices = torch.sort(expert_indices.int())
-        bins = torch.cumsum(batch_size_per_expert, 0).to(torch.int32)
-        return indices.int(), bin_ids, bins
+        from ..ops import moe as moe_ops
+
+        return moe_ops._sort_slots(expert_indices, batch_size_per_expert)
 
     def forward(self, x, expert_weights, expert_indices, batch_size_per_expert):
         """

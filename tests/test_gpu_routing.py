@@ -74,3 +74,20 @@ def test_config5_group_sizes(dev):
     hist = moe_ops.histc(assign.reshape(-1).to(dev), 64).cpu()
     assert int(hist.sum()) == 131072 and int((hist == 0).sum()) == 7 and int((hist == 1).sum()) >= 1
     assert torch.equal(hist, O.batched_histc(assign.reshape(1, -1), 64)[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64], ids=str)
+@pytest.mark.parametrize("n,experts", [(1, 1), (63, 3), (64, 64), (65, 5), (384, 64), (1023, 130), (8192, 64), (8193, 64)], ids=str)
+def test_sorted_slots_equal_a_stable_sort(dev, n, experts, dtype):
+    """Sizes around a workgroup's 64 slots, the sixteenth of the ids a wave counts, and the last size of the one-launch sort;
+    ids outside the experts' range keep their place in the order."""
+    g = torch.Generator().manual_seed(n)
+    ids = torch.randint(0, experts, (n,), generator=g)
+    if n > 64:
+        ids[5], ids[n // 2], ids[n - 1] = -3, experts + 7, torch.iinfo(torch.int32).max
+    sizes = torch.randint(0, 1000, (experts,), generator=g)
+    indices, bin_ids, bins = moe_ops._sort_slots(ids.to(dtype).to(dev), sizes.to(dev))
+    want_ids, want = torch.sort(ids, stable=True)
+    assert indices.dtype == bin_ids.dtype == bins.dtype == torch.int32
+    assert torch.equal(indices.cpu().long(), want) and torch.equal(bin_ids.cpu().long(), want_ids)
+    assert torch.equal(bins.cpu().long(), sizes.cumsum(0))
