@@ -42,8 +42,8 @@ int mi8_probe_mfma_feed(int kind, int loads, int reads, int barriers, int random
 int mi8_probe_store_rate(int rows, int waves, int workgroups, int iterations, void* window, int64_t pitch, uint32_t* cycles,
                          void* stream);
 /* One launch of the library's persistent fp8 GEMM (the kernel of mi8_gemm_fp8 for M, N >= 256, K % 128 == 0, N % 8 == 0,
- * single scales, bf16 output, contiguous operands) built with time stamps: wave 0 of workgroup w writes into
- * stamps[256 * w ..], for each of its first 16 tiles t, the low 32 bits of the shader clock at 13 points -
+ * single scales, bf16 output, contiguous operands) built with time stamps: wave 0 of workgroup w < 256 that walks whole
+ * tiles (a plan may hand others one half tile each: these record nothing) writes into stamps[256 * w ..], for each of its first 16 tiles t, the low 32 bits of the shader clock at 13 points -
  * [13 t + 0] K loop start, [+1] after three K steps, [+2] epilogue start, [+3 .. +10] the eight epilogue passes (each
  * after its staging writes have landed), [+11] last store issued, [+12] tile end (unused entries stay 0) - and in
  * [254], [255] the constant 100 MHz clock at kernel start and end.  stamps: uint32 [256 * 256] of device memory.

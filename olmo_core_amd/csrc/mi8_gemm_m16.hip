@@ -44,12 +44,15 @@ static_assert(3 * (BM / 2 + BN) * BK <= 2 * STAGE + OUT_STAGING, "the three stag
 // Tile timeline (only in the diagnostics library, which compiles this file with -DMI8_TILE_TIMELINE): wave 0 of every
 // workgroup records the shader clock at fixed points of each of its tiles - K loop start, after three K steps, epilogue
 // start, every epilogue pass, last store issued, tile end - in 1 KB of LDS of its own and copies them out when the
-// kernel ends.  A stamp costs one s_memtime and its wait (placed where nothing else the wave waits for is in flight).
+// kernel ends.  Only the first TIMELINE_WORKGROUPS workgroups with whole tiles do (a grid has up to as many again with a
+// half tile each, which has other passes).  A stamp costs one s_memtime and its wait (placed where nothing else the wave
+// waits for is in flight).
 #ifdef MI8_TILE_TIMELINE
 constexpr int TIMELINE_BYTES = 1024;
 constexpr int TIMELINE_STAMPS = 13;          // per tile
 constexpr int TIMELINE_TILES = 16;           // tiles recorded per workgroup (later tiles overwrite the last record)
-__device__ uint32_t* g_timeline = nullptr;   // [workgroups][256]: TIMELINE_TILES x TIMELINE_STAMPS, [254], [255]: 100 MHz clock at start / end
+constexpr int TIMELINE_WORKGROUPS = 256;     // what the buffer of mi8_diag_gemm_tile_timeline has room for
+__device__ uint32_t* g_timeline = nullptr;   // [TIMELINE_WORKGROUPS][256]: TIMELINE_TILES x TIMELINE_STAMPS, [254], [255]: 100 MHz clock at start / end
 #define MI8_TL(k) tl_stamp(k)
 #define MI8_TL_NEXT_TILE() (tl_ev += tl_ev < TIMELINE_STAMPS * (TIMELINE_TILES - 1) ? TIMELINE_STAMPS : 0)
 #else
@@ -111,7 +114,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
     const int wm = wave >> 1, wn = wave & 1;
     const int r16 = lane & 15, kb = lane >> 4;  // fragment row inside a tile; 32-byte K block of the lane
 #ifdef MI8_TILE_TIMELINE
-    uint32_t* const tl_out = g_timeline;
+    uint32_t* const tl_out = !kHalf && (int)blockIdx.x < TIMELINE_WORKGROUPS ? g_timeline : nullptr;
     int tl_ev = 0;
     const uint32_t tl_lds = (uint32_t)(uintptr_t)(lptr_t)(lds + LDS_BYTES - TIMELINE_BYTES);
     auto tl_put = [&](int slot, uint64_t t) __attribute__((always_inline)) {

@@ -460,3 +460,19 @@ def test_half_tiles_of_the_fused_swiglu_launch(dev, mhk):
     assert int(slots[:n].max()) == int(rslots[:rn].max())
     if want_codes:
         assert torch.equal(codes[0], ops.rowseg_max_codes(x1, x3))
+
+
+def test_tile_timeline_stays_in_its_buffer(dev):
+    """A plan with half tiles launches more workgroups than the time stamps have room for: only the first 256, which walk
+    whole tiles, record theirs."""
+    from olmo_core_amd import _C
+
+    M, N, K = 2048, 11008, 256  # 256 whole tiles and 176 half tiles
+    a, b = seeded((M, K), 1).to(E4M3).to(dev), seeded((N, K), 2).to(E4M3).to(dev)
+    s = torch.ones(1, device=dev)
+    out = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+    stamps = torch.full((1024, 256), -1, dtype=torch.int32, device=dev)
+    _C.check_diag(_C.diag().mi8_diag_gemm_tile_timeline(a.data_ptr(), s.data_ptr(), b.data_ptr(), s.data_ptr(), out.data_ptr(), M, N, K,
+                                                        0, 0, stamps.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    assert bool((stamps[256:] == -1).all()) and bool((stamps[:256, 0] != -1).all())
+    assert torch.equal(out, ops.gemm_fp8(a, s, b, s))
