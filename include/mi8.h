@@ -213,8 +213,10 @@ int mi8_gemm_fp8_swiglu(const void* a, int a_dtype, int64_t lda, const void* b1,
  * scheduling), applies the scales and rounds.  Arguments as mi8_gemm_fp8; splits in 1..min(64, ceil(K/128));
  * workspace: 16-byte aligned device memory of mi8_gemm_splitk_workspace_bytes(M, N, splits) bytes, owned by the
  * caller, free for reuse once the call's work on `stream` is done.  mi8_gemm_splitk_suggest returns the number
- * of slices the library would use for a shape (1: call mi8_gemm_fp8 instead).  No counterpart upstream: the
- * reference leaves the choice of GEMM algorithm to torch._scaled_mm's backend. */
+ * of slices the library would use for a shape (1: call mi8_gemm_fp8 instead).  Up to 64 rows K is summed in eighths
+ * (slices of ceil(ceil(K / 128) / 8) steps) whichever entry point or kernel runs, mi8_few_rows_* included, so all of
+ * them give one result; asked for those slices, mi8_gemm_fp8_splitk may add them without planes (the workspace is then
+ * not touched).  No counterpart upstream: the reference leaves the choice of GEMM algorithm to torch._scaled_mm's backend. */
 int mi8_gemm_fp8_splitk(const void* a, int a_dtype, int64_t lda, const void* b, int b_dtype, int64_t ldb,
                         int64_t M, int64_t N, int64_t K, const float* sa, int sa_is_vector, const float* sb,
                         int sb_is_vector, void* out, int out_dtype, int64_t ldc, int splits, void* workspace,
@@ -227,7 +229,8 @@ int mi8_gemm_fp8_splitk_accumulate(const void* a, int a_dtype, int64_t lda, cons
 int mi8_gemm_splitk_suggest(int64_t M, int64_t N, int64_t K);
 int64_t mi8_gemm_splitk_workspace_bytes(int64_t M, int64_t N, int splits);
 
-/* Number of GEMM kernel variants compiled in (variant ids 0..n-1; -1 lets the library choose by shape). */
+/* Number of GEMM kernel variants compiled in (variant ids 0..n-1; -1 lets the library choose by shape).  Which id is
+ * which kernel may change with the library: look a variant up by its name. */
 int mi8_gemm_num_variants(void);
 const char* mi8_gemm_variant_name(int variant);
 

@@ -22,6 +22,7 @@ struct GemmArgs {
     int sa_vec, sb_vec;
     int tiles_m, tiles_n;
     int accumulate;  // add the rounded product to what C holds (the sum of two grad_input halves) instead of overwriting
+    int slice_steps;  // (ring tiles with SLICED) K steps summed from zero before they join the sum
 };
 
 
@@ -108,6 +109,15 @@ int launch_m16_swiglu(GemmArgs& g, const uint8_t* b3, const float* sb3, uint16_t
 // a few rows of A (M <= kSkinnyMaxM) against all of B, bound by reading B once (mi8_gemm_skinny.hip): any N,
 // K % 16 == 0, any mix of single scales and scale vectors, bf16 or fp32 output
 constexpr int kSkinnyMaxM = 64;
+// Up to that many rows K is summed in eighths: slices of this many 128-byte steps (the last ones shorter or empty), each
+// from zero, added in order.  One order for every kernel a product of so few rows may run on - the few-rows kernels, a slice
+// per wave; split K, a slice per plane; ring tiles that add a slice at a time - so a layer's output does not depend on which
+// of them its options, or a training forward next to an evaluation, lead to.
+inline __host__ __device__ int eighth_steps(int64_t K)
+{
+    const int steps = (int)((K + BK - 1) / BK);
+    return (steps + 7) / 8;
+}
 int launch_skinny(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st);
 // the same kernel over the ragged grouped problems (bf16 output, per-row / per-column scale vectors):
 // forward / grad_input (T, N >= 256, K % 128 == 0) and grad_weight (N, Kl >= 256)

@@ -13,13 +13,13 @@ namespace mi8 {
 using namespace gemm;
 namespace {
 
-template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP>
+template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP, bool SLICED>
 __global__ __launch_bounds__(kRingThreads, OCC) void gemm_fp8_ring_kernel(GemmArgs g)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     int tm, tn;
     if (!tile_of_block(g, tm, tn)) return;
-    ring_tile<BM, BN, ST, CBSZ, BLGP>(g, tm * BM, tn * BN, lds);
+    ring_tile<BM, BN, ST, CBSZ, BLGP, SLICED>(g, tm * BM, tn * BN, lds);
 }
 
 // ---- split K ---------------------------------------------------------------------------------------
@@ -60,7 +60,8 @@ __global__ __launch_bounds__(kRingThreads, OCC) void gemm_fp8_splitk_kernel(Spli
 }
 
 // out[m][n] (+)= round( (sum over planes, in plane order) * (1/sa) * (1/sb) ); four columns per thread.  Bound by the
-// latency of the plane reads: four are in flight at a time (one after the other: 7-11 us where this takes 4-6).
+// latency of the plane reads: seven are in flight at a time, so that eight planes are one round of reads (one after the
+// other: 7-11 us where this takes 4-5).
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(SplitArgs a)
 {
     const GemmArgs& g = a.g;
@@ -71,16 +72,17 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(SplitArgs a)
     const int n = (int)(q % quads_per_row) * 4;
     const int64_t plane = (int64_t)g.M * a.ld_plane;
     const float* p = a.planes + (int64_t)m * a.ld_plane + n;
+    constexpr int kInFlight = 7;
     ring_v4f s = *reinterpret_cast<const ring_v4f*>(p);
-    int i = 1;
-    for (; i + 3 < a.splits; i += 4) {
-        ring_v4f t[4];
+    for (int i = 1; i < a.splits; i += kInFlight) {
+        ring_v4f t[kInFlight];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) t[u] = *reinterpret_cast<const ring_v4f*>(p + (i + u) * plane);
+        for (int u = 0; u < kInFlight; ++u)  // (past the last plane: its own again, not added)
+            t[u] = *reinterpret_cast<const ring_v4f*>(p + (i + u < a.splits ? i + u : a.splits - 1) * plane);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) s += t[u];
+        for (int u = 0; u < kInFlight; ++u)
+            if (i + u < a.splits) s += t[u];
     }
-    for (; i < a.splits; ++i) s += *reinterpret_cast<const ring_v4f*>(p + i * plane);
     // same scale arithmetic as the tile routine's own epilogue
     const float isa = g.sa_vec ? __builtin_amdgcn_rcpf(g.sa[m]) : 1.0f / g.sa[0];
     const float isb_single = g.sb_vec ? 0.0f : 1.0f / g.sb[0];
@@ -149,6 +151,29 @@ int best_ring(int64_t M, int64_t N, int64_t steps, int64_t slices, float* cost)
     return best;
 }
 
+// A few rows (more than 16: up to there the few-rows kernel always) sum K in eighths on whichever kernel, so the choice is
+// free: the few-rows kernel, whose workgroups take 32 rows of B and wait out a memory latency per step and wave; ring tiles
+// that walk all of K; ring tiles for each eighth, whose planes a second launch adds.  Constants met within 15 % on 768 x 2048
+// .. 5120 x 27648 and 17 .. 64 rows (us, in this order; 32 x 2816 x 1024: 5.6, 6.7, 8.4; 32 x 11008 x 4096: 23.4, 14.6, 19.1;
+// 32 x 4096 x 11008: 28.6, 29.2, 16.3).
+enum FewRowsKernel { kFewRows, kFewRing, kFewPlanes };
+
+// slices that are not empty
+int eighths(int64_t K) { return (int)(((K + BK - 1) / BK + eighth_steps(K) - 1) / eighth_steps(K)); }
+
+FewRowsKernel choose_few_rows(int64_t M, int64_t N, int64_t K)
+{
+    if (M <= 16) return kFewRows;
+    const float steps = (float)((K + BK - 1) / BK), bytes = (float)N * (float)K;
+    const float rounds = (float)((N + 32 * 256 - 1) / (32 * 256));
+    const float rows = 1.6f + rounds * (1.6f + eighth_steps(K) * (M <= 32 ? 1.75f : 2.6f));
+    const float walk = 4.0f + 0.29f * steps, read = 2.0f + bytes / 4.2e6f;
+    const float ring = walk > read ? walk : read;
+    const float planes = steps < 2.0f ? 1e30f : 5.0f + bytes / 5.3e6f + (float)(M * N) * 1.5e-5f;
+    if (rows <= ring && rows <= planes) return kFewRows;
+    return ring <= planes ? kFewRing : kFewPlanes;
+}
+
 // Slices for a problem, 1 = do not split: a summation order of its own, so it depends on the product alone.  Splitting
 // pays where the whole of K in one workgroup is the time (few tiles, a long K) and costs a second launch that reads the
 // planes; up to 192 tiles of 64 x 64 it is at worst even.  At least four K steps a slice.
@@ -156,7 +181,8 @@ int suggested_splits(int64_t M, int64_t N, int64_t K)
 {
     const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256), tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
     const int64_t steps = (K + BK - 1) / BK;
-    if (M <= 16 || tiles256 > 96 || steps < 8) return 1;  // (up to 16 rows: the few-rows kernel reads B once)
+    if (M <= kSkinnyMaxM) return choose_few_rows(M, N, K) == kFewRows ? 1 : eighths(K);
+    if (tiles256 > 96 || steps < 8) return 1;
     float best;
     best_ring(M, N, steps, 1, &best);
     if (M >= 256 && N >= 256 && K % BK == 0 && N % 8 == 0) {
@@ -181,7 +207,7 @@ int suggested_splits(int64_t M, int64_t N, int64_t K)
 
 // ---- variants: the ring tile shapes, then the other two kernels ----------------------------------------------------
 
-constexpr int kM16 = kNumRing, kSkinny = kNumRing + 1, kNumVariants = kNumRing + 2;
+constexpr int kM16 = kNumRing, kSkinny = kNumRing + 1, kEighths = kNumRing + 2, kNumVariants = kNumRing + 3;
 
 template <typename Args, typename Kernel>
 int launch_ring_kernel(Kernel kern, std::atomic<uint64_t>& configured, int lds_bytes, const Args& a, int tiles, int slices,
@@ -192,7 +218,7 @@ int launch_ring_kernel(Kernel kern, std::atomic<uint64_t>& configured, int lds_b
     return launch_status(what);
 }
 
-template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP>
+template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP, bool SLICED = false>
 int launch_ring(GemmArgs& g, SplitArgs* split, hipStream_t st)
 {
     GemmArgs& p = split ? split->g : g;
@@ -203,7 +229,7 @@ int launch_ring(GemmArgs& g, SplitArgs* split, hipStream_t st)
     if (split)
         return launch_ring_kernel(gemm_fp8_splitk_kernel<BM, BN, ST, OCC, CBSZ, BLGP>, configured[1], kRingLdsBytes<BM, BN, ST>,
                                   *split, tiles, split->splits, st, "mi8_gemm_fp8_splitk");
-    return launch_ring_kernel(gemm_fp8_ring_kernel<BM, BN, ST, OCC, CBSZ, BLGP>, configured[0], kRingLdsBytes<BM, BN, ST>, g,
+    return launch_ring_kernel(gemm_fp8_ring_kernel<BM, BN, ST, OCC, CBSZ, BLGP, SLICED>, configured[0], kRingLdsBytes<BM, BN, ST>, g,
                               tiles, 1, st, "mi8_gemm_fp8");
 }
 
@@ -216,6 +242,7 @@ int launch_ring_shape(int shape, GemmArgs& g, SplitArgs* split, hipStream_t st)
         case 2: return launch_ring<64, 128, 3, 2, CBSZ, BLGP>(g, split, st);
         case 3: return launch_ring<128, 128, 2, 2, CBSZ, BLGP>(g, split, st);
         case 4: return launch_ring<128, 128, 3, 1, CBSZ, BLGP>(g, split, st);
+        case kEighths: g.slice_steps = eighth_steps(g.K); return launch_ring<64, 64, 4, 2, CBSZ, BLGP, true>(g, nullptr, st);
     }
     set_error("mi8_gemm_fp8: unknown variant %d", shape);
     return MI8_ERR_ARG;
@@ -238,7 +265,8 @@ extern "C" int mi8_gemm_num_variants(void) { return kNumVariants; }
 extern "C" const char* mi8_gemm_variant_name(int variant)
 {
     if (variant < 0 || variant >= kNumVariants) return nullptr;
-    return variant == kM16 ? "256x256_dma_w4x128_m16x128" : variant == kSkinny ? "rows64x16_k8_m16x128" : kRing[variant].name;
+    return variant == kM16 ? "256x256_dma_w4x128_m16x128" : variant == kSkinny ? "rows64x16_k8_m16x128"
+           : variant == kEighths ? "64x64_ring4_eighths" : kRing[variant].name;
 }
 
 namespace {
@@ -271,12 +299,12 @@ int gemm_fp8_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b
     const bool dma_ok = (K % 128 == 0) && M >= 256 && N >= 256 && N % 8 == 0 && ldc % 8 == 0 && ldc < (1 << 22) && aligned16(out) &&
                         out_dtype == MI8_BF16 && (!sb_is_vector || aligned16(sb)) &&
                         (sa_is_vector != 0) == (sb_is_vector != 0) && (!accumulate || (M % 128 == 0 && N % 256 == 0));
-    // A few rows of A go to the kernel that streams B once; everything else to whichever of the ring tile shapes and the
-    // persistent kernel the measured costs above say is fastest for this number of tiles and K steps (all of them give
-    // the same bits).
+    // A few rows of A: see choose_few_rows; everything else goes to whichever of the ring tile shapes and the persistent
+    // kernel the measured costs above say is fastest for this number of tiles and K steps (all of them give the same bits).
     if (variant < 0) {
-        if (M <= kSkinnyMaxM) {
-            variant = kSkinny;
+        if (M <= kSkinnyMaxM) {  // (a caller that wants the planes asks for split K)
+            const FewRowsKernel few = choose_few_rows(M, N, K);
+            variant = few == kFewRows || (few == kFewPlanes && M <= 32) ? kSkinny : kEighths;
         } else {
             const int64_t steps = ceil_div(K, BK);
             float cost;
@@ -434,6 +462,9 @@ int splitk_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b_d
     s.steps_per_split = (int)per;
     s.splits = used;
     hipStream_t st = (hipStream_t)stream;
+    // the eighths of a few rows: the planes are left out where one workgroup walks all of K sooner
+    if (M <= kSkinnyMaxM && used == eighths(K) && choose_few_rows(M, N, K) == kFewRing)
+        return launch_ring_typed(kEighths, a_dtype, b_dtype, s.g, nullptr, st);
     float cost;
     const int shape = best_ring(M, N, per, used, &cost);
     if (int rc = launch_ring_typed(shape, a_dtype, b_dtype, s.g, &s, st)) return rc;

@@ -49,7 +49,8 @@ constexpr int kRingLdsBytes = ST * (BM + BN) * BK;
 constexpr int kRingThreads = 256;
 
 // C[m0 .. m0 + BM, n0 .. n0 + BN] of g's product (K may be 0: zeros).  g.sa == null: the raw fp32 sums are wanted.
-template <int BM, int BN, int ST, int CBSZ, int BLGP>
+// SLICED: K is summed in slices of g.slice_steps, each from zero, added in order (the sums of split K without its planes).
+template <int BM, int BN, int ST, int CBSZ, int BLGP, bool SLICED = false>
 __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const int n0, uint8_t* lds)
 {
     constexpr int NW = kRingThreads / 64;
@@ -113,11 +114,18 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
         }
     }
 
-    ring_v4f acc[TM][TN];
+    ring_v4f acc[TM][TN], sum[SLICED ? TM : 1][SLICED ? TN : 1];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = (ring_v4f){0, 0, 0, 0};
+    int slice_left = g.slice_steps;
+    if constexpr (SLICED) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) sum[i][j] = (ring_v4f){0, 0, 0, 0};
+    }
 
 #pragma unroll
     for (int s = 0; s < ST - 1; ++s)
@@ -153,6 +161,24 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
                     __builtin_shufflevector(fb[j][0], fb[j][1], 0, 1, 2, 3, 4, 5, 6, 7),
                     __builtin_shufflevector(fa[i][0], fa[i][1], 0, 1, 2, 3, 4, 5, 6, 7), acc[i][j], BLGP, CBSZ, 0, 0, 0, 0);
         slot = slot == ST - 1 ? 0 : slot + 1;
+        if constexpr (SLICED) {
+            if (--slice_left == 0) {
+                slice_left = g.slice_steps;
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        sum[i][j] += acc[i][j];
+                        acc[i][j] = (ring_v4f){0, 0, 0, 0};
+                    }
+            }
+        }
+    }
+    if constexpr (SLICED) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j] + acc[i][j];
     }
 
     // ---- epilogue: acc[i][j][e] of lane l is C[row = 16 i + l % 16][col = 16 j + 4 (l / 16) + e] of the wave tile.

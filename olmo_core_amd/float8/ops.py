@@ -450,7 +450,7 @@ def few_rows_swiglu(x: torch.Tensor, sx: Optional[torch.Tensor], w1q, s1, w3q, s
     """
     ``h = silu(x1) * x3`` (bf16) and its amax partials ``(slots, n_slots)`` for a few rows, ``x1`` and ``x3`` the two
     input projections, in one launch; ``x`` is e4m3 with its scale ``sx``, or (:func:`few_rows_quantises`) bf16 with
-    ``sx=None``.  Up to 16 rows ``h`` has the bits of the separate launches.
+    ``sx=None``.  ``h`` has the bits of the separate launches (every product of so few rows sums K in eighths).
     """
     _require_gpu(x, "few_rows_swiglu")
     if sx is None:

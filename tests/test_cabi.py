@@ -66,6 +66,16 @@ def test_host_only_entry_points():
     assert L.mi8_gemm_splitk_workspace_bytes(0, 30, 4) == 0
 
 
+def test_few_rows_slices():
+    """17 to 64 rows: either no split, or the non-empty eighths of K - never another order of summation."""
+    L = _C.lib()
+    for m in (17, 32, 33, 64):
+        for n in (8, 1024, 4096, 11008, 27648, 50304):
+            for steps in list(range(1, 90)) + [216, 1000]:
+                per = -(-steps // 8)
+                assert L.mi8_gemm_splitk_suggest(m, n, 128 * steps - 16) in (1, -(-steps // per)), (m, n, steps)
+
+
 def test_host_only_shape_helpers():
     """Sizes and shape predicates the callers plan with (no GPU work)."""
     L = _C.lib()

@@ -476,3 +476,26 @@ def test_tile_timeline_stays_in_its_buffer(dev):
                                                         0, 0, stamps.data_ptr(), torch.cuda.current_stream().cuda_stream))
     assert bool((stamps[256:] == -1).all()) and bool((stamps[:256, 0] != -1).all())
     assert torch.equal(out, ops.gemm_fp8(a, s, b, s))
+
+
+@pytest.mark.parametrize("mnk", [(17, 1000, 2064), (32, 40, 144), (33, 1032, 1152), (64, 520, 4096), (48, 2056, 1024), (64, 24, 27648)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
+def test_few_rows_sum_in_eighths(dev, mnk, vec):
+    """Up to 64 rows every route sums K in the same slices: the few-rows kernel, ring tiles that add a slice at a time, split K
+    over that many planes, what the library chooses, and C += product on each."""
+    M, N, K = mnk
+    a, b = seeded((M, K), 51).to(E5M2).to(dev), seeded((N, K), 52).to(E4M3).to(dev)
+    g = torch.Generator().manual_seed(53)
+    sa = (torch.rand(M if vec else 1, generator=g) + 0.5).to(dev)
+    sb = (torch.rand(N if vec else 1, generator=g) + 0.5).to(dev)
+    names = ops.gemm_variants()
+    steps = -(-K // 128)
+    slices = -(-steps // -(-steps // 8))
+    for dt in (torch.bfloat16, torch.float32):
+        want = ops.gemm_fp8(a, sa, b, sb, out_dtype=dt, variant=names.index("rows64x16_k8_m16x128"))
+        first = seeded((M, N), 54).to(dt).to(dev)
+        for kw in ({}, {"splits": 1}, {"splits": slices}, {"variant": names.index("64x64_ring4_eighths")}):
+            assert torch.equal(ops.gemm_fp8(a, sa, b, sb, out_dtype=dt, **kw), want), kw
+            if "variant" not in kw:
+                assert torch.equal(ops.gemm_fp8(a, sa, b, sb, out_dtype=dt, out=first.clone(), accumulate=True, **kw), first + want), kw

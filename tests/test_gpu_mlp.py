@@ -331,3 +331,39 @@ def test_evaluation_gives_the_training_forward(dev, mdh, kept):
         with torch.no_grad():
             got = ff(x)
         assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
+@pytest.mark.parametrize("kept", [True, False], ids=["kept_weights", "plain"])
+@pytest.mark.parametrize("mdh", [(17, 1040, 2768), (23, 4096, 11008), (32, 1024, 528), (33, 768, 2048), (48, 2048, 4096), (64, 1024, 2816)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_few_rows_have_one_result(dev, mdh, kept):
+    """17 to 64 rows: evaluation, the training forward, the three modules one by one and a checkpointed block whose first
+    run is without gradients and whose second is not all give the same bits, whichever launches they take."""
+    from torch.utils.checkpoint import checkpoint
+
+    M, D, H = mdh
+    ao = AOFloat8LinearConfig.recommended() if kept else None
+    ff, parts = _make(dev, D, H, fuse=True, ao=ao), _make(dev, D, H, fuse=False, ao=ao)
+    x, go = seeded((M, D), 1).to(dev), seeded((M, D), 2, std=1e-3).to(dev)
+    x[0, 3] = 40.0
+
+    def step(fn):
+        ff.zero_grad()
+        xd = x.clone().requires_grad_(True)
+        y = fn(xd)
+        y.backward(go)
+        return [y.detach(), xd.grad] + [p.grad.clone() for p in ff.parameters()]
+
+    plain = step(ff)
+    with torch.no_grad():
+        assert torch.equal(ff(x), plain[0]) and torch.equal(parts(x), plain[0])
+    for a, b in zip(step(lambda t: checkpoint(ff, t, use_reentrant=True)), plain):
+        assert torch.equal(a, b)
+
+
+def test_compiled_few_rows_equal_eager(dev):
+    M, D, H = 23, 1040, 2768
+    ff = _make(dev, D, H, fuse=True, ao=AOFloat8LinearConfig.recommended())
+    x = seeded((M, D), 1).to(dev)
+    with torch.no_grad():
+        assert torch.equal(torch.compile(ff, fullgraph=True)(x), ff(x))
