@@ -269,7 +269,7 @@ def gemm_fp8(
     ``a`` and ``b`` are fp8 tensors whose rows are K-contiguous; ``sa`` / ``sb`` hold one scale or one per row.
     ``out``: an ``[M, N]`` tensor of ``out_dtype`` with contiguous rows (any row pitch) to write into.
     ``splits``: slices of K summed separately and added afterwards (for problems with few output tiles);
-    -1 lets the library decide from the shape, 1 forbids splitting; a forced ``variant`` is never split.
+    -1 lets the library decide from the shape, 0 and 1 forbid splitting; a forced ``variant`` is never split.
     """
     _require_gpu(a, "gemm_fp8")
     if a.dim() != 2 or b.dim() != 2 or a.stride(1) != 1 or b.stride(1) != 1:
@@ -300,7 +300,7 @@ def gemm_fp8(
         splits = 1
     elif splits < 0:
         splits = L.mi8_gemm_splitk_suggest(M, N, K)
-    if accumulate and splits == 1:
+    if accumulate and splits <= 1:
         _C.check(
             L.mi8_gemm_fp8_accumulate(
                 a.data_ptr(), _FP8_CODE[a.dtype], a.stride(0), b.data_ptr(), _FP8_CODE[b.dtype], b.stride(0), M, N, K,
