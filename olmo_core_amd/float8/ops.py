@@ -464,6 +464,10 @@ def few_rows_swiglu(x: torch.Tensor, sx: Optional[torch.Tensor], w1q, s1, w3q, s
     h = torch.empty((M, H), dtype=torch.bfloat16, device=x.device)
     slots = torch.empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x.device)
     used = _C.c_int32(0)
+    sink = GEMM_EVENT_SINK
+    if sink is not None:
+        ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        ev0.record()
     _C.check(
         _C.lib().mi8_few_rows_swiglu(
             x.data_ptr(), int(sx is not None), x.stride(0) if M > 1 else K, sx.data_ptr() if sx is not None else None,
@@ -472,6 +476,9 @@ def few_rows_swiglu(x: torch.Tensor, sx: Optional[torch.Tensor], w1q, s1, w3q, s
         ),
         "mi8_few_rows_swiglu",
     )
+    if sink is not None:
+        ev1.record()
+        sink.append((ev0, ev1, (M, 2 * H, K)))
     return h, (slots, used.value)
 
 
@@ -484,6 +491,10 @@ def few_rows_cast_gemm(x: torch.Tensor, slots: Tuple[torch.Tensor, int], wq, sw,
     M, K = x.shape
     N = wq.shape[0]
     out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    sink = GEMM_EVENT_SINK
+    if sink is not None:
+        ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        ev0.record()
     _C.check(
         _C.lib().mi8_few_rows_cast_gemm(
             x.data_ptr(), K, slots[0].data_ptr(), slots[1], wq.data_ptr(), wq.stride(0), M, N, K, sw.data_ptr(),
@@ -491,6 +502,9 @@ def few_rows_cast_gemm(x: torch.Tensor, slots: Tuple[torch.Tensor, int], wq, sw,
         ),
         "mi8_few_rows_cast_gemm",
     )
+    if sink is not None:
+        ev1.record()
+        sink.append((ev0, ev1, (M, N, K)))
     return out
 
 

@@ -382,3 +382,19 @@ def test_compiled_few_rows_equal_eager(dev):
     x = seeded((M, D), 1).to(dev)
     with torch.no_grad():
         assert torch.equal(torch.compile(ff, fullgraph=True)(x), ff(x))
+
+
+@pytest.mark.parametrize("M", [1, 5, 17, 64, 65])
+def test_gemm_events_cover_the_products_of_an_evaluation(dev, M, monkeypatch):
+    """Every launch that holds a product is recorded, whichever launches the rows lead to."""
+    D, H = 4096, 11008
+    ff = _make(dev, D, H, fuse=True, ao=AOFloat8LinearConfig.recommended())
+    x = seeded((M, D), 1).to(dev)
+    with torch.no_grad():
+        ff(x)
+        events = []
+        monkeypatch.setattr(ops, "GEMM_EVENT_SINK", events)
+        ff(x)
+    torch.cuda.synchronize()
+    assert sum(m * n * k for _, _, (m, n, k) in events) == 3 * M * D * H
+    assert all(a.elapsed_time(b) > 0 for a, b, _ in events)
