@@ -281,7 +281,8 @@ int mi8_grouped_swiglu_bwd(const void* x1, const void* x2, const void* gh, int64
 
 /* out[R_e, :N] = (A[R_e, :K] . B_e[:N, :K]^T) / sa[r] / sb_e[n]   for every group e.
  *   A fp8 [T, lda]; B_e = b + e * b_group_stride (bytes), N rows of pitch ldb; sa float32 [T];
- *   sb_e = sb + e * sb_group_stride (floats), N values; out [T, ldc] of out_dtype. */
+ *   sb_e = sb + e * sb_group_stride (floats), N values; out [T, ldc] of out_dtype.
+ *   lda < 2^27, or T * lda < 2^32. */
 int mi8_grouped_gemm_fp8(const void* a, int a_dtype, int64_t lda, const void* b, int b_dtype, int64_t ldb,
                          int64_t b_group_stride, const int64_t* group_sizes, int32_t num_groups, int64_t T, int64_t N,
                          int64_t K, const float* sa, const float* sb, int64_t sb_group_stride, void* out,

@@ -199,7 +199,10 @@ int grouped_gemm_entry(const void* a, int a_dtype, int64_t lda, const void* b, i
     MI8_REQUIRE(aligned16(a) && aligned16(b), MI8_ERR_UNSUPPORTED, "mi8_grouped_gemm_fp8: operands must be 16-byte aligned");
     MI8_REQUIRE(N * ldb < ((int64_t)1 << 32) && T < (1 << 30) && N < (1 << 30) && K < (1 << 30), MI8_ERR_UNSUPPORTED,
                 "mi8_grouped_gemm_fp8: operand too large");
-    MI8_REQUIRE(lda < (1 << 25), MI8_ERR_UNSUPPORTED, "mi8_grouped_gemm_fp8: lda (%lld) of 2^25 or more", (long long)lda);
+    // (a ring tile addresses its rows of A, 128 or, in the smallest, 32, with 32-bit byte offsets)
+    const bool whole_a_fits = T <= (((int64_t)1 << 32) - 1) / lda;
+    MI8_REQUIRE(whole_a_fits || lda < (1 << 27), MI8_ERR_UNSUPPORTED, "mi8_grouped_gemm_fp8: lda (%lld) of 2^27 or more and an operand of 4 GiB or more",
+                (long long)lda);
     GroupedArgs g{(const uint8_t*)a, (const uint8_t*)b, out, out_dtype == MI8_F32 ? 1 : 0, lda, ldb, ldc,
                   b_group_stride, sb_group_stride, group_sizes, num_groups, T, (int)N, (int)K, sa, sb, 0,
                   accumulate ? 1 : 0};
@@ -209,7 +212,7 @@ int grouped_gemm_entry(const void* a, int a_dtype, int64_t lda, const void* b, i
     const bool fits = out_dtype == MI8_BF16 && T >= 256 && N >= 256 && K % 128 == 0 && N % 8 == 0 && ldc % 8 == 0 && aligned16(out) &&
         sb_group_stride % 4 == 0 && aligned16(sb) && lda < (1 << 23) && ldb < (1 << 23) && ldc < (1 << 22) &&
         (!accumulate || N % 256 == 0);
-    const GroupedKernel k = choose_grouped(T, num_groups, N, K, fits);
+    const GroupedKernel k = whole_a_fits || lda < (1 << 25) ? choose_grouped(T, num_groups, N, K, fits) : kRing32;
     if (k == kPersistent)
         return launch_m16_grouped((const uint8_t*)a, a_dtype, lda, (const uint8_t*)b, b_dtype, ldb, b_group_stride,
                                    group_sizes, num_groups, T, (int)N, (int)K, sa, sb, sb_group_stride, (uint16_t*)out,

@@ -108,3 +108,11 @@ def test_argument_validation_happens_before_any_gpu_call():
     assert L.mi8_amax_partials_batch(ptrs, ns, 2, 0, ctypes.c_void_p(16), None, None) == -1 and "tensor 0 is null" in _C.last_error()
     with pytest.raises(Exception):
         _C.check(-2, "x")
+
+
+def test_grouped_pitch_limits():
+    """T * lda below 4 GiB or lda below 2^27: refused by the numbers alone (the pointers are never followed)."""
+    L, p = _C.lib(), ctypes.c_void_p(256)
+
+    rc = L.mi8_grouped_gemm_fp8(p, 0, 1 << 27, p, 0, 256, 0, p, 1, 32, 1, 256, p, p, 0, p, 1, 1, None)
+    assert rc == -2 and "2^27" in _C.last_error()

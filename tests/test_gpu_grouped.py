@@ -550,3 +550,19 @@ def test_grouped_gemm_choice_exact_integers(dev, sizes, n, k, accumulate):
                 want = old[rows] + want
             assert torch.equal(out[rows], want), f"group {e}"
         start += m
+
+
+@pytest.mark.parametrize("sizes", [[2, 0, 1], [100, 1, 0, 29]], ids=["3 rows", "130 rows, 4 GiB"])
+def test_grouped_gemm_takes_a_wide_pitch(dev, sizes):
+    """Rows of A 2^25 bytes apart: any number of them."""
+    E, T, n, k, pitch = len(sizes), sum(sizes), 64, 272, 1 << 25
+    g = torch.Generator(device="cuda").manual_seed(1)
+    a = torch.empty(T * pitch, dtype=torch.uint8, device=dev).view(E4M3).as_strided((T, k), (pitch, 1))
+    values = torch.randint(-4, 5, (T, k), generator=g, device=dev).float()
+    a.copy_(values.to(E4M3))
+    b = torch.randint(-4, 5, (E * n, k), generator=g, device=dev).float()
+    one = torch.ones(max(T, E * n), device=dev)
+    out = ops.grouped_gemm_fp8(a, one[:T], b.to(E4M3), one[:E * n], torch.tensor(sizes), n=n, k=k, b_group_stride=n * k,
+                               sb_group_stride=n, out_dtype=torch.float32)
+    group = torch.repeat_interleave(torch.arange(E), torch.tensor(sizes)).to(dev)
+    assert torch.equal(out, (values[:, None, :] @ b.view(E, n, k)[group].transpose(1, 2).contiguous())[:, 0])
