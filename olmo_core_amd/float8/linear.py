@@ -34,10 +34,11 @@ __all__ = ["Float8Linear", "convert_to_float8_training", "float8_linear_function
 
 def needs_autograd(*tensors: torch.Tensor) -> bool:
     """Whether a call on these tensors has to go through an autograd function: some gradient is wanted, or
-    forward-mode differentiation is on (the function then refuses, where plain kernels would drop the tangent)."""
+    forward-mode differentiation or a transform (vmap, torch.func.grad, ...) is on, which the function refuses by name
+    where plain kernels would drop the tangent or stumble over a tensor without storage."""
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return True
-    return torch.autograd.forward_ad._current_level >= 0
+    return torch.autograd.forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
 
 
 def _is_tensorwise(c: CastConfig) -> bool:

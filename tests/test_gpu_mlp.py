@@ -398,3 +398,27 @@ def test_gemm_events_cover_the_products_of_an_evaluation(dev, M, monkeypatch):
     torch.cuda.synchronize()
     assert sum(m * n * k for _, _, (m, n, k) in events) == 3 * M * D * H
     assert all(a.elapsed_time(b) > 0 for a, b, _ in events)
+
+
+@pytest.mark.parametrize("M", [5, 300])
+def test_transforms_are_refused_by_name_without_gradients(dev, M):
+    """vmap, torch.func.grad / jvp and dual numbers: the block and the expert layer refuse as the autograd functions do, also
+    where nothing requires a gradient and where the transformed value is another one than x."""
+    import torch.autograd.forward_ad as fwd_ad
+    from torch.func import grad, jvp, vmap
+
+    from olmo_core_amd.nn import DroplessMoEMLP
+
+    D = 256
+    ff = _make(dev, D, 512, fuse=True, ao=AOFloat8LinearConfig.recommended()).requires_grad_(False)
+    experts = DroplessMoEMLP(d_model=D, hidden_size=256, num_experts=2, dtype=torch.bfloat16, init_device="cuda").requires_grad_(False)
+    sizes = torch.tensor([M - 2, 2], device=dev)
+    x, scalars = seeded((3, M, D), 1).to(dev), torch.ones(3, device=dev)
+    for fn in (ff, lambda t: experts(t, sizes)):
+        fn(x[0])
+        for call in (lambda: vmap(fn)(x), lambda: vmap(lambda s: s * fn(x[0]).float().sum())(scalars),
+                     lambda: grad(lambda s: s * fn(x[0]).float().sum())(scalars[0]), lambda: jvp(fn, (x[0],), (x[1],))):
+            with pytest.raises(RuntimeError, match="setup_context"):
+                call()
+        with fwd_ad.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
+            fn(fwd_ad.make_dual(x[0], x[1]))
