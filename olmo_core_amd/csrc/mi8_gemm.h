@@ -49,18 +49,20 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi)
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
 }
 
-// bf16(a) + bf16(b) for eight packed values, each sum formed in float32 and rounded once (what an elementwise add of
-// two bf16 tensors computes)
+// bf16(a) + bf16(b) for two or eight packed values, each sum formed in float32 and rounded once (what an elementwise add
+// of two bf16 tensors computes)
+__device__ __forceinline__ uint32_t add_bf16x2(uint32_t x, uint32_t y)
+{
+    const float lo = bits_to_f32(x << 16) + bits_to_f32(y << 16);
+    const float hi = bits_to_f32(x & 0xFFFF0000u) + bits_to_f32(y & 0xFFFF0000u);
+    return pack_bf16x2(lo, hi);
+}
+
 __device__ __forceinline__ v4i add_bf16x8(v4i a, v4i b)
 {
     v4i r;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t x = (uint32_t)a[i], y = (uint32_t)b[i];
-        const float lo = bits_to_f32(x << 16) + bits_to_f32(y << 16);
-        const float hi = bits_to_f32(x & 0xFFFF0000u) + bits_to_f32(y & 0xFFFF0000u);
-        r[i] = (int)pack_bf16x2(lo, hi);
-    }
+    for (int i = 0; i < 4; ++i) r[i] = (int)add_bf16x2((uint32_t)a[i], (uint32_t)b[i]);
     return r;
 }
 

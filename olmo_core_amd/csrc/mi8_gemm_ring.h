@@ -203,9 +203,58 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[i][j][e] = both_single ? acc[i][j][e] * one : acc[i][j][e] * isa * isb[j][e];
     }
+    const bool wide = (reinterpret_cast<uintptr_t>(g.C) & 15) == 0 && ((g.ldc | g.N) & (g.c_f32 ? 3 : 7)) == 0;
+    if (!wide) {
+        // Rows that are not whole 16-byte chunks leave an element per lane, or four bf16 values where rows are whole 8-byte
+        // chunks, consecutive lanes on consecutive columns (16 rows of the wave tile at a time through LDS; the ring is free
+        // now).  Stored from the accumulators, whose lanes hold 16 rows of four columns each, 14592 x 3967 x 1040 in float32
+        // took 188 us where this takes 127, 65536 rows in 32 groups x 1020 x 1024 213 where this takes 153.
+        const bool quads = !g.c_f32 && ((g.ldc | g.N) & 3) == 0 && (reinterpret_cast<uintptr_t>(g.C) & 7) == 0;
+        constexpr int PITCH = WTN + 4;
+        static_assert(NW * 16 * PITCH * 4 <= ST * STAGE, "output staging");
+        __syncthreads();
+        float* stg = reinterpret_cast<float*>(lds) + wave * (16 * PITCH);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) *reinterpret_cast<ring_v4f*>(stg + r16 * PITCH + 16 * j + 4 * kb) = acc[i][j];
+            if (quads) {
+                constexpr int QPR = WTN / 4;
+#pragma unroll
+                for (int it = 0; it < 16 * QPR / 64; ++it) {
+                    const int rw = (it * 64 + lane) / QPR, cw = lane % QPR * 4;
+                    const ring_v4f v = *reinterpret_cast<const ring_v4f*>(stg + rw * PITCH + cw);
+                    const int row = m0 + wm * WTM + 16 * i + rw, col = n0 + wn * WTN + cw;
+                    if (row >= g.M || col >= g.N) continue;
+                    uint2* c = reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.C) + (int64_t)row * g.ldc + col);
+                    uint2 r = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+                    if (g.accumulate) r = make_uint2(add_bf16x2(r.x, c->x), add_bf16x2(r.y, c->y));
+                    *c = r;
+                }
+                continue;
+            }
+#pragma unroll
+            for (int it = 0; it < 16 * WTN / 64; ++it) {
+                const int rw = (it * 64 + lane) / WTN, cw = lane % WTN;
+                const float v = stg[rw * PITCH + cw];
+                const int row = m0 + wm * WTM + 16 * i + rw, col = n0 + wn * WTN + cw;
+                if (row >= g.M || col >= g.N) continue;
+                const int64_t at = (int64_t)row * g.ldc + col;
+                if (g.c_f32) {
+                    float* c = reinterpret_cast<float*>(g.C) + at;
+                    *c = g.accumulate ? *c + v : v;
+                } else {
+                    uint16_t* c = reinterpret_cast<uint16_t*>(g.C) + at;
+                    uint16_t r = f32_to_bf16_bits(v);
+                    if (g.accumulate)
+                        r = f32_to_bf16_bits(bits_to_f32((uint32_t)*c << 16) + bits_to_f32((uint32_t)r << 16));
+                    *c = r;
+                }
+            }
+        }
+        return;
+    }
     if (g.c_f32) {
-        float* C = reinterpret_cast<float*>(g.C);
-        const bool wide = ((g.ldc | g.N) & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             const int row = row0 + 16 * i;
@@ -213,42 +262,14 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 const int col = col0 + 16 * j;
-                float* c = C + (int64_t)row * g.ldc + col;
-                if (wide) {
-                    if (col < g.N) {
-                        ring_v4f* c4 = reinterpret_cast<ring_v4f*>(c);
-                        *c4 = g.accumulate ? *c4 + acc[i][j] : acc[i][j];
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (col + e < g.N) c[e] = g.accumulate ? c[e] + acc[i][j][e] : acc[i][j][e];
-                }
+                if (col >= g.N) continue;
+                ring_v4f* c = reinterpret_cast<ring_v4f*>(reinterpret_cast<float*>(g.C) + (int64_t)row * g.ldc + col);
+                *c = g.accumulate ? *c + acc[i][j] : acc[i][j];
             }
         }
         return;
     }
     uint16_t* C = reinterpret_cast<uint16_t*>(g.C);
-    if (((g.ldc | g.N) & 7) != 0 || (reinterpret_cast<uintptr_t>(C) & 15) != 0) {  // rows that are not whole 16-byte chunks
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            const int row = row0 + 16 * i;
-            if (row >= g.M) continue;
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int col = col0 + 16 * j + e;
-                    if (col >= g.N) continue;
-                    uint16_t* c = C + (int64_t)row * g.ldc + col;
-                    uint16_t r = f32_to_bf16_bits(acc[i][j][e]);
-                    if (g.accumulate)  // both terms are bf16 values, summed in float32 and rounded once
-                        r = f32_to_bf16_bits(bits_to_f32((uint32_t)*c << 16) + bits_to_f32((uint32_t)r << 16));
-                    *c = r;
-                }
-        }
-        return;
-    }
     // bf16 rows leave through LDS (the ring is free now): whole row segments of the wave tile, 16 bytes per lane
     constexpr int PITCH = WTN * 2 + 16;  // (the pad spreads the rows of a store over the banks)
     static_assert(NW * WTM * PITCH <= ST * STAGE, "output staging");

@@ -510,3 +510,24 @@ def test_accumulating_keeps_what_out_holds(dev, splits):
         if splits <= -(-K // 128):
             got = ops.gemm_fp8(a, one, b, one, out_dtype=torch.float32, out=first.clone(), accumulate=True, splits=splits)
             assert torch.equal(got, first + a.float() @ b.float().t())
+
+
+@pytest.mark.parametrize("name", RING)
+@pytest.mark.parametrize("n,pad,skip", [(132, 0, 0), (132, 4, 0), (136, 8, 4), (130, 2, 0), (129, 0, 0), (132, 4, 2), (132, 4, 1)],
+                         ids=lambda v: str(v))
+def test_ring_tiles_store_rows_of_any_alignment(dev, name, n, pad, skip):
+    """Output rows that are whole 8-byte chunks, whole elements only, or start off their chunk: written and added to, and
+    nothing beside them."""
+    m, k = 137, 144
+    a, b = _int_operand((m, k), 1, E4M3).to(dev), _int_operand((n, k), 2, E4M3).to(dev)
+    one, ref = torch.ones(1, device=dev), a.float() @ b.float().t()
+    v = ops.gemm_variants().index(name)
+    for dt in (torch.bfloat16, torch.float32):
+        buf = torch.full((m * (n + pad) + 16,), 5.0, device=dev, dtype=dt)
+        out = buf[skip:skip + m * (n + pad)].view(m, n + pad)[:, :n]
+        ops.gemm_fp8(a, one, b, one, out_dtype=dt, out=out, variant=v)
+        assert torch.equal(out, ref.to(dt))
+        ops.gemm_fp8(a, one, b, one, out_dtype=dt, out=out, accumulate=True, splits=1)
+        assert torch.equal(out, ref.to(dt) + ref.to(dt))
+        out.fill_(5.0)
+        assert bool((buf == 5.0).all())
