@@ -174,9 +174,10 @@ FewRowsKernel choose_few_rows(int64_t M, int64_t N, int64_t K)
     return ring <= planes ? kFewRing : kFewPlanes;
 }
 
-// Slices for a problem, 1 = do not split: a summation order of its own, so it depends on the product alone.  Splitting
-// pays where the whole of K in one workgroup is the time (few tiles, a long K) and costs a second launch that reads the
-// planes; up to 192 tiles of 64 x 64 it is at worst even.  At least four K steps a slice.
+// Slices for a problem, 1 = do not split.  Slices are a summation order of their own, so they follow from the sizes alone.
+// Splitting pays where the whole of K in one workgroup is the time (few tiles, a long K) and costs a second launch that reads
+// the planes.  Up to 192 tiles of 64 x 64 it is at worst even, so there the unsplit estimate is not asked: such a product
+// of at least eight K steps is always split.  At least four K steps a slice.
 int suggested_splits(int64_t M, int64_t N, int64_t K)
 {
     const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256), tiles64 = ((M + 63) / 64) * ((N + 63) / 64);

@@ -989,12 +989,11 @@ namespace {
 // rounds of 256 workgroups for 1.34 rounds of work; as 256 whole and 176 half tiles it takes 79 us instead of 84.
 // 4096 x 2048 x 8192, 128 tiles, is 256 half tiles: 59 us instead of 76.  (A step of a half tile takes 0.65 us with its
 // operands in the memory-side cache, 0.85 us from HBM; a whole tile's 1.0 us, 1.35 us when all compute units have one.)
-HalfRows plan_halves(GemmArgs& g, int most_halves = 1 << 30)
+HalfRows plan_halves(GemmArgs& g, const int cus, int most_halves = 1 << 30)
 {
     const int half_rows = (g.M + 127) / 128;
     g.tiles_m = half_rows / 2;
     const int pairs = g.tiles_m * g.tiles_n, odd = (half_rows & 1) * g.tiles_n;
-    const int cus = num_compute_units();
     const float steps = (float)(g.K / BK), whole = steps * 1.05f + 5.0f, half = steps * 0.78f + 3.5f;
     // the longest share of a workgroup: half tiles are dealt first to those with fewer whole ones
     auto longest = [&](int split) {
@@ -1023,15 +1022,18 @@ HalfRows plan_halves(GemmArgs& g, int most_halves = 1 << 30)
 
 float m16_cost(int64_t M, int64_t N, int64_t K)
 {
-    // (the plan's own arithmetic, with the fixed cost of a launch; a full machine runs whole tiles at 1.35 us a step)
+    // Whether a product is cut along K hangs on this, and with it the order of its sums: the 256 units of a whole chip, not
+    // those of the device at hand, so that the sizes alone decide.  Absolute times, to be set against another kernel's: a
+    // step of a whole tile 1.0 us, rising to 1.35 as all units get one, plus the launch.  (The plan compares ways to cut one
+    // problem and takes 1.05 throughout.)
+    constexpr int cus = 256;
     GemmArgs g{};
     g.M = (int)M;
     g.N = (int)N;
     g.K = (int)K;
     g.tiles_n = (int)((N + BN - 1) / BN);
-    const HalfRows h = plan_halves(g);
+    const HalfRows h = plan_halves(g, cus);
     const float steps = (float)(K / BK);
-    const int cus = num_compute_units();
     const int q = h.n_full / cus, r = h.n_full % cus, halves = (h.n_half + cus - 1) / cus;
     float t = 3.0f + q * (steps * 1.35f + 5.0f);
     if (r) t += steps * (1.0f + 0.35f * (r > cus / 2 ? (float)(2 * r - cus) / cus : 0.0f)) + 5.0f;
@@ -1042,7 +1044,7 @@ float m16_cost(int64_t M, int64_t N, int64_t K)
 int launch_m16(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st)
 {
     g.tiles_n = (g.N + BN - 1) / BN;
-    const HalfRows rows = plan_halves(g);
+    const HalfRows rows = plan_halves(g, num_compute_units());
     if (g.sa_vec) {
         if (g.accumulate) return launch_typed(DenseProblem<true, true>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);
         return launch_typed(DenseProblem<true>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);
@@ -1054,7 +1056,7 @@ int launch_m16(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st)
 int launch_m16_codes(GemmArgs& g, uint16_t* codes, int a_dtype, int b_dtype, hipStream_t st)
 {
     g.tiles_n = (g.N + BN - 1) / BN;
-    const HalfRows rows = plan_halves(g);
+    const HalfRows rows = plan_halves(g, num_compute_units());
     DenseProblem<false, false, true> pb{g, g.lda, g.ldb, g.ldc, rows};
     pb.codes = codes;
     return launch_typed(pb, 0, true, a_dtype, b_dtype, st);
@@ -1064,7 +1066,7 @@ int launch_m16_swiglu(GemmArgs& g, const uint8_t* b3, const float* sb3, uint16_t
                       int* n_slots, uint16_t* x_codes, int a_dtype, int b_dtype, hipStream_t st)
 {
     g.tiles_n = (g.N + 127) / 128;
-    const HalfRows rows = plan_halves(g, 256);  // (4 partial maxima per workgroup, MI8_AMAX_SLOTS in all)
+    const HalfRows rows = plan_halves(g, num_compute_units(), 256);  // (4 partial maxima per workgroup, MI8_AMAX_SLOTS in all)
     SwigluProblem pb{g, g.lda, g.ldb, g.ldc, rows, (int64_t)(b3 - g.B), (int64_t)(x3 - reinterpret_cast<uint16_t*>(g.C)),
                      (int64_t)(h - reinterpret_cast<uint16_t*>(g.C)), sb3, h_slots, x_codes};
     *n_slots = 4 * rows.blocks();  // one partial maximum per wave of the grid
