@@ -60,8 +60,9 @@ __global__ __launch_bounds__(kRingThreads, OCC) void gemm_fp8_splitk_kernel(Spli
 }
 
 // out[m][n] (+)= round( (sum over planes, in plane order) * (1/sa) * (1/sb) ); four columns per thread.  Bound by the
-// latency of the plane reads: seven are in flight at a time, so that eight planes are one round of reads (one after the
-// other: 7-11 us where this takes 4-5).
+// latency of the plane reads: kInFlight are in flight at a time, seven where there are more than four planes, so that eight
+// are one round of reads (one after the other: 7-11 us where this takes 4-5).
+template <int kInFlight>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(SplitArgs a)
 {
     const GemmArgs& g = a.g;
@@ -72,13 +73,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(SplitArgs a)
     const int n = (int)(q % quads_per_row) * 4;
     const int64_t plane = (int64_t)g.M * a.ld_plane;
     const float* p = a.planes + (int64_t)m * a.ld_plane + n;
-    constexpr int kInFlight = 7;
     ring_v4f s = *reinterpret_cast<const ring_v4f*>(p);
     for (int i = 1; i < a.splits; i += kInFlight) {
         ring_v4f t[kInFlight];
 #pragma unroll
-        for (int u = 0; u < kInFlight; ++u)  // (past the last plane: its own again, not added)
-            t[u] = *reinterpret_cast<const ring_v4f*>(p + (i + u < a.splits ? i + u : a.splits - 1) * plane);
+        for (int u = 0; u < kInFlight; ++u)
+            if (i + u < a.splits) t[u] = *reinterpret_cast<const ring_v4f*>(p + (i + u) * plane);
 #pragma unroll
         for (int u = 0; u < kInFlight; ++u)
             if (i + u < a.splits) s += t[u];
@@ -470,7 +470,8 @@ int splitk_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b_d
     const int shape = best_ring(M, N, per, used, &cost);
     if (int rc = launch_ring_typed(shape, a_dtype, b_dtype, s.g, &s, st)) return rc;
     const int64_t quads = M * (s.ld_plane / 4);
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, s);
+    const auto reduce = used > 4 ? splitk_reduce_kernel<7> : used > 2 ? splitk_reduce_kernel<3> : splitk_reduce_kernel<1>;
+    hipLaunchKernelGGL(reduce, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, s);
     return launch_status("mi8_gemm_fp8_splitk");
 }
 }  // namespace
