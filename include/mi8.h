@@ -201,7 +201,7 @@ int mi8_gemm_fp8_accumulate(const void* a, int a_dtype, int64_t lda, const void*
  * larger of x1 and x3 (what mi8_rowseg_max_codes(x1, x3) computes; needs H % 64 == 0), for the backward pass's
  * mi8_swiglu_bwd_amax_from_codes. */
 int mi8_gemm_fp8_swiglu_matches_separate(int64_t M, int64_t H, int64_t K); /* host only: 1 if the fused launch takes
-    the shape and mi8_gemm_fp8 would run both projections on the same tile kernel, so that the bits agree as well */
+    the shape and the library would not cut either projection along K, so that the bits agree as well */
 int mi8_gemm_fp8_swiglu(const void* a, int a_dtype, int64_t lda, const void* b1, const void* b3, int b_dtype, int64_t ldb,
                         int64_t M, int64_t H, int64_t K, const float* sa, const float* sb1, const float* sb3, void* x1,
                         void* x3, void* h, int64_t ldc, uint32_t* slots_h, int32_t* n_slots_used, uint16_t* x_codes,
@@ -233,6 +233,9 @@ int64_t mi8_gemm_splitk_workspace_bytes(int64_t M, int64_t N, int splits);
  * which kernel may change with the library: look a variant up by its name. */
 int mi8_gemm_num_variants(void);
 const char* mi8_gemm_variant_name(int variant);
+/* Host only: the variant that -1 stands for in mi8_gemm_fp8 (accumulate != 0: in mi8_gemm_fp8_accumulate) when ldc == N, the
+ * pointers are 16-byte aligned and the scales of one kind; -1 for an empty product. */
+int mi8_gemm_variant_for(int64_t M, int64_t N, int64_t K, int out_dtype, int accumulate);
 
 /* ---------------------------------------------------------------------------------------------
  * Ragged grouped operations for the dropless-MoE expert layer.  The reference runs this layer in bf16 through

@@ -100,6 +100,7 @@ _SIGNATURES = {
     "mi8_gemm_splitk_workspace_bytes": (c_int64, [c_int64, c_int64, c_int]),
     "mi8_gemm_num_variants": (c_int, []),
     "mi8_gemm_variant_name": (c_char_p, [c_int]),
+    "mi8_gemm_variant_for": (c_int, [c_int64, c_int64, c_int64, c_int, c_int]),
     "mi8_few_rows_swiglu": (
         c_int,
         [c_void_p, c_int, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p,

@@ -261,6 +261,36 @@ int launch_ring_typed(int shape, int a_dtype, int b_dtype, GemmArgs& g, SplitArg
 
 using namespace mi8;
 
+namespace {
+// What the persistent kernel asks of a product's sizes.  (It shifts its last tile row / column back over the previous one when
+// M or N is not a whole number of half tiles (128 x 256) and rewrites the overlap with identical values: not possible when
+// accumulating.  Its output stores address a tile's 256 rows with 32-bit byte offsets: ldc < 2^22.)
+bool m16_takes(int64_t M, int64_t N, int64_t K, int64_t ldc, int out_dtype, bool accumulate)
+{
+    return K % 128 == 0 && M >= 256 && N >= 256 && N % 8 == 0 && ldc % 8 == 0 && ldc < (1 << 22) && out_dtype == MI8_BF16 &&
+           (!accumulate || (M % 128 == 0 && N % 256 == 0));
+}
+
+// A few rows of A: see choose_few_rows; everything else goes to whichever of the ring tile shapes and the persistent
+// kernel the measured costs above say is fastest for this number of tiles and K steps (all of them give the same bits).
+int chosen_variant(int64_t M, int64_t N, int64_t K, bool m16_fits)
+{
+    if (M <= kSkinnyMaxM) {  // (a caller that wants the planes asks for split K)
+        const FewRowsKernel few = choose_few_rows(M, N, K);
+        return few == kFewRows || (few == kFewPlanes && M <= 32) ? kSkinny : kEighths;
+    }
+    float cost;
+    const int ring = best_ring(M, N, ceil_div(K, BK), 1, &cost);
+    return m16_fits && m16_cost(M, N, K) < cost ? kM16 : ring;
+}
+}  // namespace
+
+extern "C" int mi8_gemm_variant_for(int64_t M, int64_t N, int64_t K, int out_dtype, int accumulate)
+{
+    if (M <= 0 || N <= 0 || K <= 0) return -1;
+    return chosen_variant(M, N, K, m16_takes(M, N, K, N, out_dtype, accumulate != 0));
+}
+
 extern "C" int mi8_gemm_num_variants(void) { return kNumVariants; }
 
 extern "C" const char* mi8_gemm_variant_name(int variant)
@@ -294,25 +324,9 @@ int gemm_fp8_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b
     GemmArgs g{(const uint8_t*)a, (const uint8_t*)b, out, out_dtype == MI8_F32 ? 1 : 0, lda, ldb, ldc, (int)M, (int)N, (int)K,
                sa, sb, sa_is_vector ? 1 : 0, sb_is_vector ? 1 : 0, 0, 0, accumulate ? 1 : 0};
     hipStream_t st = (hipStream_t)stream;
-    // (the persistent kernel shifts its last tile row / column back over the previous one when M or N is not a
-    // whole number of half tiles (128 x 256) and rewrites the overlap with identical values: not possible when accumulating)
-    // (its output stores address a tile's 256 rows with 32-bit byte offsets: ldc < 2^22)
-    const bool dma_ok = (K % 128 == 0) && M >= 256 && N >= 256 && N % 8 == 0 && ldc % 8 == 0 && ldc < (1 << 22) && aligned16(out) &&
-                        out_dtype == MI8_BF16 && (!sb_is_vector || aligned16(sb)) &&
-                        (sa_is_vector != 0) == (sb_is_vector != 0) && (!accumulate || (M % 128 == 0 && N % 256 == 0));
-    // A few rows of A: see choose_few_rows; everything else goes to whichever of the ring tile shapes and the persistent
-    // kernel the measured costs above say is fastest for this number of tiles and K steps (all of them give the same bits).
-    if (variant < 0) {
-        if (M <= kSkinnyMaxM) {  // (a caller that wants the planes asks for split K)
-            const FewRowsKernel few = choose_few_rows(M, N, K);
-            variant = few == kFewRows || (few == kFewPlanes && M <= 32) ? kSkinny : kEighths;
-        } else {
-            const int64_t steps = ceil_div(K, BK);
-            float cost;
-            variant = best_ring(M, N, steps, 1, &cost);
-            if (dma_ok && m16_cost(M, N, K) < cost) variant = kM16;
-        }
-    }
+    const bool dma_ok = m16_takes(M, N, K, ldc, out_dtype, accumulate) && aligned16(out) && (!sb_is_vector || aligned16(sb)) &&
+                        (sa_is_vector != 0) == (sb_is_vector != 0);
+    if (variant < 0) variant = chosen_variant(M, N, K, dma_ok);
     if (variant == kSkinny) return launch_skinny(g, a_dtype, b_dtype, st);
     if (variant == kM16) {
         MI8_REQUIRE(dma_ok, MI8_ERR_UNSUPPORTED,

@@ -76,6 +76,18 @@ def test_few_rows_slices():
                 assert L.mi8_gemm_splitk_suggest(m, n, 128 * steps - 16) in (1, -(-steps // per)), (m, n, steps)
 
 
+def test_variant_for():
+    """The kernel a product runs on: few rows, tiles too few or of the wrong kind for the persistent kernel, and its own."""
+    L = _C.lib()
+    name = lambda m, n, k, dt=_C.MI8_BF16, acc=0: L.mi8_gemm_variant_name(L.mi8_gemm_variant_for(m, n, k, dt, acc)).decode()  # noqa: E731
+    assert name(16, 4096, 4096) == "rows64x16_k8_m16x128" and name(64, 4096, 4096) == "64x64_ring4_eighths"
+    assert name(16384, 4096, 4096) == name(16384, 4096, 4096, acc=1) == name(16384, 4100 // 8 * 8, 4096) == "256x256_dma_w4x128_m16x128"
+    for args in ((300, 272, 144), (16384, 4096, 4112), (16384, 4096, 4096, _C.MI8_F32), (16383, 4096, 4096, _C.MI8_BF16, 1),
+                 (16384, 4104, 4096, _C.MI8_BF16, 1), (16384, 4100, 4096)):
+        assert "ring" in name(*args) and "eighths" not in name(*args), args
+    assert L.mi8_gemm_variant_for(0, 256, 256, _C.MI8_BF16, 0) == -1
+
+
 def test_host_only_shape_helpers():
     """Sizes and shape predicates the callers plan with (no GPU work)."""
     L = _C.lib()
@@ -108,6 +120,33 @@ def test_argument_validation_happens_before_any_gpu_call():
     assert L.mi8_amax_partials_batch(ptrs, ns, 2, 0, ctypes.c_void_p(16), None, None) == -1 and "tensor 0 is null" in _C.last_error()
     with pytest.raises(Exception):
         _C.check(-2, "x")
+
+
+def test_few_rows_entry_points_refuse():
+    """What the two launches of a generation step do not take, by their numbers alone (the pointers are never followed)."""
+    L, p, odd = _C.lib(), ctypes.c_void_p(256), ctypes.c_void_p(264)
+    n = ctypes.c_int32(0)
+
+    def swiglu(x=p, fp8=1, lda=256, sx=p, ldb=256, m=4, h=64, k=256, out=p):
+        return L.mi8_few_rows_swiglu(x, fp8, lda, sx, p, p, ldb, m, h, k, p, p, 0, out, p, n, None)
+
+    def cast_gemm(x=p, lda=256, slots=16, b=p, ldb=256, m=4, cols=64, k=256, out=p, ldc=64):
+        return L.mi8_few_rows_cast_gemm(x, lda, p, slots, b, ldb, m, cols, k, p, 0, out, ldc, None)
+
+    for call, code, kw, text in (
+        (swiglu, -1, dict(x=None), "null"), (swiglu, -1, dict(sx=None), "null"), (swiglu, -1, dict(out=None), "null"),
+        (swiglu, -2, dict(m=0), "rows"), (swiglu, -2, dict(m=65), "rows"), (swiglu, -2, dict(h=60), "H"), (swiglu, -2, dict(k=248), "K"),
+        (swiglu, -2, dict(h=16 * _C.AMAX_SLOTS + 8), "H"), (swiglu, -2, dict(lda=240), "pitches"), (swiglu, -2, dict(ldb=264), "pitches"),
+        (swiglu, -2, dict(x=odd), "aligned"), (swiglu, -2, dict(out=odd), "aligned"),
+        (swiglu, -2, dict(fp8=0, m=17, k=16, lda=16, ldb=16), "bf16"), (swiglu, -2, dict(fp8=0, lda=272, ldb=272), "bf16"),
+        (swiglu, -2, dict(fp8=0, m=16, k=1040, lda=1040, ldb=1040), "bf16"),
+        (cast_gemm, -1, dict(x=None), "null"), (cast_gemm, -1, dict(slots=0), "n_slots"), (cast_gemm, -1, dict(slots=_C.AMAX_SLOTS + 1), "n_slots"),
+        (cast_gemm, -2, dict(m=17), "rows"), (cast_gemm, -2, dict(cols=60), "N"), (cast_gemm, -2, dict(k=248), "K"),
+        (cast_gemm, -2, dict(m=16, k=4112, lda=4112, ldb=4112), "elements"), (cast_gemm, -2, dict(lda=252), "lda"),
+        (cast_gemm, -2, dict(ldb=264), "ldb"), (cast_gemm, -2, dict(ldc=56), "ldc"), (cast_gemm, -2, dict(ldc=66), "ldc"),
+        (cast_gemm, -2, dict(x=odd), "aligned"), (cast_gemm, -2, dict(b=odd), "aligned"),
+    ):
+        assert call(**kw) == code and text in _C.last_error(), (call.__name__, kw, _C.last_error())
 
 
 def test_grouped_pitch_limits():

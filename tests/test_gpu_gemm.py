@@ -327,8 +327,8 @@ def test_argument_errors(dev):
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
 def test_accumulating_gemm_equals_gemm_plus_add(dev, shape, vec, out_dtype):
     """out += product: the bits of `out + gemm(...)` on tensors of the output type (the new term rounded first, the
-    sum formed in float32 and rounded once), on the persistent kernel (full 256-tiles), on the general one, and for
-    shapes with few tiles and a long K, which the plain call sums in slices of K (the last two shapes)."""
+    sum formed in float32 and rounded once), on ring tiles and for shapes with few tiles and a long K, which the plain
+    call sums in slices of K (the last two shapes)."""
     M, N, K = shape
     a, b = seeded((M, K), 31, std=1e-3), seeded((N, K), 32)
     if vec:
@@ -424,8 +424,8 @@ HALF_SHAPES = [(4096, 2048, 256), (2048, 4352, 384), (2560, 2816, 128), (384, 51
 @pytest.mark.parametrize("mnk", HALF_SHAPES, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
 def test_half_tiles_of_the_persistent_kernel(dev, mnk, vec):
-    """The persistent kernel's plan of whole and half tiles against the ring tiles (same bits), with C += product where the
-    tiles do not overlap and, for single scales, the row-segment codes recorded by its epilogue."""
+    """The persistent kernel's plan of whole and half tiles against the ring tiles (same bits) and, for single scales, the
+    row-segment codes recorded by its epilogue."""
     M, N, K = mnk
     a, b = seeded((M, K), 91).to(E5M2).to(dev), seeded((N, K), 92).to(E4M3).to(dev)
     g = torch.Generator().manual_seed(93)
@@ -436,12 +436,31 @@ def test_half_tiles_of_the_persistent_kernel(dev, mnk, vec):
     want = ops.gemm_fp8(a, sa, b, sb, variant=ring)
     got = ops.gemm_fp8(a, sa, b, sb, variant=names.index("256x256_dma_w4x128_m16x128"))
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
-    first = seeded((M, N), 94).to(dev)
-    res = ops.gemm_fp8(a, sa, b, sb, out=first.clone(), accumulate=True, splits=1)
-    assert torch.equal(res, first + want)
     if not vec and ops.gemm_codes_supported(M, N, K):
         out, codes = ops.gemm_fp8_codes(a, sa, b, sb)
         assert torch.equal(out, want) and torch.equal(codes, ops.rowseg_max_codes(want))
+
+
+@pytest.mark.parametrize("mnk", [(2048, 8192, 2048), (4096, 2048, 4096), (1920, 8192, 2048), (2048, 11008, 2048)],
+                         ids=["whole", "halves", "whole+odd half row", "whole+halves"])
+@pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
+def test_persistent_kernel_accumulates_as_an_add(dev, mnk, vec):
+    """C += product on shapes that the library gives to the persistent kernel, on whole and on half tiles, also into a view
+    with a row pitch: the bits of the ring tiles' product and an elementwise add."""
+    M, N, K = mnk
+    names = ops.gemm_variants()
+    assert names[ops._C.lib().mi8_gemm_variant_for(M, N, K, ops._C.MI8_BF16, 1)] == "256x256_dma_w4x128_m16x128"
+    a, b = seeded((M, K), 91).to(E5M2).to(dev), seeded((N, K), 92).to(E4M3).to(dev)
+    g = torch.Generator().manual_seed(93)
+    sa = (torch.rand(M if vec else 1, generator=g) + 0.5).to(dev)
+    sb = (torch.rand(N if vec else 1, generator=g) + 0.5).to(dev)
+    first = seeded((M, N), 94, std=K ** 0.5).to(dev)
+    want = first + ops.gemm_fp8(a, sa, b, sb, variant=names.index("128x128_ring2"))
+    assert torch.equal(ops.gemm_fp8(a, sa, b, sb, out=first.clone(), accumulate=True), want)
+    wide = torch.full((M, N + 64), 7.0, dtype=torch.bfloat16, device=dev)
+    wide[:, :N] = first
+    ops.gemm_fp8(a, sa, b, sb, out=wide[:, :N], accumulate=True)
+    assert torch.equal(wide[:, :N], want) and bool((wide[:, N:] == 7.0).all())
 
 
 @pytest.mark.parametrize("mhk", [(4096, 1024, 256), (777, 1416, 384), (2048, 2176, 256)], ids=lambda s: "x".join(map(str, s)))

@@ -521,13 +521,13 @@ def test_grouped_dual_gemm_against_separate_products(dev, sizes):
 
 @pytest.mark.parametrize("accumulate", [False, True], ids=["", "accumulate"])
 @pytest.mark.parametrize("sizes,n,k", [
-    ([3, 0, 31, 1, 33, 0, 64, 32] * 6, 1024, 1024),   # tiles of 32 rows
-    ([64, 65, 0, 700, 63, 1] * 2, 512, 1792),         # of 64 rows
+    ([3, 0, 31, 1, 33, 0, 64, 32] * 6, 1024, 1024),   # tiles of 64 rows
+    ([64, 65, 0, 700, 63, 1] * 2, 512, 1792),         # of 32 rows
     ([130, 0, 2900, 1000], 1024, 1792),               # of 128 rows
     ([300, 0, 17, 20000, 9700], 320, 384),            # the persistent kernel, its last tile column shifted
     ([7000, 255, 0, 257, 9000], 1024, 1024),          # the persistent kernel
     ([40, 0, 301], 264, 144),                         # no multiple of a step
-], ids=["32", "64", "128", "persistent-shifted", "persistent", "ragged-k"])
+], ids=["64", "32", "128", "persistent-shifted", "persistent", "ragged-k"])
 def test_grouped_gemm_choice_exact_integers(dev, sizes, n, k, accumulate):
     """Integer operands and power-of-two scales: the product is exact in float32 whichever kernel the sizes lead to, so
     the result is its bf16 rounding (accumulating: the bf16 sum of that and the old value), and rows of no group stay."""
