@@ -13,13 +13,13 @@ namespace mi8 {
 using namespace gemm;
 namespace {
 
-template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP, bool SLICED>
-__global__ __launch_bounds__(kRingThreads, OCC) void gemm_fp8_ring_kernel(GemmArgs g)
+template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP, bool SLICED, int NW>
+__global__ __launch_bounds__(NW * 64, OCC) void gemm_fp8_ring_kernel(GemmArgs g)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     int tm, tn;
     if (!tile_of_block(g, tm, tn)) return;
-    ring_tile<BM, BN, ST, CBSZ, BLGP, SLICED>(g, tm * BM, tn * BN, lds);
+    ring_tile<BM, BN, ST, CBSZ, BLGP, SLICED, NW>(g, tm * BM, tn * BN, lds);
 }
 
 // ---- split K ---------------------------------------------------------------------------------------
@@ -114,15 +114,21 @@ struct RingShape {
     float tile;   // us per tile outside the K loop
 };
 
-// (measured on shapes from 300 x 2048 x 768 to 4096 x 2048 x 8192; the model below meets them within 15 %)
+// (measured on shapes from 300 x 2048 x 768 to 16384 x 11008 x 4112; the model below meets them within 15 %, products that
+// the stores bound aside)
 constexpr RingShape kRing[] = {
     {"64x64_ring4", 64, 64, 0.28f, 0.39f, 1.2f},
     {"128x64_ring3", 128, 64, 0.40f, 0.64f, 1.2f},
     {"64x128_ring3", 64, 128, 0.40f, 0.64f, 1.2f},
     {"128x128_ring2", 128, 128, 0.72f, 1.0f, 1.5f},
     {"128x128_ring3", 128, 128, 0.60f, 0.0f, 1.5f},
+    // Eight waves, for the large products that the persistent kernel does not take: a quarter of the barriers and half the
+    // operand bytes of 128 x 128 tiles.  us, 128x128_ring2 / this: 16384 x 4096 x 11024 834 / 601, 16384 x 11008 x 4112 865 / 676,
+    // 4096 x 4096 x 4112 84 / 63, 3000 x 3000 x 4112 in float32 76 / 57, 16384 x 11008 x 4096 in float32 734 / 671.
+    {"256x256_ring2", 256, 256, 1.6f, 0.0f, 5.0f},
 };
 constexpr int kNumRing = sizeof(kRing) / sizeof(kRing[0]);
+constexpr int kRing256 = kNumRing - 1;  // never cut along K
 constexpr float kLaunchUs = 2.6f;
 
 // time of a problem of `slices` independent slices of `steps` K steps on tile shape r, launch included
@@ -136,11 +142,12 @@ float ring_cost(const RingShape& r, int64_t M, int64_t N, int64_t steps, int64_t
     return kLaunchUs + (work > stores ? work : stores);
 }
 
+// the fastest of the four-wave shapes
 int best_ring(int64_t M, int64_t N, int64_t steps, int64_t slices, float* cost)
 {
     int best = 0;
     float c = 0.0f;
-    for (int i = 0; i < kNumRing; ++i) {
+    for (int i = 0; i < kRing256; ++i) {
         const float t = ring_cost(kRing[i], M, N, steps, slices);
         if (i == 0 || t < c) {
             best = i;
@@ -212,14 +219,14 @@ constexpr int kM16 = kNumRing, kSkinny = kNumRing + 1, kEighths = kNumRing + 2, 
 
 template <typename Args, typename Kernel>
 int launch_ring_kernel(Kernel kern, std::atomic<uint64_t>& configured, int lds_bytes, const Args& a, int tiles, int slices,
-                       hipStream_t st, const char* what)
+                       int threads, hipStream_t st, const char* what)
 {
     if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, configured, what)) return rc;
-    hipLaunchKernelGGL(kern, dim3((tiles + 7) / 8 * 8, slices), dim3(kRingThreads), lds_bytes, st, a);
+    hipLaunchKernelGGL(kern, dim3((tiles + 7) / 8 * 8, slices), dim3(threads), lds_bytes, st, a);
     return launch_status(what);
 }
 
-template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP, bool SLICED = false>
+template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP, bool SLICED = false, int NW = kRingThreads / 64>
 int launch_ring(GemmArgs& g, SplitArgs* split, hipStream_t st)
 {
     GemmArgs& p = split ? split->g : g;
@@ -227,11 +234,12 @@ int launch_ring(GemmArgs& g, SplitArgs* split, hipStream_t st)
     p.tiles_n = (p.N + BN - 1) / BN;
     const int tiles = p.tiles_m * p.tiles_n;
     static std::atomic<uint64_t> configured[2];
-    if (split)
-        return launch_ring_kernel(gemm_fp8_splitk_kernel<BM, BN, ST, OCC, CBSZ, BLGP>, configured[1], kRingLdsBytes<BM, BN, ST>,
-                                  *split, tiles, split->splits, st, "mi8_gemm_fp8_splitk");
-    return launch_ring_kernel(gemm_fp8_ring_kernel<BM, BN, ST, OCC, CBSZ, BLGP, SLICED>, configured[0], kRingLdsBytes<BM, BN, ST>, g,
-                              tiles, 1, st, "mi8_gemm_fp8");
+    if constexpr (NW * 64 == kRingThreads)  // (slices are for problems of few tiles: none of the larger workgroups' business)
+        if (split)
+            return launch_ring_kernel(gemm_fp8_splitk_kernel<BM, BN, ST, OCC, CBSZ, BLGP>, configured[1], kRingLdsBytes<BM, BN, ST>,
+                                      *split, tiles, split->splits, kRingThreads, st, "mi8_gemm_fp8_splitk");
+    return launch_ring_kernel(gemm_fp8_ring_kernel<BM, BN, ST, OCC, CBSZ, BLGP, SLICED, NW>, configured[0], kRingLdsBytes<BM, BN, ST>,
+                              g, tiles, 1, NW * 64, st, "mi8_gemm_fp8");
 }
 
 template <int CBSZ, int BLGP>
@@ -243,6 +251,7 @@ int launch_ring_shape(int shape, GemmArgs& g, SplitArgs* split, hipStream_t st)
         case 2: return launch_ring<64, 128, 3, 2, CBSZ, BLGP>(g, split, st);
         case 3: return launch_ring<128, 128, 2, 2, CBSZ, BLGP>(g, split, st);
         case 4: return launch_ring<128, 128, 3, 1, CBSZ, BLGP>(g, split, st);
+        case kRing256: return launch_ring<256, 256, 2, 1, CBSZ, BLGP, false, 8>(g, nullptr, st);
         case kEighths: g.slice_steps = eighth_steps(g.K); return launch_ring<64, 64, 4, 2, CBSZ, BLGP, true>(g, nullptr, st);
     }
     set_error("mi8_gemm_fp8: unknown variant %d", shape);
@@ -280,8 +289,12 @@ int chosen_variant(int64_t M, int64_t N, int64_t K, bool m16_fits)
         return few == kFewRows || (few == kFewPlanes && M <= 32) ? kSkinny : kEighths;
     }
     float cost;
-    const int ring = best_ring(M, N, ceil_div(K, BK), 1, &cost);
-    return m16_fits && m16_cost(M, N, K) < cost ? kM16 : ring;
+    const int64_t steps = ceil_div(K, BK);
+    const int ring = best_ring(M, N, steps, 1, &cost);
+    if (m16_fits) return m16_cost(M, N, K) < cost ? kM16 : ring;
+    // (rows that do not start on a cache line cost the small tiles, which read them more often, a quarter more, the large
+    // ones 5-7 %: 16384 x 4096 x 11008 and 11024, 616 and 834 us, 550 and 601)
+    return ring_cost(kRing[kRing256], M, N, steps, 1) < (K % BK ? 1.25f : 1.0f) * cost ? kRing256 : ring;
 }
 }  // namespace
 

@@ -4,7 +4,7 @@
 // What bounds it: these are products with fewer tiles than fill the chip once or twice at 256 x 256, so a tile's time is
 // latency (the first operand bytes, one barrier and one LDS round trip per 128-byte K step, the epilogue) and, once two
 // workgroups share a compute unit, the operand bytes that come out of L2: (BM + BN) * 128 per step at about 80 B/ns and
-// compute unit.  Hence small tiles (64 or 128 on a side, four waves of (BM / 2) x (BN / 2)), operands that go from L2
+// compute unit.  Hence small tiles (32 to 128 rows by 64 or 128 columns, four waves of (BM / 2) x (BN / 2)), operands that go from L2
 // straight to LDS (buffer loads with the LDS destination, no registers and no vector address arithmetic: one resident
 // lane offset per load and a uniform K offset), a ring of ST stages so that ST - 1 steps are in flight, and an LDS
 // footprint that lets two workgroups live on a compute unit, one computing while the other waits.
@@ -50,11 +50,12 @@ constexpr int kRingThreads = 256;
 
 // C[m0 .. m0 + BM, n0 .. n0 + BN] of g's product (K may be 0: zeros).  g.sa == null: the raw fp32 sums are wanted.
 // SLICED: K is summed in slices of g.slice_steps, each from zero, added in order (the sums of split K without its planes).
-template <int BM, int BN, int ST, int CBSZ, int BLGP, bool SLICED = false>
+// NW waves, two of them side by side along M.
+template <int BM, int BN, int ST, int CBSZ, int BLGP, bool SLICED = false, int NW = kRingThreads / 64>
 __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const int n0, uint8_t* lds)
 {
-    constexpr int NW = kRingThreads / 64;
-    constexpr int WTM = BM / 2, WTN = BN / 2;  // wave tile
+    constexpr int WAVES_N = NW / 2;
+    constexpr int WTM = BM / 2, WTN = BN / WAVES_N;  // wave tile
     constexpr int TM = WTM / 16, TN = WTN / 16;
     constexpr int STAGE = (BM + BN) * BK;
     constexpr int LA = BM / 8 / NW, LB = BN / 8 / NW, LD = LA + LB;  // loads per wave and step: 8 rows x 128 bytes each
@@ -62,10 +63,10 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / WAVES_N, wn = wave % WAVES_N;
     const int r16 = lane & 15, kb = lane >> 4;
 
-    // ---- operand loads: load i of wave w fills rows 8 (4 i + w) .. + 7; rows past the edge re-read the last one
+    // ---- operand loads: load i of wave w fills rows 8 (NW i + w) .. + 7; rows past the edge re-read the last one
     const int rows_a = g.M - m0 < BM ? g.M - m0 : BM, rows_b = g.N - n0 < BN ? g.N - n0 : BN;
     const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(g.A + (int64_t)m0 * g.lda), 0, (int)(uint32_t)((int64_t)(rows_a - 1) * g.lda + g.K), 0x00020000);
@@ -272,25 +273,31 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
     uint16_t* C = reinterpret_cast<uint16_t*>(g.C);
     // bf16 rows leave through LDS (the ring is free now): whole row segments of the wave tile, 16 bytes per lane
     constexpr int PITCH = WTN * 2 + 16;  // (the pad spreads the rows of a store over the banks)
-    static_assert(NW * WTM * PITCH <= ST * STAGE, "output staging");
+    constexpr int SR = NW * WTM * PITCH <= ST * STAGE ? WTM : WTM / 2;  // rows of the wave tile staged at a time
+    static_assert(NW * SR * PITCH <= ST * STAGE, "output staging");
     __syncthreads();
-    uint8_t* stg = lds + wave * (WTM * PITCH);
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-            *reinterpret_cast<uint2*>(stg + (16 * i + r16) * PITCH + (16 * j + 4 * kb) * 2) =
-                make_uint2(pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3]));
+    uint8_t* stg = lds + wave * (SR * PITCH);
     constexpr int LPR = WTN / 8, RPI = 64 / LPR;  // lanes per row, rows per store
 #pragma unroll
-    for (int it = 0; it < WTM / RPI; ++it) {
-        const int rw = it * RPI + lane / LPR, c8 = (lane % LPR) * 8;
-        v4i v = *reinterpret_cast<const v4i*>(stg + rw * PITCH + c8 * 2);
-        const int row = m0 + wm * WTM + rw, col = n0 + wn * WTN + c8;
-        if (row < g.M && col < g.N) {
-            v4i* c = reinterpret_cast<v4i*>(C + (int64_t)row * g.ldc + col);
-            if (g.accumulate) v = add_bf16x8(v, *c);
-            *c = v;
+    for (int part = 0; part < WTM / SR; ++part) {
+#pragma unroll
+        for (int i = 0; i < SR / 16; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const ring_v4f v = acc[part * (SR / 16) + i][j];
+                *reinterpret_cast<uint2*>(stg + (16 * i + r16) * PITCH + (16 * j + 4 * kb) * 2) =
+                    make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+            }
+#pragma unroll
+        for (int it = 0; it < SR / RPI; ++it) {
+            const int rw = it * RPI + lane / LPR, c8 = (lane % LPR) * 8;
+            v4i v = *reinterpret_cast<const v4i*>(stg + rw * PITCH + c8 * 2);
+            const int row = m0 + wm * WTM + part * SR + rw, col = n0 + wn * WTN + c8;
+            if (row < g.M && col < g.N) {
+                v4i* c = reinterpret_cast<v4i*>(C + (int64_t)row * g.ldc + col);
+                if (g.accumulate) v = add_bf16x8(v, *c);
+                *c = v;
+            }
         }
     }
 }

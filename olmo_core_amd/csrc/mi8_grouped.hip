@@ -71,8 +71,8 @@ struct GroupedWgradArgs {
     int tiles_n, tiles_k;
 };
 
-template <int BM, int BN, int ST, int CBSZ, int BLGP>
-__global__ __launch_bounds__(kRingThreads, 2) void grouped_wgrad_kernel(GroupedWgradArgs a)
+template <int BM, int BN, int ST, int CBSZ, int BLGP, int NW>
+__global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void grouped_wgrad_kernel(GroupedWgradArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int per_group = a.tiles_n * a.tiles_k;
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(kRingThreads, 2) void grouped_wgrad_kernel(GroupedW
     g.sa_vec = seg ? 1 : 0;
     g.sb_vec = seg ? 1 : 0;
     g.accumulate = 0;
-    ring_tile<BM, BN, ST, CBSZ, BLGP>(g, tn * BM, tk * BN, lds);
+    ring_tile<BM, BN, ST, CBSZ, BLGP, false, NW>(g, tn * BM, tk * BN, lds);
 }
 
 template <int BM, int BN, int ST, int CBSZ, int BLGP>
@@ -153,10 +153,10 @@ int launch_grouped_shape(GroupedArgs& a, GroupedKernel k, hipStream_t st)
     return launch_grouped<128, 128, 2, CBSZ, BLGP>(a, st);
 }
 
-template <int BM, int BN, int ST, int CBSZ, int BLGP>
+template <int BM, int BN, int ST, int CBSZ, int BLGP, int NW = kRingThreads / 64>
 int launch_wgrad(GroupedWgradArgs& a, hipStream_t st)
 {
-    auto kern = grouped_wgrad_kernel<BM, BN, ST, CBSZ, BLGP>;
+    auto kern = grouped_wgrad_kernel<BM, BN, ST, CBSZ, BLGP, NW>;
     static std::atomic<uint64_t> configured{0};
     if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), kRingLdsBytes<BM, BN, ST>, configured, "mi8_grouped_wgrad_fp8"))
         return rc;
@@ -164,16 +164,22 @@ int launch_wgrad(GroupedWgradArgs& a, hipStream_t st)
     a.tiles_k = (a.Kl + BN - 1) / BN;
     const int64_t blocks = (int64_t)a.E * a.tiles_n * a.tiles_k;
     MI8_REQUIRE(blocks < ((int64_t)1 << 31), MI8_ERR_UNSUPPORTED, "mi8_grouped_wgrad_fp8: grid too large");
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kRingThreads), (kRingLdsBytes<BM, BN, ST>), st, a);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * 64), (kRingLdsBytes<BM, BN, ST>), st, a);
     return launch_status("mi8_grouped_wgrad_fp8");
 }
 
-// small tiles until the large ones would put two workgroups on every compute unit
+// Small tiles until the middle ones would put two workgroups on every compute unit; the large ones, eight waves each, where
+// they fill the chip four times (groups differ in length, and fewer rounds do not even that out) and do not pad much more
+// than the middle ones.  us on middle / large tiles, float32: 131072 rows in 64 groups, 2048 x 1024 555 / 477, 1024 x 2048 531 / 488,
+// 512 x 1024 (two rounds) 239 / 380, 264 x 4096 (a third more padding) 342 / 387; 65536 rows in 16 groups, 1800 x 2048 351 / 313.
 template <int CBSZ, int BLGP>
 int launch_wgrad_shape(GroupedWgradArgs& a, hipStream_t st)
 {
-    if ((int64_t)a.E * ceil_div(a.N, 128) * ceil_div(a.Kl, 128) < 512) return launch_wgrad<64, 64, 4, CBSZ, BLGP>(a, st);
-    return launch_wgrad<128, 128, 2, CBSZ, BLGP>(a, st);
+    const int64_t middle = (int64_t)a.E * ceil_div(a.N, 128) * ceil_div(a.Kl, 128);
+    const int64_t large = (int64_t)a.E * ceil_div(a.N, 256) * ceil_div(a.Kl, 256);
+    if (middle < 512) return launch_wgrad<64, 64, 4, CBSZ, BLGP>(a, st);
+    if (large < 1024 || 4 * large * 5 > middle * 6) return launch_wgrad<128, 128, 2, CBSZ, BLGP>(a, st);
+    return launch_wgrad<256, 256, 2, CBSZ, BLGP, 8>(a, st);
 }
 
 bool fp8_code(int v) { return v == MI8_E4M3 || v == MI8_E5M2; }

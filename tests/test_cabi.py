@@ -85,6 +85,9 @@ def test_variant_for():
     for args in ((300, 272, 144), (16384, 4096, 4112), (16384, 4096, 4096, _C.MI8_F32), (16383, 4096, 4096, _C.MI8_BF16, 1),
                  (16384, 4104, 4096, _C.MI8_BF16, 1), (16384, 4100, 4096)):
         assert "ring" in name(*args) and "eighths" not in name(*args), args
+    # ... those of them that are large on the tiles with the persistent kernel's operand traffic
+    for args in ((16384, 11008, 4112), (16384, 4096, 11024), (8192, 5120, 27648, _C.MI8_F32), (16383, 4096, 11008, _C.MI8_BF16, 1)):
+        assert name(*args) == "256x256_ring2", args
     assert L.mi8_gemm_variant_for(0, 256, 256, _C.MI8_BF16, 0) == -1
 
 

@@ -357,11 +357,11 @@ def test_accumulating_gemm_equals_gemm_plus_add(dev, shape, vec, out_dtype):
         ops.gemm_fp8(aq, sa, bq, sb, out_dtype=out_dtype, accumulate=True)
 
 
-RING = [n for n in ("64x64_ring4", "128x64_ring3", "64x128_ring3", "128x128_ring2", "128x128_ring3")]
+RING = [n for n in ("64x64_ring4", "128x64_ring3", "64x128_ring3", "128x128_ring2", "128x128_ring3", "256x256_ring2")]
 
 
 @pytest.mark.parametrize("name", RING)
-@pytest.mark.parametrize("mnk", [(1, 1, 16), (63, 65, 128), (65, 127, 144), (129, 136, 240), (128, 128, 384), (200, 72, 656)],
+@pytest.mark.parametrize("mnk", [(1, 1, 16), (63, 65, 128), (65, 127, 144), (129, 136, 240), (128, 128, 384), (200, 72, 656), (255, 257, 144), (513, 264, 272)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_ring_tiles_at_their_edges(dev, name, mnk):
     """The ring tile shapes one row / column / K step around their tile sizes: K shorter than a step, a ragged last step
@@ -461,6 +461,20 @@ def test_persistent_kernel_accumulates_as_an_add(dev, mnk, vec):
     wide[:, :N] = first
     ops.gemm_fp8(a, sa, b, sb, out=wide[:, :N], accumulate=True)
     assert torch.equal(wide[:, :N], want) and bool((wide[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+@pytest.mark.parametrize("mnk", [(4000, 4096, 2064), (3999, 4091, 2064)], ids=lambda s: "x".join(map(str, s)))
+def test_large_ring_tiles_accumulate_as_an_add(dev, mnk, dt):
+    """C += product on the eight-wave tiles that large products of other shapes than the persistent kernel's run on."""
+    M, N, K = mnk
+    names = ops.gemm_variants()
+    assert names[ops._C.lib().mi8_gemm_variant_for(M, N, K, ops._HP_CODE[dt], 1)] == "256x256_ring2"
+    a, b = seeded((M, K), 91).to(E5M2).to(dev), seeded((N, K), 92).to(E4M3).to(dev)
+    sa, sb = (torch.rand(n, generator=torch.Generator().manual_seed(n)).to(dev) + 0.5 for n in (M, N))
+    first = seeded((M, N), 94, std=K ** 0.5).to(dt).to(dev)
+    want = first + ops.gemm_fp8(a, sa, b, sb, out_dtype=dt, variant=names.index("128x128_ring2"))
+    assert torch.equal(ops.gemm_fp8(a, sa, b, sb, out_dtype=dt, out=first.clone(), accumulate=True), want)
 
 
 @pytest.mark.parametrize("mhk", [(4096, 1024, 256), (777, 1416, 384), (2048, 2176, 256)], ids=lambda s: "x".join(map(str, s)))

@@ -151,6 +151,29 @@ def test_grouped_wgrad_exact_integers(dev, sizes):
         start += m
 
 
+@pytest.mark.parametrize("N,Kl", [(1000, 1004), (770, 1022)], ids=["1000x1004", "770x1022"])
+def test_grouped_wgrad_large_tiles_exact_integers(dev, N, Kl):
+    """Enough float32 weight gradients for the 256 x 256 tiles, partial ones in both directions: sizes that are and are not
+    whole 16-byte chunks, groups of one step, of several and of none."""
+    E = 64 if N == 1000 else 90
+    sizes = [(37 * e) % 150 if e % 7 else 0 for e in range(E)]
+    sizes[5] = 700
+    T = sum(sizes)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    sz = torch.tensor(sizes).to(dev)
+    go, x = (torch.randint(-2, 3, (T, n), generator=g, device=dev).float() for n in (N, Kl))
+    ld = ops._C.lib().mi8_grouped_padded_rows(T, E)
+    rows = torch.cat([torch.arange(m) + s for m, s in zip(sizes, _padded_starts(sizes))]).to(dev)
+    got, xt = (torch.zeros(n, ld, device=dev).index_copy_(1, rows, v.t().contiguous()) for n, v in ((N, go), (Kl, x)))
+    ones = torch.ones(E, max(N, Kl), device=dev)
+    out = ops.grouped_wgrad_fp8(got.to(E4M3), ones[:, :N].contiguous(), xt.to(E4M3), ones[:, :Kl].contiguous(), sz, tokens=T,
+                                out_dtype=torch.float32)
+    start = 0
+    for e, m in enumerate(sizes):
+        assert torch.equal(out[e], go[start:start + m].t() @ x[start:start + m]), f"group {e} (size {m})"
+        start += m
+
+
 # group-size lists for the full-tile (256 x 256, persistent) kernels: T >= 256 with groups that end inside a
 # tile, empty groups, a group larger than two tiles, a last tile that is shifted back to stay inside the matrix
 BIG_SIZE_CASES = [
