@@ -112,7 +112,8 @@ def linear(x2: torch.Tensor, weight: torch.Tensor, cfg_id: int, weight_scale: Op
 # ---- the fused SwiGLU feed-forward block (olmo_core_amd.nn.feed_forward) ------------------------------------------
 # One operator forward, one backward: a compiled transformer block keeps the launches the eager block makes (both
 # input projections and the activation in one GEMM launch, the amax of the gate gradients from row-segment codes, the
-# accumulating grad_x epilogue), bit for bit.  The forward returns y and the 13 tensors the backward takes.
+# accumulating grad_x epilogue), bit for bit.  The forward returns y and the 13 tensors the backward takes.  (Without
+# gradients the eager block makes fewer launches still, with the same bits; this one makes those of a training forward.)
 
 _N_SAVED = 13
 
