@@ -269,7 +269,8 @@ def gemm_fp8(
     ``a`` and ``b`` are fp8 tensors whose rows are K-contiguous; ``sa`` / ``sb`` hold one scale or one per row.
     ``out``: an ``[M, N]`` tensor of ``out_dtype`` with contiguous rows (any row pitch) to write into.
     ``splits``: slices of K summed separately and added afterwards (for problems with few output tiles);
-    -1 lets the library decide from the shape, 0 and 1 forbid splitting; a forced ``variant`` is never split.
+    -1 lets the library decide from the shape, 0 and 1 forbid splitting; a forced ``variant`` is never split.  More of them
+    than K has steps of 128 (or than 64) are refused; ``accumulate`` sums such a product unsplit.
     """
     _require_gpu(a, "gemm_fp8")
     if a.dim() != 2 or b.dim() != 2 or a.stride(1) != 1 or b.stride(1) != 1:
@@ -300,6 +301,8 @@ def gemm_fp8(
         splits = 1
     elif splits < 0:
         splits = L.mi8_gemm_splitk_suggest(M, N, K)
+    elif accumulate and splits > min(64, -(-K // 128)):
+        splits = 1
     if accumulate and splits <= 1:
         _C.check(
             L.mi8_gemm_fp8_accumulate(

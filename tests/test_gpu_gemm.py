@@ -534,15 +534,15 @@ def test_few_rows_sum_in_eighths(dev, mnk, vec):
                 assert torch.equal(ops.gemm_fp8(a, sa, b, sb, out_dtype=dt, out=first.clone(), accumulate=True, **kw), first + want), kw
 
 
-@pytest.mark.parametrize("splits", [-1, 0, 1, 3])
+@pytest.mark.parametrize("splits", [-1, 0, 1, 3, 100])
 def test_accumulating_keeps_what_out_holds(dev, splits):
-    """C += product for every value of `splits` (0: not split), on shapes with and without slices of their own."""
+    """C += product for every value of `splits` (0, and more than K has steps: not split), on shapes with and without slices
+    of their own."""
     for M, N, K in ((100, 200, 1040), (300, 272, 144), (16, 64, 512)):
         a, b = _int_operand((M, K), 1, E4M3).to(dev), _int_operand((N, K), 2, E4M3).to(dev)
         one, first = torch.ones(1, device=dev), _int_operand((M, N), 3, torch.float32).to(dev)
-        if splits <= -(-K // 128):
-            got = ops.gemm_fp8(a, one, b, one, out_dtype=torch.float32, out=first.clone(), accumulate=True, splits=splits)
-            assert torch.equal(got, first + a.float() @ b.float().t())
+        got = ops.gemm_fp8(a, one, b, one, out_dtype=torch.float32, out=first.clone(), accumulate=True, splits=splits)
+        assert torch.equal(got, first + a.float() @ b.float().t())
 
 
 @pytest.mark.parametrize("name", RING)
