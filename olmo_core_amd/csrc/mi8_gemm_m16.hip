@@ -986,8 +986,9 @@ namespace {
 
 // Which tiles of a dense problem are halves (tiles_n columns of tiles, nk K steps), and g.tiles_m = pairs of half rows.
 // Splitting tiles of a partial last round pays when its halves fit into one round: 2048 x 11008 x 4096 is 344 tiles, two
-// rounds of 256 workgroups for 1.34 rounds of work; as 256 whole and 176 half tiles it takes 79 us instead of 84.
-// 4096 x 2048 x 8192, 128 tiles, is 256 half tiles: 59 us instead of 76.  (A step of a half tile takes 0.65 us with its
+// rounds of 256 workgroups for 1.34 rounds of work; as 256 whole and 176 half tiles it takes 81 us in a loop of its own
+// (92 right after the casts that write its operands) instead of 87.  4096 x 2048 x 8192, 128 tiles, is 256 half tiles: 55 us
+// instead of 69.  The matrix pipe is busy 68 % and 67 % of the cycles.  (A step of a half tile takes 0.65 us with its
 // operands in the memory-side cache, 0.85 us from HBM; a whole tile's 1.0 us, 1.35 us when all compute units have one.)
 HalfRows plan_halves(GemmArgs& g, const int cus, int most_halves = 1 << 30)
 {

@@ -11,8 +11,11 @@
 //
 // The MFMA (v_mfma_f32_16x16x128_f8f6f4), the order of K and the scale arithmetic are those of the persistent kernel: a
 // product has the same bits on either.  Measured against the register-staged 128 x 128 tiles that were here before
-// (32x32x64 MFMAs, split along K where tiles were few), us per launch in a graph: 305 x 2816 x 1024 15.7 -> 5.6,
-// 1537 x 2048 x 2048 25.7 -> 12.3, 1999 x 1024 x 2816 23.4 -> 12.2, 512 x 4096 x 4096 27.9 -> 15.6.
+// (32x32x64 MFMAs, split along K where tiles were few), us per launch in a graph: 305 x 2816 x 1024 15.0 -> 6.3,
+// 1537 x 2048 x 2048 26.4 -> 15.5 (17.5 beside the casts of a training step), 1999 x 1024 x 2816 23.5 -> 11.6,
+// 512 x 4096 x 4096 26.8 -> 15.0.  Counters: 24 % of the matrix pipe's cycles busy at 1537 x 2048 x 2048, 34 % at
+// 777 x 4096 x 11008 (one workgroup to a unit: its LDS reads come between a barrier and the MFMAs), bank conflicts 2-8 % of
+// the LDS cycles, operands fetched into L2 3.3 and 2.1 times; 256 x 256 tiles at 16384 x 4096 x 11024: 59 %, 2 %, 4.8 times.
 //
 // LDS stage: [row][128 bytes], A rows then B rows; 16-byte chunk c of row r sits at c ^ swz16(r) (the swizzle of the
 // persistent kernel), applied by permuting which global chunk a lane fetches.
