@@ -215,8 +215,8 @@ int mi8_gemm_fp8_swiglu(const void* a, int a_dtype, int64_t lda, const void* b1,
  * caller, free for reuse once the call's work on `stream` is done.  mi8_gemm_splitk_suggest returns the number
  * of slices the library would use for a shape (1: call mi8_gemm_fp8 instead).  Up to 64 rows K is summed in eighths
  * (slices of ceil(ceil(K / 128) / 8) steps) whichever entry point or kernel runs, mi8_few_rows_* included, so all of
- * them give one result; asked for those slices, mi8_gemm_fp8_splitk may add them without planes (the workspace is then
- * not touched).  No counterpart upstream: the reference leaves the choice of GEMM algorithm to torch._scaled_mm's backend. */
+ * them give one result.  Where one workgroup per tile adds the slices sooner, mi8_gemm_fp8_splitk does it that way (the
+ * same sums; the workspace is then not touched).  No counterpart upstream: the reference leaves the choice of GEMM algorithm to torch._scaled_mm's backend. */
 int mi8_gemm_fp8_splitk(const void* a, int a_dtype, int64_t lda, const void* b, int b_dtype, int64_t ldb,
                         int64_t M, int64_t N, int64_t K, const float* sa, int sa_is_vector, const float* sb,
                         int sb_is_vector, void* out, int out_dtype, int64_t ldc, int splits, void* workspace,

@@ -109,26 +109,28 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(SplitArgs a)
 struct RingShape {
     const char* name;
     int bm, bn;
-    float step1;  // us per 128-byte K step with one workgroup on a compute unit ...
-    float step2;  // ... and for a pair of them sharing one (0: only one fits)
-    float tile;   // us per tile outside the K loop
+    float step0, step1;  // us per 128-byte K step with one workgroup on a compute unit: few units busy .. all of them
+    float step2;         // ... and for a pair of them sharing one (0: only one fits)
+    float tile;          // us per tile outside the K loop
+    float many, many_tile;  // step (of one or of the pair) and tile where units get three tiles and more: operands from further away
 };
 
-// (measured on shapes from 300 x 2048 x 768 to 16384 x 11008 x 4112; the model below meets them within 15 %, products that
-// the stores bound aside)
+// (fitted to 113 products each, 65 x 768 x 2048 to 1999 x 5632 x 1024 and 700 x 5120 x 27648, which the model below meets
+// within 5-8 % rms, the shape it picks on average 1 % behind the fastest; the last two to products up to 16384 x 11008 x 4112)
 constexpr RingShape kRing[] = {
-    {"64x64_ring4", 64, 64, 0.28f, 0.39f, 1.2f},
-    {"128x64_ring3", 128, 64, 0.40f, 0.64f, 1.2f},
-    {"64x128_ring3", 64, 128, 0.40f, 0.64f, 1.2f},
-    {"128x128_ring2", 128, 128, 0.72f, 1.0f, 1.5f},
-    {"128x128_ring3", 128, 128, 0.60f, 0.0f, 1.5f},
+    {"64x64_ring4", 64, 64, 0.113f, 0.181f, 0.335f, 1.33f, 0.39f, 1.2f},
+    {"128x64_ring3", 128, 64, 0.169f, 0.294f, 0.524f, 1.67f, 0.64f, 1.2f},
+    {"64x128_ring3", 64, 128, 0.171f, 0.295f, 0.533f, 1.72f, 0.64f, 1.2f},
+    {"128x128_ring2", 128, 128, 0.543f, 0.639f, 0.918f, 1.62f, 1.0f, 1.5f},
+    {"128x128_ring3", 128, 128, 0.267f, 0.45f, 0.0f, 3.0f, 0.60f, 1.5f},
     // Eight waves, for the large products that the persistent kernel does not take: a quarter of the barriers and half the
     // operand bytes of 128 x 128 tiles.  us, 128x128_ring2 / this: 16384 x 4096 x 11024 834 / 601, 16384 x 11008 x 4112 865 / 676,
     // 4096 x 4096 x 4112 84 / 63, 3000 x 3000 x 4112 in float32 76 / 57, 16384 x 11008 x 4096 in float32 734 / 671.
-    {"256x256_ring2", 256, 256, 1.6f, 0.0f, 5.0f},
+    {"256x256_ring2", 256, 256, 1.6f, 1.6f, 0.0f, 5.0f, 1.6f, 5.0f},
 };
 constexpr int kNumRing = sizeof(kRing) / sizeof(kRing[0]);
 constexpr int kRing256 = kNumRing - 1;  // never cut along K
+constexpr int kRingLastSliced = 2;      // (128 x 128 tiles have no registers left for a second set of sums)
 constexpr float kLaunchUs = 2.6f;
 
 // time of a problem of `slices` independent slices of `steps` K steps on tile shape r, launch included
@@ -136,18 +138,23 @@ float ring_cost(const RingShape& r, int64_t M, int64_t N, int64_t steps, int64_t
 {
     const int64_t tiles = ((M + r.bm - 1) / r.bm) * ((N + r.bn - 1) / r.bn) * slices;
     const int64_t per_cu = (tiles + 255) / 256;
-    const float work = per_cu == 1 || r.step2 == 0.0f ? per_cu * (steps * r.step1 + r.tile) : 0.5f * per_cu * (steps * r.step2 + r.tile);
+    const float busy = (float)tiles / 256.0f;  // (the units share what the L2s deliver)
+    const float tile = per_cu > 2 ? r.many_tile : r.tile;
+    const float alone = per_cu > 2 ? r.many : r.step0 + (r.step1 - r.step0) * (busy < 1.0f ? busy : 1.0f);
+    const float pair = per_cu > 2 ? r.many : r.step2;
+    const float work = per_cu == 1 || r.step2 == 0.0f ? per_cu * (steps * alone + tile) : 0.5f * per_cu * (steps * pair + tile);
     // A short K leaves the stores: these kernels write 3.2 MB a us (27648 x 5120 x 256: 91-100 us, the persistent kernel 66-76).
     const float stores = (float)(M * N) * (slices > 1 ? 4.0f * slices : 2.0f) / 3.2e6f;
     return kLaunchUs + (work > stores ? work : stores);
 }
 
-// the fastest of the four-wave shapes
-int best_ring(int64_t M, int64_t N, int64_t steps, int64_t slices, float* cost)
+// the fastest of the four-wave shapes (sliced: of those that are also built to add slices of K one after the other)
+int best_ring(int64_t M, int64_t N, int64_t steps, int64_t slices, float* cost, bool sliced = false)
 {
     int best = 0;
     float c = 0.0f;
     for (int i = 0; i < kRing256; ++i) {
+        if (sliced && i > kRingLastSliced) break;
         const float t = ring_cost(kRing[i], M, N, steps, slices);
         if (i == 0 || t < c) {
             best = i;
@@ -161,8 +168,8 @@ int best_ring(int64_t M, int64_t N, int64_t steps, int64_t slices, float* cost)
 // A few rows (more than 16: up to there the few-rows kernel always) sum K in eighths on whichever kernel, so the choice is
 // free: the few-rows kernel, whose workgroups take 32 rows of B and wait out a memory latency per step and wave; ring tiles
 // that walk all of K; ring tiles for each eighth, whose planes a second launch adds.  Constants met within 15 % on 768 x 2048
-// .. 5120 x 27648 and 17 .. 64 rows (us, in this order; 32 x 2816 x 1024: 5.6, 6.7, 8.4; 32 x 11008 x 4096: 23.4, 14.6, 19.1;
-// 32 x 4096 x 11008: 28.6, 29.2, 16.3).
+// .. 5120 x 27648 and 17 .. 64 rows (us, in this order; 48 x 2816 x 1024: 6.4, 5.6, 6.9; 48 x 8192 x 2048: 9.2, 6.7, 9.6;
+// 64 x 4096 x 4096: 13.0, 8.8, 12.5; 23 x 4096 x 11008: 28, 17.3, 14.0).
 enum FewRowsKernel { kFewRows, kFewRing, kFewPlanes };
 
 // slices that are not empty
@@ -174,25 +181,43 @@ FewRowsKernel choose_few_rows(int64_t M, int64_t N, int64_t K)
     const float steps = (float)((K + BK - 1) / BK), bytes = (float)N * (float)K;
     const float rounds = (float)((N + 32 * 256 - 1) / (32 * 256));
     const float rows = 1.6f + rounds * (1.6f + eighth_steps(K) * (M <= 32 ? 1.75f : 2.6f));
-    const float walk = 4.0f + 0.29f * steps, read = 2.0f + bytes / 4.2e6f;
+    const float walk = 4.2f + 0.145f * steps, read = 2.0f + bytes / 5.3e6f;
     const float ring = walk > read ? walk : read;
     const float planes = steps < 2.0f ? 1e30f : 5.0f + bytes / 5.3e6f + (float)(M * N) * 1.5e-5f;
     if (rows <= ring && rows <= planes) return kFewRows;
     return ring <= planes ? kFewRing : kFewPlanes;
 }
 
-// Slices for a problem, 1 = do not split.  Slices are a summation order of their own, so they follow from the sizes alone.
-// Splitting pays where the whole of K in one workgroup is the time (few tiles, a long K) and costs a second launch that reads
-// the planes.  Up to 192 tiles of 64 x 64 it is at worst even, so there the unsplit estimate is not asked: such a product
-// of at least eight K steps is always split.  At least four K steps a slice.
+// Slices for a problem, 1 = do not split.  Slices are a summation order of their own, so they follow from the sizes alone
+// and stay what they are when kernels get faster: few tiles and a K of at least eight steps, at least four of them a slice.
+// Which kernel sums in that order is decided apart from it (splitk_entry).  The estimate behind the line: us per K step of a
+// 64 x 64, 128 x 64 (64 x 128), 128 x 128 tile alone on a compute unit and of a pair sharing one, 0 where a pair does not fit.
+float slices_estimate(int64_t M, int64_t N, int64_t steps, int64_t slices)
+{
+    struct Line {
+        int bm, bn;
+        float step1, step2, tile;
+    };
+    constexpr Line lines[] = {{64, 64, 0.28f, 0.39f, 1.2f}, {128, 64, 0.40f, 0.64f, 1.2f}, {64, 128, 0.40f, 0.64f, 1.2f},
+                              {128, 128, 0.72f, 1.0f, 1.5f}, {128, 128, 0.60f, 0.0f, 1.5f}};
+    float best = 1e30f;
+    for (const Line& r : lines) {
+        const int64_t per_cu = (ceil_div(M, r.bm) * ceil_div(N, r.bn) * slices + 255) / 256;
+        const float work = per_cu == 1 || r.step2 == 0.0f ? per_cu * (steps * r.step1 + r.tile) : 0.5f * per_cu * (steps * r.step2 + r.tile);
+        const float stores = (float)(M * N) * (slices > 1 ? 4.0f * slices : 2.0f) / 3.2e6f;
+        const float t = 2.6f + (work > stores ? work : stores);
+        best = t < best ? t : best;
+    }
+    return best;
+}
+
 int suggested_splits(int64_t M, int64_t N, int64_t K)
 {
     const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256), tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
     const int64_t steps = (K + BK - 1) / BK;
     if (M <= kSkinnyMaxM) return choose_few_rows(M, N, K) == kFewRows ? 1 : eighths(K);
     if (tiles256 > 96 || steps < 8) return 1;
-    float best;
-    best_ring(M, N, steps, 1, &best);
+    float best = slices_estimate(M, N, steps, 1);
     if (M >= 256 && N >= 256 && K % BK == 0 && N % 8 == 0) {
         const float t = m16_cost(M, N, K);
         best = t < best ? t : best;
@@ -202,9 +227,7 @@ int suggested_splits(int64_t M, int64_t N, int64_t K)
     for (int64_t s = 2; s <= 32 && s <= steps / 4; ++s) {
         const int64_t per = (steps + s - 1) / s;
         if ((s - 1) * per >= steps) continue;  // the last slice would be empty
-        float t;
-        best_ring(M, N, per, s, &t);
-        t += 2.2f + (float)(M * N) * (4.0f * s + 2.0f) / 4.0e6f;
+        const float t = slices_estimate(M, N, per, s) + 2.2f + (float)(M * N) * (4.0f * s + 2.0f) / 4.0e6f;
         if (t < best) {
             best = t;
             splits = s;
@@ -242,9 +265,21 @@ int launch_ring(GemmArgs& g, SplitArgs* split, hipStream_t st)
                               g, tiles, 1, NW * 64, st, "mi8_gemm_fp8");
 }
 
+// K summed in slices of g.slice_steps steps by one workgroup a tile
+template <int CBSZ, int BLGP>
+int launch_sliced_shape(int shape, GemmArgs& g, hipStream_t st)
+{
+    switch (shape) {
+        case 0: return launch_ring<64, 64, 4, 2, CBSZ, BLGP, true>(g, nullptr, st);
+        case 1: return launch_ring<128, 64, 3, 2, CBSZ, BLGP, true>(g, nullptr, st);
+        default: return launch_ring<64, 128, 3, 2, CBSZ, BLGP, true>(g, nullptr, st);
+    }
+}
+
 template <int CBSZ, int BLGP>
 int launch_ring_shape(int shape, GemmArgs& g, SplitArgs* split, hipStream_t st)
 {
+    if (g.slice_steps) return launch_sliced_shape<CBSZ, BLGP>(shape, g, st);
     switch (shape) {
         case 0: return launch_ring<64, 64, 4, 2, CBSZ, BLGP>(g, split, st);
         case 1: return launch_ring<128, 64, 3, 2, CBSZ, BLGP>(g, split, st);
@@ -252,7 +287,6 @@ int launch_ring_shape(int shape, GemmArgs& g, SplitArgs* split, hipStream_t st)
         case 3: return launch_ring<128, 128, 2, 2, CBSZ, BLGP>(g, split, st);
         case 4: return launch_ring<128, 128, 3, 1, CBSZ, BLGP>(g, split, st);
         case kRing256: return launch_ring<256, 256, 2, 1, CBSZ, BLGP, false, 8>(g, nullptr, st);
-        case kEighths: g.slice_steps = eighth_steps(g.K); return launch_ring<64, 64, 4, 2, CBSZ, BLGP, true>(g, nullptr, st);
     }
     set_error("mi8_gemm_fp8: unknown variant %d", shape);
     return MI8_ERR_ARG;
@@ -347,6 +381,10 @@ int gemm_fp8_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b
                     "scales that are both single values or both vectors, and a 16-byte aligned bf16 output (M=%lld N=%lld K=%lld ldc=%lld)",
                     (long long)M, (long long)N, (long long)K, (long long)ldc);
         return launch_m16(g, a_dtype, b_dtype, st);
+    }
+    if (variant == kEighths) {
+        g.slice_steps = eighth_steps(K);
+        variant = 0;
     }
     return launch_ring_typed(variant, a_dtype, b_dtype, g, nullptr, st);
 }
@@ -490,11 +528,22 @@ int splitk_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b_d
     s.steps_per_split = (int)per;
     s.splits = used;
     hipStream_t st = (hipStream_t)stream;
-    // the eighths of a few rows: the planes are left out where one workgroup walks all of K sooner
-    if (M <= kSkinnyMaxM && used == eighths(K) && choose_few_rows(M, N, K) == kFewRing)
-        return launch_ring_typed(kEighths, a_dtype, b_dtype, s.g, nullptr, st);
-    float cost;
-    const int shape = best_ring(M, N, per, used, &cost);
+    // The planes are left out where one workgroup a tile adds the slices sooner (the eighths of a few rows: choose_few_rows).
+    // Both fitted to 550 products of 65 to 700 rows and 2 to 8 slices; us in planes / whole: 128 x 4096 x 4096 in four 13.5 / 8.6,
+    // 300 x 2048 x 2048 in three 11.7 / 6.7, 128 x 2048 x 8192 in three 10.6 / 11.6, 200 x 5120 x 27648 in six 43.8 / 61.2.
+    float planes, whole;
+    const int shape = best_ring(M, N, per, used, &planes);
+    int sliced = best_ring(M, N, steps, 1, &whole, true);
+    planes += 2.9f + (float)(M * N) * (0.89e-6f * used + 0.66e-6f);
+    bool leave_out = whole < planes;
+    if (M <= kSkinnyMaxM && used == eighths(K)) {
+        leave_out = choose_few_rows(M, N, K) == kFewRing;
+        sliced = 0;
+    }
+    if (leave_out) {
+        s.g.slice_steps = (int)per;
+        return launch_ring_typed(sliced, a_dtype, b_dtype, s.g, nullptr, st);
+    }
     if (int rc = launch_ring_typed(shape, a_dtype, b_dtype, s.g, &s, st)) return rc;
     const int64_t quads = M * (s.ld_plane / 4);
     const auto reduce = used > 4 ? splitk_reduce_kernel<7> : used > 2 ? splitk_reduce_kernel<3> : splitk_reduce_kernel<1>;

@@ -9,17 +9,23 @@
 // lane offset per load and a uniform K offset), a ring of ST stages so that ST - 1 steps are in flight, and an LDS
 // footprint that lets two workgroups live on a compute unit, one computing while the other waits.
 //
+// A step's fragments are read from LDS during the step before (two sets of registers), so that the reads (0.37 us a step of
+// a 128 x 128 tile) and the MFMAs (0.23 us) run side by side: what bounds a step is then the operands' way out of L2, 0.27 us
+// with few compute units busy and 0.40 with all of them, where it took 0.60 with the reads between a barrier and the MFMAs.
+// Tiles that share a compute unit in pairs (two stages), or that have no registers left (256 x 256), keep one set:
+// there the other workgroup or wave fills the gap.
+//
 // The MFMA (v_mfma_f32_16x16x128_f8f6f4), the order of K and the scale arithmetic are those of the persistent kernel: a
-// product has the same bits on either.  Measured against the register-staged 128 x 128 tiles that were here before
-// (32x32x64 MFMAs, split along K where tiles were few), us per launch in a graph: 305 x 2816 x 1024 15.0 -> 6.3,
-// 1537 x 2048 x 2048 26.4 -> 15.5 (17.5 beside the casts of a training step), 1999 x 1024 x 2816 23.5 -> 11.6,
-// 512 x 4096 x 4096 26.8 -> 15.0.  Counters: 24 % of the matrix pipe's cycles busy at 1537 x 2048 x 2048, 34 % at
-// 777 x 4096 x 11008 (one workgroup to a unit: its LDS reads come between a barrier and the MFMAs), bank conflicts 2-8 % of
-// the LDS cycles, operands fetched into L2 3.3 and 2.1 times; 256 x 256 tiles at 16384 x 4096 x 11024: 59 %, 2 %, 4.8 times.
+// product has the same bits on either.  us per launch in a graph, one set of fragments / two: 777 x 4096 x 11008 55.8 / 41.1
+// (128 x 128), 1537 x 2048 x 2048 14.8 / 11.3, 1999 x 1024 x 2816 12.9 / 10.0 (64 x 128), 200 x 4096 x 4096 12.1 / 9.3 (64 x 64).
+// 256 x 256 tiles at 16384 x 4096 x 11024: matrix pipe busy 59 %, bank conflicts 2 % of the LDS cycles, operands fetched into
+// L2 4.8 times.
 //
 // LDS stage: [row][128 bytes], A rows then B rows; 16-byte chunk c of row r sits at c ^ swz16(r) (the swizzle of the
 // persistent kernel), applied by permuting which global chunk a lane fetches.
 #pragma once
+#include <type_traits>
+
 #include "mi8_gemm.h"
 
 namespace mi8 {
@@ -87,6 +93,10 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
     }
     const int nk = (g.K + BK - 1) / BK;
     const bool ragged = g.K < nk * BK;
+    auto issue_one = [&](int i, int k, int slot) __attribute__((always_inline)) {
+        const bool is_a = i < LA;
+        ring_load(is_a ? da : db, lds + slot * STAGE + ((is_a ? 0 : BM) + 8 * (NW * (is_a ? i : i - LA) + wave)) * BK, off[i], k * BK);
+    };
     auto issue = [&](int k, int slot) __attribute__((always_inline)) {
         uint8_t* st = lds + slot * STAGE;
         const int at = k * BK;
@@ -99,10 +109,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < LD; ++i) {
-                const bool is_a = i < LA;
-                ring_load(is_a ? da : db, st + ((is_a ? 0 : BM) + 8 * (NW * (is_a ? i : i - LA) + wave)) * BK, off[i], at);
-            }
+            for (int i = 0; i < LD; ++i) issue_one(i, k, slot);
         }
     };
 
@@ -131,40 +138,29 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
             for (int j = 0; j < TN; ++j) sum[i][j] = (ring_v4f){0, 0, 0, 0};
     }
 
-#pragma unroll
-    for (int s = 0; s < ST - 1; ++s)
-        if (s < nk) issue(s, s);
-    int slot = 0;
-    for (int k = 0; k < nk; ++k) {
-        // this wave's loads of step k have landed (those of up to ST - 2 later steps may be in flight) ...
-        const int ahead = nk - 1 - k;
-        if (ahead >= ST - 2)
-            ring_wait<LD * (ST - 2)>();
-        else if (ST > 3 && ahead == 1)
-            ring_wait<LD>();
-        else
-            ring_wait<0>();
-        // ... every wave's have, and every wave has its fragments of step k - 1, whose slot is filled next
-        asm volatile("s_barrier" ::: "memory");
-        if (k + ST - 1 < nk) issue(k + ST - 1, slot == 0 ? ST - 1 : slot - 1);
+    // x-th fragment register pair of a step: halves q = 0, 1 of the A tiles, then of the B tiles
+    struct ReadAt { uint32_t a[2], b[2]; };
+    auto read_at = [&](int slot) __attribute__((always_inline)) {
         const uint32_t at = (uint32_t)(slot * STAGE);
-        v4i fa[TM][2], fb[TN][2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i) fa[i][q] = *reinterpret_cast<ring_frag_t>((uintptr_t)(fa_at[q] + at + i * 16 * BK));
-#pragma unroll
-            for (int j = 0; j < TN; ++j) fb[j][q] = *reinterpret_cast<ring_frag_t>((uintptr_t)(fb_at[q] + at + j * 16 * BK));
-        }
-        // D' = B . A^T: the first operand is the B fragment (its type code goes to cbsz)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                    __builtin_shufflevector(fb[j][0], fb[j][1], 0, 1, 2, 3, 4, 5, 6, 7),
-                    __builtin_shufflevector(fa[i][0], fa[i][1], 0, 1, 2, 3, 4, 5, 6, 7), acc[i][j], BLGP, CBSZ, 0, 0, 0, 0);
-        slot = slot == ST - 1 ? 0 : slot + 1;
+        ReadAt r{{fa_at[0] + at, fa_at[1] + at}, {fb_at[0] + at, fb_at[1] + at}};
+        asm volatile("" : "+v"(r.a[0]), "+v"(r.a[1]), "+v"(r.b[0]), "+v"(r.b[1]));  // (the tiles' offsets go into the instructions)
+        return r;
+    };
+    auto read_one = [&](v4i (&fa)[TM][2], v4i (&fb)[TN][2], int x, const ReadAt& r) __attribute__((always_inline)) {
+        const int t = x >> 1, q = x & 1;
+        if (t < TM)
+            fa[t][q] = *reinterpret_cast<ring_frag_t>((uintptr_t)(r.a[q] + t * 16 * BK));
+        else
+            fb[t - TM][q] = *reinterpret_cast<ring_frag_t>((uintptr_t)(r.b[q] + (t - TM) * 16 * BK));
+    };
+    // D' = B . A^T: the first operand is the B fragment (its type code goes to cbsz)
+    auto mma_one = [&](const v4i (&fa)[TM][2], const v4i (&fb)[TN][2], int x) __attribute__((always_inline)) {
+        const int i = x / TN, j = x % TN;
+        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+            __builtin_shufflevector(fb[j][0], fb[j][1], 0, 1, 2, 3, 4, 5, 6, 7),
+            __builtin_shufflevector(fa[i][0], fa[i][1], 0, 1, 2, 3, 4, 5, 6, 7), acc[i][j], BLGP, CBSZ, 0, 0, 0, 0);
+    };
+    auto end_of_step = [&]() __attribute__((always_inline)) {
         if constexpr (SLICED) {
             if (--slice_left == 0) {
                 slice_left = g.slice_steps;
@@ -176,6 +172,110 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
                         acc[i][j] = (ring_v4f){0, 0, 0, 0};
                     }
             }
+        }
+    };
+    constexpr int kMma = TM * TN, kReads = 2 * (TM + TN);
+    // Two sets of fragments: a step multiplies from one while the next step's are read into the other, and the loads of step
+    // k + ST go into the slot of step k, whose fragments have all been read.
+    constexpr bool kTwoSets = ST > 2 && 8 * kReads + 4 * kMma * (SLICED ? 2 : 1) <= 192;
+    if constexpr (kTwoSets) {
+        v4i fa[2][TM][2], fb[2][TN][2];
+        int slot = 0;
+        auto k_step = [&](int k, auto set_tag, auto steady_tag) __attribute__((always_inline)) {
+            constexpr int S = decltype(set_tag)::value;
+            auto body = [&](auto with_reads, auto with_loads) __attribute__((always_inline)) {
+                const ReadAt at = read_at(slot == ST - 1 ? 0 : slot + 1);
+#pragma unroll
+                for (int x = 0; x < kMma; ++x) {
+                    mma_one(fa[S], fb[S], x);
+                    if constexpr (decltype(with_reads)::value) {
+#pragma unroll
+                        for (int y = x * kReads / kMma; y < (x + 1) * kReads / kMma; ++y) read_one(fa[S ^ 1], fb[S ^ 1], y, at);
+                    }
+                    if constexpr (decltype(with_loads)::value) {
+#pragma unroll
+                        for (int y = x * LD / kMma; y < (x + 1) * LD / kMma; ++y) issue_one(y, k + ST, slot);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            // this wave's fragments of step k have arrived and its loads of step k + 1 have landed (those of up to ST - 2
+            // later steps may be in flight); after the barrier every wave's
+            constexpr bool kSteady = decltype(steady_tag)::value;
+            const int ahead = kSteady ? ST - 2 : nk - 2 - k;
+            if (ahead >= ST - 2)
+                ring_wait<LD * (ST - 2)>();
+            else if (ST > 3 && ahead == 1)
+                ring_wait<LD>();
+            else
+                ring_wait<0>();
+            asm volatile("s_barrier" ::: "memory");
+            if constexpr (kSteady) {
+                body(std::true_type{}, std::true_type{});
+            } else {
+                if (k + ST < nk) issue(k + ST, slot);
+                if (k + 1 < nk)
+                    body(std::true_type{}, std::false_type{});
+                else
+                    body(std::false_type{}, std::false_type{});
+            }
+            slot = slot == ST - 1 ? 0 : slot + 1;
+            end_of_step();
+        };
+        if (nk > 0) {
+#pragma unroll
+            for (int s = 0; s < ST; ++s)
+                if (s < nk) issue(s, s);
+            if (nk >= ST)
+                ring_wait<LD * (ST - 1)>();
+            else if (ST > 3 && nk == 3)
+                ring_wait<LD * 2>();
+            else if (ST > 2 && nk == 2)
+                ring_wait<LD>();
+            else
+                ring_wait<0>();
+            asm volatile("s_barrier" ::: "memory");
+            const ReadAt at = read_at(0);
+#pragma unroll
+            for (int x = 0; x < kReads; ++x) read_one(fa[0], fb[0], x, at);
+        }
+        const std::integral_constant<int, 0> set0;
+        const std::integral_constant<int, 1> set1;
+        int k = 0;
+        for (; k + 1 + ST < nk - (ragged ? 1 : 0); k += 2) {  // both steps have whole loads to issue
+            k_step(k, set0, std::true_type{});
+            k_step(k + 1, set1, std::true_type{});
+        }
+        for (; k + 1 < nk; k += 2) {
+            k_step(k, set0, std::false_type{});
+            k_step(k + 1, set1, std::false_type{});
+        }
+        if (k < nk) k_step(k, set0, std::false_type{});
+    } else {
+#pragma unroll
+        for (int s = 0; s < ST - 1; ++s)
+            if (s < nk) issue(s, s);
+        int slot = 0;
+        for (int k = 0; k < nk; ++k) {
+            // this wave's loads of step k have landed (those of up to ST - 2 later steps may be in flight) ...
+            const int ahead = nk - 1 - k;
+            if (ahead >= ST - 2)
+                ring_wait<LD * (ST - 2)>();
+            else if (ST > 3 && ahead == 1)
+                ring_wait<LD>();
+            else
+                ring_wait<0>();
+            // ... every wave's have, and every wave has its fragments of step k - 1, whose slot is filled next
+            asm volatile("s_barrier" ::: "memory");
+            if (k + ST - 1 < nk) issue(k + ST - 1, slot == 0 ? ST - 1 : slot - 1);
+            const ReadAt at = read_at(slot);
+            v4i fa[TM][2], fb[TN][2];
+#pragma unroll
+            for (int x = 0; x < kReads; ++x) read_one(fa, fb, x, at);
+#pragma unroll
+            for (int x = 0; x < kMma; ++x) mma_one(fa, fb, x);
+            slot = slot == ST - 1 ? 0 : slot + 1;
+            end_of_step();
         }
     }
     if constexpr (SLICED) {

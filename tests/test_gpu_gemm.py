@@ -564,3 +564,27 @@ def test_ring_tiles_store_rows_of_any_alignment(dev, name, n, pad, skip):
         assert torch.equal(out, ref.to(dt) + ref.to(dt))
         out.fill_(5.0)
         assert bool((buf == 5.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk, splits", [((65, 64, 272), 2), ((128, 200, 1040), 3), ((200, 2048, 1152), 5), ((130, 4100, 2064), 4),
+                                         ((700, 1024, 2816), 2), ((1000, 3000, 2048), 7)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_slices_of_k_without_planes(dev, mnk, splits, dt):
+    """Slices of K are added in order whether they pass through planes or not: the float32 sums of the slices' own products,
+    at one K step a slice, ragged last steps and slices, tiles cut at both edges, with and without `out +=`."""
+    M, N, K = mnk
+    g = torch.Generator(device=dev).manual_seed(K + splits)
+    a = torch.randn(M, K, generator=g, device=dev).to(torch.float8_e4m3fn)
+    b = torch.randn(N, K, generator=g, device=dev).to(torch.float8_e4m3fn)
+    one = torch.ones(1, device=dev)
+    per = -(-(-(-K // 128)) // splits) * 128
+    want = None
+    for k0 in range(0, K, per):
+        part = ops.gemm_fp8(a[:, k0:], one, b[:, k0:], one, k=min(per, K - k0), out_dtype=torch.float32, variant=0)
+        want = part if want is None else want + part
+    got = ops.gemm_fp8(a, one, b, one, out_dtype=dt, splits=splits)
+    assert torch.equal(got, want.to(dt))
+    first = torch.randn(M, N, generator=g, device=dev).to(dt)
+    got = ops.gemm_fp8(a, one, b, one, out_dtype=dt, splits=splits, out=first.clone(), accumulate=True)
+    assert torch.equal(got, first + want.to(dt))
