@@ -118,6 +118,46 @@ int mi8_cast_tensorwise(const void* x, int hp_dtype, int64_t rows, int64_t cols,
                         int32_t n_slots, const float* scale_in, int fp8_dtype, uint32_t flags, void* out,
                         int64_t ld_out, void* out_t, int64_t ld_t, float* scale_out, void* stream);
 
+/* mi8_cast_tensorwise for up to MI8_CAST_BATCH tensors (an input and the weights of a layer) in one launch, of bf16 and
+ * float32 mixed.  A tensor with neither slots nor scale_in has its amax taken first, into amax_ws, in one more launch for
+ * all of those.  Per tensor the arguments of mi8_cast_tensorwise (pad_t128: MI8_FLAG_PAD_T128 for this tensor; scale_out
+ * is always written); bytes and scales are those of the separate calls. */
+#define MI8_CAST_BATCH 8
+typedef struct {
+    const void* x;
+    int64_t rows, cols;
+    const uint32_t* slots;
+    const float* scale_in;
+    uint32_t* amax_ws; /* uint32 [MI8_AMAX_SLOTS], where slots and scale_in are NULL */
+    void* out;
+    int64_t ld_out;
+    void* out_t;
+    int64_t ld_t;
+    float* scale_out;
+    int32_t n_slots, hp_dtype, pad_t128;
+} mi8_cast_item;
+int mi8_cast_tensorwise_batch(const mi8_cast_item* items, int32_t count, int fp8_dtype, uint32_t flags, void* stream);
+
+/* A scale per row with a row-major copy, and a scale per column with a transposed copy, of up to MI8_CAST_BATCH tensors:
+ * per tensor the results of mi8_cast_rowwise and mi8_cast_colwise_t, two launches for all of them.
+ *   out_rows: fp8 [rows, ld_rows]; row_scale: float32 [rows]; out_t: fp8 [cols, ld_t], ld_t >= round_up(rows, 128), zero
+ *   from column `rows` to ld_t; col_scale: float32 [cols]; workspace: uint32 [mi8_two_cast_workspace_words(rows, cols)],
+ *   16-byte aligned, contents on entry unimportant. */
+typedef struct {
+    const void* x;
+    int64_t rows, cols;
+    void* out_rows;
+    int64_t ld_rows;
+    float* row_scale;
+    void* out_t;
+    int64_t ld_t;
+    float* col_scale;
+    uint32_t* workspace;
+    int32_t hp_dtype;
+} mi8_two_cast_item;
+int64_t mi8_two_cast_workspace_words(int64_t rows, int64_t cols);
+int mi8_cast_rows_and_colwise_t_batch(const mi8_two_cast_item* items, int32_t count, int fp8_dtype, uint32_t flags, void* stream);
+
 /* The dynamic tensorwise cast in one call for callers that cannot allocate device memory or hand over a
  * workspace (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): amax pass +
  * cast pass as mi8_amax_partials followed by mi8_cast_tensorwise(slots), with the partial maxima kept in an 8 KiB

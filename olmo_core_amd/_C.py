@@ -27,6 +27,23 @@ FLAG_AMAX_READY = 4
 FLAG_PAD_T128 = 8
 AMAX_SLOTS = 2048
 
+CAST_BATCH = 8
+
+
+class CastItem(ctypes.Structure):
+    """mi8_cast_item"""
+    _fields_ = [("x", c_void_p), ("rows", c_int64), ("cols", c_int64), ("slots", c_void_p), ("scale_in", c_void_p),
+                ("amax_ws", c_void_p), ("out", c_void_p), ("ld_out", c_int64), ("out_t", c_void_p), ("ld_t", c_int64),
+                ("scale_out", c_void_p), ("n_slots", c_int32), ("hp_dtype", c_int32), ("pad_t128", c_int32)]
+
+
+class TwoCastItem(ctypes.Structure):
+    """mi8_two_cast_item"""
+    _fields_ = [("x", c_void_p), ("rows", c_int64), ("cols", c_int64), ("out_rows", c_void_p), ("ld_rows", c_int64),
+                ("row_scale", c_void_p), ("out_t", c_void_p), ("ld_t", c_int64), ("col_scale", c_void_p),
+                ("workspace", c_void_p), ("hp_dtype", c_int32)]
+
+
 # name -> (restype, argtypes); mirrors include/mi8.h one to one
 _SIGNATURES = {
     "mi8_version": (c_int, []),
@@ -48,6 +65,9 @@ _SIGNATURES = {
         c_int,
         [c_void_p, c_int, c_int64, c_int64, c_int, c_uint32, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p],
     ),
+    "mi8_cast_tensorwise_batch": (c_int, [POINTER(CastItem), c_int32, c_int, c_uint32, c_void_p]),
+    "mi8_two_cast_workspace_words": (c_int64, [c_int64, c_int64]),
+    "mi8_cast_rows_and_colwise_t_batch": (c_int, [POINTER(TwoCastItem), c_int32, c_int, c_uint32, c_void_p]),
     "mi8_cast_rowwise": (
         c_int,
         [c_void_p, c_int, c_int64, c_int64, c_int, c_uint32, c_void_p, c_int64, c_void_p, c_void_p],

@@ -133,39 +133,67 @@ def _weight_operands(weight, c: Float8LinearConfig, pow2: bool, share_w: bool, w
     return wq, sw, w_saved
 
 
+def _forward_operands(x2, weights, c: Float8LinearConfig, scales, w_ops, share_x: bool, share_w: bool):
+    """:func:`_input_operands` of ``x2`` and :func:`_weight_operands` of every weight: ``(xq, sx, x_saved, [(wq, sw,
+    w_saved), ...])``.  Tensors that are cast alike share their launches."""
+    pow2 = c.round_scales_to_power_of_2
+    ci, cw = c.cast_config_input, c.cast_config_weight
+    if ci.target_dtype == cw.target_dtype and any(o is None for o in w_ops):
+        if _is_tensorwise(ci) and _is_tensorwise(cw):
+            more = [(w, dict(want_transposed=share_w, scale=s)) for w, s, o in zip(weights, scales, w_ops) if o is None]
+            (xq, xq_t, sx), *made = ops.cast_tensorwise(x2, ci.target_dtype, pow2=pow2, want_transposed=share_x, whole_steps=True,
+                                                        more=more)
+            made = iter(made)
+            ws = [next(made) if o is None else o for o in w_ops]
+            return xq, sx, (xq_t, sx) if share_x else None, [(q, s, (q_t, s) if share_w else None) for q, q_t, s in ws]
+        if _is_axiswise(ci) and _is_axiswise(cw) and share_x and share_w and all(o is None for o in w_ops):
+            (xq, sx, xq_t, sxc), *made = ops.cast_rows_and_colwise_t(x2, ci.target_dtype, pow2=pow2, more=weights)
+            return xq, sx, (xq_t, sxc), [(q, s, (q_t, sc)) for q, s, q_t, sc in made]
+    return (*_input_operands(x2, c, pow2, share_x),
+            [_weight_operands(w, c, pow2, share_w, s, o) for w, s, o in zip(weights, scales, w_ops)])
+
+
 def _forward_impl(x2, weight, c: Float8LinearConfig, weight_scale, need_gx: bool, need_gw: bool, weight_ops=None):
     """y = x2 @ weight^T in float8.  Returns ``(y, x_saved, w_saved)``: the tensors the backward needs for x and
     for the weight, each either ``(q_t, scale)`` (see :func:`_saves_quantised`) or ``None`` (keep the input).
     ``weight_ops``: ``(q, q_t, scale)`` of the weight kept by the module (:meth:`Float8Linear.weight_operands`);
     the weight is then not quantised here."""
-    pow2 = c.round_scales_to_power_of_2
-    share_x, share_w = _saves_quantised(c, need_gx, need_gw)
     if _is_disabled(c.cast_config_input):
         return torch.mm(x2, weight.t().to(x2.dtype)), None, None
-    xq, sx, x_saved = _input_operands(x2, c, pow2, share_x)
-    wq, sw, w_saved = _weight_operands(weight, c, pow2, share_w, weight_scale, weight_ops)
+    share_x, share_w = _saves_quantised(c, need_gx, need_gw)
+    xq, sx, x_saved, ((wq, sw, w_saved),) = _forward_operands(x2, (weight,), c, (weight_scale,), (weight_ops,), share_x, share_w)
     return ops.gemm_fp8(xq, sx, wq, sw, out_dtype=x2.dtype), x_saved, w_saved
 
 
+def _grad_operands(gos, c: Float8LinearConfig, need_gx: bool, need_gws):
+    """Each grad_output's operands ``(rows, cols)`` for the grad_input and the grad_weight GEMM where both are wanted and
+    quantise it alike (all of them share their launches), else ``(None, None)``."""
+    pow2 = c.round_scales_to_power_of_2
+    cg, cgw = c.cast_config_grad_output, c.cast_config_grad_output_for_grad_weight
+    made = [(None, None)] * len(gos)
+    todo = [i for i, (go, need) in enumerate(zip(gos, need_gws)) if go is not None and need_gx and need]
+    if todo and _shared_tensorwise(cg, cgw):
+        kw = dict(want_transposed=True, whole_steps=True)
+        for i, (q, q_t, s) in zip(todo, ops.cast_tensorwise_batch([(gos[i], kw) for i in todo], cg.target_dtype, pow2=pow2)):
+            made[i] = (q, s), (q_t, s)
+    elif todo and _shared_axiswise(cg, cgw):
+        for i, (q, rs, q_t, cs) in zip(todo, ops.cast_rows_and_colwise_t_batch([gos[i] for i in todo], cg.target_dtype, pow2=pow2)):
+            made[i] = (q, rs), (q_t, cs)
+    return made
+
+
 def _backward_impl(go2, c: Float8LinearConfig, N: int, x_dtype, w_dtype, x_part, w_part, x_is_q: bool, w_is_q: bool,
-                   need_gx: bool, need_gw: bool, gx_into=None):
+                   need_gx: bool, need_gw: bool, gx_into=None, go_operands=None):
     """grad_input and grad_weight from grad_output ``go2 [M, N]``; ``x_part`` / ``w_part`` are what the forward
     kept: ``(q_t, scale)`` if the flag says so, else ``(tensor,)``.  ``gx_into``: a ``[M, K]`` tensor of ``x_dtype``
     that this linear's grad_input is added to (the bits of ``gx_into + grad_input``, formed in the GEMM's epilogue)
-    and that is returned as ``gx``."""
+    and that is returned as ``gx``.  ``go_operands``: what :func:`_grad_operands` made of ``go2``."""
     pow2 = c.round_scales_to_power_of_2
     if go2.dtype != x_dtype:
         go2 = go2.to(x_dtype)
-    # quantise grad_output once if both backward GEMMs want the same tensorwise cast
-    go_rows = go_cols = None
     cg, cgw = c.cast_config_grad_output, c.cast_config_grad_output_for_grad_weight
-    if need_gx and need_gw and _shared_tensorwise(cg, cgw):
-        q, q_t, s = ops.cast_tensorwise(go2, cg.target_dtype, pow2=pow2, want_rowmajor=True, want_transposed=True,
-                                        whole_steps=True)
-        go_rows, go_cols = (q, s), (q_t, s)
-    elif need_gx and need_gw and _shared_axiswise(cg, cgw):
-        q, rs, q_t, cs = ops.cast_rows_and_colwise_t(go2, cg.target_dtype, pow2=pow2)
-        go_rows, go_cols = (q, rs), (q_t, cs)
+    # grad_output is quantised once if both backward GEMMs want the same cast
+    go_rows, go_cols = go_operands if go_operands is not None else _grad_operands([go2], c, need_gx, [need_gw])[0]
 
     gx = gw = None
     if need_gx:
@@ -229,15 +257,9 @@ def _shared_input_forward(x2, weights, c: Float8LinearConfig, scales, w_ops, nee
     ``w_saved[i]`` as :func:`_forward_impl` returns them."""
     if _is_disabled(c.cast_config_input):
         return [torch.mm(x2, w.t().to(x2.dtype)) for w in weights], None, [None] * len(weights)
-    pow2 = c.round_scales_to_power_of_2
     share_x, share_w = _saves_quantised(c, need_gx, need_gw)
-    xq, sx, x_saved = _input_operands(x2, c, pow2, share_x)
-    ys, w_saved = [], []
-    for w, ws, wo in zip(weights, scales, w_ops):
-        wq, sw, kept = _weight_operands(w, c, pow2, share_w, ws, wo)
-        ys.append(ops.gemm_fp8(xq, sx, wq, sw, out_dtype=x2.dtype))
-        w_saved.append(kept)
-    return ys, x_saved, w_saved
+    xq, sx, x_saved, ws = _forward_operands(x2, weights, c, scales, w_ops, share_x, share_w)
+    return [ops.gemm_fp8(xq, sx, wq, sw, out_dtype=x2.dtype) for wq, sw, _ in ws], x_saved, [kept for _, _, kept in ws]
 
 
 class _Float8SharedInputMatmul(torch.autograd.Function):
@@ -288,12 +310,15 @@ class _Float8SharedInputMatmul(torch.autograd.Function):
             pos += k
         gx, gws = None, [None] * n
         chain = ctx.gx_dtype == ctx.x_dtype  # the terms are added in the type the GEMMs write: by their epilogues
+        gos = [None if go is None else go.reshape(ctx.M, ctx.ns[i]) for i, go in enumerate(gos)]
+        gos = [go if go is None or go.dtype == ctx.x_dtype else go.to(ctx.x_dtype) for go in gos]
+        made = _grad_operands(gos, ctx.config, need_gx, ctx.need_gws)
         for i in reversed(range(n)):
             if gos[i] is None:
                 continue
             term, gws[i] = _backward_impl(
-                gos[i].reshape(ctx.M, ctx.ns[i]), ctx.config, ctx.ns[i], ctx.x_dtype, ctx.w_dtypes[i], x_part, w_parts[i],
-                ctx.x_is_q, ctx.w_is_q[i], need_gx, ctx.need_gws[i], gx_into=gx if chain else None,
+                gos[i], ctx.config, ctx.ns[i], ctx.x_dtype, ctx.w_dtypes[i], x_part, w_parts[i],
+                ctx.x_is_q, ctx.w_is_q[i], need_gx, ctx.need_gws[i], gx_into=gx if chain else None, go_operands=made[i],
             )
             if need_gx:
                 gx = term if chain else (term.to(ctx.gx_dtype) if gx is None else gx.add_(term))

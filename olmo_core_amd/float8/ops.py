@@ -177,6 +177,7 @@ def cast_tensorwise(
     pitch: Optional[int] = None,
     pitch_t: Optional[int] = None,
     whole_steps: bool = False,
+    more=None,
 ) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor], torch.Tensor]:
     """
     Quantise ``x [rows, cols]`` with one scale.  Returns ``(q, q_t, scale)``: ``q`` fp8 ``[rows, cols]``,
@@ -184,7 +185,12 @@ def cast_tensorwise(
     ``scale`` if given, else from amax partials (``slots`` if already computed by a producer kernel).
     ``whole_steps``: ``q_t`` is ``[cols, pad128(rows)]``, for a GEMM that contracts over the rows in steps of 128 whatever
     their number (the persistent kernel takes no other).
+    ``more``: further tensors to be cast in the same launches, as :func:`cast_tensorwise_batch` takes them; the result is
+    then the list of all results, that of ``x`` first.
     """
+    if more:
+        kw = dict(want_rowmajor=want_rowmajor, want_transposed=want_transposed, slots=slots, scale=scale, whole_steps=whole_steps)
+        return cast_tensorwise_batch([(x, kw), *more], fp8_dtype, pow2=pow2)
     x = _hp2d(x, "cast_tensorwise")
     rows, cols = x.shape
     dev = x.device
@@ -211,6 +217,54 @@ def cast_tensorwise(
         "mi8_cast_tensorwise",
     )
     return q, q_t, scale_out
+
+
+def cast_tensorwise_batch(items, fp8_dtype: torch.dtype, *, pow2: bool = False) -> list:
+    """:func:`cast_tensorwise` of several tensors on one GPU, launched together.  ``items``: up to ``CAST_BATCH`` pairs of
+    a tensor and a dict of that function's keyword arguments (``want_rowmajor``, ``want_transposed``, ``slots``, ``scale``,
+    ``whole_steps``); returns the list of its results."""
+    if len(items) == 1:
+        x, kw = items[0]
+        return [cast_tensorwise(x, fp8_dtype, pow2=pow2, **kw)]
+    if len(items) > _C.CAST_BATCH:
+        return (cast_tensorwise_batch(items[:_C.CAST_BATCH], fp8_dtype, pow2=pow2)
+                + cast_tensorwise_batch(items[_C.CAST_BATCH:], fp8_dtype, pow2=pow2))
+    xs = [_hp2d(x, "cast_tensorwise") for x, _ in items]
+    dev = xs[0].device
+    n = len(items)
+    todo = [i for i, (_, kw) in enumerate(items) if kw.get("scale") is None and kw.get("slots") is None]
+    ws = torch.empty((len(todo), _C.AMAX_SLOTS), dtype=torch.int32, device=dev) if todo else None
+    wsp = ws.data_ptr() if todo else 0
+    args = (_C.CastItem * n)()
+    out, keep = [], []
+    for i, (x, (_, kw)) in enumerate(zip(xs, items)):
+        if x.device != dev:
+            raise ValueError("cast_tensorwise_batch: tensors must be on one GPU")
+        rows, cols = x.shape
+        pad = kw.get("whole_steps", False)
+        q = torch.empty((rows, cols), dtype=fp8_dtype, device=dev) if kw.get("want_rowmajor", True) else None
+        q_t = torch.empty((cols, (pad128 if pad else pad16)(rows)), dtype=fp8_dtype, device=dev) if kw.get("want_transposed") else None
+        a = args[i]
+        a.x, a.rows, a.cols, a.hp_dtype, a.pad_t128 = x.data_ptr(), rows, cols, _HP_CODE[x.dtype], int(pad)
+        scale, slots = kw.get("scale"), kw.get("slots")
+        if scale is not None:
+            scale = scale.reshape(1).to(torch.float32)
+            keep.append(scale)
+            a.scale_in = scale.data_ptr()
+        elif slots is not None:
+            a.slots, a.n_slots = slots[0].data_ptr(), slots[1]
+        else:
+            a.amax_ws, wsp = wsp, wsp + 4 * _C.AMAX_SLOTS
+        if q is not None:
+            a.out, a.ld_out = q.data_ptr(), cols
+        if q_t is not None:
+            a.out_t, a.ld_t = q_t.data_ptr(), q_t.shape[1]
+        s = torch.empty(1, dtype=torch.float32, device=dev)  # (storages of their own: registered operators return them)
+        a.scale_out = s.data_ptr()
+        out.append((q, q_t, s))
+    _C.check(_C.lib().mi8_cast_tensorwise_batch(args, n, _FP8_CODE[fp8_dtype], _flags(pow2), _stream(xs[0])),
+             "mi8_cast_tensorwise_batch")
+    return out
 
 
 def cast_rowwise(
@@ -849,25 +903,49 @@ def swiglu_cast_rows(x1: torch.Tensor, x3: torch.Tensor, *, pow2: bool = False):
     return q, s
 
 
-_ONE_GROUP: dict = {}
-
-
 def cast_rows_and_colwise_t(
-    x: torch.Tensor, fp8_dtype: torch.dtype, *, pow2: bool = False
+    x: torch.Tensor, fp8_dtype: torch.dtype, *, pow2: bool = False, more=None
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """
-    :func:`cast_rowwise` and :func:`cast_colwise_t` of one tensor from one pair of passes (the grouped two-product
-    cast with a single group): ``(q [rows, cols], row_scale [rows], q_t [cols, rows rounded up to 128], col_scale
-    [cols])``; ``q_t`` is zero beyond ``rows``.  Bytes and scales are those of the two separate casts.
+    :func:`cast_rowwise` and :func:`cast_colwise_t` of one tensor from one pair of passes: ``(q [rows, cols], row_scale
+    [rows], q_t [cols, rows rounded up to 128], col_scale [cols])``; ``q_t`` is zero beyond ``rows``.  Bytes and scales are
+    those of the two separate casts.  ``more``: further tensors to be cast in the same launches; the result is then the
+    list of all results, that of ``x`` first.
     """
-    x = _hp2d(x, "cast_rows_and_colwise_t")
-    # one group that takes every row: the kernels clamp group sizes to the rows that exist, so one device-resident
-    # "all of them" serves every shape (no host-to-device copy per call, none at all after the first)
-    sizes = _ONE_GROUP.get(x.device)
-    if sizes is None:
-        sizes = _ONE_GROUP[x.device] = torch.tensor([1 << 62], dtype=torch.int64, device=x.device)
-    q, row_scale, q_t, col_scale = grouped_cast_rows_and_colwise_t(x, sizes, fp8_dtype, pow2=pow2)
-    return q, row_scale, q_t, col_scale.reshape(-1)
+    made = cast_rows_and_colwise_t_batch([x, *(more or ())], fp8_dtype, pow2=pow2)
+    return made if more else made[0]
+
+
+def cast_rows_and_colwise_t_batch(xs, fp8_dtype: torch.dtype, *, pow2: bool = False) -> list:
+    """:func:`cast_rows_and_colwise_t` of several tensors on one GPU, launched together."""
+    if len(xs) > _C.CAST_BATCH:
+        return (cast_rows_and_colwise_t_batch(xs[:_C.CAST_BATCH], fp8_dtype, pow2=pow2)
+                + cast_rows_and_colwise_t_batch(xs[_C.CAST_BATCH:], fp8_dtype, pow2=pow2))
+    xs = [_hp2d(x, "cast_rows_and_colwise_t") for x in xs]
+    dev = xs[0].device
+    n = len(xs)
+    L = _C.lib()
+    words = [L.mi8_two_cast_workspace_words(*x.shape) for x in xs]
+    ws = torch.empty(sum(words), dtype=torch.int32, device=dev)
+    at = ws.data_ptr()
+    args = (_C.TwoCastItem * n)()
+    out = []
+    for a, x, w in zip(args, xs, words):
+        if x.device != dev:
+            raise ValueError("cast_rows_and_colwise_t_batch: tensors must be on one GPU")
+        rows, cols = x.shape
+        ld_t = pad128(rows)
+        q = torch.empty((rows, cols), dtype=fp8_dtype, device=dev)
+        q_t = torch.empty((cols, ld_t), dtype=fp8_dtype, device=dev)
+        rs, cs = torch.empty(rows, dtype=torch.float32, device=dev), torch.empty(cols, dtype=torch.float32, device=dev)
+        a.x, a.rows, a.cols, a.hp_dtype = x.data_ptr(), rows, cols, _HP_CODE[x.dtype]
+        a.out_rows, a.ld_rows, a.row_scale = q.data_ptr(), cols, rs.data_ptr()
+        a.out_t, a.ld_t, a.col_scale, a.workspace = q_t.data_ptr(), ld_t, cs.data_ptr(), at
+        at += 4 * w
+        out.append((q, rs, q_t, cs))
+    _C.check(L.mi8_cast_rows_and_colwise_t_batch(args, n, _FP8_CODE[fp8_dtype], _flags(pow2), _stream(xs[0])),
+             "mi8_cast_rows_and_colwise_t_batch")
+    return out
 
 
 def grouped_gemm_fp8(

@@ -85,21 +85,18 @@ def _mlp_forward(x, w1, w2, w3, c, need, ws=(None, None, None), wo=(None, None, 
     # a generation step: launches that wait for one another are the time, so the activations are quantised by the GEMMs
     few_rows = not keep and STAGE_SINK is None and ops.few_rows_supported(M, H, in_dt, w_dt) and w2.shape[0] % 8 == 0
     x_in_gemm = few_rows and ops.few_rows_quantises(M, D)
-    # The amax of x and of every weight that still needs one is taken in a single launch.
-    todo = [w for w, s, o in ((w1, ws1, wo1), (w3, ws3, wo3), (w2, ws2, wo2)) if s is None and o is None]
-    if not x_in_gemm:
-        todo.insert(0, x)
-    part = {}
-    if len(todo) > 1 and all(t.dtype == todo[0].dtype and t.is_contiguous() for t in todo):
-        part = {id(t): p for t, p in zip(todo, ops.amax_partials_batch(todo))}
-    xq, xq_t, sx = (x, None, None) if x_in_gemm else ops.cast_tensorwise(
-        x, in_dt, pow2=pow2, want_transposed=need[1] or need[3], slots=part.get(id(x)), whole_steps=True)
-    w1q, w1q_t, s1 = wo1 or ops.cast_tensorwise(w1, w_dt, pow2=pow2, want_transposed=need[0], scale=ws1,
-                                                slots=part.get(id(w1)))
-    w3q, w3q_t, s3 = wo3 or ops.cast_tensorwise(w3, w_dt, pow2=pow2, want_transposed=need[0], scale=ws3,
-                                                slots=part.get(id(w3)))
-    w2q, w2q_t, s2 = wo2 or ops.cast_tensorwise(w2, w_dt, pow2=pow2, want_transposed=any_grad, scale=ws2,
-                                                slots=part.get(id(w2)))
+    # x and every weight that has no float8 copy yet are quantised together: one launch for the maxima, one for the casts
+    items = [] if x_in_gemm else [(x, dict(want_transposed=need[1] or need[3], whole_steps=True))]
+    items += [(w, dict(want_transposed=t, scale=s))
+              for w, t, s, o in ((w1, need[0], ws1, wo1), (w3, need[0], ws3, wo3), (w2, any_grad, ws2, wo2)) if o is None]
+    if in_dt == w_dt:
+        made = iter(ops.cast_tensorwise_batch(items, in_dt, pow2=pow2) if items else ())
+    else:
+        made = iter([ops.cast_tensorwise(t, in_dt if t is x else w_dt, pow2=pow2, **kw) for t, kw in items])
+    xq, xq_t, sx = (x, None, None) if x_in_gemm else next(made)
+    w1q, w1q_t, s1 = wo1 or next(made)
+    w3q, w3q_t, s3 = wo3 or next(made)
+    w2q, w2q_t, s2 = wo2 or next(made)
     if few_rows:
         h, h_slots = ops.few_rows_swiglu(xq, sx, w1q, s1, w3q, s3, pow2=pow2)
         if ops.few_rows_quantises(M, H, have_slots=True):

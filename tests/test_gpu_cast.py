@@ -337,3 +337,38 @@ def test_transposed_copy_in_whole_steps(dev, rows):
     for i in (1, 4):
         assert b[i].shape == (144, ops.pad128(rows))
         assert torch.equal(u8(a[i])[:, :rows], u8(b[i])[:, :rows]) and not u8(b[i])[:, rows:].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [torch.float8_e4m3fn, torch.float8_e5m2])
+def test_casts_of_several_tensors_in_one_launch(dev, fp8):
+    """Tensors cast together have the bytes and scales of casts one by one: single rows, tiles cut at both edges, more row
+    tiles than chunks of column maxima (4097 rows), bf16 and float32 mixed, and values that are all zero, infinite or NaN."""
+    shapes = [(1, 16), (127, 144), (128, 128), (129, 2048), (4097, 272), (300, 1040), (16, 4096)]
+    xs = [torch.randn(s, generator=torch.Generator().manual_seed(i), dtype=torch.float32).to(dev) for i, s in enumerate(shapes)]
+    xs = [x if i % 3 == 1 else x.bfloat16() for i, x in enumerate(xs)]
+    xs[2].zero_()
+    xs[3][5, 7], xs[3][6, 9] = float("inf"), float("nan")
+    raw = lambda t: t.view(torch.uint8)  # noqa: E731
+    finite = [i for i in range(len(xs)) if i != 3]
+    for pow2 in (False, True):
+        for i, (q, rs, q_t, cs) in enumerate(ops.cast_rows_and_colwise_t_batch(xs, fp8, pow2=pow2)):
+            q1, rs1 = ops.cast_rowwise(xs[i], fp8, pow2=pow2)
+            q_t1, cs1 = ops.cast_colwise_t(xs[i], fp8, pow2=pow2)
+            assert torch.equal(rs.nan_to_num(7.0), rs1.nan_to_num(7.0)) and torch.equal(cs.nan_to_num(7.0), cs1.nan_to_num(7.0))
+            if i in finite:
+                assert torch.equal(raw(q), raw(q1)) and torch.equal(raw(q_t)[:, : q_t1.shape[1]], raw(q_t1))
+            else:
+                assert torch.equal(q.float().nan_to_num(3.0), q1.float().nan_to_num(3.0))
+            assert q_t.shape[1] == ops.pad128(xs[i].shape[0]) and not raw(q_t)[:, xs[i].shape[0]:].any()
+        given = torch.full((1,), 3.0, device=dev)
+        items = [(x, dict(want_rowmajor=i % 4 != 3, want_transposed=i % 2 == 1, whole_steps=i % 3 == 0, scale=given if i == 5 else None,
+                          slots=ops.amax_partials(x) if i == 4 else None)) for i, x in enumerate(xs)]
+        for i, (q, q_t, s) in enumerate(ops.cast_tensorwise_batch(items, fp8, pow2=pow2)):
+            q1, q_t1, s1 = ops.cast_tensorwise(xs[i], fp8, pow2=pow2, **items[i][1])
+            assert torch.equal(s.nan_to_num(7.0), s1.nan_to_num(7.0))
+            for got, want in ((q, q1), (q_t, q_t1)):
+                assert (got is None) == (want is None)
+                if got is not None:
+                    assert torch.equal(got.float().nan_to_num(3.0), want.float().nan_to_num(3.0))
+    assert len(ops.cast_tensorwise_batch([(xs[6], {})] * 11, fp8)) == len(ops.cast_rows_and_colwise_t_batch([xs[6]] * 11, fp8)) == 11
