@@ -269,6 +269,28 @@ int mi8_gemm_fp8_splitk_accumulate(const void* a, int a_dtype, int64_t lda, cons
 int mi8_gemm_splitk_suggest(int64_t M, int64_t N, int64_t K);
 int64_t mi8_gemm_splitk_workspace_bytes(int64_t M, int64_t N, int splits);
 
+/* Up to MI8_GEMM_BATCH products of one pair of fp8 types in ONE launch, each as mi8_gemm_fp8 (or, where the library cuts
+ * the product along K, mi8_gemm_fp8_splitk with the suggested slices) gives it, bit for bit.  add_to_previous: the product
+ * is added to the output of the one before it (same M, N, out, ldc, out_dtype), as mi8_gemm_fp8_accumulate does; otherwise
+ * outputs must not overlap.  For the products of a layer of ordinary size, which fill a part of the chip each: whether
+ * one launch is estimated faster than one per product is what mi8_gemm_fp8_batch_pays returns (1 or 0; 0 for what
+ * mi8_gemm_fp8_batch refuses). */
+#define MI8_GEMM_BATCH 8
+typedef struct {
+    const void* a;
+    int64_t lda;
+    const void* b;
+    int64_t ldb;
+    int64_t M, N, K;
+    const float* sa;
+    const float* sb;
+    void* out;
+    int64_t ldc;
+    int32_t sa_is_vector, sb_is_vector, out_dtype, add_to_previous;
+} mi8_gemm_product;
+int mi8_gemm_fp8_batch_pays(const mi8_gemm_product* products, int32_t count);
+int mi8_gemm_fp8_batch(const mi8_gemm_product* products, int32_t count, int a_dtype, int b_dtype, void* stream);
+
 /* Number of GEMM kernel variants compiled in (variant ids 0..n-1; -1 lets the library choose by shape).  Which id is
  * which kernel may change with the library: look a variant up by its name. */
 int mi8_gemm_num_variants(void);

@@ -44,6 +44,16 @@ class TwoCastItem(ctypes.Structure):
                 ("workspace", c_void_p), ("hp_dtype", c_int32)]
 
 
+GEMM_BATCH = 8
+
+
+class GemmProduct(ctypes.Structure):
+    """mi8_gemm_product"""
+    _fields_ = [("a", c_void_p), ("lda", c_int64), ("b", c_void_p), ("ldb", c_int64), ("M", c_int64), ("N", c_int64),
+                ("K", c_int64), ("sa", c_void_p), ("sb", c_void_p), ("out", c_void_p), ("ldc", c_int64),
+                ("sa_is_vector", c_int32), ("sb_is_vector", c_int32), ("out_dtype", c_int32), ("add_to_previous", c_int32)]
+
+
 # name -> (restype, argtypes); mirrors include/mi8.h one to one
 _SIGNATURES = {
     "mi8_version": (c_int, []),
@@ -116,6 +126,8 @@ _SIGNATURES = {
         [c_void_p, c_int, c_int64, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int, c_void_p,
          c_int, c_void_p, c_int, c_int64, c_int, c_void_p, c_int64, c_void_p],
     ),
+    "mi8_gemm_fp8_batch_pays": (c_int, [POINTER(GemmProduct), c_int32]),
+    "mi8_gemm_fp8_batch": (c_int, [POINTER(GemmProduct), c_int32, c_int, c_int, c_void_p]),
     "mi8_gemm_splitk_suggest": (c_int, [c_int64, c_int64, c_int64]),
     "mi8_gemm_splitk_workspace_bytes": (c_int64, [c_int64, c_int64, c_int]),
     "mi8_gemm_num_variants": (c_int, []),

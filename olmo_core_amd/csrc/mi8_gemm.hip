@@ -104,6 +104,43 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(SplitArgs a)
     }
 }
 
+// ---- several products in one launch ------------------------------------------------------------------
+// A layer of ordinary size is a handful of products that each fill a part of the chip for 10-20 us, of which a launch of
+// their own wastes the start, the last round of tiles and the way to the next one.  Here the tiles of all of them form one
+// grid.  A product may add to the one before it (C += product, the terms of a grad_input): then one workgroup runs the
+// chain on its tile, so that every element is read and written by one lane, in order.  Every product's tiles are dealt to
+// the XCDs by themselves (an eighth each, contiguous), since products differ in length.
+struct BatchArgs {
+    GemmArgs g[MI8_GEMM_BATCH];
+    int next[MI8_GEMM_BATCH];            // the product that adds to this one's output, or -1
+    int first_slot[MI8_GEMM_BATCH + 1];  // tiles per XCD before the i-th chain
+    int head[MI8_GEMM_BATCH];            // first product of the i-th chain
+    int chains;
+};
+
+template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP, bool SLICED>
+__global__ __launch_bounds__(kRingThreads, OCC) void gemm_fp8_batch_kernel(BatchArgs a)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int xcd = (int)blockIdx.x & 7, slot = (int)blockIdx.x >> 3;
+    int c = 0;
+#pragma unroll
+    for (int i = 1; i < MI8_GEMM_BATCH; ++i)
+        if (i < a.chains && slot >= a.first_slot[i]) c = i;
+    const int per_xcd = a.first_slot[c + 1] - a.first_slot[c];
+    const int t = xcd * per_xcd + slot - a.first_slot[c];
+    int i = a.head[c];
+    if (t >= a.g[i].tiles_m * a.g[i].tiles_n) return;
+    int tm, tn;
+    tile_coords(a.g[i], t, tm, tn);
+    for (;;) {
+        ring_tile<BM, BN, ST, CBSZ, BLGP, SLICED>(a.g[i], tm * BM, tn * BN, lds);
+        i = a.next[i];
+        if (i < 0) break;
+        __syncthreads();  // the output staging has been read
+    }
+}
+
 // ---- tile shapes of the ring kernels and what a problem costs on them ---------------------------------------------
 
 struct RingShape {
@@ -297,6 +334,85 @@ int launch_ring_typed(int shape, int a_dtype, int b_dtype, GemmArgs& g, SplitArg
     if (a_dtype == MI8_E4M3)
         return b_dtype == MI8_E4M3 ? launch_ring_shape<0, 0>(shape, g, split, st) : launch_ring_shape<0, 1>(shape, g, split, st);
     return b_dtype == MI8_E4M3 ? launch_ring_shape<1, 0>(shape, g, split, st) : launch_ring_shape<1, 1>(shape, g, split, st);
+}
+
+// ---- several products in one launch: launch and cost ------------------------------------------------------------------
+
+template <int BM, int BN, int ST, int OCC, int CBSZ, int BLGP, bool SLICED>
+int launch_batch(BatchArgs& a, hipStream_t st)
+{
+    int slots = 0;
+    for (int c = 0; c < a.chains; ++c) {
+        a.first_slot[c] = slots;
+        for (int i = a.head[c]; i >= 0; i = a.next[i]) {
+            a.g[i].tiles_m = (a.g[i].M + BM - 1) / BM;
+            a.g[i].tiles_n = (a.g[i].N + BN - 1) / BN;
+        }
+        slots += (a.g[a.head[c]].tiles_m * a.g[a.head[c]].tiles_n + 7) / 8;
+    }
+    for (int c = a.chains; c <= MI8_GEMM_BATCH; ++c) a.first_slot[c] = slots;
+    static std::atomic<uint64_t> configured;
+    const auto kern = gemm_fp8_batch_kernel<BM, BN, ST, OCC, CBSZ, BLGP, SLICED>;
+    constexpr int lds_bytes = kRingLdsBytes<BM, BN, ST>;
+    if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, configured, "mi8_gemm_fp8_batch")) return rc;
+    hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(kRingThreads), lds_bytes, st, a);
+    return launch_status("mi8_gemm_fp8_batch");
+}
+
+template <int CBSZ, int BLGP>
+int launch_batch_shape(int shape, bool sliced, BatchArgs& a, hipStream_t st)
+{
+    if (sliced) {
+        if (shape == 0) return launch_batch<64, 64, 4, 2, CBSZ, BLGP, true>(a, st);
+        if (shape == 1) return launch_batch<128, 64, 3, 2, CBSZ, BLGP, true>(a, st);
+        return launch_batch<64, 128, 3, 2, CBSZ, BLGP, true>(a, st);
+    }
+    switch (shape) {
+        case 0: return launch_batch<64, 64, 4, 2, CBSZ, BLGP, false>(a, st);
+        case 1: return launch_batch<128, 64, 3, 2, CBSZ, BLGP, false>(a, st);
+        case 2: return launch_batch<64, 128, 3, 2, CBSZ, BLGP, false>(a, st);
+        case 3: return launch_batch<128, 128, 2, 2, CBSZ, BLGP, false>(a, st);
+        default: return launch_batch<128, 128, 3, 1, CBSZ, BLGP, false>(a, st);
+    }
+}
+
+// K steps that a product of these sizes sums from zero before they join the sum, 0: all of them (the order of its sums
+// wherever it runs: see eighth_steps and suggested_splits)
+int slice_steps_of(int64_t M, int64_t N, int64_t K)
+{
+    if (M <= kSkinnyMaxM) return eighth_steps(K);
+    const int splits = suggested_splits(M, N, K);
+    return splits > 1 ? (int)ceil_div(ceil_div(K, BK), splits) : 0;
+}
+
+// us of one launch over all tiles on shape r.  Chains are walked tile by tile; where units get more than one tile the load
+// evens out but for half of the longest.  (128 x 128 pairs in a training step, model / measured: three products of
+// 1537 x 2048 x 2048 36 / 42, grad_input and grad_weight of one of them 26 / 24, all six of three 78 / 70; in launches of their
+// own 16 each.)
+float batch_cost(const RingShape& r, const BatchArgs& a)
+{
+    int64_t tiles = 0;
+    float longest = 0.0f, total = 0.0f, stores = 0.0f;
+    for (int c = 0; c < a.chains; ++c) {
+        const GemmArgs& h = a.g[a.head[c]];
+        tiles += ceil_div(h.M, r.bm) * ceil_div(h.N, r.bn);
+    }
+    const bool one_round = tiles <= 256, many = tiles > 512;
+    const float busy = tiles < 256 ? (float)tiles / 256.0f : 1.0f, tile = many ? r.many_tile : r.tile;
+    const bool pairs = !one_round && r.step2 != 0.0f;
+    const float step = pairs ? (many ? r.many : r.step2) : many && !pairs ? r.many : r.step0 + (r.step1 - r.step0) * busy;
+    for (int c = 0; c < a.chains; ++c) {
+        const GemmArgs& h = a.g[a.head[c]];
+        float t = 0.0f;
+        for (int i = a.head[c]; i >= 0; i = a.next[i]) {
+            t += (float)ceil_div(a.g[i].K, BK) * step + tile;
+            stores += (float)h.M * (float)h.N * (a.g[i].c_f32 ? 4.0f : 2.0f) * (a.g[i].accumulate ? 2.0f : 1.0f) / 3.2e6f;
+        }
+        longest = t > longest ? t : longest;
+        total += t * (float)(ceil_div(h.M, r.bm) * ceil_div(h.N, r.bn)) / (pairs ? 512.0f : 256.0f);
+    }
+    const float work = one_round ? longest : 1.15f * total + 0.5f * longest;
+    return kLaunchUs + (work > stores ? work : stores);
 }
 
 }  // namespace
@@ -568,4 +684,94 @@ extern "C" int mi8_gemm_fp8_splitk_accumulate(const void* a, int a_dtype, int64_
 {
     return splitk_entry(a, a_dtype, lda, b, b_dtype, ldb, M, N, K, sa, sa_is_vector, sb, sb_is_vector, out, out_dtype, ldc,
                         splits, workspace, workspace_bytes, true, stream);
+}
+
+namespace {
+int batch_args(const mi8_gemm_product* p, int32_t count, BatchArgs& a, bool& sliced)
+{
+    const char* what = "mi8_gemm_fp8_batch";
+    MI8_REQUIRE(p, MI8_ERR_ARG, "%s: null pointer", what);
+    MI8_REQUIRE(count > 0 && count <= MI8_GEMM_BATCH, MI8_ERR_ARG, "%s: %d products (1..%d)", what, count, MI8_GEMM_BATCH);
+    a.chains = 0;
+    sliced = false;
+    for (int i = 0; i < count; ++i) {
+        const mi8_gemm_product& q = p[i];
+        MI8_REQUIRE(q.a && q.b && q.sa && q.sb && q.out, MI8_ERR_ARG, "%s: product %d: null pointer", what, i);
+        MI8_REQUIRE(q.M > 0 && q.N > 0 && q.K > 0, MI8_ERR_ARG, "%s: product %d: empty problem %lld x %lld x %lld", what, i,
+                    (long long)q.M, (long long)q.N, (long long)q.K);
+        MI8_REQUIRE(q.K % 16 == 0 && q.lda % 16 == 0 && q.ldb % 16 == 0 && q.lda >= q.K && q.ldb >= q.K && q.ldc >= q.N,
+                    MI8_ERR_UNSUPPORTED, "%s: product %d: K (%lld), lda (%lld), ldb (%lld) must be multiples of 16 with lda, ldb >= K, ldc (%lld) >= N",
+                    what, i, (long long)q.K, (long long)q.lda, (long long)q.ldb, (long long)q.ldc);
+        MI8_REQUIRE(aligned16(q.a) && aligned16(q.b), MI8_ERR_UNSUPPORTED, "%s: product %d: operands must be 16-byte aligned", what, i);
+        MI8_REQUIRE(q.M < (1 << 30) && q.N < (1 << 30) && q.K < (1 << 30) && q.M * q.lda < (int64_t)1 << 32 && q.N * q.ldb < (int64_t)1 << 32,
+                    MI8_ERR_UNSUPPORTED, "%s: product %d: operand larger than 4 GiB", what, i);
+        MI8_REQUIRE(q.out_dtype == MI8_BF16 || q.out_dtype == MI8_F32, MI8_ERR_ARG, "%s: product %d: unknown output dtype %d", what, i, q.out_dtype);
+        MI8_REQUIRE(!q.add_to_previous || (i > 0 && q.M == p[i - 1].M && q.N == p[i - 1].N && q.out == p[i - 1].out && q.ldc == p[i - 1].ldc &&
+                                           q.out_dtype == p[i - 1].out_dtype),
+                    MI8_ERR_ARG, "%s: product %d adds to the one before it: one output and sizes are wanted", what, i);
+        a.g[i] = GemmArgs{(const uint8_t*)q.a, (const uint8_t*)q.b, q.out, q.out_dtype == MI8_F32 ? 1 : 0, q.lda, q.ldb, q.ldc, (int)q.M,
+                          (int)q.N, (int)q.K, q.sa, q.sb, q.sa_is_vector ? 1 : 0, q.sb_is_vector ? 1 : 0, 0, 0, q.add_to_previous ? 1 : 0,
+                          slice_steps_of(q.M, q.N, q.K)};
+        sliced = sliced || a.g[i].slice_steps;
+        a.next[i] = -1;
+        if (q.add_to_previous)
+            a.next[i - 1] = i;
+        else
+            a.head[a.chains++] = i;
+    }
+    return MI8_OK;
+}
+
+int best_batch_shape(const BatchArgs& a, bool sliced, float* cost)
+{
+    int best = 0;
+    for (int i = 0; i <= (sliced ? kRingLastSliced : kRing256 - 1); ++i) {
+        const float t = batch_cost(kRing[i], a);
+        if (i == 0 || t < *cost) {
+            best = i;
+            *cost = t;
+        }
+    }
+    return best;
+}
+}  // namespace
+
+// One launch against a launch each (us, estimates as above, and 1 us for every launch that follows another).
+extern "C" int mi8_gemm_fp8_batch_pays(const mi8_gemm_product* products, int32_t count)
+{
+    BatchArgs a;
+    bool sliced;
+    if (batch_args(products, count, a, sliced) != MI8_OK) return 0;
+    float together = 0.0f, apart = (float)(count - 1);
+    best_batch_shape(a, sliced, &together);
+    for (int i = 0; i < count; ++i) {
+        const GemmArgs& g = a.g[i];
+        const bool acc = g.accumulate != 0;
+        float t;
+        best_ring(g.M, g.N, ceil_div(g.K, BK), 1, &t, g.slice_steps != 0);
+        if (m16_takes(g.M, g.N, g.K, g.ldc, g.c_f32 ? MI8_F32 : MI8_BF16, acc) && aligned16(g.C) && !g.slice_steps) {
+            const float p = m16_cost(g.M, g.N, g.K);
+            t = p < t ? p : t;
+        }
+        apart += t;
+    }
+    return together < apart ? 1 : 0;
+}
+
+extern "C" int mi8_gemm_fp8_batch(const mi8_gemm_product* products, int32_t count, int a_dtype, int b_dtype, void* stream)
+{
+    MI8_REQUIRE((a_dtype == MI8_E4M3 || a_dtype == MI8_E5M2) && (b_dtype == MI8_E4M3 || b_dtype == MI8_E5M2), MI8_ERR_ARG,
+                "mi8_gemm_fp8_batch: unknown fp8 dtype");
+    BatchArgs a;
+    bool sliced;
+    if (int rc = batch_args(products, count, a, sliced)) return rc;
+    float cost = 0.0f;
+    const int shape = best_batch_shape(a, sliced, &cost);
+    if (sliced)  // (whole products among sliced ones: one slice)
+        for (int i = 0; i < count; ++i)
+            if (!a.g[i].slice_steps) a.g[i].slice_steps = 1 << 30;
+    hipStream_t st = (hipStream_t)stream;
+    if (a_dtype == MI8_E4M3)
+        return b_dtype == MI8_E4M3 ? launch_batch_shape<0, 0>(shape, sliced, a, st) : launch_batch_shape<0, 1>(shape, sliced, a, st);
+    return b_dtype == MI8_E4M3 ? launch_batch_shape<1, 0>(shape, sliced, a, st) : launch_batch_shape<1, 1>(shape, sliced, a, st);
 }

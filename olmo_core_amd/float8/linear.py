@@ -196,28 +196,50 @@ def _backward_impl(go2, c: Float8LinearConfig, N: int, x_dtype, w_dtype, x_part,
     go_rows, go_cols = go_operands if go_operands is not None else _grad_operands([go2], c, need_gx, [need_gw])[0]
 
     gx = gw = None
+    products = []
     if need_gx:
         if _is_disabled(cg):
             gx = torch.mm(go2, w_part[0].to(go2.dtype))
             if gx_into is not None:
                 gx = gx_into.add_(gx)
         else:
-            if go_rows is None:
-                go_rows = _rows_operand(go2, cg, pow2)
-            w_op = (w_part[0], w_part[1]) if w_is_q else _cols_operand(w_part[0], c.cast_config_weight_for_grad_input, pow2)
-            gx = ops.gemm_fp8(go_rows[0], go_rows[1], w_op[0], w_op[1], k=N, out_dtype=x_dtype, out=gx_into,
-                              accumulate=gx_into is not None)
+            args = _grad_input_product(go2, c, N, go_rows, w_part, w_is_q)
+            if gx_into is None:
+                products.append(args)
+            else:
+                gx = ops.gemm_fp8(*args[:4], k=N, out_dtype=x_dtype, out=gx_into, accumulate=True)
     if need_gw:
         if _is_disabled(cgw):
             gw = torch.mm(go2.t(), x_part[0].to(go2.dtype))
         else:
-            if go_cols is None:
-                go_cols = _cols_operand(go2, cgw, pow2)
-            x_op = (x_part[0], x_part[1]) if x_is_q else _cols_operand(x_part[0], c.cast_config_input_for_grad_weight, pow2)
-            gw = ops.gemm_fp8(go_cols[0], go_cols[1], x_op[0], x_op[1], out_dtype=x_dtype)
-        if gw.dtype != w_dtype:
-            gw = gw.to(w_dtype)
+            products.append(_grad_weight_product(go2, c, go_cols, x_part, x_is_q))
+    if products:
+        made = ops.gemm_fp8_batch(products, out_dtype=x_dtype)
+        if need_gw and not _is_disabled(cgw):
+            gw = made.pop()
+        if made:
+            gx = made.pop()
+    if gw is not None and gw.dtype != w_dtype:
+        gw = gw.to(w_dtype)
     return gx, gw
+
+
+def _grad_input_product(go2, c: Float8LinearConfig, N: int, go_rows, w_part, w_is_q: bool, add: bool = False):
+    """The grad_input term of one linear as :func:`ops.gemm_fp8_batch` takes it."""
+    pow2 = c.round_scales_to_power_of_2
+    if go_rows is None:
+        go_rows = _rows_operand(go2, c.cast_config_grad_output, pow2)
+    w_op = w_part if w_is_q else _cols_operand(w_part[0], c.cast_config_weight_for_grad_input, pow2)
+    return (go_rows[0], go_rows[1], w_op[0], w_op[1], N, add)
+
+
+def _grad_weight_product(go2, c: Float8LinearConfig, go_cols, x_part, x_is_q: bool):
+    """The grad_weight of one linear as :func:`ops.gemm_fp8_batch` takes it."""
+    pow2 = c.round_scales_to_power_of_2
+    if go_cols is None:
+        go_cols = _cols_operand(go2, c.cast_config_grad_output_for_grad_weight, pow2)
+    x_op = x_part if x_is_q else _cols_operand(x_part[0], c.cast_config_input_for_grad_weight, pow2)
+    return (go_cols[0], go_cols[1], x_op[0], x_op[1], None, False)
 
 
 class _Float8Matmul(torch.autograd.Function):
@@ -259,7 +281,8 @@ def _shared_input_forward(x2, weights, c: Float8LinearConfig, scales, w_ops, nee
         return [torch.mm(x2, w.t().to(x2.dtype)) for w in weights], None, [None] * len(weights)
     share_x, share_w = _saves_quantised(c, need_gx, need_gw)
     xq, sx, x_saved, ws = _forward_operands(x2, weights, c, scales, w_ops, share_x, share_w)
-    return [ops.gemm_fp8(xq, sx, wq, sw, out_dtype=x2.dtype) for wq, sw, _ in ws], x_saved, [kept for _, _, kept in ws]
+    ys = ops.gemm_fp8_batch([(xq, sx, wq, sw, None, False) for wq, sw, _ in ws], out_dtype=x2.dtype)
+    return ys, x_saved, [kept for _, _, kept in ws]
 
 
 class _Float8SharedInputMatmul(torch.autograd.Function):
@@ -312,7 +335,21 @@ class _Float8SharedInputMatmul(torch.autograd.Function):
         chain = ctx.gx_dtype == ctx.x_dtype  # the terms are added in the type the GEMMs write: by their epilogues
         gos = [None if go is None else go.reshape(ctx.M, ctx.ns[i]) for i, go in enumerate(gos)]
         gos = [go if go is None or go.dtype == ctx.x_dtype else go.to(ctx.x_dtype) for go in gos]
-        made = _grad_operands(gos, ctx.config, need_gx, ctx.need_gws)
+        c = ctx.config
+        made = _grad_operands(gos, c, need_gx, ctx.need_gws)
+        order = [i for i in reversed(range(n)) if gos[i] is not None]
+        if (order and chain and not _is_disabled(c.cast_config_grad_output)
+                and not _is_disabled(c.cast_config_grad_output_for_grad_weight)):
+            products = [_grad_input_product(gos[i], c, ctx.ns[i], made[i][0], w_parts[i], ctx.w_is_q[i], add=i != order[0])
+                        for i in order if need_gx]
+            wanted = [i for i in order if ctx.need_gws[i]]
+            products += [_grad_weight_product(gos[i], c, made[i][1], x_part, ctx.x_is_q) for i in wanted]
+            outs = ops.gemm_fp8_batch(products, out_dtype=ctx.x_dtype) if products else []
+            if need_gx:
+                gx = outs.pop(0)
+            for i, gw in zip(wanted, outs):
+                gws[i] = gw if gw.dtype == ctx.w_dtypes[i] else gw.to(ctx.w_dtypes[i])
+            return (gx, None, None, None, *gws, *([None] * (2 * n)))
         for i in reversed(range(n)):
             if gos[i] is None:
                 continue

@@ -395,6 +395,53 @@ def gemm_fp8(
     return out
 
 
+def gemm_fp8_batch(products, *, out_dtype: torch.dtype = torch.bfloat16, together: Optional[bool] = None) -> list:
+    """
+    Several :func:`gemm_fp8` products of one pair of float8 types: ``products`` is a list of ``(a, sa, b, sb, k, add)``,
+    ``k`` the contracted length (``None``: that of the operands) and ``add`` whether the product is added to the one
+    before it (the bits of an elementwise add of the two outputs).  Returns the outputs of those that are not added, in
+    order.  One launch where the library estimates that it is faster than one per product (``together`` decides
+    otherwise); the results are the same bits.
+    """
+    outs = []
+    n = len(products)
+    a0, b0 = products[0][0], products[0][2]
+    if n == 1 and not products[0][5]:
+        return [gemm_fp8(*products[0][:4], k=products[0][4], out_dtype=out_dtype)]
+    _require_gpu(a0, "gemm_fp8_batch")
+    one_launch = together is not False and GEMM_EVENT_SINK is None and 1 < n <= _C.GEMM_BATCH
+    args = (_C.GemmProduct * n)() if one_launch else (None,) * n
+    for (a, sa, b, sb, k, add), p in zip(products, args):
+        M, N = a.shape[0], b.shape[0]
+        K = min(a.shape[1], b.shape[1]) if k is None else k
+        if a.dtype != a0.dtype or b.dtype != b0.dtype or a.device != a0.device or a.dtype not in _FP8_CODE or b.dtype not in _FP8_CODE:
+            raise TypeError("gemm_fp8_batch: the products must be on one GPU and of one pair of float8 types")
+        if a.stride(1) != 1 or b.stride(1) != 1:
+            raise ValueError("gemm_fp8_batch: operands must be 2-D with contiguous rows")
+        va, vb = sa.numel() != 1, sb.numel() != 1
+        if (va and sa.numel() != M) or (vb and sb.numel() != N):
+            raise ValueError(f"gemm_fp8_batch: scale sizes {sa.numel()}, {sb.numel()} do not match M={M}, N={N}")
+        if add and (not outs or tuple(outs[-1].shape) != (M, N)):
+            raise ValueError("gemm_fp8_batch: nothing of its shape to add the product to")
+        if not add:
+            outs.append(torch.empty((M, N), dtype=out_dtype, device=a.device))
+        if one_launch:
+            out = outs[-1]
+            p.a, p.lda, p.b, p.ldb = a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0)
+            p.M, p.N, p.K, p.sa, p.sb = M, N, K, sa.data_ptr(), sb.data_ptr()
+            p.out, p.ldc, p.out_dtype = out.data_ptr(), N, _HP_CODE[out_dtype]
+            p.sa_is_vector, p.sb_is_vector, p.add_to_previous = va, vb, add
+    L = _C.lib()
+    if one_launch and (together or L.mi8_gemm_fp8_batch_pays(args, n)):
+        _C.check(L.mi8_gemm_fp8_batch(args, n, _FP8_CODE[a0.dtype], _FP8_CODE[b0.dtype], _stream(a0)), "mi8_gemm_fp8_batch")
+        return outs
+    i = -1
+    for a, sa, b, sb, k, add in products:
+        i += not add
+        gemm_fp8(a, sa, b, sb, k=k, out_dtype=out_dtype, out=outs[i], accumulate=bool(add))
+    return outs
+
+
 def swiglu_gemm_supported(M: int, H: int, K: int) -> bool:
     """Shapes :func:`gemm_fp8_swiglu` takes (otherwise: two :func:`gemm_fp8` calls and :func:`swiglu_fwd`)."""
     return M >= 256 and H >= 128 and H % 8 == 0 and K % 128 == 0

@@ -110,8 +110,7 @@ def _mlp_forward(x, w1, w2, w3, c, need, ws=(None, None, None), wo=(None, None, 
         else:
             x1, x3, h, h_slots = ops.gemm_fp8_swiglu(xq, sx, w1q, s1, w3q, s3)
     else:
-        x1 = ops.gemm_fp8(xq, sx, w1q, s1, out_dtype=x.dtype)
-        x3 = ops.gemm_fp8(xq, sx, w3q, s3, out_dtype=x.dtype)
+        x1, x3 = ops.gemm_fp8_batch([(xq, sx, w1q, s1, None, False), (xq, sx, w3q, s3, None, False)], out_dtype=x.dtype)
         h, h_slots = ops.swiglu_fwd(x1, x3, want_amax=True)
     if STAGE_SINK is not None:
         STAGE_SINK.update(x1=x1.clone(), x3=x3.clone(), h=h.clone())
@@ -142,18 +141,23 @@ def _mlp_backward(gy, saved, c, dims, dtypes, need):
     need_gh = need_x or need_w1 or need_w3
     gyq, gyq_t, sgy = ops.cast_tensorwise(gy, go_dt, pow2=pow2, want_rowmajor=need_gh, want_transposed=need_w2,
                                            whole_steps=True)
-    gw2 = ops.gemm_fp8(gyq_t, sgy, hq_t, sh, out_dtype=x_dt) if need_w2 else None
-    gx = gw1 = gw3 = None
+    w2_product = (gyq_t, sgy, hq_t, sh, None, False)
+    gx = gw1 = gw2 = gw3 = None
+    if need_w2 and not need_gh:
+        gw2 = ops.gemm_fp8(*w2_product[:4], out_dtype=x_dt)
     if need_gh:
         # g1 and g3 are needed in fp8 only, and their tensorwise scales need the amax of both first.  Where the
         # forward recorded the row-segment codes of x1 and x3, the GEMM that produces gh records those of gh, and the
         # amax follows by computing a small share of the segments; otherwise a pass over the three tensors takes it.
         codes = None
         if x_codes.numel() and x_dt == torch.bfloat16 and ops.gemm_codes_supported(M, H, D):
+            if need_w2:
+                gw2 = ops.gemm_fp8(*w2_product[:4], out_dtype=x_dt)
             gh, gh_codes = ops.gemm_fp8_codes(gyq, sgy, w2q_t, s2, k=D)
             codes = (gh_codes, x_codes)
         else:
-            gh = ops.gemm_fp8(gyq, sgy, w2q_t, s2, k=D, out_dtype=x_dt)
+            gh, *rest = ops.gemm_fp8_batch([(gyq, sgy, w2q_t, s2, D, False)] + ([w2_product] if need_w2 else []), out_dtype=x_dt)
+            gw2 = rest[0] if need_w2 else None
         if STAGE_SINK is not None:
             STAGE_SINK.update(gh=gh.clone())
         need_t = need_w1 or need_w3
@@ -164,18 +168,27 @@ def _mlp_backward(gy, saved, c, dims, dtypes, need):
         if STAGE_SINK is not None:
             STAGE_SINK.update(sg1=sg1.clone(), sg3=sg3.clone(), amax_from_codes=codes is not None,
                               g1q=None if g1q is None else g1q.clone(), g3q=None if g3q is None else g3q.clone())
+        products = []
         if need_x and gx_dt == x_dt:
             # the sum of the two halves as autograd forms it (two bf16 tensors added), by the second GEMM's epilogue
-            gx = ops.gemm_fp8(g1q, sg1, w1q_t, s1, k=H, out_dtype=x_dt)
-            ops.gemm_fp8(g3q, sg3, w3q_t, s3, k=H, out_dtype=x_dt, out=gx, accumulate=True)
+            products += [(g1q, sg1, w1q_t, s1, H, False), (g3q, sg3, w3q_t, s3, H, True)]
+        elif need_x:
+            products += [(g3q, sg3, w3q_t, s3, H, False), (g1q, sg1, w1q_t, s1, H, False)]
+        if need_w1:
+            products.append((g1q_t, sg1, xq_t, sx, None, False))
+        if need_w3:
+            products.append((g3q_t, sg3, xq_t, sx, None, False))
+        outs = ops.gemm_fp8_batch(products, out_dtype=x_dt)
+        if need_w3:
+            gw3 = outs.pop()
+        if need_w1:
+            gw1 = outs.pop()
+        if need_x and gx_dt == x_dt:
+            gx = outs[0]
         elif need_x:
             # (autograd runs w3's backward first: its term is the one the other is added to)
-            gx = ops.gemm_fp8(g3q, sg3, w3q_t, s3, k=H, out_dtype=x_dt).to(gx_dt)
-            gx.add_(ops.gemm_fp8(g1q, sg1, w1q_t, s1, k=H, out_dtype=x_dt))
-        if need_w1:
-            gw1 = ops.gemm_fp8(g1q_t, sg1, xq_t, sx, out_dtype=x_dt)
-        if need_w3:
-            gw3 = ops.gemm_fp8(g3q_t, sg3, xq_t, sx, out_dtype=x_dt)
+            gx = outs[0].to(gx_dt)
+            gx.add_(outs[1])
 
     def as_param(g, dt):
         return g if g is None or g.dtype == dt else g.to(dt)

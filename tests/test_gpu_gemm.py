@@ -6,6 +6,7 @@ import torch
 
 from helpers import E4M3, E5M2, assert_gemm_close, seeded
 from oracle import float8_oracle as O
+from olmo_core_amd.exceptions import MI8KernelError
 
 pytestmark = pytest.mark.gpu
 
@@ -588,3 +589,51 @@ def test_slices_of_k_without_planes(dev, mnk, splits, dt):
     first = torch.randn(M, N, generator=g, device=dev).to(dt)
     got = ops.gemm_fp8(a, one, b, one, out_dtype=dt, splits=splits, out=first.clone(), accumulate=True)
     assert torch.equal(got, first + want.to(dt))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vec", [False, True])
+def test_products_in_one_launch(dev, dt, vec):
+    """Products launched together have the bits of a launch each: one tile and many, ragged edges and K, a product that is
+    cut along K among whole ones, up to 64 rows, a chain of three that add up, and the longest list a launch takes."""
+    g = torch.Generator(device=dev).manual_seed(int(vec))
+
+    def operands(M, N, K):
+        a = torch.randn(M, K, generator=g, device=dev).to(torch.float8_e5m2)
+        b = torch.randn(N, K, generator=g, device=dev).to(torch.float8_e4m3fn)
+        scale = lambda n: torch.exp2(torch.randint(-3, 4, (n if vec else 1,), generator=g, device=dev).float())  # noqa: E731
+        return a, scale(M), b, scale(N)
+
+    lists = [
+        [((300, 272, 144), False), ((129, 520, 1040), False)],
+        [((777, 1040, 528), False), ((777, 1040, 2064), True), ((777, 1040, 16), True), ((1040, 528, 784), False)],
+        [((40, 1024, 2816), False), ((40, 1024, 784), True), ((2000, 264, 272), False)],
+        [((100, 200, 1040), False), ((1000, 1000, 1024), False), ((100, 200, 2048), True)][:2] + [((65, 300, 128), False)],
+        [((64, 64, 128), False)] * 8,
+    ]
+    assert ops._C.lib().mi8_gemm_splitk_suggest(100, 200, 1040) > 1 and ops._C.lib().mi8_gemm_splitk_suggest(777, 1040, 2064) >= 1
+    for shapes in lists:
+        products = [(*operands(*mnk), None, add) for mnk, add in shapes]
+        apart = ops.gemm_fp8_batch(products, out_dtype=dt, together=False)
+        one = ops.gemm_fp8_batch(products, out_dtype=dt, together=True)
+        want = []
+        for a, sa, b, sb, _, add in products:  # ... and of plain products and elementwise adds
+            c = ops.gemm_fp8(a, sa, b, sb, out_dtype=dt)
+            want.append(want.pop() + c if add else c)
+        assert len(one) == len(apart) == len(want)
+        for x, y, z in zip(one, apart, want):
+            assert torch.equal(x, y) and torch.equal(x, z), shapes
+
+
+@pytest.mark.gpu
+def test_products_in_one_launch_refuse_what_one_launch_cannot_take(dev):
+    a = torch.zeros(128, 256, device=dev).to(torch.float8_e4m3fn)
+    one = torch.ones(1, device=dev)
+    with pytest.raises(ValueError, match="add"):
+        ops.gemm_fp8_batch([(a, one, a, one, None, True)])
+    with pytest.raises(TypeError, match="pair of float8"):
+        ops.gemm_fp8_batch([(a, one, a, one, None, False), (a.float().to(torch.float8_e5m2), one, a, one, None, False)])
+    with pytest.raises(MI8KernelError, match="multiples of 16"):
+        ops.gemm_fp8_batch([(a, one, a, one, 40, False)] * 2, together=True)
+    assert len(ops.gemm_fp8_batch([(a, one, a, one, None, False)] * 9)) == 9
