@@ -522,6 +522,17 @@ int mi8_moe_binned_scatter_wgrad(const void* x, const void* grad, int dtype, int
                                  const int32_t* indices, const int32_t* bins, int32_t experts, int64_t capacity,
                                  int32_t top_k, void* out, void* stream);
 
+/* A sequence of calls of this library made by one call: the launches of a layer whose kernels are shorter than the calls from
+ * an interpreter that make them.  `words`: per call the number mi8_plan_function(name) gives (-1: cannot be planned) and
+ * the call's arguments in order, one word each: a number; for an address 0 (NULL), -1 (the stream), -2
+ * (n_slots_used: not wanted) or (buffer + 1) << 48 | offset into buffers[buffer]; for an array of items (mi8_cast_item, mi8_two_cast_item,
+ * mi8_gemm_product) their number and their fields in order.  Ends with the first
+ * call that fails, returning its status.  Nothing is kept between calls; buffers must outlive the work on `stream`. */
+int mi8_plan_function(const char* name);
+int mi8_run_plan(const int64_t* words, int64_t n_words, const void* const* buffers, int32_t n_buffers, void* stream);
+/* partial maxima that mi8_gemm_fp8_swiglu writes for these sizes on the current device (its *n_slots_used) */
+int32_t mi8_gemm_fp8_swiglu_slots(int64_t M, int64_t H, int64_t K);
+
 #ifdef __cplusplus
 }
 #endif

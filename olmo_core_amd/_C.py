@@ -8,6 +8,7 @@ object is missing, every operator raises ``MI8LibraryMissing`` with the build co
 from __future__ import annotations
 
 import ctypes
+import threading
 from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_uint32, c_void_p, POINTER
 from pathlib import Path
 from typing import Optional
@@ -133,6 +134,9 @@ _SIGNATURES = {
     "mi8_gemm_num_variants": (c_int, []),
     "mi8_gemm_variant_name": (c_char_p, [c_int]),
     "mi8_gemm_variant_for": (c_int, [c_int64, c_int64, c_int64, c_int, c_int]),
+    "mi8_plan_function": (c_int, [c_char_p]),
+    "mi8_run_plan": (c_int, [c_void_p, c_int64, c_void_p, c_int32, c_void_p]),
+    "mi8_gemm_fp8_swiglu_slots": (c_int32, [c_int64, c_int64, c_int64]),
     "mi8_few_rows_swiglu": (
         c_int,
         [c_void_p, c_int, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p,
@@ -260,10 +264,16 @@ class MI8LibraryMissing(RuntimeError):
 
 _lib: Optional[ctypes.CDLL] = None
 
+# per thread: what stands in for the library while a sequence of calls is recorded (float8/plan.py)
+_recording = threading.local()
+
 
 def lib() -> ctypes.CDLL:
     """The loaded library (loads on first use)."""
     global _lib
+    recorder = getattr(_recording, "recorder", None)
+    if recorder is not None:
+        return recorder
     if _lib is None:
         if not LIB_PATH.exists():
             raise MI8LibraryMissing(

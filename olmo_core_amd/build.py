@@ -22,7 +22,7 @@ LIB_PATH = PKG_DIR / "lib" / "libmi8.so"
 DIAG_LIB_PATH = PKG_DIR / "lib" / "libmi8_diag.so"
 OBJ_DIR = PKG_DIR / "lib" / "obj"
 
-SOURCES = ["mi8_api.hip", "mi8_cast.hip", "mi8_cast_batch.hip", "mi8_gemm.hip", "mi8_gemm_m16.hip", "mi8_gemm_skinny.hip", "mi8_pointwise.hip", "mi8_swiglu_amax.hip", "mi8_grouped.hip", "mi8_permute.hip"]
+SOURCES = ["mi8_api.hip", "mi8_cast.hip", "mi8_cast_batch.hip", "mi8_gemm.hip", "mi8_gemm_m16.hip", "mi8_gemm_skinny.hip", "mi8_pointwise.hip", "mi8_swiglu_amax.hip", "mi8_grouped.hip", "mi8_permute.hip", "mi8_plan.hip"]
 # the diagnostics library: the probe kernels plus the error-text / launch helpers they share with the main library
 DIAG_SOURCES = ["mi8_api.hip", "mi8_probe.hip"]
 # ... and the persistent GEMM once more, compiled with time stamps at fixed points of every tile (object name, source, flag)

@@ -106,6 +106,7 @@ int launch_m16_codes(GemmArgs& g, uint16_t* codes, int a_dtype, int b_dtype, hip
 // the two input projections of a SwiGLU block and h = silu(x1) * x3 in one launch (g: A, B = B1, C = x1, N = H,
 // single scales sa, sb = scale of B1); writes 4 * workgroups partial maxima of |h| and their count
 // (x_codes: null, or uint16 [H / 64][M] row-segment codes of the larger of x1 and x3, H % 64 == 0)
+int m16_swiglu_slots(int64_t M, int64_t H, int64_t K);  // the number of those maxima
 int launch_m16_swiglu(GemmArgs& g, const uint8_t* b3, const float* sb3, uint16_t* x3, uint16_t* h, uint32_t* h_slots,
                       int* n_slots, uint16_t* x_codes, int a_dtype, int b_dtype, hipStream_t st);
 // a few rows of A (M <= kSkinnyMaxM) against all of B, bound by reading B once (mi8_gemm_skinny.hip): any N,

@@ -563,6 +563,12 @@ extern "C" int mi8_gemm_fp8_swiglu(const void* a, int a_dtype, int64_t lda, cons
     return rc;
 }
 
+extern "C" int32_t mi8_gemm_fp8_swiglu_slots(int64_t M, int64_t H, int64_t K)
+{
+    if (M < 256 || H < 128 || K <= 0 || M >= (1 << 30) || H >= (1 << 30) || K >= (1 << 30)) return 0;
+    return m16_swiglu_slots(M, H, K);
+}
+
 // 1 if mi8_gemm_fp8_codes takes the shape: shapes that the library never cuts along K (so that the output has the bits
 // of the plain call) whose row segments line up with the output tiles
 extern "C" int mi8_gemm_fp8_codes_supported(int64_t M, int64_t N, int64_t K)

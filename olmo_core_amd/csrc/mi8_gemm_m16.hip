@@ -1063,6 +1063,15 @@ int launch_m16_codes(GemmArgs& g, uint16_t* codes, int a_dtype, int b_dtype, hip
     return launch_typed(pb, 0, true, a_dtype, b_dtype, st);
 }
 
+int m16_swiglu_slots(int64_t M, int64_t H, int64_t K)
+{
+    GemmArgs g{};
+    g.M = (int)M;
+    g.K = (int)K;
+    g.tiles_n = (int)((H + 127) / 128);
+    return 4 * plan_halves(g, num_compute_units(), 256).blocks();
+}
+
 int launch_m16_swiglu(GemmArgs& g, const uint8_t* b3, const float* sb3, uint16_t* x3, uint16_t* h, uint32_t* h_slots,
                       int* n_slots, uint16_t* x_codes, int a_dtype, int b_dtype, hipStream_t st)
 {

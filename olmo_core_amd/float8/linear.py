@@ -26,7 +26,7 @@ from typing import Callable, Optional, Tuple
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import ops, plan
 from .native_config import CastConfig, Float8LinearConfig, ScalingGranularity, ScalingType
 
 __all__ = ["Float8Linear", "convert_to_float8_training", "float8_linear_function", "float8_projections"]
@@ -242,6 +242,69 @@ def _grad_weight_product(go2, c: Float8LinearConfig, go_cols, x_part, x_is_q: bo
     return (go_cols[0], go_cols[1], x_op[0], x_op[1], None, False)
 
 
+def _options(c: Float8LinearConfig) -> tuple:
+    """What of a config the launches of a linear follow from."""
+    out = [c.round_scales_to_power_of_2]
+    for cc in (c.cast_config_input, c.cast_config_input_for_grad_weight, c.cast_config_weight, c.cast_config_weight_for_grad_input,
+               c.cast_config_grad_output, c.cast_config_grad_output_for_grad_weight):
+        out += (id(cc.scaling_type), id(cc.scaling_granularity), cc.target_dtype)  # (ids of members of enumerations)
+    return tuple(out)
+
+
+def _planned_forward(x2, weights, c: Float8LinearConfig, scales, w_ops, need_gx: bool, need_gw: bool):
+    """:func:`_shared_input_forward` from a plan: ``(ys, kept, plan)`` or ``None``.  Only where all that the backward takes is
+    quantised here."""
+    n = len(weights)
+
+    def recorded(px, *rest):
+        given = [rest[2 * n + 3 * i:2 * n + 3 * i + 3] for i in range(n)]
+        ys, x_saved, w_saved = _shared_input_forward(px, rest[:n], c, rest[n:2 * n], [g if g[0] is not None else None for g in given],
+                                                     need_gx, need_gw)
+        if (need_gw and x_saved is None) or (need_gx and None in w_saved):
+            raise plan.Unplannable
+        return ys, (x_saved if need_gw else None, w_saved if need_gx else None)
+
+    inputs = [x2, *weights, *scales]
+    for o in w_ops:
+        inputs += (None, None, None) if o is None else o
+    return plan.call(recorded, inputs, ("linears", n, need_gx, need_gw, _options(c)), own=3 * n)
+
+
+def _planned_backward(ctx, gos, ns, need_gx: bool, need_gws):
+    """``(gx, gws)`` of a forward that ran from a plan (grad_weights in the type of x; ``None`` where nothing is wanted)."""
+    c, M, (kept,) = ctx.config, ctx.M, ctx.saved_tensors
+    gos = [None if go is None else go.reshape(M, N) for go, N in zip(gos, ns)]
+    gos = [go if go is None or (go.dtype == ctx.x_dtype and go.is_contiguous()) else go.to(ctx.x_dtype).contiguous() for go in gos]
+    order = [i for i in reversed(range(len(gos))) if gos[i] is not None]
+    wanted = [i for i in order if need_gws[i]]
+    if not order:
+        return None, [None] * len(gos)
+
+    def products(gos_, saved):
+        x_part, w_parts = saved
+        made = _grad_operands(gos_, c, need_gx, need_gws)
+        ps = [_grad_input_product(gos_[i], c, ns[i], made[i][0], w_parts[i], True, add=i != order[0]) for i in order if need_gx]
+        ps += [_grad_weight_product(gos_[i], c, made[i][1], x_part, True) for i in wanted]
+        return ops.gemm_fp8_batch(ps, out_dtype=ctx.x_dtype) if ps else []
+
+    def recorded(slab, *places):
+        return products(places, ctx.plan.saved_places(slab)), None
+
+    done = plan.call(recorded, [kept, *gos], ("backward", need_gx, tuple(need_gws)), within=ctx.plan)
+    outs = done[0] if done is not None else products(gos, ctx.plan.saved_tensors(kept))
+    outs = list(outs)
+    gx = outs.pop(0) if need_gx else None
+    gws = [None] * len(gos)
+    for i, gw in zip(wanted, outs):
+        gws[i] = gw
+    return gx, gws
+
+
+def _fp8_backward(c: Float8LinearConfig) -> bool:
+    return not (_is_disabled(c.cast_config_input) or _is_disabled(c.cast_config_grad_output)
+                or _is_disabled(c.cast_config_grad_output_for_grad_weight))
+
+
 class _Float8Matmul(torch.autograd.Function):
     """y = x @ W^T with float8 operands; x [M, K] and W [N, K] in high precision."""
 
@@ -249,6 +312,13 @@ class _Float8Matmul(torch.autograd.Function):
     def forward(ctx, x2: torch.Tensor, weight: torch.Tensor, config: Float8LinearConfig, weight_scale=None,
                 weight_ops=None):
         need_gx, need_gw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+        done = _planned_forward(x2, (weight,), config, (weight_scale,), (weight_ops,), need_gx, need_gw) if _fp8_backward(config) else None
+        ctx.plan = None
+        if done is not None:
+            (y,), kept, ctx.plan = done
+            ctx.config, ctx.M, ctx.N, ctx.x_dtype, ctx.w_dtype = config, x2.shape[0], weight.shape[0], x2.dtype, weight.dtype
+            ctx.save_for_backward(kept)
+            return y
         y, x_saved, w_saved = _forward_impl(x2, weight, config, weight_scale, need_gx, need_gw, weight_ops)
         ctx.config = config
         ctx.x_dtype, ctx.w_dtype = x2.dtype, weight.dtype
@@ -265,6 +335,9 @@ class _Float8Matmul(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, go: torch.Tensor):
+        if ctx.plan is not None:
+            gx, (gw,) = _planned_backward(ctx, [go], [ctx.N], ctx.needs_input_grad[0], [ctx.needs_input_grad[1]])
+            return gx, gw if gw is None or gw.dtype == ctx.w_dtype else gw.to(ctx.w_dtype), None, None, None
         M, K, N = ctx.shapes
         saved = ctx.saved_tensors
         gx, gw = _backward_impl(
@@ -304,6 +377,16 @@ class _Float8SharedInputMatmul(torch.autograd.Function):
         ctx.gx_dtype = x2.dtype
         if x2.dtype != act_dtype:
             x2 = x2.to(act_dtype)
+        done = None
+        if ctx.gx_dtype == x2.dtype and _fp8_backward(config):
+            done = _planned_forward(x2, weights, config, scales, w_ops, need_gx, any(need_gws))
+        ctx.plan = None
+        if done is not None:
+            ys, kept, ctx.plan = done
+            ctx.config, ctx.M, ctx.ns, ctx.x_dtype = config, x2.shape[0], [w.shape[0] for w in weights], x2.dtype
+            ctx.w_dtypes, ctx.need_gws = [w.dtype for w in weights], need_gws
+            ctx.save_for_backward(kept)
+            return tuple(ys)
         ys, x_saved, w_saved = _shared_input_forward(x2, weights, config, scales, w_ops, need_gx, any(need_gws))
         ctx.config = config
         ctx.x_dtype, ctx.w_dtypes = x2.dtype, [w.dtype for w in weights]
@@ -323,8 +406,12 @@ class _Float8SharedInputMatmul(torch.autograd.Function):
     @staticmethod
     def backward(ctx, *gos):
         n = len(ctx.ns)
-        saved = ctx.saved_tensors
         need_gx = ctx.needs_input_grad[0]
+        if ctx.plan is not None:
+            gx, gws = _planned_backward(ctx, gos, ctx.ns, need_gx, ctx.need_gws)
+            gws = [gw if gw is None or gw.dtype == dt else gw.to(dt) for gw, dt in zip(gws, ctx.w_dtypes)]
+            return (gx, None, None, None, *gws, *([None] * (2 * n)))
+        saved = ctx.saved_tensors
         x_part, pos = saved[:ctx.n_x], ctx.n_x
         w_parts = []
         for i in range(n):
@@ -362,11 +449,6 @@ class _Float8SharedInputMatmul(torch.autograd.Function):
         return (gx, None, None, None, *gws, *([None] * (2 * n)))
 
 
-@torch.compiler.disable
-def _eager_shared_input_matmul(x2, config, act_dtype, weights, scales, w_ops):
-    return _Float8SharedInputMatmul.apply(x2, config, len(weights), act_dtype, *weights, *scales, *w_ops)
-
-
 def float8_projections(x: torch.Tensor, *modules: nn.Module) -> Tuple[torch.Tensor, ...]:
     """``tuple(m(x) for m in modules)`` for linear modules applied to one tensor, e.g. ``q, k, v =
     float8_projections(x, self.w_q, self.w_k, self.w_v)`` in place of the three calls at
@@ -389,13 +471,16 @@ def float8_projections(x: torch.Tensor, *modules: nn.Module) -> Tuple[torch.Tens
     scales = [m.precomputed_weight_scale() for m in mods]
     w_ops = [m.weight_operands() for m in mods]
     if torch.is_grad_enabled() and (x2.requires_grad or any(w.requires_grad for w in weights)):
-        ys = _eager_shared_input_matmul(x2, c, act_dtype, weights, scales, w_ops)
+        # (not compiling here, so nothing is to be kept from a tracer)
+        ys = _Float8SharedInputMatmul.apply(x2, c, len(weights), act_dtype, *weights, *scales, *w_ops)
     else:
         ys = _shared_input_forward(x2.to(act_dtype), weights, c, scales, w_ops, False, False)[0]
     outs = []
     for m, y in zip(mods, ys):
-        y = y.reshape(*x.shape[:-1], m.weight.shape[0])
-        outs.append(y if m.bias is None else y + m.bias.to(y.dtype))
+        if x.dim() != 2:
+            y = y.reshape(*x.shape[:-1], y.shape[1])
+        bias = m.bias
+        outs.append(y if bias is None else y + bias.to(y.dtype))
     return tuple(outs)
 
 
@@ -457,7 +542,7 @@ def float8_linear_function(
     K = x.shape[-1]
     if weight.dim() != 2 or weight.shape[1] != K:
         raise ValueError(f"float8 linear: input features {K} do not match weight {tuple(weight.shape)}")
-    x2 = x.reshape(-1, K)
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
     cfg_id = getattr(config, "_compiled_id", -1)
     compiling = torch.compiler.is_compiling()
     if compiling and cfg_id >= 0:
@@ -466,10 +551,13 @@ def float8_linear_function(
         y = compiled.linear(x2, weight, cfg_id, weight_scale, module_id)
     elif not compiling and not (torch.is_grad_enabled() and (x2.requires_grad or weight.requires_grad)):
         # nothing to differentiate (evaluation, generation): no autograd node, nothing kept for a backward
-        y = _forward_impl(x2, weight, config, weight_scale, False, False, weight_ops)[0]
-    else:  # eager, or a config no module registered: a graph break
+        done = None if _is_disabled(config.cast_config_input) else _planned_forward(x2, (weight,), config, (weight_scale,), (weight_ops,), False, False)
+        y = done[0][0] if done is not None else _forward_impl(x2, weight, config, weight_scale, False, False, weight_ops)[0]
+    elif not compiling:
+        y = _Float8Matmul.apply(x2, weight, config, weight_scale, weight_ops)
+    else:  # a config no module registered: a graph break
         y = _eager_matmul(x2, weight, config, weight_scale, weight_ops)
-    return y.reshape(*x.shape[:-1], weight.shape[0])
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], weight.shape[0])
 
 
 class Float8Linear(nn.Linear):
@@ -499,8 +587,9 @@ class Float8Linear(nn.Linear):
         scale = None if compiling else self.precomputed_weight_scale()
         w_ops = None if compiling else self.weight_operands()
         out = float8_linear_function(input, self.weight, self.config, scale, w_ops, self._module_id)
-        if self.bias is not None:
-            out = out + self.bias.to(out.dtype)
+        bias = self.bias
+        if bias is not None:
+            out = out + bias.to(out.dtype)
         return out
 
     def precomputed_weight_scale(self) -> Optional[torch.Tensor]:

@@ -39,6 +39,13 @@ def _stream(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
+def _empty(shape, *, dtype: torch.dtype, device):
+    """``torch.empty``, or, while a sequence of calls is recorded (``plan.py``), a place in its buffers."""
+    if type(device) is torch.device:
+        return torch.empty(shape, dtype=dtype, device=device)
+    return device.place(shape, dtype)
+
+
 def _flags(pow2: bool) -> int:
     return (_C.FLAG_POW2_SCALE if pow2 else 0) | (_C.FLAG_SW_CVT if FORCE_SW_CVT else 0)
 
@@ -76,7 +83,7 @@ def amax_partials(x: torch.Tensor) -> Tuple[torch.Tensor, int]:
     """Per-workgroup partial maxima of |x| (as float32 bit patterns); returns (slots, n_used)."""
     _require_gpu(x, "amax_partials")
     xc = x if x.is_contiguous() else x.contiguous()
-    slots = torch.empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x.device)
+    slots = _empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x.device)
     used = _C.c_int32(0)
     _C.check(
         _C.lib().mi8_amax_partials(xc.data_ptr(), _HP_CODE[xc.dtype], xc.numel(), slots.data_ptr(), used, _stream(x)),
@@ -99,7 +106,7 @@ def amax_partials_batch(tensors) -> list:
     for t in tensors:
         if t.dtype != t0.dtype or t.device != t0.device or not t.is_contiguous():
             raise ValueError("amax_partials_batch: tensors must be contiguous, on one GPU and of one dtype")
-    slots = torch.empty((n, _C.AMAX_SLOTS), dtype=torch.int32, device=t0.device)
+    slots = _empty((n, _C.AMAX_SLOTS), dtype=torch.int32, device=t0.device)
     ptrs = (_C.c_void_p * n)(*[t.data_ptr() for t in tensors])
     numels = (_C.c_int64 * n)(*[t.numel() for t in tensors])
     used = (_C.c_int32 * n)()
@@ -112,7 +119,7 @@ def amax_partials_batch(tensors) -> list:
 
 def scale_from_partials(slots: torch.Tensor, n_slots: int, fp8_dtype: torch.dtype, pow2: bool = False) -> torch.Tensor:
     """Returns a float32 tensor [2] = (scale, amax)."""
-    out = torch.empty(2, dtype=torch.float32, device=slots.device)
+    out = _empty(2, dtype=torch.float32, device=slots.device)
     _C.check(
         _C.lib().mi8_scale_from_partials(
             slots.data_ptr(), n_slots, _FP8_CODE[fp8_dtype], _flags(pow2), out.data_ptr(), _stream(slots)
@@ -142,8 +149,8 @@ def multi_tensor_scales(tensors, fp8_dtype: torch.dtype, pow2: bool = False) -> 
             raise ValueError("multi_tensor_scales: every tensor needs 16-byte alignment and a multiple of 16 bytes")
     n = len(tensors)
     table = torch.tensor([[t.data_ptr() for t in tensors], [t.numel() for t in tensors]], dtype=torch.int64).to(t0.device)
-    ws = torch.empty(n, dtype=torch.int32, device=t0.device)
-    out = torch.empty(n, dtype=torch.float32, device=t0.device)
+    ws = _empty(n, dtype=torch.int32, device=t0.device)
+    out = _empty(n, dtype=torch.float32, device=t0.device)
     _C.check(
         _C.lib().mi8_multi_tensor_scales(
             table[0].data_ptr(), table[1].data_ptr(), n, _HP_CODE[t0.dtype], _FP8_CODE[fp8_dtype], _flags(pow2),
@@ -159,10 +166,10 @@ def _operand(shape: Tuple[int, int], fp8_dtype: torch.dtype, device, pitch: Opti
     any row pitch that is a multiple of 16)."""
     rows, k = shape
     if pitch is None or pitch == k:
-        return torch.empty((rows, k), dtype=fp8_dtype, device=device)
+        return _empty((rows, k), dtype=fp8_dtype, device=device)
     if pitch < k or pitch % 16:
         raise ValueError(f"operand pitch {pitch} must be a multiple of 16 and at least {k}")
-    return torch.empty((rows, pitch), dtype=fp8_dtype, device=device)[:, :k]
+    return _empty((rows, pitch), dtype=fp8_dtype, device=device)[:, :k]
 
 
 def cast_tensorwise(
@@ -200,7 +207,7 @@ def cast_tensorwise(
         slots = amax_partials(x)
     q = _operand((rows, cols), fp8_dtype, dev, pitch) if want_rowmajor else None
     q_t = _operand((cols, (pad128 if whole_steps else pad16)(rows)), fp8_dtype, dev, pitch_t) if want_transposed else None
-    scale_out = torch.empty(1, dtype=torch.float32, device=dev)
+    scale_out = _empty(1, dtype=torch.float32, device=dev)
     if scale is not None:
         scale = scale.reshape(1).to(torch.float32)
     _C.check(
@@ -233,7 +240,7 @@ def cast_tensorwise_batch(items, fp8_dtype: torch.dtype, *, pow2: bool = False) 
     dev = xs[0].device
     n = len(items)
     todo = [i for i, (_, kw) in enumerate(items) if kw.get("scale") is None and kw.get("slots") is None]
-    ws = torch.empty((len(todo), _C.AMAX_SLOTS), dtype=torch.int32, device=dev) if todo else None
+    ws = _empty((len(todo), _C.AMAX_SLOTS), dtype=torch.int32, device=dev) if todo else None
     wsp = ws.data_ptr() if todo else 0
     args = (_C.CastItem * n)()
     out, keep = [], []
@@ -242,8 +249,8 @@ def cast_tensorwise_batch(items, fp8_dtype: torch.dtype, *, pow2: bool = False) 
             raise ValueError("cast_tensorwise_batch: tensors must be on one GPU")
         rows, cols = x.shape
         pad = kw.get("whole_steps", False)
-        q = torch.empty((rows, cols), dtype=fp8_dtype, device=dev) if kw.get("want_rowmajor", True) else None
-        q_t = torch.empty((cols, (pad128 if pad else pad16)(rows)), dtype=fp8_dtype, device=dev) if kw.get("want_transposed") else None
+        q = _empty((rows, cols), dtype=fp8_dtype, device=dev) if kw.get("want_rowmajor", True) else None
+        q_t = _empty((cols, (pad128 if pad else pad16)(rows)), dtype=fp8_dtype, device=dev) if kw.get("want_transposed") else None
         a = args[i]
         a.x, a.rows, a.cols, a.hp_dtype, a.pad_t128 = x.data_ptr(), rows, cols, _HP_CODE[x.dtype], int(pad)
         scale, slots = kw.get("scale"), kw.get("slots")
@@ -259,7 +266,7 @@ def cast_tensorwise_batch(items, fp8_dtype: torch.dtype, *, pow2: bool = False) 
             a.out, a.ld_out = q.data_ptr(), cols
         if q_t is not None:
             a.out_t, a.ld_t = q_t.data_ptr(), q_t.shape[1]
-        s = torch.empty(1, dtype=torch.float32, device=dev)  # (storages of their own: registered operators return them)
+        s = _empty(1, dtype=torch.float32, device=dev)  # (storages of their own: registered operators return them)
         a.scale_out = s.data_ptr()
         out.append((q, q_t, s))
     _C.check(_C.lib().mi8_cast_tensorwise_batch(args, n, _FP8_CODE[fp8_dtype], _flags(pow2), _stream(xs[0])),
@@ -274,7 +281,7 @@ def cast_rowwise(
     x = _hp2d(x, "cast_rowwise")
     rows, cols = x.shape
     q = _operand((rows, cols), fp8_dtype, x.device, pitch)
-    s = torch.empty(rows, dtype=torch.float32, device=x.device)
+    s = _empty(rows, dtype=torch.float32, device=x.device)
     _C.check(
         _C.lib().mi8_cast_rowwise(
             x.data_ptr(), _HP_CODE[x.dtype], rows, cols, _FP8_CODE[fp8_dtype], _flags(pow2), q.data_ptr(),
@@ -292,8 +299,8 @@ def cast_colwise_t(
     x = _hp2d(x, "cast_colwise_t")
     rows, cols = x.shape
     q_t = _operand((cols, pad16(rows)), fp8_dtype, x.device, pitch_t)
-    s = torch.empty(cols, dtype=torch.float32, device=x.device)
-    ws = torch.empty(_C.lib().mi8_colamax_workspace_slots(rows, cols), dtype=torch.int32, device=x.device)
+    s = _empty(cols, dtype=torch.float32, device=x.device)
+    ws = _empty(_C.lib().mi8_colamax_workspace_slots(rows, cols), dtype=torch.int32, device=x.device)
     _C.check(
         _C.lib().mi8_cast_colwise_t(
             x.data_ptr(), _HP_CODE[x.dtype], rows, cols, _FP8_CODE[fp8_dtype], _flags(pow2), ws.data_ptr(),
@@ -340,7 +347,7 @@ def gemm_fp8(
     if accumulate and out is None:
         raise ValueError("gemm_fp8: accumulate needs the tensor to add into (out=)")
     if out is None:
-        out = torch.empty((M, N), dtype=out_dtype, device=a.device)
+        out = _empty((M, N), dtype=out_dtype, device=a.device)
     elif tuple(out.shape) != (M, N) or out.dtype != out_dtype or out.stride(1) != 1 or out.device != a.device:
         raise ValueError(f"gemm_fp8: out must be a [{M}, {N}] {out_dtype} tensor with contiguous rows on {a.device}")
     elif not out.is_inference():
@@ -368,7 +375,7 @@ def gemm_fp8(
         )
     elif splits > 1:
         # the planes come from torch's caching allocator: reuse is ordered on the stream like any other tensor
-        planes = torch.empty(L.mi8_gemm_splitk_workspace_bytes(M, N, splits), dtype=torch.uint8, device=a.device)
+        planes = _empty(L.mi8_gemm_splitk_workspace_bytes(M, N, splits), dtype=torch.uint8, device=a.device)
         _C.check(
             (L.mi8_gemm_fp8_splitk_accumulate if accumulate else L.mi8_gemm_fp8_splitk)(
                 a.data_ptr(), _FP8_CODE[a.dtype], a.stride(0), b.data_ptr(), _FP8_CODE[b.dtype], b.stride(0), M, N, K,
@@ -424,7 +431,7 @@ def gemm_fp8_batch(products, *, out_dtype: torch.dtype = torch.bfloat16, togethe
         if add and (not outs or tuple(outs[-1].shape) != (M, N)):
             raise ValueError("gemm_fp8_batch: nothing of its shape to add the product to")
         if not add:
-            outs.append(torch.empty((M, N), dtype=out_dtype, device=a.device))
+            outs.append(_empty((M, N), dtype=out_dtype, device=a.device))
         if one_launch:
             out = outs[-1]
             p.a, p.lda, p.b, p.ldb = a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0)
@@ -473,10 +480,10 @@ def gemm_fp8_swiglu(a: torch.Tensor, sa: torch.Tensor, b1: torch.Tensor, sb1: to
         raise ValueError("gemm_fp8_swiglu: single scales only")
     M, H = a.shape[0], b1.shape[0]
     K = min(a.shape[1], b1.shape[1]) if k is None else k
-    x1, x3, h = (torch.empty((M, H), dtype=torch.bfloat16, device=a.device) for _ in range(3))
-    slots = torch.empty(_C.AMAX_SLOTS, dtype=torch.int32, device=a.device)
+    x1, x3, h = (_empty((M, H), dtype=torch.bfloat16, device=a.device) for _ in range(3))
+    slots = _empty(_C.AMAX_SLOTS, dtype=torch.int32, device=a.device)
     used = _C.c_int32(0)
-    codes = torch.empty(_C.lib().mi8_rowseg_code_count(M, H), dtype=torch.int16, device=a.device) if want_codes else None
+    codes = _empty(_C.lib().mi8_rowseg_code_count(M, H), dtype=torch.int16, device=a.device) if want_codes else None
     sink = GEMM_EVENT_SINK
     if sink is not None:
         ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -516,8 +523,8 @@ def gemm_fp8_codes(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch
         raise ValueError("gemm_fp8_codes: single scales only")
     M, N = a.shape[0], b.shape[0]
     K = min(a.shape[1], b.shape[1]) if k is None else k
-    out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
-    codes = torch.empty(_C.lib().mi8_rowseg_code_count(M, N), dtype=torch.int16, device=a.device)
+    out = _empty((M, N), dtype=torch.bfloat16, device=a.device)
+    codes = _empty(_C.lib().mi8_rowseg_code_count(M, N), dtype=torch.int16, device=a.device)
     sink = GEMM_EVENT_SINK
     if sink is not None:
         ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -565,8 +572,8 @@ def few_rows_swiglu(x: torch.Tensor, sx: Optional[torch.Tensor], w1q, s1, w3q, s
     H = w1q.shape[0]
     if w1q.shape != (H, K) or w3q.shape != (H, K) or w1q.stride(0) != w3q.stride(0) or x.stride(1) != 1 or w1q.stride(1) != 1:
         raise ValueError("few_rows_swiglu: operands do not fit together")
-    h = torch.empty((M, H), dtype=torch.bfloat16, device=x.device)
-    slots = torch.empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x.device)
+    h = _empty((M, H), dtype=torch.bfloat16, device=x.device)
+    slots = _empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x.device)
     used = _C.c_int32(0)
     sink = GEMM_EVENT_SINK
     if sink is not None:
@@ -594,7 +601,7 @@ def few_rows_cast_gemm(x: torch.Tensor, slots: Tuple[torch.Tensor, int], wq, sw,
         raise ValueError("few_rows_cast_gemm: expects bfloat16 rows and a float8_e4m3fn weight of the same row length")
     M, K = x.shape
     N = wq.shape[0]
-    out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    out = _empty((M, N), dtype=torch.bfloat16, device=x.device)
     sink = GEMM_EVENT_SINK
     if sink is not None:
         ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -623,8 +630,8 @@ def swiglu_fwd(x1: torch.Tensor, x3: torch.Tensor, want_amax: bool = True):
     if x1.dtype != torch.bfloat16 or x3.dtype != torch.bfloat16 or x1.shape != x3.shape:
         raise TypeError("swiglu_fwd: expects two bfloat16 tensors of the same shape")
     x1, x3 = x1.contiguous(), x3.contiguous()
-    h = torch.empty_like(x1)
-    slots = torch.empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x1.device) if want_amax else None
+    h = _empty(x1.shape, dtype=x1.dtype, device=x1.device)
+    slots = _empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x1.device) if want_amax else None
     n = x1.numel()
     _C.check(
         _C.lib().mi8_swiglu_fwd(
@@ -639,10 +646,10 @@ def swiglu_bwd(x1: torch.Tensor, x3: torch.Tensor, gh: torch.Tensor, want_amax: 
     """Gradients of h = silu(x1) * x3 w.r.t. x1 and x3 (bf16) and optionally their amax partials."""
     _require_gpu(x1, "swiglu_bwd")
     x1, x3, gh = x1.contiguous(), x3.contiguous(), gh.contiguous()
-    g1, g3 = torch.empty_like(x1), torch.empty_like(x1)
+    g1, g3 = _empty(x1.shape, dtype=x1.dtype, device=x1.device), _empty(x1.shape, dtype=x1.dtype, device=x1.device)
     n = x1.numel()
-    s1 = torch.empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x1.device) if want_amax else None
-    s3 = torch.empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x1.device) if want_amax else None
+    s1 = _empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x1.device) if want_amax else None
+    s3 = _empty(_C.AMAX_SLOTS, dtype=torch.int32, device=x1.device) if want_amax else None
     _C.check(
         _C.lib().mi8_swiglu_bwd(
             x1.data_ptr(), x3.data_ptr(), gh.data_ptr(), g1.data_ptr(), g3.data_ptr(), n,
@@ -664,7 +671,7 @@ def rowseg_max_codes(a: torch.Tensor, b: Optional[torch.Tensor] = None) -> torch
     a = a.contiguous()
     b = b.contiguous() if b is not None else None
     rows, cols = a.shape
-    codes = torch.empty(_C.lib().mi8_rowseg_code_count(rows, cols), dtype=torch.int16, device=a.device)
+    codes = _empty(_C.lib().mi8_rowseg_code_count(rows, cols), dtype=torch.int16, device=a.device)
     _C.check(
         _C.lib().mi8_rowseg_max_codes(a.data_ptr(), b.data_ptr() if b is not None else None, rows, cols, codes.data_ptr(),
                                       _stream(a)),
@@ -683,7 +690,7 @@ def swiglu_bwd_amax_from_codes(x1: torch.Tensor, x3: torch.Tensor, gh: torch.Ten
     for c in (gh_codes, x_codes):
         if c.dtype != torch.int16 or c.numel() != n or not c.is_contiguous() or c.device != x1.device:
             raise ValueError("swiglu_bwd_amax_from_codes: codes must be the int16 arrays of rowseg_max_codes for this shape")
-    state = torch.empty(_C.lib().mi8_swiglu_amax_state_words(rows, cols), dtype=torch.int32, device=x1.device)
+    state = _empty(_C.lib().mi8_swiglu_amax_state_words(rows, cols), dtype=torch.int32, device=x1.device)
     _C.check(
         _C.lib().mi8_swiglu_bwd_amax_from_codes(x1.data_ptr(), x3.data_ptr(), gh.data_ptr(), rows, cols, gh_codes.data_ptr(),
                                                 x_codes.data_ptr(), state.data_ptr(), _stream(x1)),
@@ -717,8 +724,8 @@ def swiglu_bwd_cast(
         state = swiglu_bwd_amax_from_codes(x1, x3, gh, codes[0], codes[1])
         s1, s3, used = state[0:1], state[1:2], 1
     else:
-        s1 = torch.empty(_C.AMAX_SLOTS, dtype=torch.int32, device=dev)
-        s3 = torch.empty(_C.AMAX_SLOTS, dtype=torch.int32, device=dev)
+        s1 = _empty(_C.AMAX_SLOTS, dtype=torch.int32, device=dev)
+        s3 = _empty(_C.AMAX_SLOTS, dtype=torch.int32, device=dev)
         _C.check(
             _C.lib().mi8_swiglu_bwd(x1.data_ptr(), x3.data_ptr(), gh.data_ptr(), None, None, n, s1.data_ptr(), s3.data_ptr(),
                                     _stream(x1)),
@@ -727,7 +734,7 @@ def swiglu_bwd_cast(
         used = _C.lib().mi8_amax_slots_for(n)
     q = [_operand((rows, cols), fp8_dtype, dev) if want_rowmajor else None for _ in range(2)]
     q_t = [_operand((cols, (pad128 if whole_steps else pad16)(rows)), fp8_dtype, dev) if want_transposed else None for _ in range(2)]
-    scales = [torch.empty(1, dtype=torch.float32, device=dev) for _ in range(2)]
+    scales = [_empty(1, dtype=torch.float32, device=dev) for _ in range(2)]
     ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
     _C.check(
         _C.lib().mi8_swiglu_bwd_cast(
@@ -769,8 +776,8 @@ def grouped_cast_colwise_t(
     sizes = _sizes_i64(group_sizes, x.device)
     E = sizes.numel()
     ld_t = grouped_padded_rows(T, E)
-    q_t = torch.empty((cols, ld_t), dtype=fp8_dtype, device=x.device)
-    scale = torch.empty((E, cols), dtype=torch.float32, device=x.device)
+    q_t = _empty((cols, ld_t), dtype=fp8_dtype, device=x.device)
+    scale = _empty((E, cols), dtype=torch.float32, device=x.device)
     ws = torch.zeros(E * cols, dtype=torch.int32, device=x.device)
     _C.check(
         _C.lib().mi8_grouped_cast_colwise_t(
@@ -797,7 +804,7 @@ def grouped_swiglu_fwd(x1: torch.Tensor, x2: torch.Tensor, group_sizes: torch.Te
     T, cols = x1.shape
     sizes = _sizes_i64(group_sizes, x1.device)
     E = sizes.numel()
-    h = torch.empty_like(x1)
+    h = _empty(x1.shape, dtype=x1.dtype, device=x1.device)
     ws = _grouped_amax_workspace(T, cols, E, x1.device)
     _C.check(
         _C.lib().mi8_grouped_swiglu_fwd(x1.data_ptr(), x2.data_ptr(), T, cols, sizes.data_ptr(), E, h.data_ptr(),
@@ -817,7 +824,7 @@ def grouped_swiglu_bwd(x1: torch.Tensor, x2: torch.Tensor, gh: torch.Tensor, gro
     T, cols = x1.shape
     sizes = _sizes_i64(group_sizes, x1.device)
     E = sizes.numel()
-    g1, g2 = torch.empty_like(x1), torch.empty_like(x1)
+    g1, g2 = _empty(x1.shape, dtype=x1.dtype, device=x1.device), _empty(x1.shape, dtype=x1.dtype, device=x1.device)
     ws1 = _grouped_amax_workspace(T, cols, E, x1.device)
     ws2 = _grouped_amax_workspace(T, cols, E, x1.device)
     _C.check(
@@ -844,10 +851,10 @@ def grouped_cast_rows_and_colwise_t(
     sizes = _sizes_i64(group_sizes, x.device)
     E = sizes.numel()
     ld_t = grouped_padded_rows(T, E)
-    q_t = torch.empty((cols, ld_t), dtype=fp8_dtype, device=x.device)
-    scale = torch.empty((E, cols), dtype=torch.float32, device=x.device)
-    q = torch.empty((T, cols), dtype=fp8_dtype, device=x.device)
-    row_scale = torch.empty(T, dtype=torch.float32, device=x.device)
+    q_t = _empty((cols, ld_t), dtype=fp8_dtype, device=x.device)
+    scale = _empty((E, cols), dtype=torch.float32, device=x.device)
+    q = _empty((T, cols), dtype=fp8_dtype, device=x.device)
+    row_scale = _empty(T, dtype=torch.float32, device=x.device)
     flags = _flags(pow2)
     if amax is None:
         ws = _grouped_amax_workspace(T, cols, E, x.device)
@@ -888,10 +895,10 @@ def gather_cast_rows_and_colwise_t(
     sizes = _sizes_i64(group_sizes, x.device)
     E = sizes.numel()
     ld_t = grouped_padded_rows(T, E)
-    q_t = torch.empty((cols, ld_t), dtype=fp8_dtype, device=x.device)
-    scale = torch.empty((E, cols), dtype=torch.float32, device=x.device)
-    q = torch.empty((T, cols), dtype=fp8_dtype, device=x.device)
-    row_scale = torch.empty(T, dtype=torch.float32, device=x.device)
+    q_t = _empty((cols, ld_t), dtype=fp8_dtype, device=x.device)
+    scale = _empty((E, cols), dtype=torch.float32, device=x.device)
+    q = _empty((T, cols), dtype=fp8_dtype, device=x.device)
+    row_scale = _empty(T, dtype=torch.float32, device=x.device)
     ws = _grouped_amax_workspace(T, cols, E, x.device)
     wp, wd = None, 0
     if weights is not None:
@@ -923,8 +930,8 @@ def gather_cast_rows(x: torch.Tensor, indices: torch.Tensor, top_k: int, *, pow2
         raise ValueError(f"gather_cast_rows: expected {T} indices on {x.device}")
     if indices.dtype != torch.int32 or not indices.is_contiguous():
         indices = indices.to(torch.int32).contiguous()
-    q = torch.empty((T, cols), dtype=torch.float8_e4m3fn, device=x.device)
-    s = torch.empty(T, dtype=torch.float32, device=x.device)
+    q = _empty((T, cols), dtype=torch.float8_e4m3fn, device=x.device)
+    s = _empty(T, dtype=torch.float32, device=x.device)
     _C.check(
         _C.lib().mi8_moe_gather_cast_rows(x.data_ptr(), tokens, cols, indices.data_ptr(), top_k, _flags(pow2), q.data_ptr(),
                                           cols, s.data_ptr(), _stream(x)),
@@ -940,8 +947,8 @@ def swiglu_cast_rows(x1: torch.Tensor, x3: torch.Tensor, *, pow2: bool = False):
         raise ValueError("swiglu_cast_rows: expects two bfloat16 matrices of one shape")
     x1, x3 = x1.contiguous(), x3.contiguous()
     rows, cols = x1.shape
-    q = torch.empty((rows, cols), dtype=torch.float8_e4m3fn, device=x1.device)
-    s = torch.empty(rows, dtype=torch.float32, device=x1.device)
+    q = _empty((rows, cols), dtype=torch.float8_e4m3fn, device=x1.device)
+    s = _empty(rows, dtype=torch.float32, device=x1.device)
     _C.check(
         _C.lib().mi8_swiglu_cast_rows(x1.data_ptr(), x3.data_ptr(), rows, cols, _flags(pow2), q.data_ptr(), cols,
                                       s.data_ptr(), _stream(x1)),
@@ -973,7 +980,7 @@ def cast_rows_and_colwise_t_batch(xs, fp8_dtype: torch.dtype, *, pow2: bool = Fa
     n = len(xs)
     L = _C.lib()
     words = [L.mi8_two_cast_workspace_words(*x.shape) for x in xs]
-    ws = torch.empty(sum(words), dtype=torch.int32, device=dev)
+    ws = _empty(sum(words), dtype=torch.int32, device=dev)
     at = ws.data_ptr()
     args = (_C.TwoCastItem * n)()
     out = []
@@ -982,9 +989,9 @@ def cast_rows_and_colwise_t_batch(xs, fp8_dtype: torch.dtype, *, pow2: bool = Fa
             raise ValueError("cast_rows_and_colwise_t_batch: tensors must be on one GPU")
         rows, cols = x.shape
         ld_t = pad128(rows)
-        q = torch.empty((rows, cols), dtype=fp8_dtype, device=dev)
-        q_t = torch.empty((cols, ld_t), dtype=fp8_dtype, device=dev)
-        rs, cs = torch.empty(rows, dtype=torch.float32, device=dev), torch.empty(cols, dtype=torch.float32, device=dev)
+        q = _empty((rows, cols), dtype=fp8_dtype, device=dev)
+        q_t = _empty((cols, ld_t), dtype=fp8_dtype, device=dev)
+        rs, cs = _empty(rows, dtype=torch.float32, device=dev), _empty(cols, dtype=torch.float32, device=dev)
         a.x, a.rows, a.cols, a.hp_dtype = x.data_ptr(), rows, cols, _HP_CODE[x.dtype]
         a.out_rows, a.ld_rows, a.row_scale = q.data_ptr(), cols, rs.data_ptr()
         a.out_t, a.ld_t, a.col_scale, a.workspace = q_t.data_ptr(), ld_t, cs.data_ptr(), at
@@ -1026,7 +1033,7 @@ def grouped_gemm_fp8(
             torch._C._increment_version((out,))
         fn, what = _C.lib().mi8_grouped_gemm_fp8_accumulate, "mi8_grouped_gemm_fp8_accumulate"
     else:
-        out = torch.empty((T, n), dtype=out_dtype, device=a.device)
+        out = _empty((T, n), dtype=out_dtype, device=a.device)
         fn, what = _C.lib().mi8_grouped_gemm_fp8, "mi8_grouped_gemm_fp8"
     _C.check(
         fn(
@@ -1065,7 +1072,7 @@ def grouped_gemm_fp8_dual(
     if sa1.numel() != T or sa2.numel() != T or sb1.shape != sb2.shape:
         raise ValueError("grouped_gemm_fp8_dual: one scale per row of a1 / a2, column scales of one shape")
     sizes = _sizes_i64(group_sizes, a1.device)
-    out = torch.empty((T, n), dtype=torch.bfloat16, device=a1.device)
+    out = _empty((T, n), dtype=torch.bfloat16, device=a1.device)
     _C.check(
         _C.lib().mi8_grouped_gemm_fp8_dual(
             a1.data_ptr(), a2.data_ptr(), _FP8_CODE[a1.dtype], a1.stride(0), b1.data_ptr(), b2.data_ptr(), _FP8_CODE[b1.dtype],
@@ -1093,7 +1100,7 @@ def grouped_wgrad_fp8(
     E, N, Kl = sizes.numel(), a_t.shape[0], b_t.shape[0]
     if a_t.stride(0) != b_t.stride(0):
         raise ValueError("grouped_wgrad_fp8: both operands must share the padded token pitch")
-    out = torch.empty((E, N, Kl), dtype=out_dtype, device=a_t.device)
+    out = _empty((E, N, Kl), dtype=out_dtype, device=a_t.device)
     _C.check(
         _C.lib().mi8_grouped_wgrad_fp8(
             a_t.data_ptr(), _FP8_CODE[a_t.dtype], b_t.data_ptr(), _FP8_CODE[b_t.dtype], a_t.stride(0),

@@ -16,7 +16,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from ..float8 import ops
+from ..float8 import ops, plan
 from ..float8.linear import Float8Linear, _shared_tensorwise, needs_autograd
 
 __all__ = ["FeedForward", "swiglu"]
@@ -196,6 +196,31 @@ def _mlp_backward(gy, saved, c, dims, dtypes, need):
     return gx, as_param(gw1, w1_dt), as_param(gw2, w2_dt), as_param(gw3, w3_dt)
 
 
+def _planned_forward(x, weights, c, need, ws, wo, keep: bool):
+    """:func:`_mlp_forward` from a plan: ``([y], kept, plan)`` or ``None``."""
+    if STAGE_SINK is not None:
+        return None
+    pow2 = c.round_scales_to_power_of_2
+    options = ("mlp", need, keep, pow2, c.cast_config_input.target_dtype, c.cast_config_weight.target_dtype,
+               c.cast_config_grad_output.target_dtype, FUSE_SWIGLU_EPILOGUE, SWIGLU_AMAX_FROM_CODES)
+
+    def recorded(px, p1, p2, p3, *rest):
+        given = tuple(rest[3 + 3 * i:6 + 3 * i] if rest[3 + 3 * i] is not None else None for i in range(3))
+        y, saved = _mlp_forward(px, p1, p2, p3, c, need, rest[:3], given, keep)
+        return [y], saved if keep else None
+
+    if None not in wo and not keep:  # generation: what is needed of three weights are their row-major float8 copies
+
+        def kept_weights(px, q1, q2, q3, t1, t2, t3):
+            return [_mlp_forward(px, q1, q2, q3, c, need, (None,) * 3, ((q1, None, t1), (q2, None, t2), (q3, None, t3)), False)[0]], None
+
+        return plan.call(kept_weights, [x, *(o[0] for o in wo), *(o[2] for o in wo)], options, own=6)
+    inputs = [x, *weights, *ws]
+    for o in wo:
+        inputs += (None, None, None) if o is None else o
+    return plan.call(recorded, inputs, options, own=9)
+
+
 class _Float8SwiGLUMLP(torch.autograd.Function):
     """The fused block as an eager autograd function (a traced graph takes the registered operators of
     ``olmo_core_amd.float8.compiled`` instead, which run the same two routines)."""
@@ -203,7 +228,13 @@ class _Float8SwiGLUMLP(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w1, w2, w3, config, ws1=None, ws2=None, ws3=None, wo1=None, wo2=None, wo3=None):
         need = tuple(ctx.needs_input_grad[:4])
-        y, saved = _mlp_forward(x, w1, w2, w3, config, need, (ws1, ws2, ws3), (wo1, wo2, wo3))
+        done = _planned_forward(x, (w1, w2, w3), config, need, (ws1, ws2, ws3), (wo1, wo2, wo3), True)
+        ctx.plan = None
+        if done is not None:
+            (y,), kept, ctx.plan = done
+            saved = (kept,)
+        else:
+            y, saved = _mlp_forward(x, w1, w2, w3, config, need, (ws1, ws2, ws3), (wo1, wo2, wo3))
         ctx.config = config
         ctx.dtypes = (x.dtype, w1.dtype, w2.dtype, w3.dtype)
         ctx.dims = (x.shape[0], x.shape[1], w1.shape[0])
@@ -212,21 +243,40 @@ class _Float8SwiGLUMLP(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gy):
-        grads = _mlp_backward(gy, ctx.saved_tensors, ctx.config, ctx.dims, ctx.dtypes, tuple(ctx.needs_input_grad[:4]))
-        return grads + (None,) * 7
+        need = tuple(ctx.needs_input_grad[:4])
+        if ctx.plan is None:
+            return _mlp_backward(gy, ctx.saved_tensors, ctx.config, ctx.dims, ctx.dtypes, need) + (None,) * 7
+        (kept,), bf16 = ctx.saved_tensors, torch.bfloat16
+        done = None
+        if STAGE_SINK is None and ctx.dtypes[0] == bf16:
+            if gy.dtype != bf16 or not gy.is_contiguous():
+                gy = gy.to(bf16).contiguous()
+
+            def recorded(slab, pgy):
+                grads = _mlp_backward(pgy, ctx.plan.saved_places(slab), ctx.config, ctx.dims, (bf16,) * 4, need)
+                return [g for g in grads if g is not None], None
+
+            done = plan.call(recorded, [kept, gy], ("backward", need), within=ctx.plan)
+        if done is None:
+            return _mlp_backward(gy, ctx.plan.saved_tensors(kept), ctx.config, ctx.dims, ctx.dtypes, need) + (None,) * 7
+        grads = iter(done[0])
+        grads = [next(grads) if n else None for n in need]
+        return (*(g if g is None or g.dtype == dt else g.to(dt) for g, dt in zip(grads, ctx.dtypes)), *(None,) * 7)
 
 
 def _fusable_modules(ff: "FeedForward", same_object: bool = False) -> bool:
     """The three projections are float8 modules of one tensorwise config without bias.  same_object: only accept one
     shared config object (what a model conversion hands to every module), without comparing configs field by field:
     the form a traced graph evaluates."""
-    if not ff.fuse_float8:
-        return False
-    for m in (ff.w1, ff.w2, ff.w3):
+    return ff.fuse_float8 and _fusable((ff.w1, ff.w2, ff.w3), same_object)
+
+
+def _fusable(mods, same_object: bool = False) -> bool:
+    for m in mods:
         if not isinstance(m, Float8Linear) or m.bias is not None:
             return False
-    c = ff.w1.config
-    for m in (ff.w2, ff.w3):
+    c = mods[0].config
+    for m in mods[1:]:
         if m.config is not c and (same_object or m.config != c):
             return False
     return (
@@ -234,11 +284,6 @@ def _fusable_modules(ff: "FeedForward", same_object: bool = False) -> bool:
         and _shared_tensorwise(c.cast_config_weight, c.cast_config_weight_for_grad_input)
         and _shared_tensorwise(c.cast_config_grad_output, c.cast_config_grad_output_for_grad_weight)
     )
-
-
-@torch.compiler.disable
-def _fused_mlp(x2, w1, w2, w3, config, ws1=None, ws2=None, ws3=None, wo1=None, wo2=None, wo3=None):
-    return _Float8SwiGLUMLP.apply(x2, w1, w2, w3, config, ws1, ws2, ws3, wo1, wo2, wo3)
 
 
 class FeedForward(nn.Module):
@@ -280,18 +325,20 @@ class FeedForward(nn.Module):
                 y = compiled.swiglu_mlp(x2, self.w1.weight, self.w2.weight, self.w3.weight, cfg_id,
                                         (self.w1._module_id, self.w2._module_id, self.w3._module_id))
                 return y.reshape(*x.shape[:-1], self.w2.weight.shape[0])
-        elif xa.is_cuda and act_dtype == torch.bfloat16 and _fusable_modules(self):
-            x2 = xa.reshape(-1, xa.shape[-1])
-            weights = (self.w1.weight, self.w2.weight, self.w3.weight)
-            scales = tuple(m.precomputed_weight_scale() for m in (self.w1, self.w2, self.w3))
-            operands = tuple(m.weight_operands() for m in (self.w1, self.w2, self.w3))
+        elif xa.is_cuda and act_dtype == torch.bfloat16 and self.fuse_float8 and _fusable(mods := (self.w1, self.w2, self.w3)):
+            x2 = xa if xa.dim() == 2 else xa.reshape(-1, xa.shape[-1])
+            c = mods[0].config
+            weights = tuple(m.weight for m in mods)
+            scales = tuple(m.precomputed_weight_scale() for m in mods)
+            operands = tuple(m.weight_operands() for m in mods)
             if needs_autograd(x2, *weights):
-                y = _fused_mlp(x2, *weights, self.w1.config, *scales, *operands)
+                y = _Float8SwiGLUMLP.apply(x2, *weights, c, *scales, *operands)  # (not compiling: no tracer to keep it from)
             else:
                 # nothing to differentiate: no transposed float8 copies, nothing kept for a backward (an autograd
                 # function reports its inputs' requires_grad also where gradients are off)
-                y = _mlp_forward(x2, *weights, self.w1.config, (False,) * 4, scales, operands, keep=False)[0]
-            return y.reshape(*x.shape[:-1], self.w2.weight.shape[0])
+                done = _planned_forward(x2, weights, c, (False,) * 4, scales, operands, False)
+                y = done[0][0] if done is not None else _mlp_forward(x2, *weights, c, (False,) * 4, scales, operands, keep=False)[0]
+            return y if xa.dim() == 2 else y.reshape(*x.shape[:-1], y.shape[1])
         x1, x3 = self.w1(x), self.w3(x)
         if x1.is_cuda and x1.dtype == torch.bfloat16 and not compiling:
             h = swiglu(x1, x3)

@@ -18,7 +18,7 @@ import math
 import torch
 import torch.nn as nn
 
-from ..float8 import ops
+from ..float8 import ops, plan
 from ..float8.linear import needs_autograd
 
 __all__ = ["DroplessMoEMLP", "float8_dropless_mlp"]
@@ -226,6 +226,18 @@ def _forward_only(x, w1, w2, w3, sizes, E, pow2, indices, top_k, kept, scatter_w
     return y
 
 
+def _planned_forward_only(x, w1, w2, w3, sizes, E, pow2, indices, top_k, kept, scatter_weights):
+    """:func:`_forward_only` with kept weights from a plan, or ``None``."""
+    (w1q, s1, _, _), (w3q, s3, _, _), (_, _, w2t, s2) = kept
+
+    def recorded(px, p1, p2, p3, psizes, pindices, pweights, q1, t1, q3, t3, q2, t2):
+        made = ((q1, t1, None, None), (q3, t3, None, None), (None, None, q2, t2))
+        return [_forward_only(px, p1, p2, p3, psizes, E, pow2, pindices, top_k, made, pweights)], None
+
+    done = plan.call(recorded, [x, w1, w2, w3, sizes, indices, scatter_weights, w1q, s1, w3q, s3, w2t, s2], ("experts", E, pow2, top_k))
+    return None if done is None else done[0][0]
+
+
 @torch.compiler.disable
 def float8_dropless_mlp(x, w1, w2, w3, batch_size_per_expert, num_experts: int, pow2: bool = True, indices=None,
                         top_k: int = 1, kept=None, scatter_weights=None):
@@ -238,7 +250,9 @@ def float8_dropless_mlp(x, w1, w2, w3, batch_size_per_expert, num_experts: int, 
     differentiable = (x, w1, w2, w3) if scatter_weights is None else (x, w1, w2, w3, scatter_weights)
     if (STAGE_SINK is None and x.dtype == torch.bfloat16 and x.numel() and max(x.shape[1], w1.shape[0] // num_experts) <= 65536
             and not needs_autograd(*differentiable)):  # (the per-row casts hold a row of at most 65536 in registers)
-        return _forward_only(x, w1, w2, w3, batch_size_per_expert, num_experts, pow2, indices, top_k, kept, scatter_weights)
+        args = (x, w1, w2, w3, batch_size_per_expert, num_experts, pow2, indices, top_k, kept, scatter_weights)
+        y = _planned_forward_only(*args) if kept is not None else None
+        return _forward_only(*args) if y is None else y
     return _Float8DroplessMLP.apply(x, w1, w2, w3, batch_size_per_expert, num_experts, pow2, indices, top_k, kept,
                                     scatter_weights)
 

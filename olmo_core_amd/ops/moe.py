@@ -22,13 +22,10 @@ from typing import Any, Optional
 import torch
 
 from .. import _C
+from ..float8.ops import _empty, _stream
 
 _DT = {torch.bfloat16: _C.MI8_BF16, torch.float32: _C.MI8_F32, torch.float16: _C.MI8_F16}
 _RAW = (torch.float8_e4m3fn, torch.float8_e5m2, torch.uint8, torch.int8)
-
-
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _dt(x: torch.Tensor, what: str, allow_raw: bool = False) -> int:
@@ -110,9 +107,9 @@ def _scatter(x, indices, weights, top_k: int) -> torch.Tensor:
         raise ValueError(f"scatter: {n} rows, {indices.shape[0]} indices, top_k {top_k} do not fit together")
     tokens = n // top_k
     w, wp, wd = _weights(weights, n, "scatter")
-    out = torch.empty((tokens, hidden), dtype=x.dtype, device=x.device)
+    out = _empty((tokens, hidden), dtype=x.dtype, device=x.device)
     if out.numel():
-        inverse = torch.empty(n, dtype=torch.int32, device=x.device)
+        inverse = _empty(n, dtype=torch.int32, device=x.device)
         _C.check(
             _C.lib().mi8_moe_scatter(x.data_ptr(), _dt(x, "scatter"), tokens, hidden, indices.data_ptr(), wp, wd, top_k,
                                      inverse.data_ptr(), out.data_ptr(), _stream(x)),
