@@ -189,10 +189,12 @@ __device__ __forceinline__ uint2 quantise8(uint4 v, float s)
                       quant4<MI8_E4M3, false>(f[4], f[5], f[6], f[7], s, s, s, s));
 }
 
-template <int MT, int U, int KIND, bool DUAL>
-__global__ __launch_bounds__(kFewThreads, MT == 1 ? 6 : MT == 2 ? 4 : 2) void few_rows_kernel(FewRowsArgs a)
+// WHOLE: a wave's share of K is at most U steps, all of which it requests at the start.
+template <int MT, int U, int KIND, bool DUAL, bool WHOLE>
+__global__ __launch_bounds__(kFewThreads, WHOLE ? (U > 8 ? 2 : 4) : MT == 1 ? 6 : MT == 2 ? 4 : 2) void few_rows_kernel(FewRowsArgs a)
 {
     constexpr int NB = DUAL ? 2 : 1;
+    constexpr int UX = WHOLE ? 1 : U;  // steps of A read ahead
     extern __shared__ __attribute__((aligned(16))) uint8_t aq[];  // kSlots, kAmax: A in e4m3, [M][K]
     __shared__ v4f red[kSkinnyWaves][MT][64];
     __shared__ uint32_t smem[kSkinnyWaves];
@@ -211,11 +213,11 @@ __global__ __launch_bounds__(kFewThreads, MT == 1 ? 6 : MT == 2 ? 4 : 2) void fe
     const uint8_t* wp[NB];
     wp[0] = g.B + (int64_t)n_row * g.ldb + kg * 32;
     if constexpr (DUAL) wp[1] = a.B3 + (int64_t)n_row * g.ldb + kg * 32;
-    v4i w[U][NB][2], w_next[U][NB][2];
+    v4i w[U][NB][2], w_next[WHOLE ? 1 : U][NB][2];
     auto inside = [&](int s, int h) { return s < s_end && s * kStep + kg * 32 + 16 * h < g.K; };
-    auto load_w = [&](v4i(&to)[U][NB][2], int s) {
+    auto load_w = [&](auto& to, int s) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < (int)(sizeof(to) / sizeof(to[0])); ++u)
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -278,44 +280,54 @@ __global__ __launch_bounds__(kFewThreads, MT == 1 ? 6 : MT == 2 ? 4 : 2) void fe
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[nb][mt] = v4f{0, 0, 0, 0};
 
-    v4i x[U][MT][2], x_next[U][MT][2];
-    auto load_x = [&](v4i(&to)[U][MT][2], int s) {
+    v4i x[UX][MT][2], x_next[UX][MT][2];
+    auto load_x = [&](v4i(&to)[UX][MT][2], int s) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < UX; ++u)
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
                     to[u][mt][h] = load16(xp[mt] + (int64_t)(s + u) * kStep + 16 * h, inside(s + u, h));
     };
-    load_x(x, s_begin);
-    for (int s = s_begin; s < s_end; s += U) {
-        load_w(w_next, s + U);
-        load_x(x_next, s + U);
+    auto step = [&](const v4i(&xs)[MT][2], const v4i(&ws)[NB][2]) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
+        for (int mt = 0; mt < MT; ++mt) {
+            const v8i fx = __builtin_shufflevector(xs[mt][0], xs[mt][1], 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const v8i fx = __builtin_shufflevector(x[u][mt][0], x[u][mt][1], 0, 1, 2, 3, 4, 5, 6, 7);
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) {
-                    const v8i fw = __builtin_shufflevector(w[u][nb][0], w[u][nb][1], 0, 1, 2, 3, 4, 5, 6, 7);
-                    acc[nb][mt] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fw, fx, acc[nb][mt], 0, 0, 0, 0, 0, 0);
-                }
+            for (int nb = 0; nb < NB; ++nb) {
+                const v8i fw = __builtin_shufflevector(ws[nb][0], ws[nb][1], 0, 1, 2, 3, 4, 5, 6, 7);
+                acc[nb][mt] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fw, fx, acc[nb][mt], 0, 0, 0, 0, 0, 0);
             }
         }
+    };
+    load_x(x, s_begin);
+    if constexpr (WHOLE) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {  // (steps past the share multiply zeros)
+            if (s_begin + u >= s_end) break;
+            load_x(u & 1 ? x : x_next, s_begin + u + 1);
+            step(u & 1 ? x_next[0] : x[0], w[u]);
+        }
+    } else {
+        for (int s = s_begin; s < s_end; s += U) {
+            load_w(w_next, s + U);
+            load_x(x_next, s + U);
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
+            for (int u = 0; u < U; ++u) step(x[u], w[u]);
 #pragma unroll
-                for (int h = 0; h < 2; ++h) w[u][nb][h] = w_next[u][nb][h];
+            for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+                for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+                    for (int h = 0; h < 2; ++h) w[u][nb][h] = w_next[u][nb][h];
 #pragma unroll
-                for (int h = 0; h < 2; ++h) x[u][mt][h] = x_next[u][mt][h];
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) x[u][mt][h] = x_next[u][mt][h];
+        }
     }
 
     const int m = (wave < MT ? wave : 0) * 16 + r16;  // wave mt finishes block mt of the rows of A
@@ -354,15 +366,15 @@ __global__ __launch_bounds__(kFewThreads, MT == 1 ? 6 : MT == 2 ? 4 : 2) void fe
     }
 }
 
-template <int MT, int U, int KIND, bool DUAL>
+template <int MT, int U, int KIND, bool DUAL, bool WHOLE = false>
 int launch_few_rows(const FewRowsArgs& a, hipStream_t st, const char* what)
 {
     static std::atomic<uint64_t> configured;
     if constexpr (KIND == kSlots)
-        if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(few_rows_kernel<MT, U, KIND, DUAL>), kLdsElems, configured, what))
+        if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(few_rows_kernel<MT, U, KIND, DUAL, WHOLE>), kLdsElems, configured, what))
             return rc;
     const int lds = KIND == kFp8 ? 0 : a.g.M * a.g.K;  // (K % 16 == 0)
-    hipLaunchKernelGGL((few_rows_kernel<MT, U, KIND, DUAL>), dim3((a.g.N + 15) / 16), dim3(kFewThreads), lds, st, a);
+    hipLaunchKernelGGL((few_rows_kernel<MT, U, KIND, DUAL, WHOLE>), dim3((a.g.N + 15) / 16), dim3(kFewThreads), lds, st, a);
     return launch_status(what);
 }
 
@@ -438,5 +450,14 @@ extern "C" int mi8_few_rows_cast_gemm(const void* x, int64_t lda, const uint32_t
     a.slots_in = slots;
     a.n_slots = n_slots;
     a.pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
-    return launch_few_rows<1, 2, kSlots, false>(a, (hipStream_t)stream, "mi8_few_rows_cast_gemm");
+    // Where all workgroups fit on the chip at once with the registers for it (one to a compute unit up to N = 4096, two up to
+    // 8192 and eight steps), each wave requests its whole share of K before the maxima are folded and A is converted: all of
+    // B is under way meanwhile.
+    const char* what = "mi8_few_rows_cast_gemm";
+    hipStream_t st = (hipStream_t)stream;
+    const int share = eighth_steps(K);
+    if (N <= 8192 && share <= 4) return launch_few_rows<1, 4, kSlots, false, true>(a, st, what);
+    if (N <= 8192 && share <= 8) return launch_few_rows<1, 8, kSlots, false, true>(a, st, what);
+    if (N <= 4096 && share <= 12) return launch_few_rows<1, 12, kSlots, false, true>(a, st, what);
+    return launch_few_rows<1, 2, kSlots, false>(a, st, what);
 }
