@@ -137,6 +137,7 @@ _SIGNATURES = {
     "mi8_plan_function": (c_int, [c_char_p]),
     "mi8_run_plan": (c_int, [c_void_p, c_int64, c_void_p, c_int32, c_void_p]),
     "mi8_gemm_fp8_swiglu_slots": (c_int32, [c_int64, c_int64, c_int64]),
+    "mi8_few_rows_swiglu_slots": (c_int32, [c_int64, c_int64, c_int64, c_int]),
     "mi8_few_rows_swiglu": (
         c_int,
         [c_void_p, c_int, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p,

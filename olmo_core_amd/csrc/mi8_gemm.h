@@ -23,6 +23,10 @@ struct GemmArgs {
     int tiles_m, tiles_n;
     int accumulate;  // add the rounded product to what C holds (the sum of two grad_input halves) instead of overwriting
     int slice_steps;  // (ring tiles with SLICED) K steps summed from zero before they join the sum
+    // (ring tiles with DUAL) the second matrix and its scale, and a partial maximum of |C| per workgroup
+    const uint8_t* B3;
+    const float* sb3;
+    uint32_t* slots_out;
 };
 
 
@@ -122,6 +126,10 @@ inline __host__ __device__ int eighth_steps(int64_t K)
     return (steps + 7) / 8;
 }
 int launch_skinny(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st);
+// C = h = silu(A B^T) * (A B3^T) of e4m3 operands, single scales, up to 64 rows of A, on ring tiles of 64 rows by 32 columns of
+// each product (mi8_gemm.hip); writes dual_ring_slots(N) partial maxima
+int launch_dual_ring(GemmArgs& g, hipStream_t st);
+inline int dual_ring_slots(int64_t N) { return (int)((N + 31) / 32); }
 // the same kernel over the ragged grouped problems (bf16 output, per-row / per-column scale vectors):
 // forward / grad_input (T, N >= 256, K % 128 == 0) and grad_weight (N, Kl >= 256)
 int launch_m16_grouped(const uint8_t* a, int a_dtype, int64_t lda, const uint8_t* b, int b_dtype, int64_t ldb,

@@ -22,6 +22,17 @@ __global__ __launch_bounds__(NW * 64, OCC) void gemm_fp8_ring_kernel(GemmArgs g)
     ring_tile<BM, BN, ST, CBSZ, BLGP, SLICED, NW>(g, tm * BM, tn * BN, lds);
 }
 
+// A few rows through both input projections of a SwiGLU block and the activation (see ring_tile); K in eighths.  Bound by
+// reading the weights, 3.7 TB/s at 90 MB and 5.0 at 283 (weights from HBM; six stages instead of four change nothing).
+template <int BM>
+__global__ __launch_bounds__(kRingThreads, BM == 32 ? 3 : 2) void dual_ring_kernel(GemmArgs g)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    int tm, tn;
+    if (!tile_of_block(g, tm, tn)) return;
+    ring_tile<BM, 64, 4, 0, 0, true, kRingThreads / 64, true>(g, 0, tn * 32, lds);
+}
+
 // ---- split K ---------------------------------------------------------------------------------------
 // A problem with few output tiles and a long K leaves most compute units idle while every busy one pays a
 // memory latency per 128-byte K step.  Here blockIdx.y cuts K into slices: every (tile, slice) workgroup runs
@@ -335,6 +346,19 @@ int launch_ring_typed(int shape, int a_dtype, int b_dtype, GemmArgs& g, SplitArg
         return b_dtype == MI8_E4M3 ? launch_ring_shape<0, 0>(shape, g, split, st) : launch_ring_shape<0, 1>(shape, g, split, st);
     return b_dtype == MI8_E4M3 ? launch_ring_shape<1, 0>(shape, g, split, st) : launch_ring_shape<1, 1>(shape, g, split, st);
 }
+
+}  // namespace
+int gemm::launch_dual_ring(GemmArgs& g, hipStream_t st)
+{
+    g.tiles_m = 1;
+    g.tiles_n = dual_ring_slots(g.N);
+    g.slice_steps = eighth_steps(g.K);
+    static std::atomic<uint64_t> configured[2];
+    const char* what = "mi8_few_rows_swiglu";
+    if (g.M <= 32) return launch_ring_kernel(dual_ring_kernel<32>, configured[0], kRingLdsBytes<32, 64, 4>, g, g.tiles_n, 1, kRingThreads, st, what);
+    return launch_ring_kernel(dual_ring_kernel<64>, configured[1], kRingLdsBytes<64, 64, 4>, g, g.tiles_n, 1, kRingThreads, st, what);
+}
+namespace {
 
 // ---- several products in one launch: launch and cost ------------------------------------------------------------------
 

@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "mi8_gemm.h"
+#include "mi8_swiglu.h"
 
 namespace mi8 {
 namespace gemm {
@@ -52,6 +53,20 @@ __device__ __forceinline__ void ring_wait()
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x70);
 }
 
+// the same for all but the loads of `steps` steps (0 .. MOST) of LD loads each
+template <int LD, int MOST>
+__device__ __forceinline__ void ring_wait_steps(int steps)
+{
+    if constexpr (MOST == 0) {
+        ring_wait<0>();
+    } else {
+        if (steps >= MOST)
+            ring_wait<LD * MOST>();
+        else
+            ring_wait_steps<LD, MOST - 1>(steps);
+    }
+}
+
 template <int BM, int BN, int ST>
 constexpr int kRingLdsBytes = ST * (BM + BN) * BK;
 
@@ -60,7 +75,9 @@ constexpr int kRingThreads = 256;
 // C[m0 .. m0 + BM, n0 .. n0 + BN] of g's product (K may be 0: zeros).  g.sa == null: the raw fp32 sums are wanted.
 // SLICED: K is summed in slices of g.slice_steps, each from zero, added in order (the sums of split K without its planes).
 // NW waves, two of them side by side along M.
-template <int BM, int BN, int ST, int CBSZ, int BLGP, bool SLICED = false, int NW = kRingThreads / 64>
+// DUAL (32 or 64 rows by 64 B rows, single scales): C[.., n0 .. n0 + 32] = silu(A B^T) * (A B3^T).  B rows 32 w .. of the stage, those of the
+// wave column w, are 16 rows of B and the same 16 of B3, so that a lane holds both products of the same elements.
+template <int BM, int BN, int ST, int CBSZ, int BLGP, bool SLICED = false, int NW = kRingThreads / 64, bool DUAL = false>
 __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const int n0, uint8_t* lds)
 {
     constexpr int WAVES_N = NW / 2;
@@ -68,7 +85,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
     constexpr int TM = WTM / 16, TN = WTN / 16;
     constexpr int STAGE = (BM + BN) * BK;
     constexpr int LA = BM / 8 / NW, LB = BN / 8 / NW, LD = LA + LB;  // loads per wave and step: 8 rows x 128 bytes each
-    static_assert(LA * 8 * NW == BM && LB * 8 * NW == BN && ST >= 2 && ST <= 4 && LD * (ST - 2) < 64, "tile shape");
+    static_assert(LA * 8 * NW == BM && LB * 8 * NW == BN && ST >= 2 && LD * (ST - 1) < 64, "tile shape");
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -76,17 +93,21 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
     const int r16 = lane & 15, kb = lane >> 4;
 
     // ---- operand loads: load i of wave w fills rows 8 (NW i + w) .. + 7; rows past the edge re-read the last one
-    const int rows_a = g.M - m0 < BM ? g.M - m0 : BM, rows_b = g.N - n0 < BN ? g.N - n0 : BN;
+    constexpr int BNC = DUAL ? BN / 2 : BN;  // columns of C
+    static_assert(!DUAL || (BM <= 64 && BN == 64 && NW == 4 && TN == 2), "dual tile shape");
+    const int rows_a = g.M - m0 < BM ? g.M - m0 : BM, rows_b = g.N - n0 < BNC ? g.N - n0 : BNC;
+    const uint8_t* const b_base = DUAL && (wave & 2) ? g.B3 : g.B;  // (a wave's loads of B are of one matrix)
     const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(g.A + (int64_t)m0 * g.lda), 0, (int)(uint32_t)((int64_t)(rows_a - 1) * g.lda + g.K), 0x00020000);
     const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(g.B + (int64_t)n0 * g.ldb), 0, (int)(uint32_t)((int64_t)(rows_b - 1) * g.ldb + g.K), 0x00020000);
+        (void*)(b_base + (int64_t)n0 * g.ldb), 0, (int)(uint32_t)((int64_t)(rows_b - 1) * g.ldb + g.K), 0x00020000);
     const int lr = lane >> 3, chunk16 = ((lane & 7) ^ swz16(lr)) * 16;
     int off[LD];
 #pragma unroll
     for (int i = 0; i < LD; ++i) {
         const bool is_a = i < LA;
         int r = 8 * (NW * (is_a ? i : i - LA) + wave) + lr;
+        if (DUAL && !is_a) r = 16 * (r >> 5) + (r & 15);
         const int last = (is_a ? rows_a : rows_b) - 1;
         r = r < last ? r : last;
         off[i] = (int)((uint32_t)r * (uint32_t)(is_a ? g.lda : g.ldb)) + chunk16;
@@ -203,12 +224,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
             // later steps may be in flight); after the barrier every wave's
             constexpr bool kSteady = decltype(steady_tag)::value;
             const int ahead = kSteady ? ST - 2 : nk - 2 - k;
-            if (ahead >= ST - 2)
-                ring_wait<LD * (ST - 2)>();
-            else if (ST > 3 && ahead == 1)
-                ring_wait<LD>();
-            else
-                ring_wait<0>();
+            ring_wait_steps<LD, ST - 2>(ahead);
             asm volatile("s_barrier" ::: "memory");
             if constexpr (kSteady) {
                 body(std::true_type{}, std::true_type{});
@@ -226,14 +242,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
 #pragma unroll
             for (int s = 0; s < ST; ++s)
                 if (s < nk) issue(s, s);
-            if (nk >= ST)
-                ring_wait<LD * (ST - 1)>();
-            else if (ST > 3 && nk == 3)
-                ring_wait<LD * 2>();
-            else if (ST > 2 && nk == 2)
-                ring_wait<LD>();
-            else
-                ring_wait<0>();
+            ring_wait_steps<LD, ST - 1>(nk - 1);
             asm volatile("s_barrier" ::: "memory");
             const ReadAt at = read_at(0);
 #pragma unroll
@@ -258,13 +267,7 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
         int slot = 0;
         for (int k = 0; k < nk; ++k) {
             // this wave's loads of step k have landed (those of up to ST - 2 later steps may be in flight) ...
-            const int ahead = nk - 1 - k;
-            if (ahead >= ST - 2)
-                ring_wait<LD * (ST - 2)>();
-            else if (ST > 3 && ahead == 1)
-                ring_wait<LD>();
-            else
-                ring_wait<0>();
+            ring_wait_steps<LD, ST - 2>(nk - 1 - k);
             // ... every wave's have, and every wave has its fragments of step k - 1, whose slot is filled next
             asm volatile("s_barrier" ::: "memory");
             if (k + ST - 1 < nk) issue(k + ST - 1, slot == 0 ? ST - 1 : slot - 1);
@@ -285,6 +288,29 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
             for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j] + acc[i][j];
     }
 
+    if constexpr (DUAL) {
+        const float isa = 1.0f / g.sa[0], f1 = isa * (1.0f / g.sb[0]), f3 = isa * (1.0f / g.sb3[0]);
+        const int col = n0 + 16 * wn + 4 * kb;  // (N % 8 == 0)
+        uint32_t hm = 0;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int row = m0 + wm * WTM + 16 * i + r16;
+            const ring_v4f x1 = acc[i][0], x3 = acc[i][TN - 1];
+            const uint2 h = swiglu_fwd4(make_uint2(pack_bf16x2(x1[0] * f1, x1[1] * f1), pack_bf16x2(x1[2] * f1, x1[3] * f1)),
+                                        make_uint2(pack_bf16x2(x3[0] * f3, x3[1] * f3), pack_bf16x2(x3[2] * f3, x3[3] * f3)));
+            if (row < g.M && col < g.N) {
+                *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.C) + (int64_t)row * g.ldc + col) = h;
+                hm = umax32(hm, (max_code8(h.x, h.y, h.x, h.y) & 0xFFFFu) << 16);
+            }
+        }
+        hm = wave_umax(hm);
+        __syncthreads();  // (the ring is free now)
+        uint32_t* maxima = reinterpret_cast<uint32_t*>(lds);
+        if (lane == 0) maxima[wave] = hm;
+        __syncthreads();
+        if (tid == 0) g.slots_out[n0 / BNC] = umax32(umax32(maxima[0], maxima[1]), umax32(maxima[2], maxima[3]));
+        return;
+    }
     // ---- epilogue: acc[i][j][e] of lane l is C[row = 16 i + l % 16][col = 16 j + 4 (l / 16) + e] of the wave tile.
     // Single scales are inverted with an IEEE division, scale vectors with v_rcp_f32 (exact for the power-of-two scales
     // of the axiswise recipes, within 1 ulp otherwise).

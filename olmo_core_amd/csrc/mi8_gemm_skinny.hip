@@ -397,6 +397,23 @@ int launch_skinny(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st)
 using namespace mi8;
 using namespace mi8::gemm;
 
+namespace {
+// Whether the float8 rows go to the ring tiles (mi8_gemm.hip), which fetch A once per 32 columns of both products where the
+// kernel above reads it from L2 for every 16: more rows, or more bytes of weights, make that the time.  us, above / ring:
+// 16 x 8192 x 2048 9.9 / 9.0, 23 x 11008 x 4096 28.5 / 25.3, 48 x 11008 x 4096 43.6 / 27.1, 64 x 8192 x 2048 18.5 / 9.3,
+// 4 x 27648 x 5120 66.6 / 56.6, 64 x 27648 x 5120 135 / 70; 8 x 11008 x 4096 24.3 / 24.2, 32 x 2816 x 1024 5.6 / 5.8.
+bool dual_on_ring(int64_t M, int64_t H, int64_t K)
+{
+    const int64_t bytes = 2 * H * K;
+    return M > 32 || (bytes >= 16 << 20 && M > 8) || (bytes >= 200 << 20 && M > 3);
+}
+}  // namespace
+
+extern "C" int32_t mi8_few_rows_swiglu_slots(int64_t M, int64_t H, int64_t K, int x_is_fp8)
+{
+    return x_is_fp8 && dual_on_ring(M, H, K) ? dual_ring_slots(H) : (int32_t)((H + 15) / 16);
+}
+
 extern "C" int mi8_few_rows_swiglu(const void* x, int x_is_fp8, int64_t lda, const float* sx, const void* b1, const void* b3,
                                    int64_t ldb, int64_t M, int64_t H, int64_t K, const float* sb1, const float* sb3,
                                    uint32_t flags, void* h, uint32_t* slots_h, int32_t* n_slots_used, void* stream)
@@ -422,9 +439,15 @@ extern "C" int mi8_few_rows_swiglu(const void* x, int x_is_fp8, int64_t lda, con
     a.sb3 = sb3;
     a.pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
     a.slots_out = slots_h;
-    *n_slots_used = (int32_t)((H + 15) / 16);
+    *n_slots_used = mi8_few_rows_swiglu_slots(M, H, K, x_is_fp8);
     hipStream_t st = (hipStream_t)stream;
     if (!x_is_fp8) return launch_few_rows<1, 1, kAmax, true>(a, st, "mi8_few_rows_swiglu");
+    if (dual_on_ring(M, H, K)) {
+        a.g.B3 = a.B3;
+        a.g.sb3 = sb3;
+        a.g.slots_out = slots_h;
+        return launch_dual_ring(a.g, st);
+    }
     if (M <= 16) return launch_few_rows<1, 1, kFp8, true>(a, st, "mi8_few_rows_swiglu");
     if (M <= 32) return launch_few_rows<2, 1, kFp8, true>(a, st, "mi8_few_rows_swiglu");
     return launch_few_rows<4, 1, kFp8, true>(a, st, "mi8_few_rows_swiglu");

@@ -170,7 +170,7 @@ class _Recorder:
         if name == "mi8_amax_partials":
             return self.real.mi8_amax_slots_for(args[2])
         if name == "mi8_few_rows_swiglu":
-            return (args[8] + 15) // 16
+            return self.real.mi8_few_rows_swiglu_slots(*args[7:10], args[1])
         if name == "mi8_gemm_fp8_swiglu":
             return self.real.mi8_gemm_fp8_swiglu_slots(*args[7:10])
         raise Unplannable(name)

@@ -637,3 +637,17 @@ def test_products_in_one_launch_refuse_what_one_launch_cannot_take(dev):
     with pytest.raises(MI8KernelError, match="multiples of 16"):
         ops.gemm_fp8_batch([(a, one, a, one, 40, False)] * 2, together=True)
     assert len(ops.gemm_fp8_batch([(a, one, a, one, None, False)] * 9)) == 9
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M, H, K", [(33, 8, 16), (64, 264, 272), (48, 72, 2064), (9, 8192, 1040), (32, 2056, 4112), (23, 4096, 2048)])
+def test_few_rows_swiglu_on_ring_tiles(dev, M, H, K):
+    """h and its maxima have the bits of the separate launches: columns that end inside a tile, a ragged K, 32 and 64 row tiles."""
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    x, w1, w3 = (torch.randn(n, K, generator=g, device=dev).to(torch.float8_e4m3fn) for n in (M, H, H))
+    sx, s1, s3 = (torch.full((1,), v, device=dev) for v in (3.0, 5.0, 7.0))
+    h, (slots, n) = ops.few_rows_swiglu(x, sx, w1, s1, w3, s3)
+    x1, x3 = ops.gemm_fp8(x, sx, w1, s1), ops.gemm_fp8(x, sx, w3, s3)
+    want, _ = ops.swiglu_fwd(x1, x3)
+    assert torch.equal(h, want) and n == (H + 31) // 32
+    assert slots[:n].max().item() == h.abs().float().max().view(1).view(torch.int32).item()
