@@ -46,7 +46,8 @@ typedef enum mi8_hp {
     MI8_BF16 = 0,
     MI8_F32 = 1,
     MI8_F16 = 2,  /* token-permutation entry points only */
-    MI8_RAW8 = 3  /* opaque 1-byte elements (fp8 rows): unweighted permutation only */
+    MI8_RAW8 = 3, /* opaque 1-byte elements (fp8 rows): unweighted permutation only */
+    MI8_F32_OF_BF16 = 4 /* GEMM outputs only: float32 that holds the values a bf16 output would (gradients of float32 weights) */
 } mi8_hp;
 
 /* flags shared by the cast entry points */
@@ -211,7 +212,7 @@ int mi8_cast_colwise_t(const void* x, int hp_dtype, int64_t rows, int64_t cols, 
  *   A: fp8 [M, lda] row-major, B: fp8 [N, ldb] row-major - both operands K-contiguous; K % 16 == 0,
  *   lda, ldb % 16 == 0.  a_dtype / b_dtype may differ (e5m2 x e4m3 for the gradient GEMMs).
  *   sa: quantisation scale(s) of A - one float32 if sa_rows == 0, else float32 [M]; sb likewise ([N]).
- *   out: [M, ldc] of out_dtype (MI8_BF16 or MI8_F32), ldc >= N.
+ *   out: [M, ldc] of out_dtype (MI8_BF16, MI8_F32 or MI8_F32_OF_BF16), ldc >= N.
  *   variant: -1 picks a tile configuration from the shape; 0..mi8_gemm_num_variants()-1 forces one.
  * ------------------------------------------------------------------------------------------- */
 int mi8_gemm_fp8(const void* a, int a_dtype, int64_t lda, const void* b, int b_dtype, int64_t ldb, int64_t M,

@@ -21,7 +21,7 @@ import os
 LIB_PATH = Path(os.environ.get("MI8_LIBRARY") or (Path(__file__).resolve().parent / "lib" / "libmi8.so"))
 
 MI8_E4M3, MI8_E5M2 = 0, 1
-MI8_BF16, MI8_F32, MI8_F16, MI8_RAW8 = 0, 1, 2, 3
+MI8_BF16, MI8_F32, MI8_F16, MI8_RAW8, MI8_F32_OF_BF16 = 0, 1, 2, 3, 4
 FLAG_POW2_SCALE = 1
 FLAG_SW_CVT = 2
 FLAG_AMAX_READY = 4

@@ -10,11 +10,14 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 constexpr int BK = 128;  // bytes of K per LDS stage
 
+inline int c_f32_of(int out_dtype) { return out_dtype == MI8_BF16 ? 0 : out_dtype == MI8_F32 ? 1 : 2; }
+inline bool gemm_out_dtype(int v) { return v == MI8_BF16 || v == MI8_F32 || v == MI8_F32_OF_BF16; }
+
 struct GemmArgs {
     const uint8_t* A;
     const uint8_t* B;
     void* C;
-    int c_f32;
+    int c_f32;  // 0: bf16, 1: float32, 2: float32 that holds the bf16 values
     int64_t lda, ldb, ldc;
     int M, N, K;
     const float* sa;
@@ -43,6 +46,8 @@ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f)
     __bf16 h = (__bf16)f;  // round-to-nearest-even; v_cvt_pk_bf16_f32 on gfx950
     return __builtin_bit_cast(uint16_t, h);
 }
+
+__device__ __forceinline__ float round_to_bf16(float f) { return bits_to_f32((uint32_t)f32_to_bf16_bits(f) << 16); }
 
 // Two floats -> two bf16 (round-to-nearest-even) in one dword, low half first: a single v_cvt_pk_bf16_f32.
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));

@@ -102,7 +102,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(SplitArgs a)
     for (int j = 0; j < 4; ++j) {
         if (n + j >= g.N) break;
         const float isb = g.sb_vec ? __builtin_amdgcn_rcpf(g.sb[n + j]) : isb_single;
-        const float r = both_single ? s[j] * (isa * isb) : s[j] * isa * isb;
+        float r = both_single ? s[j] * (isa * isb) : s[j] * isa * isb;
+        if (g.c_f32 == 2) r = round_to_bf16(r);
         if (g.c_f32) {
             float* c = reinterpret_cast<float*>(g.C) + (int64_t)m * g.ldc + n + j;
             *c = g.accumulate ? *c + r : r;
@@ -450,7 +451,8 @@ namespace {
 // accumulating.  Its output stores address a tile's 256 rows with 32-bit byte offsets: ldc < 2^22.)
 bool m16_takes(int64_t M, int64_t N, int64_t K, int64_t ldc, int out_dtype, bool accumulate)
 {
-    return K % 128 == 0 && M >= 256 && N >= 256 && N % 8 == 0 && ldc % 8 == 0 && ldc < (1 << 22) && out_dtype == MI8_BF16 &&
+    return K % 128 == 0 && M >= 256 && N >= 256 && N % 8 == 0 && ldc % 8 == 0 && ldc < (out_dtype == MI8_BF16 ? 1 << 22 : 1 << 21) &&
+           (out_dtype == MI8_BF16 || (out_dtype == MI8_F32_OF_BF16 && !accumulate)) &&
            (!accumulate || (M % 128 == 0 && N % 256 == 0));
 }
 
@@ -506,9 +508,9 @@ int gemm_fp8_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b
     MI8_REQUIRE(M * lda < (int64_t)1 << 32 && N * ldb < (int64_t)1 << 32 && M < (1 << 30) && N < (1 << 30) &&
                     K < (1 << 30),
                 MI8_ERR_UNSUPPORTED, "mi8_gemm_fp8: operand larger than 4 GiB");
-    MI8_REQUIRE(out_dtype == MI8_BF16 || out_dtype == MI8_F32, MI8_ERR_ARG, "mi8_gemm_fp8: unknown output dtype %d",
+    MI8_REQUIRE(gemm_out_dtype(out_dtype), MI8_ERR_ARG, "mi8_gemm_fp8: unknown output dtype %d",
                 out_dtype);
-    GemmArgs g{(const uint8_t*)a, (const uint8_t*)b, out, out_dtype == MI8_F32 ? 1 : 0, lda, ldb, ldc, (int)M, (int)N, (int)K,
+    GemmArgs g{(const uint8_t*)a, (const uint8_t*)b, out, c_f32_of(out_dtype), lda, ldb, ldc, (int)M, (int)N, (int)K,
                sa, sb, sa_is_vector ? 1 : 0, sb_is_vector ? 1 : 0, 0, 0, accumulate ? 1 : 0};
     hipStream_t st = (hipStream_t)stream;
     const bool dma_ok = m16_takes(M, N, K, ldc, out_dtype, accumulate) && aligned16(out) && (!sb_is_vector || aligned16(sb)) &&
@@ -518,7 +520,7 @@ int gemm_fp8_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b
     if (variant == kM16) {
         MI8_REQUIRE(dma_ok, MI8_ERR_UNSUPPORTED,
                     "mi8_gemm_fp8: the direct-to-LDS variant needs M, N >= 256, K %% 128 == 0, N %% 8 == 0, ldc %% 8 == 0, "
-                    "scales that are both single values or both vectors, and a 16-byte aligned bf16 output (M=%lld N=%lld K=%lld ldc=%lld)",
+                    "scales that are both single values or both vectors, and a 16-byte aligned output of bf16 values (M=%lld N=%lld K=%lld ldc=%lld)",
                     (long long)M, (long long)N, (long long)K, (long long)ldc);
         return launch_m16(g, a_dtype, b_dtype, st);
     }
@@ -656,7 +658,7 @@ int splitk_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b_d
     MI8_REQUIRE(M * lda < (int64_t)1 << 32 && N * ldb < (int64_t)1 << 32 && M < (1 << 30) && N < (1 << 30) &&
                     K < (1 << 30),
                 MI8_ERR_UNSUPPORTED, "mi8_gemm_fp8_splitk: operand larger than 4 GiB");
-    MI8_REQUIRE(out_dtype == MI8_BF16 || out_dtype == MI8_F32, MI8_ERR_ARG,
+    MI8_REQUIRE(gemm_out_dtype(out_dtype), MI8_ERR_ARG,
                 "mi8_gemm_fp8_splitk: unknown output dtype %d", out_dtype);
     const int64_t steps = (K + BK - 1) / BK;
     MI8_REQUIRE(splits >= 1 && splits <= 64 && splits <= steps, MI8_ERR_ARG,
@@ -667,7 +669,7 @@ int splitk_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b_d
                 "mi8_gemm_fp8_splitk: workspace of %lld bytes, %lld needed", (long long)workspace_bytes,
                 (long long)mi8_gemm_splitk_workspace_bytes(M, N, used));
     SplitArgs s{};
-    s.g = GemmArgs{(const uint8_t*)a, (const uint8_t*)b, out, out_dtype == MI8_F32 ? 1 : 0, lda, ldb, ldc, (int)M,
+    s.g = GemmArgs{(const uint8_t*)a, (const uint8_t*)b, out, c_f32_of(out_dtype), lda, ldb, ldc, (int)M,
                    (int)N, (int)K, sa, sb, sa_is_vector ? 1 : 0, sb_is_vector ? 1 : 0, 0, 0, accumulate ? 1 : 0};
     s.planes = (float*)workspace;
     s.ld_plane = (N + 3) / 4 * 4;
@@ -735,11 +737,11 @@ int batch_args(const mi8_gemm_product* p, int32_t count, BatchArgs& a, bool& sli
         MI8_REQUIRE(aligned16(q.a) && aligned16(q.b), MI8_ERR_UNSUPPORTED, "%s: product %d: operands must be 16-byte aligned", what, i);
         MI8_REQUIRE(q.M < (1 << 30) && q.N < (1 << 30) && q.K < (1 << 30) && q.M * q.lda < (int64_t)1 << 32 && q.N * q.ldb < (int64_t)1 << 32,
                     MI8_ERR_UNSUPPORTED, "%s: product %d: operand larger than 4 GiB", what, i);
-        MI8_REQUIRE(q.out_dtype == MI8_BF16 || q.out_dtype == MI8_F32, MI8_ERR_ARG, "%s: product %d: unknown output dtype %d", what, i, q.out_dtype);
+        MI8_REQUIRE(gemm_out_dtype(q.out_dtype), MI8_ERR_ARG, "%s: product %d: unknown output dtype %d", what, i, q.out_dtype);
         MI8_REQUIRE(!q.add_to_previous || (i > 0 && q.M == p[i - 1].M && q.N == p[i - 1].N && q.out == p[i - 1].out && q.ldc == p[i - 1].ldc &&
                                            q.out_dtype == p[i - 1].out_dtype),
                     MI8_ERR_ARG, "%s: product %d adds to the one before it: one output and sizes are wanted", what, i);
-        a.g[i] = GemmArgs{(const uint8_t*)q.a, (const uint8_t*)q.b, q.out, q.out_dtype == MI8_F32 ? 1 : 0, q.lda, q.ldb, q.ldc, (int)q.M,
+        a.g[i] = GemmArgs{(const uint8_t*)q.a, (const uint8_t*)q.b, q.out, c_f32_of(q.out_dtype), q.lda, q.ldb, q.ldc, (int)q.M,
                           (int)q.N, (int)q.K, q.sa, q.sb, q.sa_is_vector ? 1 : 0, q.sb_is_vector ? 1 : 0, 0, 0, q.add_to_previous ? 1 : 0,
                           slice_steps_of(q.M, q.N, q.K)};
         sliced = sliced || a.g[i].slice_steps;
@@ -779,7 +781,7 @@ extern "C" int mi8_gemm_fp8_batch_pays(const mi8_gemm_product* products, int32_t
         const bool acc = g.accumulate != 0;
         float t;
         best_ring(g.M, g.N, ceil_div(g.K, BK), 1, &t, g.slice_steps != 0);
-        if (m16_takes(g.M, g.N, g.K, g.ldc, g.c_f32 ? MI8_F32 : MI8_BF16, acc) && aligned16(g.C) && !g.slice_steps) {
+        if (m16_takes(g.M, g.N, g.K, g.ldc, g.c_f32 == 0 ? MI8_BF16 : g.c_f32 == 1 ? MI8_F32 : MI8_F32_OF_BF16, acc) && aligned16(g.C) && !g.slice_steps) {
             const float p = m16_cost(g.M, g.N, g.K);
             t = p < t ? p : t;
         }

@@ -455,7 +455,8 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
                 else
                     __builtin_amdgcn_s_waitcnt(vmcnt(8 + 12 * kPasses));
             } else {
-                __builtin_amdgcn_s_waitcnt(vmcnt(8 + (Problem::kOutCodes ? 10 : 8) * kPasses));
+                constexpr int stores = (Problem::kOutF32 ? 16 : Problem::kOutCodes ? 10 : 8) * kPasses;
+                __builtin_amdgcn_s_waitcnt(vmcnt(8 + stores < 63 ? 8 + stores : 63));  // (the counter has six bits)
             }
         };
         auto k_step = [&](bool fresh, auto set_tag) __attribute__((always_inline)) {
@@ -616,7 +617,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
         const bool zero_tile = td.nk == 0;  // nothing accumulated; the scales may be unset
         const uint8_t* sc_slot = lds + 2 * STAGE + OUT_STAGING + (cp_seq & kSlotMask) * kSlotBytes;
         if (!zero_tile) ++cp_seq;
-        const int ldc_bytes = (int)pb.ldc * 2;
+        const int ldc_bytes = (int)pb.ldc * (Problem::kOutF32 ? 4 : 2);
         const uint32_t c_lane_off = (uint32_t)((lane >> 3) * ldc_bytes + (lane & 7) * 16);
         __amdgpu_buffer_rsrc_t c_rows;
         if constexpr (Problem::kMaskRows)
@@ -625,6 +626,8 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
         // memory only after the arithmetic of the next pass, so that each pass exposes one LDS round trip instead
         // of two.
         v4i staged[4];  // (an ext-vector type: arrays of HIP's uint4 struct end up in scratch)
+        // kOutF32: a lane takes four bf16 values at a time, stored as 16 bytes of float32 (whole 128-byte lines per store:
+        // eight stores a pass); staged[it] holds those of the row's two halves
         // Accumulating problems (C += product): what C holds at the addresses of a pass is fetched one pass ahead
         // of the stores that replace it, with the same coalesced 16-byte accesses, and added to the staged rows as
         // an elementwise bf16 add would (float32 sum of the two bf16 values, one rounding).
@@ -691,10 +694,22 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
             } else {
                 // the tile's 256 rows as one buffer: a uniform offset per instruction + one lane offset shared by all passes
                 const __amdgpu_buffer_rsrc_t c_tile = out_rows(td.c, 256 * ldc_bytes);
+                if constexpr (Problem::kOutF32) {
+#pragma unroll
+                    for (int it = 0; it < 4; ++it)
+#pragma unroll
+                        for (int half = 0; half < 2; ++half) {
+                            const uint32_t a = (uint32_t)staged[it][2 * half], b = (uint32_t)staged[it][2 * half + 1];
+                            const v4i v = {(int)(a << 16), (int)(a & 0xFFFF0000u), (int)(b << 16), (int)(b & 0xFFFF0000u)};
+                            __builtin_amdgcn_raw_buffer_store_b128(v, c_tile, c_lane_off,
+                                                                   (rt + it * 8) * ldc_bytes + (wn * WT + jq * 64 + half * 32) * 4, kOutStoreAux);
+                        }
+                } else {
 #pragma unroll
                 for (int it = 0; it < 4; ++it)
                     __builtin_amdgcn_raw_buffer_store_b128(staged[it], c_tile, c_lane_off,
                                                            (rt + it * 8) * ldc_bytes + (wn * WT + jq * 64) * 2, kOutStoreAux);
+                }
             }
         };
         if constexpr (Problem::kSwiglu) {
@@ -876,7 +891,17 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
 #pragma unroll
                 for (int it = 0; it < 4; ++it) {
                     const int rw = it * 8 + (lane >> 3);
-                    staged[it] = *reinterpret_cast<const v4i*>(stg + rw * 128 + (((lane & 7) ^ ((rw >> 1) & 7)) << 4));
+                    if constexpr (Problem::kOutF32) {
+#pragma unroll
+                        for (int half = 0; half < 2; ++half) {
+                            const int chunk = (half * 4 + ((lane & 7) >> 1)) ^ ((rw >> 1) & 7);
+                            const uint2 v = *reinterpret_cast<const uint2*>(stg + rw * 128 + chunk * 16 + (lane & 1) * 8);
+                            staged[it][2 * half] = (int)v.x;
+                            staged[it][2 * half + 1] = (int)v.y;
+                        }
+                    } else {
+                        staged[it] = *reinterpret_cast<const v4i*>(stg + rw * 128 + (((lane & 7) ^ ((rw >> 1) & 7)) << 4));
+                    }
                 }
                 asm volatile("" ::: "memory");
             }
@@ -1046,6 +1071,10 @@ int launch_m16(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st)
 {
     g.tiles_n = (g.N + BN - 1) / BN;
     const HalfRows rows = plan_halves(g, num_compute_units());
+    if (g.c_f32) {
+        if (g.sa_vec) return launch_typed(DenseProblem<true, false, false, true>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);
+        return launch_typed(DenseProblem<false, false, false, true>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);
+    }
     if (g.sa_vec) {
         if (g.accumulate) return launch_typed(DenseProblem<true, true>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);
         return launch_typed(DenseProblem<true>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);

@@ -333,6 +333,14 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& g, const int m0, const
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[i][j][e] = both_single ? acc[i][j][e] * one : acc[i][j][e] * isa * isb[j][e];
     }
+    if (g.c_f32 == 2) {  // (uniform)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[i][j][e] = round_to_bf16(acc[i][j][e]);
+    }
     const bool wide = (reinterpret_cast<uintptr_t>(g.C) & 15) == 0 && ((g.ldc | g.N) & (g.c_f32 ? 3 : 7)) == 0;
     if (!wide) {
         // Rows that are not whole 16-byte chunks leave an element per lane, or four bf16 values where rows are whole 8-byte

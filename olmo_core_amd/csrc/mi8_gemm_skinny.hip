@@ -123,7 +123,8 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_fp8_skinny_kernel(Gemm
             const int n = n0 + nb * 16 + kg * 4 + j;
             if (n >= g.N) continue;
             const float isb = g.sb_vec ? __builtin_amdgcn_rcpf(g.sb[n]) : isb_scalar;
-            const float v = both_single ? sum[j] * (isa * isb) : sum[j] * isa * isb;
+            float v = both_single ? sum[j] * (isa * isb) : sum[j] * isa * isb;
+            if (g.c_f32 == 2) v = round_to_bf16(v);
             if (g.c_f32) {
                 float* c = reinterpret_cast<float*>(g.C) + (int64_t)m * g.ldc + n;
                 *c = g.accumulate ? *c + v : v;

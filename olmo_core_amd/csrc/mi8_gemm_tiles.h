@@ -64,7 +64,8 @@ struct HalfRows {
 // CODES: the epilogue also records, per row segment (64 consecutive columns of a row) of C, the largest magnitude it
 // wrote as a 16-bit code (mi8_swiglu.h; codes[(column / 64) * M + row], N % 64 == 0: shifted tiles then start on
 // segment boundaries).
-template <bool VEC, bool ACC = false, bool CODES = false>
+// F32: C is float32 that holds the bf16 values.
+template <bool VEC, bool ACC = false, bool CODES = false, bool F32 = false>
 struct DenseProblem {
     GemmArgs g;
     int64_t lda, ldb, ldc;
@@ -74,6 +75,7 @@ struct DenseProblem {
     static constexpr bool kVecScales = VEC;  // both scales are vectors (per row / per column) or both single
     static constexpr bool kAccumulate = ACC;  // C += the rounded product
     static constexpr bool kOutCodes = CODES;
+    static constexpr bool kOutF32 = F32;
     // (scale vectors applied inside the MFMAs, as the grouped problems do, change nothing here: the K = 4096 rowwise GEMMs
     // of an attention block ran in 3.00-3.02 ms per step either way - under the power limit a shorter epilogue is paid
     // back by a lower clock)
@@ -107,7 +109,7 @@ struct DenseProblem {
         d.nk = g.K / BK;
         d.sa = g.sa + (VEC ? m0 : 0);
         d.sb = g.sb + (VEC ? n0 : 0);
-        d.c = reinterpret_cast<uint16_t*>(g.C) + (int64_t)m0 * g.ldc + n0;
+        d.c = reinterpret_cast<uint16_t*>(g.C) + ((int64_t)m0 * g.ldc + n0) * (F32 ? 2 : 1);
         d.row_lo = 0;
         d.row_hi = height;
         d.m0 = m0;
@@ -131,7 +133,7 @@ struct SwigluProblem {
     const float* sb3;       // scale of B3
     uint32_t* h_slots;      // [4 * workgroups] partial maxima of |h| (float32 bit patterns)
     uint16_t* x_codes;      // null, or [H / 64][M] codes of the larger of x1 and x3 per row segment (H % 64 == 0)
-    static constexpr bool kVecScales = false, kAccumulate = false, kSwiglu = true, kOutCodes = false;
+    static constexpr bool kVecScales = false, kAccumulate = false, kSwiglu = true, kOutCodes = false, kOutF32 = false;
     static constexpr bool kMaskRows = false, kXcdRanges = true, kMfmaScale = false, kTwoSegments = false, kHalves = true;
     using Cache = NoCache;
     __device__ __forceinline__ Cache prepare() const { return Cache{}; }
@@ -228,7 +230,7 @@ __device__ __forceinline__ GroupSpan locate_group_cached(const GroupCache& c, co
 template <bool ACC = false>
 struct GroupedProblem {
     static constexpr bool kAccumulate = ACC;
-    static constexpr bool kSwiglu = false, kOutCodes = false, kMfmaScale = true, kTwoSegments = false;
+    static constexpr bool kSwiglu = false, kOutCodes = false, kOutF32 = false, kMfmaScale = true, kTwoSegments = false;
     const uint8_t* A;
     const uint8_t* B;
     uint16_t* C;
@@ -278,7 +280,7 @@ struct GroupedProblem {
 // no second launch, no read-modify-write of the output.  A1, A2 share a row pitch, B1, B2 a row pitch and group stride,
 // the column scales a group stride; K1, K2 are multiples of 256 (an even number of steps each).
 struct GroupedDualProblem {
-    static constexpr bool kAccumulate = false, kSwiglu = false, kOutCodes = false, kMfmaScale = true, kTwoSegments = true;
+    static constexpr bool kAccumulate = false, kSwiglu = false, kOutCodes = false, kOutF32 = false, kMfmaScale = true, kTwoSegments = true;
     static constexpr bool kVecScales = true, kMaskRows = true, kXcdRanges = true, kHalves = false;
     GroupedProblem<false> first;  // A1, B1, C, pitches, sizes, N, K = K1, sa1, sb1
     int64_t lda, ldb, ldc;        // (copies of first's, under the names the kernel reads)
@@ -333,7 +335,7 @@ struct GroupedWgradProblem {
     const float* sa;  // [E, N]
     const float* sb;  // [E, Kl]
     static constexpr bool kVecScales = true, kMaskRows = false, kXcdRanges = false, kHalves = false;
-    static constexpr bool kAccumulate = false, kSwiglu = false, kOutCodes = false, kMfmaScale = false, kTwoSegments = false;
+    static constexpr bool kAccumulate = false, kSwiglu = false, kOutCodes = false, kOutF32 = false, kMfmaScale = false, kTwoSegments = false;
     using Cache = WgradCache;
     __device__ __forceinline__ Cache prepare() const
     {

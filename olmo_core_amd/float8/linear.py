@@ -212,7 +212,7 @@ def _backward_impl(go2, c: Float8LinearConfig, N: int, x_dtype, w_dtype, x_part,
         if _is_disabled(cgw):
             gw = torch.mm(go2.t(), x_part[0].to(go2.dtype))
         else:
-            products.append(_grad_weight_product(go2, c, go_cols, x_part, x_is_q))
+            products.append(_grad_weight_product(go2, c, go_cols, x_part, x_is_q, w_dtype))
     if products:
         made = ops.gemm_fp8_batch(products, out_dtype=x_dtype)
         if need_gw and not _is_disabled(cgw):
@@ -233,13 +233,13 @@ def _grad_input_product(go2, c: Float8LinearConfig, N: int, go_rows, w_part, w_i
     return (go_rows[0], go_rows[1], w_op[0], w_op[1], N, add)
 
 
-def _grad_weight_product(go2, c: Float8LinearConfig, go_cols, x_part, x_is_q: bool):
-    """The grad_weight of one linear as :func:`ops.gemm_fp8_batch` takes it."""
+def _grad_weight_product(go2, c: Float8LinearConfig, go_cols, x_part, x_is_q: bool, w_dtype):
+    """The grad_weight of one linear as :func:`ops.gemm_fp8_batch` takes it (written as float32 for a float32 weight)."""
     pow2 = c.round_scales_to_power_of_2
     if go_cols is None:
         go_cols = _cols_operand(go2, c.cast_config_grad_output_for_grad_weight, pow2)
     x_op = x_part if x_is_q else _cols_operand(x_part[0], c.cast_config_input_for_grad_weight, pow2)
-    return (go_cols[0], go_cols[1], x_op[0], x_op[1], None, False)
+    return (go_cols[0], go_cols[1], x_op[0], x_op[1], None, False, w_dtype)
 
 
 def _options(c: Float8LinearConfig) -> tuple:
@@ -284,7 +284,7 @@ def _planned_backward(ctx, gos, ns, need_gx: bool, need_gws):
         x_part, w_parts = saved
         made = _grad_operands(gos_, c, need_gx, need_gws)
         ps = [_grad_input_product(gos_[i], c, ns[i], made[i][0], w_parts[i], True, add=i != order[0]) for i in order if need_gx]
-        ps += [_grad_weight_product(gos_[i], c, made[i][1], x_part, True) for i in wanted]
+        ps += [_grad_weight_product(gos_[i], c, made[i][1], x_part, True, ctx.w_dtypes[i]) for i in wanted]
         return ops.gemm_fp8_batch(ps, out_dtype=ctx.x_dtype) if ps else []
 
     def recorded(slab, *places):
@@ -317,6 +317,7 @@ class _Float8Matmul(torch.autograd.Function):
         if done is not None:
             (y,), kept, ctx.plan = done
             ctx.config, ctx.M, ctx.N, ctx.x_dtype, ctx.w_dtype = config, x2.shape[0], weight.shape[0], x2.dtype, weight.dtype
+            ctx.w_dtypes = [weight.dtype]
             ctx.save_for_backward(kept)
             return y
         y, x_saved, w_saved = _forward_impl(x2, weight, config, weight_scale, need_gx, need_gw, weight_ops)
@@ -430,7 +431,7 @@ class _Float8SharedInputMatmul(torch.autograd.Function):
             products = [_grad_input_product(gos[i], c, ctx.ns[i], made[i][0], w_parts[i], ctx.w_is_q[i], add=i != order[0])
                         for i in order if need_gx]
             wanted = [i for i in order if ctx.need_gws[i]]
-            products += [_grad_weight_product(gos[i], c, made[i][1], x_part, ctx.x_is_q) for i in wanted]
+            products += [_grad_weight_product(gos[i], c, made[i][1], x_part, ctx.x_is_q, ctx.w_dtypes[i]) for i in wanted]
             outs = ops.gemm_fp8_batch(products, out_dtype=ctx.x_dtype) if products else []
             if need_gx:
                 gx = outs.pop(0)

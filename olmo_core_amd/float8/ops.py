@@ -323,6 +323,7 @@ def gemm_fp8(
     out: Optional[torch.Tensor] = None,
     splits: int = -1,
     accumulate: bool = False,
+    rounded: bool = False,
 ) -> torch.Tensor:
     """
     ``out[M, N] = (a[M, :k] @ b[N, :k].T) / sa / sb`` with fp32 accumulation on the fp8 matrix cores.
@@ -332,6 +333,7 @@ def gemm_fp8(
     ``splits``: slices of K summed separately and added afterwards (for problems with few output tiles);
     -1 lets the library decide from the shape, 0 and 1 forbid splitting; a forced ``variant`` is never split.  More of them
     than K has steps of 128 (or than 64) are refused; ``accumulate`` sums such a product unsplit.
+    ``rounded`` (float32 ``out_dtype``): the values that a bfloat16 output would have.
     """
     _require_gpu(a, "gemm_fp8")
     if a.dim() != 2 or b.dim() != 2 or a.stride(1) != 1 or b.stride(1) != 1:
@@ -358,6 +360,7 @@ def gemm_fp8(
         ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         ev0.record()
     L = _C.lib()
+    code = _C.MI8_F32_OF_BF16 if rounded and out_dtype == torch.float32 else _HP_CODE[out_dtype]
     if variant >= 0:
         splits = 1
     elif splits < 0:
@@ -369,7 +372,7 @@ def gemm_fp8(
             L.mi8_gemm_fp8_accumulate(
                 a.data_ptr(), _FP8_CODE[a.dtype], a.stride(0), b.data_ptr(), _FP8_CODE[b.dtype], b.stride(0), M, N, K,
                 sa.data_ptr(), int(sa.numel() != 1), sb.data_ptr(), int(sb.numel() != 1),
-                out.data_ptr(), _HP_CODE[out_dtype], out.stride(0), _stream(a),
+                out.data_ptr(), code, out.stride(0), _stream(a),
             ),
             "mi8_gemm_fp8_accumulate",
         )
@@ -381,7 +384,7 @@ def gemm_fp8(
                 a.data_ptr(), _FP8_CODE[a.dtype], a.stride(0), b.data_ptr(), _FP8_CODE[b.dtype], b.stride(0), M, N, K,
                 sa.data_ptr(), int(sa.numel() != 1),
                 sb.data_ptr(), int(sb.numel() != 1),
-                out.data_ptr(), _HP_CODE[out_dtype], out.stride(0), splits, planes.data_ptr(), planes.numel(),
+                out.data_ptr(), code, out.stride(0), splits, planes.data_ptr(), planes.numel(),
                 _stream(a),
             ),
             "mi8_gemm_fp8_splitk",
@@ -392,7 +395,7 @@ def gemm_fp8(
                 a.data_ptr(), _FP8_CODE[a.dtype], a.stride(0), b.data_ptr(), _FP8_CODE[b.dtype], b.stride(0), M, N, K,
                 sa.data_ptr(), int(sa.numel() != 1),
                 sb.data_ptr(), int(sb.numel() != 1),
-                out.data_ptr(), _HP_CODE[out_dtype], out.stride(0), variant, _stream(a),
+                out.data_ptr(), code, out.stride(0), variant, _stream(a),
             ),
             "mi8_gemm_fp8",
         )
@@ -406,19 +409,24 @@ def gemm_fp8_batch(products, *, out_dtype: torch.dtype = torch.bfloat16, togethe
     """
     Several :func:`gemm_fp8` products of one pair of float8 types: ``products`` is a list of ``(a, sa, b, sb, k, add)``,
     ``k`` the contracted length (``None``: that of the operands) and ``add`` whether the product is added to the one
-    before it (the bits of an elementwise add of the two outputs).  Returns the outputs of those that are not added, in
+    before it (the bits of an elementwise add of the two outputs).  A seventh element ``torch.float32`` wants the product
+    of a bfloat16 ``out_dtype`` as float32 values (the gradient of a float32 weight).  Returns the outputs of those that are not added, in
     order.  One launch where the library estimates that it is faster than one per product (``together`` decides
     otherwise); the results are the same bits.
     """
     outs = []
     n = len(products)
     a0, b0 = products[0][0], products[0][2]
+    wide = lambda p: len(p) > 6 and p[6] == torch.float32 and out_dtype == torch.bfloat16  # noqa: E731
     if n == 1 and not products[0][5]:
-        return [gemm_fp8(*products[0][:4], k=products[0][4], out_dtype=out_dtype)]
+        p = products[0]
+        return [gemm_fp8(*p[:4], k=p[4], out_dtype=torch.float32 if wide(p) else out_dtype, rounded=wide(p))]
     _require_gpu(a0, "gemm_fp8_batch")
     one_launch = together is not False and GEMM_EVENT_SINK is None and 1 < n <= _C.GEMM_BATCH
     args = (_C.GemmProduct * n)() if one_launch else (None,) * n
-    for (a, sa, b, sb, k, add), p in zip(products, args):
+    for product, p in zip(products, args):
+        a, sa, b, sb, k, add = product[:6]
+        f32 = wide(product)
         M, N = a.shape[0], b.shape[0]
         K = min(a.shape[1], b.shape[1]) if k is None else k
         if a.dtype != a0.dtype or b.dtype != b0.dtype or a.device != a0.device or a.dtype not in _FP8_CODE or b.dtype not in _FP8_CODE:
@@ -431,21 +439,22 @@ def gemm_fp8_batch(products, *, out_dtype: torch.dtype = torch.bfloat16, togethe
         if add and (not outs or tuple(outs[-1].shape) != (M, N)):
             raise ValueError("gemm_fp8_batch: nothing of its shape to add the product to")
         if not add:
-            outs.append(_empty((M, N), dtype=out_dtype, device=a.device))
+            outs.append(_empty((M, N), dtype=torch.float32 if f32 else out_dtype, device=a.device))
         if one_launch:
             out = outs[-1]
             p.a, p.lda, p.b, p.ldb = a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0)
             p.M, p.N, p.K, p.sa, p.sb = M, N, K, sa.data_ptr(), sb.data_ptr()
-            p.out, p.ldc, p.out_dtype = out.data_ptr(), N, _HP_CODE[out_dtype]
+            p.out, p.ldc, p.out_dtype = out.data_ptr(), N, _C.MI8_F32_OF_BF16 if f32 else _HP_CODE[out_dtype]
             p.sa_is_vector, p.sb_is_vector, p.add_to_previous = va, vb, add
     L = _C.lib()
     if one_launch and (together or L.mi8_gemm_fp8_batch_pays(args, n)):
         _C.check(L.mi8_gemm_fp8_batch(args, n, _FP8_CODE[a0.dtype], _FP8_CODE[b0.dtype], _stream(a0)), "mi8_gemm_fp8_batch")
         return outs
     i = -1
-    for a, sa, b, sb, k, add in products:
+    for product in products:
+        a, sa, b, sb, k, add = product[:6]
         i += not add
-        gemm_fp8(a, sa, b, sb, k=k, out_dtype=out_dtype, out=outs[i], accumulate=bool(add))
+        gemm_fp8(a, sa, b, sb, k=k, out_dtype=outs[i].dtype, out=outs[i], accumulate=bool(add), rounded=wide(product))
     return outs
 
 

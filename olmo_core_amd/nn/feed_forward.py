@@ -141,10 +141,11 @@ def _mlp_backward(gy, saved, c, dims, dtypes, need):
     need_gh = need_x or need_w1 or need_w3
     gyq, gyq_t, sgy = ops.cast_tensorwise(gy, go_dt, pow2=pow2, want_rowmajor=need_gh, want_transposed=need_w2,
                                            whole_steps=True)
-    w2_product = (gyq_t, sgy, hq_t, sh, None, False)
+    # (the weights' gradients leave the GEMMs in the weights' type: float32 that holds the bf16 values under autocast)
+    w2_product = (gyq_t, sgy, hq_t, sh, None, False, w2_dt)
     gx = gw1 = gw2 = gw3 = None
     if need_w2 and not need_gh:
-        gw2 = ops.gemm_fp8(*w2_product[:4], out_dtype=x_dt)
+        (gw2,) = ops.gemm_fp8_batch([w2_product], out_dtype=x_dt)
     if need_gh:
         # g1 and g3 are needed in fp8 only, and their tensorwise scales need the amax of both first.  Where the
         # forward recorded the row-segment codes of x1 and x3, the GEMM that produces gh records those of gh, and the
@@ -152,7 +153,7 @@ def _mlp_backward(gy, saved, c, dims, dtypes, need):
         codes = None
         if x_codes.numel() and x_dt == torch.bfloat16 and ops.gemm_codes_supported(M, H, D):
             if need_w2:
-                gw2 = ops.gemm_fp8(*w2_product[:4], out_dtype=x_dt)
+                (gw2,) = ops.gemm_fp8_batch([w2_product], out_dtype=x_dt)
             gh, gh_codes = ops.gemm_fp8_codes(gyq, sgy, w2q_t, s2, k=D)
             codes = (gh_codes, x_codes)
         else:
@@ -175,9 +176,9 @@ def _mlp_backward(gy, saved, c, dims, dtypes, need):
         elif need_x:
             products += [(g3q, sg3, w3q_t, s3, H, False), (g1q, sg1, w1q_t, s1, H, False)]
         if need_w1:
-            products.append((g1q_t, sg1, xq_t, sx, None, False))
+            products.append((g1q_t, sg1, xq_t, sx, None, False, w1_dt))
         if need_w3:
-            products.append((g3q_t, sg3, xq_t, sx, None, False))
+            products.append((g3q_t, sg3, xq_t, sx, None, False, w3_dt))
         outs = ops.gemm_fp8_batch(products, out_dtype=x_dt)
         if need_w3:
             gw3 = outs.pop()
@@ -253,15 +254,14 @@ class _Float8SwiGLUMLP(torch.autograd.Function):
                 gy = gy.to(bf16).contiguous()
 
             def recorded(slab, pgy):
-                grads = _mlp_backward(pgy, ctx.plan.saved_places(slab), ctx.config, ctx.dims, (bf16,) * 4, need)
+                grads = _mlp_backward(pgy, ctx.plan.saved_places(slab), ctx.config, ctx.dims, ctx.dtypes, need)
                 return [g for g in grads if g is not None], None
 
-            done = plan.call(recorded, [kept, gy], ("backward", need), within=ctx.plan)
+            done = plan.call(recorded, [kept, gy], ("backward", need), within=ctx.plan)  # (the forward's plan knows the types)
         if done is None:
             return _mlp_backward(gy, ctx.plan.saved_tensors(kept), ctx.config, ctx.dims, ctx.dtypes, need) + (None,) * 7
         grads = iter(done[0])
-        grads = [next(grads) if n else None for n in need]
-        return (*(g if g is None or g.dtype == dt else g.to(dt) for g, dt in zip(grads, ctx.dtypes)), *(None,) * 7)
+        return (*(next(grads) if n else None for n in need), *(None,) * 7)
 
 
 def _fusable_modules(ff: "FeedForward", same_object: bool = False) -> bool:

@@ -651,3 +651,30 @@ def test_few_rows_swiglu_on_ring_tiles(dev, M, H, K):
     want, _ = ops.swiglu_fwd(x1, x3)
     assert torch.equal(h, want) and n == (H + 31) // 32
     assert slots[:n].max().item() == h.abs().float().max().view(1).view(torch.int32).item()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vec", [False, True])
+def test_float32_outputs_of_bf16_values(dev, vec):
+    """float32 outputs that hold the bf16 values: every kernel, tiles shifted back over their neighbours and half tiles of the
+    persistent one, planes, rows that are not whole 16-byte chunks; one by one and together with bf16 products."""
+    g = torch.Generator(device=dev).manual_seed(3)
+    names = ops.gemm_variants()
+    for M, N, K in ((1, 64, 128), (40, 272, 1040), (300, 264, 256), (257, 1000, 384), (640, 2056, 512), (777, 331, 528), (2048, 2816, 1024)):
+        a = torch.randn(M, K, generator=g, device=dev).to(torch.float8_e5m2)
+        b = torch.randn(N, K, generator=g, device=dev).to(torch.float8_e4m3fn)
+        sa, sb = (torch.rand(n if vec else 1, generator=g, device=dev) + 0.5 for n in (M, N))
+        for v in range(-1, len(names)):
+            try:
+                want = ops.gemm_fp8(a, sa, b, sb, variant=v)
+            except MI8KernelError:
+                continue
+            got = ops.gemm_fp8(a, sa, b, sb, variant=v, out_dtype=torch.float32, rounded=True)
+            assert torch.equal(got, want.float()), (M, N, K, v)
+        if K > 256:
+            want = ops.gemm_fp8(a, sa, b, sb, splits=3)
+            assert torch.equal(ops.gemm_fp8(a, sa, b, sb, splits=3, out_dtype=torch.float32, rounded=True), want.float())
+        products = [(a, sa, b, sb, None, False, torch.float32), (a, sa, b, sb, None, False)]
+        for together in (False, True):
+            x, y = ops.gemm_fp8_batch(products, together=together)
+            assert x.dtype == torch.float32 and y.dtype == torch.bfloat16 and torch.equal(x, y.float())
