@@ -143,7 +143,8 @@ int mi8_cast_tensorwise_batch(const mi8_cast_item* items, int32_t count, int fp8
  * per tensor the results of mi8_cast_rowwise and mi8_cast_colwise_t, two launches for all of them.
  *   out_rows: fp8 [rows, ld_rows]; row_scale: float32 [rows]; out_t: fp8 [cols, ld_t], ld_t >= round_up(rows, 128), zero
  *   from column `rows` to ld_t; col_scale: float32 [cols]; workspace: uint32 [mi8_two_cast_workspace_words(rows, cols)],
- *   16-byte aligned, contents on entry unimportant. */
+ *   16-byte aligned, contents on entry unimportant.  group_rows (0: rows): every group_rows rows, a multiple of 128 that
+ *   divides rows, have column scales of their own, col_scale [rows / group_rows, cols] (the weights of experts). */
 typedef struct {
     const void* x;
     int64_t rows, cols;
@@ -154,6 +155,7 @@ typedef struct {
     int64_t ld_t;
     float* col_scale;
     uint32_t* workspace;
+    int64_t group_rows;
     int32_t hp_dtype;
 } mi8_two_cast_item;
 int64_t mi8_two_cast_workspace_words(int64_t rows, int64_t cols);

@@ -42,7 +42,7 @@ class TwoCastItem(ctypes.Structure):
     """mi8_two_cast_item"""
     _fields_ = [("x", c_void_p), ("rows", c_int64), ("cols", c_int64), ("out_rows", c_void_p), ("ld_rows", c_int64),
                 ("row_scale", c_void_p), ("out_t", c_void_p), ("ld_t", c_int64), ("col_scale", c_void_p),
-                ("workspace", c_void_p), ("hp_dtype", c_int32)]
+                ("workspace", c_void_p), ("group_rows", c_int64), ("hp_dtype", c_int32)]
 
 
 GEMM_BATCH = 8

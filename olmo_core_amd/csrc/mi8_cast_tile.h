@@ -140,11 +140,52 @@ __device__ __forceinline__ void tile_load(const void* x, int64_t row_end, int64_
         }
 }
 
-// Quantise a loaded tile with the eight per-column scales of this lane (all equal for a tensorwise cast).
+// The same tile as it is in memory, half the registers for bf16: for kernels that have it in flight while they make the scales.
+template <int HP>
+struct RawTile {
+    static constexpr int NV = HpVec<HP>::kBytes / 2;  // 16-byte vectors per eight elements
+    uint4 v[2][4][NV];
+    __device__ __forceinline__ void load(const void* x, int64_t row_end, int64_t cols, int64_t row0, int64_t col0)
+    {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const int64_t c8 = col0 + 8 * (lane & 15);
+        const char* xb = reinterpret_cast<const char*>(x);
+#pragma unroll
+        for (int it = 0; it < 2; ++it)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t r = row0 + 32 * wave + 16 * it + 4 * (lane >> 4) + j;
+#pragma unroll
+                for (int k = 0; k < NV; ++k) {
+                    v[it][j][k] = make_uint4(0, 0, 0, 0);
+                    if (c8 < cols && r < row_end) v[it][j][k] = load_stream16(xb + (r * cols + c8) * HpVec<HP>::kBytes + 16 * k);
+                }
+            }
+    }
+    __device__ __forceinline__ void operator()(int it, int j, float (&f)[8]) const
+    {
+        const uint4 a = v[it][j][0], b = v[it][j][NV - 1];
+        if constexpr (HP == MI8_BF16) {
+            const uint32_t d[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                f[2 * k] = bits_to_f32(d[k] << 16);
+                f[2 * k + 1] = bits_to_f32(d[k] & 0xFFFF0000u);
+            }
+        } else {
+            const uint32_t d[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) f[k] = bits_to_f32(d[k]);
+        }
+    }
+};
+
+// Quantise a loaded tile (values(it, j, f): a thread's eight of row 16 it + j) with the eight per-column scales of this lane
+// (all equal for a tensorwise cast).
 // Row-major bytes go to out[r, c]; the transposed bytes go to out_t[c, dst0 + (r - row0)] as 16-byte chunks,
 // chunks at or beyond dst_end are not written.
-template <int FP8, bool SW>
-__device__ __forceinline__ void tile_quantise(const float (&f)[2][4][8], int64_t row_end, int64_t cols, int64_t row0, int64_t col0,
+template <int FP8, bool SW, typename Values>
+__device__ __forceinline__ void tile_quantise(const Values& values, int64_t row_end, int64_t cols, int64_t row0, int64_t col0,
                                               const float (&sc)[8], uint8_t* out, int64_t ld_out, uint8_t* out_t, int64_t ld_t,
                                               int64_t dst0, int64_t dst_end, uint32_t* lds_t, uint8_t* out_r = nullptr,
                                               int64_t ld_r = 0, const float* row_scale = nullptr, int64_t row_scale_row0 = 0)
@@ -172,7 +213,8 @@ __device__ __forceinline__ void tile_quantise(const float (&f)[2][4][8], int64_t
         for (int j = 0; j < 4; ++j) {
             const int64_t r = row0 + 32 * wave + 16 * it + 4 * g + j;
             const bool ok = col_ok && r < row_end;
-            const float* v = f[it][j];
+            float v[8];
+            values(it, j, v);
             lo[j] = quant4<FP8, SW>(v[0], v[1], v[2], v[3], sc[0], sc[1], sc[2], sc[3]);
             hi[j] = quant4<FP8, SW>(v[4], v[5], v[6], v[7], sc[4], sc[5], sc[6], sc[7]);
             if (!ok) lo[j] = hi[j] = 0;  // padding is zero bytes whatever the scale is (0 * NaN is NaN)
@@ -222,7 +264,11 @@ __device__ __forceinline__ void tile_cast_body(const void* x, int64_t row_end, i
 {
     float f[2][4][8];
     tile_load<HP>(x, row_end, cols, row0, col0, f, gather, top_k, src_rows, gather_w, gather_w_dtype);
-    tile_quantise<FP8, SW>(f, row_end, cols, row0, col0, sc, out, ld_out, out_t, ld_t, dst0, dst_end, lds_t, out_r, ld_r,
+    const auto values = [&](int it, int j, float(&v)[8]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = f[it][j][k];
+    };
+    tile_quantise<FP8, SW>(values, row_end, cols, row0, col0, sc, out, ld_out, out_t, ld_t, dst0, dst_end, lds_t, out_r, ld_r,
                            row_scale, row_scale_row0);
 }
 

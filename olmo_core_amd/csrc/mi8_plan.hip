@@ -92,7 +92,7 @@ struct Get<const mi8_two_cast_item*> {
         for (int i = 0; i < n; ++i) {
             mi8_two_cast_item& t = r.two_casts[i];
             get(r, t.x), get(r, t.rows), get(r, t.cols), get(r, t.out_rows), get(r, t.ld_rows), get(r, t.row_scale), get(r, t.out_t);
-            get(r, t.ld_t), get(r, t.col_scale), get(r, t.workspace), get(r, t.hp_dtype);
+            get(r, t.ld_t), get(r, t.col_scale), get(r, t.workspace), get(r, t.group_rows), get(r, t.hp_dtype);
         }
         return r.two_casts;
     }

@@ -979,11 +979,13 @@ def cast_rows_and_colwise_t(
     return made if more else made[0]
 
 
-def cast_rows_and_colwise_t_batch(xs, fp8_dtype: torch.dtype, *, pow2: bool = False) -> list:
-    """:func:`cast_rows_and_colwise_t` of several tensors on one GPU, launched together."""
+def cast_rows_and_colwise_t_batch(xs, fp8_dtype: torch.dtype, *, pow2: bool = False, groups: int = 1) -> list:
+    """:func:`cast_rows_and_colwise_t` of several tensors on one GPU, launched together.  ``groups``: the rows of every tensor
+    are that many equal groups with column scales of their own, ``[groups, cols]`` (experts' weights; groups of a multiple
+    of 128 rows): bytes and scales of :func:`grouped_cast_rows_and_colwise_t`."""
     if len(xs) > _C.CAST_BATCH:
-        return (cast_rows_and_colwise_t_batch(xs[:_C.CAST_BATCH], fp8_dtype, pow2=pow2)
-                + cast_rows_and_colwise_t_batch(xs[_C.CAST_BATCH:], fp8_dtype, pow2=pow2))
+        return (cast_rows_and_colwise_t_batch(xs[:_C.CAST_BATCH], fp8_dtype, pow2=pow2, groups=groups)
+                + cast_rows_and_colwise_t_batch(xs[_C.CAST_BATCH:], fp8_dtype, pow2=pow2, groups=groups))
     xs = [_hp2d(x, "cast_rows_and_colwise_t") for x in xs]
     dev = xs[0].device
     n = len(xs)
@@ -1000,7 +1002,12 @@ def cast_rows_and_colwise_t_batch(xs, fp8_dtype: torch.dtype, *, pow2: bool = Fa
         ld_t = pad128(rows)
         q = _empty((rows, cols), dtype=fp8_dtype, device=dev)
         q_t = _empty((cols, ld_t), dtype=fp8_dtype, device=dev)
-        rs, cs = _empty(rows, dtype=torch.float32, device=dev), _empty(cols, dtype=torch.float32, device=dev)
+        rs = _empty(rows, dtype=torch.float32, device=dev)
+        cs = _empty(cols if groups == 1 else (groups, cols), dtype=torch.float32, device=dev)
+        if groups > 1:
+            if rows % groups:
+                raise ValueError(f"cast_rows_and_colwise_t_batch: {rows} rows are not {groups} equal groups")
+            a.group_rows = rows // groups
         a.x, a.rows, a.cols, a.hp_dtype = x.data_ptr(), rows, cols, _HP_CODE[x.dtype]
         a.out_rows, a.ld_rows, a.row_scale = q.data_ptr(), cols, rs.data_ptr()
         a.out_t, a.ld_t, a.col_scale, a.workspace = q_t.data_ptr(), ld_t, cs.data_ptr(), at

@@ -341,12 +341,13 @@ def test_transposed_copy_in_whole_steps(dev, rows):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("fp8", [torch.float8_e4m3fn, torch.float8_e5m2])
-def test_casts_of_several_tensors_in_one_launch(dev, fp8):
+@pytest.mark.parametrize("types", ["mixed", "bf16", "float32"])
+def test_casts_of_several_tensors_in_one_launch(dev, fp8, types):
     """Tensors cast together have the bytes and scales of casts one by one: single rows, tiles cut at both edges, more row
-    tiles than chunks of column maxima (4097 rows), bf16 and float32 mixed, and values that are all zero, infinite or NaN."""
+    tiles than chunks of column maxima (4097 rows), bf16, float32 and both, and values that are all zero, infinite or NaN."""
     shapes = [(1, 16), (127, 144), (128, 128), (129, 2048), (4097, 272), (300, 1040), (16, 4096)]
     xs = [torch.randn(s, generator=torch.Generator().manual_seed(i), dtype=torch.float32).to(dev) for i, s in enumerate(shapes)]
-    xs = [x if i % 3 == 1 else x.bfloat16() for i, x in enumerate(xs)]
+    xs = [x if types == "float32" or types == "mixed" and i % 3 == 1 else x.bfloat16() for i, x in enumerate(xs)]
     xs[2].zero_()
     xs[3][5, 7], xs[3][6, 9] = float("inf"), float("nan")
     raw = lambda t: t.view(torch.uint8)  # noqa: E731

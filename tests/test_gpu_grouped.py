@@ -589,3 +589,19 @@ def test_grouped_gemm_takes_a_wide_pitch(dev, sizes):
                                sb_group_stride=n, out_dtype=torch.float32)
     group = torch.repeat_interleave(torch.arange(E), torch.tensor(sizes)).to(dev)
     assert torch.equal(out, (values[:, None, :] @ b.view(E, n, k)[group].transpose(1, 2).contiguous())[:, 0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E, H, D", [(2, 128, 16), (5, 256, 144), (3, 1408, 1040), (2, 4224, 272)])
+def test_experts_weights_cast_together(dev, E, H, D):
+    """Weights of equal groups of rows, cast together, have the bytes and scales of the ragged grouped cast: one row tile a group
+    and several, groups of more row tiles (33) than partial maxima are kept of, tensors of one type and of both."""
+    ws = [seeded((E * H, D), 3 + i).to(dev) for i in range(2)] + [seeded((E * H, D), 9).to(dev).float()]
+    ws[0][H:].mul_(3.0)
+    ws[1][5, 7] = 0.0
+    equal = torch.full((E,), H, dtype=torch.int64, device=dev)
+    for pow2, some in ((False, ws), (True, ws[:2]), (True, ws[2:])):
+        for w, (q, rs, q_t, cs) in zip(some, ops.cast_rows_and_colwise_t_batch(some, torch.float8_e4m3fn, pow2=pow2, groups=E)):
+            q1, rs1, q_t1, cs1 = ops.grouped_cast_rows_and_colwise_t(w, equal, torch.float8_e4m3fn, pow2=pow2)
+            assert torch.equal(rs, rs1) and torch.equal(cs, cs1) and torch.equal(q.view(torch.uint8), q1.view(torch.uint8))
+            assert torch.equal(q_t.view(torch.uint8), q_t1.view(torch.uint8)[:, : E * H])
