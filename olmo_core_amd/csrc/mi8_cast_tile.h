@@ -70,26 +70,33 @@ constexpr int kTile = 128;
 __device__ __forceinline__ int64_t gathered_row(const int32_t* gather, int top_k, int64_t src_rows, int64_t r, bool ok)
 {
     if (!ok) return -1;
-    const int64_t slot = gather[r];
-    return (slot < 0 || slot >= src_rows * top_k) ? -1 : slot / top_k;
+    const int32_t slot = gather[r];  // (src_rows * top_k < 2^31: a 32-bit division)
+    return (slot < 0 || slot >= src_rows * top_k) ? -1 : (int64_t)((uint32_t)slot / (uint32_t)top_k);
 }
 
-// Weight of the slot that logical row r holds (weighted gather: the row is the token's row times this weight, the
-// product rounded to the element type as the gather kernel does); 1 without weights.
-__device__ __forceinline__ float gathered_weight(const int32_t* gather, const void* w, int w_dtype, int64_t r, bool ok)
+// Weight of a slot of the weighted gather: the row is the token's row times this weight, the product rounded to the element type
+// as the gather kernel does.
+__device__ __forceinline__ float slot_weight(const void* w, int w_dtype, int64_t slot)
 {
-    if (!w || !ok) return 1.0f;
-    const int64_t slot = gather[r];
     if (w_dtype == MI8_F32) return reinterpret_cast<const float*>(w)[slot];
     const uint16_t v = reinterpret_cast<const uint16_t*>(w)[slot];
     return w_dtype == MI8_BF16 ? bits_to_f32((uint32_t)v << 16) : (float)__builtin_bit_cast(_Float16, v);
 }
 
+// the 16 bytes of a row times the row's gather weight, each product rounded to the element type
 template <int HP>
-__device__ __forceinline__ float round_to_hp(float f)
+__device__ __forceinline__ uint4 scale_vec(uint4 v, float w)
 {
-    if constexpr (HP == MI8_BF16) return (float)(__bf16)f;
-    return f;
+    uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (HP == MI8_BF16) {
+            d[i] = pack_bf16(bits_to_f32(d[i] << 16) * w, bits_to_f32(d[i] & 0xFFFF0000u) * w);
+        } else {
+            d[i] = f32_to_bits(bits_to_f32(d[i]) * w);
+        }
+    }
+    return make_uint4(d[0], d[1], d[2], d[3]);
 }
 
 // LDS holds the transposed tile as 128 columns x 128 row-bytes.  Two columns share a 256-byte line; the
@@ -103,64 +110,46 @@ __device__ __forceinline__ int tile_lds_chunk(int col, int part /* 0..7: which 1
     return (col >> 1) * 16 + ((((col & 1) << 3) | part) ^ key);
 }
 
-// A thread's share of the 128 x 128 tile at (row0, col0): rows 32 wave + 16 it + 4 (lane / 16) + j, eight columns from
-// 8 (lane % 16); rows >= row_end and columns >= cols read as zero.  The loads need nothing but the position, so that they
-// can be in flight while the scales are made.
-template <int HP>
-__device__ __forceinline__ void tile_load(const void* x, int64_t row_end, int64_t cols, int64_t row0, int64_t col0, float (&f)[2][4][8],
-                                          const int32_t* gather = nullptr, int top_k = 1, int64_t src_rows = 0,
-                                          const void* gather_w = nullptr, int gather_w_dtype = 0)
-{
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int cl = lane & 15, g = lane >> 4;
-    const int64_t c8 = col0 + 8 * cl;
-    const bool col_ok = c8 < cols;
-    const char* xb = reinterpret_cast<const char*>(x);
-#pragma unroll
-    for (int it = 0; it < 2; ++it)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t r = row0 + 32 * wave + 16 * it + 4 * g + j;
-            bool ok = col_ok && r < row_end;
-            int64_t src = r;
-            if (gather) {  // row r of the expert-sorted side is row gather[r] / top_k of x (uniform branch)
-                src = gathered_row(gather, top_k, src_rows, r, r < row_end);
-                ok = ok && src >= 0;
-            }
-            if (gather)  // (uniform) a token's row is read top_k times: it stays cached
-                HpVec<HP>::load8(xb + (src * cols + c8) * HpVec<HP>::kBytes, ok, f[it][j]);
-            else
-                HpVec<HP>::template load8<true>(xb + (src * cols + c8) * HpVec<HP>::kBytes, ok, f[it][j]);
-            if (gather_w) {  // (uniform) weighted gather: the product, rounded to the element type
-                const float w = gathered_weight(gather, gather_w, gather_w_dtype, r, ok);
-#pragma unroll
-                for (int k = 0; k < 8; ++k) f[it][j][k] = round_to_hp<HP>(f[it][j][k] * w);
-            }
-        }
-}
-
-// The same tile as it is in memory, half the registers for bf16: for kernels that have it in flight while they make the scales.
+// A thread's share of the 128 x 128 tile at (row0, col0) as it is in memory (bf16: half the registers of its values): rows
+// 32 wave + 16 it + 4 (lane / 16) + j, eight columns from 8 (lane % 16); rows >= row_end and columns >= cols read as zero.
+// The loads need nothing but the position, so that they can be in flight while the scales are made.
+// GATHER: row r is row src[r - row0] of x, a row of zeros where that is negative.
 template <int HP>
 struct RawTile {
     static constexpr int NV = HpVec<HP>::kBytes / 2;  // 16-byte vectors per eight elements
     uint4 v[2][4][NV];
-    __device__ __forceinline__ void load(const void* x, int64_t row_end, int64_t cols, int64_t row0, int64_t col0)
+    __device__ __forceinline__ static int row_of(int it, int j) { return 32 * ((int)threadIdx.x >> 6) + 16 * it + 4 * (((int)threadIdx.x & 63) >> 4) + j; }
+    template <bool GATHER = false>
+    __device__ __forceinline__ void load(const void* x, int64_t row_end, int64_t cols, int64_t row0, int64_t col0, const int32_t* src = nullptr)
     {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int64_t c8 = col0 + 8 * (lane & 15);
+        const int64_t c8 = col0 + 8 * (threadIdx.x & 15);
         const char* xb = reinterpret_cast<const char*>(x);
 #pragma unroll
         for (int it = 0; it < 2; ++it)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int64_t r = row0 + 32 * wave + 16 * it + 4 * (lane >> 4) + j;
+                const int64_t r = row0 + row_of(it, j);
+                const int64_t from = GATHER ? (int64_t)src[row_of(it, j)] : r;
+                const bool ok = c8 < cols && r < row_end && from >= 0;
 #pragma unroll
                 for (int k = 0; k < NV; ++k) {
                     v[it][j][k] = make_uint4(0, 0, 0, 0);
-                    if (c8 < cols && r < row_end) v[it][j][k] = load_stream16(xb + (r * cols + c8) * HpVec<HP>::kBytes + 16 * k);
+                    const char* p = xb + (from * cols + c8) * HpVec<HP>::kBytes + 16 * k;
+                    // (gathered: a token's row is read top_k times, it stays cached)
+                    if (ok) v[it][j][k] = GATHER ? *reinterpret_cast<const uint4*>(p) : load_stream16(p);
                 }
             }
+    }
+    // the weighted gather's product; weights[row]: 1 for a row of zeros
+    __device__ __forceinline__ void scale_rows(const float* weights, bool col_ok)
+    {
+#pragma unroll
+        for (int it = 0; it < 2; ++it)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int k = 0; k < NV; ++k)
+                    if (col_ok) v[it][j][k] = scale_vec<HP>(v[it][j][k], weights[row_of(it, j)]);
     }
     __device__ __forceinline__ void operator()(int it, int j, float (&f)[8]) const
     {
@@ -254,23 +243,6 @@ __device__ __forceinline__ void tile_quantise(const Values& values, int64_t row_
 }
 
 // Both: rows [row0, row0 + 128) of x (rows >= row_end read as zero and produce zero bytes), columns [col0, col0 + 128).
-template <int HP, int FP8, bool SW>
-__device__ __forceinline__ void tile_cast_body(const void* x, int64_t row_end, int64_t cols, int64_t row0, int64_t col0,
-                                               const float (&sc)[8], uint8_t* out, int64_t ld_out, uint8_t* out_t, int64_t ld_t,
-                                               int64_t dst0, int64_t dst_end, uint32_t* lds_t,
-                                               uint8_t* out_r = nullptr, int64_t ld_r = 0, const float* row_scale = nullptr,
-                                               int64_t row_scale_row0 = 0, const int32_t* gather = nullptr, int top_k = 1,
-                                               int64_t src_rows = 0, const void* gather_w = nullptr, int gather_w_dtype = 0)
-{
-    float f[2][4][8];
-    tile_load<HP>(x, row_end, cols, row0, col0, f, gather, top_k, src_rows, gather_w, gather_w_dtype);
-    const auto values = [&](int it, int j, float(&v)[8]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = f[it][j][k];
-    };
-    tile_quantise<FP8, SW>(values, row_end, cols, row0, col0, sc, out, ld_out, out_t, ld_t, dst0, dst_end, lds_t, out_r, ld_r,
-                           row_scale, row_scale_row0);
-}
 
 }  // namespace
 }  // namespace mi8

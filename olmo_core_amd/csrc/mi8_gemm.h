@@ -50,12 +50,9 @@ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f)
 __device__ __forceinline__ float round_to_bf16(float f) { return bits_to_f32((uint32_t)f32_to_bf16_bits(f) << 16); }
 
 // Two floats -> two bf16 (round-to-nearest-even) in one dword, low half first: a single v_cvt_pk_bf16_f32.
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi)
 {
-    const f32x2_t f = {lo, hi};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
+    return pack_bf16(lo, hi);
 }
 
 // bf16(a) + bf16(b) for two or eight packed values, each sum formed in float32 and rounded once (what an elementwise add

@@ -7,16 +7,12 @@
 
 namespace mi8 {
 
-__device__ __forceinline__ float bf16_round(float f)
+// two values rounded to bf16: one conversion for both
+__device__ __forceinline__ void bf16_round2(float& a, float& b)
 {
-    __bf16 h = (__bf16)f;
-    return (float)h;
-}
-
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi)
-{
-    __bf16 a = (__bf16)lo, b = (__bf16)hi;
-    return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+    const uint32_t p = pack_bf16(a, b);
+    a = bits_to_f32(p << 16);
+    b = bits_to_f32(p & 0xFFFF0000u);
 }
 
 // 1 / (1 + e^-x) on the hardware exp2 and reciprocal (about one ulp each): the result feeds a bf16 rounding, and
@@ -51,9 +47,11 @@ __device__ __forceinline__ uint4 swiglu_fwd8(uint4 x1, uint4 x3)
     unpack8(x1, a);
     unpack8(x3, b);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const float s = bf16_round(a[k] * sigmoid_f32(a[k]));  // silu output as a bf16 tensor
-        o[k] = s * b[k];
+    for (int k = 0; k < 8; k += 2) {
+        float s0 = a[k] * sigmoid_f32(a[k]), s1 = a[k + 1] * sigmoid_f32(a[k + 1]);
+        bf16_round2(s0, s1);  // silu output as a bf16 tensor
+        o[k] = s0 * b[k];
+        o[k + 1] = s1 * b[k + 1];
     }
     return pack8(o);
 }
@@ -67,9 +65,11 @@ __device__ __forceinline__ uint2 swiglu_fwd4(uint2 x1, uint2 x3)
                         bits_to_f32(x3.y & 0xFFFF0000u)};
     float o[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const float s = bf16_round(a[k] * sigmoid_f32(a[k]));
-        o[k] = s * b[k];
+    for (int k = 0; k < 4; k += 2) {
+        float s0 = a[k] * sigmoid_f32(a[k]), s1 = a[k + 1] * sigmoid_f32(a[k + 1]);
+        bf16_round2(s0, s1);
+        o[k] = s0 * b[k];
+        o[k + 1] = s1 * b[k + 1];
     }
     return make_uint2(pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3]));
 }
@@ -82,12 +82,21 @@ __device__ __forceinline__ void swiglu_bwd8(uint4 x1, uint4 x3, uint4 gh, uint4&
     unpack8(x3, b);
     unpack8(gh, g);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const float sig = sigmoid_f32(a[k]);
-        const float s = bf16_round(a[k] * sig);    // saved silu output
-        o3[k] = g[k] * s;                          // d/dx3
-        const float gs = bf16_round(g[k] * b[k]);  // gradient reaching silu's output
-        o1[k] = gs * (sig * (1.0f + a[k] * (1.0f - sig)));
+    for (int k = 0; k < 8; k += 2) {
+        const float sig[2] = {sigmoid_f32(a[k]), sigmoid_f32(a[k + 1])};
+        float s[2], gs[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            s[i] = a[k + i] * sig[i];
+            gs[i] = g[k + i] * b[k + i];
+        }
+        bf16_round2(s[0], s[1]);    // saved silu output
+        bf16_round2(gs[0], gs[1]);  // gradient reaching silu's output
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            o3[k + i] = g[k + i] * s[i];  // d/dx3
+            o1[k + i] = gs[i] * (sig[i] * (1.0f + a[k + i] * (1.0f - sig[i])));
+        }
     }
     g1 = pack8(o1);
     g3 = pack8(o3);

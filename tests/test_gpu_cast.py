@@ -373,3 +373,18 @@ def test_casts_of_several_tensors_in_one_launch(dev, fp8, types):
                 if got is not None:
                     assert torch.equal(got.float().nan_to_num(3.0), want.float().nan_to_num(3.0))
     assert len(ops.cast_tensorwise_batch([(xs[6], {})] * 11, fp8)) == len(ops.cast_rows_and_colwise_t_batch([xs[6]] * 11, fp8)) == 11
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [torch.float8_e4m3fn, torch.float8_e5m2])
+@pytest.mark.parametrize("scale", [1.0, 0.37, 3e38])
+def test_every_bf16_value_saturates_and_keeps_nan(dev, fp8, scale):
+    """A given scale, all 65536 bf16 values: the product in float32, clamped to the largest fp8 value (infinities too), NaN kept."""
+    x = torch.arange(65536, dtype=torch.int32).to(torch.uint16).view(torch.bfloat16).reshape(512, 128)
+    q, q_t, _ = ops.cast_tensorwise(x.to(dev), fp8, want_transposed=True, scale=torch.full((1,), scale, device=dev))
+    top = torch.finfo(fp8).max
+    want = (x.float() * scale).clamp(-top, top).to(fp8)
+    assert torch.equal(q.cpu().float().nan_to_num(0.3), want.float().nan_to_num(0.3))
+    assert torch.equal(q_t.cpu().float().nan_to_num(0.3)[:, :512], want.float().t().nan_to_num(0.3))
+    nan = want.float().isnan()
+    assert torch.equal(q.cpu().view(torch.uint8)[~nan], want.view(torch.uint8)[~nan])  # (the sign of zero too)
