@@ -768,13 +768,18 @@ int best_batch_shape(const BatchArgs& a, bool sliced, float* cost)
 }
 }  // namespace
 
-// One launch against a launch each (us, estimates as above, and 1 us for every launch that follows another).
+// One launch against a launch each: us, estimates as above; in a step operands come from memory rather than from the last
+// repetition's L2, so a product on its own takes 1.2 times its estimate, and every launch that follows another 2 us.  Fitted to 66 sets
+// of two to six products, 400-4000 rows of 1024 and 2048 (replayed graphs, operands of four sets in turn): 0.3 % over the better of the two
+// on average, 5 % before the two constants; the largest misses 5 %.  us together / apart: the six products of three projections'
+// backward, 1537 x 2048 61 / 84, 4000 x 2048 146 / 153; grad_input and grad_weight of one 21 / 27, 4000 rows 47 / 41; of two
+// projections 1024 -> 2816, 3000 rows 46 / 61.
 extern "C" int mi8_gemm_fp8_batch_pays(const mi8_gemm_product* products, int32_t count)
 {
     BatchArgs a;
     bool sliced;
     if (batch_args(products, count, a, sliced) != MI8_OK) return 0;
-    float together = 0.0f, apart = (float)(count - 1);
+    float together = 0.0f, apart = 2.0f * (float)(count - 1);
     best_batch_shape(a, sliced, &together);
     for (int i = 0; i < count; ++i) {
         const GemmArgs& g = a.g[i];
@@ -785,7 +790,7 @@ extern "C" int mi8_gemm_fp8_batch_pays(const mi8_gemm_product* products, int32_t
             const float p = m16_cost(g.M, g.N, g.K);
             t = p < t ? p : t;
         }
-        apart += t;
+        apart += 1.2f * t;
     }
     return together < apart ? 1 : 0;
 }
