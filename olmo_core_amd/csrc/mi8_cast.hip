@@ -354,7 +354,7 @@ struct GroupedCastArgs {
 __device__ __forceinline__ bool locate_padded_tile(const int64_t* sizes, int E, int64_t T, int p, int& e,
                                                    int64_t& row0, int64_t& row_end)
 {
-    if (E <= 4) {  // a handful of groups (one: the dense two-product cast): walking them is cheaper than a scan
+    if (E <= 4) {  // a handful of groups: walking them is cheaper than a scan
         int64_t before = 0;
         int tiles = 0;
         for (e = 0; e < E; ++e) {
