@@ -291,6 +291,9 @@ class Plan:
 _plans: dict = {}
 _seen: dict = {}
 
+# The hooks that saved tensors go through on this thread (activation checkpointing, offloading), or None.
+_saved_tensor_hooks = torch._C._autograd._top_saved_tensors_default_hooks
+
 
 def _plannable(inputs) -> bool:
     for t in inputs:
@@ -315,8 +318,12 @@ def call(fn: Callable, inputs: Sequence[Optional[torch.Tensor]], options: tuple,
     """``(outputs, kept, plan)`` of ``fn(*inputs)`` replayed from its plan, or ``None`` where it has none (yet): then the
     caller runs ``fn`` itself.  ``fn`` returns the tensors to be returned and a tree of those to be kept; what it does must
     follow from the shapes and types of ``inputs`` and from ``options`` (hashable, ``fn`` named in it) alone.  ``within``: the
-    plan that this one continues.  ``own``: how many of the last inputs are this package's own tensors (contiguous, aligned)."""
-    if _observed() or not _plannable(inputs[:-own] if own else inputs):
+    plan that this one continues.  ``own``: how many of the last inputs are this package's own tensors (contiguous, aligned).
+
+    A forward under saved-tensor hooks has no plan: it would save one buffer where ``fn`` itself saves the tensors, and
+    which of the two runs depends on how often the sizes were met.  Hooks see every saved tensor, and checkpointing refuses a
+    re-run that saves other tensors than the first run did."""
+    if (within is None and _saved_tensor_hooks(True) is not None) or _observed() or not _plannable(inputs[:-own] if own else inputs):
         return None
     key = [options, inputs[0].device.index]
     for t in inputs:

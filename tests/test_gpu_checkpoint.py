@@ -13,7 +13,8 @@ from helpers import seeded
 
 pytestmark = pytest.mark.gpu
 
-from olmo_core_amd.float8 import AOFloat8LinearRecipe, Float8Config  # noqa: E402
+from olmo_core_amd.float8 import AOFloat8LinearRecipe, Float8Config, plan  # noqa: E402
+from olmo_core_amd.float8.linear import float8_projections  # noqa: E402
 from olmo_core_amd.nn import FeedForward  # noqa: E402
 
 
@@ -65,3 +66,51 @@ def test_checkpointed_block_reruns_bit_identically(dev, recipe, fuse):
     for name, a, b, c in zip(names, plain, full, selected):
         assert torch.equal(a, b), f"{name}: full re-run differs from the plain call"
         assert torch.equal(a, c), f"{name}: selected-ops re-run differs from the plain call"
+
+
+@pytest.mark.parametrize("recipe", ["tensorwise", "rowwise"])
+@pytest.mark.parametrize("what", ["linear", "projections", "block"])
+def test_sizes_whose_first_call_is_checkpointed(dev, monkeypatch, recipe, what):
+    """No call on these sizes came before: the first run, its re-run in the backward, the same layer again and a second layer
+    of its sizes save the same tensors, however often the sizes were met, and give the bits of plain calls."""
+    monkeypatch.setattr(plan, "_plans", {})
+    monkeypatch.setattr(plan, "_seen", {})
+    if what == "block":
+        layers = [_block(dev, recipe, True, 256, 512) for _ in range(2)]
+    else:
+        layers = [torch.nn.ModuleList([torch.nn.Linear(256, 256, bias=False, dtype=torch.bfloat16, device=dev) for _ in range(3)]) for _ in range(2)]
+        for m in layers:
+            Float8Config(ao_recipe=AOFloat8LinearRecipe(recipe)).apply_float8_linear(m)
+    model = torch.nn.ModuleList(layers)
+    one = {"block": lambda m, t: m(t), "linear": lambda m, t: m[0](t), "projections": lambda m, t: sum(float8_projections(t, *m))}[what]
+    x, go = seeded((77, 256), 1).to(dev), seeded((77, 256), 2, std=1e-3).to(dev)
+
+    def run(call):
+        model.zero_grad()
+        xd = x.clone().requires_grad_(True)
+        y = xd
+        for m in layers:
+            y = call(lambda t, m=m: one(m, t), y)
+        y.backward(go)
+        return [y.detach(), xd.grad, *(p.grad for p in model.parameters() if p.grad is not None)]
+
+    rerun = [run(lambda f, t: checkpoint(f, t, use_reentrant=False)) for _ in range(3)]
+    plain = [run(lambda f, t: f(t)) for _ in range(3)]
+    assert plan._plans  # (the plain calls' sizes have come back by now)
+    rerun.append(run(lambda f, t: checkpoint(f, t, use_reentrant=False)))
+    for got in (*plain[1:], *rerun):
+        assert len(got) == len(plain[0]) and all(torch.equal(a, b) for a, b in zip(got, plain[0]))
+
+
+def test_saved_tensor_hooks_see_the_tensors(dev, monkeypatch):
+    """Hooks on saved tensors see the same ones on the first call of a set of sizes and on later ones."""
+    monkeypatch.setattr(plan, "_plans", {})
+    monkeypatch.setattr(plan, "_seen", {})
+    ff = _block(dev, "tensorwise", True, 256, 512)
+    seen = []
+    for _ in range(4):
+        packed = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append((t.shape, t.dtype)) or t, lambda t: t):
+            ff(seeded((90, 256), 1).to(dev).requires_grad_(True)).sum().backward()
+        seen.append(packed)
+    assert len(seen[0]) == 13 and all(p == seen[0] for p in seen)
