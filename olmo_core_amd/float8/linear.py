@@ -214,7 +214,7 @@ def _backward_impl(go2, c: Float8LinearConfig, N: int, x_dtype, w_dtype, x_part,
         else:
             products.append(_grad_weight_product(go2, c, go_cols, x_part, x_is_q, w_dtype))
     if products:
-        made = ops.gemm_fp8_batch(products, out_dtype=x_dtype)
+        made = ops.gemm_fp8_products(products, out_dtype=x_dtype)
         if need_gw and not _is_disabled(cgw):
             gw = made.pop()
         if made:
@@ -285,7 +285,7 @@ def _planned_backward(ctx, gos, ns, need_gx: bool, need_gws):
         made = _grad_operands(gos_, c, need_gx, need_gws)
         ps = [_grad_input_product(gos_[i], c, ns[i], made[i][0], w_parts[i], True, add=i != order[0]) for i in order if need_gx]
         ps += [_grad_weight_product(gos_[i], c, made[i][1], x_part, True, ctx.w_dtypes[i]) for i in wanted]
-        return ops.gemm_fp8_batch(ps, out_dtype=ctx.x_dtype) if ps else []
+        return ops.gemm_fp8_products(ps, out_dtype=ctx.x_dtype)
 
     def recorded(slab, *places):
         return products(places, ctx.plan.saved_places(slab)), None
@@ -432,7 +432,7 @@ class _Float8SharedInputMatmul(torch.autograd.Function):
                         for i in order if need_gx]
             wanted = [i for i in order if ctx.need_gws[i]]
             products += [_grad_weight_product(gos[i], c, made[i][1], x_part, ctx.x_is_q, ctx.w_dtypes[i]) for i in wanted]
-            outs = ops.gemm_fp8_batch(products, out_dtype=ctx.x_dtype) if products else []
+            outs = ops.gemm_fp8_products(products, out_dtype=ctx.x_dtype)
             if need_gx:
                 gx = outs.pop(0)
             for i, gw in zip(wanted, outs):

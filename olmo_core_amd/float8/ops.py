@@ -458,6 +458,18 @@ def gemm_fp8_batch(products, *, out_dtype: torch.dtype = torch.bfloat16, togethe
     return outs
 
 
+def gemm_fp8_products(products, *, out_dtype: torch.dtype = torch.bfloat16) -> list:
+    """:func:`gemm_fp8_batch` of products whose pairs of float8 types may differ (grad_input contracts with the weight's type,
+    grad_weight with the input's): neighbours of one pair together."""
+    outs, start = [], 0
+    for i in range(1, len(products) + 1):
+        a, b = products[start][0], products[start][2]
+        if i == len(products) or products[i][0].dtype != a.dtype or products[i][2].dtype != b.dtype:
+            outs += gemm_fp8_batch(products[start:i], out_dtype=out_dtype)
+            start = i
+    return outs
+
+
 def swiglu_gemm_supported(M: int, H: int, K: int) -> bool:
     """Shapes :func:`gemm_fp8_swiglu` takes (otherwise: two :func:`gemm_fp8` calls and :func:`swiglu_fwd`)."""
     return M >= 256 and H >= 128 and H % 8 == 0 and K % 128 == 0

@@ -157,7 +157,7 @@ def _mlp_backward(gy, saved, c, dims, dtypes, need):
             gh, gh_codes = ops.gemm_fp8_codes(gyq, sgy, w2q_t, s2, k=D)
             codes = (gh_codes, x_codes)
         else:
-            gh, *rest = ops.gemm_fp8_batch([(gyq, sgy, w2q_t, s2, D, False)] + ([w2_product] if need_w2 else []), out_dtype=x_dt)
+            gh, *rest = ops.gemm_fp8_products([(gyq, sgy, w2q_t, s2, D, False)] + ([w2_product] if need_w2 else []), out_dtype=x_dt)
             gw2 = rest[0] if need_w2 else None
         if STAGE_SINK is not None:
             STAGE_SINK.update(gh=gh.clone())
@@ -179,7 +179,7 @@ def _mlp_backward(gy, saved, c, dims, dtypes, need):
             products.append((g1q_t, sg1, xq_t, sx, None, False, w1_dt))
         if need_w3:
             products.append((g3q_t, sg3, xq_t, sx, None, False, w3_dt))
-        outs = ops.gemm_fp8_batch(products, out_dtype=x_dt)
+        outs = ops.gemm_fp8_products(products, out_dtype=x_dt)
         if need_w3:
             gw3 = outs.pop()
         if need_w1:

@@ -514,3 +514,47 @@ def test_forward_replays_from_a_captured_graph(dev, tokens):
             torch.cuda.synchronize()
             eager = model(x_new)
             assert torch.equal(y_static, eager), i
+
+
+@pytest.mark.parametrize("granularity", ["tensorwise", "axiswise"])
+@pytest.mark.parametrize("x_dt, w_dt, go_dt", [(E5M2, E4M3, E5M2), (E4M3, E5M2, E5M2), (E5M2, E4M3, E4M3)], ids=["x", "w", "x_not_go"])
+def test_input_and_weight_in_different_float8_types(dev, x_dt, w_dt, go_dt, granularity):
+    """grad_input contracts with the weight's type, grad_weight with the input's, and a config may set them apart: a linear
+    against the oracle, and projections of one input and the fused block against the modules one by one."""
+    from olmo_core_amd.float8.linear import float8_projections
+    from olmo_core_amd.float8.native_config import CastConfig, ScalingGranularity
+    from olmo_core_amd.nn import FeedForward
+
+    cast = lambda dt: CastConfig(scaling_granularity=ScalingGranularity(granularity), target_dtype=dt)  # noqa: E731
+    config = Float8LinearConfig(cast_config_input=cast(x_dt), cast_config_weight=cast(w_dt), cast_config_grad_output=cast(go_dt),
+                                round_scales_to_power_of_2=granularity == "axiswise")
+    spec = O.LinearSpec(*(O.CastSpec(O.DYNAMIC, granularity, dt) for dt in (x_dt, w_dt, go_dt)),
+                        round_scales_to_power_of_2=granularity == "axiswise")
+    M, K, N = 300, 256, 272
+    x, go = seeded((M, K), 1), seeded((M, N), 2, std=1e-3)
+
+    def run(fwd, params, *gos):
+        for p in params:
+            p.grad = None
+        xd = x.to(dev).requires_grad_(True)
+        ys = fwd(xd)
+        torch.autograd.backward(ys, [g.to(dev) for g in gos])
+        return [*ys, xd.grad, *(p.grad for p in params)]
+
+    q, k = (convert_to_float8_training(nn.Linear(K, N, bias=False, dtype=torch.bfloat16, device=dev), config=config) for _ in range(2))
+    ref = O.linear_fwd_bwd(x, q.weight.detach().cpu(), None, go, spec)
+    for _ in range(4):  # (later calls replay a plan)
+        got = run(lambda t: [q(t)], [q.weight], go)
+        for a, b in zip(got, (ref.out, ref.grad_input, ref.grad_weight)):
+            assert_gemm_close(a, b)
+    apart = run(lambda t: [q(t), k(t)], [q.weight, k.weight], go, -go)
+    ff = FeedForward(d_model=K, hidden_size=528, bias=False, dtype=torch.bfloat16, init_device="cuda")
+    convert_to_float8_training(ff, config=config)
+    ff.fuse_float8 = False
+    block = run(lambda t: [ff(t)], list(ff.parameters()), seeded((M, K), 3, std=1e-3))
+    ff.fuse_float8 = True
+    for _ in range(4):
+        for a, b in zip(run(lambda t: float8_projections(t, q, k), [q.weight, k.weight], go, -go), apart):
+            assert torch.equal(a, b)
+        for a, b in zip(run(lambda t: [ff(t)], list(ff.parameters()), seeded((M, K), 3, std=1e-3)), block):
+            assert torch.equal(a, b)
