@@ -535,7 +535,7 @@ int mi8_plan_function(const char* name);
 int mi8_run_plan(const int64_t* words, int64_t n_words, const void* const* buffers, int32_t n_buffers, void* stream);
 /* partial maxima that mi8_gemm_fp8_swiglu writes for these sizes on the current device (its *n_slots_used) */
 int32_t mi8_gemm_fp8_swiglu_slots(int64_t M, int64_t H, int64_t K);
-int32_t mi8_few_rows_swiglu_slots(int64_t M, int64_t H, int64_t K, int x_is_fp8); /* (as well for mi8_few_rows_swiglu) */
+int32_t mi8_few_rows_swiglu_slots(int64_t M, int64_t H, int64_t K, int x_is_fp8); /* (of mi8_few_rows_swiglu, operands without padding: lda = ldb = K) */
 
 #ifdef __cplusplus
 }

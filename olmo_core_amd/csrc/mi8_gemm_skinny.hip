@@ -403,8 +403,11 @@ namespace {
 // kernel above reads it from L2 for every 16: more rows, or more bytes of weights, make that the time.  us, above / ring:
 // 16 x 8192 x 2048 9.9 / 9.0, 23 x 11008 x 4096 28.5 / 25.3, 48 x 11008 x 4096 43.6 / 27.1, 64 x 8192 x 2048 18.5 / 9.3,
 // 4 x 27648 x 5120 66.6 / 56.6, 64 x 27648 x 5120 135 / 70; 8 x 11008 x 4096 24.3 / 24.2, 32 x 2816 x 1024 5.6 / 5.8.
-bool dual_on_ring(int64_t M, int64_t H, int64_t K)
+// Ring tiles address the rows of a tile, all of A and 32 of each matrix, with 32-bit offsets; the kernel above with 64-bit ones.
+bool dual_on_ring(int64_t M, int64_t H, int64_t K, int64_t lda, int64_t ldb)
 {
+    constexpr int64_t most = (int64_t)1 << 32;
+    if (lda >= most || ldb >= most || M * lda >= most || 32 * ldb >= most) return false;
     const int64_t bytes = 2 * H * K;
     return M > 32 || (bytes >= 16 << 20 && M > 8) || (bytes >= 200 << 20 && M > 3);
 }
@@ -412,7 +415,7 @@ bool dual_on_ring(int64_t M, int64_t H, int64_t K)
 
 extern "C" int32_t mi8_few_rows_swiglu_slots(int64_t M, int64_t H, int64_t K, int x_is_fp8)
 {
-    return x_is_fp8 && dual_on_ring(M, H, K) ? dual_ring_slots(H) : (int32_t)((H + 15) / 16);
+    return x_is_fp8 && dual_on_ring(M, H, K, K, K) ? dual_ring_slots(H) : (int32_t)((H + 15) / 16);
 }
 
 extern "C" int mi8_few_rows_swiglu(const void* x, int x_is_fp8, int64_t lda, const float* sx, const void* b1, const void* b3,
@@ -440,10 +443,11 @@ extern "C" int mi8_few_rows_swiglu(const void* x, int x_is_fp8, int64_t lda, con
     a.sb3 = sb3;
     a.pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
     a.slots_out = slots_h;
-    *n_slots_used = mi8_few_rows_swiglu_slots(M, H, K, x_is_fp8);
+    const bool on_ring = x_is_fp8 && dual_on_ring(M, H, K, lda, ldb);
+    *n_slots_used = on_ring ? dual_ring_slots(H) : (int32_t)((H + 15) / 16);
     hipStream_t st = (hipStream_t)stream;
     if (!x_is_fp8) return launch_few_rows<1, 1, kAmax, true>(a, st, "mi8_few_rows_swiglu");
-    if (dual_on_ring(M, H, K)) {
+    if (on_ring) {
         a.g.B3 = a.B3;
         a.g.sb3 = sb3;
         a.g.slots_out = slots_h;

@@ -76,6 +76,14 @@ def test_few_rows_slices():
                 assert L.mi8_gemm_splitk_suggest(m, n, 128 * steps - 16) in (1, -(-steps // per)), (m, n, steps)
 
 
+def test_few_rows_swiglu_on_ring_tiles_only_where_offsets_fit():
+    """Ring tiles have 32-bit offsets into a tile's rows (a partial maximum per 32 columns of h); rows that are further apart stay
+    on the kernel with 64-bit addresses (one per 16)."""
+    slots = lambda m, k: _C.lib().mi8_few_rows_swiglu_slots(m, 64, k, 1)  # noqa: E731
+    assert slots(64, 4096) == slots(64, (1 << 26) - 16) == slots(32, (1 << 27) - 16) == 2
+    assert slots(64, 1 << 26) == slots(33, 1 << 27) == slots(32, 1 << 27) == slots(9, 1 << 27) == 4
+
+
 def test_variant_for():
     """The kernel a product runs on: few rows, tiles too few or of the wrong kind for the persistent kernel, and its own."""
     L = _C.lib()

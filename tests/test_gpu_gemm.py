@@ -654,6 +654,22 @@ def test_few_rows_swiglu_on_ring_tiles(dev, M, H, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [9, 33, 40])
+def test_few_rows_swiglu_takes_a_wide_pitch(dev, M):
+    """Rows of x and of both weights 2^27 bytes apart: offsets into a tile's rows beyond 32 bits."""
+    H, K, pitch = 40, 272, 1 << 27
+    buf = torch.empty(H * pitch, dtype=torch.uint8, device=dev).view(torch.float8_e4m3fn).view(H, pitch)
+    g = torch.Generator(device=dev).manual_seed(M)
+    x, w1, w3 = (buf[:n, 512 * i:512 * i + K] for i, n in enumerate((M, H, H)))
+    for t in (x, w1, w3):
+        t.copy_(torch.randn(t.shape, generator=g, device=dev).to(torch.float8_e4m3fn))
+    sx, s1, s3 = (torch.full((1,), v, device=dev) for v in (3.0, 5.0, 7.0))
+    h, (slots, n) = ops.few_rows_swiglu(x, sx, w1, s1, w3, s3)
+    want, (want_slots, m) = ops.few_rows_swiglu(x.contiguous(), sx, w1.contiguous(), s1, w3.contiguous(), s3)
+    assert torch.equal(h, want) and int(slots[:n].max()) == int(want_slots[:m].max())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("vec", [False, True])
 def test_float32_outputs_of_bf16_values(dev, vec):
     """float32 outputs that hold the bf16 values: every kernel, tiles shifted back over their neighbours and half tiles of the
