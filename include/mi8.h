@@ -226,7 +226,8 @@ int mi8_gemm_fp8(const void* a, int a_dtype, int64_t lda, const void* b, int b_d
  * tensors of out_dtype.  This is how the grad_input of a block whose input feeds two linears (w1 and w3 of the
  * feed-forward block, src/olmo_core/nn/feed_forward.py:171) is summed by autograd; here the second GEMM adds into the
  * first one's output and the separate elementwise pass over [M, N] disappears.  Arguments as mi8_gemm_fp8 (the kernel
- * is chosen by shape). */
+ * is chosen by shape), out_dtype MI8_BF16 or MI8_F32: MI8_F32_OF_BF16 is for products that are not added to anything, here
+ * and in the other entry points that add. */
 int mi8_gemm_fp8_accumulate(const void* a, int a_dtype, int64_t lda, const void* b, int b_dtype, int64_t ldb, int64_t M,
                             int64_t N, int64_t K, const float* sa, int sa_is_vector, const float* sb, int sb_is_vector,
                             void* out, int out_dtype, int64_t ldc, void* stream);
@@ -299,7 +300,7 @@ int mi8_gemm_fp8_batch(const mi8_gemm_product* products, int32_t count, int a_dt
 int mi8_gemm_num_variants(void);
 const char* mi8_gemm_variant_name(int variant);
 /* Host only: the variant that -1 stands for in mi8_gemm_fp8 (accumulate != 0: in mi8_gemm_fp8_accumulate) when ldc == N, the
- * pointers are 16-byte aligned and the scales of one kind; -1 for an empty product. */
+ * pointers are 16-byte aligned and the scales of one kind; -1 for an empty product and for a sum in MI8_F32_OF_BF16. */
 int mi8_gemm_variant_for(int64_t M, int64_t N, int64_t K, int out_dtype, int accumulate);
 
 /* ---------------------------------------------------------------------------------------------

@@ -476,7 +476,7 @@ int chosen_variant(int64_t M, int64_t N, int64_t K, bool m16_fits)
 
 extern "C" int mi8_gemm_variant_for(int64_t M, int64_t N, int64_t K, int out_dtype, int accumulate)
 {
-    if (M <= 0 || N <= 0 || K <= 0) return -1;
+    if (M <= 0 || N <= 0 || K <= 0 || (accumulate && out_dtype == MI8_F32_OF_BF16)) return -1;
     return chosen_variant(M, N, K, m16_takes(M, N, K, N, out_dtype, accumulate != 0));
 }
 
@@ -510,6 +510,7 @@ int gemm_fp8_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b
                 MI8_ERR_UNSUPPORTED, "mi8_gemm_fp8: operand larger than 4 GiB");
     MI8_REQUIRE(gemm_out_dtype(out_dtype), MI8_ERR_ARG, "mi8_gemm_fp8: unknown output dtype %d",
                 out_dtype);
+    MI8_REQUIRE(!accumulate || out_dtype != MI8_F32_OF_BF16, MI8_ERR_UNSUPPORTED, "mi8_gemm_fp8_accumulate: a sum is not rounded to bf16 values");
     GemmArgs g{(const uint8_t*)a, (const uint8_t*)b, out, c_f32_of(out_dtype), lda, ldb, ldc, (int)M, (int)N, (int)K,
                sa, sb, sa_is_vector ? 1 : 0, sb_is_vector ? 1 : 0, 0, 0, accumulate ? 1 : 0};
     hipStream_t st = (hipStream_t)stream;
@@ -660,6 +661,8 @@ int splitk_entry(const void* a, int a_dtype, int64_t lda, const void* b, int b_d
                 MI8_ERR_UNSUPPORTED, "mi8_gemm_fp8_splitk: operand larger than 4 GiB");
     MI8_REQUIRE(gemm_out_dtype(out_dtype), MI8_ERR_ARG,
                 "mi8_gemm_fp8_splitk: unknown output dtype %d", out_dtype);
+    MI8_REQUIRE(!accumulate || out_dtype != MI8_F32_OF_BF16, MI8_ERR_UNSUPPORTED,
+                "mi8_gemm_fp8_splitk_accumulate: a sum is not rounded to bf16 values");
     const int64_t steps = (K + BK - 1) / BK;
     MI8_REQUIRE(splits >= 1 && splits <= 64 && splits <= steps, MI8_ERR_ARG,
                 "mi8_gemm_fp8_splitk: splits (%d) must be in 1..min(64, K steps = %lld)", splits, (long long)steps);
@@ -741,6 +744,8 @@ int batch_args(const mi8_gemm_product* p, int32_t count, BatchArgs& a, bool& sli
         MI8_REQUIRE(!q.add_to_previous || (i > 0 && q.M == p[i - 1].M && q.N == p[i - 1].N && q.out == p[i - 1].out && q.ldc == p[i - 1].ldc &&
                                            q.out_dtype == p[i - 1].out_dtype),
                     MI8_ERR_ARG, "%s: product %d adds to the one before it: one output and sizes are wanted", what, i);
+        MI8_REQUIRE(!q.add_to_previous || q.out_dtype != MI8_F32_OF_BF16, MI8_ERR_UNSUPPORTED, "%s: product %d: a sum is not rounded to bf16 values",
+                    what, i);
         a.g[i] = GemmArgs{(const uint8_t*)q.a, (const uint8_t*)q.b, q.out, c_f32_of(q.out_dtype), q.lda, q.ldb, q.ldc, (int)q.M,
                           (int)q.N, (int)q.K, q.sa, q.sb, q.sa_is_vector ? 1 : 0, q.sb_is_vector ? 1 : 0, 0, 0, q.add_to_previous ? 1 : 0,
                           slice_steps_of(q.M, q.N, q.K)};

@@ -333,7 +333,7 @@ def gemm_fp8(
     ``splits``: slices of K summed separately and added afterwards (for problems with few output tiles);
     -1 lets the library decide from the shape, 0 and 1 forbid splitting; a forced ``variant`` is never split.  More of them
     than K has steps of 128 (or than 64) are refused; ``accumulate`` sums such a product unsplit.
-    ``rounded`` (float32 ``out_dtype``): the values that a bfloat16 output would have.
+    ``rounded`` (float32 ``out_dtype``, not with ``accumulate``): the values that a bfloat16 output would have.
     """
     _require_gpu(a, "gemm_fp8")
     if a.dim() != 2 or b.dim() != 2 or a.stride(1) != 1 or b.stride(1) != 1:
@@ -348,6 +348,9 @@ def gemm_fp8(
         raise ValueError(f"gemm_fp8: scale sizes {sa.numel()}, {sb.numel()} do not match M={M}, N={N}")
     if accumulate and out is None:
         raise ValueError("gemm_fp8: accumulate needs the tensor to add into (out=)")
+    rounded = rounded and out_dtype == torch.float32
+    if accumulate and rounded:
+        raise ValueError("gemm_fp8: a sum is not rounded to bfloat16 values (accumulate with rounded)")
     if out is None:
         out = _empty((M, N), dtype=out_dtype, device=a.device)
     elif tuple(out.shape) != (M, N) or out.dtype != out_dtype or out.stride(1) != 1 or out.device != a.device:
@@ -360,7 +363,7 @@ def gemm_fp8(
         ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         ev0.record()
     L = _C.lib()
-    code = _C.MI8_F32_OF_BF16 if rounded and out_dtype == torch.float32 else _HP_CODE[out_dtype]
+    code = _C.MI8_F32_OF_BF16 if rounded else _HP_CODE[out_dtype]
     if variant >= 0:
         splits = 1
     elif splits < 0:
@@ -410,7 +413,7 @@ def gemm_fp8_batch(products, *, out_dtype: torch.dtype = torch.bfloat16, togethe
     Several :func:`gemm_fp8` products of one pair of float8 types: ``products`` is a list of ``(a, sa, b, sb, k, add)``,
     ``k`` the contracted length (``None``: that of the operands) and ``add`` whether the product is added to the one
     before it (the bits of an elementwise add of the two outputs).  A seventh element ``torch.float32`` wants the product
-    of a bfloat16 ``out_dtype`` as float32 values (the gradient of a float32 weight).  Returns the outputs of those that are not added, in
+    of a bfloat16 ``out_dtype`` as float32 values (the gradient of a float32 weight; no term of a sum).  Returns the outputs of those that are not added, in
     order.  One launch where the library estimates that it is faster than one per product (``together`` decides
     otherwise); the results are the same bits.
     """
@@ -438,6 +441,8 @@ def gemm_fp8_batch(products, *, out_dtype: torch.dtype = torch.bfloat16, togethe
             raise ValueError(f"gemm_fp8_batch: scale sizes {sa.numel()}, {sb.numel()} do not match M={M}, N={N}")
         if add and (not outs or tuple(outs[-1].shape) != (M, N)):
             raise ValueError("gemm_fp8_batch: nothing of its shape to add the product to")
+        if add and (f32 or outs[-1].dtype != out_dtype):
+            raise ValueError("gemm_fp8_batch: a sum is not rounded to bfloat16 values (float32 product that is added or added to)")
         if not add:
             outs.append(_empty((M, N), dtype=torch.float32 if f32 else out_dtype, device=a.device))
         if one_launch:

@@ -133,6 +133,17 @@ def test_argument_validation_happens_before_any_gpu_call():
         _C.check(-2, "x")
 
 
+def test_sums_are_not_rounded_to_bf16_values():
+    """MI8_F32_OF_BF16 holds what a bf16 output would; of a sum that is a value rounded twice, which no entry point that adds forms."""
+    L, p = _C.lib(), 1 << 20  # (16-byte aligned; never read: refused before any launch)
+    args = (p, _C.MI8_E4M3, 256, p, _C.MI8_E4M3, 256, 128, 128, 256, p, 0, p, 0, p, _C.MI8_F32_OF_BF16, 128)
+    assert L.mi8_gemm_fp8_accumulate(*args, None) == -2
+    assert L.mi8_gemm_fp8_splitk_accumulate(*args, 2, p, 1 << 30, None) == -2
+    chain = (_C.GemmProduct * 2)(*(_C.GemmProduct(p, 256, p, 256, 128, 128, 256, p, p, p, 128, 0, 0, _C.MI8_F32_OF_BF16, i) for i in range(2)))
+    assert L.mi8_gemm_fp8_batch(chain, 2, _C.MI8_E4M3, _C.MI8_E4M3, None) == -2 and not L.mi8_gemm_fp8_batch_pays(chain, 2)
+    assert L.mi8_gemm_variant_for(512, 512, 256, _C.MI8_F32_OF_BF16, 1) == -1 != L.mi8_gemm_variant_for(512, 512, 256, _C.MI8_F32_OF_BF16, 0)
+
+
 def test_few_rows_entry_points_refuse():
     """What the two launches of a generation step do not take, by their numbers alone (the pointers are never followed)."""
     L, p, odd = _C.lib(), ctypes.c_void_p(256), ctypes.c_void_p(264)

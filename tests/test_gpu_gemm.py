@@ -637,6 +637,13 @@ def test_products_in_one_launch_refuse_what_one_launch_cannot_take(dev):
     with pytest.raises(MI8KernelError, match="multiples of 16"):
         ops.gemm_fp8_batch([(a, one, a, one, 40, False)] * 2, together=True)
     assert len(ops.gemm_fp8_batch([(a, one, a, one, None, False)] * 9)) == 9
+    f32, add = (a, one, a, one, None, False, torch.float32), (a, one, a, one, None, True)
+    for together in (None, False, True):  # a sum of float32 values that are rounded to bf16
+        for chain in ([f32, add], [f32, (*add, torch.float32)], [f32[:6], (*add, torch.float32)]):
+            with pytest.raises(ValueError, match="sum is not rounded"):
+                ops.gemm_fp8_batch(chain, together=together)
+    with pytest.raises(ValueError, match="sum is not rounded"):
+        ops.gemm_fp8(a, one, a, one, out=torch.zeros(128, 128, device=dev), out_dtype=torch.float32, accumulate=True, rounded=True)
 
 
 @pytest.mark.gpu
