@@ -108,3 +108,26 @@ def test_sizes_that_do_not_come_back_are_not_recorded(dev, runs):
         for tokens in range(1, 9):
             lin(seeded((tokens, 128), 1).to(dev))
     assert not plan._plans and len(plan._seen) == 8 and not runs
+
+
+@pytest.mark.parametrize("name, tokens, kept", [
+    ("swiglu_fwd", 300, False), ("few_rows_swiglu", 23, True), ("few_rows_cast_gemm", 3, True), ("gemm_fp8_swiglu", 4096, False),
+    ("gemm_fp8_codes", 4096, False), ("swiglu_bwd_cast", 300, False), ("gemm_fp8_products", 300, False), ("cast_tensorwise", 300, False)])
+def test_replaced_operations_are_called(dev, runs, monkeypatch, name, tokens, kept):
+    """An operation that is replaced after its calls were recorded is called again."""
+    model = FeedForward(d_model=256, hidden_size=2048, bias=False, dtype=torch.bfloat16, init_device="cuda")
+    Float8Config(ao=AOFloat8LinearConfig.recommended() if kept else AOFloat8LinearConfig()).apply_float8_linear(_fill(model))
+    x, go = seeded((tokens, 256), 1).to(dev), seeded((tokens, 256), 2, std=1e-3).to(dev)
+
+    def step():
+        if not kept:
+            return _step(model, x, lambda t: [model(t)], [go])
+        with torch.no_grad():
+            return [model(x)]
+
+    want = [step() for _ in range(4)][-1]
+    n, called, real = len(runs), [], getattr(plan.ops, name)
+    assert n
+    monkeypatch.setattr(plan.ops, name, lambda *a, **k: called.append(1) or real(*a, **k))
+    got = step()
+    assert called and len(runs) == n and all(torch.equal(a, b) for a, b in zip(got, want))
