@@ -226,6 +226,7 @@ class Plan:
         self._buffers = ctypes.c_void_p * self.n_buffers
         self._saved = self._rebase(saved, where)
         self.then: dict = {}  # plans of the backward, which depend on where this one keeps what it keeps
+        self.used = False  # replayed since its table was last full
 
     @staticmethod
     def _put(where, number, n, sizes, totals, buffer) -> None:
@@ -290,6 +291,12 @@ class Plan:
         return outs, kept
 
 
+class _NoPlan:
+    """Stands in the table for a sequence that cannot be recorded."""
+
+    used = False
+
+
 _plans: dict = {}
 _seen: dict = {}
 
@@ -314,6 +321,19 @@ def _observed() -> bool:
     """Someone watches single launches (measurement hooks) or has put a function of theirs in the place of an operation of
     :mod:`ops`, any of which a recorded sequence may have called (0.9 us for the 43 of them)."""
     return ops.GEMM_EVENT_SINK is not None or ops.FORCE_SW_CVT or _operations(_OPS) != _ORIGINALS
+
+
+def _remember(plans: dict, key: tuple, plan) -> None:
+    """A full table gives up what was not replayed since it was last full, or else its older half: sizes that come back stay
+    where others come once."""
+    if len(plans) >= _MOST_PLANS:
+        for k, p in list(plans.items()):
+            if not p.used:
+                plans.pop(k, None)
+            p.used = False
+        for k in list(plans)[:len(plans) - _MOST_PLANS // 2] if len(plans) >= _MOST_PLANS else ():
+            plans.pop(k, None)
+    plans[key] = plan
 
 
 def call(fn: Callable, inputs: Sequence[Optional[torch.Tensor]], options: tuple, within: Optional[Plan] = None,
@@ -346,10 +366,10 @@ def call(fn: Callable, inputs: Sequence[Optional[torch.Tensor]], options: tuple,
         try:
             plan = Plan(fn, [(tuple(t.shape), t.dtype) if t is not None else None for t in inputs], inputs[0].device.index)
         except Exception:  # (what it is that cannot be done on placeholders, or at all, the caller's own run says)
-            plan = False
-        if len(plans) >= _MOST_PLANS:
-            plans.clear()
-        plans[key] = plan
-    if plan is False:
+            plan = _NoPlan()
+        _remember(plans, key, plan)
+    else:
+        plan.used = True
+    if type(plan) is _NoPlan:
         return None
     return (*plan.run(inputs), plan)
