@@ -261,7 +261,7 @@ def _planned_forward(x2, weights, c: Float8LinearConfig, scales, w_ops, need_gx:
         ys, x_saved, w_saved = _shared_input_forward(px, rest[:n], c, rest[n:2 * n], [g if g[0] is not None else None for g in given],
                                                      need_gx, need_gw)
         if (need_gw and x_saved is None) or (need_gx and None in w_saved):
-            raise plan.Unplannable
+            raise plan.Unplannable("an input is kept")
         return ys, (x_saved if need_gw else None, w_saved if need_gx else None)
 
     inputs = [x2, *weights, *scales]

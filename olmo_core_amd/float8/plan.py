@@ -17,6 +17,7 @@ and backward 391 / 194 (the GPU 182); four attention projections of 1537 tokens 
 from __future__ import annotations
 
 import ctypes
+import logging
 import operator
 import types
 from typing import Callable, Optional, Sequence
@@ -25,6 +26,8 @@ import torch
 
 from .. import _C
 from . import ops
+
+_log = logging.getLogger(__name__)
 
 _OFFSET = (1 << 48) - 1
 _STREAM, _IGNORED = -1, -2
@@ -96,15 +99,18 @@ class _Place:
     def is_inference(self) -> bool:  # (no version counter to move)
         return True
 
-    def to(self, dtype) -> "_Place":
-        if dtype != self.dtype:
-            raise Unplannable
+    def to(self, *args, **kwargs) -> "_Place":
+        if kwargs or len(args) != 1 or args[0] != self.dtype:
+            raise Unplannable("a conversion")
         return self
+
+    def __getattr__(self, name: str):
+        raise Unplannable(f"tensor.{name}")
 
     def reshape(self, *shape) -> "_Place":
         out = _Place(self.device, shape[0] if len(shape) == 1 and not isinstance(shape[0], int) else shape, self.dtype, self.address)
         if out.numel() != self.numel():
-            raise Unplannable
+            raise Unplannable("a reshape")
         return out
 
     def new_empty(self, shape) -> "_Place":
@@ -112,7 +118,7 @@ class _Place:
 
     def __getitem__(self, i) -> "_Place":
         if not isinstance(i, slice) or i.step not in (None, 1) or len(self.shape) != 1 or not i.stop:
-            raise Unplannable
+            raise Unplannable("an index")
         start = i.start or 0
         return _Place(self.device, i.stop - start, self.dtype, self.address + start * self.dtype.itemsize)
 
@@ -203,7 +209,7 @@ class Plan:
         for k, o in enumerate(outs):
             number = (o.address >> 48) - 1
             if number < n or o.address & _OFFSET or number in where:
-                raise Unplannable
+                raise Unplannable("an output that is no buffer of its own")
             where[number] = (n + 2 + k, 0)
             self.outs.append((o.shape, o.dtype))
         totals = [0, 0]
@@ -213,7 +219,7 @@ class Plan:
             self._put(where, number, n, rec.sizes, totals, 0)
         self.temporary, self.kept = totals
         if sum(totals) + sum(rec.sizes[k - n] for k, (b, _) in where.items() if b >= n + 2) > _MOST_BYTES:
-            raise Unplannable
+            raise Unplannable("more than _MOST_BYTES")
         words = list(rec.words)
         for at in rec.addresses:
             number = (words[at] >> 48) - 1
@@ -231,12 +237,12 @@ class Plan:
     @staticmethod
     def _put(where, number, n, sizes, totals, buffer) -> None:
         if number < n:
-            raise Unplannable  # an input is kept as it is
+            raise Unplannable("an input is kept")
         if number not in where:
             where[number] = (n + buffer, totals[buffer])
             totals[buffer] += (sizes[number - n] + _ALIGN - 1) // _ALIGN * _ALIGN
         elif where[number][0] != n + buffer and buffer == 1:
-            raise Unplannable  # an output is kept
+            raise Unplannable("an output is kept")
 
     def _rebase(self, tree, where):
         if isinstance(tree, _Place):
@@ -292,9 +298,12 @@ class Plan:
 
 
 class _NoPlan:
-    """Stands in the table for a sequence that cannot be recorded."""
+    """Stands in the table for a sequence that cannot be recorded, with the reason."""
 
     used = False
+
+    def __init__(self, reason: str):
+        self.reason = reason
 
 
 _plans: dict = {}
@@ -365,8 +374,11 @@ def call(fn: Callable, inputs: Sequence[Optional[torch.Tensor]], options: tuple,
             return None
         try:
             plan = Plan(fn, [(tuple(t.shape), t.dtype) if t is not None else None for t in inputs], inputs[0].device.index)
-        except Exception:  # (what it is that cannot be done on placeholders, or at all, the caller's own run says)
-            plan = _NoPlan()
+        except Unplannable as e:
+            plan = _NoPlan(str(e))
+        except Exception as e:  # of a call that the caller's own run refuses as well, or of this file
+            plan = _NoPlan(f"{type(e).__name__}: {e}")
+            _log.warning("%s: not recorded, its calls are made one by one (%s)", options[0], plan.reason)
         _remember(plans, key, plan)
     else:
         plan.used = True

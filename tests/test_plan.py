@@ -2,6 +2,9 @@
 
 import types
 
+import pytest
+import torch
+
 from olmo_core_amd.float8 import plan
 
 
@@ -23,3 +26,25 @@ def test_sizes_that_come_back_outlive_sizes_that_do_not():
     keys = list(table)
     plan._remember(table, "new", entry())
     assert list(table) == [*keys[-(most // 2):], "new"]
+
+
+@pytest.mark.parametrize("fail, reason, warned", [
+    (lambda p: p.float(), "tensor.float", False), (lambda p: p.to(torch.int32), "a conversion", False),
+    (lambda p: p.to(device="cpu", dtype=torch.bfloat16), "a conversion", False), (lambda p: p[::2], "an index", False),
+    (lambda p: {}["slot"], "KeyError: 'slot'", True), (lambda p: plan.ops.gemm_fp8(p, p, p, p), "TypeError: gemm_fp8: operands must be float8", True)])
+def test_what_cannot_be_recorded_says_why(monkeypatch, caplog, fail, reason, warned):
+    """A sequence that does what placeholders cannot has no plan and the reason; any other error is reported as well."""
+    monkeypatch.setattr(plan, "_plans", {})
+    monkeypatch.setattr(plan, "_seen", {})
+    monkeypatch.setattr(plan, "_plannable", lambda inputs: True)
+    x = torch.zeros(16, 16, dtype=torch.bfloat16)
+
+    def fn(p):
+        fail(p)
+        return [], None
+
+    for _ in range(6):
+        assert plan.call(fn, [x], ("a test",)) is None
+    (entry,) = plan._plans.values()
+    assert entry.reason.startswith(reason)
+    assert [r.levelname for r in caplog.records] == ["WARNING"] * warned
