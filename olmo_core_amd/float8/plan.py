@@ -8,8 +8,8 @@ type and a place in a buffer), notes the calls it makes, and from then on makes 
 buffer for everything temporary, one for what a backward takes, and the outputs.
 
 Nothing of an input is kept: a plan belongs to sizes and options, holds no address and no tensor, and is the same for
-every stream and thread.  Sizes are recorded when they are met for the second time, so that inputs whose sizes never come
-back cost a lookup.  us of a call among others, call by call / replayed: feed-forward block of 1999 tokens, 1024 / 2816, forward
+every stream and thread.  Sizes are recorded when they are met for the third time (``_RECORD_AT``): those that never come back
+cost a lookup, unless three or more layers of a model have them.  us of a call among others, call by call / replayed: feed-forward block of 1999 tokens, 1024 / 2816, forward
 and backward 391 / 194 (the GPU 182); four attention projections of 1537 tokens x 2048 535 / 306; generation of 23 tokens at
 4096 / 11008 69 / 55, of one token at 768 / 2048 40 / 27; 64 experts of 2048 x 1024, 48 tokens x top-8 92 / 70.
 """
@@ -37,6 +37,12 @@ _ALIGN = 256
 # they are used up than together at the end.
 _MOST_BYTES = 512 << 20
 _MOST_PLANS, _MOST_SEEN = 512, 4096
+
+# The time a set of sizes is met at which it is recorded.  Recording against what each later call saves, us: forward and
+# backward of a block of 1999 tokens, 1024 / 2816, 586 against 200; a linear of 100 tokens, 1024 x 1024, 103 against 19; a block
+# generating 23 tokens, 4096 / 11008, 163 against 28, one token, 768 / 2048, 90 against 8.  It pays after 3 to 11 more calls, so not
+# for sizes that two layers meet once in a forward of their own.
+_RECORD_AT = 3
 
 _QUERIES = {
     "mi8_gemm_splitk_suggest", "mi8_gemm_splitk_workspace_bytes", "mi8_gemm_fp8_batch_pays", "mi8_amax_slots_for",
@@ -367,11 +373,13 @@ def call(fn: Callable, inputs: Sequence[Optional[torch.Tensor]], options: tuple,
     plans = _plans if within is None else within.then
     plan = plans.get(key)
     if plan is None:
-        if within is None and key not in _seen:
-            if len(_seen) >= _MOST_SEEN:
-                _seen.clear()
-            _seen[key] = True
-            return None
+        if within is None:
+            met = _seen.get(key, 0) + 1
+            if met < _RECORD_AT:
+                if len(_seen) >= _MOST_SEEN:
+                    _seen.clear()
+                _seen[key] = met
+                return None
         try:
             plan = Plan(fn, [(tuple(t.shape), t.dtype) if t is not None else None for t in inputs], inputs[0].device.index)
         except Unplannable as e:

@@ -1,5 +1,5 @@
-"""Recorded sequences of launches (olmo_core_amd/float8/plan.py): a layer's third call on one set of sizes, which replays the
-plan recorded on the second, has the bits of the first, which made its calls one by one."""
+"""Recorded sequences of launches (olmo_core_amd/float8/plan.py): a layer's third call on one set of sizes, which records its
+plan and replays it, has the bits of the first, which made its calls one by one."""
 
 import pytest
 import torch

@@ -48,3 +48,17 @@ def test_what_cannot_be_recorded_says_why(monkeypatch, caplog, fail, reason, war
     (entry,) = plan._plans.values()
     assert entry.reason.startswith(reason)
     assert [r.levelname for r in caplog.records] == ["WARNING"] * warned
+
+
+def test_sizes_met_twice_are_not_recorded(monkeypatch):
+    """Two layers of one size, sequence lengths that come once: no recording, which costs more than a replay saves."""
+    monkeypatch.setattr(plan, "_plans", {})
+    monkeypatch.setattr(plan, "_seen", {})
+    monkeypatch.setattr(plan, "_plannable", lambda inputs: True)
+    recorded = []
+    for tokens in range(1, 9):
+        for _ in range(2):
+            plan.call(lambda p: recorded.append(tokens) or p.float(), [torch.zeros(tokens, 16)], ("a test",))
+    assert not recorded and not plan._plans
+    plan.call(lambda p: recorded.append(3) or p.float(), [torch.zeros(3, 16)], ("a test",))
+    assert recorded == [3] and len(plan._plans) == 1
