@@ -254,6 +254,8 @@ def _options(c: Float8LinearConfig) -> tuple:
 def _planned_forward(x2, weights, c: Float8LinearConfig, scales, w_ops, need_gx: bool, need_gw: bool):
     """:func:`_shared_input_forward` from a plan: ``(ys, kept, plan)`` or ``None``.  Only where all that the backward takes is
     quantised here."""
+    if need_gx and any(o is not None for o in w_ops):
+        return None
     n = len(weights)
 
     def recorded(px, *rest):

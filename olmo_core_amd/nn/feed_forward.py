@@ -199,8 +199,8 @@ def _mlp_backward(gy, saved, c, dims, dtypes, need):
 
 def _planned_forward(x, weights, c, need, ws, wo, keep: bool):
     """:func:`_mlp_forward` from a plan: ``([y], kept, plan)`` or ``None``."""
-    if STAGE_SINK is not None:
-        return None
+    if STAGE_SINK is not None or x.dtype != torch.bfloat16 or (keep and any(o is not None for o in wo)):
+        return None  # (a conversion of x, and kept weights among what the backward takes, are not recorded)
     pow2 = c.round_scales_to_power_of_2
     options = ("mlp", need, keep, pow2, c.cast_config_input.target_dtype, c.cast_config_weight.target_dtype,
                c.cast_config_grad_output.target_dtype, FUSE_SWIGLU_EPILOGUE, SWIGLU_AMAX_FROM_CODES)

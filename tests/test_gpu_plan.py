@@ -131,3 +131,18 @@ def test_replaced_operations_are_called(dev, runs, monkeypatch, name, tokens, ke
     monkeypatch.setattr(plan.ops, name, lambda *a, **k: called.append(1) or real(*a, **k))
     got = step()
     assert called and len(runs) == n and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("kept, autocast", [(True, False), (False, True)])
+def test_forms_without_a_plan_are_not_looked_up(dev, runs, kept, autocast):
+    """Training with kept float8 weights, and float32 activations under autocast, have no plans: no lookup, no attempt."""
+    model = nn.ModuleDict({"ff": FeedForward(d_model=256, hidden_size=512, bias=False, dtype=torch.bfloat16, init_device="cuda"),
+                           "q": nn.Linear(256, 256, bias=False, dtype=torch.bfloat16, device=dev),
+                           "k": nn.Linear(256, 256, bias=False, dtype=torch.bfloat16, device=dev)})
+    Float8Config(ao=AOFloat8LinearConfig.recommended() if kept else AOFloat8LinearConfig()).apply_float8_linear(_fill(model))
+    x = seeded((300, 256), 1).to(dev)
+    x, go = (x.float() if autocast else x), seeded((300, 256), 2, std=1e-3).to(dev)
+    fwd = lambda t: [model["ff"](t), *float8_projections(t, model["q"], model["k"])]  # noqa: E731
+    got = [_step(model, x, fwd, [go] * 3, autocast) for _ in range(4)]
+    assert not plan._seen and not plan._plans and not runs
+    assert all(torch.equal(a, b) for a, b in zip(got[0], got[3]))
