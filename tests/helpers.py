@@ -2,9 +2,12 @@
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
+from olmo_core_amd import _C
 from oracle import float8_oracle as O
 
 E4M3, E5M2 = torch.float8_e4m3fn, torch.float8_e5m2
@@ -91,3 +94,59 @@ def assert_bf16_pointwise_close(got, ref, what="", max_frac=1e-2, ulps=2):
         step = (gi - ri).abs()[diff]
         tiny = (r.float().abs()[diff] < 1e-30) & (g.float().abs()[diff] < 1e-30)
         assert bool(((step <= ulps) | tiny).all()), f"{what}: an element differs by more than {ulps} bf16 steps"
+
+
+class _Watched:
+    """A function of the library that tells what it is called with."""
+
+    def __init__(self, fn, tell):
+        self.fn, self.tell, self.argtypes = fn, tell, fn.argtypes
+
+    def __call__(self, *args):
+        self.tell(*args)
+        return self.fn(*args)
+
+
+def watch_casts(monkeypatch) -> list:
+    """``(address, rows, cols)`` of every tensor the library is asked to quantise from now on: cast alone, in a list, or by a
+    call that a plan replays (include/mi8.h: mi8_run_plan), which goes on being replayed."""
+    seen: list = []
+    alone = {"mi8_cast_tensorwise", "mi8_cast_rowwise", "mi8_cast_colwise_t"}
+    lists = {"mi8_cast_tensorwise_batch", "mi8_cast_rows_and_colwise_t_batch"}
+    real, loaded = _C.lib, _C.lib()
+    numbers = {loaded.mi8_plan_function(name.encode()): name for name in _C.EXPORTED_SYMBOLS}
+
+    def replayed(words, n_words, buffers, n_buffers, stream):
+        at = iter(words[:n_words])
+
+        def one(kind):
+            v = next(at)
+            if kind is not ctypes.c_void_p or v in (0, -1, -2):
+                return v
+            return buffers[(v >> 48) - 1] + (v & ((1 << 48) - 1))
+
+        for number in at:
+            name, args = numbers[number], []
+            for kind in _C._SIGNATURES[name][1]:
+                item = getattr(kind, "_type_", None)
+                if isinstance(item, type) and issubclass(item, ctypes.Structure):
+                    args.append([{f: one(k) for f, k in item._fields_} for _ in range(next(at))])
+                else:
+                    args.append(one(kind))
+            if name in alone:
+                seen.append((args[0], args[2], args[3]))
+            elif name in lists:
+                seen.extend((t["x"], t["rows"], t["cols"]) for t in args[0])
+
+    class Library:
+        def __getattr__(self, name):
+            fn = getattr(loaded, name)
+            if name in alone:
+                return _Watched(fn, lambda *a: seen.append((a[0], a[2], a[3])))
+            if name in lists:
+                return _Watched(fn, lambda items, *a: seen.extend((t.x, t.rows, t.cols) for t in items))
+            return _Watched(fn, replayed) if name == "mi8_run_plan" else fn
+
+    library = Library()
+    monkeypatch.setattr(_C, "lib", lambda: real() if getattr(_C._recording, "recorder", None) is not None else library)
+    return seen

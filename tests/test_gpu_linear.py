@@ -5,13 +5,13 @@ import pytest
 import torch
 import torch.nn as nn
 
-from helpers import E4M3, E5M2, assert_bytes_equal, assert_gemm_close, assert_scale_equal, seeded
+from helpers import E4M3, E5M2, assert_bytes_equal, assert_gemm_close, assert_scale_equal, seeded, watch_casts
 from oracle import float8_oracle as O
 
 pytestmark = pytest.mark.gpu
 
 from olmo_core_amd.float8 import AOFloat8LinearConfig, AOFloat8LinearRecipe, Float8Config  # noqa: E402
-from olmo_core_amd.float8 import ops  # noqa: E402
+from olmo_core_amd.float8 import ops, plan  # noqa: E402
 from olmo_core_amd.float8.linear import Float8Linear, convert_to_float8_training  # noqa: E402
 from olmo_core_amd.float8.native_config import Float8LinearConfig  # noqa: E402
 
@@ -310,15 +310,8 @@ def test_kept_weight_operands(dev, monkeypatch):
     assert all(m.weight_operands() is None for m in plain.modules() if isinstance(m, Float8Linear))
 
     weight_ptrs = {m.weight.data_ptr() for m in kept.modules() if isinstance(m, Float8Linear)}
-    casts = []
-    real_cast = ops.cast_tensorwise
-
-    def counting_cast(x, *a, **k):
-        if x.data_ptr() in weight_ptrs:
-            casts.append(x.data_ptr())
-        return real_cast(x, *a, **k)
-
-    monkeypatch.setattr(ops, "cast_tensorwise", counting_cast)
+    quantised = watch_casts(monkeypatch)
+    weight_casts = lambda: sum(at in weight_ptrs for at, _, _ in quantised)  # noqa: E731
 
     def step(model, x):
         xg = x.clone().requires_grad_(True)
@@ -331,7 +324,7 @@ def test_kept_weight_operands(dev, monkeypatch):
         y0, g0 = step(plain, x)
         y1, g1 = step(kept, x)
         assert torch.equal(y0, y1) and torch.equal(g0, g1), i
-        assert len(casts) == 4, (i, len(casts))  # w1, w2, w3, proj: once each, in the first micro-batch only
+        assert weight_casts() == 4, (i, weight_casts())  # w1, w2, w3, proj: once each, in the first micro-batch only
     for (n0, p0), (n1, p1) in zip(plain.named_parameters(), kept.named_parameters()):
         assert n0 == n1 and torch.equal(p0.grad, p1.grad), n0
 
@@ -346,13 +339,15 @@ def test_kept_weight_operands(dev, monkeypatch):
         y0, g0 = step(plain, x)
         y1, g1 = step(kept, x)
         assert torch.equal(y0, y1) and torch.equal(g0, g1)
-    assert len(casts) == 8
+    assert weight_casts() == 8
 
     # generation-style use: no gradients, frozen weights, nothing is quantised again
+    monkeypatch.setattr(plan, "_plans", {})
     with torch.no_grad():
-        for x in xs:
+        for x in xs * 2:
             assert torch.equal(kept["proj"](kept["ff"](x)), plain["proj"](plain["ff"](x)))
-    assert len(casts) == 8
+    assert [type(p) for key, p in plan._plans.items() if key[0][0] == "mlp"] == [plan.Plan] * 2
+    assert weight_casts() == 8  # (nor by a call that a plan replays)
 
 
 
@@ -380,26 +375,18 @@ def test_projections_of_one_input(dev, recipe, shape, monkeypatch):
     M, K, ns = shape
     mods = _projection_modules(dev, recipe, K, ns, bias_on=(1,))
     gos = [seeded((2, M // 2, N), 50 + i, std=1e-3).to(dev) for i, N in enumerate(ns)]
-    calls = {"n": 0}
-    for name in ("cast_tensorwise", "cast_rows_and_colwise_t", "cast_rowwise"):
-        orig = getattr(ops, name)
-
-        def counted(t, *a, _orig=orig, **k):
-            if t.shape == (M, K):
-                calls["n"] += 1
-            return _orig(t, *a, **k)
-
-        monkeypatch.setattr(ops, name, counted)
+    quantised = watch_casts(monkeypatch)
+    input_casts = lambda: sum((rows, cols) == (M, K) for _, rows, cols in quantised)  # noqa: E731
 
     def run(fused, used=(0, 1, 2)):
-        calls["n"] = 0
+        quantised.clear()
         x = seeded((2, M // 2, K), 7).to(dev).requires_grad_(True)
         for m in mods:
             m.weight.grad = None
             if m.bias is not None:
                 m.bias.grad = None
         ys = float8_projections(x, *mods) if fused else tuple(m(x) for m in mods)
-        n_fwd = calls["n"]
+        n_fwd = input_casts()
         torch.autograd.backward([ys[i] for i in used], [gos[i] for i in used])
         grads = [None if m.weight.grad is None else m.weight.grad.clone() for m in mods]
         return n_fwd, ys, x.grad, grads, mods[1].bias.grad
@@ -415,9 +402,9 @@ def test_projections_of_one_input(dev, recipe, shape, monkeypatch):
     # no gradients: same outputs, one cast; frozen weights: only grad_x
     with torch.no_grad():
         xs = seeded((M, K), 11).to(dev)
-        calls["n"] = 0
+        quantised.clear()
         outs = float8_projections(xs, *mods)
-        assert calls["n"] == 1
+        assert input_casts() == 1
         for o, m in zip(outs, mods):
             assert torch.equal(o, m(xs))
     for m in mods:

@@ -4,7 +4,7 @@ bits), both vs the oracle's composition (tolerance), and the fused amax against 
 import pytest
 import torch
 
-from helpers import E4M3, E5M2, assert_gemm_close, assert_scale_equal, gemm_errors, seeded
+from helpers import E4M3, E5M2, assert_gemm_close, assert_scale_equal, gemm_errors, seeded, watch_casts
 from oracle import float8_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -268,15 +268,8 @@ def test_compiled_modules_use_their_kept_weights(dev, monkeypatch):
                            "proj": nn.Linear(D, 256, bias=True, dtype=torch.bfloat16)}).to(dev)
     Float8Config(ao=AOFloat8LinearConfig.recommended()).apply_float8_linear(model)
     weight_shapes = {(H, D), (D, H), (256, D)}
-    casts = []
-    orig = ops.cast_tensorwise
-
-    def counted(t, *a, **k):
-        if tuple(t.shape) in weight_shapes:
-            casts.append(tuple(t.shape))
-        return orig(t, *a, **k)
-
-    monkeypatch.setattr(ops, "cast_tensorwise", counted)
+    quantised = watch_casts(monkeypatch)
+    weight_casts = lambda: sum((rows, cols) in weight_shapes for _, rows, cols in quantised)  # noqa: E731
 
     def fwd(m, x):
         return m["proj"](m["ff"](x))
@@ -290,19 +283,19 @@ def test_compiled_modules_use_their_kept_weights(dev, monkeypatch):
         y = compiled(xd)
         y.backward(go)
         outs.append((y, xd.grad))
-    assert len(casts) == 4, casts  # w1, w2, w3 and the projection, once each for the three micro-batches
+    assert weight_casts() == 4, quantised  # w1, w2, w3 and the projection, once each for the three micro-batches
     model.zero_grad()
     for x, (y1, g1) in zip(xs, outs):
         xd = x.clone().requires_grad_(True)
         y0 = fwd(model, xd)
         y0.backward(go)
         assert torch.equal(y0, y1) and torch.equal(xd.grad, g1)
-    assert len(casts) == 4
+    assert weight_casts() == 4
     with torch.no_grad():  # a weight update is seen: the copies are made again
         for p in model.parameters():
             p.mul_(1.5)
     y = compiled(xs[0])
-    assert len(casts) == 8 and torch.equal(y, fwd(model, xs[0]))
+    assert weight_casts() == 8 and torch.equal(y, fwd(model, xs[0]))
 
 
 @pytest.mark.parametrize("kept", [True, False], ids=["kept_weights", "plain"])
