@@ -361,6 +361,13 @@ def _shared_input_forward(x2, weights, c: Float8LinearConfig, scales, w_ops, nee
     return ys, x_saved, [kept for _, _, kept in ws]
 
 
+# Elements of the grad_outputs of linears of one input up to which they are quantised, and their products handed over, together:
+# all of their float8 copies, two bytes an element, are held until then.  Beyond, one linear after the other.  Forward and backward
+# of three projections with scales per row, together / one by one: 16384 x 4096 2046 / 2068 us, the backward's own peak 608 / 352 MiB,
+# 16384 x 2048 834 / 843 us, 312 / 184 MiB; with one scale 2000 / 1999 and 805 / 800 us.
+_MOST_TOGETHER = 256 << 20
+
+
 class _Float8SharedInputMatmul(torch.autograd.Function):
     """``ys[i] = x @ W_i^T`` for several weights applied to ONE input (the q, k and v projections of an attention
     block, reference src/olmo_core/nn/attention/__init__.py:582): x is quantised once by construction, one copy of
@@ -426,9 +433,10 @@ class _Float8SharedInputMatmul(torch.autograd.Function):
         gos = [None if go is None else go.reshape(ctx.M, ctx.ns[i]) for i, go in enumerate(gos)]
         gos = [go if go is None or go.dtype == ctx.x_dtype else go.to(ctx.x_dtype) for go in gos]
         c = ctx.config
-        made = _grad_operands(gos, c, need_gx, ctx.need_gws)
         order = [i for i in reversed(range(n)) if gos[i] is not None]
-        if (order and chain and not _is_disabled(c.cast_config_grad_output)
+        together = sum(gos[i].numel() for i in order) <= _MOST_TOGETHER
+        made = _grad_operands(gos, c, need_gx, ctx.need_gws) if together else [None] * n
+        if (order and together and chain and not _is_disabled(c.cast_config_grad_output)
                 and not _is_disabled(c.cast_config_grad_output_for_grad_weight)):
             products = [_grad_input_product(gos[i], c, ctx.ns[i], made[i][0], w_parts[i], ctx.w_is_q[i], add=i != order[0])
                         for i in order if need_gx]

@@ -419,6 +419,35 @@ def test_projections_of_one_input(dev, recipe, shape, monkeypatch):
     assert torch.equal(outs[0], mods[0](xs)) and torch.equal(outs[1], plain(xs))
 
 
+@pytest.mark.parametrize("recipe", RECIPES)
+def test_large_projections_go_backward_one_by_one(dev, recipe, monkeypatch):
+    """Above a number of elements the grad_outputs are quantised one after the other: the same bits, one float8 pair held."""
+    from olmo_core_amd.float8 import linear
+
+    M, K = 4096, 1024
+    mods = _projection_modules(dev, recipe, K, (K,) * 4)
+    x, gos = seeded((M, K), 1).to(dev), [seeded((M, K), 2 + i, std=1e-3).to(dev) for i in range(4)]
+    monkeypatch.setattr(plan, "call", lambda *a, **k: None)
+
+    def run(most):
+        monkeypatch.setattr(linear, "_MOST_TOGETHER", most)
+        for m in mods:
+            m.weight.grad = None
+        xd = x.clone().requires_grad_(True)
+        ys = linear.float8_projections(xd, *mods)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        torch.autograd.backward(ys, gos)
+        return [xd.grad, *(m.weight.grad for m in mods)], torch.cuda.max_memory_allocated() - before
+
+    run(4 * M * K)
+    (a, held), (b, less) = run(4 * M * K), run(4 * M * K - 1)
+    assert all(torch.equal(p, q) for p, q in zip(a, b))
+    if recipe != "rowwise_with_gw_hp":  # (its grad_outputs are quantised for one product only, never together)
+        assert held - less >= 2 * (2 * M * K)  # two pairs and more
+
+
 @pytest.mark.parametrize("recipe", ["tensorwise", "rowwise"])
 def test_projections_under_autocast(dev, recipe):
     """Float32 activations under autocast: every module converts its own input, so autograd adds the three grad_input
