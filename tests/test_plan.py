@@ -31,6 +31,7 @@ def test_sizes_that_come_back_outlive_sizes_that_do_not():
 @pytest.mark.parametrize("fail, reason, warned", [
     (lambda p: p.float(), "tensor.float", False), (lambda p: p.to(torch.int32), "a conversion", False),
     (lambda p: p.to(device="cpu", dtype=torch.bfloat16), "a conversion", False), (lambda p: p[::2], "an index", False),
+    (lambda p: p.device.place((plan._MOST_BYTES + 1,), torch.uint8), "more than _MOST_BYTES", False),
     (lambda p: {}["slot"], "KeyError: 'slot'", True), (lambda p: plan.ops.gemm_fp8(p, p, p, p), "TypeError: gemm_fp8: operands must be float8", True)])
 def test_what_cannot_be_recorded_says_why(monkeypatch, caplog, fail, reason, warned):
     """A sequence that does what placeholders cannot has no plan and the reason; any other error is reported as well."""
