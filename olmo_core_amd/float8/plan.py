@@ -38,7 +38,7 @@ _ALIGN = 256
 # MiB: 121 + 99 386 / 267, 136 / 150; 169 + 137 395 / 349, 194 / 218; 225 + 181 432 / 434, 264 / 292; 238 + 207 440 / 442,
 # 211 / 242; 308 + 262 608 / 597, 292 / 339; 385 + 321 711 / 705, 378 / 444; 322 + 390 626 / 631, 404 / 556; 463 + 420 984 / 985.
 # Of three projections 154 + 155 467 / 422, 228 + 227 594 / 597, 352 + 352 1052 / 1049.
-_MOST_BYTES = 256 << 20
+_MOST_BYTES = 320 << 20
 _MOST_PLANS, _MOST_SEEN = 512, 4096
 
 # The time a set of sizes is met at which it is recorded.  Recording against what each later call saves, us: forward and
