@@ -142,7 +142,7 @@ int mi8_cast_tensorwise_batch(const mi8_cast_item* items, int32_t count, int fp8
 /* A scale per row with a row-major copy, and a scale per column with a transposed copy, of up to MI8_CAST_BATCH tensors:
  * per tensor the results of mi8_cast_rowwise and mi8_cast_colwise_t, two launches for all of them.
  *   out_rows: fp8 [rows, ld_rows]; row_scale: float32 [rows]; out_t: fp8 [cols, ld_t], ld_t >= round_up(rows, 128), zero
- *   from column `rows` to ld_t; col_scale: float32 [cols]; workspace: uint32 [mi8_two_cast_workspace_words(rows, cols)],
+ *   from column `rows` to round_up(rows, 128) and not written beyond; col_scale: float32 [cols]; workspace: uint32 [mi8_two_cast_workspace_words(rows, cols)],
  *   16-byte aligned, contents on entry unimportant.  group_rows (0: rows): every group_rows rows, a multiple of 128 that
  *   divides rows, have column scales of their own, col_scale [rows / group_rows, cols] (the weights of experts). */
 typedef struct {

@@ -388,3 +388,24 @@ def test_every_bf16_value_saturates_and_keeps_nan(dev, fp8, scale):
     assert torch.equal(q_t.cpu().float().nan_to_num(0.3)[:, :512], want.float().t().nan_to_num(0.3))
     nan = want.float().isnan()
     assert torch.equal(q.cpu().view(torch.uint8)[~nan], want.view(torch.uint8)[~nan])  # (the sign of zero too)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows, group_rows", [(1, 0), (128, 0), (300, 0), (512, 256)])
+def test_two_scale_cast_into_a_wider_pitch(dev, rows, group_rows):
+    """out_t rows that are further apart than the rows rounded up to 128: zeros up to there, the bytes beyond are the caller's."""
+    cols, end = 144, ops.pad128(rows)
+    ld_t = end + 48
+    x = torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows)).bfloat16().to(dev)
+    (want_q, want_rs, want_t, want_cs), = ops.cast_rows_and_colwise_t_batch([x], torch.float8_e4m3fn, groups=rows // group_rows if group_rows else 1)
+    q = torch.full((rows, cols + 32), 0x55, dtype=torch.uint8, device=dev)
+    q_t = torch.full((cols, ld_t), 0x55, dtype=torch.uint8, device=dev)
+    rs, cs = torch.empty_like(want_rs), torch.empty_like(want_cs)
+    L = ops._C.lib()
+    ws = torch.empty(L.mi8_two_cast_workspace_words(rows, cols), dtype=torch.int32, device=dev)
+    item = (ops._C.TwoCastItem * 1)(ops._C.TwoCastItem(x.data_ptr(), rows, cols, q.data_ptr(), cols + 32, rs.data_ptr(), q_t.data_ptr(), ld_t,
+                                                       cs.data_ptr(), ws.data_ptr(), group_rows, ops._C.MI8_BF16))
+    ops._C.check(L.mi8_cast_rows_and_colwise_t_batch(item, 1, ops._C.MI8_E4M3, 0, ops._stream(x)), "mi8_cast_rows_and_colwise_t_batch")
+    assert torch.equal(q[:, :cols], want_q.view(torch.uint8)) and bool((q[:, cols:] == 0x55).all())
+    assert torch.equal(q_t[:, :end], want_t.view(torch.uint8)) and bool((q_t[:, end:] == 0x55).all())
+    assert not q_t[:, rows:end].any() and torch.equal(rs, want_rs) and torch.equal(cs, want_cs)
