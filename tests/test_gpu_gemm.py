@@ -596,7 +596,7 @@ def test_slices_of_k_without_planes(dev, mnk, splits, dt):
 @pytest.mark.parametrize("vec", [False, True])
 def test_products_in_one_launch(dev, dt, vec):
     """Products launched together have the bits of a launch each: one tile and many, ragged edges and K, a product that is
-    cut along K among whole ones, up to 64 rows, a chain of three that add up, and the longest list a launch takes."""
+    cut along K among whole ones and in a sum, up to 64 rows, a chain of three that add up, and the longest list a launch takes."""
     g = torch.Generator(device=dev).manual_seed(int(vec))
 
     def operands(M, N, K):
@@ -609,10 +609,12 @@ def test_products_in_one_launch(dev, dt, vec):
         [((300, 272, 144), False), ((129, 520, 1040), False)],
         [((777, 1040, 528), False), ((777, 1040, 2064), True), ((777, 1040, 16), True), ((1040, 528, 784), False)],
         [((40, 1024, 2816), False), ((40, 1024, 784), True), ((2000, 264, 272), False)],
-        [((100, 200, 1040), False), ((1000, 1000, 1024), False), ((100, 200, 2048), True)][:2] + [((65, 300, 128), False)],
+        [((100, 200, 1040), False), ((1000, 1000, 1024), False), ((65, 300, 128), False)],
+        [((100, 200, 1040), False), ((100, 200, 2048), True), ((100, 200, 128), True), ((1000, 1000, 1024), False)],
         [((64, 64, 128), False)] * 8,
     ]
-    assert ops._C.lib().mi8_gemm_splitk_suggest(100, 200, 1040) > 1 and ops._C.lib().mi8_gemm_splitk_suggest(777, 1040, 2064) >= 1
+    cut = [ops._C.lib().mi8_gemm_splitk_suggest(100, 200, k) for k in (1040, 2048, 128)]
+    assert cut[0] != cut[1] and min(cut[:2]) > 1 and cut[2] == 1  # (terms of one sum, cut along K in two ways and not at all)
     for shapes in lists:
         products = [(*operands(*mnk), None, add) for mnk, add in shapes]
         apart = ops.gemm_fp8_batch(products, out_dtype=dt, together=False)
