@@ -242,7 +242,5 @@ __device__ __forceinline__ void tile_quantise(const Values& values, int64_t row_
     }
 }
 
-// Both: rows [row0, row0 + 128) of x (rows >= row_end read as zero and produce zero bytes), columns [col0, col0 + 128).
-
 }  // namespace
 }  // namespace mi8

@@ -180,7 +180,6 @@ __device__ __forceinline__ void transpose4x4_bytes(uint32_t r0, uint32_t r1, uin
     c3 = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
 }
 
-// Eight consecutive high-precision elements starting at a 16-byte aligned address -> float[8]
 // Streaming accesses (the nt bit): for data a kernel reads for the last time, or writes for a later kernel to read.
 // Such lines take no space from data that is about to be read again - in a two-pass cast the second pass's
 // outputs otherwise evict what the first pass left of the input in the memory-side cache (16384 x 11008: amax + cast
@@ -201,6 +200,7 @@ __device__ __forceinline__ void store_stream8(void* p, uint32_t lo, uint32_t hi)
     __builtin_nontemporal_store((u32x2_t){lo, hi}, reinterpret_cast<u32x2_t*>(p));
 }
 
+// Eight consecutive high-precision elements starting at a 16-byte aligned address -> float[8]
 template <int HP>
 struct HpVec;
 template <>

@@ -305,7 +305,7 @@ __global__ __launch_bounds__(kFewThreads, WHOLE ? (U > 8 ? 2 : 4) : MT == 1 ? 6 
     load_x(x, s_begin);
     if constexpr (WHOLE) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {  // (steps past the share multiply zeros)
+        for (int u = 0; u < U; ++u) {
             if (s_begin + u >= s_end) break;
             load_x(u & 1 ? x : x_next, s_begin + u + 1);
             step(u & 1 ? x_next[0] : x[0], w[u]);
@@ -403,6 +403,8 @@ namespace {
 // kernel above reads it from L2 for every 16: more rows, or more bytes of weights, make that the time.  us, above / ring:
 // 16 x 8192 x 2048 9.9 / 9.0, 23 x 11008 x 4096 28.5 / 25.3, 48 x 11008 x 4096 43.6 / 27.1, 64 x 8192 x 2048 18.5 / 9.3,
 // 4 x 27648 x 5120 66.6 / 56.6, 64 x 27648 x 5120 135 / 70; 8 x 11008 x 4096 24.3 / 24.2, 32 x 2816 x 1024 5.6 / 5.8.
+// The line at 200 MB for four rows, below it 20480 x 4096 36.0 / 37.2, 32768 x 2048 28.3 / 30.0, 12288 x 8192 41.1 / 40.2, above
+// 20480 x 5120 49.4 / 43.1, 27648 x 4096 46.6 / 45.3, 24576 x 6144 62.5 / 53.5, 22016 x 8192 72.1 / 67.5, 28672 x 8192 86.2 / 85.9.
 // Ring tiles address the rows of a tile, all of A and 32 of each matrix, with 32-bit offsets; the kernel above with 64-bit ones.
 bool dual_on_ring(int64_t M, int64_t H, int64_t K, int64_t lda, int64_t ldb)
 {
@@ -455,7 +457,7 @@ extern "C" int mi8_few_rows_swiglu(const void* x, int x_is_fp8, int64_t lda, con
     }
     if (M <= 16) return launch_few_rows<1, 1, kFp8, true>(a, st, "mi8_few_rows_swiglu");
     if (M <= 32) return launch_few_rows<2, 1, kFp8, true>(a, st, "mi8_few_rows_swiglu");
-    return launch_few_rows<4, 1, kFp8, true>(a, st, "mi8_few_rows_swiglu");
+    return launch_few_rows<4, 1, kFp8, true>(a, st, "mi8_few_rows_swiglu");  // (rows too far apart for ring tiles)
 }
 
 extern "C" int mi8_few_rows_cast_gemm(const void* x, int64_t lda, const uint32_t* slots, int32_t n_slots, const void* b,

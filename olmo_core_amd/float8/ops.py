@@ -97,7 +97,9 @@ AMAX_BATCH = 8
 
 def amax_partials_batch(tensors) -> list:
     """:func:`amax_partials` of up to ``AMAX_BATCH`` contiguous GPU tensors of one dtype in one launch: a list of
-    ``(slots, n_used)`` in the order given (same values as separate calls)."""
+    ``(slots, n_used)`` in the order given (same values as separate calls).  For callers that take the maxima ahead of their
+    casts (``cast_tensorwise(..., slots=)``); the layers' casts of several tensors take them in the launch of
+    :func:`cast_tensorwise_batch`."""
     n = len(tensors)
     if not 0 < n <= AMAX_BATCH:
         raise ValueError(f"amax_partials_batch: {n} tensors (1..{AMAX_BATCH})")
