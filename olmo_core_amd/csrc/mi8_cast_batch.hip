@@ -176,7 +176,9 @@ __device__ __forceinline__ void two_amax_body(const TwoCastItem& t, int block, u
 #pragma unroll
         for (int k = 0; k < 4; ++k) acc[v][k] = 0;
     uint32_t* const row_out = t.row_part + (int64_t)ct * t.tiles_m * kTile;
-    const int last = (chunk + 1) * t.chunk_tiles < t.tiles_m ? (chunk + 1) * t.chunk_tiles : t.tiles_m;
+    const int group = chunk / t.group_chunks;
+    const int first = group * t.group_tiles + (chunk - group * t.group_chunks) * t.chunk_tiles, end = (group + 1) * t.group_tiles;
+    const int last = first + t.chunk_tiles < end ? first + t.chunk_tiles : end;
     // half a tile of rows in flight while the half before it is folded
     constexpr int kHalf = kTile / 32;
     uint4 v[2][kHalf][NV];
@@ -205,9 +207,9 @@ __device__ __forceinline__ void two_amax_body(const TwoCastItem& t, int block, u
             if (cl == 0) row_out[row0 + 16 * i] = m;  // (the table has whole tiles of rows)
         }
     };
-    int64_t row0 = (int64_t)chunk * t.chunk_tiles * kTile + rg;
+    int64_t row0 = (int64_t)first * kTile + rg;
     load_half(v[0], row0);
-    for (int rt = chunk * t.chunk_tiles; rt < last; ++rt, row0 += kTile) {
+    for (int rt = first; rt < last; ++rt, row0 += kTile) {
         load_half(v[1], row0 + kTile / 2);
         fold_half(v[0], row0);
         if (rt + 1 < last) load_half(v[0], row0 + kTile);
@@ -309,15 +311,10 @@ __global__ __launch_bounds__(kThreads) void two_cast_items_kernel(TwoCastItems a
 
 bool valid_hp(int v) { return v == MI8_BF16 || v == MI8_F32; }
 
-// row tiles per chunk of the column partials: at most 32 chunks to fold (16384 x 4096: 75 us; 64 chunks 76.6, 16 chunks 88); of a
-// group of rows a divisor of its tiles, so that a chunk has rows of one group only
-int chunk_tiles_for(int64_t tiles_m) { return (int)ceil_div(tiles_m, 32); }
-int chunk_tiles_of_group(int64_t tiles)
-{
-    int c = 1;
-    while (tiles % c || tiles / c > 32) ++c;
-    return c;
-}
+// row tiles per chunk of the column partials: at most 32 chunks of a group of rows (or of all) to fold (16384 x 4096: 75 us; 64 chunks
+// 76.6, 16 chunks 88); the last chunk of a group is shorter, so that a chunk has rows of one group only
+// (three weights of 8 x 5504 x 1024, 43 tiles a group: 165 us, in chunks that divide a group - here all of it - 239)
+int chunk_tiles_for(int64_t group_tiles) { return (int)ceil_div(group_tiles, 32); }
 
 template <typename Kernel, typename Args>
 int launch_items(Kernel kern, const Args& a, int64_t blocks, hipStream_t st, const char* what)
@@ -444,12 +441,12 @@ extern "C" int mi8_cast_rows_and_colwise_t_batch(const mi8_two_cast_item* items,
         const mi8_two_cast_item& t = items[i];
         const int64_t tiles_m = ceil_div(t.rows, kTile), tiles_n = ceil_div(t.cols, kTile);
         const int64_t group_tiles = t.group_rows ? t.group_rows / kTile : tiles_m;  // (of the rows that share column scales)
-        const int chunk = t.group_rows ? chunk_tiles_of_group(group_tiles) : chunk_tiles_for(tiles_m);
-        const int64_t chunks = ceil_div(tiles_m, chunk);
+        const int chunk = chunk_tiles_for(group_tiles);
+        const int64_t group_chunks = ceil_div(group_tiles, chunk), chunks = tiles_m / group_tiles * group_chunks;
         MI8_REQUIRE(blocks + tiles_m * tiles_n < ((int64_t)1 << 31), MI8_ERR_UNSUPPORTED, "%s: grid too large", what);
         a.t[i] = TwoCastItem{t.x, t.rows, t.cols, (uint8_t*)t.out_rows, t.ld_rows, t.row_scale, (uint8_t*)t.out_t, t.ld_t, t.col_scale,
                              t.workspace, t.workspace + chunks * tiles_n * kTile, t.hp_dtype == MI8_F32, (int)tiles_m, (int)tiles_n,
-                             chunk, (int)group_tiles, (int)ceil_div(group_tiles, chunk), (int)blocks, (int)chunk_blocks};
+                             chunk, (int)group_tiles, (int)group_chunks, (int)blocks, (int)chunk_blocks};
         blocks += tiles_m * tiles_n;
         chunk_blocks += chunks * tiles_n;
     }

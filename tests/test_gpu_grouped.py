@@ -592,10 +592,11 @@ def test_grouped_gemm_takes_a_wide_pitch(dev, sizes):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("E, H, D", [(2, 128, 16), (5, 256, 144), (3, 1408, 1040), (2, 4224, 272)])
+@pytest.mark.parametrize("E, H, D", [(2, 128, 16), (5, 256, 144), (3, 1408, 1040), (2, 4224, 272), (3, 4736, 144), (2, 8320, 16), (2, 16256, 16)])
 def test_experts_weights_cast_together(dev, E, H, D):
     """Weights of equal groups of rows, cast together, have the bytes and scales of the ragged grouped cast: one row tile a group
-    and several, groups of more row tiles (33) than partial maxima are kept of, tensors of one type and of both."""
+    and several, groups of more row tiles than partial maxima are kept of (33, 37, 65, 127: chunks of two, three and four, the last
+    of a group shorter), tensors of one type and of both."""
     ws = [seeded((E * H, D), 3 + i).to(dev) for i in range(2)] + [seeded((E * H, D), 9).to(dev).float()]
     ws[0][H:].mul_(3.0)
     ws[1][5, 7] = 0.0
