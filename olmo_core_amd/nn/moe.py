@@ -39,12 +39,13 @@ def _cast_weights(ws, E: int, H: int, pow2: bool) -> list:
     """Both float8 copies of the experts' weights ``[E * H, D]``: per weight ``(q, row_scale, q_t, col_scale [E, D])``, expert e's
     columns of ``q_t`` from ``e * round_up(H, 128)`` on.
 
-    Together in two launches up to half a GB, where the launches and the clearing of every weight's amax show: three bf16 weights
-    of 8 x 1024 x 1024 take 37.5 us against 65.5 one by one, 8 x 1792 x 1024 57 against 72, 32 x 512 x 1024 61 against 77,
-    64 x 1024 x 1024 (402 MB) 216 against 241.  Beyond, both are at the memory's rate (64 x 1024 x 2048, 805 MB: 474 against 468;
-    8 x 4096 x 4096: 464 against 463).
+    Together in two launches up to 192 MiB, where the launches and the clearing of every weight's amax show; beyond, the second
+    pass over one weight finds more of it in the memory-side cache when no other weight was read in between.  us for three
+    bf16 weights, together / one by one: 8 x 1024 x 1024 37 / 65, 8 x 1792 x 1024 54 / 65, 8 x 8192 x 512 108 / 117,
+    8 x 1024 x 4096 (192 MiB) 112 / 120, 2 x 2048 x 8192 (192) 119 / 117; 8 x 2816 x 2048 (264) 173 / 164, 32 x 1024 x 2048 (384)
+    237 / 225, 2 x 14336 x 2048 (336) 219 / 192, 64 x 1024 x 1024 (384) 219 / 225.
     """
-    together = sum(w.numel() * w.element_size() for w in ws) <= 512 << 20
+    together = sum(w.numel() * w.element_size() for w in ws) <= 192 << 20
     if together and H % 128 == 0 and E > 1 and all(w.dtype in (torch.bfloat16, torch.float32) for w in ws):
         return ops.cast_rows_and_colwise_t_batch(ws, _E4M3, pow2=pow2, groups=E)
     equal = torch.full((E,), H, dtype=torch.int64, device=ws[0].device)  # the weights as equal-size groups
