@@ -366,10 +366,13 @@ def call(fn: Callable, inputs: Sequence[Optional[torch.Tensor]], options: tuple,
     re-run that saves other tensors than the first run did."""
     if (within is None and _saved_tensor_hooks(True) is not None) or _observed() or not _plannable(inputs[:-own] if own else inputs):
         return None
-    key = [options, inputs[0].device.index]
+    index = inputs[0].get_device()
+    key = [options, index]
     for t in inputs:
         if t is None:
             key.append(None)
+        elif t.get_device() != index:
+            return None  # (a plan launches on one GPU; the calls one by one refuse what they quantise together)
         else:
             key += (t.shape, t.dtype)
     key = tuple(key)
@@ -384,7 +387,7 @@ def call(fn: Callable, inputs: Sequence[Optional[torch.Tensor]], options: tuple,
                 _seen[key] = met
                 return None
         try:
-            plan = Plan(fn, [(tuple(t.shape), t.dtype) if t is not None else None for t in inputs], inputs[0].device.index)
+            plan = Plan(fn, [(tuple(t.shape), t.dtype) if t is not None else None for t in inputs], index)
         except Unplannable as e:
             plan = _NoPlan(str(e))
         except Exception as e:  # of a call that the caller's own run refuses as well, or of this file

@@ -63,3 +63,22 @@ def test_sizes_met_twice_are_not_recorded(monkeypatch):
     assert not recorded and not plan._plans
     plan.call(lambda p: recorded.append(3) or p.float(), [torch.zeros(3, 16)], ("a test",))
     assert recorded == [3] and len(plan._plans) == 1
+
+
+def test_inputs_on_two_gpus_have_no_plan(monkeypatch):
+    """A recorded sequence has one stream and takes no look at devices: an input that lives on another GPU goes to the calls one by
+    one, which refuse it where they quantise it, however often its sizes were met and also where the sizes have a plan."""
+    monkeypatch.setattr(plan, "_plans", {})
+    monkeypatch.setattr(plan, "_seen", {})
+    monkeypatch.setattr(plan, "_plannable", lambda inputs: True)
+    monkeypatch.setattr(plan, "Plan", lambda *a: types.SimpleNamespace(run=lambda inputs: ([], None), used=False))
+    on = lambda index: types.SimpleNamespace(shape=(16, 16), dtype=torch.bfloat16, get_device=lambda: index,  # noqa: E731
+                                             device=types.SimpleNamespace(index=index))
+    for own in (0, 1):
+        for _ in range(4):
+            assert plan.call(None, [on(0), None, on(1)], ("a test",), own=own) is None
+        assert not plan._plans
+    for _ in range(2):
+        assert plan.call(None, [on(0), None, on(0)], ("a test",)) is None
+    assert plan.call(None, [on(0), None, on(0)], ("a test",)) is not None
+    assert plan.call(None, [on(0), None, on(1)], ("a test",)) is None
