@@ -33,12 +33,12 @@ _OFFSET = (1 << 48) - 1
 _STREAM, _IGNORED = -1, -2
 _ALIGN = 256
 
-# Sizes above which a sequence is not planned: its launches are long enough, and its temporaries are better given back as
-# they are used up than together at the end.  Forward and backward of a block, MiB of the two plans, us call by call / replayed, peak
-# MiB: 121 + 99 386 / 267, 136 / 150; 169 + 137 395 / 349, 194 / 218; 225 + 181 432 / 434, 264 / 292; 238 + 207 440 / 442,
-# 211 / 242; 308 + 262 608 / 597, 292 / 339; 385 + 321 711 / 705, 378 / 444; 322 + 390 626 / 631, 404 / 556; 463 + 420 984 / 985.
-# Of three projections 154 + 155 467 / 422, 228 + 227 594 / 597, 352 + 352 1052 / 1049.
-_MOST_BYTES = 320 << 20
+# Sizes above which a sequence is not planned: its launches are long enough, and a buffer for all temporaries holds more than
+# they do one by one.  Forward and backward of a block, MiB of the two plans, us call by call / replayed, peak MiB: 67 + 57 418 / 202,
+# 68 / 78; 121 + 99 419 / 273, 130 / 150; 221 + 178 464 / 468, 260 / 286; 322 + 233 652 / 650, 404 / 399; 385 + 417 (float32 weights)
+# 805 / 802 (on other boxes 771 / 759, 786 / 777), 378 / 444; 434 + 313 837 / 834, 532 / 542; 463 + 420 1008 / 1010, 365 / 408; 520 + 426
+# 1055 / 1056, 539 / 626.  Of three projections 154 + 155 484 / 432, 220 / 223; 283 + 286 842 / 840, 460 / 434; 357 + 358 1127 / 1128.
+_MOST_BYTES = 448 << 20
 _MOST_PLANS, _MOST_SEEN = 512, 4096
 
 # The time a set of sizes is met at which it is recorded.  Recording against what each later call saves, us: forward and
@@ -139,7 +139,8 @@ class _Recorder:
         self.device = _Device(index, self)
         self.real = _C.lib()
         self.words: list = []
-        self.addresses: list = []  # positions of addresses in words
+        self.addresses: list = []  # positions of addresses in words, and the number of their call
+        self.calls = 0
         self.sizes: list = []      # bytes of the places, numbered after the inputs
         self.n_inputs = n_inputs
 
@@ -161,7 +162,7 @@ class _Recorder:
         if kind is ctypes.c_void_p:
             value = int(value or 0)
             if value:
-                self.addresses.append(len(self.words))
+                self.addresses.append((len(self.words), self.calls))
         self.words.append(int(value))
 
     def _note(self, name: str, number: int, kinds, args) -> int:
@@ -181,6 +182,7 @@ class _Recorder:
             else:
                 self._word(a, kind)
         self.words.append(_STREAM)
+        self.calls += 1
         return 0
 
     def _slots(self, name: str, args) -> int:
@@ -199,6 +201,38 @@ def _places(tree):
     elif isinstance(tree, (tuple, list)):
         for t in tree:
             yield from _places(t)
+
+
+def _pack(temporaries: dict):
+    """``(offsets, bytes)`` of temporaries ``{name: (bytes, first call, last call)}`` in one buffer.  Two that no call has in common
+    may share bytes, as they do where the allocator is given each back after its last use (the calls of a plan follow one
+    another on one stream).  The largest first, each at the lowest offset that is free.
+
+    Bytes are shared where that saves a quarter of them, else every temporary has its own, which is up to 1 % faster.  us of
+    forward and backward, shared / of their own, MiB of the backward's temporaries: block of 4096 tokens, 2048 / 8192, float32 weights
+    766 / 759, 192 / 209, bfloat16 707 / 701; of 6000 tokens, 1024 / 2816 353 / 351, 12000 623 / 625, 194 / 350; three projections of
+    8192 x 2048 410 / 413, 16384 x 2048 807 / 811, 192 / 288."""
+    rounded = {name: (size + _ALIGN - 1) // _ALIGN * _ALIGN for name, (size, _, _) in temporaries.items()}
+    live: dict = {}
+    for name, (_, first, last) in temporaries.items():
+        for c in range(first, last + 1):
+            live[c] = live.get(c, 0) + rounded[name]
+    offsets, end, placed = {}, 0, []
+    if 4 * max(live.values(), default=0) > 3 * sum(rounded.values()):
+        for name, size in rounded.items():
+            offsets[name], end = end, end + size
+        return offsets, end
+    for name, size in sorted(rounded.items(), key=lambda t: -t[1]):
+        _, first, last = temporaries[name]
+        at = 0
+        for lo, hi in sorted((lo, hi) for lo, hi, f, l in placed if f <= last and first <= l):
+            if lo - at >= size:
+                break
+            at = max(at, hi)
+        offsets[name] = at
+        placed.append((at, at + size, first, last))
+        end = max(end, at + size)
+    return offsets, end
 
 
 class Plan:
@@ -221,16 +255,18 @@ class Plan:
                 raise Unplannable("an output that is no buffer of its own")
             where[number] = (n + 2 + k, 0)
             self.outs.append((o.shape, o.dtype))
-        totals = [0, 0]
+        self.kept = 0
         for p in _places(saved):
-            self._put(where, (p.address >> 48) - 1, n, rec.sizes, totals, 1)
-        for number in range(n, n + len(rec.sizes)):
-            self._put(where, number, n, rec.sizes, totals, 0)
-        self.temporary, self.kept = totals
-        if sum(totals) + sum(rec.sizes[k - n] for k, (b, _) in where.items() if b >= n + 2) > _MOST_BYTES:
-            raise Unplannable("more than _MOST_BYTES")
+            self._keep(where, (p.address >> 48) - 1, n, rec.sizes)
         words = list(rec.words)
-        for at in rec.addresses:
+        calls: dict = {number: [] for number in range(n, n + len(rec.sizes)) if number not in where}  # of the temporaries
+        for at, number_of_call in rec.addresses:
+            calls.get((words[at] >> 48) - 1, []).append(number_of_call)
+        offsets, self.temporary = _pack({number: (rec.sizes[number - n], c[0] if c else -1, c[-1] if c else -1) for number, c in calls.items()})
+        if self.temporary + self.kept + sum(rec.sizes[k - n] for k, (b, _) in where.items() if b >= n + 2) > _MOST_BYTES:
+            raise Unplannable("more than _MOST_BYTES")
+        where.update((number, (n, at)) for number, at in offsets.items())
+        for at, _ in rec.addresses:
             number = (words[at] >> 48) - 1
             if number >= n:
                 b, off = where[number]
@@ -243,14 +279,13 @@ class Plan:
         self.then: dict = {}  # plans of the backward, which depend on where this one keeps what it keeps
         self.used = False  # replayed since its table was last full
 
-    @staticmethod
-    def _put(where, number, n, sizes, totals, buffer) -> None:
+    def _keep(self, where, number, n, sizes) -> None:
         if number < n:
             raise Unplannable("an input is kept")
         if number not in where:
-            where[number] = (n + buffer, totals[buffer])
-            totals[buffer] += (sizes[number - n] + _ALIGN - 1) // _ALIGN * _ALIGN
-        elif where[number][0] != n + buffer and buffer == 1:
+            where[number] = (n + 1, self.kept)
+            self.kept += (sizes[number - n] + _ALIGN - 1) // _ALIGN * _ALIGN
+        elif where[number][0] != n + 1:
             raise Unplannable("an output is kept")
 
     def _rebase(self, tree, where):

@@ -62,6 +62,24 @@ def test_feed_forward(dev, runs, tokens, d, h, autocast):
     _check(lambda s: _step(model, seeded((tokens, d), s).to(dev), lambda x: [model(x)], [go], autocast), runs, 2)
 
 
+def test_replays_hold_no_more_than_the_calls(dev, runs):
+    """A block whose backward, call by call, gives back half of its temporaries before it takes the next: so does its plan."""
+    model = FeedForward(d_model=1024, hidden_size=2816, bias=False, dtype=torch.bfloat16, init_device="cuda")
+    Float8Config(ao_recipe=AOFloat8LinearRecipe.tensorwise).apply_float8_linear(_fill(model))
+    go, peaks = seeded((12000, 1024), 5, std=1e-3).to(dev), []
+
+    def step(s):
+        x = seeded((12000, 1024), s).to(dev)
+        torch.cuda.reset_peak_memory_stats()
+        held = torch.cuda.memory_allocated()
+        out = _step(model, x, lambda t: [model(t)], [go])
+        peaks.append(torch.cuda.max_memory_allocated() - held)
+        return out
+
+    _check(step, runs, 2)
+    assert peaks[-1] <= 1.05 * peaks[0]
+
+
 @pytest.mark.parametrize("tokens", [1, 16, 23, 65, 777])
 def test_evaluation(dev, runs, tokens):
     model = FeedForward(d_model=256, hidden_size=768, bias=False, dtype=torch.bfloat16, init_device="cuda")

@@ -1,5 +1,7 @@
 """The tables of recorded sequences (olmo_core_amd/float8/plan.py), on the CPU."""
 
+import itertools
+import random
 import types
 
 import pytest
@@ -82,3 +84,21 @@ def test_inputs_on_two_gpus_have_no_plan(monkeypatch):
         assert plan.call(None, [on(0), None, on(0)], ("a test",)) is None
     assert plan.call(None, [on(0), None, on(0)], ("a test",)) is not None
     assert plan.call(None, [on(0), None, on(1)], ("a test",)) is None
+
+
+def test_temporaries_share_bytes_only_in_different_calls():
+    """Intervals of calls that overlap get bytes of their own, all within the buffer; what has no call in common is reused."""
+    rng = random.Random(1)
+    for _ in range(300):
+        calls = rng.randint(1, 20)
+        t = {i: (rng.choice((0, 1, 255, 256, 257, rng.randint(1, 1 << 20))), *sorted(rng.choices(range(calls), k=2))) for i in range(rng.randint(0, 25))}
+        at, size = plan._pack(t)
+        assert at.keys() == t.keys() and all(a >= 0 and a % plan._ALIGN == 0 and a + t[i][0] <= size for i, a in at.items())
+        for (i, a), (j, b) in itertools.combinations(at.items(), 2):
+            if t[i][1] <= t[j][2] and t[j][1] <= t[i][2]:
+                assert a + t[i][0] <= b or b + t[j][0] <= a
+        rounded = {i: -(-v[0] // plan._ALIGN) * plan._ALIGN for i, v in t.items()}
+        most = max((sum(rounded[i] for i, v in t.items() if v[1] <= c <= v[2]) for c in range(calls)), default=0)
+        assert most <= size <= sum(rounded.values())
+    assert plan._pack({"a": (512, 0, 1), "b": (512, 2, 3), "c": (100, 1, 2)}) == ({"a": 0, "b": 0, "c": 512}, 768)
+    assert plan._pack({}) == ({}, 0)
