@@ -120,6 +120,7 @@ struct TileCastArgs {
     int64_t ld_t;
     float* scale_out;  // scalar modes: [1]; per-column mode: [cols]; may be null
     int64_t t_end;     // columns of out_t written: rows and the zeros after them
+    bool stream;
 };
 
 template <int HP, int FP8, bool SW, int MODE>
@@ -170,7 +171,7 @@ __global__ __launch_bounds__(kThreads) void tile_cast_kernel(TileCastArgs a)
         for (int i = 0; i < 8; ++i) sc[i] = s;
     }
 
-    tile_quantise<FP8, SW>(values, a.rows, a.cols, row0, col0, sc, a.out, a.ld_out, a.out_t, a.ld_t, row0, a.t_end, lds_t);
+    tile_quantise<FP8, SW>(values, a.rows, a.cols, row0, col0, sc, a.out, a.ld_out, a.out_t, a.ld_t, row0, a.t_end, lds_t, a.stream);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -265,6 +266,7 @@ struct RowCastArgs {
     const int32_t* gather;  // kRowGather: [rows], x is [src_rows, cols]
     int top_k;
     int64_t src_rows;
+    bool stream;
 };
 
 template <int HP, int FP8, bool SW, int TPR /* 64 or 256 */, int NV /* 8-element vectors per lane */, int SRC>
@@ -310,7 +312,7 @@ __global__ __launch_bounds__(kThreads) void rowwise_cast_kernel(RowCastArgs a)
         if (row_ok && v < nvec) {
             const uint32_t lo = quant4<FP8, SW>(f[i][0], f[i][1], f[i][2], f[i][3], s, s, s, s);
             const uint32_t hi = quant4<FP8, SW>(f[i][4], f[i][5], f[i][6], f[i][7], s, s, s, s);
-            store_stream8(orow + (int64_t)v * 8, lo, hi);
+            store_out8(orow + (int64_t)v * 8, lo, hi, a.stream);
         }
     }
 }
@@ -343,6 +345,7 @@ struct GroupedCastArgs {
     int64_t src_rows;
     const void* gather_w;  // optional weight per slot (weighted gather), of element type gather_w_dtype
     int gather_w_dtype;
+    bool stream;
 };
 
 // Tile p of the padded row space (128 rows each; group e owns ceil(m_e / 128) consecutive tiles) -> its group,
@@ -517,6 +520,7 @@ struct SwigluBwdCastArgs {
     float* scale_out1;  // [1]
     float* scale_out3;
     int64_t t_end;  // columns of the transposed copies written
+    bool stream;
 };
 
 template <int FP8, bool SW>
@@ -579,7 +583,7 @@ __global__ __launch_bounds__(kThreads) void swiglu_bwd_cast_kernel(SwigluBwdCast
                 lo[j] = quant4<FP8, SW>(v[0], v[1], v[2], v[3], sc[o], sc[o], sc[o], sc[o]);
                 hi[j] = quant4<FP8, SW>(v[4], v[5], v[6], v[7], sc[o], sc[o], sc[o], sc[o]);
                 if (!ok) lo[j] = hi[j] = 0;  // padding is zero bytes whatever the scale is (0 * NaN is NaN)
-                if (out[o] && ok) store_stream8(out[o] + r * a.ld_out + c8, lo[j], hi[j]);
+                if (out[o] && ok) store_out8(out[o] + r * a.ld_out + c8, lo[j], hi[j], a.stream);
             }
             if (want_t) {
                 uint32_t t[8];
@@ -606,7 +610,7 @@ __global__ __launch_bounds__(kThreads) void swiglu_bwd_cast_kernel(SwigluBwdCast
                 const uint4 v = reinterpret_cast<const uint4*>(lds_t[o])[tile_lds_chunk(col, part)];
                 const int64_t c = col0 + col;
                 const int64_t d = row0 + 16 * part;
-                if (c < a.cols && d < dst_end) store_stream16(out_t[o] + c * a.ld_t + d, v);
+                if (c < a.cols && d < dst_end) store_out16(out_t[o] + c * a.ld_t + d, v, a.stream);
             }
     }
 }
@@ -746,7 +750,7 @@ __global__ __launch_bounds__(kThreads) void grouped_tile_cast_kernel(GroupedCast
     for (int i = 0; i < 8; ++i) sc[i] = s_scale[8 * cl + i];
     const int64_t dst0 = (int64_t)kTile * rt;
     if (GATHER && a.gather_w) values.scale_rows(rows.w, col0 + 8 * cl < a.cols);
-    tile_quantise<FP8, SW>(values, row_end, a.cols, row0, col0, sc, nullptr, 0, a.out_t, a.ld_t, dst0, a.ld_t, lds_t, a.out_r, a.ld_r,
+    tile_quantise<FP8, SW>(values, row_end, a.cols, row0, col0, sc, nullptr, 0, a.out_t, a.ld_t, dst0, a.ld_t, lds_t, a.stream, a.out_r, a.ld_r,
                            s_row_scale, row0);
 }
 
@@ -1069,7 +1073,8 @@ extern "C" int mi8_cast_tensorwise(const void* x, int hp_dtype, int64_t rows, in
         return launch_status("mi8_cast_tensorwise");
     }
     TileCastArgs a{x, rows, cols, slots, n_slots, scale_in, (flags & MI8_FLAG_POW2_SCALE) != 0,
-                   (uint8_t*)out, ld_out, (uint8_t*)out_t, ld_t, scale_out, t_end};
+                   (uint8_t*)out, ld_out, (uint8_t*)out_t, ld_t, scale_out, t_end,
+                   streams_outputs(rows * cols * ((out ? 1 : 0) + (out_t ? 1 : 0)))};
     dispatch_tile_cast(hp_dtype, fp8_dtype, (flags & MI8_FLAG_SW_CVT) != 0, slots ? kScalarFromSlots : kScalarFromPtr,
                        a, (hipStream_t)stream);
     return launch_status("mi8_cast_tensorwise");
@@ -1169,7 +1174,8 @@ extern "C" int mi8_swiglu_bwd_cast(const void* x1, const void* x3, const void* g
                     (long long)ld_t);
     SwigluBwdCastArgs a{(const uint4*)x1, (const uint4*)x3, (const uint4*)gh, rows, cols, slots_g1, slots_g3, n_slots,
                         (flags & MI8_FLAG_POW2_SCALE) != 0, (uint8_t*)out1, (uint8_t*)out3, ld_out, (uint8_t*)out1_t,
-                        (uint8_t*)out3_t, ld_t, scale_out1, scale_out3, t_end};
+                        (uint8_t*)out3_t, ld_t, scale_out1, scale_out3, t_end,
+                        streams_outputs(2 * rows * cols * ((out1 ? 1 : 0) + (out1_t ? 1 : 0)))};
     const dim3 grid((unsigned)ceil_div(cols, kTile), (unsigned)ceil_div(rows, kTile));
     hipStream_t st = (hipStream_t)stream;
     const bool sw = flags & MI8_FLAG_SW_CVT;
@@ -1196,7 +1202,7 @@ extern "C" int mi8_cast_rowwise(const void* x, int hp_dtype, int64_t rows, int64
     MI8_REQUIRE(aligned16(x) && aligned16(out), MI8_ERR_UNSUPPORTED, "mi8_cast_rowwise: pointers must be 16-byte aligned");
     const bool pow2 = flags & MI8_FLAG_POW2_SCALE, sw = flags & MI8_FLAG_SW_CVT;
     hipStream_t st = (hipStream_t)stream;
-    const RowCastArgs a{x, rows, cols, pow2, (uint8_t*)out, ld_out, scale_out, nullptr, nullptr, 0, 0};
+    const RowCastArgs a{x, rows, cols, pow2, (uint8_t*)out, ld_out, scale_out, nullptr, nullptr, 0, 0, streams_outputs(rows * cols)};
     int rc;
 #define MI8_ROW(HP_, FP8_) \
     rc = sw ? launch_rowwise<HP_, FP8_, true>(a, st) : launch_rowwise<HP_, FP8_, false>(a, st)
@@ -1235,7 +1241,7 @@ extern "C" int mi8_moe_gather_cast_rows(const void* x, int64_t tokens, int64_t c
     int rc = check_expert_rows("mi8_moe_gather_cast_rows", tokens * top_k, cols, x, out, ld_out, scale_out);
     if (rc != MI8_OK) return rc;
     const RowCastArgs a{x, tokens * top_k, cols, (flags & MI8_FLAG_POW2_SCALE) != 0, (uint8_t*)out, ld_out, scale_out,
-                        nullptr, indices, top_k, tokens};
+                        nullptr, indices, top_k, tokens, streams_outputs(tokens * top_k * cols)};
     rc = (flags & MI8_FLAG_SW_CVT) ? launch_rowwise<MI8_BF16, MI8_E4M3, true, kRowGather>(a, (hipStream_t)stream)
                                    : launch_rowwise<MI8_BF16, MI8_E4M3, false, kRowGather>(a, (hipStream_t)stream);
     MI8_REQUIRE(rc == MI8_OK, rc, "mi8_moe_gather_cast_rows: unsupported row length %lld", (long long)cols);
@@ -1248,7 +1254,8 @@ extern "C" int mi8_swiglu_cast_rows(const void* x1, const void* x3, int64_t rows
     int rc = check_expert_rows("mi8_swiglu_cast_rows", rows, cols, x1, out, ld_out, scale_out);
     if (rc != MI8_OK) return rc;
     MI8_REQUIRE(x3 && aligned16(x3), MI8_ERR_ARG, "mi8_swiglu_cast_rows: x3 must be given and 16-byte aligned");
-    const RowCastArgs a{x1, rows, cols, (flags & MI8_FLAG_POW2_SCALE) != 0, (uint8_t*)out, ld_out, scale_out, x3, nullptr, 0, 0};
+    const RowCastArgs a{x1, rows, cols, (flags & MI8_FLAG_POW2_SCALE) != 0, (uint8_t*)out, ld_out, scale_out, x3, nullptr, 0, 0,
+                        streams_outputs(rows * cols)};
     rc = (flags & MI8_FLAG_SW_CVT) ? launch_rowwise<MI8_BF16, MI8_E4M3, true, kRowSwiglu>(a, (hipStream_t)stream)
                                    : launch_rowwise<MI8_BF16, MI8_E4M3, false, kRowSwiglu>(a, (hipStream_t)stream);
     MI8_REQUIRE(rc == MI8_OK, rc, "mi8_swiglu_cast_rows: unsupported row length %lld", (long long)cols);
@@ -1285,7 +1292,7 @@ extern "C" int mi8_cast_colwise_t(const void* x, int hp_dtype, int64_t rows, int
     int rc = launch_status("mi8_cast_colwise_t(amax)");
     if (rc != MI8_OK) return rc;
     TileCastArgs a{x, rows, cols, workspace, n_chunks, nullptr, (flags & MI8_FLAG_POW2_SCALE) != 0,
-                   nullptr, 0, (uint8_t*)out_t, ld_t, scale_out, round_up(rows, 16)};
+                   nullptr, 0, (uint8_t*)out_t, ld_t, scale_out, round_up(rows, 16), streams_outputs(rows * cols)};
     dispatch_tile_cast(hp_dtype, fp8_dtype, (flags & MI8_FLAG_SW_CVT) != 0, kPerColumnFromWorkspace, a, st);
     return launch_status("mi8_cast_colwise_t(cast)");
 }
@@ -1325,7 +1332,7 @@ int grouped_cast_launch(const char* what, const void* x, int hp_dtype, int64_t T
     const bool pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
     GroupedCastArgs a{x, T, cols, group_sizes, num_groups, pow2, amax_ws, (uint8_t*)out_t, ld_t, scale_out,
                       out_rows ? row_amax_ws : nullptr, (uint8_t*)out_rows, ld_rows, row_scale_out, gather, top_k, src_rows, gather_w,
-                      gather_w_dtype};
+                      gather_w_dtype, streams_outputs(T * cols * (out_rows ? 2 : 1))};
     hipStream_t st = (hipStream_t)stream;
     dim3 grid((unsigned)ceil_div(cols, kTile), (unsigned)ptiles);
     int rc = MI8_OK;

@@ -46,7 +46,7 @@ struct AmaxItems {
 struct CastItems {
     CastItem t[MI8_CAST_BATCH];
     int count;
-    bool pow2;
+    bool pow2, stream;
 };
 
 template <typename Items>
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(kThreads) void amax_items_kernel(AmaxItems a)
 }
 
 template <int HP, int FP8, bool SW>
-__device__ __forceinline__ void cast_item(const CastItem& t, int tile, bool pow2, uint32_t* lds_t, uint32_t* smem)
+__device__ __forceinline__ void cast_item(const CastItem& t, int tile, bool pow2, bool stream, uint32_t* lds_t, uint32_t* smem)
 {
     const int64_t row0 = (int64_t)(tile / t.tiles_n) * kTile, col0 = (int64_t)(tile % t.tiles_n) * kTile;
     RawTile<HP> values;
@@ -108,7 +108,7 @@ __device__ __forceinline__ void cast_item(const CastItem& t, int tile, bool pow2
     float sc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) sc[i] = s;
-    tile_quantise<FP8, SW>(values, t.rows, t.cols, row0, col0, sc, t.out, t.ld_out, t.out_t, t.ld_t, row0, t.t_end, lds_t);
+    tile_quantise<FP8, SW>(values, t.rows, t.cols, row0, col0, sc, t.out, t.ld_out, t.out_t, t.ld_t, row0, t.t_end, lds_t, stream);
 }
 
 // MIX: bf16, float32, or both
@@ -122,9 +122,9 @@ __global__ __launch_bounds__(kThreads) void cast_items_kernel(CastItems a)
     const int block = (int)blockIdx.x;
     const CastItem& t = a.t[item_of_block(a, block)];
     if (MIX == kAllF32 || (MIX == kMixed && t.fp32))
-        cast_item<MI8_F32, FP8, SW>(t, block - t.first, a.pow2, lds_t, smem);
+        cast_item<MI8_F32, FP8, SW>(t, block - t.first, a.pow2, a.stream, lds_t, smem);
     else
-        cast_item<MI8_BF16, FP8, SW>(t, block - t.first, a.pow2, lds_t, smem);
+        cast_item<MI8_BF16, FP8, SW>(t, block - t.first, a.pow2, a.stream, lds_t, smem);
 }
 
 // ---- a scale per row (row-major copy) and a scale per column (transposed copy) of several tensors -----------------------
@@ -157,7 +157,7 @@ struct TwoCastItem {
 struct TwoCastItems {
     TwoCastItem t[MI8_CAST_BATCH];
     int count;
-    bool pow2;
+    bool pow2, stream;
 };
 
 template <int HP>
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(kThreads) void two_amax_items_kernel(TwoCastItems a
 }
 
 template <int HP, int FP8, bool SW>
-__device__ __forceinline__ void two_cast_item(const TwoCastItem& t, int tile, bool pow2, uint32_t* lds_t, uint32_t (&parts)[2][4][kTile],
+__device__ __forceinline__ void two_cast_item(const TwoCastItem& t, int tile, bool pow2, bool stream, uint32_t* lds_t, uint32_t (&parts)[2][4][kTile],
                                               float (&s_scale)[2][kTile])
 {
     const int rt = tile / t.tiles_n, ct = tile % t.tiles_n;
@@ -291,7 +291,7 @@ __device__ __forceinline__ void two_cast_item(const TwoCastItem& t, int tile, bo
     float sc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) sc[i] = s_scale[0][8 * (tid & 15) + i];
-    tile_quantise<FP8, SW>(values, t.rows, t.cols, row0, col0, sc, nullptr, 0, t.out_t, t.ld_t, row0, t.ld_t, lds_t, t.out_r, t.ld_r,
+    tile_quantise<FP8, SW>(values, t.rows, t.cols, row0, col0, sc, nullptr, 0, t.out_t, t.ld_t, row0, t.ld_t, lds_t, stream, t.out_r, t.ld_r,
                            s_scale[1], row0);
 }
 
@@ -304,9 +304,9 @@ __global__ __launch_bounds__(kThreads) void two_cast_items_kernel(TwoCastItems a
     const int block = (int)blockIdx.x;
     const TwoCastItem& t = a.t[item_of_block(a, block)];
     if (MIX == kAllF32 || (MIX == kMixed && t.fp32))
-        two_cast_item<MI8_F32, FP8, SW>(t, block - t.first, a.pow2, lds_t, parts, s_scale);
+        two_cast_item<MI8_F32, FP8, SW>(t, block - t.first, a.pow2, a.stream, lds_t, parts, s_scale);
     else
-        two_cast_item<MI8_BF16, FP8, SW>(t, block - t.first, a.pow2, lds_t, parts, s_scale);
+        two_cast_item<MI8_BF16, FP8, SW>(t, block - t.first, a.pow2, a.stream, lds_t, parts, s_scale);
 }
 
 bool valid_hp(int v) { return v == MI8_BF16 || v == MI8_F32; }
@@ -370,7 +370,7 @@ extern "C" int mi8_cast_tensorwise_batch(const mi8_cast_item* items, int32_t cou
     CastItems ca{};
     ca.count = count;
     ca.pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
-    int64_t amax_blocks = 0, cast_blocks = 0;
+    int64_t amax_blocks = 0, cast_blocks = 0, bytes = 0;
     for (int i = 0; i < count; ++i) {
         const mi8_cast_item& t = items[i];
         MI8_REQUIRE(t.x && t.scale_out && (t.out || t.out_t) && (t.slots || t.scale_in || t.amax_ws), MI8_ERR_ARG, "%s: tensor %d: null pointer", what, i);
@@ -396,7 +396,9 @@ extern "C" int mi8_cast_tensorwise_batch(const mi8_cast_item* items, int32_t cou
         ca.t[i] = CastItem{t.x, t.rows, t.cols, slots, t.scale_in, (uint8_t*)t.out, t.ld_out, (uint8_t*)t.out_t, t.ld_t, t_end,
                            t.scale_out, n_slots, fp32, (int)tiles_n, (int)cast_blocks};
         cast_blocks += tiles;
+        bytes += t.rows * t.cols * ((t.out ? 1 : 0) + (t.out_t ? 1 : 0));
     }
+    ca.stream = streams_outputs(bytes);
     hipStream_t st = (hipStream_t)stream;
     if (am.count)
         if (int rc = launch_items(amax_items_kernel, am, amax_blocks, st, what)) return rc;
@@ -436,7 +438,7 @@ extern "C" int mi8_cast_rows_and_colwise_t_batch(const mi8_two_cast_item* items,
     TwoCastItems a{};
     a.count = count;
     a.pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
-    int64_t blocks = 0, chunk_blocks = 0;
+    int64_t blocks = 0, chunk_blocks = 0, bytes = 0;
     for (int i = 0; i < count; ++i) {
         const mi8_two_cast_item& t = items[i];
         const int64_t tiles_m = ceil_div(t.rows, kTile), tiles_n = ceil_div(t.cols, kTile);
@@ -449,6 +451,8 @@ extern "C" int mi8_cast_rows_and_colwise_t_batch(const mi8_two_cast_item* items,
                              chunk, (int)group_tiles, (int)group_chunks, (int)blocks, (int)chunk_blocks};
         blocks += tiles_m * tiles_n;
         chunk_blocks += chunks * tiles_n;
+        bytes += 2 * t.rows * t.cols;
     }
+    a.stream = streams_outputs(bytes);
     return launch_two_cast(a, fp8_dtype, (flags & MI8_FLAG_SW_CVT) != 0, chunk_blocks, blocks, (hipStream_t)stream, what);
 }

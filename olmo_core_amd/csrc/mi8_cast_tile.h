@@ -172,12 +172,13 @@ struct RawTile {
 // Quantise a loaded tile (values(it, j, f): a thread's eight of row 16 it + j) with the eight per-column scales of this lane
 // (all equal for a tensorwise cast).
 // Row-major bytes go to out[r, c]; the transposed bytes go to out_t[c, dst0 + (r - row0)] as 16-byte chunks,
-// chunks at or beyond dst_end are not written.
+// chunks at or beyond dst_end are not written.  stream: see streams_outputs.
 template <int FP8, bool SW, typename Values>
 __device__ __forceinline__ void tile_quantise(const Values& values, int64_t row_end, int64_t cols, int64_t row0, int64_t col0,
                                               const float (&sc)[8], uint8_t* out, int64_t ld_out, uint8_t* out_t, int64_t ld_t,
-                                              int64_t dst0, int64_t dst_end, uint32_t* lds_t, uint8_t* out_r = nullptr,
-                                              int64_t ld_r = 0, const float* row_scale = nullptr, int64_t row_scale_row0 = 0)
+                                              int64_t dst0, int64_t dst_end, uint32_t* lds_t,
+                                              bool stream, uint8_t* out_r = nullptr, int64_t ld_r = 0, const float* row_scale = nullptr,
+                                              int64_t row_scale_row0 = 0)
 {
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
@@ -207,12 +208,12 @@ __device__ __forceinline__ void tile_quantise(const Values& values, int64_t row_
             lo[j] = quant4<FP8, SW>(v[0], v[1], v[2], v[3], sc[0], sc[1], sc[2], sc[3]);
             hi[j] = quant4<FP8, SW>(v[4], v[5], v[6], v[7], sc[4], sc[5], sc[6], sc[7]);
             if (!ok) lo[j] = hi[j] = 0;  // padding is zero bytes whatever the scale is (0 * NaN is NaN)
-            if (out && ok) store_stream8(out + r * ld_out + c8, lo[j], hi[j]);
+            if (out && ok) store_out8(out + r * ld_out + c8, lo[j], hi[j], stream);
             if (out_r && ok) {  // the same values quantised with the row's own scale
                 const float sr = srow[it][j];
                 const uint32_t rl = quant4<FP8, SW>(v[0], v[1], v[2], v[3], sr, sr, sr, sr);
                 const uint32_t rh = quant4<FP8, SW>(v[4], v[5], v[6], v[7], sr, sr, sr, sr);
-                store_stream8(out_r + r * ld_r + c8, rl, rh);
+                store_out8(out_r + r * ld_r + c8, rl, rh, stream);
             }
         }
         if (out_t) {
@@ -237,7 +238,7 @@ __device__ __forceinline__ void tile_quantise(const Values& values, int64_t row_
             const uint4 v = reinterpret_cast<const uint4*>(lds_t)[tile_lds_chunk(col, part)];
             const int64_t c = col0 + col;
             const int64_t d = dst0 + 16 * part;
-            if (c < cols && d < dst_end) store_stream16(out_t + c * ld_t + d, v);
+            if (c < cols && d < dst_end) store_out16(out_t + c * ld_t + d, v, stream);
         }
     }
 }

@@ -31,6 +31,14 @@ static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t
 static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 static inline int64_t round_up(int64_t a, int64_t b) { return ceil_div(a, b) * b; }
 
+// Whether a cast that writes `bytes` of float8 stores them streaming (the nt bit).  What it writes is what the next products
+// read, so as long as it fits the memory-side cache (256 MB) it is left there: a tile's K loop runs at the rate its operands arrive, and
+// from HBM they come in 128-byte pieces of as many rows as there are tiles (1537 x 2048 x 2048: 9.7 us streamed, 6.7 left in the
+// cache; 777 x 4096 x 11008 46 and 32).  Beyond, the copies would only displace each other and the input.  us of a step, streamed / kept:
+// block of 1024 tokens, 2048 / 8192 (50 MB a launch) 352 / 327, of 4096 in float32 789 / 765 (117 MB), of 4096, 4096 / 11008 1552 / 1527 (180 MB);
+// four projections of 4096 x 2048 386 / 361; 64 experts of 2048 x 1024, 131072 rows (268 MB) 4470 / 4735.
+static inline bool streams_outputs(int64_t bytes) { return bytes > (int64_t)192 << 20; }
+
 // ---- device side ---------------------------------------------------------------------------------
 
 template <int FP8>
@@ -180,7 +188,7 @@ __device__ __forceinline__ void transpose4x4_bytes(uint32_t r0, uint32_t r1, uin
     c3 = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
 }
 
-// Streaming accesses (the nt bit): for data a kernel reads for the last time, or writes for a later kernel to read.
+// Streaming accesses (the nt bit): for data a kernel reads for the last time, or writes more of than the memory-side cache holds.
 // Such lines take no space from data that is about to be read again - in a two-pass cast the second pass's
 // outputs otherwise evict what the first pass left of the input in the memory-side cache (16384 x 11008: amax + cast
 // 232 -> 181 us); rows gathered several times and tables read again keep the default.
@@ -198,6 +206,29 @@ __device__ __forceinline__ void store_stream16(void* p, uint4 v)
 __device__ __forceinline__ void store_stream8(void* p, uint32_t lo, uint32_t hi)
 {
     __builtin_nontemporal_store((u32x2_t){lo, hi}, reinterpret_cast<u32x2_t*>(p));
+}
+
+// A cast's outputs, whichever way the launch stores them (uniform; see streams_outputs).  (The empty statements keep the
+// compiler from merging the two stores into one without the bit.)
+__device__ __forceinline__ void store_out16(void* p, uint4 v, bool stream)
+{
+    if (stream) {
+        asm volatile("");
+        store_stream16(p, v);
+        asm volatile("");
+    } else {
+        *reinterpret_cast<u32x4_t*>(p) = (u32x4_t){v.x, v.y, v.z, v.w};
+    }
+}
+__device__ __forceinline__ void store_out8(void* p, uint32_t lo, uint32_t hi, bool stream)
+{
+    if (stream) {
+        asm volatile("");
+        store_stream8(p, lo, hi);
+        asm volatile("");
+    } else {
+        *reinterpret_cast<u32x2_t*>(p) = (u32x2_t){lo, hi};
+    }
 }
 
 // Eight consecutive high-precision elements starting at a 16-byte aligned address -> float[8]

@@ -409,3 +409,20 @@ def test_two_scale_cast_into_a_wider_pitch(dev, rows, group_rows):
     assert torch.equal(q[:, :cols], want_q.view(torch.uint8)) and bool((q[:, cols:] == 0x55).all())
     assert torch.equal(q_t[:, :end], want_t.view(torch.uint8)) and bool((q_t[:, end:] == 0x55).all())
     assert not q_t[:, rows:end].any() and torch.equal(rs, want_rs) and torch.equal(cs, want_cs)
+
+
+@pytest.mark.parametrize("rows", [12288, 12304], ids=["kept_in_cache", "streamed"])
+def test_outputs_around_the_line_of_streaming_stores(dev, rows):
+    """Two copies of 12288 x 8192 are the most that is left in the memory-side cache, 16 more rows are stored past it: the same bytes
+    as casts of a sixteenth of the rows each, which every kernel keeps in the cache."""
+    cols, part = 8192, rows // 16
+    x = seeded((64, cols), 5).to(dev).repeat(rows // 64 + 1, 1)[:rows].contiguous()
+    s = torch.tensor([0.37], device=dev)
+    q, q_t, _ = ops.cast_tensorwise(x, E4M3, scale=s, want_transposed=True)
+    rq, rs, rq_t, _ = ops.cast_rows_and_colwise_t(x, E4M3)
+    for i in range(0, rows, part):
+        p, p_t, _ = ops.cast_tensorwise(x[i:i + part], E4M3, scale=s, want_transposed=True)
+        assert torch.equal(u8(q[i:i + part]), u8(p)) and torch.equal(u8(q_t[:, i:i + part]), u8(p_t[:, :part])), i
+        p, ps, p_t, _ = ops.cast_rows_and_colwise_t(x[i:i + part], E4M3)  # (every part holds each of the 64 rows: the same column scales)
+        assert torch.equal(u8(rq[i:i + part]), u8(p)) and torch.equal(rs[i:i + part], ps), i
+        assert torch.equal(u8(rq_t[:, i:i + part]), u8(p_t[:, :part])), i
