@@ -106,7 +106,7 @@ __device__ __forceinline__ bool tile_of_block(const GemmArgs& g, int& tm, int& t
 // persistent direct-to-LDS kernel, four waves of 128 x 128 on 16x16x128 MFMAs (mi8_gemm_m16.hip); requires
 // M, N >= 256, K % 128 == 0, N % 8 == 0, ldc % 8 == 0, a 16-byte aligned bf16 output
 int launch_m16(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st);  // (honours g.accumulate)
-float m16_cost(int64_t M, int64_t N, int64_t K);  // us such a launch takes, as a model fitted to measurements
+float m16_cost(int64_t M, int64_t N, int64_t K, bool quarters);  // us such a launch takes, as a model fitted to measurements
 // the same with single scales, also recording the row-segment codes of C (uint16 [N / 64][M], N % 64 == 0)
 int launch_m16_codes(GemmArgs& g, uint16_t* codes, int a_dtype, int b_dtype, hipStream_t st);
 // the two input projections of a SwiGLU block and h = silu(x1) * x3 in one launch (g: A, B = B1, C = x1, N = H,

@@ -268,7 +268,7 @@ int suggested_splits(int64_t M, int64_t N, int64_t K)
     if (tiles256 > 96 || steps < 8) return 1;
     float best = slices_estimate(M, N, steps, 1);
     if (M >= 256 && N >= 256 && K % BK == 0 && N % 8 == 0) {
-        const float t = m16_cost(M, N, K);
+        const float t = m16_cost(M, N, K, false);
         best = t < best ? t : best;
     }
     if (tiles64 <= 192) best = 1e30f;
@@ -467,7 +467,7 @@ int chosen_variant(int64_t M, int64_t N, int64_t K, bool m16_fits)
     float cost;
     const int64_t steps = ceil_div(K, BK);
     const int ring = best_ring(M, N, steps, 1, &cost);
-    if (m16_fits) return m16_cost(M, N, K) < cost ? kM16 : ring;
+    if (m16_fits) return m16_cost(M, N, K, true) < cost ? kM16 : ring;
     // (rows that do not start on a cache line cost the small tiles, which read them more often, a quarter more, the large
     // ones 5-7 %: 16384 x 4096 x 11008 and 11024, 616 and 834 us, 550 and 601)
     return ring_cost(kRing[kRing256], M, N, steps, 1) < (K % BK ? 1.25f : 1.0f) * cost ? kRing256 : ring;
@@ -792,7 +792,7 @@ extern "C" int mi8_gemm_fp8_batch_pays(const mi8_gemm_product* products, int32_t
         float t;
         best_ring(g.M, g.N, ceil_div(g.K, BK), 1, &t, g.slice_steps != 0);
         if (m16_takes(g.M, g.N, g.K, g.ldc, g.c_f32 == 0 ? MI8_BF16 : g.c_f32 == 1 ? MI8_F32 : MI8_F32_OF_BF16, acc) && aligned16(g.C) && !g.slice_steps) {
-            const float p = m16_cost(g.M, g.N, g.K);
+            const float p = m16_cost(g.M, g.N, g.K, true);
             t = p < t ? p : t;
         }
         apart += 1.2f * t;

@@ -96,17 +96,18 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t out_rows(void* p, int bytes)
 // s_waitcnt: at most n vector memory operations of this wave outstanding, the other counters untouched
 constexpr int vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
 
-// Workgroup `block` of `blocks` that walk the problem's whole tiles (kHalf: one half tile each, 128 x 256: the waves take
-// 64 x 128).
-template <typename Problem, int CBSZ_A, int BLGP_B, bool kHalf>
+// Workgroup `block` of `blocks` that walk the problem's whole tiles (kRows = 256), or have a half (128 x 256: the waves take
+// 64 x 128) or a quarter of a tile (64 x 256: 32 x 128) each.
+template <typename Problem, int CBSZ_A, int BLGP_B, int kRows>
 __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, const int blocks)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    constexpr int WTM = kHalf ? WT / 2 : WT;          // rows of a wave's part of the tile
-    constexpr int kRowsA = kHalf ? BM / 2 : BM;       // A rows of a stage
-    constexpr int kStage = (kRowsA + BN) * BK;
-    constexpr int kLoadsA = kHalf ? kLoads / 2 : kLoads;
-    constexpr int kPasses = kHalf ? 2 : 4;            // epilogue: blocks of 32 rows of the wave's part
+    static_assert(kRows == BM || kRows == BM / 2 || kRows == BM / 4, "whole tiles, halves, quarters");
+    constexpr bool kPart = kRows < BM;
+    constexpr int WTM = kRows / 2;                    // rows of a wave's part of the tile
+    constexpr int kStage = (kRows + BN) * BK;
+    constexpr int kLoadsA = kRows / 32;
+    constexpr int kPasses = kRows / 64;               // epilogue: blocks of 32 rows of the wave's part
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -114,7 +115,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
     const int wm = wave >> 1, wn = wave & 1;
     const int r16 = lane & 15, kb = lane >> 4;  // fragment row inside a tile; 32-byte K block of the lane
 #ifdef MI8_TILE_TIMELINE
-    uint32_t* const tl_out = !kHalf && (int)blockIdx.x < TIMELINE_WORKGROUPS ? g_timeline : nullptr;
+    uint32_t* const tl_out = !kPart && (int)blockIdx.x < TIMELINE_WORKGROUPS ? g_timeline : nullptr;
     int tl_ev = 0;
     const uint32_t tl_lds = (uint32_t)(uintptr_t)(lptr_t)(lds + LDS_BYTES - TIMELINE_BYTES);
     auto tl_put = [&](int slot, uint64_t t) __attribute__((always_inline)) {
@@ -144,7 +145,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
         for (int q = 0; q < 2; ++q) {
             const uint32_t chunk = (uint32_t)((2 * kb + q) ^ swz16(r16));
             ra[q] = lds0 + (uint32_t)((wm * WTM + r16) * BK) + (chunk << 4);
-            rb[q] = lds0 + (uint32_t)(kRowsA * BK + (wn * WT + r16) * BK) + (chunk << 4);
+            rb[q] = lds0 + (uint32_t)(kRows * BK + (wn * WT + r16) * BK) + (chunk << 4);
         }
     }
     auto flip_read_stage = [&](int to_stage) __attribute__((always_inline)) {
@@ -176,7 +177,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
         dv[k] = (uint32_t)((int64_t)lr * ld) + ((uint32_t)((lane & 7) ^ swz16(8 * (k & 1) + lr)) << 4);
     }
     // x in 0..15: the first eight -> A rows 8 x, the rest -> B rows 8 (x - 8).  A half tile has 128 rows of A: wave w fetches
-    // rows [32 w, +32) with the first four.
+    // rows [32 w, +32) with the first four; a quarter has 64: rows [16 w, +16) with the first two.
     auto dma_one = [&](const uint8_t* a_origin, const uint8_t* b_origin, int stage, int x) __attribute__((always_inline)) {
         const bool is_a = x < kLoads;
         const int p = x % kLoads;
@@ -185,7 +186,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
         asm volatile("" : "+s"(rows));  // opaque: the sum stays one add at the load instead of sixteen resident registers
         const uint32_t o = dv[(is_a ? 0 : 2) + (p & 1)] + rows;
         const uint8_t* src = (is_a ? a_origin : b_origin) + o;
-        uint8_t* dst = lds + stage * kStage + (is_a ? 0 : kRowsA * BK) + row * BK;
+        uint8_t* dst = lds + stage * kStage + (is_a ? 0 : kRows * BK) + row * BK;
         __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)dst, 16, 0, 0);
     };
 
@@ -218,8 +219,8 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
     auto scale_dma = [&](const TileDesc& d) __attribute__((always_inline)) {
         if constexpr (Problem::kVecScales) {
             uint8_t* slot = lds + 2 * STAGE + OUT_STAGING + (ld_seq & kSlotMask) * kSlotBytes + wave * 256;
-            // (a half tile has 128 rows, and the scales may end with them: its upper half repeats the lower one)
-            const int row = (wave * 64 + lane) & (kHalf ? 127 : 255);
+            // (the scales may end with a part's rows: they are repeated)
+            const int row = (wave * 64 + lane) & (kRows - 1);
             __builtin_amdgcn_global_load_lds((gptr_t)(d.sa + row), (lptr_t)slot, 4, 0, 0);
             __builtin_amdgcn_global_load_lds((gptr_t)(d.sb + wave * 64 + lane), (lptr_t)(slot + 1024), 4, 0, 0);
             if constexpr (Problem::kTwoSegments) {
@@ -235,8 +236,8 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
     // its workgroups striding through it; tiles of unequal cost are strided over the whole grid instead
     const typename Problem::Cache cache = pb.prepare();
     int total;
-    if constexpr (kHalf)
-        total = pb.half_tiles();
+    if constexpr (kPart)
+        total = pb.template part_tiles<kRows>();
     else
         total = pb.total_tiles(cache);
     int first_tile, tile_stride, my_tiles;
@@ -262,8 +263,8 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
         return;
     }
     auto my_tile = [&](int idx) __attribute__((always_inline)) {
-        if constexpr (kHalf)
-            return pb.half_tile(first_tile + idx * tile_stride);
+        if constexpr (kPart)
+            return pb.template part_tile<kRows>(first_tile + idx * tile_stride);
         else
             return pb.tile(first_tile + idx * tile_stride, cache);
     };
@@ -319,7 +320,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
         }
         if (ld_kt >= ld_nk) next_load_tile();
     };
-    if constexpr (!kHalf) next_load_tile();
+    if constexpr (!kPart) next_load_tile();
 
     v4f acc[2 * kPasses][NT];
     // D' = B . A^T : the first MFMA operand is the B fragment (its type code goes to cbsz).  `fresh`: the tile's
@@ -367,7 +368,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
     };
 
     // ---- prologue: stages of steps 0 and 1, fragments of step 0 ----------------------------------------
-    if (!kHalf && ld_a != nullptr) {  // uniform
+    if (!kPart && ld_a != nullptr) {  // uniform
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
 #pragma unroll
@@ -381,7 +382,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
     // fragments a step's phase A starts from: A tiles 0-3 and all B tiles of the stage the read addresses point at
     auto read_step_head = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < (WTM < 64 ? WTM / 16 : 4); ++t) {
             read_a(fa_lo[t], t, 0);
             read_a(fa_lo[t], t, 1);
         }
@@ -391,7 +392,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
             read_b(fb[0][t], t, 1);
         }
     };
-    if constexpr (!kHalf) {
+    if constexpr (!kPart) {
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's direct loads have landed
         __syncthreads();
         read_step_head();
@@ -491,17 +492,18 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
             advance_load_cursor();
             ++step;
         };
-        if constexpr (kHalf) {
+        if constexpr (kPart) {
             // A half tile: half the rows of A, hence a third less of a stage, half the accumulators and room for a second set of
             // A fragments too.  So there are three stages, every fragment of a step is read during the step before, and a
             // stage is free for step s + 3 as soon as step s starts: one barrier a step, its loads two steps ahead of
             // their wait, its 24 fragment reads (1140 cycles of LDS for the four waves, against 1024 of MFMAs) spread over
             // all of it.  Without its loads and reads the loop takes 0.53 us a step, with either 0.60, with both 0.65;
             // operands that come from HBM make it 0.85.  One tile per workgroup: nothing is prefetched across tiles, and the
-            // output staging takes the place of the stages.
+            // output staging takes the place of the stages.  A quarter tile is the same with half the MFMAs (512 cycles) for 20
+            // fragment reads and ten loads, 960 cycles of LDS: 0.41-0.54 us a step.
             const uint8_t* a_src = td.a;
             const uint8_t* b_src = td.b + b_wave_shift;
-            constexpr int kStepLoads = kLoadsA + kLoads;
+            constexpr int kStepLoads = kLoadsA + kLoads, kTilesA = WTM / 16, kMma = kTilesA * NT;
             auto fetch = [&](int x, int slot) __attribute__((always_inline)) {  // x-th load of the step a_src / b_src point at
                 dma_one(a_src, b_src, slot, x < kLoadsA ? x : kLoads + x - kLoadsA);
             };
@@ -527,7 +529,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
 #pragma unroll
                 for (int j = 0; j < NT; ++j) acc[i][j] = (v4f){0, 0, 0, 0};
             int slot = 0;
-            auto half_step = [&](int kt, auto set_tag) __attribute__((always_inline)) {
+            auto part_step = [&](int kt, auto set_tag) __attribute__((always_inline)) {
                 constexpr int S = decltype(set_tag)::value;
                 auto& fa = S ? fa_hi : fa_lo;
                 auto& fa_next = S ? fa_lo : fa_hi;
@@ -545,12 +547,17 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
                 }
                 auto body = [&](auto with_loads) __attribute__((always_inline)) {
 #pragma unroll
-                    for (int x = 0; x < 32; ++x) {
-                        const int j = x >> 2, i = x & 3;
+                    for (int x = 0; x < kMma; ++x) {
+                        const int j = x / kTilesA, i = x % kTilesA;
                         mma(fa[i], fb[S][j], acc[i][j], false, i, j);
-                        if (x < 8) read_a(fa_next[x >> 1], x >> 1, x & 1);
-                        if (x >= 8 && x < 24) read_b(fb[S ^ 1][(x - 8) >> 1], (x - 8) >> 1, x & 1);
-                        if (decltype(with_loads)::value && x % 2 == 1 && x / 2 < kStepLoads) fetch(x / 2, slot);
+#pragma unroll
+                        for (int y = x * 32 / kMma; y < (x + 1) * 32 / kMma; ++y) {  // (one read an MFMA, two in a quarter)
+                            if (y < 2 * kTilesA)
+                                read_a(fa_next[y >> 1], y >> 1, y & 1);
+                            else if (y < 2 * kTilesA + 2 * NT)
+                                read_b(fb[S ^ 1][(y - 2 * kTilesA) >> 1], (y - 2 * kTilesA) >> 1, y & 1);
+                            if (decltype(with_loads)::value && y % 2 == 1 && y / 2 < kStepLoads) fetch(y / 2, slot);
+                        }
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 };
@@ -565,10 +572,10 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
             };
             int kt = 0;
             for (; kt + 1 < td.nk; kt += 2) {
-                half_step(kt, std::integral_constant<int, 0>{});
-                half_step(kt + 1, std::integral_constant<int, 1>{});
+                part_step(kt, std::integral_constant<int, 0>{});
+                part_step(kt + 1, std::integral_constant<int, 1>{});
             }
-            if (kt < td.nk) half_step(kt, std::integral_constant<int, 0>{});
+            if (kt < td.nk) part_step(kt, std::integral_constant<int, 0>{});
             __builtin_amdgcn_s_waitcnt(vmcnt(0) & 0xF0FF);
             asm volatile("s_barrier" ::: "memory");  // nobody reads the stages any more
         } else if (td.nk > 0) {
@@ -612,7 +619,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
         // (the copies below are opaque to the compiler's hazard handling: the last MFMA has retired after these)
         MI8_TL(2);
         asm volatile("s_nop 15\n\ts_nop 15");
-        uint8_t* stg = lds + (kHalf ? 0 : 2 * STAGE) + wave * 4096;
+        uint8_t* stg = lds + (kPart ? 0 : 2 * STAGE) + wave * 4096;
         const uint32_t stg_lds = (uint32_t)(uintptr_t)(lptr_t)stg;
         const bool zero_tile = td.nk == 0;  // nothing accumulated; the scales may be unset
         const uint8_t* sc_slot = lds + 2 * STAGE + OUT_STAGING + (cp_seq & kSlotMask) * kSlotBytes;
@@ -927,7 +934,7 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
         // again here makes those 96 registers free during the epilogue, which otherwise spills (and every
         // reload from scratch waits on the in-order vector memory counter, i.e. on the stores above).
         __builtin_amdgcn_sched_barrier(0);  // (or the scheduler moves these reads up into the epilogue)
-        if constexpr (!kHalf) read_step_head();
+        if constexpr (!kPart) read_step_head();
         MI8_TL(12);
         MI8_TL_NEXT_TILE();
     }
@@ -951,19 +958,22 @@ __device__ __forceinline__ void m16_tiles(const Problem& pb, const int block, co
     }
 }
 
-// Workgroups [0, whole_blocks) walk the whole tiles, the others have a half tile each; the dispatcher starts those as compute
-// units fall free.  (Two separate bodies: as branches of one tile loop they share 256 accumulators across control flow and the
+// Workgroups [0, whole_blocks) walk the whole tiles, the others have a half or a quarter of a tile each; the dispatcher starts
+// those as compute units fall free.  (Separate bodies: as branches of one tile loop they share 256 accumulators across control flow and the
 // kernel spills.)
 template <typename Problem, int CBSZ_A, int BLGP_B>
 __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
 {
-    if constexpr (Problem::kHalves) {
-        if ((int)blockIdx.x < pb.rows.whole_blocks)
-            m16_tiles<Problem, CBSZ_A, BLGP_B, false>(pb, (int)blockIdx.x, pb.rows.whole_blocks);
+    if constexpr (Problem::kParts) {
+        const int halves = (int)blockIdx.x - pb.rows.whole_blocks, quarters = halves - pb.rows.half_blocks;
+        if (halves < 0)
+            m16_tiles<Problem, CBSZ_A, BLGP_B, BM>(pb, (int)blockIdx.x, pb.rows.whole_blocks);
+        else if (quarters < 0)
+            m16_tiles<Problem, CBSZ_A, BLGP_B, BM / 2>(pb, halves, pb.rows.half_blocks);
         else
-            m16_tiles<Problem, CBSZ_A, BLGP_B, true>(pb, (int)blockIdx.x - pb.rows.whole_blocks, (int)gridDim.x - pb.rows.whole_blocks);
+            m16_tiles<Problem, CBSZ_A, BLGP_B, BM / 4>(pb, quarters, pb.rows.quarter_blocks);
     } else {
-        m16_tiles<Problem, CBSZ_A, BLGP_B, false>(pb, (int)blockIdx.x, (int)gridDim.x);
+        m16_tiles<Problem, CBSZ_A, BLGP_B, BM>(pb, (int)blockIdx.x, (int)gridDim.x);
     }
 }
 
@@ -990,7 +1000,7 @@ int launch(const Problem& pb, int max_tiles, bool persistent, hipStream_t st)
     if (int rc = reserve_dynamic_lds(reinterpret_cast<const void*>(kern), LDS_BYTES, configured, "mi8 16x16x128 GEMM"))
         return rc;
     int blocks = persistent ? persistent_blocks(max_tiles) : max_tiles;
-    if constexpr (Problem::kHalves) blocks = pb.rows.blocks();
+    if constexpr (Problem::kParts) blocks = pb.rows.blocks();
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kThreads), LDS_BYTES, st, pb);
     return launch_status("mi8 16x16x128 GEMM");
 }
@@ -1009,13 +1019,16 @@ int launch_typed(const Problem& pb, int max_tiles, bool persistent, int a_dtype,
 
 namespace {
 
+// us per K step and besides for a quarter tile (0.41 a step with half of the compute units busy, 0.54 with all of them)
+constexpr float kQuarterStep = 0.48f, kQuarterTile = 2.5f;
+
 // Which tiles of a dense problem are halves (tiles_n columns of tiles, nk K steps), and g.tiles_m = pairs of half rows.
 // Splitting tiles of a partial last round pays when its halves fit into one round: 2048 x 11008 x 4096 is 344 tiles, two
 // rounds of 256 workgroups for 1.34 rounds of work; as 256 whole and 176 half tiles it takes 81 us in a loop of its own
 // (92 right after the casts that write its operands) instead of 87.  4096 x 2048 x 8192, 128 tiles, is 256 half tiles: 55 us
 // instead of 69.  The matrix pipe is busy 68 % and 67 % of the cycles.  (A step of a half tile takes 0.65 us with its
 // operands in the memory-side cache, 0.85 us from HBM; a whole tile's 1.0 us, 1.35 us when all compute units have one.)
-HalfRows plan_halves(GemmArgs& g, const int cus, int most_halves = 1 << 30)
+RowPlan plan_halves(GemmArgs& g, const int cus, int most_halves = 1 << 30)
 {
     const int half_rows = (g.M + 127) / 128;
     g.tiles_m = half_rows / 2;
@@ -1031,7 +1044,7 @@ HalfRows plan_halves(GemmArgs& g, const int cus, int most_halves = 1 << 30)
     };
     if (odd > most_halves) {
         g.tiles_m = (g.M + BM - 1) / BM;
-        return HalfRows{g.tiles_m * g.tiles_n, 0, 0, persistent_blocks(g.tiles_m * g.tiles_n), 0};
+        return RowPlan{g.tiles_m * g.tiles_n, 0, 0, persistent_blocks(g.tiles_m * g.tiles_n), 0, 0, 0, 0};
     }
     int split = 0;
     float best = longest(0);
@@ -1041,12 +1054,81 @@ HalfRows plan_halves(GemmArgs& g, const int cus, int most_halves = 1 << 30)
             split = c;
             best = longest(c);
         }
-    return HalfRows{pairs - split, 2 * split + odd, 2 * split, persistent_blocks(pairs - split), (2 * split + odd + 7) / 8 * 8};
+    return RowPlan{pairs - split, 2 * split + odd, 2 * split, persistent_blocks(pairs - split), (2 * split + odd + 7) / 8 * 8, 0, 0, 0};
+}
+
+// us until the last of `cus` units is done: whole tiles in rounds, then every half and quarter to the unit that is free first
+float makespan(const RowPlan& p, const int cus, const float steps)
+{
+    struct { float load; int units; } have[5];  // (units that are free at the same time)
+    const int q = p.n_full / cus, r = p.n_full % cus;
+    const float whole = steps * 1.05f + 5.0f;
+    int n = 1;
+    have[0] = {q * whole, cus - r};
+    if (r) have[n++] = {(q + 1) * whole, r};
+    auto deal = [&](int left, float each) {
+        while (left > 0) {
+            int first = 0;
+            for (int i = 1; i < n; ++i)
+                if (have[i].load < have[first].load) first = i;
+            if (left >= have[first].units) {
+                left -= have[first].units;
+                have[first].load += each;
+            } else {
+                have[first].units -= left;
+                have[n++] = {have[first].load + each, left};
+                left = 0;
+            }
+        }
+    };
+    deal(p.n_half, steps * 0.78f + 3.5f);
+    deal(p.n_quarter, steps * kQuarterStep + kQuarterTile);
+    float last = 0.0f;
+    for (int i = 0; i < n; ++i) last = have[i].load > last ? have[i].load : last;
+    return last;
+}
+
+// The same with quarter tiles where they shorten it: a row of them at the end instead of a half row that is less than half
+// full, and quarters of the last whole tiles.  us with halves only / with quarters: both projections and SwiGLU of 777 x 11008 x
+// 4096, whose 258 whole tiles and 86 pieces of nine rows are 256 whole tiles and 94 quarters, 85.4 / 71.0; 4160 x 4096 x 4096 (a row
+// of quarters beside whole tiles) 69.6 / 63.6.  A product of quarters alone, 1537 x 2048 x 2048, takes 12.7 (15.7 in halves), as
+// long as on ring tiles; 1024 x 4096 x 4096 21.0 (26.5), ring tiles 19.9.
+RowPlan plan_parts(GemmArgs& g, const int cus, int most_parts = 1 << 30)
+{
+    RowPlan best = plan_halves(g, cus, most_parts);
+    const float steps = (float)(g.K / BK);
+    const int quarter_rows = (g.M + 63) / 64, tail = quarter_rows & 3, rows = quarter_rows >> 2;
+    if (best.n_half == 0 && tail == 0) return best;  // (whole tiles alone are best)
+    const int pairs = rows * g.tiles_n, half_row = (tail >> 1) * g.tiles_n, quarter_row = (tail & 1) * g.tiles_n;
+    float time = makespan(best, cus, steps);
+    bool better = false;
+    const int splits[3] = {0, pairs % cus, pairs < cus ? pairs : pairs % cus + cus};
+    for (int c = 0; c < 3; ++c) {
+        const int split = splits[c];
+        if ((c && (split == 0 || split == splits[c - 1])) || split > pairs) continue;
+        for (int part = 0; part <= (split ? 4 : 0); ++part) {  // a share of the split tiles in quarters, the others in halves
+            const int fours = split * part / 4, twos = split - fours;
+            RowPlan p{pairs - split, 2 * twos + half_row, 2 * twos, persistent_blocks(pairs - split), 0, 4 * fours + quarter_row, 4 * fours, 0};
+            if (p.n_half + p.n_quarter > most_parts) continue;
+            const float t = makespan(p, cus, steps);
+            if (t < 0.97f * time) {
+                time = t;
+                best = p;
+                better = true;
+            }
+        }
+    }
+    if (better) {
+        g.tiles_m = rows;
+        best.half_blocks = (best.n_half + 7) / 8 * 8;
+        best.quarter_blocks = (best.n_quarter + 7) / 8 * 8;
+    }
+    return best;
 }
 
 }  // namespace
 
-float m16_cost(int64_t M, int64_t N, int64_t K)
+float m16_cost(int64_t M, int64_t N, int64_t K, bool quarters)
 {
     // Whether a product is cut along K hangs on this, and with it the order of its sums: the 256 units of a whole chip, not
     // those of the device at hand, so that the sizes alone decide.  Absolute times, to be set against another kernel's: a
@@ -1058,19 +1140,29 @@ float m16_cost(int64_t M, int64_t N, int64_t K)
     g.N = (int)N;
     g.K = (int)K;
     g.tiles_n = (int)((N + BN - 1) / BN);
-    const HalfRows h = plan_halves(g, cus);
+    const RowPlan p = quarters ? plan_parts(g, cus) : plan_halves(g, cus);
     const float steps = (float)(K / BK);
-    const int q = h.n_full / cus, r = h.n_full % cus, halves = (h.n_half + cus - 1) / cus;
+    const int q = p.n_full / cus, r = p.n_full % cus;
     float t = 3.0f + q * (steps * 1.35f + 5.0f);
     if (r) t += steps * (1.0f + 0.35f * (r > cus / 2 ? (float)(2 * r - cus) / cus : 0.0f)) + 5.0f;
-    if (halves && !(r && h.n_half <= cus - r)) t += halves * (steps * 0.78f + 3.5f);
+    int idle = r ? cus - r : 0;  // units that wait for the others
+    auto add = [&](int n, float each) {
+        if (n > idle) {
+            const int rounds = (n + cus - 1) / cus;
+            t += rounds * each;
+            idle += rounds * cus;
+        }
+        idle -= n;
+    };
+    add(p.n_half, steps * 0.78f + 3.5f);
+    add(p.n_quarter, steps * kQuarterStep + kQuarterTile);
     return t;
 }
 
 int launch_m16(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st)
 {
     g.tiles_n = (g.N + BN - 1) / BN;
-    const HalfRows rows = plan_halves(g, num_compute_units());
+    const RowPlan rows = plan_parts(g, num_compute_units());
     if (g.c_f32) {
         if (g.sa_vec) return launch_typed(DenseProblem<true, false, false, true>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);
         return launch_typed(DenseProblem<false, false, false, true>{g, g.lda, g.ldb, g.ldc, rows}, 0, true, a_dtype, b_dtype, st);
@@ -1086,7 +1178,7 @@ int launch_m16(GemmArgs& g, int a_dtype, int b_dtype, hipStream_t st)
 int launch_m16_codes(GemmArgs& g, uint16_t* codes, int a_dtype, int b_dtype, hipStream_t st)
 {
     g.tiles_n = (g.N + BN - 1) / BN;
-    const HalfRows rows = plan_halves(g, num_compute_units());
+    const RowPlan rows = plan_parts(g, num_compute_units());
     DenseProblem<false, false, true> pb{g, g.lda, g.ldb, g.ldc, rows};
     pb.codes = codes;
     return launch_typed(pb, 0, true, a_dtype, b_dtype, st);
@@ -1098,14 +1190,14 @@ int m16_swiglu_slots(int64_t M, int64_t H, int64_t K)
     g.M = (int)M;
     g.K = (int)K;
     g.tiles_n = (int)((H + 127) / 128);
-    return 4 * plan_halves(g, num_compute_units(), 256).blocks();
+    return 4 * plan_parts(g, num_compute_units(), 256).blocks();
 }
 
 int launch_m16_swiglu(GemmArgs& g, const uint8_t* b3, const float* sb3, uint16_t* x3, uint16_t* h, uint32_t* h_slots,
                       int* n_slots, uint16_t* x_codes, int a_dtype, int b_dtype, hipStream_t st)
 {
     g.tiles_n = (g.N + 127) / 128;
-    const HalfRows rows = plan_halves(g, num_compute_units(), 256);  // (4 partial maxima per workgroup, MI8_AMAX_SLOTS in all)
+    const RowPlan rows = plan_parts(g, num_compute_units(), 256);  // (4 partial maxima per workgroup, MI8_AMAX_SLOTS in all)
     SwigluProblem pb{g, g.lda, g.ldb, g.ldc, rows, (int64_t)(b3 - g.B), (int64_t)(x3 - reinterpret_cast<uint16_t*>(g.C)),
                      (int64_t)(h - reinterpret_cast<uint16_t*>(g.C)), sb3, h_slots, x_codes};
     *n_slots = 4 * rows.blocks();  // one partial maximum per wave of the grid

@@ -32,30 +32,36 @@ struct TileDesc {
 
 struct NoCache {};
 
-// Rows of a kHalves problem.  The M rows are ceil(M / 128) half rows of tiles: pairs of them make the 256-row tiles, an odd
-// one at the end is a row of half tiles (128 x 256).  The last tiles of the order may be split into their two halves, so
-// that a partial last round of whole tiles becomes a round of half tiles on twice as many compute units.  Half tiles
-// are numbered by themselves: the halves of the split pairs, then the odd half row.  Every tile is complete: the last one
-// of either kind is shifted back over its predecessor (M >= 256), recomputes the overlap with the same K order and
+// Rows of a kParts problem.  g.tiles_m rows of whole tiles (256 rows) are followed by at most one row of half tiles (128 x 256)
+// and one of quarters (64 x 256).  The last whole tiles of the order may be split, some into their halves, the last ones into
+// their quarters, so that a partial last round of whole tiles becomes a round of smaller ones on more compute units.  Halves and
+// quarters are numbered by themselves: those of the split tiles, then the row at the end.  Every tile is complete: one that
+// would pass the last row is shifted back over its predecessor (M >= 256), recomputes the overlap with the same K order and
 // rewrites identical values.
-struct HalfRows {
-    int n_full;       // whole tiles
-    int n_half;       // half tiles
-    int n_split;      // how many of these are halves of split tiles (the rest: the odd half row)
-    int whole_blocks;  // workgroups that walk the whole tiles
-    int half_blocks;   // workgroups with a half tile each
-    __host__ __device__ int blocks() const { return whole_blocks + half_blocks; }
-    __device__ __forceinline__ void half(const GemmArgs& g, int i, int& m0, int& tn) const
+struct RowPlan {
+    int n_full;         // whole tiles
+    int n_half;         // half tiles
+    int n_split;        // how many of these are halves of split tiles (the rest: the row of half tiles)
+    int whole_blocks;   // workgroups that walk the whole tiles
+    int half_blocks;    // workgroups with a half tile each
+    int n_quarter;      // the same for quarters, those of split tiles first
+    int n_split4;
+    int quarter_blocks;
+    __host__ __device__ int blocks() const { return whole_blocks + half_blocks + quarter_blocks; }
+    template <int kRows>
+    __device__ __forceinline__ void part(const GemmArgs& g, int i, int& m0, int& tn) const
     {
-        int tm, row;
-        if (i < n_split) {
-            tile_coords(g, n_full + (i >> 1), tm, tn);
-            row = 2 * tm + (i & 1);
+        constexpr int kPer = BM / kRows;
+        const int split = kRows == BM / 2 ? n_split : n_split4;
+        int tm, row0;
+        if (i < split) {
+            tile_coords(g, n_full + (kRows == BM / 2 ? 0 : n_split / 2) + i / kPer, tm, tn);
+            row0 = tm * BM + i % kPer * kRows;
         } else {
-            tn = i - n_split;
-            row = 2 * g.tiles_m;
+            tn = i - split;
+            row0 = g.tiles_m * BM + (kRows == BM / 4 && n_half > n_split ? BM / 2 : 0);
         }
-        m0 = (row * 128 + 128 <= g.M) ? row * 128 : g.M - 128;
+        m0 = row0 + kRows <= g.M ? row0 : g.M - kRows;
     }
 };
 
@@ -69,9 +75,9 @@ template <bool VEC, bool ACC = false, bool CODES = false, bool F32 = false>
 struct DenseProblem {
     GemmArgs g;
     int64_t lda, ldb, ldc;
-    HalfRows rows;
+    RowPlan rows;
     uint16_t* codes = nullptr;  // (CODES)
-    static constexpr bool kHalves = true;
+    static constexpr bool kParts = true;
     static constexpr bool kVecScales = VEC;  // both scales are vectors (per row / per column) or both single
     static constexpr bool kAccumulate = ACC;  // C += the rounded product
     static constexpr bool kOutCodes = CODES;
@@ -87,18 +93,20 @@ struct DenseProblem {
     __device__ __forceinline__ float single_sa() const { return g.sa[0]; }
     __device__ __forceinline__ float single_sb() const { return g.sb[0]; }
     __device__ __forceinline__ int total_tiles(const Cache&) const { return rows.n_full; }
-    __device__ __forceinline__ int half_tiles() const { return rows.n_half; }
+    template <int kRows>
+    __device__ __forceinline__ int part_tiles() const { return kRows == BM / 2 ? rows.n_half : rows.n_quarter; }
     __device__ __forceinline__ TileDesc tile(int t, const Cache&) const
     {
         int tm, tn;
         tile_coords(g, t, tm, tn);
         return at((tm * BM + BM <= g.M) ? tm * BM : g.M - BM, tn, BM);
     }
-    __device__ __forceinline__ TileDesc half_tile(int i) const
+    template <int kRows>
+    __device__ __forceinline__ TileDesc part_tile(int i) const
     {
         int m0, tn;
-        rows.half(g, i, m0, tn);
-        return at(m0, tn, BM / 2);
+        rows.part<kRows>(g, i, m0, tn);
+        return at(m0, tn, kRows);
     }
     __device__ __forceinline__ TileDesc at(int m0, int tn, int height) const
     {
@@ -126,7 +134,7 @@ struct DenseProblem {
 struct SwigluProblem {
     GemmArgs g;             // A, B = B1, C = x1; N = H; tiles_n counts 128-column tiles; sa, sb = scale of A, of B1
     int64_t lda, ldb, ldc;
-    HalfRows rows;
+    RowPlan rows;
     int64_t b3_offset;      // bytes from B1 to B3
     int64_t x3_offset;      // elements from x1 to x3 and to h (same pitch ldc)
     int64_t h_offset;
@@ -134,24 +142,26 @@ struct SwigluProblem {
     uint32_t* h_slots;      // [4 * workgroups] partial maxima of |h| (float32 bit patterns)
     uint16_t* x_codes;      // null, or [H / 64][M] codes of the larger of x1 and x3 per row segment (H % 64 == 0)
     static constexpr bool kVecScales = false, kAccumulate = false, kSwiglu = true, kOutCodes = false, kOutF32 = false;
-    static constexpr bool kMaskRows = false, kXcdRanges = true, kMfmaScale = false, kTwoSegments = false, kHalves = true;
+    static constexpr bool kMaskRows = false, kXcdRanges = true, kMfmaScale = false, kTwoSegments = false, kParts = true;
     using Cache = NoCache;
     __device__ __forceinline__ Cache prepare() const { return Cache{}; }
     __device__ __forceinline__ float single_sa() const { return g.sa[0]; }
     __device__ __forceinline__ float single_sb() const { return g.sb[0]; }
     __device__ __forceinline__ int total_tiles(const Cache&) const { return rows.n_full; }
-    __device__ __forceinline__ int half_tiles() const { return rows.n_half; }
+    template <int kRows>
+    __device__ __forceinline__ int part_tiles() const { return kRows == BM / 2 ? rows.n_half : rows.n_quarter; }
     __device__ __forceinline__ TileDesc tile(int t, const Cache&) const
     {
         int tm, tn;
         tile_coords(g, t, tm, tn);
         return at((tm * BM + BM <= g.M) ? tm * BM : g.M - BM, tn, BM);
     }
-    __device__ __forceinline__ TileDesc half_tile(int i) const
+    template <int kRows>
+    __device__ __forceinline__ TileDesc part_tile(int i) const
     {
         int m0, tn;
-        rows.half(g, i, m0, tn);
-        return at(m0, tn, BM / 2);
+        rows.part<kRows>(g, i, m0, tn);
+        return at(m0, tn, kRows);
     }
     __device__ __forceinline__ TileDesc at(int m0, int tn, int height) const
     {
@@ -241,7 +251,7 @@ struct GroupedProblem {
     int N, K, tiles_n;
     const float* sa;
     const float* sb;
-    static constexpr bool kVecScales = true, kMaskRows = true, kXcdRanges = true, kHalves = false;
+    static constexpr bool kVecScales = true, kMaskRows = true, kXcdRanges = true, kParts = false;
     using Cache = GroupCache;
     __device__ __forceinline__ Cache prepare() const { return build_group_cache<BM>(sizes, E, T); }
     __device__ __forceinline__ int total_tiles(const Cache& c) const
@@ -281,7 +291,7 @@ struct GroupedProblem {
 // the column scales a group stride; K1, K2 are multiples of 256 (an even number of steps each).
 struct GroupedDualProblem {
     static constexpr bool kAccumulate = false, kSwiglu = false, kOutCodes = false, kOutF32 = false, kMfmaScale = true, kTwoSegments = true;
-    static constexpr bool kVecScales = true, kMaskRows = true, kXcdRanges = true, kHalves = false;
+    static constexpr bool kVecScales = true, kMaskRows = true, kXcdRanges = true, kParts = false;
     GroupedProblem<false> first;  // A1, B1, C, pitches, sizes, N, K = K1, sa1, sb1
     int64_t lda, ldb, ldc;        // (copies of first's, under the names the kernel reads)
     const uint8_t* A2;
@@ -334,7 +344,7 @@ struct GroupedWgradProblem {
     int N, Kl, tiles_n, tiles_k;
     const float* sa;  // [E, N]
     const float* sb;  // [E, Kl]
-    static constexpr bool kVecScales = true, kMaskRows = false, kXcdRanges = false, kHalves = false;
+    static constexpr bool kVecScales = true, kMaskRows = false, kXcdRanges = false, kParts = false;
     static constexpr bool kAccumulate = false, kSwiglu = false, kOutCodes = false, kOutF32 = false, kMfmaScale = false, kTwoSegments = false;
     using Cache = WgradCache;
     __device__ __forceinline__ Cache prepare() const

@@ -496,6 +496,23 @@ def test_half_tiles_of_the_fused_swiglu_launch(dev, mhk):
         assert torch.equal(codes[0], ops.rowseg_max_codes(x1, x3))
 
 
+# quarter tiles (64 x 256): all of them, a row of them at the end (whole, and shifted back), whole and half tiles beside them
+@pytest.mark.parametrize("mnk", [(450, 512, 384), (777, 1032, 256), (4160, 4096, 128), (3000, 5632, 256)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
+def test_quarter_tiles_of_the_persistent_kernel(dev, mnk, vec):
+    test_half_tiles_of_the_persistent_kernel(dev, mnk, vec)
+
+
+@pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
+def test_quarter_tiles_accumulate_as_an_add(dev, vec):
+    test_persistent_kernel_accumulates_as_an_add(dev, (3328, 5632, 256), vec)  # 256 whole tiles and 120 quarters
+
+
+@pytest.mark.parametrize("mhk", [(450, 520, 128), (777, 11008, 384), (3000, 5632, 256)], ids=lambda s: "x".join(map(str, s)))
+def test_quarter_tiles_of_the_fused_swiglu_launch(dev, mhk):
+    test_half_tiles_of_the_fused_swiglu_launch(dev, mhk)
+
+
 def test_tile_timeline_stays_in_its_buffer(dev):
     """A plan with half tiles launches more workgroups than the time stamps have room for: only the first 256, which walk
     whole tiles, record theirs."""
