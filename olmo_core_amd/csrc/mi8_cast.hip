@@ -345,7 +345,6 @@ struct GroupedCastArgs {
     int64_t src_rows;
     const void* gather_w;  // optional weight per slot (weighted gather), of element type gather_w_dtype
     int gather_w_dtype;
-    bool stream;
 };
 
 // Tile p of the padded row space (128 rows each; group e owns ceil(m_e / 128) consecutive tiles) -> its group,
@@ -750,7 +749,7 @@ __global__ __launch_bounds__(kThreads) void grouped_tile_cast_kernel(GroupedCast
     for (int i = 0; i < 8; ++i) sc[i] = s_scale[8 * cl + i];
     const int64_t dst0 = (int64_t)kTile * rt;
     if (GATHER && a.gather_w) values.scale_rows(rows.w, col0 + 8 * cl < a.cols);
-    tile_quantise<FP8, SW>(values, row_end, a.cols, row0, col0, sc, nullptr, 0, a.out_t, a.ld_t, dst0, a.ld_t, lds_t, a.stream, a.out_r, a.ld_r,
+    tile_quantise<FP8, SW>(values, row_end, a.cols, row0, col0, sc, nullptr, 0, a.out_t, a.ld_t, dst0, a.ld_t, lds_t, true, a.out_r, a.ld_r,
                            s_row_scale, row0);
 }
 
@@ -1332,7 +1331,7 @@ int grouped_cast_launch(const char* what, const void* x, int hp_dtype, int64_t T
     const bool pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
     GroupedCastArgs a{x, T, cols, group_sizes, num_groups, pow2, amax_ws, (uint8_t*)out_t, ld_t, scale_out,
                       out_rows ? row_amax_ws : nullptr, (uint8_t*)out_rows, ld_rows, row_scale_out, gather, top_k, src_rows, gather_w,
-                      gather_w_dtype, streams_outputs(T * cols * (out_rows ? 2 : 1))};
+                      gather_w_dtype};
     hipStream_t st = (hipStream_t)stream;
     dim3 grid((unsigned)ceil_div(cols, kTile), (unsigned)ptiles);
     int rc = MI8_OK;
