@@ -240,3 +240,22 @@ def test_routed_layer_without_gradients_has_the_same_bits(dev, tokens, keep):
     with torch.no_grad():
         got = layer(x, w, idx, sizes)
     assert torch.equal(got, want.detach())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=str)
+@pytest.mark.parametrize("tokens,top_k,hidden", [(1, 1, 8), (48, 8, 2048), (3, 64, 2056), (100, 7, 4096), (1024, 8, 264), (8192, 1, 16)], ids=str)
+@pytest.mark.parametrize("weighted", [False, True])
+def test_scatter_of_few_slots_equals_that_of_many(dev, tokens, top_k, hidden, weighted, dtype):
+    """The one-launch scatter against the general one, which the same problem several times over goes to; some slots unfilled."""
+    g = torch.Generator().manual_seed(tokens + hidden)
+    n = tokens * top_k
+    x = torch.randn(n, hidden, generator=g).to(dtype).to(dev)
+    w = torch.rand(n, generator=g).to(dtype).to(dev) if weighted else None
+    indices = torch.randperm(n, generator=g).int()
+    if n > 64:
+        indices[3], indices[n // 2], indices[n - 1] = -1, n + 2, torch.iinfo(torch.int32).max
+    times = 8192 // n + 1
+    many = torch.cat([torch.where((indices >= 0) & (indices < n), indices + n * i, -1) for i in range(times)])
+    got = ops._scatter(x, indices.to(dev), w, top_k)
+    want = ops._scatter(x.repeat(times, 1), many.int().to(dev), w.repeat(times) if weighted else None, top_k)
+    assert torch.equal(got, want[:tokens])
