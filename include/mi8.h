@@ -477,6 +477,12 @@ int64_t mi8_moe_sort_slots_max(void);
 int mi8_moe_sort_slots(const void* ids, int ids_are_64, int64_t n, const int64_t* sizes, int32_t experts, int32_t* indices,
                        int32_t* bin_ids, int32_t* bins, void* stream);
 
+/* The same for any n < 2^30 and up to 256 experts.  workspace: int32 [mi8_moe_sort_workspace_words(n, experts)] (0: not taken),
+ * overwritten. */
+int64_t mi8_moe_sort_workspace_words(int64_t n, int32_t experts);
+int mi8_moe_sort_many_slots(const void* ids, int ids_are_64, int64_t n, const int64_t* sizes, int32_t experts, int32_t* workspace,
+                            int32_t* indices, int32_t* bin_ids, int32_t* bins, void* stream);
+
 /* out[i, :] = x[indices[i] / top_k, :] * weights[indices[i]]           out: [tokens * top_k, hidden] */
 int mi8_moe_gather(const void* x, int dtype, int64_t tokens, int64_t hidden, const int32_t* indices,
                    const void* weights, int w_dtype, int32_t top_k, void* out, void* stream);

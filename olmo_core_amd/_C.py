@@ -88,6 +88,11 @@ _SIGNATURES = {
         c_int,
         [c_void_p, c_int, c_int64, c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_void_p],
     ),
+    "mi8_moe_sort_workspace_words": (c_int64, [c_int64, c_int32]),
+    "mi8_moe_sort_many_slots": (
+        c_int,
+        [c_void_p, c_int, c_int64, c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
+    ),
     "mi8_moe_gather_cast_rows": (
         c_int,
         [c_void_p, c_int64, c_int64, c_void_p, c_int32, c_uint32, c_void_p, c_int64, c_void_p, c_void_p],

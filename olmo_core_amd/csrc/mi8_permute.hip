@@ -495,10 +495,26 @@ int launch_wgrad(PermuteArgs& a, int dtype, int64_t rows, hipStream_t st)
 // have its id or a smaller one, plus the number of slots after it with a smaller one.  A workgroup places 64 slots, one
 // per lane; its 16 waves count over a sixteenth of the ids each (wave-uniform, so scalar loads and two vector
 // instructions an id).  A call with few tokens is a chain of short launches: the conversion, sort, prefix sum and their
-// copies were eleven of them.  Counting is n^2, so larger inputs stay with the radix sort.  us on the device, this and the
+// copies were eleven of them.  Counting is n^2, so larger inputs have a sort of their own.  us on the device, this and the
 // chain it replaces: 384 slots 3.6 / 27, 2048 7.4 / 30, 8192 15.8 / 37.
 constexpr int kSortThreads = 1024;
 constexpr int64_t kSortSlots = 8192;
+
+// the inclusive prefix sums of the experts' counts, by one wave
+__device__ __forceinline__ void write_bins(const int64_t* __restrict__ sizes, int experts, int32_t* __restrict__ bins, int lane)
+{
+    int64_t sum = 0;
+    for (int base = 0; base < experts; base += 64) {
+        int64_t v = base + lane < experts ? sizes[base + lane] : 0;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int64_t o = __shfl_up(v, d, 64);
+            if (lane >= d) v += o;
+        }
+        if (base + lane < experts) bins[base + lane] = (int32_t)(sum + v);
+        sum += __shfl(v, 63, 64);
+    }
+}
 
 template <typename ID>
 __global__ __launch_bounds__(kSortThreads) void sort_slots_kernel(const ID* __restrict__ ids, int n,
@@ -533,25 +549,125 @@ __global__ __launch_bounds__(kSortThreads) void sort_slots_kernel(const ID* __re
         indices[at] = e;
         bin_ids[at] = id;
     }
-    if (wave == 1 && blockIdx.x == 0) {  // the inclusive prefix sums of the experts' counts
-        int64_t sum = 0;
-        for (int base = 0; base < experts; base += 64) {
-            int64_t v = base + lane < experts ? sizes[base + lane] : 0;
+    if (wave == 1 && blockIdx.x == 0) write_bins(sizes, experts, bins, lane);
+}
+
+// The same for more slots: a stable counting sort in two launches, which count the ids of every 1024 slots and place them.  (A
+// radix sort of 131072 slots with its conversions and the scan of the sizes is 16 dependent launches, 93 us; with these two a step of 16384 tokens takes 67 us less.)  An id that
+// names no expert sorts as any other number would: counted, over all slots, for every such slot.
+constexpr int kSortExperts = 256;  // (16 tables of that many counts in LDS)
+
+__device__ __forceinline__ int sort_bucket(int32_t id, int experts) { return id < 0 ? 0 : id >= experts ? experts + 1 : id + 1; }
+
+template <typename ID>
+__global__ __launch_bounds__(kSortThreads) void count_slots_kernel(const ID* __restrict__ ids, int n, int experts, int32_t* __restrict__ counts)
+{
+    __shared__ int32_t count[kSortExperts + 2];
+    const int tid = threadIdx.x, e = (int)blockIdx.x * kSortThreads + tid;
+    if (tid < experts + 2) count[tid] = 0;
+    __syncthreads();
+    if (e < n) atomicAdd(&count[sort_bucket((int32_t)ids[e], experts)], 1);
+    __syncthreads();
+    if (tid < experts + 2) counts[(int64_t)blockIdx.x * (experts + 2) + tid] = count[tid];
+}
+
+template <typename ID>
+__global__ __launch_bounds__(kSortThreads) void place_slots_kernel(const ID* __restrict__ ids, int n, const int64_t* __restrict__ sizes,
+                                                                   int experts, const int32_t* __restrict__ counts,
+                                                                   int32_t* __restrict__ indices, int32_t* __restrict__ bin_ids,
+                                                                   int32_t* __restrict__ bins)
+{
+    constexpr int kWaves = kSortThreads / 64;
+    __shared__ int32_t of_wave[kWaves][kSortExperts + 2], before[kSortExperts + 2], total[kSortExperts + 2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, buckets = experts + 2;
+    for (int b = tid; b < kWaves * (kSortExperts + 2); b += kSortThreads) (&of_wave[0][0])[b] = 0;
+    if (tid < buckets) before[tid] = total[tid] = 0;
+    __syncthreads();
+    // slots of each bucket in the blocks before this one and in all: as many threads a bucket as there are
+    const int parts = kSortThreads / buckets, part = tid / buckets, bucket = tid - part * buckets;
+    if (part < parts) {
+        int32_t sum = 0, mine = 0;
+#pragma unroll 4
+        for (int b = part; b < (int)gridDim.x; b += parts) {
+            const int32_t c = counts[(int64_t)b * buckets + bucket];
+            sum += c;
+            if (b < (int)blockIdx.x) mine += c;
+        }
+        atomicAdd(&total[bucket], sum);
+        atomicAdd(&before[bucket], mine);
+    }
+    // place among the wave's slots of one bucket
+    const int e = (int)blockIdx.x * kSortThreads + tid;
+    const int32_t id = e < n ? (int32_t)ids[e] : 0;
+    const int b = sort_bucket(id, experts);
+    uint64_t same = __ballot(e < n);
+    for (int bit = 0; (buckets - 1) >> bit; ++bit) {
+        const uint64_t set = __ballot((b >> bit) & 1);
+        same &= (b >> bit) & 1 ? set : ~set;
+    }
+    const int rank = __popcll(same & (((uint64_t)1 << lane) - 1));
+    if (e < n && rank == 0) of_wave[wave][b] = __popcll(same);
+    __syncthreads();
+    if (wave == 0) {  // where each bucket starts
+        int32_t sum = 0;
+        for (int base = 0; base < buckets; base += 64) {
+            const int32_t own = base + lane < buckets ? total[base + lane] : 0;
+            int32_t v = own;
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) {
-                const int64_t o = __shfl_up(v, d, 64);
+                const int32_t o = __shfl_up(v, d, 64);
                 if (lane >= d) v += o;
             }
-            if (base + lane < experts) bins[base + lane] = (int32_t)(sum + v);
+            if (base + lane < buckets) before[base + lane] += sum + v - own;
             sum += __shfl(v, 63, 64);
         }
     }
+    __syncthreads();
+    if (e < n) {
+        int32_t at = before[b] + rank;
+        for (int w = 0; w < wave; ++w) at += of_wave[w][b];
+        if (b == 0 || b == experts + 1) {
+            at = b == 0 ? 0 : n - total[b];
+            for (int j = 0; j < n; ++j) {
+                const int32_t other = (int32_t)ids[j];
+                if (sort_bucket(other, experts) == b && (other < id || (other == id && j < e))) ++at;
+            }
+        }
+        indices[at] = e;
+        bin_ids[at] = id;
+    }
+    if (wave == 1 && blockIdx.x == 0) write_bins(sizes, experts, bins, lane);
 }
 
 }  // namespace
 }  // namespace mi8
 
 using namespace mi8;
+
+extern "C" int64_t mi8_moe_sort_workspace_words(int64_t n, int32_t experts)
+{
+    return n > 0 && n < (1 << 30) && experts > 0 && experts <= kSortExperts ? ceil_div(n, kSortThreads) * (experts + 2) : 0;
+}
+
+extern "C" int mi8_moe_sort_many_slots(const void* ids, int ids_are_64, int64_t n, const int64_t* sizes, int32_t experts,
+                                       int32_t* workspace, int32_t* indices, int32_t* bin_ids, int32_t* bins, void* stream)
+{
+    MI8_REQUIRE(ids && sizes && workspace && indices && bin_ids && bins, MI8_ERR_ARG, "mi8_moe_sort_many_slots: null pointer");
+    MI8_REQUIRE(mi8_moe_sort_workspace_words(n, experts) > 0, MI8_ERR_UNSUPPORTED,
+                "mi8_moe_sort_many_slots: needs 1..2^30 - 1 slots and 1..%d experts (got %lld, %d)", kSortExperts, (long long)n, experts);
+    const dim3 grid((unsigned)ceil_div(n, kSortThreads)), threads(kSortThreads);
+    hipStream_t st = (hipStream_t)stream;
+    if (ids_are_64) {
+        hipLaunchKernelGGL(count_slots_kernel<int64_t>, grid, threads, 0, st, (const int64_t*)ids, (int)n, experts, workspace);
+        hipLaunchKernelGGL(place_slots_kernel<int64_t>, grid, threads, 0, st, (const int64_t*)ids, (int)n, sizes, experts, workspace, indices,
+                           bin_ids, bins);
+    } else {
+        hipLaunchKernelGGL(count_slots_kernel<int32_t>, grid, threads, 0, st, (const int32_t*)ids, (int)n, experts, workspace);
+        hipLaunchKernelGGL(place_slots_kernel<int32_t>, grid, threads, 0, st, (const int32_t*)ids, (int)n, sizes, experts, workspace, indices,
+                           bin_ids, bins);
+    }
+    return launch_status("mi8_moe_sort_many_slots");
+}
 
 extern "C" int64_t mi8_moe_sort_slots_max(void) { return kSortSlots; }
 

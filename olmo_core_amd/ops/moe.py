@@ -58,16 +58,25 @@ def _weights(w: Optional[torch.Tensor], n: int, what: str):
 
 def _sort_slots(ids: torch.Tensor, sizes: torch.Tensor):
     """``(indices, bin_ids, bins)``: the slots stably sorted by expert id, their ids, the inclusive prefix sums of
-    ``sizes`` (all int32).  One launch up to ``mi8_moe_sort_slots_max()`` slots; torch's sort beyond, for other types and
-    wherever something other than plain GPU tensors is at work (tracing, vmap, subclasses)."""
+    ``sizes`` (all int32).  One launch up to ``mi8_moe_sort_slots_max()`` slots, two beyond; torch's sort for other types, more
+    than 256 experts with that many slots, and wherever something other than plain GPU tensors is at work (tracing, vmap, subclasses)."""
     n = ids.numel()
     if (type(ids) is torch.Tensor and type(sizes) is torch.Tensor and not torch.compiler.is_compiling() and ids.is_cuda
             and sizes.device == ids.device and ids.dim() == sizes.dim() == 1 and ids.dtype in (torch.int32, torch.int64)
             and sizes.dtype == torch.int64 and ids.is_contiguous() and sizes.is_contiguous() and sizes.numel()
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._functorch.peek_interpreter_stack() is None
-            and 0 < n <= _C.lib().mi8_moe_sort_slots_max()):
+            and 0 < n and (n <= _C.lib().mi8_moe_sort_slots_max() or _C.lib().mi8_moe_sort_workspace_words(n, sizes.shape[0]))):
         indices, bin_ids = (torch.empty(n, dtype=torch.int32, device=ids.device) for _ in range(2))
         bins = torch.empty(sizes.shape[0], dtype=torch.int32, device=ids.device)
+        if n > _C.lib().mi8_moe_sort_slots_max():
+            counts = torch.empty(_C.lib().mi8_moe_sort_workspace_words(n, sizes.shape[0]), dtype=torch.int32, device=ids.device)
+            _C.check(
+                _C.lib().mi8_moe_sort_many_slots(ids.data_ptr(), int(ids.dtype == torch.int64), n, sizes.data_ptr(), sizes.shape[0],
+                                                 counts.data_ptr(), indices.data_ptr(), bin_ids.data_ptr(), bins.data_ptr(),
+                                                 _stream(ids)),
+                "mi8_moe_sort_many_slots",
+            )
+            return indices, bin_ids, bins
         _C.check(
             _C.lib().mi8_moe_sort_slots(ids.data_ptr(), int(ids.dtype == torch.int64), n, sizes.data_ptr(), sizes.shape[0],
                                         indices.data_ptr(), bin_ids.data_ptr(), bins.data_ptr(), _stream(ids)),

@@ -91,3 +91,10 @@ def test_sorted_slots_equal_a_stable_sort(dev, n, experts, dtype):
     assert indices.dtype == bin_ids.dtype == bins.dtype == torch.int32
     assert torch.equal(indices.cpu().long(), want) and torch.equal(bin_ids.cpu().long(), want_ids)
     assert torch.equal(bins.cpu().long(), sizes.cumsum(0))
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64], ids=str)
+@pytest.mark.parametrize("n,experts", [(8193, 1), (9216, 8), (9217, 126), (40000, 127), (131072, 64), (131073, 256), (8200, 257)], ids=str)
+def test_many_slots_sorted_equal_a_stable_sort(dev, n, experts, dtype):
+    """Around the 1024 slots of a workgroup, the bits of a bucket number and the most experts that the two launches take."""
+    test_sorted_slots_equal_a_stable_sort(dev, n, experts, dtype)
