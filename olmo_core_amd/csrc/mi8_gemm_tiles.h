@@ -193,20 +193,11 @@ __device__ __forceinline__ GroupCache build_group_cache(const int64_t* sizes, in
 {
     GroupCache c{0, 0, 0, 0, E <= 64};
     if (!c.valid) return c;
-    const int lane = (int)threadIdx.x & 63;
-    int64_t m = (lane < E) ? sizes[lane] : 0;
-    m = m < 0 ? 0 : (m > T ? T : m);
-    int64_t end = wave_inclusive_sum(m, lane);
-    int64_t start = end - m;
-    end = end < T ? end : T;
-    start = start < T ? start : T;
-    const int64_t me = end - start;
-    const int64_t un = (me + U - 1) / U;
-    const int64_t uend = wave_inclusive_sum(un, lane);
-    c.start = (int)start;  // T < 2^30 is checked on the host
-    c.m = (int)me;
-    c.ubefore = (int)(uend - un);
-    c.uend = (int)uend;
+    const GroupLane g = group_of_lane<U>(sizes, (int)threadIdx.x & 63, E, (uint32_t)T, 0, 0);  // (T < 2^30 is checked on the host)
+    c.start = (int)g.start;
+    c.m = (int)g.m;
+    c.ubefore = (int)(g.uend - g.un);
+    c.uend = (int)g.uend;
     return c;
 }
 

@@ -606,3 +606,27 @@ def test_experts_weights_cast_together(dev, E, H, D):
             q1, rs1, q_t1, cs1 = ops.grouped_cast_rows_and_colwise_t(w, equal, torch.float8_e4m3fn, pow2=pow2)
             assert torch.equal(rs, rs1) and torch.equal(cs, cs1) and torch.equal(q.view(torch.uint8), q1.view(torch.uint8))
             assert torch.equal(q_t.view(torch.uint8), q_t1.view(torch.uint8)[:, : E * H])
+
+
+@pytest.mark.parametrize("E", [5, 15, 17, 33, 64, 65, 200])
+def test_groups_are_found_in_any_list_of_sizes(dev, E):
+    """Empty groups, sizes below zero (empty) and sizes that pass the last row (cut there), around the 16 lanes of a row of the
+    prefix sums, the 64 of a wave and beyond: every group's transposed cast against a cast of its rows alone."""
+    g = torch.Generator().manual_seed(E)
+    sizes = torch.randint(0, 300, (E,), generator=g)
+    sizes[torch.rand(E, generator=g) < 0.3] = 0
+    sizes[1], sizes[E // 2] = -7, 129
+    T = int(sizes.clamp(min=0).sum()) - int(sizes.clamp(min=0)[E - 2:].sum()) + 40
+    sizes[E - 2] = 1 << 40
+    x = seeded((T, 32), seed=E).to(dev)
+    q_t, scale = ops.grouped_cast_colwise_t(x, sizes, E4M3)
+    row = column = 0
+    for e, m in enumerate(sizes.clamp(min=0).tolist()):
+        m = min(m, T - row)
+        if m:
+            want, want_scale = ops.cast_colwise_t(x[row:row + m].contiguous(), E4M3)
+            assert torch.equal(scale[e], want_scale.reshape(-1)), e
+            assert torch.equal(q_t[:, column:column + m].view(torch.uint8), want[:, :m].view(torch.uint8)), e
+        row += m
+        column += (m + 127) // 128 * 128
+    assert row == T
