@@ -1097,29 +1097,34 @@ RowPlan plan_parts(GemmArgs& g, const int cus, int most_parts = 1 << 30)
 {
     RowPlan best = plan_halves(g, cus, most_parts);
     const float steps = (float)(g.K / BK);
-    const int quarter_rows = (g.M + 63) / 64, tail = quarter_rows & 3, rows = quarter_rows >> 2;
-    if (best.n_half == 0 && tail == 0) return best;  // (whole tiles alone are best)
-    const int pairs = rows * g.tiles_n, half_row = (tail >> 1) * g.tiles_n, quarter_row = (tail & 1) * g.tiles_n;
+    const int quarter_rows = (g.M + 63) / 64;
+    if (best.n_half == 0 && quarter_rows % 4 == 0) return best;  // (whole tiles alone are best)
     float time = makespan(best, cus, steps);
-    bool better = false;
-    const int splits[3] = {0, pairs % cus, pairs < cus ? pairs : pairs % cus + cus};
-    for (int c = 0; c < 3; ++c) {
-        const int split = splits[c];
-        if ((c && (split == 0 || split == splits[c - 1])) || split > pairs) continue;
-        for (int part = 0; part <= (split ? 4 : 0); ++part) {  // a share of the split tiles in quarters, the others in halves
-            const int fours = split * part / 4, twos = split - fours;
-            RowPlan p{pairs - split, 2 * twos + half_row, 2 * twos, persistent_blocks(pairs - split), 0, 4 * fours + quarter_row, 4 * fours, 0};
-            if (p.n_half + p.n_quarter > most_parts) continue;
-            const float t = makespan(p, cus, steps);
-            if (t < 0.97f * time) {
-                time = t;
-                best = p;
-                better = true;
+    int tiles_m = 0;
+    // rows at the end as a half and a quarter row, or as one more row of whole tiles (all or the last of which may be split),
+    // which repeats some of the rows before: not where the tiles add to C
+    for (int up = 0; up <= (quarter_rows % 4 && !g.accumulate ? 1 : 0); ++up) {
+        const int rows = quarter_rows / 4 + up, tail = up ? 0 : quarter_rows % 4;
+        const int pairs = rows * g.tiles_n, half_row = (tail >> 1) * g.tiles_n, quarter_row = (tail & 1) * g.tiles_n;
+        const int splits[3] = {0, pairs % cus, pairs < cus ? pairs : pairs % cus + cus};
+        for (int c = 0; c < 3; ++c) {
+            const int split = splits[c];
+            if ((c && (split == 0 || split == splits[c - 1])) || split > pairs) continue;
+            for (int part = 0; part <= (split ? 4 : 0); ++part) {  // a share of the split tiles in quarters, the others in halves
+                const int fours = split * part / 4, twos = split - fours;
+                RowPlan p{pairs - split, 2 * twos + half_row, 2 * twos, persistent_blocks(pairs - split), 0, 4 * fours + quarter_row, 4 * fours, 0};
+                if (p.n_half + p.n_quarter > most_parts) continue;
+                const float t = makespan(p, cus, steps);
+                if (t < 0.97f * time) {
+                    time = t;
+                    best = p;
+                    tiles_m = rows;
+                }
             }
         }
     }
-    if (better) {
-        g.tiles_m = rows;
+    if (tiles_m) {
+        g.tiles_m = tiles_m;
         best.half_blocks = (best.n_half + 7) / 8 * 8;
         best.quarter_blocks = (best.n_quarter + 7) / 8 * 8;
     }
