@@ -117,6 +117,7 @@ _SIGNATURES = {
          c_int, c_void_p, c_int, c_int64, c_void_p],
     ),
     "mi8_gemm_fp8_swiglu_matches_separate": (c_int, [c_int64, c_int64, c_int64]),
+    "mi8_gemm_fp8_swiglu_pays": (c_int, [c_int64, c_int64, c_int64]),
     "mi8_gemm_fp8_swiglu": (
         c_int,
         [c_void_p, c_int, c_int64, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p,

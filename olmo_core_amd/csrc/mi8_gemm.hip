@@ -551,13 +551,24 @@ extern "C" int mi8_gemm_fp8_accumulate(const void* a, int a_dtype, int64_t lda, 
 }
 
 // 1 if mi8_gemm_fp8_swiglu takes the shape AND the library would not cut either projection along K (then the fused
-// launch reproduces the three-call route bit for bit: all kernels that do not split sum in one order); fewer tiles go to
-// the separate calls
+// launch reproduces the three-call route bit for bit: all kernels that do not split sum in one order), for products of many tiles,
+// which are never cut
 extern "C" int mi8_gemm_fp8_swiglu_matches_separate(int64_t M, int64_t H, int64_t K)
 {
     if (M < 256 || H < 256 || K <= 0 || K % 128 || H % 8) return 0;
     const int64_t tiles256 = ((M + 255) / 256) * ((H + 255) / 256);
     return tiles256 > 96 ? 1 : 0;
+}
+
+// The same for any number of tiles: with few the fused launch, in whole, half and quarter tiles, is the faster one too.  us fused /
+// two products in one launch and the activation: 256 x 11008 x 4096 29.2 / 43.8, 300 44.5 / 56.9; 640 x 8192 x 2048 28.3 / 37.8;
+// 1999 x 2816 x 1024 20.8 / 28.3; 777 x 2048 x 768 9.4 / 14.8, 256 8.6 / 9.3; 256 x 512 x 512 7.5 / 8.0.  (From K = 512 on, the
+// widths that models have: below, the gain is of launches alone, 1-8 us, and the separate ones stay.)
+extern "C" int mi8_gemm_fp8_swiglu_pays(int64_t M, int64_t H, int64_t K)
+{
+    if (mi8_gemm_fp8_swiglu_matches_separate(M, H, K)) return 1;
+    if (M < 256 || H < 256 || K < 512 || K % 128 || H % 8) return 0;
+    return suggested_splits(M, H, K) == 1 ? 1 : 0;
 }
 
 extern "C" int mi8_gemm_fp8_swiglu(const void* a, int a_dtype, int64_t lda, const void* b1, const void* b3, int b_dtype,

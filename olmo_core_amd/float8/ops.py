@@ -488,6 +488,11 @@ def swiglu_gemm_matches_separate(M: int, H: int, K: int) -> bool:
     return bool(_C.lib().mi8_gemm_fp8_swiglu_matches_separate(M, H, K))
 
 
+def swiglu_gemm_pays(M: int, H: int, K: int) -> bool:
+    """Shapes for which :func:`gemm_fp8_swiglu` gives those bits and is the faster route, of any number of tiles."""
+    return bool(_C.lib().mi8_gemm_fp8_swiglu_pays(M, H, K))
+
+
 def gemm_fp8_swiglu(a: torch.Tensor, sa: torch.Tensor, b1: torch.Tensor, sb1: torch.Tensor, b3: torch.Tensor,
                     sb3: torch.Tensor, *, k: Optional[int] = None, want_codes: bool = False):
     """

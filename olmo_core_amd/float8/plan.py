@@ -49,7 +49,7 @@ _RECORD_AT = 3
 
 _QUERIES = {
     "mi8_gemm_splitk_suggest", "mi8_gemm_splitk_workspace_bytes", "mi8_gemm_fp8_batch_pays", "mi8_amax_slots_for",
-    "mi8_colamax_workspace_slots", "mi8_two_cast_workspace_words", "mi8_gemm_fp8_swiglu_matches_separate",
+    "mi8_colamax_workspace_slots", "mi8_two_cast_workspace_words", "mi8_gemm_fp8_swiglu_matches_separate", "mi8_gemm_fp8_swiglu_pays",
     "mi8_gemm_fp8_codes_supported", "mi8_rowseg_code_count", "mi8_swiglu_amax_state_words", "mi8_gemm_fp8_swiglu_slots",
 }
 

@@ -58,11 +58,11 @@ def swiglu(x1: torch.Tensor, x3: torch.Tensor) -> torch.Tensor:
 
 def _use_codes(M: int, D: int, H: int, any_grad: bool) -> bool:
     """Whether the fused forward launch records the row-segment codes of x1 and x3 for the backward pass."""
-    return any_grad and SWIGLU_AMAX_FROM_CODES and H % 64 == 0
+    return any_grad and SWIGLU_AMAX_FROM_CODES and H % 64 == 0 and ops.gemm_codes_supported(M, H, D)
 
 
 def _fused_launch_ok(M: int, D: int, H: int) -> bool:
-    return FUSE_SWIGLU_EPILOGUE and ops.swiglu_gemm_matches_separate(M, H, D)
+    return FUSE_SWIGLU_EPILOGUE and ops.swiglu_gemm_pays(M, H, D)
 
 
 def _mlp_forward(x, w1, w2, w3, c, need, ws=(None, None, None), wo=(None, None, None), keep=True):
