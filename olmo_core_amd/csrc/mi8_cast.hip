@@ -123,7 +123,7 @@ struct TileCastArgs {
     bool stream;
 };
 
-template <int HP, int FP8, bool SW, int MODE>
+template <int HP, int FP8, bool SW, int MODE, bool STREAM>
 __global__ __launch_bounds__(kThreads) void tile_cast_kernel(TileCastArgs a)
 {
     __shared__ __attribute__((aligned(16))) uint32_t lds_t[kTile * kTile / 4];
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(kThreads) void tile_cast_kernel(TileCastArgs a)
         for (int i = 0; i < 8; ++i) sc[i] = s;
     }
 
-    tile_quantise<FP8, SW>(values, a.rows, a.cols, row0, col0, sc, a.out, a.ld_out, a.out_t, a.ld_t, row0, a.t_end, lds_t, a.stream);
+    tile_quantise<FP8, SW>(values, a.rows, a.cols, row0, col0, sc, a.out, a.ld_out, a.out_t, a.ld_t, row0, a.t_end, lds_t, STREAM);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -305,14 +305,13 @@ __global__ __launch_bounds__(kThreads) void rowwise_cast_kernel(RowCastArgs a)
         m = block_umax(m, smem);
     const float s = scale_from_amax_bits<FP8>(m, a.pow2);
     if (row_ok && lane == 0) a.scale_out[row] = s;
-    uint8_t* orow = a.out + row * a.ld_out;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int v = lane + TPR * i;
         if (row_ok && v < nvec) {
             const uint32_t lo = quant4<FP8, SW>(f[i][0], f[i][1], f[i][2], f[i][3], s, s, s, s);
             const uint32_t hi = quant4<FP8, SW>(f[i][4], f[i][5], f[i][6], f[i][7], s, s, s, s);
-            store_out8(orow + (int64_t)v * 8, lo, hi, a.stream);
+            store_out8(a.out, row * a.ld_out + (int64_t)v * 8, lo, hi, a.stream);
         }
     }
 }
@@ -582,7 +581,7 @@ __global__ __launch_bounds__(kThreads) void swiglu_bwd_cast_kernel(SwigluBwdCast
                 lo[j] = quant4<FP8, SW>(v[0], v[1], v[2], v[3], sc[o], sc[o], sc[o], sc[o]);
                 hi[j] = quant4<FP8, SW>(v[4], v[5], v[6], v[7], sc[o], sc[o], sc[o], sc[o]);
                 if (!ok) lo[j] = hi[j] = 0;  // padding is zero bytes whatever the scale is (0 * NaN is NaN)
-                if (out[o] && ok) store_out8(out[o] + r * a.ld_out + c8, lo[j], hi[j], a.stream);
+                if (out[o] && ok) store_out8(out[o], r * a.ld_out + c8, lo[j], hi[j], a.stream);
             }
             if (want_t) {
                 uint32_t t[8];
@@ -609,7 +608,7 @@ __global__ __launch_bounds__(kThreads) void swiglu_bwd_cast_kernel(SwigluBwdCast
                 const uint4 v = reinterpret_cast<const uint4*>(lds_t[o])[tile_lds_chunk(col, part)];
                 const int64_t c = col0 + col;
                 const int64_t d = row0 + 16 * part;
-                if (c < a.cols && d < dst_end) store_out16(out_t[o] + c * a.ld_t + d, v, a.stream);
+                if (c < a.cols && d < dst_end) store_out16(out_t[o], c * a.ld_t + d, v, a.stream);
             }
     }
 }
@@ -755,20 +754,21 @@ __global__ __launch_bounds__(kThreads) void grouped_tile_cast_kernel(GroupedCast
 
 // ---- dispatch helpers ------------------------------------------------------------------------------
 
+// (two kernels: a launch of a few rows is as long as the code it fetches)
+template <int HP, int FP8, bool SW, int MODE>
+void launch_tile_cast_mode(const TileCastArgs& a, dim3 grid, hipStream_t st)
+{
+    const auto kern = a.stream ? tile_cast_kernel<HP, FP8, SW, MODE, true> : tile_cast_kernel<HP, FP8, SW, MODE, false>;
+    hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, st, a);
+}
+
 template <int HP, int FP8, bool SW>
 void launch_tile_cast(int mode, const TileCastArgs& a, dim3 grid, hipStream_t st)
 {
     switch (mode) {
-        case kScalarFromSlots:
-            hipLaunchKernelGGL((tile_cast_kernel<HP, FP8, SW, kScalarFromSlots>), grid, dim3(kThreads), 0, st, a);
-            break;
-        case kScalarFromPtr:
-            hipLaunchKernelGGL((tile_cast_kernel<HP, FP8, SW, kScalarFromPtr>), grid, dim3(kThreads), 0, st, a);
-            break;
-        default:
-            hipLaunchKernelGGL((tile_cast_kernel<HP, FP8, SW, kPerColumnFromWorkspace>), grid, dim3(kThreads), 0,
-                               st, a);
-            break;
+        case kScalarFromSlots: return launch_tile_cast_mode<HP, FP8, SW, kScalarFromSlots>(a, grid, st);
+        case kScalarFromPtr: return launch_tile_cast_mode<HP, FP8, SW, kScalarFromPtr>(a, grid, st);
+        default: return launch_tile_cast_mode<HP, FP8, SW, kPerColumnFromWorkspace>(a, grid, st);
     }
 }
 
@@ -1073,7 +1073,7 @@ extern "C" int mi8_cast_tensorwise(const void* x, int hp_dtype, int64_t rows, in
     }
     TileCastArgs a{x, rows, cols, slots, n_slots, scale_in, (flags & MI8_FLAG_POW2_SCALE) != 0,
                    (uint8_t*)out, ld_out, (uint8_t*)out_t, ld_t, scale_out, t_end,
-                   streams_outputs(rows * cols * ((out ? 1 : 0) + (out_t ? 1 : 0)))};
+                   streams_outputs(rows * cols * ((out ? 1 : 0) + (out_t ? 1 : 0)), out ? rows * ld_out : 0, out_t ? cols * ld_t : 0)};
     dispatch_tile_cast(hp_dtype, fp8_dtype, (flags & MI8_FLAG_SW_CVT) != 0, slots ? kScalarFromSlots : kScalarFromPtr,
                        a, (hipStream_t)stream);
     return launch_status("mi8_cast_tensorwise");
@@ -1174,7 +1174,7 @@ extern "C" int mi8_swiglu_bwd_cast(const void* x1, const void* x3, const void* g
     SwigluBwdCastArgs a{(const uint4*)x1, (const uint4*)x3, (const uint4*)gh, rows, cols, slots_g1, slots_g3, n_slots,
                         (flags & MI8_FLAG_POW2_SCALE) != 0, (uint8_t*)out1, (uint8_t*)out3, ld_out, (uint8_t*)out1_t,
                         (uint8_t*)out3_t, ld_t, scale_out1, scale_out3, t_end,
-                        streams_outputs(2 * rows * cols * ((out1 ? 1 : 0) + (out1_t ? 1 : 0)))};
+                        streams_outputs(2 * rows * cols * ((out1 ? 1 : 0) + (out1_t ? 1 : 0)), out1 ? rows * ld_out : 0, out1_t ? cols * ld_t : 0)};
     const dim3 grid((unsigned)ceil_div(cols, kTile), (unsigned)ceil_div(rows, kTile));
     hipStream_t st = (hipStream_t)stream;
     const bool sw = flags & MI8_FLAG_SW_CVT;
@@ -1201,7 +1201,8 @@ extern "C" int mi8_cast_rowwise(const void* x, int hp_dtype, int64_t rows, int64
     MI8_REQUIRE(aligned16(x) && aligned16(out), MI8_ERR_UNSUPPORTED, "mi8_cast_rowwise: pointers must be 16-byte aligned");
     const bool pow2 = flags & MI8_FLAG_POW2_SCALE, sw = flags & MI8_FLAG_SW_CVT;
     hipStream_t st = (hipStream_t)stream;
-    const RowCastArgs a{x, rows, cols, pow2, (uint8_t*)out, ld_out, scale_out, nullptr, nullptr, 0, 0, streams_outputs(rows * cols)};
+    const RowCastArgs a{x, rows, cols, pow2, (uint8_t*)out, ld_out, scale_out, nullptr, nullptr, 0, 0,
+                        streams_rows(rows * cols, rows * ld_out)};
     int rc;
 #define MI8_ROW(HP_, FP8_) \
     rc = sw ? launch_rowwise<HP_, FP8_, true>(a, st) : launch_rowwise<HP_, FP8_, false>(a, st)
@@ -1240,7 +1241,7 @@ extern "C" int mi8_moe_gather_cast_rows(const void* x, int64_t tokens, int64_t c
     int rc = check_expert_rows("mi8_moe_gather_cast_rows", tokens * top_k, cols, x, out, ld_out, scale_out);
     if (rc != MI8_OK) return rc;
     const RowCastArgs a{x, tokens * top_k, cols, (flags & MI8_FLAG_POW2_SCALE) != 0, (uint8_t*)out, ld_out, scale_out,
-                        nullptr, indices, top_k, tokens, streams_outputs(tokens * top_k * cols)};
+                        nullptr, indices, top_k, tokens, streams_rows(tokens * top_k * cols, tokens * top_k * ld_out)};
     rc = (flags & MI8_FLAG_SW_CVT) ? launch_rowwise<MI8_BF16, MI8_E4M3, true, kRowGather>(a, (hipStream_t)stream)
                                    : launch_rowwise<MI8_BF16, MI8_E4M3, false, kRowGather>(a, (hipStream_t)stream);
     MI8_REQUIRE(rc == MI8_OK, rc, "mi8_moe_gather_cast_rows: unsupported row length %lld", (long long)cols);
@@ -1254,7 +1255,7 @@ extern "C" int mi8_swiglu_cast_rows(const void* x1, const void* x3, int64_t rows
     if (rc != MI8_OK) return rc;
     MI8_REQUIRE(x3 && aligned16(x3), MI8_ERR_ARG, "mi8_swiglu_cast_rows: x3 must be given and 16-byte aligned");
     const RowCastArgs a{x1, rows, cols, (flags & MI8_FLAG_POW2_SCALE) != 0, (uint8_t*)out, ld_out, scale_out, x3, nullptr, 0, 0,
-                        streams_outputs(rows * cols)};
+                        streams_rows(rows * cols, rows * ld_out)};
     rc = (flags & MI8_FLAG_SW_CVT) ? launch_rowwise<MI8_BF16, MI8_E4M3, true, kRowSwiglu>(a, (hipStream_t)stream)
                                    : launch_rowwise<MI8_BF16, MI8_E4M3, false, kRowSwiglu>(a, (hipStream_t)stream);
     MI8_REQUIRE(rc == MI8_OK, rc, "mi8_swiglu_cast_rows: unsupported row length %lld", (long long)cols);
@@ -1291,7 +1292,7 @@ extern "C" int mi8_cast_colwise_t(const void* x, int hp_dtype, int64_t rows, int
     int rc = launch_status("mi8_cast_colwise_t(amax)");
     if (rc != MI8_OK) return rc;
     TileCastArgs a{x, rows, cols, workspace, n_chunks, nullptr, (flags & MI8_FLAG_POW2_SCALE) != 0,
-                   nullptr, 0, (uint8_t*)out_t, ld_t, scale_out, round_up(rows, 16), streams_outputs(rows * cols)};
+                   nullptr, 0, (uint8_t*)out_t, ld_t, scale_out, round_up(rows, 16), streams_outputs(rows * cols, cols * ld_t)};
     dispatch_tile_cast(hp_dtype, fp8_dtype, (flags & MI8_FLAG_SW_CVT) != 0, kPerColumnFromWorkspace, a, st);
     return launch_status("mi8_cast_colwise_t(cast)");
 }

@@ -6,6 +6,8 @@
 // for the other.  A call among others, us, tensor by tensor / together: one projection of 116 tokens, 4096 x 4096, input and
 // weight 51.1 / 37.9; of 2048 tokens, 4096 x 11008, 132.9 / 128.6; forward and backward of four projections on 1537 tokens of 2048
 // with scales per row and column (ten tensors, 30 launches before, 8 now) 633 / 470.
+#include <algorithm>
+
 #include "../../include/mi8.h"
 #include "mi8_cast_tile.h"
 
@@ -370,7 +372,7 @@ extern "C" int mi8_cast_tensorwise_batch(const mi8_cast_item* items, int32_t cou
     CastItems ca{};
     ca.count = count;
     ca.pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
-    int64_t amax_blocks = 0, cast_blocks = 0, bytes = 0;
+    int64_t amax_blocks = 0, cast_blocks = 0, bytes = 0, end = 0;
     for (int i = 0; i < count; ++i) {
         const mi8_cast_item& t = items[i];
         MI8_REQUIRE(t.x && t.scale_out && (t.out || t.out_t) && (t.slots || t.scale_in || t.amax_ws), MI8_ERR_ARG, "%s: tensor %d: null pointer", what, i);
@@ -397,8 +399,9 @@ extern "C" int mi8_cast_tensorwise_batch(const mi8_cast_item* items, int32_t cou
                            t.scale_out, n_slots, fp32, (int)tiles_n, (int)cast_blocks};
         cast_blocks += tiles;
         bytes += t.rows * t.cols * ((t.out ? 1 : 0) + (t.out_t ? 1 : 0));
+        end = std::max({end, t.out ? t.rows * t.ld_out : 0, t.out_t ? t.cols * t.ld_t : 0});
     }
-    ca.stream = streams_outputs(bytes);
+    ca.stream = streams_outputs(bytes, end);
     hipStream_t st = (hipStream_t)stream;
     if (am.count)
         if (int rc = launch_items(amax_items_kernel, am, amax_blocks, st, what)) return rc;
@@ -438,7 +441,7 @@ extern "C" int mi8_cast_rows_and_colwise_t_batch(const mi8_two_cast_item* items,
     TwoCastItems a{};
     a.count = count;
     a.pow2 = (flags & MI8_FLAG_POW2_SCALE) != 0;
-    int64_t blocks = 0, chunk_blocks = 0, bytes = 0;
+    int64_t blocks = 0, chunk_blocks = 0, bytes = 0, end = 0;
     for (int i = 0; i < count; ++i) {
         const mi8_two_cast_item& t = items[i];
         const int64_t tiles_m = ceil_div(t.rows, kTile), tiles_n = ceil_div(t.cols, kTile);
@@ -452,7 +455,8 @@ extern "C" int mi8_cast_rows_and_colwise_t_batch(const mi8_two_cast_item* items,
         blocks += tiles_m * tiles_n;
         chunk_blocks += chunks * tiles_n;
         bytes += 2 * t.rows * t.cols;
+        end = std::max({end, t.rows * t.ld_rows, t.cols * t.ld_t});
     }
-    a.stream = streams_outputs(bytes);
+    a.stream = streams_outputs(bytes, end);
     return launch_two_cast(a, fp8_dtype, (flags & MI8_FLAG_SW_CVT) != 0, chunk_blocks, blocks, (hipStream_t)stream, what);
 }

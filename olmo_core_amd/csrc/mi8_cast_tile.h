@@ -208,12 +208,12 @@ __device__ __forceinline__ void tile_quantise(const Values& values, int64_t row_
             lo[j] = quant4<FP8, SW>(v[0], v[1], v[2], v[3], sc[0], sc[1], sc[2], sc[3]);
             hi[j] = quant4<FP8, SW>(v[4], v[5], v[6], v[7], sc[4], sc[5], sc[6], sc[7]);
             if (!ok) lo[j] = hi[j] = 0;  // padding is zero bytes whatever the scale is (0 * NaN is NaN)
-            if (out && ok) store_out8(out + r * ld_out + c8, lo[j], hi[j], stream);
+            if (out && ok) store_out8(out, r * ld_out + c8, lo[j], hi[j], stream);
             if (out_r && ok) {  // the same values quantised with the row's own scale
                 const float sr = srow[it][j];
                 const uint32_t rl = quant4<FP8, SW>(v[0], v[1], v[2], v[3], sr, sr, sr, sr);
                 const uint32_t rh = quant4<FP8, SW>(v[4], v[5], v[6], v[7], sr, sr, sr, sr);
-                store_out8(out_r + r * ld_r + c8, rl, rh, stream);
+                store_out8(out_r, r * ld_r + c8, rl, rh, stream);
             }
         }
         if (out_t) {
@@ -238,7 +238,7 @@ __device__ __forceinline__ void tile_quantise(const Values& values, int64_t row_
             const uint4 v = reinterpret_cast<const uint4*>(lds_t)[tile_lds_chunk(col, part)];
             const int64_t c = col0 + col;
             const int64_t d = dst0 + 16 * part;
-            if (c < cols && d < dst_end) store_out16(out_t + c * ld_t + d, v, stream);
+            if (c < cols && d < dst_end) store_out16(out_t, c * ld_t + d, v, stream);
         }
     }
 }

@@ -39,7 +39,16 @@ static inline int64_t round_up(int64_t a, int64_t b) { return ceil_div(a, b) * b
 // four projections of 4096 x 2048 386 / 361; 64 experts of 2048 x 1024, 131072 rows (268 MB) 4470 / 4735.
 // The grouped casts stream at any size: their products gained nothing, and what a launch leaves in the L2s it writes back before
 // it ends (4008 rows of 64 experts, 2048 columns: 12.6 / 15.0 a launch, a step 1000 / 1011).
-static inline bool streams_outputs(int64_t bytes) { return bytes > (int64_t)192 << 20; }
+// (A few rows, up to 1 MiB, are read once by the products that follow: block of 23 tokens 49.4 / 49.8.)
+// (end, end2: bytes from the start of the outputs to their ends; the other stores take 31-bit offsets.)
+static inline bool streams_outputs(int64_t bytes, int64_t end, int64_t end2 = 0)
+{
+    return bytes > (int64_t)192 << 20 || bytes <= (int64_t)1 << 20 || end >= 0x7FFFFFF0 || end2 >= 0x7FFFFFF0;
+}
+// A cast of rows alone also streams the copies of small weights (8 to 24 MiB), which the products of a few rows that follow read once.  us of a linear without
+// gradients, copies of 17 MB (4096 x 4096) streamed / kept: 1 row 22.9 / 24.2, 200 33.1 / 32.9, 2048 52.2 / 49.5; (2048 x 8192) 22.8 / 24.1, 31.8 /
+// 33.1, 46.7 / 46.7; of 45 MB (4096 x 11008) 42.7 / 41.8, 54.9 / 51.3, 110.7 / 104.4.
+static inline bool streams_rows(int64_t bytes, int64_t end) { return (bytes > (int64_t)8 << 20 && bytes <= (int64_t)24 << 20) || streams_outputs(bytes, end); }
 
 // ---- device side ---------------------------------------------------------------------------------
 
@@ -210,27 +219,24 @@ __device__ __forceinline__ void store_stream8(void* p, uint32_t lo, uint32_t hi)
     __builtin_nontemporal_store((u32x2_t){lo, hi}, reinterpret_cast<u32x2_t*>(p));
 }
 
-// A cast's outputs, whichever way the launch stores them (uniform; see streams_outputs).  (The empty statements keep the
-// compiler from merging the two stores into one without the bit.)
-__device__ __forceinline__ void store_out16(void* p, uint4 v, bool stream)
+// A cast's outputs at `at` bytes from the (uniform) start of a tensor, whichever way the launch stores them (see
+// streams_outputs).  What is left in the memory-side cache is written through the L2 (sc0 sc1): left there as dirty lines it would be
+// written back when the kernel ends (a linear of 9 rows, 4096 x 4096 27.3 / 25.3 us, of 777 39.5 / 38.4, of 2048, 4096 x 11008 120.2 / 119.8).
+__device__ __forceinline__ void store_out16(uint8_t* out, int64_t at, uint4 v, bool stream)
 {
-    if (stream) {
-        asm volatile("");
-        store_stream16(p, v);
-        asm volatile("");
-    } else {
-        *reinterpret_cast<u32x4_t*>(p) = (u32x4_t){v.x, v.y, v.z, v.w};
-    }
+    if (stream)
+        store_stream16(out + at, v);
+    else
+        __builtin_amdgcn_raw_buffer_store_b128((u32x4_t){v.x, v.y, v.z, v.w}, __builtin_amdgcn_make_buffer_rsrc(out, 0, 0x7FFFFFFF, 0x00020000),
+                                               (int)at, 0, 1 | 16);
 }
-__device__ __forceinline__ void store_out8(void* p, uint32_t lo, uint32_t hi, bool stream)
+__device__ __forceinline__ void store_out8(uint8_t* out, int64_t at, uint32_t lo, uint32_t hi, bool stream)
 {
-    if (stream) {
-        asm volatile("");
-        store_stream8(p, lo, hi);
-        asm volatile("");
-    } else {
-        *reinterpret_cast<u32x2_t*>(p) = (u32x2_t){lo, hi};
-    }
+    if (stream)
+        store_stream8(out + at, lo, hi);
+    else
+        __builtin_amdgcn_raw_buffer_store_b64((u32x2_t){lo, hi}, __builtin_amdgcn_make_buffer_rsrc(out, 0, 0x7FFFFFFF, 0x00020000), (int)at,
+                                              0, 1 | 16);
 }
 
 // Eight consecutive high-precision elements starting at a 16-byte aligned address -> float[8]
