@@ -51,6 +51,11 @@ int mi8_probe_store_rate(int rows, int waves, int workgroups, int iterations, vo
 int mi8_diag_gemm_tile_timeline(const void* a, const float* sa, const void* b, const float* sb, void* out, int64_t M, int64_t N,
                                 int64_t K, int a_dtype, int b_dtype, uint32_t* stamps, void* stream);
 
+/* How that kernel cuts a product (swiglu: both projections of mi8_gemm_fp8_swiglu; accumulate: of mi8_gemm_fp8_accumulate) into tiles on
+ * a chip of `compute_units` units; host only.  plan[7]: rows of 256-row tiles, whole tiles, half tiles, how many of these are halves of
+ * split tiles (the rest: a row of half tiles at the end), quarter tiles, how many of these are quarters of split tiles, workgroups. */
+int mi8_diag_gemm_plan(int64_t M, int64_t N, int64_t K, int swiglu, int accumulate, int compute_units, int32_t* plan);
+
 #ifdef __cplusplus
 }
 #endif

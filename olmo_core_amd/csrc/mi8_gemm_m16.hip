@@ -980,9 +980,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_fp8_m16_kernel(Problem pb)
 // Workgroups of a persistent launch: one per compute unit, or, for fewer tiles, as many as the tiles need - rounded
 // up to a multiple of 8, because every XCD takes an eighth of the tiles (rounded up) and needs that many workgroups
 // to finish in one round (43 tiles on 43 workgroups: XCDs with 5 workgroups for 6 tiles).
-int persistent_blocks(int max_tiles)
+int persistent_blocks(int max_tiles, const int blocks = num_compute_units())
 {
-    const int blocks = num_compute_units();
     const int wanted = (max_tiles + 7) / 8 * 8;
     return blocks > wanted ? wanted : blocks;
 }
@@ -1022,13 +1021,23 @@ namespace {
 // us per K step and besides for a quarter tile (0.41 a step with half of the compute units busy, 0.54 with all of them)
 constexpr float kQuarterStep = 0.48f, kQuarterTile = 2.5f;
 
+constexpr int round_up_8(int n) { return (n + 7) / 8 * 8; }
+
+// What a plan may have at most: half and quarter tiles, and workgroups in all
+struct PartLimits {
+    int parts = 1 << 30, blocks = 1 << 30;
+    bool allow(const RowPlan& p) const { return p.n_half + p.n_quarter <= parts && p.blocks() <= blocks; }
+};
+// (four partial maxima of |h| per workgroup)
+constexpr PartLimits kSwigluLimits{256, MI8_AMAX_SLOTS / 4};
+
 // Which tiles of a dense problem are halves (tiles_n columns of tiles, nk K steps), and g.tiles_m = pairs of half rows.
 // Splitting tiles of a partial last round pays when its halves fit into one round: 2048 x 11008 x 4096 is 344 tiles, two
 // rounds of 256 workgroups for 1.34 rounds of work; as 256 whole and 176 half tiles it takes 81 us in a loop of its own
 // (92 right after the casts that write its operands) instead of 87.  4096 x 2048 x 8192, 128 tiles, is 256 half tiles: 55 us
 // instead of 69.  The matrix pipe is busy 68 % and 67 % of the cycles.  (A step of a half tile takes 0.65 us with its
 // operands in the memory-side cache, 0.85 us from HBM; a whole tile's 1.0 us, 1.35 us when all compute units have one.)
-RowPlan plan_halves(GemmArgs& g, const int cus, int most_halves = 1 << 30)
+RowPlan plan_halves(GemmArgs& g, const int cus, const PartLimits limits = {})
 {
     const int half_rows = (g.M + 127) / 128;
     g.tiles_m = half_rows / 2;
@@ -1042,19 +1051,22 @@ RowPlan plan_halves(GemmArgs& g, const int cus, int most_halves = 1 << 30)
         const float more = r > 0 ? (q + 1) * whole + (h + (hr > cus - r ? 1 : 0)) * half : 0.0f;
         return less > more ? less : more;
     };
-    if (odd > most_halves) {
+    auto with = [&](int split) {
+        return RowPlan{pairs - split, 2 * split + odd, 2 * split, persistent_blocks(pairs - split, cus), round_up_8(2 * split + odd), 0, 0, 0};
+    };
+    if (!limits.allow(with(0))) {
         g.tiles_m = (g.M + BM - 1) / BM;
-        return RowPlan{g.tiles_m * g.tiles_n, 0, 0, persistent_blocks(g.tiles_m * g.tiles_n), 0, 0, 0, 0};
+        return RowPlan{g.tiles_m * g.tiles_n, 0, 0, persistent_blocks(g.tiles_m * g.tiles_n, cus), 0, 0, 0, 0};
     }
     int split = 0;
     float best = longest(0);
     const int candidates[2] = {pairs % cus, pairs < cus ? pairs : pairs % cus + cus};
     for (int c : candidates)
-        if (c > 0 && c <= pairs && 2 * c + odd <= most_halves && longest(c) < 0.97f * best) {
+        if (c > 0 && c <= pairs && limits.allow(with(c)) && longest(c) < 0.97f * best) {
             split = c;
             best = longest(c);
         }
-    return RowPlan{pairs - split, 2 * split + odd, 2 * split, persistent_blocks(pairs - split), (2 * split + odd + 7) / 8 * 8, 0, 0, 0};
+    return with(split);
 }
 
 // us until the last of `cus` units is done: whole tiles in rounds, then every half and quarter to the unit that is free first
@@ -1093,9 +1105,9 @@ float makespan(const RowPlan& p, const int cus, const float steps)
 // 4096, whose 258 whole tiles and 86 pieces of nine rows are 256 whole tiles and 94 quarters, 85.4 / 71.0; 4160 x 4096 x 4096 (a row
 // of quarters beside whole tiles) 69.6 / 63.6.  A product of quarters alone, 1537 x 2048 x 2048, takes 12.7 (15.7 in halves), as
 // long as on ring tiles; 1024 x 4096 x 4096 21.0 (26.5), ring tiles 19.9.
-RowPlan plan_parts(GemmArgs& g, const int cus, int most_parts = 1 << 30)
+RowPlan plan_parts(GemmArgs& g, const int cus, const PartLimits limits = {})
 {
-    RowPlan best = plan_halves(g, cus, most_parts);
+    RowPlan best = plan_halves(g, cus, limits);
     const float steps = (float)(g.K / BK);
     const int quarter_rows = (g.M + 63) / 64;
     if (best.n_half == 0 && quarter_rows % 4 == 0) return best;  // (whole tiles alone are best)
@@ -1112,8 +1124,9 @@ RowPlan plan_parts(GemmArgs& g, const int cus, int most_parts = 1 << 30)
             if ((c && (split == 0 || split == splits[c - 1])) || split > pairs) continue;
             for (int part = 0; part <= (split ? 4 : 0); ++part) {  // a share of the split tiles in quarters, the others in halves
                 const int fours = split * part / 4, twos = split - fours;
-                RowPlan p{pairs - split, 2 * twos + half_row, 2 * twos, persistent_blocks(pairs - split), 0, 4 * fours + quarter_row, 4 * fours, 0};
-                if (p.n_half + p.n_quarter > most_parts) continue;
+                const int halves = 2 * twos + half_row, quarters = 4 * fours + quarter_row;
+                const RowPlan p{pairs - split, halves, 2 * twos, persistent_blocks(pairs - split, cus), round_up_8(halves), quarters, 4 * fours, round_up_8(quarters)};
+                if (!limits.allow(p)) continue;
                 const float t = makespan(p, cus, steps);
                 if (t < 0.97f * time) {
                     time = t;
@@ -1123,11 +1136,7 @@ RowPlan plan_parts(GemmArgs& g, const int cus, int most_parts = 1 << 30)
             }
         }
     }
-    if (tiles_m) {
-        g.tiles_m = tiles_m;
-        best.half_blocks = (best.n_half + 7) / 8 * 8;
-        best.quarter_blocks = (best.n_quarter + 7) / 8 * 8;
-    }
+    if (tiles_m) g.tiles_m = tiles_m;
     return best;
 }
 
@@ -1195,14 +1204,16 @@ int m16_swiglu_slots(int64_t M, int64_t H, int64_t K)
     g.M = (int)M;
     g.K = (int)K;
     g.tiles_n = (int)((H + 127) / 128);
-    return 4 * plan_parts(g, num_compute_units(), 256).blocks();
+    return 4 * plan_parts(g, num_compute_units(), kSwigluLimits).blocks();
 }
 
 int launch_m16_swiglu(GemmArgs& g, const uint8_t* b3, const float* sb3, uint16_t* x3, uint16_t* h, uint32_t* h_slots,
                       int* n_slots, uint16_t* x_codes, int a_dtype, int b_dtype, hipStream_t st)
 {
     g.tiles_n = (g.N + 127) / 128;
-    const RowPlan rows = plan_parts(g, num_compute_units(), 256);  // (4 partial maxima per workgroup, MI8_AMAX_SLOTS in all)
+    const RowPlan rows = plan_parts(g, num_compute_units(), kSwigluLimits);
+    MI8_REQUIRE(4 * rows.blocks() <= MI8_AMAX_SLOTS, MI8_ERR_UNSUPPORTED, "mi8_gemm_fp8_swiglu: %d workgroups of four partial maxima, room for %d",
+                rows.blocks(), MI8_AMAX_SLOTS);
     SwigluProblem pb{g, g.lda, g.ldb, g.ldc, rows, (int64_t)(b3 - g.B), (int64_t)(x3 - reinterpret_cast<uint16_t*>(g.C)),
                      (int64_t)(h - reinterpret_cast<uint16_t*>(g.C)), sb3, h_slots, x_codes};
     *n_slots = 4 * rows.blocks();  // one partial maximum per wave of the grid
@@ -1276,5 +1287,25 @@ extern "C" int mi8_diag_gemm_tile_timeline(const void* a, const float* sa, const
                     hipMemcpyToSymbol(HIP_SYMBOL(gemm::g_timeline), &none, sizeof(none)) == hipSuccess,
                 MI8_ERR_LAUNCH, "mi8_diag_gemm_tile_timeline: launch or reset failed");
     return rc;
+}
+
+// (declared in mi8_diag.h) The tiles a dense problem is cut into; host only.
+extern "C" int mi8_diag_gemm_plan(int64_t M, int64_t N, int64_t K, int swiglu, int accumulate, int compute_units, int32_t* plan)
+{
+    using namespace mi8;
+    MI8_REQUIRE(plan && compute_units > 0, MI8_ERR_ARG, "mi8_diag_gemm_plan: null pointer or no compute units");
+    MI8_REQUIRE(M >= 256 && N >= (swiglu ? 128 : 256) && K >= 128 && K % 128 == 0 && M < (1 << 24) && N < (1 << 20) && K < (1 << 30) && !(swiglu && accumulate),
+                MI8_ERR_UNSUPPORTED, "mi8_diag_gemm_plan: needs M, N >= 256 (N >= 128 for SwiGLU, which adds to nothing), K a multiple of 128");
+    gemm::GemmArgs g{};
+    g.M = (int)M;
+    g.N = (int)N;
+    g.K = (int)K;
+    g.accumulate = accumulate;
+    const int64_t columns = swiglu ? 128 : 256;
+    g.tiles_n = (int)ceil_div(N, columns);
+    const gemm::RowPlan p = gemm::plan_parts(g, compute_units, swiglu ? gemm::kSwigluLimits : gemm::PartLimits{});
+    const int32_t counts[7] = {g.tiles_m, p.n_full, p.n_half, p.n_split, p.n_quarter, p.n_split4, p.blocks()};
+    for (int i = 0; i < 7; ++i) plan[i] = counts[i];
+    return MI8_OK;
 }
 #endif

@@ -177,3 +177,20 @@ def test_grouped_pitch_limits():
 
     rc = L.mi8_grouped_gemm_fp8(p, 0, 1 << 27, p, 0, 256, 0, p, 1, 32, 1, 256, p, p, 0, p, 1, 1, None)
     assert rc == -2 and "2^27" in _C.last_error()
+
+
+def _plan(M, N, K, swiglu=0, accumulate=0, units=256):
+    """How the persistent kernel cuts a product: names and counts as mi8_diag.h lists them."""
+    counts = (ctypes.c_int32 * 7)()
+    assert _C.diag().mi8_diag_gemm_plan(M, N, K, swiglu, accumulate, units, ctypes.addressof(counts)) == 0
+    return dict(zip(("rows", "whole", "halves", "split_halves", "quarters", "split_quarters", "blocks"), counts))
+
+
+@pytest.mark.parametrize("units", [256, 304])
+def test_partial_maxima_of_the_fused_swiglu_launch_have_room(units):
+    """Four words per workgroup, MI8_AMAX_SLOTS in all, whatever mix of tiles a plan has and whatever rounds its launch up."""
+    for M in (*range(256, 6000, 192), 5952, 777, 1999):
+        for tiles in (*range(1, 140, 3), 49, 96):
+            for K in (128, 512, 4096, 28672):
+                plan = _plan(M, 128 * tiles, K, swiglu=1, units=units)
+                assert 4 * plan["blocks"] <= _C.AMAX_SLOTS, (M, tiles, K, plan)
