@@ -553,22 +553,91 @@ __global__ __launch_bounds__(kSortThreads) void sort_slots_kernel(const ID* __re
 }
 
 // The same for more slots: a stable counting sort in two launches, which count the ids of every 1024 slots and place them.  (A
-// radix sort of 131072 slots with its conversions and the scan of the sizes is 16 dependent launches, 93 us; with these two a step of 16384 tokens takes 67 us less.)  An id that
-// names no expert sorts as any other number would: counted, over all slots, for every such slot.
+// radix sort of 131072 slots with its conversions and the scan of the sizes is 16 dependent launches, 93 us; with these two a step of 16384 tokens takes 67 us less.)
+// An id that names no expert sorts as any other number would.  Where all that are too small, or all that are too large, are one
+// number, as those of dropped slots are, they are one more bucket (131072 slots 18 us).  Else the first launch's sorted lists of
+// them, one a workgroup, are searched by every such slot (all 131072 of any numbers 450 us, radix sort 66).
 constexpr int kSortExperts = 256;  // (16 tables of that many counts in LDS)
 
 __device__ __forceinline__ int sort_bucket(int32_t id, int experts) { return id < 0 ? 0 : id >= experts ? experts + 1 : id + 1; }
 
+// the lists: behind the counts, 1024 words a workgroup
+__device__ __forceinline__ int32_t* others_of(int32_t* counts, int experts) { return counts + (int64_t)gridDim.x * (experts + 2); }
+__device__ __forceinline__ const int32_t* others_of(const int32_t* counts, int experts) { return counts + (int64_t)gridDim.x * (experts + 2); }
+
+// the place of a workgroup's slot `at` among those of its slots whose ids name no expert
+__device__ __forceinline__ int32_t rank_of_other(const int32_t* id_of, int at, int experts)
+{
+    const int32_t id = id_of[at];
+    int32_t rank = 0;
+#pragma unroll 4
+    for (int j = 0; j < kSortThreads; j += 4) {
+        const int4 four = reinterpret_cast<const int4*>(id_of)[j / 4];
+        const int32_t v[4] = {four.x, four.y, four.z, four.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rank += (uint32_t)v[i] >= (uint32_t)experts && (v[i] < id || (v[i] == id && j + i < at)) ? 1 : 0;
+    }
+    return rank;
+}
+
+// how many entries of the other workgroups' lists come before one of this workgroup's: eight lists are searched at a time
+__device__ __forceinline__ int32_t others_before(const int32_t* __restrict__ counts, int experts, int32_t id)
+{
+    const int32_t* __restrict__ others = others_of(counts, experts);
+    const int blocks = (int)gridDim.x, own = (int)blockIdx.x;
+    constexpr int U = 8;
+    int32_t sum = 0;
+    for (int first = 0; first < blocks; first += U) {
+        int len[U], at[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int block = first + u;
+            const int32_t* c = counts + (int64_t)(block < blocks ? block : own) * (experts + 2);
+            len[u] = block < blocks && block != own ? c[0] + c[experts + 1] : 0;
+            at[u] = 0;
+        }
+        for (int step = kSortThreads; step; step >>= 1) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (at[u] + step <= len[u]) {
+                    const int32_t v = others[(int64_t)(first + u) * kSortThreads + at[u] + step - 1];
+                    if (v < id || (v == id && first + u < own)) at[u] += step;
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) sum += at[u];
+    }
+    return sum;
+}
+
 template <typename ID>
 __global__ __launch_bounds__(kSortThreads) void count_slots_kernel(const ID* __restrict__ ids, int n, int experts, int32_t* __restrict__ counts)
 {
-    __shared__ int32_t count[kSortExperts + 2];
+    __shared__ int32_t count[kSortExperts + 2], least[2], most[2], filled[2];  // (the last three: ids too small, too large)
+    __shared__ __attribute__((aligned(16))) int32_t id_of[kSortThreads];
     const int tid = threadIdx.x, e = (int)blockIdx.x * kSortThreads + tid;
+    const int32_t id = e < n ? (int32_t)ids[e] : 0;
+    const int b = sort_bucket(id, experts), side = b != 0;
+    const bool other = b == 0 || b == experts + 1;  // (not the lanes beyond n)
+    id_of[tid] = id;
     if (tid < experts + 2) count[tid] = 0;
+    if (tid < 2) {
+        least[tid] = INT32_MAX;
+        most[tid] = INT32_MIN;
+        filled[tid] = 0;
+    }
     __syncthreads();
-    if (e < n) atomicAdd(&count[sort_bucket((int32_t)ids[e], experts)], 1);
+    if (e < n) atomicAdd(&count[b], 1);
+    if (other) {
+        atomicMin(&least[side], id);
+        atomicMax(&most[side], id);
+    }
     __syncthreads();
     if (tid < experts + 2) counts[(int64_t)blockIdx.x * (experts + 2) + tid] = count[tid];
+    if (other) {
+        const int at = least[side] == most[side] ? (side ? count[0] : 0) + atomicAdd(&filled[side], 1) : rank_of_other(id_of, tid, experts);
+        others_of(counts, experts)[(int64_t)blockIdx.x * kSortThreads + at] = id;
+    }
 }
 
 template <typename ID>
@@ -579,9 +648,15 @@ __global__ __launch_bounds__(kSortThreads) void place_slots_kernel(const ID* __r
 {
     constexpr int kWaves = kSortThreads / 64;
     __shared__ int32_t of_wave[kWaves][kSortExperts + 2], before[kSortExperts + 2], total[kSortExperts + 2];
+    __shared__ int32_t slot_at[kSortThreads], least[2], most[2];  // (ids too small, too large)
+    __shared__ __attribute__((aligned(16))) int32_t id_of[kSortThreads];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, buckets = experts + 2;
     for (int b = tid; b < kWaves * (kSortExperts + 2); b += kSortThreads) (&of_wave[0][0])[b] = 0;
     if (tid < buckets) before[tid] = total[tid] = 0;
+    if (tid < 2) {
+        least[tid] = INT32_MAX;
+        most[tid] = INT32_MIN;
+    }
     __syncthreads();
     // slots of each bucket in the blocks before this one and in all: as many threads a bucket as there are
     const int parts = kSortThreads / buckets, part = tid / buckets, bucket = tid - part * buckets;
@@ -600,6 +675,7 @@ __global__ __launch_bounds__(kSortThreads) void place_slots_kernel(const ID* __r
     const int e = (int)blockIdx.x * kSortThreads + tid;
     const int32_t id = e < n ? (int32_t)ids[e] : 0;
     const int b = sort_bucket(id, experts);
+    id_of[tid] = id;
     uint64_t same = __ballot(e < n);
     for (int bit = 0; (buckets - 1) >> bit; ++bit) {
         const uint64_t set = __ballot((b >> bit) & 1);
@@ -608,6 +684,16 @@ __global__ __launch_bounds__(kSortThreads) void place_slots_kernel(const ID* __r
     const int rank = __popcll(same & (((uint64_t)1 << lane) - 1));
     if (e < n && rank == 0) of_wave[wave][b] = __popcll(same);
     __syncthreads();
+    const int others = total[0] + total[experts + 1];
+    for (int i = tid; i < (others ? 2 * (int)gridDim.x : 0); i += kSortThreads) {
+        const int32_t* c = counts + (int64_t)(i >> 1) * buckets;
+        const int32_t low = c[0], len = i & 1 ? c[experts + 1] : low;
+        if (len) {
+            const int32_t* list = others_of(counts, experts) + (int64_t)(i >> 1) * kSortThreads + (i & 1 ? low : 0);
+            atomicMin(&least[i & 1], list[0]);
+            atomicMax(&most[i & 1], list[len - 1]);
+        }
+    }
     if (wave == 0) {  // where each bucket starts
         int32_t sum = 0;
         for (int base = 0; base < buckets; base += 64) {
@@ -623,18 +709,24 @@ __global__ __launch_bounds__(kSortThreads) void place_slots_kernel(const ID* __r
         }
     }
     __syncthreads();
-    if (e < n) {
+    const bool several = least[0] < most[0] || least[1] < most[1], other = b == 0 || b == experts + 1;
+    if (e < n && !(several && other)) {
         int32_t at = before[b] + rank;
         for (int w = 0; w < wave; ++w) at += of_wave[w][b];
-        if (b == 0 || b == experts + 1) {
-            at = b == 0 ? 0 : n - total[b];
-            for (int j = 0; j < n; ++j) {
-                const int32_t other = (int32_t)ids[j];
-                if (sort_bucket(other, experts) == b && (other < id || (other == id && j < e))) ++at;
-            }
-        }
         indices[at] = e;
         bin_ids[at] = id;
+    }
+    if (several) {  // (uniform) lane i takes the i-th of the workgroup's list, so that a wave searches close by
+        if (other) slot_at[rank_of_other(id_of, tid, experts)] = tid;
+        __syncthreads();
+        const int32_t* c = counts + (int64_t)blockIdx.x * buckets;
+        if (tid < c[0] + c[experts + 1]) {
+            const int slot = slot_at[tid];
+            const int32_t its_id = id_of[slot];
+            const int32_t at = (its_id < 0 ? 0 : n - others) + tid + others_before(counts, experts, its_id);
+            indices[at] = (int)blockIdx.x * kSortThreads + slot;
+            bin_ids[at] = its_id;
+        }
     }
     if (wave == 1 && blockIdx.x == 0) write_bins(sizes, experts, bins, lane);
 }
@@ -646,7 +738,7 @@ using namespace mi8;
 
 extern "C" int64_t mi8_moe_sort_workspace_words(int64_t n, int32_t experts)
 {
-    return n > 0 && n < (1 << 30) && experts > 0 && experts <= kSortExperts ? ceil_div(n, kSortThreads) * (experts + 2) : 0;
+    return n > 0 && n < (1 << 30) && experts > 0 && experts <= kSortExperts ? ceil_div(n, kSortThreads) * (experts + 2 + kSortThreads) : 0;
 }
 
 extern "C" int mi8_moe_sort_many_slots(const void* ids, int ids_are_64, int64_t n, const int64_t* sizes, int32_t experts,
