@@ -479,8 +479,8 @@ int64_t mi8_moe_sort_slots_max(void);
 int mi8_moe_sort_slots(const void* ids, int ids_are_64, int64_t n, const int64_t* sizes, int32_t experts, int32_t* indices,
                        int32_t* bin_ids, int32_t* bins, void* stream);
 
-/* The same for any n < 2^30 and up to 256 experts.  workspace: int32 [mi8_moe_sort_workspace_words(n, experts)] (0: not taken),
- * overwritten. */
+/* The same for more slots and up to 256 experts, as long as ceil(n / 1024)^2 * (experts + 2) <= 3e8 (2^20 slots of 256 experts,
+ * 2^21 of 64).  workspace: int32 [mi8_moe_sort_workspace_words(n, experts)] (0: not taken), overwritten. */
 int64_t mi8_moe_sort_workspace_words(int64_t n, int32_t experts);
 int mi8_moe_sort_many_slots(const void* ids, int ids_are_64, int64_t n, const int64_t* sizes, int32_t experts, int32_t* workspace,
                             int32_t* indices, int32_t* bin_ids, int32_t* bins, void* stream);

@@ -554,10 +554,14 @@ __global__ __launch_bounds__(kSortThreads) void sort_slots_kernel(const ID* __re
 
 // The same for more slots: a stable counting sort in two launches, which count the ids of every 1024 slots and place them.  (A
 // radix sort of 131072 slots with its conversions and the scan of the sizes is 16 dependent launches, 93 us; with these two a step of 16384 tokens takes 67 us less.)
+// Every workgroup of the second reads the counts of all, so the reads grow with the square of the slots, and the radix sort
+// has what passes kSortCounts of them.  us, this and that: 8 experts, 2^22 slots 74 / 221 (168 million counts); 64, 2^20 33 / 191, 2^21 87 / 153 (277),
+// 2^22 270 / 222; 256, 2^19 33 / 155, 2^20 90 / 197 (271), 2^21 309 / 154.
 // An id that names no expert sorts as any other number would.  Where all that are too small, or all that are too large, are one
 // number, as those of dropped slots are, they are one more bucket (131072 slots 18 us).  Else the first launch's sorted lists of
 // them, one a workgroup, are searched by every such slot (all 131072 of any numbers 450 us, radix sort 66).
 constexpr int kSortExperts = 256;  // (16 tables of that many counts in LDS)
+constexpr int64_t kSortCounts = 300000000;
 
 __device__ __forceinline__ int sort_bucket(int32_t id, int experts) { return id < 0 ? 0 : id >= experts ? experts + 1 : id + 1; }
 
@@ -738,7 +742,9 @@ using namespace mi8;
 
 extern "C" int64_t mi8_moe_sort_workspace_words(int64_t n, int32_t experts)
 {
-    return n > 0 && n < (1 << 30) && experts > 0 && experts <= kSortExperts ? ceil_div(n, kSortThreads) * (experts + 2 + kSortThreads) : 0;
+    if (n <= 0 || n >= (1 << 30) || experts <= 0 || experts > kSortExperts) return 0;
+    const int64_t blocks = ceil_div(n, kSortThreads);
+    return blocks * blocks * (experts + 2) <= kSortCounts ? blocks * (experts + 2 + kSortThreads) : 0;
 }
 
 extern "C" int mi8_moe_sort_many_slots(const void* ids, int ids_are_64, int64_t n, const int64_t* sizes, int32_t experts,
@@ -746,7 +752,8 @@ extern "C" int mi8_moe_sort_many_slots(const void* ids, int ids_are_64, int64_t 
 {
     MI8_REQUIRE(ids && sizes && workspace && indices && bin_ids && bins, MI8_ERR_ARG, "mi8_moe_sort_many_slots: null pointer");
     MI8_REQUIRE(mi8_moe_sort_workspace_words(n, experts) > 0, MI8_ERR_UNSUPPORTED,
-                "mi8_moe_sort_many_slots: needs 1..2^30 - 1 slots and 1..%d experts (got %lld, %d)", kSortExperts, (long long)n, experts);
+                "mi8_moe_sort_many_slots: needs 1..%d experts and no more slots than mi8_moe_sort_workspace_words takes (got %lld, %d)", kSortExperts,
+                (long long)n, experts);
     const dim3 grid((unsigned)ceil_div(n, kSortThreads)), threads(kSortThreads);
     hipStream_t st = (hipStream_t)stream;
     if (ids_are_64) {

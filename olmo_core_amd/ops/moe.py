@@ -58,8 +58,8 @@ def _weights(w: Optional[torch.Tensor], n: int, what: str):
 
 def _sort_slots(ids: torch.Tensor, sizes: torch.Tensor):
     """``(indices, bin_ids, bins)``: the slots stably sorted by expert id, their ids, the inclusive prefix sums of
-    ``sizes`` (all int32).  One launch up to ``mi8_moe_sort_slots_max()`` slots, two beyond; torch's sort for other types, more
-    than 256 experts with that many slots, and wherever something other than plain GPU tensors is at work (tracing, vmap, subclasses)."""
+    ``sizes`` (all int32).  One launch up to ``mi8_moe_sort_slots_max()`` slots, two beyond; torch's sort for other types, for
+    more slots or experts than ``mi8_moe_sort_workspace_words`` takes, and wherever something other than plain GPU tensors is at work (tracing, vmap, subclasses)."""
     n = ids.numel()
     if (type(ids) is torch.Tensor and type(sizes) is torch.Tensor and not torch.compiler.is_compiling() and ids.is_cuda
             and sizes.device == ids.device and ids.dim() == sizes.dim() == 1 and ids.dtype in (torch.int32, torch.int64)

@@ -194,3 +194,12 @@ def test_partial_maxima_of_the_fused_swiglu_launch_have_room(units):
             for K in (128, 512, 4096, 28672):
                 plan = _plan(M, 128 * tiles, K, swiglu=1, units=units)
                 assert 4 * plan["blocks"] <= _C.AMAX_SLOTS, (M, tiles, K, plan)
+
+
+def test_slots_that_the_counting_sort_takes():
+    """Its second launch reads every workgroup's counts in every workgroup: what passes 3e8 of them is for the caller's sort."""
+    words = _C.lib().mi8_moe_sort_workspace_words
+    for n, experts in ((8193, 1), (131072, 64), (1 << 20, 256), (1 << 21, 64), (1 << 22, 8)):
+        assert words(n, experts) >= -(-n // 1024) * (experts + 2 + 1024), (n, experts)
+    for n, experts in ((1 << 21, 256), (1 << 22, 64), (1 << 24, 1), ((1 << 30) - 1, 1), (1 << 30, 8), (131072, 257), (0, 8), (8193, 0)):
+        assert words(n, experts) == 0, (n, experts)
