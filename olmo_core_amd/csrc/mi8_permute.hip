@@ -272,10 +272,20 @@ __global__ __launch_bounds__(kThreads) void scatter_reduce_kernel(PermuteArgs a,
 
 // The scatter of few slots in one launch.  A call with few tokens is a chain of short launches, and three of them - clearing the
 // inverse, filling it, one wave a token - were its last 17 us (48 tokens of 8 slots, 2048 columns; now 6.4).  Here
-// a workgroup finds the rows of its token among all slots itself (n / 256 loads a lane, so up to kFewSlots), and its lanes
-// have one 16-byte chunk of a row each, eight rows in flight.  Sums as above; a slot named twice takes the later row.
+// a workgroup finds the rows of its token among all slots itself, and its lanes have one 16-byte chunk of a row each, eight rows in
+// flight.  Sums as above; a slot named twice takes the later row.
 constexpr int64_t kFewSlots = 8192;
 constexpr int kFewTopK = 64;
+
+// So the slots are read as often as there are workgroups: up to 2^22 of them in all, 2^23 where half the lanes have no chunk to wait
+// for.  us, this and the three launches, tokens x slots of a token x bf16 columns: 512 x 8 x 4096 (2^22) 13.5 / 21.1, 1024 x 4 x 2048 9.5 / 11.6, 2048 x 1 x
+// 2048 10.9 / 13.1; 1024 x 8 x 2048 (2^23) 17.6 / 14.8, x 1024 9.7 / 13.3; 2048 x 2 x 2048 13.8 / 13.0, x 1024 10.5 / 11.2; 2048 x 4 x 1024 (2^24)
+// 15.9 / 13.2, x 64 12.3 / 11.0; 8192 x 1 x 4096 (2^27) 101 / 59.
+bool scatter_in_one_launch(const PermuteArgs& a, int64_t tokens, int64_t chunks)
+{
+    const int64_t columns = ceil_div(chunks, kThreads);
+    return a.vec && a.n <= kFewSlots && a.top_k <= kFewTopK && columns <= 65535 && tokens * a.n * columns <= (chunks <= 128 ? 1 << 23 : 1 << 22);
+}
 
 template <int DT, bool SCALE>
 __global__ __launch_bounds__(kThreads) void scatter_few_kernel(PermuteArgs a)
@@ -441,8 +451,9 @@ template <bool BINNED>
 int launch_scatter(PermuteArgs& a, int dtype, int64_t rows, int64_t tokens, hipStream_t st)
 {
     const bool scale = a.weights != nullptr;
-    if (!BINNED && a.vec && a.n <= kFewSlots && a.top_k <= kFewTopK) {
-        const dim3 grid((unsigned)tokens, (unsigned)ceil_div(a.hidden * elem_size(dtype) / 16, kThreads));
+    const int64_t chunks = a.hidden * elem_size(dtype) / 16;
+    if (!BINNED && scatter_in_one_launch(a, tokens, chunks)) {
+        const dim3 grid((unsigned)tokens, (unsigned)ceil_div(chunks, kThreads));
 #define MI8_S(DT_)                                                                                                   \
     if (scale)                                                                                                       \
         hipLaunchKernelGGL((scatter_few_kernel<DT_, true>), grid, dim3(kThreads), 0, st, a);                         \

@@ -243,7 +243,7 @@ def test_routed_layer_without_gradients_has_the_same_bits(dev, tokens, keep):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=str)
-@pytest.mark.parametrize("tokens,top_k,hidden", [(1, 1, 8), (48, 8, 2048), (3, 64, 2056), (100, 7, 4096), (1024, 8, 264), (8192, 1, 16)], ids=str)
+@pytest.mark.parametrize("tokens,top_k,hidden", [(1, 1, 8), (48, 8, 2048), (3, 64, 2056), (100, 7, 4096), (1024, 8, 264), (2048, 1, 16)], ids=str)
 @pytest.mark.parametrize("weighted", [False, True])
 def test_scatter_of_few_slots_equals_that_of_many(dev, tokens, top_k, hidden, weighted, dtype):
     """The one-launch scatter against the general one, which the same problem several times over goes to; some slots unfilled."""
@@ -259,3 +259,26 @@ def test_scatter_of_few_slots_equals_that_of_many(dev, tokens, top_k, hidden, we
     got = ops._scatter(x, indices.to(dev), w, top_k)
     want = ops._scatter(x.repeat(times, 1), many.int().to(dev), w.repeat(times) if weighted else None, top_k)
     assert torch.equal(got, want[:tokens])
+
+
+@pytest.mark.parametrize("tokens,top_k,hidden,one", [
+    (512, 8, 4096, True), (1024, 4, 2048, True), (1024, 8, 1024, True), (8192, 1, 16, False), (1024, 8, 2048, False), (2048, 4, 64, False),
+    (1, 1, 65536 * 2048, False)], ids=str)
+def test_scatter_in_one_launch_only_where_the_slots_are_read_few_times(dev, tokens, top_k, hidden, one):
+    """Whether the one launch ran shows in the workspace, which it leaves alone; a row of 256 MiB has more column blocks than a
+    launch may."""
+    n = tokens * top_k
+    x = torch.randn(n, min(hidden, 8192), device=dev).bfloat16().repeat(1, max(hidden // 8192, 1))
+    indices = torch.randperm(n, device=dev).int()
+    inverse = torch.full((n,), -7, dtype=torch.int32, device=dev)
+    out = torch.empty(tokens, hidden, dtype=torch.bfloat16, device=dev)
+    lib = ops._C.lib()
+    ops._C.check(lib.mi8_moe_scatter(x.data_ptr(), ops._C.MI8_BF16, tokens, hidden, indices.data_ptr(), None, 0, top_k, inverse.data_ptr(),
+                                     out.data_ptr(), torch.cuda.current_stream().cuda_stream), "mi8_moe_scatter")
+    assert bool((inverse == -7).all()) == one
+    slots = torch.empty_like(x)
+    slots[indices.long()] = x
+    want = torch.zeros(tokens, hidden, device=dev)
+    for j in range(top_k):  # float32 sums in slot order, rounded once
+        want += slots.view(tokens, top_k, hidden)[:, j]
+    assert torch.equal(out, want.bfloat16())
