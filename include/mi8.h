@@ -54,6 +54,7 @@ typedef enum mi8_hp {
 #define MI8_FLAG_POW2_SCALE 1u /* round every scale down to a power of two (ao.py:167 round_scales_to_power_of_2) */
 #define MI8_FLAG_SW_CVT 2u     /* convert with integer arithmetic instead of v_cvt_pk_{fp8,bf8}_f32 (same bytes) */
 #define MI8_FLAG_PAD_T128 8u   /* transposed copies of tensorwise casts: zero columns up to a multiple of 128 instead of 16 */
+#define MI8_FLAG_READ_BY_FEW_ROWS 16u /* mi8_cast_rowwise: the copy is a weight that a product of at most 256 rows reads (same bytes) */
 #define MI8_FLAG_AMAX_READY 4u /* grouped casts: the amax workspaces already hold the amax of x (see mi8_grouped_swiglu_*) */
 
 /* Number of uint32 slots a tensorwise amax workspace must have. */

@@ -26,6 +26,7 @@ FLAG_POW2_SCALE = 1
 FLAG_SW_CVT = 2
 FLAG_AMAX_READY = 4
 FLAG_PAD_T128 = 8
+FLAG_READ_BY_FEW_ROWS = 16
 AMAX_SLOTS = 2048
 
 CAST_BATCH = 8

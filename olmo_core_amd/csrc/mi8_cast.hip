@@ -1202,7 +1202,7 @@ extern "C" int mi8_cast_rowwise(const void* x, int hp_dtype, int64_t rows, int64
     const bool pow2 = flags & MI8_FLAG_POW2_SCALE, sw = flags & MI8_FLAG_SW_CVT;
     hipStream_t st = (hipStream_t)stream;
     const RowCastArgs a{x, rows, cols, pow2, (uint8_t*)out, ld_out, scale_out, nullptr, nullptr, 0, 0,
-                        streams_rows(rows * cols, rows * ld_out)};
+                        streams_rows(rows, cols, ld_out, (flags & MI8_FLAG_READ_BY_FEW_ROWS) != 0)};
     int rc;
 #define MI8_ROW(HP_, FP8_) \
     rc = sw ? launch_rowwise<HP_, FP8_, true>(a, st) : launch_rowwise<HP_, FP8_, false>(a, st)
@@ -1241,7 +1241,7 @@ extern "C" int mi8_moe_gather_cast_rows(const void* x, int64_t tokens, int64_t c
     int rc = check_expert_rows("mi8_moe_gather_cast_rows", tokens * top_k, cols, x, out, ld_out, scale_out);
     if (rc != MI8_OK) return rc;
     const RowCastArgs a{x, tokens * top_k, cols, (flags & MI8_FLAG_POW2_SCALE) != 0, (uint8_t*)out, ld_out, scale_out,
-                        nullptr, indices, top_k, tokens, streams_rows(tokens * top_k * cols, tokens * top_k * ld_out)};
+                        nullptr, indices, top_k, tokens, streams_outputs(tokens * top_k * cols, tokens * top_k * ld_out)};
     rc = (flags & MI8_FLAG_SW_CVT) ? launch_rowwise<MI8_BF16, MI8_E4M3, true, kRowGather>(a, (hipStream_t)stream)
                                    : launch_rowwise<MI8_BF16, MI8_E4M3, false, kRowGather>(a, (hipStream_t)stream);
     MI8_REQUIRE(rc == MI8_OK, rc, "mi8_moe_gather_cast_rows: unsupported row length %lld", (long long)cols);
@@ -1255,7 +1255,7 @@ extern "C" int mi8_swiglu_cast_rows(const void* x1, const void* x3, int64_t rows
     if (rc != MI8_OK) return rc;
     MI8_REQUIRE(x3 && aligned16(x3), MI8_ERR_ARG, "mi8_swiglu_cast_rows: x3 must be given and 16-byte aligned");
     const RowCastArgs a{x1, rows, cols, (flags & MI8_FLAG_POW2_SCALE) != 0, (uint8_t*)out, ld_out, scale_out, x3, nullptr, 0, 0,
-                        streams_rows(rows * cols, rows * ld_out)};
+                        streams_outputs(rows * cols, rows * ld_out)};
     rc = (flags & MI8_FLAG_SW_CVT) ? launch_rowwise<MI8_BF16, MI8_E4M3, true, kRowSwiglu>(a, (hipStream_t)stream)
                                    : launch_rowwise<MI8_BF16, MI8_E4M3, false, kRowSwiglu>(a, (hipStream_t)stream);
     MI8_REQUIRE(rc == MI8_OK, rc, "mi8_swiglu_cast_rows: unsupported row length %lld", (long long)cols);

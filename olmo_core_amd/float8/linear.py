@@ -110,8 +110,8 @@ def _input_operands(x2, c: Float8LinearConfig, pow2: bool, share_x: bool):
     return xq, sx, x_saved
 
 
-def _weight_operands(weight, c: Float8LinearConfig, pow2: bool, share_w: bool, weight_scale=None, weight_ops=None):
-    """``(wq, sw, w_saved)`` for the forward GEMM: the weight's by-rows operand, its scale(s), and what the backward
+def _weight_operands(weight, c: Float8LinearConfig, pow2: bool, share_w: bool, rows: int, weight_scale=None, weight_ops=None):
+    """``(wq, sw, w_saved)`` for the forward GEMM of ``rows`` rows: the weight's by-rows operand, its scale(s), and what the backward
     keeps for grad_input (``(q_t, scale)`` or ``None``: keep the weight itself)."""
     w_saved = None
     if weight_ops is not None:
@@ -129,7 +129,7 @@ def _weight_operands(weight, c: Float8LinearConfig, pow2: bool, share_w: bool, w
         wq, sw, wq_t, swc = ops.cast_rows_and_colwise_t(weight, c.cast_config_weight.target_dtype, pow2=pow2)
         w_saved = (wq_t, swc)
     else:
-        wq, sw = ops.cast_rowwise(weight, c.cast_config_weight.target_dtype, pow2=pow2)
+        wq, sw = ops.cast_rowwise(weight, c.cast_config_weight.target_dtype, pow2=pow2, product_rows=rows)
     return wq, sw, w_saved
 
 
@@ -150,7 +150,7 @@ def _forward_operands(x2, weights, c: Float8LinearConfig, scales, w_ops, share_x
             (xq, sx, xq_t, sxc), *made = ops.cast_rows_and_colwise_t(x2, ci.target_dtype, pow2=pow2, more=weights)
             return xq, sx, (xq_t, sxc), [(q, s, (q_t, sc)) for q, s, q_t, sc in made]
     return (*_input_operands(x2, c, pow2, share_x),
-            [_weight_operands(w, c, pow2, share_w, s, o) for w, s, o in zip(weights, scales, w_ops)])
+            [_weight_operands(w, c, pow2, share_w, x2.shape[0], s, o) for w, s, o in zip(weights, scales, w_ops)])
 
 
 def _forward_impl(x2, weight, c: Float8LinearConfig, weight_scale, need_gx: bool, need_gw: bool, weight_ops=None):

@@ -277,16 +277,18 @@ def cast_tensorwise_batch(items, fp8_dtype: torch.dtype, *, pow2: bool = False) 
 
 
 def cast_rowwise(
-    x: torch.Tensor, fp8_dtype: torch.dtype, *, pow2: bool = False, pitch: Optional[int] = None
+    x: torch.Tensor, fp8_dtype: torch.dtype, *, pow2: bool = False, pitch: Optional[int] = None, product_rows: Optional[int] = None
 ) -> Tuple[torch.Tensor, torch.Tensor]:
-    """One scale per row: returns (q fp8 [rows, cols], scale float32 [rows])."""
+    """One scale per row: returns (q fp8 [rows, cols], scale float32 [rows]).  ``product_rows``: for a weight, the rows of the
+    product that reads it (how the bytes are stored, not what they are)."""
     x = _hp2d(x, "cast_rowwise")
+    few = _C.FLAG_READ_BY_FEW_ROWS if product_rows is not None and product_rows <= 256 else 0
     rows, cols = x.shape
     q = _operand((rows, cols), fp8_dtype, x.device, pitch)
     s = _empty(rows, dtype=torch.float32, device=x.device)
     _C.check(
         _C.lib().mi8_cast_rowwise(
-            x.data_ptr(), _HP_CODE[x.dtype], rows, cols, _FP8_CODE[fp8_dtype], _flags(pow2), q.data_ptr(),
+            x.data_ptr(), _HP_CODE[x.dtype], rows, cols, _FP8_CODE[fp8_dtype], _flags(pow2) | few, q.data_ptr(),
             q.stride(0), s.data_ptr(), _stream(x),
         ),
         "mi8_cast_rowwise",

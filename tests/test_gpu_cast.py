@@ -426,3 +426,27 @@ def test_outputs_around_the_line_of_streaming_stores(dev, rows):
         p, ps, p_t, _ = ops.cast_rows_and_colwise_t(x[i:i + part], E4M3)  # (every part holds each of the 64 rows: the same column scales)
         assert torch.equal(u8(rq[i:i + part]), u8(p)) and torch.equal(rs[i:i + part], ps), i
         assert torch.equal(u8(rq_t[:, i:i + part]), u8(p_t[:, :part])), i
+
+
+@pytest.mark.parametrize("rows", [6144, 7000, 12288, 12304])
+def test_rows_cast_for_a_product_of_few_rows(dev, rows, monkeypatch):
+    """12 to 24 MiB and the sizes beside them, stored for products of few and of many rows: the same bytes; a linear says how many
+    rows its product has."""
+    x = seeded((64, 2048), 6).to(dev).repeat(rows // 64 + 1, 1)[:rows].contiguous()
+    want, want_s = (t[:rows] for t in ops.cast_rowwise(x[:64].contiguous(), E4M3))
+    want, want_s = want.view(torch.uint8).repeat(rows // 64 + 1, 1)[:rows], want_s.repeat(rows // 64 + 1)[:rows]
+    for product_rows in (None, 1, 256, 257):
+        q, s = ops.cast_rowwise(x, E4M3, product_rows=product_rows)
+        assert torch.equal(q.view(torch.uint8), want) and torch.equal(s, want_s), product_rows
+
+    from olmo_core_amd.float8.linear import Float8Linear
+    from olmo_core_amd.float8.native_config import Float8LinearConfig
+
+    seen, real = [], ops.cast_rowwise
+    monkeypatch.setattr(ops, "cast_rowwise", lambda t, *a, **k: (seen.append((t.shape[0], k.get("product_rows"))), real(t, *a, **k))[1])
+    lin = Float8Linear.from_float(torch.nn.Linear(2048, rows, bias=False, dtype=torch.bfloat16, device=dev),
+                                  Float8LinearConfig.from_recipe_name("rowwise"))
+    with torch.no_grad():
+        for m in (3, 300):
+            lin(x[:m])
+    assert seen == [(3, None), (rows, 3), (300, None), (rows, 300)]
