@@ -150,3 +150,22 @@ def watch_casts(monkeypatch) -> list:
     library = Library()
     monkeypatch.setattr(_C, "lib", lambda: real() if getattr(_C._recording, "recorder", None) is not None else library)
     return seen
+
+
+# M, N, K of products (swiglu: of each of two projections) and the kinds of tiles the persistent kernel's plan has for them on 256
+# units: W whole; h, q halves and quarters of split tiles; H, Q a row of half or quarter tiles at the end, H-, Q- one that is
+# shifted back over its predecessor; + the last row of tiles repeats rows of the one before
+HALF_PLANS = {
+    (4096, 2048, 256): "h", (2048, 4352, 384): "W", (2560, 2816, 128): "h", (1152, 3328, 128): "H h", (1130, 3328, 128): "H- h",
+    (1300, 6400, 384): "H- W",
+}
+QUARTER_PLANS = {
+    (450, 512, 384): "+ q", (384, 512, 640): "+ q", (777, 1032, 256): "Q- q", (4160, 4096, 128): "Q W", (3000, 5632, 256): "H Q- W",
+    (3456, 4864, 128): "+ W q", (1600, 5120, 384): "Q h", (700, 11008, 384): "H Q- h", (640, 43776, 128): "H W h q",
+}
+HALF_SWIGLU_PLANS = {(4096, 1024, 256): "h", (1130, 1664, 128): "H- h", (1600, 2560, 128): "H- W", (2048, 2176, 256): "W"}
+QUARTER_SWIGLU_PLANS = {(450, 520, 128): "+ q", (777, 1416, 384): "Q- q", (777, 11008, 384): "Q- W q", (3000, 5632, 256): "H Q- W"}
+ACCUMULATE_PLANS = {
+    (2048, 8192, 2048): "W", (4096, 2048, 4096): "h", (1920, 8192, 2048): "H W", (2048, 11008, 2048): "W h", (3328, 5632, 256): "W q",
+    (640, 43776, 128): "H W h q",
+}

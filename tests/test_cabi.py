@@ -6,6 +6,7 @@ from pathlib import Path
 
 import pytest
 
+import helpers
 from olmo_core_amd import _C
 
 ROOT = Path(__file__).resolve().parent.parent
@@ -203,3 +204,18 @@ def test_slots_that_the_counting_sort_takes():
         assert words(n, experts) >= -(-n // 1024) * (experts + 2 + 1024), (n, experts)
     for n, experts in ((1 << 21, 256), (1 << 22, 64), (1 << 24, 1), ((1 << 30) - 1, 1), (1 << 30, 8), (131072, 257), (0, 8), (8193, 0)):
         assert words(n, experts) == 0, (n, experts)
+
+
+@pytest.mark.parametrize("plans,how", [("HALF_PLANS", {}), ("QUARTER_PLANS", {}), ("HALF_SWIGLU_PLANS", dict(swiglu=1)),
+                                       ("QUARTER_SWIGLU_PLANS", dict(swiglu=1)), ("ACCUMULATE_PLANS", dict(accumulate=1))], ids=str)
+def test_sizes_of_the_tile_tests_have_the_tiles_they_are_for(plans, how):
+    for (M, N, K), kinds in getattr(helpers, plans).items():
+        p = _plan(M, N, K, **how)
+        end = 256 * p["rows"]  # where the rows at the end start
+        found = ["W"] * (p["whole"] > 0) + ["h"] * (p["split_halves"] > 0) + ["q"] * (p["split_quarters"] > 0) + ["+"] * (end > M)
+        if p["halves"] > p["split_halves"]:
+            found.append("H" if end + 128 <= M else "H-")
+            end += 128
+        if p["quarters"] > p["split_quarters"]:
+            found.append("Q" if end + 64 <= M else "Q-")
+        assert " ".join(sorted(found)) == kinds, (M, N, K, p)

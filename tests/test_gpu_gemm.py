@@ -4,7 +4,8 @@ exactness on integer-valued operands."""
 import pytest
 import torch
 
-from helpers import E4M3, E5M2, assert_gemm_close, seeded
+from helpers import (ACCUMULATE_PLANS, E4M3, E5M2, HALF_PLANS, HALF_SWIGLU_PLANS, QUARTER_PLANS, QUARTER_SWIGLU_PLANS, assert_gemm_close,
+                     seeded)
 from oracle import float8_oracle as O
 from olmo_core_amd.exceptions import MI8KernelError
 
@@ -417,12 +418,9 @@ def test_split_k_accumulates_as_an_add(dev, mnk, dt):
     assert torch.equal(got, want)
 
 
-# half rows of tiles (128 x 256): every tile split, a partial last round split, an odd half row at the end (alone, and
-# shifted back over its predecessor), whole tiles only
-HALF_SHAPES = [(4096, 2048, 256), (2048, 4352, 384), (2560, 2816, 128), (384, 512, 640), (777, 1032, 256), (1300, 6400, 384)]
-
-
-@pytest.mark.parametrize("mnk", HALF_SHAPES, ids=lambda s: "x".join(map(str, s)))
+# half tiles (128 x 256): every tile split, a row of them at the end (whole, and shifted back over its predecessor), beside whole
+# tiles and beside split ones; whole tiles only
+@pytest.mark.parametrize("mnk", HALF_PLANS, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
 def test_half_tiles_of_the_persistent_kernel(dev, mnk, vec):
     """The persistent kernel's plan of whole and half tiles against the ring tiles (same bits) and, for single scales, the
@@ -442,11 +440,10 @@ def test_half_tiles_of_the_persistent_kernel(dev, mnk, vec):
         assert torch.equal(out, want) and torch.equal(codes, ops.rowseg_max_codes(want))
 
 
-@pytest.mark.parametrize("mnk", [(2048, 8192, 2048), (4096, 2048, 4096), (1920, 8192, 2048), (2048, 11008, 2048)],
-                         ids=["whole", "halves", "whole+odd half row", "whole+halves"])
+@pytest.mark.parametrize("mnk", ACCUMULATE_PLANS, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
 def test_persistent_kernel_accumulates_as_an_add(dev, mnk, vec):
-    """C += product on shapes that the library gives to the persistent kernel, on whole and on half tiles, also into a view
+    """C += product on shapes that the library gives to the persistent kernel, on whole, half and quarter tiles, also into a view
     with a row pitch: the bits of the ring tiles' product and an elementwise add."""
     M, N, K = mnk
     names = ops.gemm_variants()
@@ -478,7 +475,7 @@ def test_large_ring_tiles_accumulate_as_an_add(dev, mnk, dt):
     assert torch.equal(ops.gemm_fp8(a, sa, b, sb, out_dtype=dt, out=first.clone(), accumulate=True), want)
 
 
-@pytest.mark.parametrize("mhk", [(4096, 1024, 256), (777, 1416, 384), (2048, 2176, 256)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("mhk", HALF_SWIGLU_PLANS, ids=lambda s: "x".join(map(str, s)))
 def test_half_tiles_of_the_fused_swiglu_launch(dev, mhk):
     M, H, K = mhk
     xq, _, sx = ops.cast_tensorwise(seeded((M, K), 61).to(dev), E4M3)
@@ -496,19 +493,15 @@ def test_half_tiles_of_the_fused_swiglu_launch(dev, mhk):
         assert torch.equal(codes[0], ops.rowseg_max_codes(x1, x3))
 
 
-# quarter tiles (64 x 256): all of them, a row of them at the end (whole, and shifted back), whole and half tiles beside them
-@pytest.mark.parametrize("mnk", [(450, 512, 384), (777, 1032, 256), (4160, 4096, 128), (3000, 5632, 256)], ids=lambda s: "x".join(map(str, s)))
+# quarter tiles (64 x 256): all of them, a row of them at the end (whole, and shifted back), split tiles of whole and repeated rows,
+# whole, split and half tiles beside them
+@pytest.mark.parametrize("mnk", QUARTER_PLANS, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
 def test_quarter_tiles_of_the_persistent_kernel(dev, mnk, vec):
     test_half_tiles_of_the_persistent_kernel(dev, mnk, vec)
 
 
-@pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
-def test_quarter_tiles_accumulate_as_an_add(dev, vec):
-    test_persistent_kernel_accumulates_as_an_add(dev, (3328, 5632, 256), vec)  # 256 whole tiles and 120 quarters
-
-
-@pytest.mark.parametrize("mhk", [(450, 520, 128), (777, 11008, 384), (3000, 5632, 256)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("mhk", QUARTER_SWIGLU_PLANS, ids=lambda s: "x".join(map(str, s)))
 def test_quarter_tiles_of_the_fused_swiglu_launch(dev, mhk):
     test_half_tiles_of_the_fused_swiglu_launch(dev, mhk)
 
