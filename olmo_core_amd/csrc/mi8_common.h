@@ -46,11 +46,11 @@ static inline bool streams_outputs(int64_t bytes, int64_t end, int64_t end2 = 0)
     return bytes > (int64_t)192 << 20 || bytes <= (int64_t)1 << 20 || end >= 0x7FFFFFF0 || end2 >= 0x7FFFFFF0;
 }
 // A weight that a product of few rows reads (MI8_FLAG_READ_BY_FEW_ROWS: up to 256) is read once, and of rows up to 2048 long 12 to 24 MiB
-// are streamed for it.  us of a linear with a scale per row, streamed / kept: 2048 -> 8192 (16.8 MB) 1 row 22.7 / 23.7, 64 30.0 / 31.3, 256 32.4 / 33.9,
-// 777 40.3 / 37.6, 2048 47.8 / 46.8; 1024 -> 20480 64 33.5 / 36.0; 2048 -> 11264 (23.1) 34.8 / 36.5; below and beyond 2048 -> 5120 (10.5) 24.0 / 22.8,
-// 64 -> 25.2 MB 35.5 / 36.5 and 256 40.1 / 38.2; longer rows 4096 -> 4096 34.8 / 34.5, -> 5120 38.3 / 35.1, 8192 -> 2048 30.3 / 32.4, 256
-// 40.9 / 36.9.  (Activations and the rows of experts are kept: 4096 x 4096 42.0 / 38.1, 8192 x 2048 48.0 / 50.3, 9000 x 2048 60.6 / 57.6, a layer of 8
-// experts, 4096 tokens of 1024 157 / 137.)
+// are streamed for it.  us of a linear with a scale per row, streamed / kept: 2048 -> 8192 (16.8 MB) of 1 row 22.7 / 23.7, 64 rows 30.0 / 31.3, 256 32.4 /
+// 33.9, 777 40.3 / 37.6, 2048 47.8 / 46.8; of 64 rows 1024 -> 20480 33.5 / 36.0, 2048 -> 11264 (23.1 MB) 34.8 / 36.5.  Beside that, of 64 rows: 2048 -> 5120
+// (10.5 MB) 24.0 / 22.8, -> 12288 (25.2 MB) 35.5 / 36.5 and of 256 40.1 / 38.2; longer rows 4096 -> 4096 34.8 / 34.5, -> 5120 38.3 / 35.1, 8192 -> 2048 30.3 /
+// 32.4 and of 256 40.9 / 36.9.  (Activations and the rows of experts are kept: 4096 x 4096 42.0 / 38.1, 8192 x 2048 48.0 / 50.3, 9000 x 2048 60.6 / 57.6, a layer
+// of 8 experts, 4096 tokens of 1024 157 / 137.)
 static inline bool streams_rows(int64_t rows, int64_t cols, int64_t ld_out, bool by_few_rows)
 {
     const int64_t bytes = rows * cols;
