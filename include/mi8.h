@@ -247,7 +247,7 @@ int mi8_gemm_fp8_accumulate(const void* a, int a_dtype, int64_t lda, const void*
  * mi8_swiglu_bwd_amax_from_codes. */
 int mi8_gemm_fp8_swiglu_matches_separate(int64_t M, int64_t H, int64_t K); /* host only: 1 if the fused launch takes
     the shape, which has more than 96 tiles of 256 x 256: the library then cuts neither projection along K, so that the bits agree as well */
-int mi8_gemm_fp8_swiglu_pays(int64_t M, int64_t H, int64_t K); /* host only: 1 for those shapes and for those of fewer
+int mi8_gemm_fp8_swiglu_pays(int64_t M, int64_t H, int64_t K); /* host only: 1 for those shapes and, with K >= 512, for those of fewer
     tiles whose projections would not be cut along K */
 int mi8_gemm_fp8_swiglu(const void* a, int a_dtype, int64_t lda, const void* b1, const void* b3, int b_dtype, int64_t ldb,
                         int64_t M, int64_t H, int64_t K, const float* sa, const float* sb1, const float* sb3, void* x1,

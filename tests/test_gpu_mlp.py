@@ -157,17 +157,17 @@ def test_swiglu_fused_into_the_projection_gemm(dev, mhk, a_fp8):
     assert_bf16_pointwise_close(h, O.swiglu(x1.cpu(), x3.cpu()), "h vs oracle")
 
 
-@pytest.mark.parametrize("mdh", [(256, 512, 256), (300, 768, 2048), (400, 640, 264), (1999, 1024, 2816), (256, 4096, 1024), (512, 1152, 512), (300, 256, 2048), (777, 128, 320), (4000, 384, 1040)],
+@pytest.mark.parametrize("mdh", [(256, 512, 256), (300, 768, 2048), (400, 640, 264), (1999, 1024, 2816), (256, 4096, 1024), (512, 1152, 512), (300, 256, 2048)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_fused_launch_of_few_tiles_gives_identical_block_results(dev, mdh):
-    """The block on both routes where the projections have at most 96 tiles; where the library would cut them along K the block keeps
-    the separate launches."""
+    """The block on both routes where the projections have at most 96 tiles; where the library would cut them along K, or K is short,
+    the block keeps the separate launches."""
     from olmo_core_amd.nn import feed_forward as ff_mod
 
     M, D, H = mdh
     assert not ops.swiglu_gemm_matches_separate(M, H, D)
-    assert ops.swiglu_gemm_pays(M, H, D) == (ops._C.lib().mi8_gemm_splitk_suggest(M, H, D) == 1)
-    assert ops.swiglu_gemm_pays(M, H, D) == (mdh not in [(256, 4096, 1024), (512, 1152, 512)])
+    assert ops.swiglu_gemm_pays(M, H, D) == (D >= 512 and ops._C.lib().mi8_gemm_splitk_suggest(M, H, D) == 1)
+    assert ops.swiglu_gemm_pays(M, H, D) == (mdh not in [(256, 4096, 1024), (512, 1152, 512), (300, 256, 2048)])
     x, go = seeded((M, D), 1).to(dev), seeded((M, D), 2, std=1e-3).to(dev)
     res = []
     for flag in (True, False):
