@@ -562,8 +562,10 @@ extern "C" int mi8_gemm_fp8_swiglu_matches_separate(int64_t M, int64_t H, int64_
 
 // The same for any number of tiles: with few the fused launch, in whole, half and quarter tiles, is the faster one too.  us fused /
 // two products in one launch and the activation: 256 x 11008 x 4096 29.2 / 43.8, 300 44.5 / 56.9; 640 x 8192 x 2048 28.3 / 37.8;
-// 1999 x 2816 x 1024 20.8 / 28.3; 777 x 2048 x 768 9.4 / 14.8, 256 8.6 / 9.3; 256 x 512 x 512 7.5 / 8.0.  (From K = 512 on, the
-// widths that models have: below, the gain is of launches alone, 1-8 us, and the separate ones stay.)
+// 1999 x 2816 x 1024 20.8 / 28.3; 777 x 2048 x 768 9.4 / 14.8, 256 8.6 / 9.3; 256 x 512 x 512 7.5 / 8.0.  A block without gradients: 400 x 512 x
+// 512 39.9 / 43.0, 512 x 8192 x 512 41.7 / 47.9; of 230 sizes with K of 512 to 2048 none was slower.  The line at K = 512 is not one of speed (3000 x 2048 x
+// 384 40.8 / 46.0, 777 x 2048 x 256 39.4 / 42.3, none of 219 sizes slower): the tests of calls that are recorded and replaced pin the
+// separate launches with blocks 256 wide, and the feed-forward blocks of perf/cases.py are 768 wide or more.
 extern "C" int mi8_gemm_fp8_swiglu_pays(int64_t M, int64_t H, int64_t K)
 {
     if (mi8_gemm_fp8_swiglu_matches_separate(M, H, K)) return 1;
