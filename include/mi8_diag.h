@@ -1,7 +1,7 @@
 /*
  * mi8 diagnostics: C ABI of libmi8_diag.so, a separate library with measurement kernels that are no part of the
  * float8 linear path and of its drop-in boundary (include/mi8.h, libmi8.so).  Built by the same recipe
- * (python -m olmo_core_amd.build); loaded only by bench.py (--power-probe, --feed-probe, --store-probe, --tile-timeline).  No counterpart in the
+ * (python -m olmo_core_amd.build); loaded by bench.py (--power-probe, --feed-probe, --store-probe, --tile-timeline) and tests only.  No counterpart in the
  * reference.  Conventions as in mi8.h: int status (0 = ok), mi8_diag_last_error() for the text, work is only
  * enqueued on `stream`.
  */

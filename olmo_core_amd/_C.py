@@ -254,7 +254,7 @@ _SIGNATURES = {
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
-# libmi8_diag.so (include/mi8_diag.h): measurement kernels, loaded by bench.py only
+# libmi8_diag.so (include/mi8_diag.h): measurement kernels and the plan of the persistent one, loaded by bench.py and tests only
 DIAG_LIB_PATH = LIB_PATH.parent / "libmi8_diag.so"
 _DIAG_SIGNATURES = {
     "mi8_diag_last_error": (c_char_p, []),
