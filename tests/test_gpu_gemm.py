@@ -4,8 +4,7 @@ exactness on integer-valued operands."""
 import pytest
 import torch
 
-from helpers import (ACCUMULATE_PLANS, E4M3, E5M2, HALF_PLANS, HALF_SWIGLU_PLANS, QUARTER_PLANS, QUARTER_SWIGLU_PLANS, assert_gemm_close,
-                     seeded)
+from helpers import E4M3, E5M2, HALF_PLANS, HALF_SWIGLU_PLANS, QUARTER_PLANS, QUARTER_SWIGLU_PLANS, assert_gemm_close, seeded
 from oracle import float8_oracle as O
 from olmo_core_amd.exceptions import MI8KernelError
 
@@ -440,10 +439,11 @@ def test_half_tiles_of_the_persistent_kernel(dev, mnk, vec):
         assert torch.equal(out, want) and torch.equal(codes, ops.rowseg_max_codes(want))
 
 
-@pytest.mark.parametrize("mnk", ACCUMULATE_PLANS, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("mnk", [(2048, 8192, 2048), (4096, 2048, 4096), (1920, 8192, 2048), (2048, 11008, 2048)],
+                         ids=["whole", "halves", "whole+odd half row", "whole+halves"])
 @pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
 def test_persistent_kernel_accumulates_as_an_add(dev, mnk, vec):
-    """C += product on shapes that the library gives to the persistent kernel, on whole, half and quarter tiles, also into a view
+    """C += product on shapes that the library gives to the persistent kernel, on whole and on half tiles, also into a view
     with a row pitch: the bits of the ring tiles' product and an elementwise add."""
     M, N, K = mnk
     names = ops.gemm_variants()
@@ -499,6 +499,16 @@ def test_half_tiles_of_the_fused_swiglu_launch(dev, mhk):
 @pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
 def test_quarter_tiles_of_the_persistent_kernel(dev, mnk, vec):
     test_half_tiles_of_the_persistent_kernel(dev, mnk, vec)
+
+
+@pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
+def test_quarter_tiles_accumulate_as_an_add(dev, vec):
+    test_persistent_kernel_accumulates_as_an_add(dev, (3328, 5632, 256), vec)  # 256 whole tiles and 120 quarters
+
+
+@pytest.mark.parametrize("vec", [False, True], ids=["single-scales", "scale-vectors"])
+def test_tiles_of_all_kinds_accumulate_as_an_add(dev, vec):
+    test_persistent_kernel_accumulates_as_an_add(dev, (640, 43776, 128), vec)
 
 
 @pytest.mark.parametrize("mhk", QUARTER_SWIGLU_PLANS, ids=lambda s: "x".join(map(str, s)))
